@@ -145,6 +145,28 @@ def load() -> C.CDLL:
     return lib
 
 
+class HipKernelError(RuntimeError):
+    """A C-ABI call returned a negative status."""
+
+
+_host = None
+
+
+def host():
+    """The native host path of the ops (csrc/host_ops.cpp); raises if it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError("linearnexus_amd/_host.so is missing or does not load: build it with `python -m linearnexus_amd.build` "
+                               "(there is no CPU or PyTorch fallback for these ops)") from e
+        module.set_kernel_error(HipKernelError)
+        _host = module
+    return _host
+
+
 def profile_enable(on: bool) -> None:
     """Turns per-kernel HIP-event timing on or off for the calling thread."""
     load().lnx_profile_enable(int(on))
@@ -156,10 +178,6 @@ def profile_read(capacity: int = 8192):
     ms = (C.c_float * capacity)()
     n = load().lnx_profile_read(capacity, names, ms)
     return [(names[i].decode(), float(ms[i])) for i in range(min(n, capacity))]
-
-
-class HipKernelError(RuntimeError):
-    """A C-ABI call returned a negative status."""
 
 
 def check(status: int, what: str) -> None:

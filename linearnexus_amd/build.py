@@ -1,7 +1,8 @@
-"""Builds liblinearnexus_hip.so for gfx950 with hipcc (cross-compiles without a GPU).
+"""Builds liblinearnexus_hip.so for gfx950 with hipcc (cross-compiles without a GPU) and _host.so, the host path of the
+Python ops, with g++.
 
-Usage: ``python -m linearnexus_amd.build``.  The library is written next to this file so
-that it travels with the source tree; nothing is installed.
+Usage: ``python -m linearnexus_amd.build``.  The libraries are written next to this file so
+that they travel with the source tree; nothing is installed.
 """
 from __future__ import annotations
 
@@ -13,6 +14,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liblinearnexus_hip.so")
+HOST = os.path.join(HERE, "_host.so")
 SOURCES = ["c_api.hip", "recurrent.hip", "chunk_fwd.hip", "chunk_bwd.hip", "chunk_direct.hip", "conv1d.hip", "dplr.hip", "rmsnorm_gated.hip", "kda_gate.hip", "gdn_gate.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffast-math", "-fno-finite-math-only",
@@ -34,16 +36,45 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_host() -> str:
+    """csrc/host_ops.cpp against torch's headers."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    obj = os.path.join(CSRC, "host_ops.o")
+    inc = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", *(f"-I{i}" for i in inc),
+           "-c", os.path.join(CSRC, "host_ops.cpp"), "-o", obj]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on host_ops.cpp:\n" + r.stderr)
+    return obj
+
+
+def _link_host(obj: str) -> None:
+    from torch.utils import cpp_extension
+
+    cmd = ["g++", "-shared", "-o", HOST, obj, f"-L{HERE}", "-llinearnexus_hip", *(f"-L{p}" for p in cpp_extension.library_paths()),
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("linking _host.so failed:\n" + r.stderr)
+
+
 def build(verbose: bool = True) -> str:
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
-    with ThreadPoolExecutor(max_workers=min(4, len(srcs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(5, len(srcs) + 1)) as ex:
+        host_obj = ex.submit(_compile_host)
         objs = list(ex.map(_compile, srcs))
+        host_obj = host_obj.result()
     cmd = ["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr)
+    _link_host(host_obj)
     if verbose:
-        print(f"built {LIB} from {', '.join(srcs)}")
+        print(f"built {LIB} from {', '.join(srcs)} and {HOST} from host_ops.cpp")
     build_c_abi_smoke(verbose)
     build_xla_ffi(verbose)
     return LIB

@@ -21,7 +21,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from ._lib import GATE_NONE, GATE_SCALAR, GATE_VECTOR, LNX_BF16, LNX_F32, ScanArgs
+from ._lib import LNX_BF16, LNX_F32
 
 Tensor = torch.Tensor
 _DT = {torch.float32: LNX_F32, torch.bfloat16: LNX_BF16}
@@ -32,15 +32,7 @@ CHUNK = 64  # the kernels' chunk length; results do not depend on it
 # helpers
 # --------------------------------------------------------------------------------------
 
-def _stream(t: Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
-
-
-def _ptr(t: Optional[Tensor]) -> Optional[int]:
-    return None if t is None else t.data_ptr()
-
-
-def _check_inputs(q: Tensor, k: Tensor, v: Tensor) -> int:
+def _check_inputs(q: Tensor, k: Tensor, v: Tensor) -> None:
     for name, t in (("q", q), ("k", k), ("v", v)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{name} must be a torch.Tensor on an AMD GPU, got {type(t).__name__}")
@@ -52,7 +44,6 @@ def _check_inputs(q: Tensor, k: Tensor, v: Tensor) -> int:
         raise RuntimeError(f"q, k, v must share one dtype, got {q.dtype}, {k.dtype}, {v.dtype}")
     if q.shape != k.shape or q.shape[:-1] != v.shape[:-1]:
         raise RuntimeError(f"shape mismatch: q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)}")
-    return _DT[q.dtype]
 
 
 def _f32(t: Tensor) -> Tensor:
@@ -80,71 +71,14 @@ def _promote(q: Tensor, k: Tensor, v: Tensor):
     return q.to(torch.float32), k.to(torch.float32), v.to(torch.float32), q.dtype
 
 
-# Memory layout of the token tensors.  The ops take the reference's head-first [B, H, T, .] shapes; a caller
-# whose data lives token-first -- [B, T, H, .], what the reference's blocks hold before they transpose
-# (delta_net.py:645-647) -- passes ``x.transpose(1, 2)`` views, and the kernels then read and write that
-# memory in place (``token_first`` in the argument block) instead of working on contiguous copies.
-
-def _is_token_first(x: Tensor) -> bool:
-    return x.dim() >= 3 and not x.is_contiguous() and x.transpose(1, 2).is_contiguous()
-
-
-def _as_layout(x: Optional[Tensor], token_first: bool) -> Optional[Tensor]:
-    """``x`` (logical [B, H, T, ...]) with dense memory in the chosen layout; no copy when it already has it."""
-    if x is None:
-        return None
-    if x.data_ptr() % 16:  # a dense view that starts inside a 16-byte vector of its storage: the kernels need a copy
-        x = x.clone(memory_format=torch.preserve_format)
-    if token_first:
-        return x if _is_token_first(x) else x.transpose(1, 2).contiguous().transpose(1, 2)
-    return x.contiguous()
-
-
-def _empty_layout(B, H, T, tail, dtype, device, token_first: bool) -> Tensor:
-    if token_first:
-        return torch.empty((B, T, H) + tuple(tail), dtype=dtype, device=device).transpose(1, 2)
-    return torch.empty((B, H, T) + tuple(tail), dtype=dtype, device=device)
-
-
-def _dense(x: Tensor):
-    """A contiguous tensor over x's memory (or a copy) and the function that maps results back to x's layout."""
-    if x.is_contiguous():
-        return x, (lambda y: y)
-    if x.dim() >= 4 and _is_token_first(x):  # with fewer dimensions the transposition would move the last axis itself
-        return x.transpose(1, 2), (lambda y: y.transpose(1, 2))
-    return x.contiguous(), (lambda y: y)
-
-
 def _squeeze_beta(beta: Tensor, ndim: int) -> Tensor:
     # delta_net.py:166-167, :257-258, :378-379 -- a trailing singleton is accepted
     return beta.squeeze(-1) if beta.dim() == ndim else beta
 
 
-def _gate_kind(g: Optional[Tensor], lead_shape, dk: int) -> int:
-    if g is None:
-        return GATE_NONE
-    if tuple(g.shape) == tuple(lead_shape):
-        return GATE_SCALAR
-    if tuple(g.shape) == tuple(lead_shape) + (dk,):
-        return GATE_VECTOR
-    raise RuntimeError(f"gate shape {tuple(g.shape)} matches neither {tuple(lead_shape)} nor {tuple(lead_shape) + (dk,)}")
-
-
 # Test hooks: the tiling overrides of ``lnx_scan_args`` (0 = the library's choice).  The GPU tests set them to reach both
 # slab widths of the sequential kernels, and the grouped form of the fp32 output kernel, at small shapes.
 _test_hooks = {"scan_slab": 0, "out_slabs": 0}
-
-
-def _base_args(B, H, T, dk, dv, dtype, o_dtype, gate, l2norm, scale) -> ScanArgs:
-    a = ScanArgs()
-    a.test_scan_slab, a.test_out_slabs = _test_hooks["scan_slab"], _test_hooks["out_slabs"]
-    a.B, a.H, a.T, a.dk, a.dv = B, H, T, dk, dv
-    a.chunk = CHUNK
-    a.dtype, a.o_dtype, a.gate = dtype, o_dtype, gate
-    a.use_qk_l2norm = int(bool(l2norm))
-    a.nseq = 0
-    a.scale = float(scale)
-    return a
 
 
 # --------------------------------------------------------------------------------------
@@ -203,13 +137,20 @@ class KDAState(_GatedState):
 # --------------------------------------------------------------------------------------
 
 def _step(q, k, v, g, beta, state, scale, l2norm, o_dtype_from_state, inplace):
+    # contiguous inputs of one kernel dtype with fp32 beta, g and state and no gradient wanted: a decode loop's calls
+    out = _lib.host().step(q, k, v, g, beta, state, scale, l2norm, o_dtype_from_state, inplace)
+    return _step_general(q, k, v, g, beta, state, scale, l2norm, o_dtype_from_state, inplace) if out is None else out
+
+
+def _step_general(q, k, v, g, beta, state, scale, l2norm, o_dtype_from_state, inplace):
     q, k, v, back = _promote(q, k, v)
     if back is not None:
         o, s_out = _step(q, k, v, g, beta, state, scale, l2norm, o_dtype_from_state, inplace)
         return (o if o_dtype_from_state else o.to(back)), s_out
-    dt = _check_inputs(q, k, v)
+    _check_inputs(q, k, v)
     if q.dim() != 3:
         raise RuntimeError(f"step ops take [B, H, d] vectors, got q {tuple(q.shape)}")
+    beta = _squeeze_beta(beta, 3)
     if _wants_grad(q, k, v, g, beta, state):
         if inplace:
             raise RuntimeError("inplace=True overwrites the state a backward pass would need")
@@ -217,35 +158,24 @@ def _step(q, k, v, g, beta, state, scale, l2norm, o_dtype_from_state, inplace):
         # values do not depend on whether a gradient is wanted
         up = (lambda t: t.to(torch.float32)) if (l2norm and q.dtype != torch.float32) else (lambda t: t)
         o, s_out = _chunk(up(q)[:, :, None], up(k)[:, :, None], up(v)[:, :, None], None if g is None else g[:, :, None],
-                          _squeeze_beta(beta, 3)[:, :, None], scale, state, CHUNK, l2norm,
+                          beta[:, :, None], scale, state, CHUNK, l2norm,
                           torch.float32 if (o_dtype_from_state or l2norm) else q.dtype, False, None)
         return o[:, :, 0].to(state.dtype if o_dtype_from_state else q.dtype), s_out
     B, H, dk = q.shape
     dv = v.shape[-1]
-    beta = _squeeze_beta(beta, 3)
-    gate = _gate_kind(g, (B, H), dk)
+    if g is not None and tuple(g.shape) not in ((B, H), (B, H, dk)):
+        raise RuntimeError(f"gate shape {tuple(g.shape)} matches neither {(B, H)} nor {(B, H, dk)}")
+    if tuple(beta.shape) != (B, H):
+        raise RuntimeError(f"beta shape {tuple(beta.shape)} != {(B, H)}")
     if tuple(state.shape) != (B, H, dk, dv):
         raise RuntimeError(f"state shape {tuple(state.shape)} != {(B, H, dk, dv)}")
-    if scale is None:
-        scale = dk ** -0.5
-    if inplace:
-        if state.dtype != torch.float32 or not state.is_contiguous():
-            raise RuntimeError("inplace=True needs a contiguous float32 state")
-        s_in = s_out = state
-    else:
-        s_in = _f32(state)
-        s_out = torch.empty_like(s_in)
-    o_t = torch.float32 if o_dtype_from_state else q.dtype
-    o = torch.empty(B, H, dv, dtype=o_t, device=q.device)
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-    beta = _f32(beta)
-    g = None if g is None else _f32(g)
-    a = _base_args(B, H, 1, dk, dv, dt, _DT[o_t], gate, l2norm, scale)
-    a.q, a.k, a.v, a.beta, a.g = _ptr(q), _ptr(k), _ptr(v), _ptr(beta), _ptr(g)
-    a.initial_state, a.final_state, a.o = _ptr(s_in), _ptr(s_out), _ptr(o)
-    lib = _lib.load()
-    _lib.check(lib.lnx_decode_step(a, _stream(q)), "lnx_decode_step")
-    return o, s_out
+    if inplace and (state.dtype != torch.float32 or not state.is_contiguous()):
+        raise RuntimeError("inplace=True needs a contiguous float32 state")
+    out = _lib.host().step(q.contiguous(), k.contiguous(), v.contiguous(), None if g is None else _f32(g), _f32(beta),
+                           _f32(state), scale, l2norm, o_dtype_from_state, inplace)
+    if out is None:
+        raise RuntimeError("beta, g and state must be on the GPU of q, k and v")
+    return out
 
 
 def delta_rule_step(q, k, v, beta, state, scale=None, *, inplace=False) -> Tuple[Tensor, Tensor]:
@@ -267,28 +197,6 @@ def kda_step(q, k, v, g, beta, state, scale=None, use_qk_l2norm=True, *, inplace
 # token-by-token scan
 # --------------------------------------------------------------------------------------
 
-def _seq_setup(q, k, v, g, beta, initial_state, cu_seqlens):
-    dt = _check_inputs(q, k, v)
-    if q.dim() != 4:
-        raise RuntimeError(f"scan ops take [B, H, T, d] tensors, got q {tuple(q.shape)}")
-    B, H, T, dk = q.shape
-    dv = v.shape[-1]
-    beta = _squeeze_beta(beta, 4)
-    if tuple(beta.shape) != (B, H, T):
-        raise RuntimeError(f"beta shape {tuple(beta.shape)} != {(B, H, T)}")
-    gate = _gate_kind(g, (B, H, T), dk)
-    nseq = 0
-    if cu_seqlens is not None:
-        if B != 1:
-            raise RuntimeError("cu_seqlens needs a packed batch with B == 1")
-        cu_seqlens = _check_cu_seqlens(cu_seqlens, T).to(device=q.device, dtype=torch.int32).contiguous()
-        nseq = cu_seqlens.numel() - 1
-    nstate = nseq if nseq else B
-    if initial_state is not None and tuple(initial_state.shape) != (nstate, H, dk, dv):
-        raise RuntimeError(f"initial_state shape {tuple(initial_state.shape)} != {(nstate, H, dk, dv)}")
-    return dt, B, H, T, dk, dv, beta, gate, nseq, nstate, cu_seqlens
-
-
 def _check_cu_seqlens(cu, T: int) -> Tensor:
     """``cu_seqlens`` as an integer tensor.  A table that lives on the host (list, numpy array, CPU tensor) is
     validated here: one-dimensional, at least two entries, ``cu[0] == 0``, non-decreasing, ``cu[-1] == T`` -- every
@@ -308,6 +216,13 @@ def _check_cu_seqlens(cu, T: int) -> Tensor:
     return cu
 
 
+def _packed_table(cu_seqlens, q: Tensor) -> Optional[Tensor]:
+    """The checked table as the kernels read it: int32 on q's device."""
+    if cu_seqlens is None:
+        return None
+    return _check_cu_seqlens(cu_seqlens, q.shape[2]).to(device=q.device, dtype=torch.int32).contiguous()
+
+
 def _recurrent(q, k, v, g, beta, scale, initial_state, l2norm, cu_seqlens=None):
     q, k, v, back = _promote(q, k, v)
     if back is not None:
@@ -319,24 +234,8 @@ def _recurrent(q, k, v, g, beta, scale, initial_state, l2norm, cu_seqlens=None):
                            l2norm, torch.float32, False, cu_seqlens)
             return o.to(q.dtype), sT
         return _chunk(q, k, v, g, beta, scale, initial_state, CHUNK, l2norm, q.dtype, False, cu_seqlens)
-    dt, B, H, T, dk, dv, beta, gate, nseq, nstate, cu = _seq_setup(q, k, v, g, beta, initial_state, cu_seqlens)
-    if scale is None:
-        scale = dk ** -0.5
-    tf = all(_is_token_first(t) for t in (q, k, v))
-    q, k, v = _as_layout(q, tf), _as_layout(k, tf), _as_layout(v, tf)
-    beta = _as_layout(beta.to(torch.float32), tf)
-    g = None if g is None else _as_layout(g.to(torch.float32), tf)
-    s0 = None if initial_state is None else _f32(initial_state)
-    o = _empty_layout(B, H, T, (dv,), q.dtype, q.device, tf)
-    sT = torch.empty(nstate, H, dk, dv, dtype=torch.float32, device=q.device)
-    a = _base_args(B, H, T, dk, dv, dt, dt, gate, l2norm, scale)
-    a.nseq = nseq
-    a.token_first = int(tf)
-    a.q, a.k, a.v, a.beta, a.g = _ptr(q), _ptr(k), _ptr(v), _ptr(beta), _ptr(g)
-    a.initial_state, a.final_state, a.o, a.cu_seqlens = _ptr(s0), _ptr(sT), _ptr(o), _ptr(cu)
-    lib = _lib.load()
-    _lib.check(lib.lnx_recurrent_fwd(a, _stream(q)), "lnx_recurrent_fwd")
-    return o, sT
+    cu = None if cu_seqlens is None else _packed_table(cu_seqlens, q)
+    return _lib.host().recurrent(q, k, v, g, beta, initial_state, scale, l2norm, cu)
 
 
 def delta_rule_recurrent(q, k, v, beta, initial_state=None, scale=None, backend=None, *, cu_seqlens=None):
@@ -362,155 +261,25 @@ def kda_recurrent(q, k, v, g, beta, scale=None, initial_state=None, use_qk_l2nor
 def l2norm_rows(x: Tensor) -> Tensor:
     """``x / (|x|_2 + 1e-6)`` over the last dimension, in x's dtype (gated_deltanet.py:273-275; what the DeltaNet
     block applies to q and k before the op, delta_net.py:566-575).  Differentiable."""
-    if _wants_grad(x):
-        return _L2Norm.apply(x)
-    return _l2norm_rows_fwd(x)
-
-
-def _l2norm_rows_fwd(x: Tensor) -> Tensor:
-    x, back = _dense(x)
-    y = torch.empty_like(x)
-    d = x.shape[-1]
-    _lib.check(_lib.load().lnx_l2norm_fwd(_ptr(x), _ptr(y), x.numel() // d, d, _DT[x.dtype], _stream(x)), "lnx_l2norm_fwd")
-    return back(y)
+    return _lib.host().l2norm(x)
 
 
 def _l2norm_rows_bwd(x: Tensor, dy: Tensor) -> Tensor:
-    x, back = _dense(x)
-    dy = back(dy)  # same logical shape; bring it to x's dense memory order (back is its own inverse)
-    dy = dy if dy.is_contiguous() else dy.contiguous()
-    dx = torch.empty_like(x)
-    d = x.shape[-1]
-    _lib.check(_lib.load().lnx_l2norm_bwd(_ptr(x), _ptr(dy), _ptr(dx), x.numel() // d, d, _DT[x.dtype], _stream(x)),
-               "lnx_l2norm_bwd")
-    return back(dx)
-
-
-class _L2Norm(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x):
-        ctx.save_for_backward(x)
-        return _l2norm_rows_fwd(x)
-
-    @staticmethod
-    def backward(ctx, dy):
-        (x,) = ctx.saved_tensors
-        return _l2norm_rows_bwd(x, dy.to(x.dtype))
+    return _lib.host().l2norm_bwd(x, dy)
 
 
 def _chunk_forward(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens, forward_only,
                    dv_total=None, want_o=True, raw_gate=None):
-    """One lnx_chunk_fwd call.  ``dv_total`` > v's columns: the state has dv_total value columns of which v holds the
-    first ones and the others are zero (``value_cols``); ``want_o=False``: final states only.  Both forward-only.
-    ``raw_gate = (A_log, g_bias or None, threshold)``: ``g`` is the raw per-channel gate projection in q's dtype and the
-    kernels apply kda_gate's activation themselves."""
-    dt, B, H, T, dk, dv_in, beta, gate, nseq, nstate, cu = _seq_setup(q, k, v, g, beta, None, cu_seqlens)
-    dv = dv_in if dv_total is None else dv_total
-    if initial_state is not None and tuple(initial_state.shape) != (nstate, H, dk, dv):
-        raise RuntimeError(f"initial_state shape {tuple(initial_state.shape)} != {(nstate, H, dk, dv)}")
-    tf = all(_is_token_first(t) for t in (q, k, v))  # [B,T,H,.] memory behind transposed views: used in place
-    q_in, k_in = _as_layout(q, tf), _as_layout(k, tf)
-    v = _as_layout(v, tf)
-    beta_f = _as_layout(beta.to(torch.float32), tf)
-    g_f = None if g is None else _as_layout(g if raw_gate is not None else g.to(torch.float32), tf)
-    s0 = None if initial_state is None else _f32(initial_state)
-    o = _empty_layout(B, H, T, (dv,), o_dtype, q.device, tf) if want_o else None
-    sT = torch.empty(nstate, H, dk, dv, dtype=torch.float32, device=q.device)
-    a = _base_args(B, H, T, dk, dv, dt, _DT[o_dtype], gate, False, scale)
-    lib = _lib.load()
-    # The reference's chunk path normalises in the input dtype before anything else (gated_deltanet.py:273-275,
-    # kda.py:379-381).  Where the kernels scale the rows themselves (no normalised copies, gradients carried through
-    # the normalisation inside lnx_chunk_bwd) they get the raw q and k; otherwise the rows are normalised first.
-    fused = bool(l2norm) and bool(lib.lnx_chunk_fuses_l2norm(a))
-    a.use_qk_l2norm = int(fused)
-    qn = _l2norm_rows_fwd(q_in) if l2norm and not fused else q_in
-    kn = _l2norm_rows_fwd(k_in) if l2norm and not fused else k_in
-    a.nseq = nseq
-    a.token_first = int(tf)
-    a.forward_only = int(forward_only)
-    a.value_cols = 0 if dv == dv_in else dv_in
-    a.q, a.k, a.v, a.beta, a.g = _ptr(qn), _ptr(kn), _ptr(v), _ptr(beta_f), _ptr(g_f)
-    a.initial_state, a.final_state, a.o, a.cu_seqlens = _ptr(s0), _ptr(sT), _ptr(o), _ptr(cu)
-    gate_keep = ()
-    if raw_gate is not None:
-        A32 = raw_gate[0].detach().to(torch.float32).contiguous()
-        b32 = None if raw_gate[1] is None else raw_gate[1].detach().to(torch.float32).contiguous()
-        a.g, a.gate_raw, a.gate_A_log, a.gate_bias, a.gate_threshold = None, _ptr(g_f), _ptr(A32), _ptr(b32), float(raw_gate[2])
-        gate_keep = (A32, b32)
-    lib = _lib.load()
-    nbytes = int(lib.lnx_chunk_workspace_bytes(a))
-    if nbytes == 0 and T > 0 and B > 0:
-        _lib.check(-2, "lnx_chunk_workspace_bytes")
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=q.device)
-    a.workspace, a.workspace_bytes = _ptr(ws), nbytes
-    _lib.check(lib.lnx_chunk_fwd(a, _stream(q)), "lnx_chunk_fwd")
-    saved = (q_in, k_in, qn, kn, v, beta_f, g_f, s0, cu, ws) + gate_keep
-    meta = (dt, B, H, T, dk, dv, gate, nseq, float(scale), bool(l2norm), o_dtype, beta.dtype,
-            None if g is None else g.dtype, initial_state is not None, tf, fused)
-    return o, sT, saved, meta
-
-
-class _ChunkScan(torch.autograd.Function):
-    """Pairs lnx_chunk_fwd with lnx_chunk_bwd (the role ``jax.custom_vjp`` plays for a JAX caller)."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens, grad_mode=True,
-                A_log=None, g_bias=None, threshold=None):
-        # nothing to differentiate (inference): the kernels skip what only the backward reads.  `grad_mode` is the
-        # caller's torch.is_grad_enabled() -- inside forward() it is always off, and needs_input_grad alone is still set
-        # for leaves that require grad under torch.no_grad()
-        raw_gate = None if A_log is None else (A_log, g_bias, threshold)
-        o, sT, saved, meta = _chunk_forward(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens,
-                                            forward_only=not (grad_mode and any(ctx.needs_input_grad)), raw_gate=raw_gate)
-        ctx.save_for_backward(*saved)
-        ctx.meta = meta
-        ctx.raw_gate = None if A_log is None else (float(threshold), A_log.dtype, None if g_bias is None else g_bias.dtype)
-        # an output that takes no part in the loss arrives in backward() as None, not as a tensor of zeros that a fill
-        # kernel wrote and lnx_chunk_bwd would read: a null d_final_state is the kernels' "no gradient"
-        ctx.set_materialize_grads(False)
-        return o, sT
-
-    @staticmethod
-    def backward(ctx, d_o, d_sT):
-        q_in, k_in, qn, kn, v, beta_f, g_f, s0, cu, ws = ctx.saved_tensors[:10]
-        dt, B, H, T, dk, dv, gate, nseq, scale, l2norm, o_dtype, beta_dt, g_dt, has_s0, tf, fused = ctx.meta
-        dev = qn.device
-        d_o = torch.zeros(B, H, T, dv, dtype=qn.dtype, device=dev) if d_o is None else d_o.to(qn.dtype)
-        d_o = _as_layout(d_o, tf)
-        d_sT = None if d_sT is None else _f32(d_sT)
-        dq, dk_, dv_ = torch.empty_like(qn), torch.empty_like(kn), torch.empty_like(v)
-        dbeta = torch.empty_like(beta_f)
-        dg = None if g_f is None else torch.empty_like(g_f)
-        nstate = nseq if nseq else B
-        ds0 = torch.empty(nstate, H, dk, dv, dtype=torch.float32, device=dev) if has_s0 else None
-        a = _base_args(B, H, T, dk, dv, dt, _DT[o_dtype], gate, fused, scale)
-        a.nseq = nseq
-        a.token_first = int(tf)
-        a.q, a.k, a.v, a.beta, a.g = _ptr(qn), _ptr(kn), _ptr(v), _ptr(beta_f), _ptr(g_f)
-        a.initial_state, a.cu_seqlens = _ptr(s0), _ptr(cu)
-        a.d_o, a.d_final_state = _ptr(d_o), _ptr(d_sT)
-        a.d_q, a.d_k, a.d_v, a.d_beta, a.d_g, a.d_initial_state = (_ptr(dq), _ptr(dk_), _ptr(dv_), _ptr(dbeta),
-                                                                   _ptr(dg), _ptr(ds0))
-        a.workspace, a.workspace_bytes = _ptr(ws), ws.numel()
-        dA = dbias = None
-        if ctx.raw_gate is not None:  # g is the raw gate projection: its gradient and the activation's parameter gradients
-            A32, b32 = ctx.saved_tensors[10:12]
-            dA = torch.empty_like(A32)
-            dbias = None if b32 is None else torch.empty_like(b32)
-            a.g, a.d_g = None, None
-            a.gate_raw, a.gate_A_log, a.gate_bias, a.gate_threshold = _ptr(g_f), _ptr(A32), _ptr(b32), ctx.raw_gate[0]
-            a.d_gate_raw, a.d_gate_A_log, a.d_gate_bias = _ptr(dg), _ptr(dA), _ptr(dbias)
-        _lib.check(_lib.load().lnx_chunk_bwd(a, _stream(qn)), "lnx_chunk_bwd")
-        if l2norm and not fused:
-            dq = _l2norm_rows_bwd(q_in, dq)
-            dk_ = _l2norm_rows_bwd(k_in, dk_)
-        dbeta = dbeta.to(beta_dt)
-        if dg is not None:
-            dg = dg.to(g_dt)
-        if ctx.raw_gate is not None:
-            dA = dA.to(ctx.raw_gate[1])
-            dbias = None if dbias is None else dbias.to(ctx.raw_gate[2])
-        return dq, dk_, dv_, dg, dbeta, ds0, None, None, None, None, None, dA, dbias, None
+    """One chunked scan, ``(o, final_state)``.  Without ``forward_only`` the call is a node of the autograd graph
+    whose backward is lnx_chunk_bwd; with it the kernels skip what only a backward pass reads.  ``dv_total`` > v's
+    columns: the state has dv_total value columns of which v holds the first ones and the others are zero
+    (``value_cols``); ``want_o=False``: final states only.  Both forward-only.  ``raw_gate = (A_log, g_bias or None,
+    threshold)``: ``g`` is the raw per-channel gate projection in q's dtype and the kernels apply kda_gate's
+    activation themselves."""
+    A_log, g_bias, threshold = raw_gate or (None, None, 0.0)
+    return _lib.host().chunk(q, k, v, g, beta, initial_state, scale, l2norm, _DT[o_dtype], _packed_table(cu_seqlens, q),
+                             forward_only, dv_total or 0, want_o, A_log, g_bias, threshold,
+                             _test_hooks["scan_slab"], _test_hooks["out_slabs"])
 
 
 _CHUNK_DK = (64, 128, 256)  # key head dimensions the chunk kernels are built for
@@ -551,7 +320,7 @@ def _segmented_forward(q, k, v, g, beta, scale, initial_state, l2norm, o_dtype, 
     q1, k1, v1, g1, beta1 = fold(q), fold(k), fold(v), fold(g), fold(_squeeze_beta(beta, 4))
     s_ext = torch.zeros(nseg, rows, dk, dv + dk, dtype=torch.float32, device=q.device)
     s_ext[..., dv:] = torch.eye(dk, dtype=torch.float32, device=q.device)
-    _, ab, _, _ = _chunk_forward(q1, k1, v1, g1, beta1, s_ext, scale, l2norm, o_dtype, cu, forward_only=True,
+    _, ab = _chunk_forward(q1, k1, v1, g1, beta1, s_ext, scale, l2norm, o_dtype, cu, forward_only=True,
                                  dv_total=dv + dk, want_o=False)  # v's columns followed by dk zero columns
     del s_ext
     Bs, As = ab[..., :dv], ab[..., dv:]
@@ -562,7 +331,7 @@ def _segmented_forward(q, k, v, g, beta, scale, initial_state, l2norm, o_dtype, 
         s_in[i] = cur
         if i + 1 < nseg:
             cur = torch.baddbmm(Bs[i], As[i], cur)
-    o, sT = _ChunkScan.apply(q1, k1, v1, g1, beta1, s_in, scale, l2norm, o_dtype, cu, torch.is_grad_enabled())
+    o, sT = _chunk_forward(q1, k1, v1, g1, beta1, s_in, scale, l2norm, o_dtype, cu, forward_only=True)
     return o.reshape(B, H, T, dv), sT[nseg - 1].reshape(B, H, dk, dv)
 
 
@@ -581,12 +350,13 @@ def _chunk(q, k, v, g, beta, scale, initial_state, chunk_size, l2norm, o_dtype, 
     dk, dv = q.shape[-1], v.shape[-1]
     dkp = next((c for c in _CHUNK_DK if dk <= c), None)
     dvp = -(-dv // 64) * 64
+    forward_only = not _wants_grad(q, k, v, g, beta, initial_state)
     if dkp is None or q.dim() != 4 or (dkp, dvp) == (dk, dv):
-        if dkp is not None and q.dim() == 4 and cu_seqlens is None and not _wants_grad(q, k, v, g, beta, initial_state):
+        if forward_only and dkp is not None and q.dim() == 4 and cu_seqlens is None:
             nseg = _prefill_segments(q.shape[0], q.shape[1], q.shape[2], dv)
             if nseg > 1:
                 return _segmented_forward(q, k, v, g, beta, scale, initial_state, l2norm, o_dtype, nseg)
-        return _ChunkScan.apply(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens, torch.is_grad_enabled())
+        return _chunk_forward(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens, forward_only=forward_only)[:2]
     # Head dimensions between the kernels' sizes (the reference's own tests use dk = 8, 16, dv = 8, 32):
     # zero channels are exact.  A zero key/query channel adds nothing to any <q,k>, <k,k> or |x|_2, the state rows
     # and columns it would feed stay zero, and the padded value columns are independent of the others; autograd
@@ -597,7 +367,7 @@ def _chunk(q, k, v, g, beta, scale, initial_state, chunk_size, l2norm, o_dtype, 
         g = pad(g, (0, dkp - dk))
     if initial_state is not None:
         initial_state = pad(initial_state, (0, dvp - dv, 0, dkp - dk))
-    o, sT = _ChunkScan.apply(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens, torch.is_grad_enabled())
+    o, sT = _chunk_forward(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens, forward_only=forward_only)[:2]
     return o[..., :dv], sT[..., :dk, :dv]
 
 
@@ -645,5 +415,6 @@ def kda_chunkwise_raw_gate(q, k, v, g_raw, beta, A_log, g_bias=None, scale=None,
         raise RuntimeError(f"A_log must be [{H}] and g_bias [{H * dk}]")
     if scale is None:
         scale = dk ** -0.5
-    return _ChunkScan.apply(q, k, v, g_raw, beta, initial_state, scale, use_qk_l2norm, output_dtype, cu_seqlens,
-                            torch.is_grad_enabled(), A_log, g_bias, float(threshold))
+    return _chunk_forward(q, k, v, g_raw, beta, initial_state, scale, use_qk_l2norm, output_dtype, cu_seqlens,
+                          forward_only=not _wants_grad(q, k, v, g_raw, beta, initial_state, A_log, g_bias),
+                          raw_gate=(A_log, g_bias, float(threshold)))[:2]
