@@ -4,7 +4,7 @@
 //   y = x * rsqrt(mean(x^2) + eps) * weight * sigmoid(gate)        (gate NULL: no gate)
 // Streaming kernels: LPR lanes share a row of LPR 16-byte vectors, a wavefront covers 64 / LPR rows per pass,
 // and the loads of four passes are issued together.  The backward also keeps d_weight partial sums in
-// registers over all passes of a wavefront and adds them with one atomic per column and workgroup.
+// registers over all passes of a wavefront and leaves one partial row per workgroup.
 #include "lnx_common.h"
 #include "mma_tiles.h"
 #include "reduce_rows.h"
@@ -12,7 +12,7 @@
 namespace {
 
 constexpr int UNR = 4;         // passes whose loads are in flight together
-constexpr int BWD_STEPS = 8;   // steps (of UNR passes) per wavefront in the backward: rows per d_weight atomic
+constexpr int BWD_STEPS = 8;   // most steps (of UNR passes) per wavefront in the backward: rows per partial row of d_weight
 
 __device__ __forceinline__ float sigmoidf(float z) { return 1.f / (1.f + __expf(-z)); }
 
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void rmsnorm_gated_fwd_kernel(const T* x, cons
 //   dx = rstd (u - xn mean(u xn));  dgate = dy xn w s (1 - s);  dweight = sum over rows of dy xn s.
 template <typename T, int LPR>
 __global__ __launch_bounds__(256) void rmsnorm_gated_bwd_kernel(const T* x, const T* gate, const float* w, const T* dy,
-                                                                T* dx, T* dgate, float* dw, int64_t rows, float eps) {
+                                                                T* dx, T* dgate, float* dw, int64_t rows, float eps, int steps) {
   typedef typename Vec16<T>::V V;
   constexpr int VN = Vec16<T>::N, RPW = 64 / LPR, D = LPR * VN;
   const int lane = threadIdx.x & 63, sub = lane / LPR, li = lane % LPR;
@@ -69,8 +69,8 @@ __global__ __launch_bounds__(256) void rmsnorm_gated_bwd_kernel(const T* x, cons
   float wv[VN], dwv[VN];
 #pragma unroll
   for (int e = 0; e < VN; ++e) wv[e] = w[li * VN + e], dwv[e] = 0.f;
-  for (int step = 0; step < BWD_STEPS; ++step) {
-    const int64_t r0 = (wave * BWD_STEPS + step) * (RPW * UNR) + sub;
+  for (int step = 0; step < steps; ++step) {
+    const int64_t r0 = (wave * steps + step) * (RPW * UNR) + sub;
     if (r0 - sub >= rows) break;
     V xv[UNR], gv[UNR], yv[UNR];
 #pragma unroll
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256) void rmsnorm_gated_fwd_wide_kernel(const T* x,
 
 template <typename T, int NV>
 __global__ __launch_bounds__(256) void rmsnorm_gated_bwd_wide_kernel(const T* x, const T* gate, const float* w, const T* dy,
-                                                                     T* dx, T* dgate, float* dw, int64_t rows, int d, float eps) {
+                                                                     T* dx, T* dgate, float* dw, int64_t rows, int d, float eps, int steps) {
   typedef typename Vec16<T>::V V;
   constexpr int VN = Vec16<T>::N;
   const int lane = threadIdx.x & 63, wv_i = threadIdx.x >> 6;
@@ -210,8 +210,8 @@ __global__ __launch_bounds__(256) void rmsnorm_gated_bwd_wide_kernel(const T* x,
       wv[j][e] = ((lane + 64 * j) * VN < d) ? w[(lane + 64 * j) * VN + e] : 0.f;
       dwv[j][e] = 0.f;
     }
-  for (int step = 0; step < BWD_STEPS; ++step) {
-    const int64_t r0 = (wave * BWD_STEPS + step) * UNRW;
+  for (int step = 0; step < steps; ++step) {
+    const int64_t r0 = (wave * steps + step) * UNRW;
     if (r0 >= rows) break;
     V xv[UNRW][NV], gv[UNRW][NV], yv[UNRW][NV];
 #pragma unroll
@@ -335,8 +335,17 @@ void launch_fwd(int l, int d, const void* x, const void* gate, const float* w, v
   }
 }
 
+// Steps per wavefront of the backward: as many as leave two wavefronts per SIMD (2048), so that a small call fills the
+// chip before it saves partial rows ([2,2007,16,128] bf16: 8 steps, 502 waves: 37 us; 2 steps, 2007 waves: 16 us).
+int bwd_steps(int l, int64_t rows) {
+  const int64_t step_rows = l ? (int64_t)(64 / l) * UNR : UNRW, all = (rows + step_rows - 1) / step_rows;
+  int s = BWD_STEPS;
+  while (s > 1 && (all + s - 1) / s < 2048) s >>= 1;
+  return s;
+}
+
 int64_t bwd_blocks(int l, int64_t rows) {
-  const int64_t per_wave = l ? (int64_t)(64 / l) * UNR * BWD_STEPS : (int64_t)UNRW * BWD_STEPS;
+  const int64_t per_wave = (l ? (int64_t)(64 / l) * UNR : UNRW) * bwd_steps(l, rows);
   return ((rows + per_wave - 1) / per_wave + 3) / 4;
 }
 
@@ -344,11 +353,12 @@ template <typename T>
 void launch_bwd(int l, int d, const void* x, const void* gate, const float* w, const void* dy, void* dx, void* dgate, float* dw,
                 int64_t rows, float eps, hipStream_t st) {
   dim3 grid((unsigned)bwd_blocks(l, rows));
+  const int steps = bwd_steps(l, rows);
   if (l) {
-    LNX_LPR_SWITCH(rmsnorm_gated_bwd_kernel, (const T*)x, (const T*)gate, w, (const T*)dy, (T*)dx, (T*)dgate, dw, rows, eps)
+    LNX_LPR_SWITCH(rmsnorm_gated_bwd_kernel, (const T*)x, (const T*)gate, w, (const T*)dy, (T*)dx, (T*)dgate, dw, rows, eps, steps)
   } else {
     const int nv = wide_vectors<T>(d);
-    LNX_NV_SWITCH(rmsnorm_gated_bwd_wide_kernel, (const T*)x, (const T*)gate, w, (const T*)dy, (T*)dx, (T*)dgate, dw, rows, d, eps)
+    LNX_NV_SWITCH(rmsnorm_gated_bwd_wide_kernel, (const T*)x, (const T*)gate, w, (const T*)dy, (T*)dx, (T*)dgate, dw, rows, d, eps, steps)
   }
 }
 
