@@ -280,6 +280,33 @@ uint64_t lnx_dplr_recurrent_bwd_workspace_bytes(int32_t B, int32_t H, int32_t T,
 int lnx_dplr_recurrent_bwd(const lnx_dplr_bwd_args* a, void* hip_stream);
 
 /*
+ * The same scan and its backward pass over chunks of 64 tokens on the matrix cores, in fp32 like the token kernels, for
+ * heads of dk = dv = 64.  lnx_dplr_chunk_fits tells whether these kernels take a shape (T >= 16).  `args` as for
+ * lnx_dplr_recurrent_fwd with o_dtype == dtype and 16-byte aligned tensors; the forward call leaves what the backward call
+ * needs in `kept` (NULL: no backward pass will follow).  lnx_dplr_chunk_bytes gives the bytes of `kept` (LNX_DPLR_KEPT, both
+ * calls) and of the scratch areas (forward with kept, forward without, backward), which hold nothing between calls and are
+ * bounded (about 1 GiB) however long the sequence is.  The token gradients dq,
+ * dk, dv, da, db have args->dtype; dgk and d_initial_state (may be NULL) are fp32; d_final_state may be NULL (zero).  No
+ * atomics: the result is the same from run to run.
+ */
+enum { LNX_DPLR_KEPT = 0, LNX_DPLR_FWD_SCRATCH = 1, LNX_DPLR_BWD_SCRATCH = 2, LNX_DPLR_ONLY_SCRATCH = 3 };
+typedef struct lnx_dplr_chunk_grads {
+  const void* d_o;
+  const float* d_final_state;
+  void* dq;
+  void* dk;
+  void* dv;
+  void* da;
+  void* db;
+  float* dgk;
+  float* d_initial_state;
+} lnx_dplr_chunk_grads;
+int lnx_dplr_chunk_fits(int32_t B, int32_t H, int32_t T, int32_t dk, int32_t dv);
+uint64_t lnx_dplr_chunk_bytes(int32_t B, int32_t H, int32_t T, int32_t what);
+int lnx_dplr_chunk_fwd(const lnx_dplr_args* args, void* kept, void* scratch, void* hip_stream);
+int lnx_dplr_chunk_bwd(const lnx_dplr_args* args, const lnx_dplr_chunk_grads* grads, void* kept, void* scratch, void* hip_stream);
+
+/*
  * RMSNorm with an optional sigmoid gate over the rows of [rows, d] matrices, the output epilogue of the reference's
  * blocks: y = x * rsqrt(mean(x^2) + eps) * weight * sigmoid(gate).  Replaces FusedRMSNormGated.__call__
  * (linearnexus/modules/linear_attn/kda.py:664-700) and o_norm(o) * sigmoid(g_out) (gated_deltanet.py:854-862).

@@ -820,14 +820,39 @@ Tensor dplr_call(bool step, const Tensor& q, const Tensor& k, const Tensor& v, c
   return o;
 }
 
+Tensor work_area(const Tensor& like, uint64_t bytes) { return at::empty({(int64_t)std::max<uint64_t>(bytes, 1)}, like.options().dtype(at::kByte)); }
+
+// Whether the chunked kernels take a scan (lnx_dplr_chunk_fits, and tensors that start on 16-byte boundaries)
+bool dplr_chunked(std::initializer_list<const Tensor*> ts, const Tensor& v) {
+  const Tensor& q = **ts.begin();
+  if (!lnx_dplr_chunk_fits((int32_t)q.size(0), (int32_t)q.size(1), (int32_t)q.size(2), (int32_t)q.size(3), (int32_t)v.size(3))) return false;
+  for (const Tensor* t : ts)
+    if (reinterpret_cast<uintptr_t>(t->data_ptr()) % 16) return false;
+  return true;
+}
+
+// The scan; `kept`: receives the chunked kernels' tensors for the backward pass (undefined where the token kernels ran)
+Tensor dplr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& a, const Tensor& b, const Tensor& gk, const Tensor& s_in, const Tensor& s_out, double scale,
+                    Tensor* kept) {
+  if (!dplr_chunked({&q, &k, &v, &a, &b, &gk}, v)) return dplr_call(false, q, k, v, a, b, gk, s_in, s_out, scale);
+  lnx_dplr_args r = dplr_args(q, k, v, a, b, gk, s_in, scale, false);
+  Tensor o = at::empty_like(v);
+  r.o = ptr(o), r.final_state = fptr(s_out);
+  if (kept) *kept = work_area(q, lnx_dplr_chunk_bytes(r.B, r.H, r.T, LNX_DPLR_KEPT));
+  const Tensor ws = work_area(q, lnx_dplr_chunk_bytes(r.B, r.H, r.T, kept ? LNX_DPLR_FWD_SCRATCH : LNX_DPLR_ONLY_SCRATCH));
+  check_status(lnx_dplr_chunk_fwd(&r, kept ? ptr(*kept) : nullptr, ptr(ws), stream_of(q)), "lnx_dplr_chunk_fwd");
+  return o;
+}
+
 Tensor dplr_state(const Tensor& q, const Tensor& v) { return at::empty({q.size(0), q.size(1), q.size(-1), v.size(-1)}, q.options().dtype(at::kFloat)); }
 
 struct DplrFn : Function<DplrFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor& a0, const Tensor& b0, const Tensor& gk0, const OptT& s0,
                                double scale) {
     const Tensor q = q0.contiguous(), k = k0.contiguous(), v = v0.contiguous(), a = a0.contiguous(), b = b0.contiguous(), gk = f32(gk0), s_in = f32(undef(s0));
-    const Tensor s_out = dplr_state(q, v), o = dplr_call(false, q, k, v, a, b, gk, s_in, s_out, scale);
-    ctx->save_for_backward({q, k, v, a, b, gk, s_in});
+    Tensor kept;
+    const Tensor s_out = dplr_state(q, v), o = dplr_forward(q, k, v, a, b, gk, s_in, s_out, scale, &kept);
+    ctx->save_for_backward({q, k, v, a, b, gk, s_in, kept});
     ctx->saved_data["i"] = std::vector<int64_t>{(int64_t)gk0.scalar_type(), (int64_t)(s0.has_value() ? s0->scalar_type() : at::kFloat), s0.has_value() && s0->requires_grad()};
     ctx->saved_data["d"] = scale;
     ctx->set_materialize_grads(false);
@@ -840,9 +865,18 @@ struct DplrFn : Function<DplrFn> {
     const int64_t B = q.size(0), H = q.size(1), T = q.size(2), dk = q.size(3), dv = v.size(3);
     const auto dt = q.scalar_type();
     const auto fo = q.options().dtype(at::kFloat);
+    const lnx_dplr_args args = dplr_args(q, k, v, a, b, gk, s_in, ctx->saved_data["d"].toDouble(), false);
+    const Tensor d_o = grads[0].defined() ? as_layout(grads[0].to(dt), false) : at::zeros_like(v), d_s = f32(grads[1]);
+    if (const Tensor& kept = s[7]; kept.defined()) {
+      Tensor r[5] = {at::empty_like(q), at::empty_like(k), at::empty_like(v), at::empty_like(a), at::empty_like(b)}, dgk = at::empty_like(gk), d0;
+      if (s_in.defined() && m[2]) d0 = at::empty_like(s_in);
+      const Tensor ws = work_area(q, lnx_dplr_chunk_bytes(args.B, args.H, args.T, LNX_DPLR_BWD_SCRATCH));
+      const lnx_dplr_chunk_grads cg{ptr(d_o), fptr(d_s), ptr(r[0]), ptr(r[1]), ptr(r[2]), ptr(r[3]), ptr(r[4]), fptr(dgk), fptr(d0)};
+      check_status(lnx_dplr_chunk_bwd(&args, &cg, ptr(kept), ptr(ws), stream_of(q)), "lnx_dplr_chunk_bwd");
+      return {r[0], r[1], r[2], r[3], r[4], dgk.to((at::ScalarType)m[0]), d0.defined() ? d0.to((at::ScalarType)m[1]) : d0, Tensor()};
+    }
     lnx_dplr_bwd_args g{};
-    g.fwd = dplr_args(q, k, v, a, b, gk, s_in, ctx->saved_data["d"].toDouble(), false);
-    const Tensor d_o = grads[0].defined() ? grads[0].to(dt).contiguous() : at::zeros_like(v), d_s = f32(grads[1]);
+    g.fwd = args;
     Tensor tok = at::empty({5, B, H, T, dk}, fo), dvv = at::empty({B, H, T, dv}, fo), ds0;
     if (s_in.defined() && m[2]) ds0 = at::empty_like(s_in);
     const uint64_t nws = lnx_dplr_recurrent_bwd_workspace_bytes((int32_t)B, (int32_t)H, (int32_t)T, (int32_t)dk, (int32_t)dv);
@@ -864,7 +898,7 @@ std::pair<Tensor, Tensor> dplr_scan(const Tensor& q, const Tensor& k, const Tens
     return {r[0], r[1]};
   }
   const Tensor s_out = dplr_state(q, v);
-  return {dplr_call(false, q.contiguous(), k.contiguous(), v.contiguous(), a.contiguous(), b.contiguous(), f32(gk), f32(s0), s_out, scale), s_out};
+  return {dplr_forward(q.contiguous(), k.contiguous(), v.contiguous(), a.contiguous(), b.contiguous(), f32(gk), f32(s0), s_out, scale, nullptr), s_out};
 }
 
 // dplr(q, k, v, a, b, gk, scale, initial_state)

@@ -509,19 +509,19 @@ __device__ __forceinline__ void mm16_store(float* dst, int ld, floatx4 c, int la
 
 // In-LDS inverse of the unit lower-triangular matrix I + A (A strictly lower, 64x64, fp32,
 // leading dimension LNX_LDA):  Tm = (I + A)^-1.  `sA` is read only; `sT` receives the full
-// matrix (upper triangle zero); `sX` is a [32][36] fp32 scratch.  Must be called by all 256
-// threads.  Diagonal 16x16 blocks by forward substitution, then two levels of block merges
+// matrix (upper triangle zero); `sX` is a [32][36] fp32 scratch.  Must be called by all THREADS
+// threads of the workgroup, of which the first 256 work.  Diagonal 16x16 blocks by forward substitution, then two levels of block merges
 //   [[L0, 0], [B, L1]]^-1 = [[L0^-1, 0], [-L1^-1 B L0^-1, L1^-1]].
 // In place (sT == sA, INPLACE): A's upper triangle and diagonal must hold zeros; every block of A is read for the last
 // time before the barrier that precedes the write of the same block of Tm.
-template <bool INPLACE = false>
+template <bool INPLACE = false, int THREADS = 256>
 __device__ __forceinline__ void tri_inverse_64(const float* sA, float* sT, float* sX, int tid) {
   const int wave = tid >> 6, lane = tid & 63;
   if (!INPLACE) {
-    for (int idx = tid; idx < 64 * LNX_LDA; idx += 256) sT[idx] = 0.f;
+    for (int idx = tid; idx < 64 * LNX_LDA; idx += THREADS) sT[idx] = 0.f;
     lds_barrier();
   }
-  if (lane < 16) {
+  if (lane < 16 && wave < 4) {
     const int r0 = 16 * wave, c = lane;
     float d[16];
 #pragma unroll
@@ -550,12 +550,12 @@ __device__ __forceinline__ void tri_inverse_64(const float* sA, float* sT, float
   lds_barrier();
   // level 2: the 32x32 lower-left block, one 16x16 output per wave
   const int bi = 16 * (wave >> 1), bj = 16 * (wave & 1);
-  {
+  if (THREADS == 256 || wave < 4) {
     floatx4 x = mm16_f32(sA + (32 + bi) * LNX_LDA, LNX_LDA, sT + bj, LNX_LDA, 32, lane);
     mm16_store(sX + bi * 36 + bj, 36, x, lane, 1.f);
   }
   lds_barrier();
-  {
+  if (THREADS == 256 || wave < 4) {
     floatx4 y = mm16_f32(sT + (32 + bi) * LNX_LDA + 32, LNX_LDA, sX + bj, 36, 32, lane);
     mm16_store(sT + (32 + bi) * LNX_LDA + bj, LNX_LDA, y, lane, -1.f);
   }
