@@ -21,8 +21,7 @@
 //   bwd_chunk  (one workgroup per chunk, all in parallel)                         dq, dk, dbeta, dg from q, k, v, dO, the
 //              two saved states and D, dR as the scans left them (dv leaves the reverse scan)
 //
-// Both scans split their waves into one compute wave per 32 value columns of the slab (two for the 64-column slabs:
-// matrix work on the tiles in LDS, the fp32 state in MFMA accumulators for the whole sequence) and four mover waves
+// Both scans split their waves into one compute wave per 16 value columns of the slab (matrix work on the tiles in LDS, the fp32 state in MFMA accumulators for the whole sequence) and four mover waves
 // (global loads two chunks ahead into registers, the next chunk's tiles into LDS, LDS -> global copies of results as
 // whole rows); all five input tiles and the per-token scalars are double-buffered in LDS, so two LDS-only barriers per
 // chunk suffice.  bwd_chunk brings its slabs in with loads that go straight to LDS (mma_tiles.h).
@@ -35,7 +34,13 @@ namespace {
 
 using T = bf16_t;
 typedef Mma<T> M;
+typedef Mma16 S16;
 template <typename X> __device__ __forceinline__ X* at(char* ws, uint64_t off) { return reinterpret_cast<X*>(ws + off); }
+
+// dst[l16][4 g ..] = accumulator tile of 16 rows (transposed store: this lane's column, four consecutive rows, 8 bytes)
+__device__ __forceinline__ void store_t(const floatx4& a, T* dst, int ld, int lane) {
+  store4(dst + (lane & 15) * ld + 4 * (lane >> 4), a);
+}
 
 // dst[col][row0 + ...] = fragment (transposed store, four consecutive rows per 8-byte vector)
 __device__ __forceinline__ void store_frag_t(const floatx16& a, T* dst, int ld, int lane) {
@@ -47,35 +52,43 @@ __device__ __forceinline__ void store_frag_t(const floatx16& a, T* dst, int ld, 
 }
 
 // Zeroes the 224 vectors above the diagonal (row r, columns 8 c .. 8 c + 7 with 8 c > r) of `ntile` consecutive
-// [64][ld] tiles of `stride` elements; 256 threads.  Group g of eight rows has 7 - g such vectors per row.
-__device__ __forceinline__ void zero_upper_triangles(T* tiles, int ntile, int stride, int ld, int tid) {
+// [64][ld] tiles of `stride` elements, columns in the order CHAIN; 256 threads.  Group g of eight rows has 7 - g such vectors per row.
+template <bool CHAIN> __device__ __forceinline__ void zero_upper_triangles(T* tiles, int ntile, int stride, int ld, int tid) {
   if (tid >= 512 - LNX_TRI_VECS) return;
   int g = 0;
   while (56 * (g + 1) - 4 * (g + 1) * g <= tid) ++g;  // vectors of the groups before g + 1
   const int o = tid - (56 * g - 4 * g * (g - 1)), per = 7 - g;
   const int r = 8 * g + o / per, c = g + 1 + (o - (o / per) * per);
-  for (int t = 0; t < ntile; ++t) *reinterpret_cast<Vec16<T>::V*>(tiles + t * stride + r * ld + 8 * c) = vec_zero<T>();
+  for (int t = 0; t < ntile; ++t) S16::put<CHAIN>(tiles + t * stride + r * ld + S16::pos<CHAIN>(8 * c), vec_zero<T>());
 }
 
 // Per-token scalars of one chunk in LDS, written by the movers when they commit a chunk
 struct Scal {
-  enum { BETA = 0, GAM = 64, R = 128, SG = 192, DEC = 256, SIZE = 320 };  // beta, e^G, e^{G_C - G}, scale e^G, e^{G_C}
+  enum { BETA = 0, GAM = 64, R = 128, SG = 192, DEC = 256, SIZE = 320 };  // beta, beta e^G / |k|, e^{G_C - G} / |k|, scale e^G / |q|, e^{G_C}
 };
 
 // ---------------------------------------------------------------------------------------
-// scan_fwd.  A compute wave owns a 32-column strip of the value slab: its [dk x 32] part of the state stays in MFMA
+// scan_fwd.  A compute wave owns a 16-column strip of the value slab: its [dk x 16] part of the state stays in MFMA
 // accumulators for the whole sequence, and the chain  S -> Y = K S -> R -> D = Tm R -> S'  never leaves the wave's
-// registers -- an accumulator fragment is the B operand of the next product as it is (Mma::from_acc), only the A
-// operands (K, Q, Tm, Pm rows) come from LDS.  All five input tiles are double-buffered, so the movers write chunk
+// registers -- two accumulator tiles are the B operand of the next product as they are (Mma16::from_acc), only the A
+// operands (K, Q, Tm, Pm rows) come from LDS.  Strips of 16 columns put a slab's chain on twice as many SIMDs as strips of 32:
+// B2 H16 T2007 d128 (32 chunks in a row, 128 workgroups) 65 -> 49 us forward and 74 -> 57 us in reverse, one prompt of 1000
+// tokens 32 -> 23 us, B8 H16 T4096 204 -> 190 and 217 -> 206 us.  What is left of a chunk's 1.5 us there: a SIMD takes 1 KB of
+// LDS reads in about 16 cycles, and a strip reads 60 KB of operands whatever its width.  All five input tiles are double-buffered, so the movers write chunk
 // n + 1 while chunk n is being read and two barriers per chunk are enough:
 //   B1    buffers of chunk n complete           compute: S^T -> LDS (saved states), Y, Q S, R, D (-> LDS, transposed), O -> LDS
 //                                               movers:  loads of chunk n + 2; chunk n + 1 -> the other buffers
 //   Bmid  O, S^T and D^T are in LDS             compute: state update        movers: O, S^T, D^T -> global
 // ---------------------------------------------------------------------------------------
 template <int DK, int BVW> struct FScanL {
-  static constexpr int PAD = M::PAD, LDK = DK + PAD, LDC = LNX_C + PAD, BV = BVW, LDV = BV + PAD, NCW = BV / 32;
-  static constexpr int kK = 64 * LDK, kST = BV * LDK, kV = 64 * LDV, kC = 64 * LDC;
-  static constexpr int kDT = BV * LDC;
+  // 32-column slabs are taken where the chip has room for more workgroups, so what counts there is the time of a chunk's
+  // chain: operand tiles in chain order, rows 32 bytes off a multiple of 64 (Mma16).  64-column slabs are bound by what the
+  // movers carry.
+  static constexpr bool CHAIN = BVW == 32;
+  static constexpr int BV = BVW, PAD = M::PAD, OPAD = CHAIN ? 16 : 8, LDK = DK + OPAD, LDC = LNX_C + OPAD, LDV = BV + PAD, NCW = BV / 16;
+  static constexpr int LDS = DK + PAD, LDD = LNX_C + PAD;  // of the tiles on their way out: states, D or dR
+  static constexpr int kK = 64 * LDK, kST = BV * LDS, kV = 64 * LDV, kC = 64 * LDC;
+  static constexpr int kDT = BV * LDD;
   // [2] x (K, Q, V, Tm, Pm) | O | S^T | D^T | scalars [2]
   static constexpr size_t bytes = sizeof(T) * (2 * (2 * kK + kV + 2 * kC) + kV + kST + kDT) + sizeof(float) * 2 * Scal::SIZE;
   static constexpr int threads = 64 * NCW + 256;
@@ -84,8 +97,9 @@ template <int DK, int BVW> struct FScanL {
 template <int DK, int GATE, int BVW, typename OT>
 __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(DirectParams p) {
   typedef FScanL<DK, BVW> L;
-  constexpr int LDK = L::LDK, LDC = L::LDC, BV = L::BV, LDV = L::LDV, NCW = L::NCW;
-  constexpr int KT = DK / 32;  // row tiles of the state strip
+  constexpr int LDK = L::LDK, LDC = L::LDC, BV = L::BV, LDV = L::LDV, NCW = L::NCW, LDS = L::LDS, LDD = L::LDD;
+  constexpr bool CHAIN = L::CHAIN;
+  constexpr int KT = DK / 16;  // row tiles of the state strip
   static_assert(DK == 64 || DK == 128, "dk = 64 or 128");
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);  // [2][64][LDK]
@@ -119,19 +133,17 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     struct Tiles {
       RowTile K, Q;
       ValTile V;
-      TriRegs<T> Tm, P;  // lower-triangular tiles, packed in the workspace
-      float g, gc, b;
-      float fq[RowTile::IT], nk[RowTile::IT];  // factors of the token each of this thread's Q / K vectors belongs to
+      TriRegs<T, CHAIN> Tm, P;  // lower-triangular tiles, packed in the workspace
+      float g, gc, b, fq, nk;  // per-token scalars of token mt % 64
       float bv[ValTile::IT];  // beta of the token each of its V vectors belongs to
       int len;
     };
     Tiles ta, tb;
     ta.g = ta.gc = ta.b = tb.g = tb.gc = tb.b = 0.f;
     ta.Tm.init(LDC, mt), ta.P.init(LDC, mt), tb.Tm.init(LDC, mt), tb.P.init(LDC, mt);
-    zero_upper_triangles(sTm, 4, L::kC, LDC, mt);  // both buffers of Tm and Pm: the packed tiles never write there
+    zero_upper_triangles<CHAIN>(sTm, 4, L::kC, LDC, mt);  // both buffers of Tm and Pm: the packed tiles never write there
     ta.len = tb.len = 0;
-#pragma unroll
-    for (int it = 0; it < RowTile::IT; ++it) ta.fq[it] = tb.fq[it] = ta.nk[it] = tb.nk[it] = 0.f;
+    ta.fq = tb.fq = ta.nk = tb.nk = 0.f;
 #pragma unroll
     for (int it = 0; it < ValTile::IT; ++it) ta.bv[it] = tb.bv[it] = 0.f;
     // part 0: K, 1: Q, 2: the rest; < 0: everything
@@ -153,36 +165,22 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
         R.g = G[t];
         R.gc = G[63];
       }
-#pragma unroll
-      for (int it = 0; it < RowTile::IT; ++it) {
-        R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
-        R.nk[it] = at<const float>(p.ws, p.off.Nk)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
-      }
+      R.fq = at<const float>(p.ws, p.off.Fq)[slot * 64 + t];
+      R.nk = at<const float>(p.ws, p.off.Nk)[slot * 64 + t];
       R.b = p.beta[tbase + (int64_t)min(t, R.len - 1) * p.geom.ts];
 #pragma unroll
       for (int it = 0; it < ValTile::IT; ++it)
         R.bv[it] = p.beta[tbase + (int64_t)min(min((mt + 256 * it) / ValTile::VPR, 63), R.len - 1) * p.geom.ts];
     };
+    // K and Q rows go to LDS as they are: their factors (1 / |k|, scale e^G / |q|) are rows of the products' results or of
+    // the other operand and enter there in fp32, sixteen multiplications per compute wave instead of a conversion both
+    // ways for every element in the movers
     auto commit = [&](const Tiles& R, int pb, int part = -1) {
-      {  // K rows normalised; Q rows normalised and scaled by scale e^{G_i}: the outputs then need no scaling of their own
-        T* dstk = sK + pb * L::kK;
-        T* dst = sQ + pb * L::kK;
 #pragma unroll
-        for (int it = 0; it < RowTile::IT; ++it) {
-          const int idx = mt + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
-          if (part < 0 || part == 0) {
-            typename Vec16<T>::V y = R.K.x[it];
-#pragma unroll
-            for (int e = 0; e < RowTile::N; ++e) y[e] = (bf16_t)((float)y[e] * R.nk[it]);
-            *reinterpret_cast<typename Vec16<T>::V*>(dstk + r * LDK + c) = y;
-          }
-          if (part < 0 || part == 1) {
-            typename Vec16<T>::V x = R.Q.x[it];
-#pragma unroll
-            for (int e = 0; e < RowTile::N; ++e) x[e] = (bf16_t)((float)x[e] * R.fq[it]);
-            *reinterpret_cast<typename Vec16<T>::V*>(dst + r * LDK + c) = x;
-          }
-        }
+      for (int it = 0; it < RowTile::IT; ++it) {
+        const int idx = mt + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
+        if (part < 0 || part == 0) S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), R.K.x[it]);
+        if (part < 0 || part == 1) S16::put<CHAIN>(sQ + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), R.Q.x[it]);
       }
       if (part == 0 || part == 1) return;
       {  // V rows scaled by beta_i: R = beta V - (beta e^G) Y
@@ -201,8 +199,9 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
       if (mt < 64) {
         float* sc = sSc + pb * Scal::SIZE;
         const float gam = (GATE == LNX_GATE_SCALAR) ? __expf(R.g) : 1.f;
-        sc[Scal::GAM + mt] = (mt < R.len) ? R.b * gam : 0.f;  // beta e^G
-        sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) : 1.f;
+        sc[Scal::GAM + mt] = (mt < R.len) ? R.b * gam * R.nk : 0.f;
+        sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) * R.nk : R.nk;
+        sc[Scal::SG + mt] = R.fq;
         if (mt == 0) sc[Scal::DEC] = (GATE == LNX_GATE_SCALAR) ? __expf(R.gc) : 1.f;
       }
     };
@@ -236,8 +235,8 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
       }
       if (p.save) {
         const int64_t slot = (int64_t)row * N + n;
-        unstage_tile<T, BV, DK, true>(at<T>(p.ws, p.off.SnT) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sST, LDK, BV, mt);
-        unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT, LDC, BV, mt);
+        unstage_tile<T, BV, DK, true>(at<T>(p.ws, p.off.SnT) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sST, LDS, BV, mt);
+        unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT, LDD, BV, mt);
       }
       lds_barrier();  // B1 of the next chunk
     };
@@ -260,31 +259,29 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     return;
   }
 
-  // ---------------- compute waves: wave w owns value columns [32 w, 32 w + 32) of the slab ----------------
-  const int vs = 32 * wave;
-  const int fr = lane & 31;
-  floatx16 S[KT];
+  // ---------------- compute waves: wave w owns value columns [16 w, 16 w + 16) of the slab ----------------
+  const int vs = 16 * wave;
+  const int l16 = lane & 15, g4 = 4 * (lane >> 4);
+  floatx4 S[KT];
 #pragma unroll
-  for (int ci = 0; ci < KT; ++ci)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) S[ci][e] = 0.f;
+  for (int ci = 0; ci < KT; ++ci) S[ci] = floatx4{0.f, 0.f, 0.f, 0.f};
   if (p.s0) {
-    const float* s0 = p.s0 + (int64_t)sidx * DK * p.dv + v0 + vs;
+    const float* s0 = p.s0 + (int64_t)sidx * DK * p.dv + v0 + vs + l16;
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) S[ci][e] = s0[(int64_t)(32 * ci + frag_row(e, lane)) * p.dv + frag_col(lane)];
+      for (int e = 0; e < 4; ++e) S[ci][e] = s0[(int64_t)(16 * ci + g4 + e) * p.dv];
     // the loads complete here: left pending into the loop, every iteration would count them down again
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) asm volatile("" : "+v"(S[ci][e]));
+      for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(S[ci][e]));
   }
   lds_barrier();  // B1 of the first chunk
   // Every LDS read is issued well ahead of the product that consumes it (A fragments two steps ahead, the next
-  // phase's first fragments and scalars during the current phase's last steps): a wave alone on its SIMD has nothing
-  // else to cover the LDS latency with.  The scheduling fences pin that order.
-  constexpr int NK = DK / 16;  // 16-wide steps over dk
+  // phase's first fragments and scalars during the current phase's last steps): a compute wave has nothing else to cover
+  // the LDS latency with.  The scheduling fences pin that order.
+  constexpr int NK = DK / 32;  // 32-wide steps over dk
   for (int n = c0; n < c1; ++n) {
     const int pb = (n - c0) & 1;
     const T* sKc = sK + pb * L::kK;
@@ -295,167 +292,129 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     const float* sc = sSc + pb * Scal::SIZE;
     if (p.save) {
 #pragma unroll
-      for (int ci = 0; ci < KT; ++ci) store_frag_t(S[ci], sST + vs * LDK + 32 * ci, LDK, lane);
+      for (int ci = 0; ci < KT; ++ci) store_t(S[ci], sST + vs * LDS + 16 * ci, LDS, lane);
     }
     // ---- Y = K S (lane = value column) and (Q~ S)^T (lane = token): the state fragments are the shared operand ----
-    floatx16 y[2], o[2];
+    floatx4 y[4], o[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 4; ++i) y[i] = o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    S16::Frag fa[2][4], fb[2][4];  // [step mod 2][token tile]
+    bf16x4 vr[4];                  // beta V at this lane's accumulator positions
+    floatx4 sv[4];                 // per-row scalars at this lane's accumulator positions: beta e^G / |k|, later e^{G_C - G} / |k|
+    S16::Frag tm[6], pm[6];        // [token tile, step]: (0,0) (1,0) (2,0) (3,0) (2,1) (3,1): Tm and Pm are lower-triangular
 #pragma unroll
-      for (int e = 0; e < 16; ++e) y[i][e] = o[i][e] = 0.f;
-    M::Frag fa[3][2], fb[3][2];  // [step mod 3][row tile]
-    bf16x4 vr[2][4];             // beta V at this lane's accumulator positions
-    floatx4 sv[2][4];            // per-row scalars at this lane's accumulator positions: beta e^G, later e^{G_C - G}
+    for (int i = 0; i < 4; ++i) fa[0][i] = S16::load<CHAIN>(sKc + (16 * i + l16) * LDK, lane);
 #pragma unroll
-    for (int s_ = 0; s_ < 2; ++s_)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        fa[s_][i] = M::load_chain(sKc + (32 * i + fr) * LDK + 16 * s_, lane);
-        fb[s_][i] = M::load_chain(sQc + (32 * i + fr) * LDK + 16 * s_, lane);
-      }
+    for (int i = 0; i < 4; ++i) fb[0][i] = S16::load<CHAIN>(sQc + (16 * i + l16) * LDK, lane);
+    // at most 16 LDS reads are in flight (the wave's counter ends at 15): K of the next step goes out ahead of this step's
+    // products, Q behind them
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      if (ks + 2 < NK) {
+      const S16::Frag b = S16::from_acc(S[2 * ks], S[2 * ks + 1]);
+      if (ks + 1 < NK) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          fa[(ks + 2) % 3][i] = M::load_chain(sKc + (32 * i + fr) * LDK + 16 * (ks + 2), lane);
-          fb[(ks + 2) % 3][i] = M::load_chain(sQc + (32 * i + fr) * LDK + 16 * (ks + 2), lane);
-        }
+        for (int i = 0; i < 4; ++i) fa[(ks + 1) & 1][i] = S16::load<CHAIN>(sKc + (16 * i + l16) * LDK + 32 * (ks + 1), lane);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vr[i] = S16::rows4(sVc, LDV, 16 * i, vs, lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::GAM + 16 * i + g4);
       }
-      if (ks == NK - 2) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 4; ++i) S16::mma(y[i], fa[ks & 1][i], b);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            vr[i][q] = M::load_acc_rows_raw(sVc, LDV, 32 * i, q, vs, lane);
-            sv[i][q] = load4(sc + Scal::GAM + 32 * i + 8 * q + 4 * (lane >> 5));
-          }
-      }
-      const M::Frag b = M::from_acc(S[ks >> 1], ks & 1);
+      for (int i = 0; i < 4; ++i) S16::mma(o[i], b, fb[ks & 1][i]);
+      if (ks + 1 < NK) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        M::mma(y[i], fa[ks % 3][i], b);
-        M::mma(o[i], b, fb[ks % 3][i]);
+        for (int i = 0; i < 4; ++i) fb[(ks + 1) & 1][i] = S16::load<CHAIN>(sQc + (16 * i + l16) * LDK + 32 * (ks + 1), lane);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tm[i] = S16::load<CHAIN>(sTc + (16 * i + l16) * LDC, lane);
+#pragma unroll
+        for (int i = 2; i < 4; ++i) tm[i + 2] = S16::load<CHAIN>(sTc + (16 * i + l16) * LDC + 32, lane);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    // Tm and Pm are lower-triangular: the first 32 rows of D and of the outputs take the first 32 tokens only, so the two
-    // products need 6 MFMAs each, not 8, and the work on the first half (R, D, scaling, conversions, stores) runs in the
-    // shadow of the second half's MFMAs.  tm[i][ks], pm[i][ks]: row tile i, 16-token step ks (i = 0: ks < 2).
-    M::Frag tm0[2], tm1[4], pm0[2], pm1[4];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      tm0[ks] = M::load_chain(sTc + fr * LDC + 16 * ks, lane);
-      tm1[ks] = M::load_chain(sTc + (32 + fr) * LDC + 16 * ks, lane);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- R = beta V - (beta e^G) Y, in place of Y: tokens 0 .. 31 ----
+    // ---- R = beta V - (beta e^G) Y, in place of Y; D = Tm R: the first half of the rows takes the first 32 tokens only ----
     auto form_r = [&](int i) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) y[i][4 * q + u] = (float)vr[i][q][u] - sv[i][q][u] * y[i][4 * q + u];
+      for (int u = 0; u < 4; ++u) y[i][u] = (float)vr[i][u] - sv[i][u] * y[i][u];
     };
-    form_r(0);
-    M::Frag br[4];
-    br[0] = M::from_acc(y[0], 0), br[1] = M::from_acc(y[0], 1);
+    floatx4 d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float fq[4];  // scale e^G / |q| of this lane's token in each tile of o
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fq[i] = sc[Scal::SG + 16 * i + l16];
+    form_r(0), form_r(1);
+    const S16::Frag br0 = S16::from_acc(y[0], y[1]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S16::mma(d[i], tm[i], br0);
+    form_r(2), form_r(3);
+    const S16::Frag br1 = S16::from_acc(y[2], y[3]);
     __builtin_amdgcn_sched_barrier(0);
-    // ---- D = Tm R: the steps over tokens 0 .. 31, with R of tokens 32 .. 63 formed meanwhile ----
-    floatx16 d[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 4; ++i) pm[i] = S16::load<CHAIN>(sPc + (16 * i + l16) * LDC, lane);
+    S16::mma(d[2], tm[4], br1);
+    S16::mma(d[3], tm[5], br1);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) d[i][e] = 0.f;
+    for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::R + 16 * i + g4);  // e^{G_C - G} / |k| for the state update
 #pragma unroll
-    for (int ks = 2; ks < 4; ++ks) tm1[ks] = M::load_chain(sTc + (32 + fr) * LDC + 16 * ks, lane);
-    M::mma(d[0], tm0[0], br[0]);
-    M::mma(d[1], tm1[0], br[0]);
-    M::mma(d[0], tm0[1], br[1]);
-    M::mma(d[1], tm1[1], br[1]);
-    form_r(1);
-    br[2] = M::from_acc(y[1], 0), br[3] = M::from_acc(y[1], 1);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      pm0[ks] = M::load_chain(sPc + fr * LDC + 16 * ks, lane);
-      pm1[ks] = M::load_chain(sPc + (32 + fr) * LDC + 16 * ks, lane);
-    }
-    if (GATE == LNX_GATE_SCALAR) {  // e^{G_C - G} for the state update
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sv[i][q] = load4(sc + Scal::R + 32 * i + 8 * q + 4 * (lane >> 5));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- the last two steps of D's second half; the first half goes on to the outputs ----
-    M::Frag fu[2][KT];  // K^T fragments of the state update, [step parity][row tile of the state]
-    M::Frag bd[4];      // D as the outputs' operand; br becomes the state update's operand (rows scaled by e^{G_C - G})
-    M::mma(d[1], tm1[2], br[2]);
-    M::mma(d[1], tm1[3], br[3]);
-    store_frag_t(d[0], sDT + vs * LDC, LDC, lane);  // also when nothing is saved: a branch here would split the schedule
-    bd[0] = M::from_acc(d[0], 0), bd[1] = M::from_acc(d[0], 1);
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- O^T = (Q~ S)^T + D^T Pm^T ----
-#pragma unroll
-    for (int ks = 2; ks < 4; ++ks) pm1[ks] = M::load_chain(sPc + (32 + fr) * LDC + 16 * ks, lane);
-    M::mma(o[0], bd[0], pm0[0]);
-    M::mma(o[1], bd[0], pm1[0]);
-    M::mma(o[0], bd[1], pm0[1]);
-    M::mma(o[1], bd[1], pm1[1]);
-    store_frag_t(d[1], sDT + vs * LDC + 32, LDC, lane);
-    bd[2] = M::from_acc(d[1], 0), bd[3] = M::from_acc(d[1], 1);
-#pragma unroll
-    for (int ci = 0; ci < KT; ++ci) fu[0][ci] = M::load_t_chain(sKc, LDK, 0, 32 * ci, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    M::mma(o[1], bd[2], pm1[2]);
-    M::mma(o[1], bd[3], pm1[3]);
-    store_frag_t(o[0], sO + vs, LDV, lane);  // [token][value column]
-    // the state update's operand while the last products finish: D rows scaled by e^{G_C - G}
-    if (GATE == LNX_GATE_SCALAR) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) d[i][4 * q + u] *= sv[i][q][u];
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) br[ks] = M::from_acc(d[ks >> 1], ks & 1);
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) br[ks] = bd[ks];
-    }
+    for (int i = 0; i < 4; ++i) o[i] *= fq[i];
     const float dec = (GATE == LNX_GATE_SCALAR) ? sc[Scal::DEC] : 1.f;
     __builtin_amdgcn_sched_barrier(0);
-    store_frag_t(o[1], sO + 32 * LDV + vs, LDV, lane);
-    lds_barrier();  // Bmid
-    // ---- S <- e^{G_C} S + K^T (e^{G_C - G} D) ----
+    // ---- O^T = (Q~ S)^T + D^T Pm^T ----
+    const S16::Frag bd0 = S16::from_acc(d[0], d[1]);
+#pragma unroll
+    for (int i = 2; i < 4; ++i) pm[i + 2] = S16::load<CHAIN>(sPc + (16 * i + l16) * LDC + 32, lane);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S16::mma(o[i], bd0, pm[i]);
+    S16::Frag fu[2][KT];  // K^T fragments of the state update, [step][row tile of the state]
+#pragma unroll
+    for (int ci = 0; ci < 4; ++ci) fu[0][ci] = S16::load_cols<CHAIN>(sKc, LDK, 0, ci, lane);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) store_t(d[i], sDT + vs * LDD + 16 * i, LDD, lane);  // also when nothing is saved: a branch here would split the schedule
+    const S16::Frag bd1 = S16::from_acc(d[2], d[3]);
+    S16::mma(o[2], bd1, pm[4]);
+    S16::mma(o[3], bd1, pm[5]);
+    // the state update's operand while the last products finish: D rows scaled by e^{G_C - G}
+    const S16::Frag bu0 = S16::from_acc(d[0] * sv[0], d[1] * sv[1]), bu1 = S16::from_acc(d[2] * sv[2], d[3] * sv[3]);
     if (GATE == LNX_GATE_SCALAR) {
 #pragma unroll
-      for (int ci = 0; ci < KT; ++ci)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) S[ci][e] *= dec;
+      for (int ci = 0; ci < KT; ++ci) S[ci] *= dec;
     }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (ks + 1 < 4) {
+    for (int i = 0; i < 4; ++i) store_t(o[i], sO + 16 * i * LDV + vs, LDV, lane);  // [token][value column]
+    lds_barrier();  // Bmid
+    // ---- S <- e^{G_C} S + K^T (e^{G_C - G} D) ----
 #pragma unroll
-        for (int ci = 0; ci < KT; ++ci) fu[(ks + 1) & 1][ci] = M::load_t_chain(sKc, LDK, 16 * (ks + 1), 32 * ci, lane);
-      }
+    for (int ci = 4; ci < KT; ++ci) fu[0][ci] = S16::load_cols<CHAIN>(sKc, LDK, 0, ci, lane);
 #pragma unroll
-      for (int ci = 0; ci < KT; ++ci) M::mma(S[ci], fu[ks & 1][ci], br[ks]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int ci = 0; ci < 4; ++ci) S16::mma(S[ci], fu[0][ci], bu0);
+#pragma unroll
+    for (int ci = 0; ci < 4; ++ci) fu[1][ci] = S16::load_cols<CHAIN>(sKc, LDK, 32, ci, lane);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ci = 4; ci < KT; ++ci) S16::mma(S[ci], fu[0][ci], bu0);
+#pragma unroll
+    for (int ci = 4; ci < KT; ++ci) fu[1][ci] = S16::load_cols<CHAIN>(sKc, LDK, 32, ci, lane);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci) S16::mma(S[ci], fu[1][ci], bu1);
     lds_barrier();  // B1 of the next chunk
   }
-  float* out = p.sT_out + (int64_t)sidx * DK * p.dv + v0 + vs + frag_col(lane);
+  float* out = p.sT_out + (int64_t)sidx * DK * p.dv + v0 + vs + l16;
 #pragma unroll
   for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) out[(int64_t)(32 * ci + frag_row(e, lane)) * p.dv] = S[ci][e];
+    for (int e = 0; e < 4; ++e) out[(int64_t)(16 * ci + g4 + e) * p.dv] = S[ci][e];
 }
 
 template <int DK, int GATE, typename OT>
 int launch_scan_fwd(const DirectParams& p, int nstate, hipStream_t st) {
-  // 32-column slabs (one compute wave) when 64-column ones would occupy at most half of the chip
+  // 32-column slabs (two compute waves) when 64-column ones would occupy at most half of the chip
   const bool narrow = lnx_narrow_slabs((int64_t)nstate * p.geom.H * (p.dv / 64), p.slab);
   auto k = narrow ? scan_fwd_kernel<DK, GATE, 32, OT> : scan_fwd_kernel<DK, GATE, 64, OT>;
   const size_t b = narrow ? FScanL<DK, 32>::bytes : FScanL<DK, 64>::bytes;
@@ -469,7 +428,7 @@ int launch_scan_fwd(const DirectParams& p, int nstate, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------------------
-// scan_bwd: the reverse pass, same organisation as scan_fwd.  A compute wave owns a 32-column strip of dS (the
+// scan_bwd: the reverse pass, same organisation as scan_fwd.  A compute wave owns a 16-column strip of dS (the
 // gradient of the state leaving the chunk); the chain  dS' -> Z = K dS' -> dD -> dR = Tm^T dD -> dY -> dS  stays in
 // its registers.  Needs no forward state: only K, Q, dO, Tm, Pm and the per-token scalars.
 //   B1    buffers of chunk n complete           compute: dS'^T -> LDS (saved), Z, Pm^T dO, dD, dR (-> LDS, transposed),
@@ -478,9 +437,14 @@ int launch_scan_fwd(const DirectParams& p, int nstate, hipStream_t st) {
 //   Bmid  dS'^T, dR^T and dv are in LDS         compute: dS update          movers: dS'^T, dR^T -> workspace, dv out
 // ---------------------------------------------------------------------------------------
 template <int DK, int BVW> struct BScanL {
-  static constexpr int PAD = M::PAD, LDK = DK + PAD, LDC = LNX_C + PAD, BV = BVW, LDV = BV + PAD, NCW = BV / 32;
-  static constexpr int kK = 64 * LDK, kST = BV * LDK, kV = 64 * LDV, kC = 64 * LDC;
-  static constexpr int kDT = BV * LDC;
+  // 32-column slabs are taken where the chip has room for more workgroups, so what counts there is the time of a chunk's
+  // chain: operand tiles in chain order, rows 32 bytes off a multiple of 64 (Mma16).  64-column slabs are bound by what the
+  // movers carry.
+  static constexpr bool CHAIN = BVW == 32;
+  static constexpr int BV = BVW, PAD = M::PAD, OPAD = CHAIN ? 16 : 8, LDK = DK + OPAD, LDC = LNX_C + OPAD, LDV = BV + PAD, NCW = BV / 16;
+  static constexpr int LDS = DK + PAD, LDD = LNX_C + PAD;  // of the tiles on their way out: states, D or dR
+  static constexpr int kK = 64 * LDK, kST = BV * LDS, kV = 64 * LDV, kC = 64 * LDC;
+  static constexpr int kDT = BV * LDD;
   // [2] x (K, scaled Q, dO, Tm, Pm) | dS'^T | dR^T | dv | scalars [2]
   static constexpr size_t bytes = sizeof(T) * (2 * (2 * kK + kV + 2 * kC) + kST + kDT + kV) + sizeof(float) * 2 * Scal::SIZE;
   static constexpr int threads = 64 * NCW + 256;
@@ -489,8 +453,9 @@ template <int DK, int BVW> struct BScanL {
 template <int DK, int GATE, int BVW>
 __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(DirectParams p) {
   typedef BScanL<DK, BVW> L;
-  constexpr int LDK = L::LDK, LDC = L::LDC, BV = L::BV, LDV = L::LDV, NCW = L::NCW;
-  constexpr int KT = DK / 32;
+  constexpr int LDK = L::LDK, LDC = L::LDC, BV = L::BV, LDV = L::LDV, NCW = L::NCW, LDS = L::LDS, LDD = L::LDD;
+  constexpr bool CHAIN = L::CHAIN;
+  constexpr int KT = DK / 16;
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);  // [2][64][LDK]
   T* sQ = sK + 2 * L::kK;              // rows scaled by scale e^G
@@ -522,18 +487,16 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
     struct Tiles {
       RowTile K, Q;
       TileRegs<T, 64, BV> dO;
-      TriRegs<T> Tm, P;  // lower-triangular tiles, packed in the workspace
-      float g, gc, b;
-      float fq[RowTile::IT], nk[RowTile::IT];  // factors of the token each of this thread's Q / K vectors belongs to
+      TriRegs<T, CHAIN> Tm, P;  // lower-triangular tiles, packed in the workspace
+      float g, gc, b, fq, nk;  // per-token scalars of token mt % 64
       int len;
     };
     Tiles ta, tb;
     ta.g = ta.gc = ta.b = tb.g = tb.gc = tb.b = 0.f;
     ta.Tm.init(LDC, mt), ta.P.init(LDC, mt), tb.Tm.init(LDC, mt), tb.P.init(LDC, mt);
-    zero_upper_triangles(sTm, 4, L::kC, LDC, mt);  // both buffers of Tm and Pm: the packed tiles never write there
+    zero_upper_triangles<CHAIN>(sTm, 4, L::kC, LDC, mt);  // both buffers of Tm and Pm: the packed tiles never write there
     ta.len = tb.len = 0;
-#pragma unroll
-    for (int it = 0; it < RowTile::IT; ++it) ta.fq[it] = tb.fq[it] = ta.nk[it] = tb.nk[it] = 0.f;
+    ta.fq = tb.fq = ta.nk = tb.nk = 0.f;
     auto fetch = [&](Tiles& R, int n, int part = -1) {  // part 0: K, 1: Q, 2: the rest; < 0: everything
       const int64_t slot = (int64_t)row * N + n;
       int tok0;
@@ -551,33 +514,19 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
         R.g = G[t];
         R.gc = G[63];
       }
-#pragma unroll
-      for (int it = 0; it < RowTile::IT; ++it) {
-        R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
-        R.nk[it] = at<const float>(p.ws, p.off.Nk)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
-      }
+      R.fq = at<const float>(p.ws, p.off.Fq)[slot * 64 + t];
+      R.nk = at<const float>(p.ws, p.off.Nk)[slot * 64 + t];
       R.b = p.beta[tbase + (int64_t)min(t, R.len - 1) * p.geom.ts];
     };
+    // K and Q rows go to LDS as they are: their factors (1 / |k|, scale e^G / |q|) are rows of the products' results or of
+    // the other operand and enter there in fp32, sixteen multiplications per compute wave instead of a conversion both
+    // ways for every element in the movers
     auto commit = [&](const Tiles& R, int pb, int part = -1) {
-      {  // K rows normalised; Q rows normalised and scaled by scale e^{G_i}: (scale diag(e^G) Q)^T dO needs no scaled copy of dO
-        T* dstk = sK + pb * L::kK;
-        T* dst = sQ + pb * L::kK;
 #pragma unroll
-        for (int it = 0; it < RowTile::IT; ++it) {
-          const int idx = mt + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
-          if (part < 0 || part == 0) {
-            typename Vec16<T>::V y = R.K.x[it];
-#pragma unroll
-            for (int e = 0; e < RowTile::N; ++e) y[e] = (bf16_t)((float)y[e] * R.nk[it]);
-            *reinterpret_cast<typename Vec16<T>::V*>(dstk + r * LDK + c) = y;
-          }
-          if (part < 0 || part == 1) {
-            typename Vec16<T>::V x = R.Q.x[it];
-#pragma unroll
-            for (int e = 0; e < RowTile::N; ++e) x[e] = (bf16_t)((float)x[e] * R.fq[it]);
-            *reinterpret_cast<typename Vec16<T>::V*>(dst + r * LDK + c) = x;
-          }
-        }
+      for (int it = 0; it < RowTile::IT; ++it) {
+        const int idx = mt + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
+        if (part < 0 || part == 0) S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), R.K.x[it]);
+        if (part < 0 || part == 1) S16::put<CHAIN>(sQ + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), R.Q.x[it]);
       }
       if (part == 0 || part == 1) return;
       R.dO.store(sdO + pb * L::kV, LDV, mt);
@@ -588,8 +537,9 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
         const float gam = (GATE == LNX_GATE_SCALAR) ? __expf(R.g) : 1.f;
         const float bt = (mt < R.len) ? R.b : 0.f;
         sc[Scal::BETA + mt] = bt;
-        sc[Scal::GAM + mt] = bt * gam;  // beta e^G: dY = -(beta e^G) dR
-        sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) : 1.f;
+        sc[Scal::GAM + mt] = bt * gam * R.nk;  // dY = -(beta e^G) dR
+        sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) * R.nk : R.nk;
+        sc[Scal::SG + mt] = R.fq;
         if (mt == 0) sc[Scal::DEC] = (GATE == LNX_GATE_SCALAR) ? __expf(R.gc) : 1.f;
       }
     };
@@ -610,8 +560,8 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
       }
       lds_barrier();  // Bmid
       const int64_t slot = (int64_t)row * N + n;
-      unstage_tile<T, BV, DK, true>(at<T>(p.ws, p.off.dSn) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sdST, LDK, BV, mt);
-      unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.dD) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sdRT, LDC, BV, mt);
+      unstage_tile<T, BV, DK, true>(at<T>(p.ws, p.off.dSn) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sdST, LDS, BV, mt);
+      unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.dD) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sdRT, LDD, BV, mt);
       int tok0, len;
       chunk_span(span, n, tok0, len);
       unstage_tile_checked<T, 64, BV>(p.dv_out + tok_index(p.geom, row, tok0) * p.dv + v0, tsv, sdV, LDV, len, mt);
@@ -636,24 +586,26 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
   }
 
   // ---------------- compute waves ----------------
-  const int vs = 32 * wave;
-  const int fr = lane & 31;
-  floatx16 dS[KT];
+  const int vs = 16 * wave;
+  const int l16 = lane & 15, g4 = 4 * (lane >> 4);
+  floatx4 dS[KT];
 #pragma unroll
-  for (int ci = 0; ci < KT; ++ci)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) dS[ci][e] = 0.f;
+  for (int ci = 0; ci < KT; ++ci) dS[ci] = floatx4{0.f, 0.f, 0.f, 0.f};
   if (p.d_sT) {
-    const float* src = p.d_sT + (int64_t)sidx * DK * p.dv + v0 + vs;
+    const float* src = p.d_sT + (int64_t)sidx * DK * p.dv + v0 + vs + l16;
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) dS[ci][e] = src[(int64_t)(32 * ci + frag_row(e, lane)) * p.dv + frag_col(lane)];
+      for (int e = 0; e < 4; ++e) dS[ci][e] = src[(int64_t)(16 * ci + g4 + e) * p.dv];
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(dS[ci][e]));  // complete here, as in scan_fwd
   }
   lds_barrier();  // B1 of the first chunk
   // LDS reads are issued ahead of the products that consume them, as in scan_fwd.  The products that do not depend on
   // the incoming dS' (Pm^T dO, Q~^T dO) fill the gaps of the chain  dS' -> Z -> dD -> dR -> dY -> dS.
-  constexpr int NK = DK / 16;
+  constexpr int NK = DK / 32;
   for (int n = c1 - 1; n >= c0; --n) {
     const int pb = (c1 - 1 - n) & 1;
     const T* sKc = sK + pb * L::kK;
@@ -662,162 +614,124 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
     const T* sTc = sTm + pb * L::kC;
     const T* sPc = sP + pb * L::kC;
     const float* sc = sSc + pb * Scal::SIZE;
-    M::Frag fa[3][2], fp[2][2], fo[2];
-    floatx4 sv[2][4];  // per-row scalars at this lane's accumulator positions: e^{G_C - G}, later beta e^G
+    S16::Frag fa[2][4];  // K rows, [step mod 2][token tile]
+    S16::Frag ft[6];     // Pm^T, then Tm^T: [token tile, step] (0,1) (1,1) (2,1) (3,1) (0,0) (1,0): upper-triangular
+    S16::Frag fo[2];     // dO
+    floatx4 sv[4];       // per-row scalars at this lane's accumulator positions: e^{G_C - G} / |k|, later beta e^G / |k|
+    auto load_tri = [&](const T* tile) {
 #pragma unroll
-    for (int s_ = 0; s_ < 2; ++s_)
+      for (int i = 0; i < 4; ++i) ft[i] = S16::load_cols<CHAIN>(tile, LDC, 32, i, lane);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) fa[s_][i] = M::load_chain(sKc + (32 * i + fr) * LDK + 16 * s_, lane);
-    fp[0][0] = M::load_t(sPc, LDC, 0, 0, lane);  // Pm^T and Tm^T are upper-triangular: row tile 1 takes steps 2, 3 only
-    fo[0] = M::load_t(sOc, LDV, 0, vs, lane);
+      for (int i = 0; i < 2; ++i) ft[i + 4] = S16::load_cols<CHAIN>(tile, LDC, 0, i, lane);
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fa[0][i] = S16::load<CHAIN>(sKc + (16 * i + l16) * LDK, lane);
+#pragma unroll
+    for (int s_ = 0; s_ < 2; ++s_) fo[s_] = S16::load_t(sOc, LDV, 32 * s_, vs, lane);
     // the state gradient as the B operand of Z = K dS'; its accumulators are then free to take the next dS
-    M::Frag bs[NK];
+    S16::Frag bs[NK];
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) bs[ks] = M::from_acc(dS[ks >> 1], ks & 1);
+    for (int ks = 0; ks < NK; ++ks) bs[ks] = S16::from_acc(dS[2 * ks], dS[2 * ks + 1]);
 #pragma unroll
-    for (int ci = 0; ci < KT; ++ci) store_frag_t(dS[ci], sdST + vs * LDK + 32 * ci, LDK, lane);
+    for (int ci = 0; ci < KT; ++ci) store_t(dS[ci], sdST + vs * LDS + 16 * ci, LDS, lane);
     const float dec = (GATE == LNX_GATE_SCALAR) ? sc[Scal::DEC] : 1.f;
-    __builtin_amdgcn_sched_barrier(0);
     // ---- Z = K dS' and the chunk-local part Pm^T dO ----
-    floatx16 z[2], dd[2];
+    floatx4 z[4], dd[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) z[i][e] = dd[i][e] = 0.f;
+    for (int i = 0; i < 4; ++i) z[i] = dd[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      if (ks + 2 < NK) {
+      if (ks + 1 < NK) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) fa[(ks + 2) % 3][i] = M::load_chain(sKc + (32 * i + fr) * LDK + 16 * (ks + 2), lane);
+        for (int i = 0; i < 4; ++i) fa[(ks + 1) & 1][i] = S16::load<CHAIN>(sKc + (16 * i + l16) * LDK + 32 * (ks + 1), lane);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::R + 16 * i + g4);
       }
-      if (ks + 1 < 4) {
+      if (ks == 0) load_tri(sPc);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-          if (i == 0 || ks + 1 >= 2) fp[(ks + 1) & 1][i] = M::load_t(sPc, LDC, 16 * (ks + 1), 32 * i, lane);
-        fo[(ks + 1) & 1] = M::load_t(sOc, LDV, 16 * (ks + 1), vs, lane);
-      }
-      if (ks == NK - 2) {
+      for (int i = 0; i < 4; ++i) S16::mma(z[i], fa[ks & 1][i], bs[ks]);
+      if (ks == NK - 1) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 4; ++i) S16::mma(dd[i], ft[i], fo[1]);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) sv[i][q] = load4(sc + Scal::R + 32 * i + 8 * q + 4 * (lane >> 5));
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) M::mma(z[i], fa[ks % 3][i], bs[ks]);
-      if (ks < 4) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          if (i == 0 || ks >= 2) M::mma(dd[i], fp[ks & 1][i], fo[ks & 1]);
+        for (int i = 0; i < 2; ++i) S16::mma(dd[i], ft[i + 4], fo[0]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    // first fragments of Tm^T, and of the (scale e^G Q)^T dO product that fills the wait for Z
-    M::Frag fq[2][KT];
+    // ---- dS <- e^{G_C} dS' + (scale e^G Q)^T dO fills the wait for Z; Tm^T is fetched behind it ----
+    S16::Frag fq[2][KT];
 #pragma unroll
-    for (int s_ = 0; s_ < 2; ++s_) fa[s_][0] = M::load_t_chain(sTc, LDC, 16 * s_, 0, lane);
-#pragma unroll
-    for (int ci = 0; ci < KT; ++ci) fq[0][ci] = M::load_t(sQc, LDK, 0, 32 * ci, lane);
-    fo[0] = M::load_t(sOc, LDV, 0, vs, lane);
+    for (int ci = 0; ci < KT; ++ci) fq[0][ci] = S16::load_cols<CHAIN>(sQc, LDK, 0, ci, lane);
+    load_tri(sTc);
     if (GATE == LNX_GATE_SCALAR) {
 #pragma unroll
-      for (int ci = 0; ci < KT; ++ci)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) dS[ci][e] *= dec;
+      for (int ci = 0; ci < KT; ++ci) dS[ci] *= dec;
     }
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- dS <- e^{G_C} dS' + (scale e^G Q)^T dO ----
+    // dO rows times scale e^G / |q|, the operand of the Q^T dO product
+    S16::Frag foq[2];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (ks + 1 < 4) {
-#pragma unroll
-        for (int ci = 0; ci < KT; ++ci) fq[(ks + 1) & 1][ci] = M::load_t(sQc, LDK, 16 * (ks + 1), 32 * ci, lane);
-        fo[(ks + 1) & 1] = M::load_t(sOc, LDV, 16 * (ks + 1), vs, lane);
-      }
-#pragma unroll
-      for (int ci = 0; ci < KT; ++ci) M::mma(dS[ci], fq[ks & 1][ci], fo[ks & 1]);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int s_ = 0; s_ < 2; ++s_) {
+      const floatx4 f0 = load4(sc + Scal::SG + 32 * s_ + g4), f1 = load4(sc + Scal::SG + 32 * s_ + 16 + g4);
+      foq[s_] = S16::from_acc(f0 * floatx4{(float)fo[s_][0], (float)fo[s_][1], (float)fo[s_][2], (float)fo[s_][3]},
+                              f1 * floatx4{(float)fo[s_][4], (float)fo[s_][5], (float)fo[s_][6], (float)fo[s_][7]});
     }
     // ---- dD = Pm^T dO + e^{G_C - G} Z ----
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 4; ++i) dd[i] += sv[i] * z[i];
+    S16::Frag bd0 = S16::from_acc(dd[0], dd[1]), bd1 = S16::from_acc(dd[2], dd[3]);
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+    for (int ci = 0; ci < KT; ++ci) S16::mma(dS[ci], fq[0][ci], foq[0]);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) dd[i][4 * q + u] += sv[i][q][u] * z[i][4 * q + u];
-    M::Frag bd[4];
+    for (int ci = 0; ci < KT; ++ci) fq[1][ci] = S16::load_cols<CHAIN>(sQc, LDK, 32, ci, lane);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) bd[ks] = M::from_acc(dd[ks >> 1], ks & 1);
+    for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::GAM + 16 * i + g4);
     __builtin_amdgcn_sched_barrier(0);
     // ---- dR = Tm^T dD (lane = value column, in z) and once more with the operands exchanged (lane = token, in dd), which
     //      is the orientation dv = beta dR leaves in ----
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 4; ++i) z[i] = dd[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 16; ++e) z[i][e] = dd[i][e] = 0.f;
-    M::Frag fu[2][KT];  // K^T fragments of the dS update
+    for (int i = 0; i < 4; ++i) S16::mma(z[i], ft[i], bd1);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (ks + 2 < 4) {
+    for (int i = 0; i < 2; ++i) S16::mma(z[i], ft[i + 4], bd0);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) fa[(ks + 2) % 3][i] = M::load_t_chain(sTc, LDC, 16 * (ks + 2), 32 * i, lane);
-      } else if (ks == 2) {
+    for (int i = 0; i < 4; ++i) S16::mma(dd[i], bd1, ft[i]);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) S16::mma(dd[i], bd0, ft[i + 4]);
+    S16::Frag fu[2][KT];  // K^T fragments of the dS update
 #pragma unroll
-          for (int q = 0; q < 4; ++q) sv[i][q] = load4(sc + Scal::GAM + 32 * i + 8 * q + 4 * (lane >> 5));
-      } else {
+    for (int ci = 0; ci < KT; ++ci) fu[0][ci] = S16::load_cols<CHAIN>(sKc, LDK, 0, ci, lane);
+    float bl[4];
 #pragma unroll
-        for (int ci = 0; ci < KT; ++ci) fu[0][ci] = M::load_t_chain(sKc, LDK, 0, 32 * ci, lane);
-      }
+    for (int i = 0; i < 4; ++i) bl[i] = sc[Scal::BETA + 16 * i + l16];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        if (i == 0 || ks >= 2) M::mma(z[i], fa[ks % 3][i], bd[ks]);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        if (i == 0 || ks >= 2) M::mma(dd[i], bd[ks], fa[ks % 3][i]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    const float bl0 = sc[Scal::BETA + fr], bl1 = sc[Scal::BETA + 32 + fr];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) store_frag_t(z[i], sdRT + vs * LDC + 32 * i, LDC, lane);
-    // dY = -beta e^G dR
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) z[i][4 * q + u] *= -sv[i][q][u];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) bd[ks] = M::from_acc(z[ks >> 1], ks & 1);
+    for (int ci = 0; ci < KT; ++ci) S16::mma(dS[ci], fq[1][ci], foq[1]);
     __builtin_amdgcn_sched_barrier(0);
-    // dv = beta dR: fragment dd[i] holds tokens 32 i .. (one per lane) x the strip's value columns
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      dd[0][e] *= bl0;
-      dd[1][e] *= bl1;
-    }
+    for (int i = 0; i < 4; ++i) store_t(z[i], sdRT + vs * LDD + 16 * i, LDD, lane);
+    // dY = -beta e^G dR
+    bd0 = S16::from_acc(-sv[0] * z[0], -sv[1] * z[1]);
+    bd1 = S16::from_acc(-sv[2] * z[2], -sv[3] * z[3]);
+    // dv = beta dR: tile dd[i] holds tokens 16 i .. (one per lane) x the strip's value columns
 #pragma unroll
-    for (int i = 0; i < 2; ++i) store_frag_t(dd[i], sdV + 32 * i * LDV + vs, LDV, lane);
+    for (int i = 0; i < 4; ++i) store_t(dd[i] * bl[i], sdV + 16 * i * LDV + vs, LDV, lane);
     lds_barrier();  // Bmid
     // ---- dS += K^T dY ----
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (ks + 1 < 4) {
+    for (int ci = 0; ci < KT; ++ci) fu[1][ci] = S16::load_cols<CHAIN>(sKc, LDK, 32, ci, lane);
 #pragma unroll
-        for (int ci = 0; ci < KT; ++ci) fu[(ks + 1) & 1][ci] = M::load_t_chain(sKc, LDK, 16 * (ks + 1), 32 * ci, lane);
-      }
+    for (int ci = 0; ci < KT; ++ci) S16::mma(dS[ci], fu[0][ci], bd0);
 #pragma unroll
-      for (int ci = 0; ci < KT; ++ci) M::mma(dS[ci], fu[ks & 1][ci], bd[ks]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int ci = 0; ci < KT; ++ci) S16::mma(dS[ci], fu[1][ci], bd1);
     lds_barrier();  // B1 of the next chunk
   }
   if (p.ds0) {
-    float* out = p.ds0 + (int64_t)sidx * DK * p.dv + v0 + vs + frag_col(lane);
+    float* out = p.ds0 + (int64_t)sidx * DK * p.dv + v0 + vs + l16;
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) out[(int64_t)(32 * ci + frag_row(e, lane)) * p.dv] = dS[ci][e];
+      for (int e = 0; e < 4; ++e) out[(int64_t)(16 * ci + g4 + e) * p.dv] = dS[ci][e];
   }
 }
 

@@ -97,6 +97,70 @@ template <> struct Mma<bf16_t> {
   }
 };
 
+// 16 x 16 x 32 products of bf16 operands, for waves that own 16 columns.  Accumulator: element r of lane (l16 = lane & 15,
+// g = lane >> 4) is row 4 g + r, column l16.  Contraction order ("chain order"): lane group g holds the indices
+// 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3 of a step of 32, which is how two accumulator tiles of 16 rows lie in
+// registers, so a result is the next product's operand without a trip through LDS.
+struct Mma16 {
+  typedef bf16x8 Frag;
+  typedef short short4_ __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) short4_ lds_short4;
+  static __device__ __forceinline__ void mma(floatx4& c, const Frag& a, const Frag& b) {
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ Frag join(bf16x4 lo, bf16x4 hi) {
+    typedef unsigned uint4_ __attribute__((ext_vector_type(4)));
+    typedef unsigned uint2_ __attribute__((ext_vector_type(2)));
+    const uint2_ a = __builtin_bit_cast(uint2_, lo), b = __builtin_bit_cast(uint2_, hi);
+    return __builtin_bit_cast(Frag, (uint4_{a[0], a[1], b[0], b[1]}));
+  }
+  static __device__ __forceinline__ Frag from_acc(floatx4 lo, floatx4 hi) { return join(pack_bf16x4(lo), pack_bf16x4(hi)); }
+  // Tiles whose rows are operands ([rows][k], k along the row) lie in LDS in one of two column orders.  Plain: an operand is
+  // two 8-byte reads.  CHAIN: inside each block of 32 columns, position 8 g + j holds column 4 g + j (j < 4) or
+  // 16 + 4 g + j - 4, so an operand is one ds_read_b128 per step, and an aligned vector of eight columns is written in two
+  // halves.  Measured per KB of the CU's LDS: ds_read_b128 3.9 cycles where rows are 32 bytes off a multiple of 64 (288, 160)
+  // and 6.6 at 272 or 144; two ds_read_b64 5.4; the ds_read2_b64 that hipcc makes of them 12 - 16 (hence the volatile reads);
+  // writes 7.5 - 13 in one piece, 9 - 16 in two.  A wave can have 15 reads in flight, so a wave whose chain waits for its reads
+  // wants CHAIN; where the movers' writes are what a chunk waits for, plain is the better one.
+  template <bool CHAIN> static __device__ __forceinline__ int pos(int c) {  // of the vector at column c, c % 8 == 0
+    return CHAIN ? (c & ~31) + ((c >> 3) & 1) * 16 + ((c >> 4) & 1) * 4 : c;
+  }
+  template <bool CHAIN> static __device__ __forceinline__ void put(bf16_t* p, bf16x8 v) {  // p: the row at pos(c)
+    if (CHAIN) {
+      *reinterpret_cast<bf16x4*>(p) = bf16x4{v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<bf16x4*>(p + 8) = bf16x4{v[4], v[5], v[6], v[7]};
+    } else {
+      *reinterpret_cast<bf16x8*>(p) = v;
+    }
+  }
+  // operand rows: p points at (this lane's row l16, first column of the step)
+  template <bool CHAIN> static __device__ __forceinline__ Frag load(const bf16_t* p, int lane) {
+    if (CHAIN) return *reinterpret_cast<const bf16x8*>(p + 8 * (lane >> 4));
+    typedef float float2_ __attribute__((ext_vector_type(2)));
+    typedef const volatile __attribute__((address_space(3))) float2_ lds_float2;
+    lds_float2* q = (lds_float2*)(p + 4 * (lane >> 4));
+    const float2_ lo = q[0], hi = q[4];
+    return join(__builtin_bit_cast(bf16x4, lo), __builtin_bit_cast(bf16x4, hi));
+  }
+  // operand from the columns 16 ci + l16 of such a tile (contraction along the tile's rows)
+  template <bool CHAIN> static __device__ __forceinline__ Frag load_cols(const bf16_t* tile, int ld, int k0, int ci, int lane) {
+    const int s = lane & 15;
+    const bf16_t* p = tile + (k0 + 4 * (lane >> 4) + (s >> 2)) * ld + (CHAIN ? 32 * (ci >> 1) + 4 * (ci & 1) + 8 * (s & 3) : 16 * ci + 4 * (s & 3));
+    return join(__builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(p))),
+                __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(p + 16 * ld))));
+  }
+  // four consecutive rows r0 + 4 g .. of column c0 + l16 of a row-major tile: one transposing read
+  static __device__ __forceinline__ bf16x4 rows4(const bf16_t* tile, int ld, int r0, int c0, int lane) {
+    const int s = lane & 15;
+    const bf16_t* p = tile + (r0 + 4 * (lane >> 4) + (s >> 2)) * ld + c0 + 4 * (s & 3);
+    return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(p)));
+  }
+  // the same from a plain row-major [k][rows] tile, rows c0 + l16
+  static __device__ __forceinline__ Frag load_t(const bf16_t* tile, int ld, int k0, int c0, int lane) {
+    return join(rows4(tile, ld, k0, c0, lane), rows4(tile, ld, k0 + 16, c0, lane));
+  }
+};
+
 template <> struct Mma<float> {
   static constexpr int KS = 8;
   static constexpr int VEC = 4;
@@ -336,8 +400,8 @@ __device__ __forceinline__ void tri_vec_pos(int idx, int& r, int& c) {  // idx <
   c = o - q * (g + 1);
 }
 // The packed tile in the registers of 256 threads (vector tid, and vector 256 + tid for tid < 32) between its global
-// loads and its LDS stores, like TileRegs; the LDS tile's upper part is zeroed once by the caller and never written.
-template <typename T> struct TriRegs {
+// loads and its LDS stores (columns in the order CHAIN of Mma16), like TileRegs; the LDS tile's upper part is zeroed once by the caller and never written.
+template <typename T, bool CHAIN> struct TriRegs {
   static_assert(sizeof(T) == 2, "packed triangles are a 2-byte format");
   typename Vec16<T>::V x[2];
   int o0, o1;  // LDS element offsets of this thread's two vectors for a leading dimension fixed at init
@@ -345,10 +409,10 @@ template <typename T> struct TriRegs {
   __device__ __forceinline__ void init(int ld, int tid) {
     int r, c;
     tri_vec_pos(tid, r, c);
-    o0 = r * ld + 8 * c;
+    o0 = r * ld + Mma16::pos<CHAIN>(8 * c);
     second = tid < LNX_TRI_VECS - 256;
     tri_vec_pos(second ? 256 + tid : LNX_TRI_VECS - 1, r, c);
-    o1 = r * ld + 8 * c;
+    o1 = r * ld + Mma16::pos<CHAIN>(8 * c);
   }
   __device__ __forceinline__ void load(const T* src, int tid) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(src), 0, LNX_TRI_VECS * 16, 0x00020000);
@@ -357,8 +421,8 @@ template <typename T> struct TriRegs {
     x[1] = __builtin_bit_cast(typename Vec16<T>::V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * (256 + tid), 0, 0));
   }
   __device__ __forceinline__ void store(T* dst) const {
-    *reinterpret_cast<typename Vec16<T>::V*>(dst + o0) = x[0];
-    if (second) *reinterpret_cast<typename Vec16<T>::V*>(dst + o1) = x[1];
+    Mma16::put<CHAIN>(dst + o0, x[0]);
+    if (second) Mma16::put<CHAIN>(dst + o1, x[1]);
   }
 };
 

@@ -9,6 +9,7 @@ DEV = "cuda"
 
 
 def _close(got, want, tol=1e-5):
+    got, want = got.detach(), want.detach()
     e = float((got.double() - want.double()).abs().max() / want.double().abs().max().clamp_min(1e-30))
     assert e < tol, e
 
