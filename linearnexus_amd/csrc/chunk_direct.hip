@@ -37,9 +37,9 @@ typedef Mma<T> M;
 typedef Mma16 S16;
 template <typename X> __device__ __forceinline__ X* at(char* ws, uint64_t off) { return reinterpret_cast<X*>(ws + off); }
 
-// dst[l16][4 g ..] = accumulator tile of 16 rows (transposed store: this lane's column, four consecutive rows, 8 bytes)
+// dst[l16][grp ..] = accumulator tile in Mma16's order of rows (transposed store: this lane's column, four consecutive rows, 8 bytes)
 __device__ __forceinline__ void store_t(const floatx4& a, T* dst, int ld, int lane) {
-  store4(dst + (lane & 15) * ld + 4 * (lane >> 4), a);
+  store4(dst + (lane & 15) * ld + S16::grp(lane), a);
 }
 
 // dst[col][row0 + ...] = fragment (transposed store, four consecutive rows per 8-byte vector)
@@ -62,9 +62,16 @@ template <bool CHAIN> __device__ __forceinline__ void zero_upper_triangles(T* ti
   for (int t = 0; t < ntile; ++t) S16::put<CHAIN>(tiles + t * stride + r * ld + S16::pos<CHAIN>(8 * c), vec_zero<T>());
 }
 
+// A row's elements times its factor, rounded back
+__device__ __forceinline__ typename Vec16<T>::V scaled(typename Vec16<T>::V x, float f) {
+#pragma unroll
+  for (int e = 0; e < Vec16<T>::N; ++e) x[e] = (bf16_t)((float)x[e] * f);
+  return x;
+}
+
 // Per-token scalars of one chunk in LDS, written by the movers when they commit a chunk
 struct Scal {
-  enum { BETA = 0, GAM = 64, R = 128, SG = 192, DEC = 256, SIZE = 320 };  // beta, beta e^G / |k|, e^{G_C - G} / |k|, scale e^G / |q|, e^{G_C}
+  enum { BETA = 0, GAM = 64, R = 128, DEC = 192, SIZE = 256 };  // beta, beta e^G, e^{G_C - G}, e^{G_C}
 };
 
 // ---------------------------------------------------------------------------------------
@@ -72,9 +79,11 @@ struct Scal {
 // accumulators for the whole sequence, and the chain  S -> Y = K S -> R -> D = Tm R -> S'  never leaves the wave's
 // registers -- two accumulator tiles are the B operand of the next product as they are (Mma16::from_acc), only the A
 // operands (K, Q, Tm, Pm rows) come from LDS.  Strips of 16 columns put a slab's chain on twice as many SIMDs as strips of 32:
-// B2 H16 T2007 d128 (32 chunks in a row, 128 workgroups) 65 -> 49 us forward and 74 -> 57 us in reverse, one prompt of 1000
-// tokens 32 -> 23 us, B8 H16 T4096 204 -> 190 and 217 -> 206 us.  What is left of a chunk's 1.5 us there: a SIMD takes 1 KB of
-// LDS reads in about 16 cycles, and a strip reads 60 KB of operands whatever its width.  All five input tiles are double-buffered, so the movers write chunk
+// B2 H16 T2007 d128 (32 chunks in a row, 128 workgroups) 65 -> 57 us forward and 74 -> 59 us in reverse, one prompt of 1000
+// tokens 34 -> 29 us, B8 H16 T4096 204 -> 198 and 217 -> 207 us; the bits are those of 32-column strips (Mma16).  What is left of
+// a chunk's 1.7 us there: a SIMD takes 1 KB of LDS reads in about 16 cycles, and a strip reads 60 KB of operands whatever its
+// width; then the movers' conversions of K and Q rows.
+//  All five input tiles are double-buffered, so the movers write chunk
 // n + 1 while chunk n is being read and two barriers per chunk are enough:
 //   B1    buffers of chunk n complete           compute: S^T -> LDS (saved states), Y, Q S, R, D (-> LDS, transposed), O -> LDS
 //                                               movers:  loads of chunk n + 2; chunk n + 1 -> the other buffers
@@ -134,7 +143,8 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
       RowTile K, Q;
       ValTile V;
       TriRegs<T, CHAIN> Tm, P;  // lower-triangular tiles, packed in the workspace
-      float g, gc, b, fq, nk;  // per-token scalars of token mt % 64
+      float g, gc, b;  // per-token scalars of token mt % 64
+      float fq[RowTile::IT], nk[RowTile::IT];  // factors of the token each of this thread's Q / K vectors belongs to
       float bv[ValTile::IT];  // beta of the token each of its V vectors belongs to
       int len;
     };
@@ -143,7 +153,8 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     ta.Tm.init(LDC, mt), ta.P.init(LDC, mt), tb.Tm.init(LDC, mt), tb.P.init(LDC, mt);
     zero_upper_triangles<CHAIN>(sTm, 4, L::kC, LDC, mt);  // both buffers of Tm and Pm: the packed tiles never write there
     ta.len = tb.len = 0;
-    ta.fq = tb.fq = ta.nk = tb.nk = 0.f;
+#pragma unroll
+    for (int it = 0; it < RowTile::IT; ++it) ta.fq[it] = tb.fq[it] = ta.nk[it] = tb.nk[it] = 0.f;
 #pragma unroll
     for (int it = 0; it < ValTile::IT; ++it) ta.bv[it] = tb.bv[it] = 0.f;
     // part 0: K, 1: Q, 2: the rest; < 0: everything
@@ -165,22 +176,25 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
         R.g = G[t];
         R.gc = G[63];
       }
-      R.fq = at<const float>(p.ws, p.off.Fq)[slot * 64 + t];
-      R.nk = at<const float>(p.ws, p.off.Nk)[slot * 64 + t];
+#pragma unroll
+      for (int it = 0; it < RowTile::IT; ++it) {
+        R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
+        R.nk[it] = at<const float>(p.ws, p.off.Nk)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
+      }
       R.b = p.beta[tbase + (int64_t)min(t, R.len - 1) * p.geom.ts];
 #pragma unroll
       for (int it = 0; it < ValTile::IT; ++it)
         R.bv[it] = p.beta[tbase + (int64_t)min(min((mt + 256 * it) / ValTile::VPR, 63), R.len - 1) * p.geom.ts];
     };
-    // K and Q rows go to LDS as they are: their factors (1 / |k|, scale e^G / |q|) are rows of the products' results or of
-    // the other operand and enter there in fp32, sixteen multiplications per compute wave instead of a conversion both
-    // ways for every element in the movers
+    // K rows normalised (their own bits where nothing is to be normalised), Q rows normalised and scaled by scale e^{G_i}
     auto commit = [&](const Tiles& R, int pb, int part = -1) {
 #pragma unroll
       for (int it = 0; it < RowTile::IT; ++it) {
         const int idx = mt + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
-        if (part < 0 || part == 0) S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), R.K.x[it]);
-        if (part < 0 || part == 1) S16::put<CHAIN>(sQ + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), R.Q.x[it]);
+        if (part < 0 || part == 0)
+          S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), p.l2norm ? scaled(R.K.x[it], R.nk[it]) : R.K.x[it]);
+        if (part < 0 || part == 1)
+          S16::put<CHAIN>(sQ + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), scaled(R.Q.x[it], R.fq[it]));
       }
       if (part == 0 || part == 1) return;
       {  // V rows scaled by beta_i: R = beta V - (beta e^G) Y
@@ -199,9 +213,8 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
       if (mt < 64) {
         float* sc = sSc + pb * Scal::SIZE;
         const float gam = (GATE == LNX_GATE_SCALAR) ? __expf(R.g) : 1.f;
-        sc[Scal::GAM + mt] = (mt < R.len) ? R.b * gam * R.nk : 0.f;
-        sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) * R.nk : R.nk;
-        sc[Scal::SG + mt] = R.fq;
+        sc[Scal::GAM + mt] = (mt < R.len) ? R.b * gam : 0.f;
+        sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) : 1.f;
         if (mt == 0) sc[Scal::DEC] = (GATE == LNX_GATE_SCALAR) ? __expf(R.gc) : 1.f;
       }
     };
@@ -261,7 +274,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
 
   // ---------------- compute waves: wave w owns value columns [16 w, 16 w + 16) of the slab ----------------
   const int vs = 16 * wave;
-  const int l16 = lane & 15, g4 = 4 * (lane >> 4);
+  const int l16 = lane & 15, lr = S16::row(lane), g4 = S16::grp(lane);
   floatx4 S[KT];
 #pragma unroll
   for (int ci = 0; ci < KT; ++ci) S[ci] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -270,7 +283,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[ci][e] = s0[(int64_t)(16 * ci + g4 + e) * p.dv];
+      for (int e = 0; e < 4; ++e) S[ci][e] = s0[(int64_t)(S16::row0(ci) + g4 + e) * p.dv];
     // the loads complete here: left pending into the loop, every iteration would count them down again
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)
@@ -292,7 +305,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     const float* sc = sSc + pb * Scal::SIZE;
     if (p.save) {
 #pragma unroll
-      for (int ci = 0; ci < KT; ++ci) store_t(S[ci], sST + vs * LDS + 16 * ci, LDS, lane);
+      for (int ci = 0; ci < KT; ++ci) store_t(S[ci], sST + vs * LDS + S16::row0(ci), LDS, lane);
     }
     // ---- Y = K S (lane = value column) and (Q~ S)^T (lane = token): the state fragments are the shared operand ----
     floatx4 y[4], o[4];
@@ -300,10 +313,10 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     for (int i = 0; i < 4; ++i) y[i] = o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
     S16::Frag fa[2][4], fb[2][4];  // [step mod 2][token tile]
     bf16x4 vr[4];                  // beta V at this lane's accumulator positions
-    floatx4 sv[4];                 // per-row scalars at this lane's accumulator positions: beta e^G / |k|, later e^{G_C - G} / |k|
+    floatx4 sv[4];                 // per-row scalars at this lane's accumulator positions: beta e^G, later e^{G_C - G}
     S16::Frag tm[6], pm[6];        // [token tile, step]: (0,0) (1,0) (2,0) (3,0) (2,1) (3,1): Tm and Pm are lower-triangular
 #pragma unroll
-    for (int i = 0; i < 4; ++i) fa[0][i] = S16::load<CHAIN>(sKc + (16 * i + l16) * LDK, lane);
+    for (int i = 0; i < 4; ++i) fa[0][i] = S16::load<CHAIN>(sKc + (S16::row0(i) + lr) * LDK, lane);
 #pragma unroll
     for (int i = 0; i < 4; ++i) fb[0][i] = S16::load<CHAIN>(sQc + (16 * i + l16) * LDK, lane);
     // at most 16 LDS reads are in flight (the wave's counter ends at 15): K of the next step goes out ahead of this step's
@@ -313,12 +326,12 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
       const S16::Frag b = S16::from_acc(S[2 * ks], S[2 * ks + 1]);
       if (ks + 1 < NK) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) fa[(ks + 1) & 1][i] = S16::load<CHAIN>(sKc + (16 * i + l16) * LDK + 32 * (ks + 1), lane);
+        for (int i = 0; i < 4; ++i) fa[(ks + 1) & 1][i] = S16::load<CHAIN>(sKc + (S16::row0(i) + lr) * LDK + 32 * (ks + 1), lane);
       } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) vr[i] = S16::rows4(sVc, LDV, 16 * i, vs, lane);
+        for (int i = 0; i < 4; ++i) vr[i] = S16::rows4(sVc, LDV, S16::row0(i) + g4, vs, lane);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::GAM + 16 * i + g4);
+        for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::GAM + S16::row0(i) + g4);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) S16::mma(y[i], fa[ks & 1][i], b);
@@ -330,9 +343,9 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
         for (int i = 0; i < 4; ++i) fb[(ks + 1) & 1][i] = S16::load<CHAIN>(sQc + (16 * i + l16) * LDK + 32 * (ks + 1), lane);
       } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) tm[i] = S16::load<CHAIN>(sTc + (16 * i + l16) * LDC, lane);
+        for (int i = 0; i < 4; ++i) tm[i] = S16::load<CHAIN>(sTc + (S16::row0(i) + lr) * LDC, lane);
 #pragma unroll
-        for (int i = 2; i < 4; ++i) tm[i + 2] = S16::load<CHAIN>(sTc + (16 * i + l16) * LDC + 32, lane);
+        for (int i = 2; i < 4; ++i) tm[i + 2] = S16::load<CHAIN>(sTc + (S16::row0(i) + lr) * LDC + 32, lane);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -344,9 +357,6 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     floatx4 d[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) d[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float fq[4];  // scale e^G / |q| of this lane's token in each tile of o
-#pragma unroll
-    for (int i = 0; i < 4; ++i) fq[i] = sc[Scal::SG + 16 * i + l16];
     form_r(0), form_r(1);
     const S16::Frag br0 = S16::from_acc(y[0], y[1]);
 #pragma unroll
@@ -359,9 +369,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     S16::mma(d[2], tm[4], br1);
     S16::mma(d[3], tm[5], br1);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::R + 16 * i + g4);  // e^{G_C - G} / |k| for the state update
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] *= fq[i];
+    for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::R + S16::row0(i) + g4);  // e^{G_C - G} for the state update
     const float dec = (GATE == LNX_GATE_SCALAR) ? sc[Scal::DEC] : 1.f;
     __builtin_amdgcn_sched_barrier(0);
     // ---- O^T = (Q~ S)^T + D^T Pm^T ----
@@ -374,7 +382,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
 #pragma unroll
     for (int ci = 0; ci < 4; ++ci) fu[0][ci] = S16::load_cols<CHAIN>(sKc, LDK, 0, ci, lane);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) store_t(d[i], sDT + vs * LDD + 16 * i, LDD, lane);  // also when nothing is saved: a branch here would split the schedule
+    for (int i = 0; i < 4; ++i) store_t(d[i], sDT + vs * LDD + S16::row0(i), LDD, lane);  // also when nothing is saved: a branch here would split the schedule
     const S16::Frag bd1 = S16::from_acc(d[2], d[3]);
     S16::mma(o[2], bd1, pm[4]);
     S16::mma(o[3], bd1, pm[5]);
@@ -386,7 +394,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) store_t(o[i], sO + 16 * i * LDV + vs, LDV, lane);  // [token][value column]
+    for (int i = 0; i < 4; ++i) store4(sO + (16 * i + l16) * LDV + vs + 4 * (lane >> 4), o[i]);  // [token][value column]
     lds_barrier();  // Bmid
     // ---- S <- e^{G_C} S + K^T (e^{G_C - G} D) ----
 #pragma unroll
@@ -409,7 +417,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
 #pragma unroll
   for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) out[(int64_t)(16 * ci + g4 + e) * p.dv] = S[ci][e];
+    for (int e = 0; e < 4; ++e) out[(int64_t)(S16::row0(ci) + g4 + e) * p.dv] = S[ci][e];
 }
 
 template <int DK, int GATE, typename OT>
@@ -488,7 +496,8 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
       RowTile K, Q;
       TileRegs<T, 64, BV> dO;
       TriRegs<T, CHAIN> Tm, P;  // lower-triangular tiles, packed in the workspace
-      float g, gc, b, fq, nk;  // per-token scalars of token mt % 64
+      float g, gc, b;  // per-token scalars of token mt % 64
+      float fq[RowTile::IT], nk[RowTile::IT];  // factors of the token each of this thread's Q / K vectors belongs to
       int len;
     };
     Tiles ta, tb;
@@ -496,7 +505,8 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
     ta.Tm.init(LDC, mt), ta.P.init(LDC, mt), tb.Tm.init(LDC, mt), tb.P.init(LDC, mt);
     zero_upper_triangles<CHAIN>(sTm, 4, L::kC, LDC, mt);  // both buffers of Tm and Pm: the packed tiles never write there
     ta.len = tb.len = 0;
-    ta.fq = tb.fq = ta.nk = tb.nk = 0.f;
+#pragma unroll
+    for (int it = 0; it < RowTile::IT; ++it) ta.fq[it] = tb.fq[it] = ta.nk[it] = tb.nk[it] = 0.f;
     auto fetch = [&](Tiles& R, int n, int part = -1) {  // part 0: K, 1: Q, 2: the rest; < 0: everything
       const int64_t slot = (int64_t)row * N + n;
       int tok0;
@@ -514,19 +524,22 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
         R.g = G[t];
         R.gc = G[63];
       }
-      R.fq = at<const float>(p.ws, p.off.Fq)[slot * 64 + t];
-      R.nk = at<const float>(p.ws, p.off.Nk)[slot * 64 + t];
+#pragma unroll
+      for (int it = 0; it < RowTile::IT; ++it) {
+        R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
+        R.nk[it] = at<const float>(p.ws, p.off.Nk)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
+      }
       R.b = p.beta[tbase + (int64_t)min(t, R.len - 1) * p.geom.ts];
     };
-    // K and Q rows go to LDS as they are: their factors (1 / |k|, scale e^G / |q|) are rows of the products' results or of
-    // the other operand and enter there in fp32, sixteen multiplications per compute wave instead of a conversion both
-    // ways for every element in the movers
+    // K rows normalised (their own bits where nothing is to be normalised), Q rows normalised and scaled by scale e^{G_i}
     auto commit = [&](const Tiles& R, int pb, int part = -1) {
 #pragma unroll
       for (int it = 0; it < RowTile::IT; ++it) {
         const int idx = mt + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
-        if (part < 0 || part == 0) S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), R.K.x[it]);
-        if (part < 0 || part == 1) S16::put<CHAIN>(sQ + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), R.Q.x[it]);
+        if (part < 0 || part == 0)
+          S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), p.l2norm ? scaled(R.K.x[it], R.nk[it]) : R.K.x[it]);
+        if (part < 0 || part == 1)
+          S16::put<CHAIN>(sQ + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), scaled(R.Q.x[it], R.fq[it]));
       }
       if (part == 0 || part == 1) return;
       R.dO.store(sdO + pb * L::kV, LDV, mt);
@@ -537,9 +550,8 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
         const float gam = (GATE == LNX_GATE_SCALAR) ? __expf(R.g) : 1.f;
         const float bt = (mt < R.len) ? R.b : 0.f;
         sc[Scal::BETA + mt] = bt;
-        sc[Scal::GAM + mt] = bt * gam * R.nk;  // dY = -(beta e^G) dR
-        sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) * R.nk : R.nk;
-        sc[Scal::SG + mt] = R.fq;
+        sc[Scal::GAM + mt] = bt * gam;  // dY = -(beta e^G) dR
+        sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) : 1.f;
         if (mt == 0) sc[Scal::DEC] = (GATE == LNX_GATE_SCALAR) ? __expf(R.gc) : 1.f;
       }
     };
@@ -587,7 +599,7 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
 
   // ---------------- compute waves ----------------
   const int vs = 16 * wave;
-  const int l16 = lane & 15, g4 = 4 * (lane >> 4);
+  const int l16 = lane & 15, lr = S16::row(lane), g4 = S16::grp(lane);
   floatx4 dS[KT];
 #pragma unroll
   for (int ci = 0; ci < KT; ++ci) dS[ci] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -596,7 +608,7 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dS[ci][e] = src[(int64_t)(16 * ci + g4 + e) * p.dv];
+      for (int e = 0; e < 4; ++e) dS[ci][e] = src[(int64_t)(S16::row0(ci) + g4 + e) * p.dv];
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
@@ -617,15 +629,16 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
     S16::Frag fa[2][4];  // K rows, [step mod 2][token tile]
     S16::Frag ft[6];     // Pm^T, then Tm^T: [token tile, step] (0,1) (1,1) (2,1) (3,1) (0,0) (1,0): upper-triangular
     S16::Frag fo[2];     // dO
-    floatx4 sv[4];       // per-row scalars at this lane's accumulator positions: e^{G_C - G} / |k|, later beta e^G / |k|
-    auto load_tri = [&](const T* tile) {
+    floatx4 sv[4];       // per-row scalars at this lane's accumulator positions: e^{G_C - G}, later beta e^G
+    auto load_tri = [&](const T* tile, auto natural) {
+      constexpr bool NATURAL = decltype(natural)::value;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) ft[i] = S16::load_cols<CHAIN>(tile, LDC, 32, i, lane);
+      for (int i = 0; i < 4; ++i) ft[i] = S16::load_cols<CHAIN, NATURAL>(tile, LDC, 32, i, lane);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) ft[i + 4] = S16::load_cols<CHAIN>(tile, LDC, 0, i, lane);
+      for (int i = 0; i < 2; ++i) ft[i + 4] = S16::load_cols<CHAIN, NATURAL>(tile, LDC, 0, i, lane);
     };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) fa[0][i] = S16::load<CHAIN>(sKc + (16 * i + l16) * LDK, lane);
+    for (int i = 0; i < 4; ++i) fa[0][i] = S16::load<CHAIN>(sKc + (S16::row0(i) + lr) * LDK, lane);
 #pragma unroll
     for (int s_ = 0; s_ < 2; ++s_) fo[s_] = S16::load_t(sOc, LDV, 32 * s_, vs, lane);
     // the state gradient as the B operand of Z = K dS'; its accumulators are then free to take the next dS
@@ -633,7 +646,7 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) bs[ks] = S16::from_acc(dS[2 * ks], dS[2 * ks + 1]);
 #pragma unroll
-    for (int ci = 0; ci < KT; ++ci) store_t(dS[ci], sdST + vs * LDS + 16 * ci, LDS, lane);
+    for (int ci = 0; ci < KT; ++ci) store_t(dS[ci], sdST + vs * LDS + S16::row0(ci), LDS, lane);
     const float dec = (GATE == LNX_GATE_SCALAR) ? sc[Scal::DEC] : 1.f;
     // ---- Z = K dS' and the chunk-local part Pm^T dO ----
     floatx4 z[4], dd[4];
@@ -643,79 +656,71 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
     for (int ks = 0; ks < NK; ++ks) {
       if (ks + 1 < NK) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) fa[(ks + 1) & 1][i] = S16::load<CHAIN>(sKc + (16 * i + l16) * LDK + 32 * (ks + 1), lane);
+        for (int i = 0; i < 4; ++i) fa[(ks + 1) & 1][i] = S16::load<CHAIN>(sKc + (S16::row0(i) + lr) * LDK + 32 * (ks + 1), lane);
       } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::R + 16 * i + g4);
+        for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::R + S16::row0(i) + g4);
       }
-      if (ks == 0) load_tri(sPc);
+      if (ks == 0) load_tri(sPc, std::true_type{});
 #pragma unroll
       for (int i = 0; i < 4; ++i) S16::mma(z[i], fa[ks & 1][i], bs[ks]);
       if (ks == NK - 1) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S16::mma(dd[i], ft[i], fo[1]);
-#pragma unroll
         for (int i = 0; i < 2; ++i) S16::mma(dd[i], ft[i + 4], fo[0]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S16::mma(dd[i], ft[i], fo[1]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
     // ---- dS <- e^{G_C} dS' + (scale e^G Q)^T dO fills the wait for Z; Tm^T is fetched behind it ----
     S16::Frag fq[2][KT];
 #pragma unroll
-    for (int ci = 0; ci < KT; ++ci) fq[0][ci] = S16::load_cols<CHAIN>(sQc, LDK, 0, ci, lane);
-    load_tri(sTc);
+    for (int ci = 0; ci < KT; ++ci) fq[0][ci] = S16::load_cols<CHAIN, true>(sQc, LDK, 0, ci, lane);
+    load_tri(sTc, std::false_type{});
     if (GATE == LNX_GATE_SCALAR) {
 #pragma unroll
       for (int ci = 0; ci < KT; ++ci) dS[ci] *= dec;
-    }
-    // dO rows times scale e^G / |q|, the operand of the Q^T dO product
-    S16::Frag foq[2];
-#pragma unroll
-    for (int s_ = 0; s_ < 2; ++s_) {
-      const floatx4 f0 = load4(sc + Scal::SG + 32 * s_ + g4), f1 = load4(sc + Scal::SG + 32 * s_ + 16 + g4);
-      foq[s_] = S16::from_acc(f0 * floatx4{(float)fo[s_][0], (float)fo[s_][1], (float)fo[s_][2], (float)fo[s_][3]},
-                              f1 * floatx4{(float)fo[s_][4], (float)fo[s_][5], (float)fo[s_][6], (float)fo[s_][7]});
     }
     // ---- dD = Pm^T dO + e^{G_C - G} Z ----
 #pragma unroll
     for (int i = 0; i < 4; ++i) dd[i] += sv[i] * z[i];
     S16::Frag bd0 = S16::from_acc(dd[0], dd[1]), bd1 = S16::from_acc(dd[2], dd[3]);
 #pragma unroll
-    for (int ci = 0; ci < KT; ++ci) S16::mma(dS[ci], fq[0][ci], foq[0]);
+    for (int ci = 0; ci < KT; ++ci) S16::mma(dS[ci], fq[0][ci], fo[0]);
 #pragma unroll
-    for (int ci = 0; ci < KT; ++ci) fq[1][ci] = S16::load_cols<CHAIN>(sQc, LDK, 32, ci, lane);
+    for (int ci = 0; ci < KT; ++ci) fq[1][ci] = S16::load_cols<CHAIN, true>(sQc, LDK, 32, ci, lane);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::GAM + 16 * i + g4);
+    for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::GAM + S16::row0(i) + g4);
     __builtin_amdgcn_sched_barrier(0);
     // ---- dR = Tm^T dD (lane = value column, in z) and once more with the operands exchanged (lane = token, in dd), which
     //      is the orientation dv = beta dR leaves in ----
 #pragma unroll
     for (int i = 0; i < 4; ++i) z[i] = dd[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) S16::mma(z[i], ft[i], bd1);
-#pragma unroll
     for (int i = 0; i < 2; ++i) S16::mma(z[i], ft[i + 4], bd0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) S16::mma(dd[i], bd1, ft[i]);
-#pragma unroll
     for (int i = 0; i < 2; ++i) S16::mma(dd[i], bd0, ft[i + 4]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S16::mma(z[i], ft[i], bd1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S16::mma(dd[i], bd1, ft[i]);
     S16::Frag fu[2][KT];  // K^T fragments of the dS update
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci) fu[0][ci] = S16::load_cols<CHAIN>(sKc, LDK, 0, ci, lane);
     float bl[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) bl[i] = sc[Scal::BETA + 16 * i + l16];
+    for (int i = 0; i < 4; ++i) bl[i] = sc[Scal::BETA + S16::row0(i) + lr];
 #pragma unroll
-    for (int ci = 0; ci < KT; ++ci) S16::mma(dS[ci], fq[1][ci], foq[1]);
+    for (int ci = 0; ci < KT; ++ci) S16::mma(dS[ci], fq[1][ci], fo[1]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) store_t(z[i], sdRT + vs * LDD + 16 * i, LDD, lane);
+    for (int i = 0; i < 4; ++i) store_t(z[i], sdRT + vs * LDD + S16::row0(i), LDD, lane);
     // dY = -beta e^G dR
     bd0 = S16::from_acc(-sv[0] * z[0], -sv[1] * z[1]);
     bd1 = S16::from_acc(-sv[2] * z[2], -sv[3] * z[3]);
     // dv = beta dR: tile dd[i] holds tokens 16 i .. (one per lane) x the strip's value columns
 #pragma unroll
-    for (int i = 0; i < 4; ++i) store_t(dd[i] * bl[i], sdV + 16 * i * LDV + vs, LDV, lane);
+    for (int i = 0; i < 4; ++i) store4(sdV + (S16::row0(i) + lr) * LDV + vs + 4 * (lane >> 4), dd[i] * bl[i]);
     lds_barrier();  // Bmid
     // ---- dS += K^T dY ----
 #pragma unroll
@@ -731,7 +736,7 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) out[(int64_t)(16 * ci + g4 + e) * p.dv] = dS[ci][e];
+      for (int e = 0; e < 4; ++e) out[(int64_t)(S16::row0(ci) + g4 + e) * p.dv] = dS[ci][e];
   }
 }
 

@@ -97,10 +97,13 @@ template <> struct Mma<bf16_t> {
   }
 };
 
-// 16 x 16 x 32 products of bf16 operands, for waves that own 16 columns.  Accumulator: element r of lane (l16 = lane & 15,
-// g = lane >> 4) is row 4 g + r, column l16.  Contraction order ("chain order"): lane group g holds the indices
-// 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3 of a step of 32, which is how two accumulator tiles of 16 rows lie in
-// registers, so a result is the next product's operand without a trip through LDS.
+// 16 x 16 x 32 products of bf16 operands, for waves that own 16 columns.  Lane: l16 = lane & 15, g = lane >> 4.  The product adds
+// its eight contraction slots of group 0 first, then those of groups 1, 2, 3 -- the order in which two 32 x 32 x 16 products
+// add theirs -- so with group g holding what (step g >> 1, half g & 1) holds there, both give the same bits, and 16- and
+// 32-column strips can be exchanged freely.  In the order that chained products use ("chain order") group g holds the indices
+// grp(g) + 0 .. 3 and grp(g) + 8 .. 11 of a step of 32, grp(g) = 16 (g >> 1) + 4 (g & 1); in natural order 8 g .. 8 g + 7.
+// Accumulators that become operands: tile i of a column of tiles covers the rows  row0(i) + grp(g) + r  (element r of group
+// g), row0(i) = 32 (i >> 1) + 8 (i & 1), so tiles 2 s and 2 s + 1 in registers are the operand of step s in chain order.
 struct Mma16 {
   typedef bf16x8 Frag;
   typedef short short4_ __attribute__((ext_vector_type(4)));
@@ -114,16 +117,19 @@ struct Mma16 {
     const uint2_ a = __builtin_bit_cast(uint2_, lo), b = __builtin_bit_cast(uint2_, hi);
     return __builtin_bit_cast(Frag, (uint4_{a[0], a[1], b[0], b[1]}));
   }
+  static __device__ __forceinline__ int row0(int i) { return 32 * (i >> 1) + 8 * (i & 1); }
+  static __device__ __forceinline__ int grp(int lane) { return 16 * ((lane >> 5) & 1) + 4 * ((lane >> 4) & 1); }
+  static __device__ __forceinline__ int row(int lane) { return 16 * ((lane >> 3) & 1) + (lane & 7); }  // of operand row l16 in such a tile
   static __device__ __forceinline__ Frag from_acc(floatx4 lo, floatx4 hi) { return join(pack_bf16x4(lo), pack_bf16x4(hi)); }
   // Tiles whose rows are operands ([rows][k], k along the row) lie in LDS in one of two column orders.  Plain: an operand is
-  // two 8-byte reads.  CHAIN: inside each block of 32 columns, position 8 g + j holds column 4 g + j (j < 4) or
-  // 16 + 4 g + j - 4, so an operand is one ds_read_b128 per step, and an aligned vector of eight columns is written in two
+  // two 8-byte reads.  CHAIN: inside each block of 32 columns, position 8 g + j holds column grp(g) + j (j < 4) or
+  // grp(g) + 4 + j, so an operand is one ds_read_b128 per step, and an aligned vector of eight columns is written in two
   // halves.  Measured per KB of the CU's LDS: ds_read_b128 3.9 cycles where rows are 32 bytes off a multiple of 64 (288, 160)
   // and 6.6 at 272 or 144; two ds_read_b64 5.4; the ds_read2_b64 that hipcc makes of them 12 - 16 (hence the volatile reads);
   // writes 7.5 - 13 in one piece, 9 - 16 in two.  A wave can have 15 reads in flight, so a wave whose chain waits for its reads
   // wants CHAIN; where the movers' writes are what a chunk waits for, plain is the better one.
   template <bool CHAIN> static __device__ __forceinline__ int pos(int c) {  // of the vector at column c, c % 8 == 0
-    return CHAIN ? (c & ~31) + ((c >> 3) & 1) * 16 + ((c >> 4) & 1) * 4 : c;
+    return CHAIN ? (c & ~31) + ((c >> 4) & 1) * 16 + ((c >> 3) & 1) * 4 : c;
   }
   template <bool CHAIN> static __device__ __forceinline__ void put(bf16_t* p, bf16x8 v) {  // p: the row at pos(c)
     if (CHAIN) {
@@ -133,31 +139,32 @@ struct Mma16 {
       *reinterpret_cast<bf16x8*>(p) = v;
     }
   }
-  // operand rows: p points at (this lane's row l16, first column of the step)
+  // operand rows in chain order: p points at (this lane's row, first column of the step)
   template <bool CHAIN> static __device__ __forceinline__ Frag load(const bf16_t* p, int lane) {
     if (CHAIN) return *reinterpret_cast<const bf16x8*>(p + 8 * (lane >> 4));
     typedef float float2_ __attribute__((ext_vector_type(2)));
     typedef const volatile __attribute__((address_space(3))) float2_ lds_float2;
-    lds_float2* q = (lds_float2*)(p + 4 * (lane >> 4));
-    const float2_ lo = q[0], hi = q[4];
+    lds_float2* q = (lds_float2*)(p + grp(lane));
+    const float2_ lo = q[0], hi = q[2];
     return join(__builtin_bit_cast(bf16x4, lo), __builtin_bit_cast(bf16x4, hi));
   }
-  // operand from the columns 16 ci + l16 of such a tile (contraction along the tile's rows)
-  template <bool CHAIN> static __device__ __forceinline__ Frag load_cols(const bf16_t* tile, int ld, int k0, int ci, int lane) {
+  // operand from the columns of tile ci of such a tile (contraction along the tile's rows from k0)
+  template <bool CHAIN, bool NATURAL = false> static __device__ __forceinline__ Frag load_cols(const bf16_t* tile, int ld, int k0, int ci, int lane) {
     const int s = lane & 15;
-    const bf16_t* p = tile + (k0 + 4 * (lane >> 4) + (s >> 2)) * ld + (CHAIN ? 32 * (ci >> 1) + 4 * (ci & 1) + 8 * (s & 3) : 16 * ci + 4 * (s & 3));
+    const bf16_t* p = tile + (k0 + (NATURAL ? 8 * (lane >> 4) : grp(lane)) + (s >> 2)) * ld + 32 * (ci >> 1) +
+                      (CHAIN ? 4 * (ci & 1) + 8 * (s & 3) : 8 * (ci & 1) + 16 * ((s >> 1) & 1) + 4 * (s & 1));
     return join(__builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(p))),
-                __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(p + 16 * ld))));
+                __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(p + (NATURAL ? 4 : 8) * ld))));
   }
-  // four consecutive rows r0 + 4 g .. of column c0 + l16 of a row-major tile: one transposing read
+  // four consecutive rows from r0 of column c0 + l16 of a row-major tile (r0 may differ between groups of 16 lanes): one transposing read
   static __device__ __forceinline__ bf16x4 rows4(const bf16_t* tile, int ld, int r0, int c0, int lane) {
     const int s = lane & 15;
-    const bf16_t* p = tile + (r0 + 4 * (lane >> 4) + (s >> 2)) * ld + c0 + 4 * (s & 3);
+    const bf16_t* p = tile + (r0 + (s >> 2)) * ld + c0 + 4 * (s & 3);
     return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(p)));
   }
-  // the same from a plain row-major [k][rows] tile, rows c0 + l16
+  // operand in natural order from a plain row-major [k][columns] tile, columns c0 + l16
   static __device__ __forceinline__ Frag load_t(const bf16_t* tile, int ld, int k0, int c0, int lane) {
-    return join(rows4(tile, ld, k0, c0, lane), rows4(tile, ld, k0 + 16, c0, lane));
+    return join(rows4(tile, ld, k0 + 8 * (lane >> 4), c0, lane), rows4(tile, ld, k0 + 8 * (lane >> 4) + 4, c0, lane));
   }
 };
 
