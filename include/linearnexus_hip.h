@@ -150,6 +150,16 @@ int lnx_recurrent_fwd(const lnx_scan_args* a, void* hip_stream);
 uint64_t lnx_chunk_workspace_bytes(const lnx_scan_args* a);
 int lnx_chunk_fwd(const lnx_scan_args* a, void* hip_stream);
 /*
+ * lnx_chunk_fwd of one long sequence (B == 1, no cu_seqlens, forward_only = 1) as nseg segments of whole chunks that run in
+ * parallel, for calls with too few (head, value slab) chains to fill the GPU.  The scan is linear in the state: a first pass
+ * from [0 | I] leaves [B_i | A_i] with S_out = A_i S_in + B_i per segment, these are chained, and a second pass from the
+ * chained states gives the outputs.  nseg must be the number of segments of ceil(ceil(T / 64) / nseg) chunks that T tokens
+ * make.  final_state is [nseg, H, dk, dv] here: the states at the end of every segment, the last one being the final state.
+ * The workspace takes lnx_chunk_fwd_segmented_bytes(a, nseg).
+ */
+uint64_t lnx_chunk_fwd_segmented_bytes(const lnx_scan_args* a, int32_t nseg);
+int lnx_chunk_fwd_segmented(const lnx_scan_args* a, int32_t nseg, void* hip_stream);
+/*
  * 1 when lnx_chunk_fwd / lnx_chunk_bwd apply the in-op normalisation of q and k themselves for these arguments
  * (use_qk_l2norm = 1: gated_deltanet.py:273-275, kda.py:379-381 normalise inside the op, and it is their default):
  * q, k, v in bf16, dk <= 128, no per-channel gate.  The rows are scaled where the kernels stage them and the

@@ -1322,33 +1322,32 @@ __global__ void copy_state_kernel(const float* src, float* dst, int64_t n) {
 }
 
 // packed batches: slot table [N][2] = (token0, len), then seq_chunk0[nseq + 1], then the sequence
-// indices by decreasing length (ties by index).  One workgroup: the first chunk slot of every sequence by a serial
-// prefix over the (few) sequences, then all threads fill the slots, each finding its sequence by bisection.
-__global__ void build_table_kernel(const int32_t* cu, int nseq, int N, int T, int32_t* tab) {
-  int32_t* chunk0 = tab + 2 * N;
-  int32_t* order = chunk0 + nseq + 1;
+// indices by decreasing length (ties by index).  One workgroup: every thread sums the slots of the sequences before its own
+// (independent loads; a serial prefix waited for each), then all threads fill the slots, each finding its sequence by
+// bisection in LDS.
+constexpr int TABLE_LDS = 1024;  // sequences whose first slots fit there
+__global__ __launch_bounds__(1024) void build_table_kernel(const int32_t* cu, int nseq, int N, int T, int32_t* tab) {
+  __shared__ int32_t first_slot[TABLE_LDS + 1];
+  int32_t* out0 = tab + 2 * N;
+  int32_t* chunk0 = nseq <= TABLE_LDS ? first_slot : out0;
+  int32_t* order = out0 + nseq + 1;
   // a malformed table (entries outside [0, T] or decreasing) must not send any kernel outside the tensors
   auto first = [&](int s) { return seq_first(cu, s, T); };
   auto length = [&](int s) { return seq_end(cu, s, T) - seq_first(cu, s, T); };
   for (int s = threadIdx.x; s < nseq; s += blockDim.x) {
     const int ls = length(s);
-    int rank = 0;
+    int rank = 0, c = 0;
     for (int u = 0; u < nseq; ++u) {
       const int lu = length(u);
       rank += (lu > ls) || (lu == ls && u < s);
+      if (u < s) c += (lu + LNX_C - 1) / LNX_C;
     }
     order[rank] = s;
-  }
-  if (threadIdx.x == 0) {
-    int c = 0;
-    for (int s = 0; s < nseq; ++s) {
-      chunk0[s] = min(c, N);
-      c += (length(s) + LNX_C - 1) / LNX_C;
-    }
-    chunk0[nseq] = min(c, N);
+    out0[s] = chunk0[s] = min(c, N);
+    if (s == nseq - 1) out0[nseq] = chunk0[nseq] = min(c + (ls + LNX_C - 1) / LNX_C, N);
   }
   __threadfence_block();
-  __syncthreads();  // chunk0 is read back from global memory by the other threads
+  __syncthreads();  // chunk0 is read back by the other threads, from global memory where it does not fit LDS
   const int total = chunk0[nseq];
   for (int c = threadIdx.x; c < N; c += blockDim.x) {
     int t0 = 0, len = 0;
@@ -1482,8 +1481,10 @@ void launch_prepare_lite(const FwdParams& p, hipStream_t st) {
   hipLaunchKernelGGL(k, dim3((unsigned)((int64_t)p.geom.rows * p.geom.N)), dim3(256), b, st, p);
 }
 
-int launch_direct_fwd(const lnx_scan_args* a, const FwdParams& p, int nstate, hipStream_t st) {
-  if (a->dk == 128) {
+int launch_direct_fwd(const lnx_scan_args* a, const FwdParams& p, int nstate, bool prepared, hipStream_t st) {
+  if (prepared) {
+    // Tm, Pm, G and the row factors do not depend on the values or the states
+  } else if (a->dk == 128) {
     if (a->gate == LNX_GATE_SCALAR) launch_prepare_lite<128, LNX_GATE_SCALAR>(p, st);
     else launch_prepare_lite<128, LNX_GATE_NONE>(p, st);
   } else {
@@ -1504,8 +1505,9 @@ int launch_direct_fwd(const lnx_scan_args* a, const FwdParams& p, int nstate, hi
   return LNX_OK;
 }
 
-// The forward pass on a caller-chosen workspace (a->workspace is not looked at).
-int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_bytes, hipStream_t st) {
+// The forward pass on a caller-chosen workspace (a->workspace is not looked at).  `prepared`: the same call but for v, dv and
+// the states has just used this workspace, whose sequence table and value-independent tensors are taken over.
+int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_bytes, hipStream_t st, bool prepared = false) {
   const bool packed = a->cu_seqlens != nullptr;
   const int nstate = packed ? a->nseq : a->B;
   if (nstate == 0) return LNX_OK;
@@ -1521,8 +1523,8 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
     return lnx_set_error(LNX_ERR_WORKSPACE, "workspace of %llu bytes needed, %llu given", (unsigned long long)w.total,
                          (unsigned long long)workspace_bytes);
   char* ws = reinterpret_cast<char*>(workspace);
-  if (packed)
-    hipLaunchKernelGGL(build_table_kernel, dim3(1), dim3(256), 0, st, a->cu_seqlens, a->nseq, lnx_chunk_slots(a), a->T,
+  if (packed && !prepared)
+    hipLaunchKernelGGL(build_table_kernel, dim3(1), dim3(1024), 0, st, a->cu_seqlens, a->nseq, lnx_chunk_slots(a), a->T,
                        reinterpret_cast<int32_t*>(ws + w.tab));
   FwdParams p;
   p.geom.H = a->H; p.geom.T = a->T; p.geom.N = lnx_chunk_slots(a); p.geom.nseq = a->nseq;
@@ -1541,7 +1543,7 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
   p.l2norm = a->use_qk_l2norm;
   p.ws = ws; p.off = w;
   int rc;
-  if (lnx_chunk_direct(a)) return launch_direct_fwd(a, p, nstate, st);
+  if (lnx_chunk_direct(a)) return launch_direct_fwd(a, p, nstate, prepared, st);
   if (a->dtype == LNX_BF16)  // dk <= 128 without a per-channel gate went to the direct-solve kernels above
     rc = (a->dk == 256)   ? launch_fwd_gate<bf16_t, 256>(a->gate, p, nstate, st)
          : (a->dk == 128) ? launch_fwd<bf16_t, 128, LNX_GATE_VECTOR>(p, nstate, st)
@@ -1555,6 +1557,101 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
   if (e != hipSuccess) return lnx_set_error(LNX_ERR_LAUNCH, "chunk forward launch: %s", hipGetErrorString(e));
   return LNX_OK;
 }
+
+// ---------------------------------------------------------------------------------------
+// A long sequence in segments (lnx_chunk_fwd_segmented).  setup: cu_seqlens of the segments and their states [0 | I].
+// chain: s_in[0] = s0, s_in[i + 1] = B_i + A_i s_in[i], where segment i left [B_i | A_i] in ab [n, H, dk, dv + dk].
+// One workgroup per (head, 16 value columns): the columns stay in LDS (transposed) for all segments, wave w forms rows
+// 16 w .. on the fp32 matrix cores (16x16x4) with its rows of the next A_i on their way meanwhile.  A step waits for 64 KB
+// of A_i from L2 and 4 products of 32 in a row: 16 segments of 4 heads d128 21 us, where a batched library product and
+// two copies per step took 310 us.
+// ---------------------------------------------------------------------------------------
+__global__ void segment_setup_kernel(int32_t* cu, int n, int seg, int T, float* ab, int dk, int dv, int64_t total) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i <= n) cu[i] = min((int)i * seg, T);
+  const int w = (dk + dv) / 4;
+  if (i >= total / 4) return;
+  const int c = 4 * (int)(i % w), r = (int)((i / w) % dk);
+  floatx4 x;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = c + e - dv == r ? 1.f : 0.f;
+  store4(ab + 4 * i, x);
+}
+
+template <int DK> constexpr int segment_chain_threads = DK == 64 ? 256 : 512;
+template <int DK>
+__global__ __launch_bounds__(segment_chain_threads<DK>) void segment_chain_kernel(const float* ab, const float* s0, float* s_in, int n, int H, int dv) {
+  constexpr int THREADS = segment_chain_threads<DK>, PW = DK / (THREADS / 4), NT = DK / 16;  // row tiles of a wave; 16-wide steps over k
+  constexpr int LD = DK + 4;
+  __shared__ __align__(16) float sS[2][16 * LD];  // [column][k]
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, kq = lane >> 4;
+  const int h = blockIdx.x, v0 = 16 * blockIdx.y;
+  const int ldab = dv + DK;
+  auto tile = [&](int t) { return PW * wave + t; };
+  struct Rows {
+    floatx4 a[PW][NT], b[PW];
+  };
+  auto fetch = [&](Rows& r, int i) {
+    const float* m = ab + ((int64_t)i * H + h) * DK * ldab;
+#pragma unroll
+    for (int t = 0; t < PW; ++t) {
+#pragma unroll
+      for (int s = 0; s < NT; ++s) r.a[t][s] = load4(m + (int64_t)(16 * tile(t) + l16) * ldab + dv + 16 * s + 4 * kq);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r.b[t][e] = m[(int64_t)(16 * tile(t) + 4 * kq + e) * ldab + v0 + l16];
+    }
+  };
+  for (int i = tid; i < DK * 16; i += THREADS) sS[0][(i & 15) * LD + (i >> 4)] = s0 ? s0[((int64_t)h * DK + (i >> 4)) * dv + v0 + (i & 15)] : 0.f;
+  constexpr bool AHEAD = DK <= 128;  // two sets of registers: the next rows are requested before this step's products
+  Rows ra, rb;
+  fetch(ra, 0);
+  // no load behind a branch, where its wait could not be counted: the last steps fetch and multiply what nobody reads
+  auto step = [&](Rows& r, Rows& next, int i) {
+    lds_barrier();
+    const float* cur = sS[i & 1];
+    if (AHEAD) fetch(next, min(i + 1, n - 1));
+    float* out = s_in + ((int64_t)i * H + h) * DK * dv + v0;
+    for (int j = tid; j < DK * 16; j += THREADS) out[(int64_t)(j >> 4) * dv + (j & 15)] = cur[(j & 15) * LD + (j >> 4)];
+    floatx4 acc[PW][2];
+#pragma unroll
+    for (int t = 0; t < PW; ++t) acc[t][0] = r.b[t], acc[t][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NT; ++s) {
+      const floatx4 x = load4(cur + l16 * LD + 16 * s + 4 * kq);
+#pragma unroll
+      for (int t = 0; t < PW; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[t][s & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.a[t][s][e], x[e], acc[t][s & 1], 0, 0, 0);
+    }
+    if (!AHEAD) fetch(r, min(i + 1, n - 1));
+#pragma unroll
+    for (int t = 0; t < PW; ++t) store4(sS[(i + 1) & 1] + l16 * LD + 16 * tile(t) + 4 * kq, acc[t][0] + acc[t][1]);
+  };
+  for (int i = 0; i < n; i += 2) {
+    step(ra, AHEAD ? rb : ra, i);
+    if (i + 1 < n) step(AHEAD ? rb : ra, ra, i + 1);
+  }
+}
+
+// The two passes' arguments and where the parts of the workspace lie.
+struct Segmented {
+  lnx_scan_args first, second;
+  int seg, n;
+  uint64_t cu, ab, s_in, ws_bytes, total;
+  explicit Segmented(const lnx_scan_args* a, int nseg) {
+    const int chunks = (a->T + LNX_C - 1) / LNX_C;
+    seg = (chunks + nseg - 1) / nseg * LNX_C, n = (a->T + seg - 1) / seg;
+    first = second = *a;
+    first.nseq = second.nseq = n;
+    first.cu_seqlens = second.cu_seqlens = reinterpret_cast<const int32_t*>(16);  // only their presence enters the layout
+    first.dv = a->dv + a->dk, first.value_cols = a->dv, first.o = nullptr;
+    ws_bytes = std::max(lnx_chunk_ws_layout(&first).total, lnx_chunk_ws_layout(&second).total);
+    cu = ws_bytes, ab = cu + lnx_align256((uint64_t)(n + 1) * 4);
+    const uint64_t states = (uint64_t)n * a->H * a->dk;
+    s_in = ab + lnx_align256(states * (a->dv + a->dk) * 4);
+    total = s_in + states * a->dv * 4;
+  }
+};
 
 // Library-owned scratch of lnx_chunk_fwd_static: one copy per GPU, at its own address on each, alive until the
 // process ends.  The name below is a host-side handle only; device code gets the address looked up per device.
@@ -1598,6 +1695,37 @@ extern "C" int lnx_chunk_fwd(const lnx_scan_args* a, void* stream) {
   int rc = lnx_chunk_check(a, false);
   if (rc != LNX_OK) return rc;
   return chunk_fwd_on(a, a->workspace, a->workspace_bytes, (hipStream_t)stream);
+}
+
+extern "C" uint64_t lnx_chunk_fwd_segmented_bytes(const lnx_scan_args* a, int32_t nseg) {
+  if (!a || a->B != 1 || a->H <= 0 || a->T <= 0 || nseg <= 0 || a->cu_seqlens || (a->dk != 64 && a->dk != 128 && a->dk != 256) || a->dv <= 0 || a->dv % 64 != 0)
+    return 0;
+  return Segmented(a, nseg).total;
+}
+
+extern "C" int lnx_chunk_fwd_segmented(const lnx_scan_args* a, int32_t nseg, void* stream) {
+  int rc = lnx_chunk_check(a, false);
+  if (rc != LNX_OK) return rc;
+  if (a->B != 1 || a->T <= 0 || a->cu_seqlens || !a->forward_only || !a->o || a->value_cols != 0 || nseg <= 0)
+    return lnx_set_error(LNX_ERR_SHAPE, "lnx_chunk_fwd_segmented takes one dense sequence (B = %d, T = %d, nseg = %d), forward_only and an output", a->B, a->T, nseg);
+  Segmented g(a, nseg);
+  if (g.n != nseg) return lnx_set_error(LNX_ERR_SHAPE, "%d tokens make %d segments of whole chunks, not %d", a->T, g.n, nseg);
+  if (!a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 15) || a->workspace_bytes < g.total)
+    return lnx_set_error(LNX_ERR_WORKSPACE, "an aligned workspace of %llu bytes needed, %llu given", (unsigned long long)g.total, (unsigned long long)a->workspace_bytes);
+  hipStream_t st = (hipStream_t)stream;
+  char* ws = reinterpret_cast<char*>(a->workspace);
+  int32_t* cu = reinterpret_cast<int32_t*>(ws + g.cu);
+  float *ab = reinterpret_cast<float*>(ws + g.ab), *s_in = reinterpret_cast<float*>(ws + g.s_in);
+  const int64_t total = (int64_t)g.n * a->H * a->dk * (a->dv + a->dk);
+  hipLaunchKernelGGL(segment_setup_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, st, cu, g.n, g.seg, a->T, ab, a->dk, a->dv, total);
+  g.first.cu_seqlens = g.second.cu_seqlens = cu;
+  g.first.initial_state = ab, g.first.final_state = ab;  // every workgroup of the scan reads its columns before it writes them
+  g.second.initial_state = s_in;
+  if ((rc = chunk_fwd_on(&g.first, ws, g.ws_bytes, st)) != LNX_OK) return rc;
+  auto chain = a->dk == 256 ? segment_chain_kernel<256> : a->dk == 128 ? segment_chain_kernel<128> : segment_chain_kernel<64>;
+  lnx_profile_mark("segment_chain", st);
+  hipLaunchKernelGGL(chain, dim3(a->H, a->dv / 16), dim3(a->dk == 64 ? 256 : 512), 0, st, ab, a->initial_state, s_in, g.n, a->H, a->dv);
+  return chunk_fwd_on(&g.second, ws, g.ws_bytes, st, lnx_chunk_direct(a));
 }
 
 extern "C" int lnx_chunk_fwd_static_init(void) {

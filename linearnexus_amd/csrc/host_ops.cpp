@@ -352,8 +352,8 @@ PyObject* py_l2norm_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 // What one chunk call is given besides its tensors.
 struct ChunkOptions {
   double scale = 1.0, threshold = 0.0;
-  bool l2norm = false, forward_only = false, want_o = true, raw_gate = false;
-  int64_t o_dtype = 0, dv_total = 0;  // dv_total > 0: the state has that many value columns, v holds the first ones
+  bool l2norm = false, forward_only = false;
+  int64_t o_dtype = 0;
   int64_t scan_slab = 0, out_slabs = 0;  // test hooks of lnx_scan_args
   Tensor cu;                             // sequence table of a packed batch, or undefined
 };
@@ -377,8 +377,7 @@ std::pair<Tensor, Tensor> chunk_forward(const Tensor& q, const Tensor& k, const 
                                         const Tensor& A_log, const Tensor& g_bias, const ChunkOptions& opt_, ChunkCall& c) {
   const Tensor& cu = opt_.cu;
   const SeqShape s = seq_shape(q, k, v, g, beta, cu);
-  const int64_t dv = opt_.dv_total ? opt_.dv_total : s.dv;
-  check_state(s0, s, dv);
+  check_state(s0, s, s.dv);
   const bool tf = is_token_first(q) && is_token_first(k) && is_token_first(v);
   c.q_in = as_layout(q, tf), c.k_in = as_layout(k, tf), c.v = as_layout(v, tf);
   c.beta = as_layout(beta.to(at::kFloat), tf);
@@ -386,9 +385,9 @@ std::pair<Tensor, Tensor> chunk_forward(const Tensor& q, const Tensor& k, const 
   c.s0 = f32(s0), c.cu = cu;
   c.A = f32(A_log), c.bias = f32(g_bias);
   const auto o_t = type_of(opt_.o_dtype);
-  const Tensor o = opt_.want_o ? empty_layout(s.B, s.H, s.T, dv, q.options().dtype(o_t), tf) : Tensor();
-  const Tensor sT = at::empty({s.nstate, s.H, s.dk, dv}, q.options().dtype(at::kFloat));
-  lnx_scan_args a = base_args(s.B, s.H, s.T, s.dk, dv, code_of(q.scalar_type()), (int)opt_.o_dtype, s.gate, false, opt_.scale);
+  const Tensor o = empty_layout(s.B, s.H, s.T, s.dv, q.options().dtype(o_t), tf);
+  const Tensor sT = at::empty({s.nstate, s.H, s.dk, s.dv}, q.options().dtype(at::kFloat));
+  lnx_scan_args a = base_args(s.B, s.H, s.T, s.dk, s.dv, code_of(q.scalar_type()), (int)opt_.o_dtype, s.gate, false, opt_.scale);
   a.test_scan_slab = (int32_t)opt_.scan_slab, a.test_out_slabs = (int32_t)opt_.out_slabs;
   // The reference's chunk path normalises in the input dtype before anything else (gated_deltanet.py:273-275,
   // kda.py:379-381).  Where the kernels scale the rows themselves (no normalised copies, gradients carried through the
@@ -401,7 +400,6 @@ std::pair<Tensor, Tensor> chunk_forward(const Tensor& q, const Tensor& k, const 
   a.nseq = (int32_t)s.nseq;
   a.token_first = tf;
   a.forward_only = opt_.forward_only;
-  a.value_cols = dv == s.dv ? 0 : (int32_t)s.dv;
   a.q = ptr(c.qn), a.k = ptr(c.kn), a.v = ptr(c.v), a.beta = fptr(c.beta), a.g = fptr(c.g);
   a.initial_state = fptr(c.s0), a.final_state = fptr(sT), a.o = ptr(o), a.cu_seqlens = static_cast<const int32_t*>(ptr(cu));
   set_gate(a, c, opt_.threshold);
@@ -473,18 +471,56 @@ struct ChunkFn : Function<ChunkFn> {
   }
 };
 
-// chunk(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu, forward_only, dv_total, want_o, A_log, g_bias, threshold,
+// chunk_segmented(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, nseg): (o, final state) of a forward-only call on dense
+// sequences, cut into about nseg segments that run in parallel (lnx_chunk_fwd_segmented); batch rows become heads.
+PyObject* py_chunk_segmented(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  LNX_BEGIN
+  Args in(args, nargs, 10, "chunk_segmented");
+  at::NoGradGuard no_grad;
+  const Tensor q0 = in.tensor(0, "q"), k0 = in.tensor(1, "k"), v0 = in.tensor(2, "v"), g0 = in.maybe(3, "g"), s00 = in.maybe(5, "initial_state");
+  const Tensor beta0 = squeeze_beta(in.tensor(4, "beta"), 4);
+  const SeqShape s = seq_shape(q0, k0, v0, g0, beta0, Tensor());
+  check_state(s00, s, s.dv);
+  const int64_t rows = s.B * s.H, chunks = (s.T + 63) / 64, per = (chunks + in.integer(9) - 1) / in.integer(9), nseg = (chunks + per - 1) / per;
+  auto fold = [&](const Tensor& t) {
+    if (!t.defined() || s.B == 1) return t;
+    std::vector<int64_t> sizes = t.sizes().vec();
+    sizes[0] = 1, sizes[1] = rows;
+    return t.reshape(sizes);
+  };
+  const Tensor q1 = fold(q0), k1 = fold(k0), v1 = fold(v0);
+  const bool tf = is_token_first(q1) && is_token_first(k1) && is_token_first(v1);
+  Tensor q = as_layout(q1, tf), k = as_layout(k1, tf);
+  const Tensor v = as_layout(v1, tf), beta = as_layout(fold(beta0).to(at::kFloat), tf), g = g0.defined() ? as_layout(fold(g0).to(at::kFloat), tf) : g0, s0 = f32(s00);
+  const int64_t o_dtype = in.integer(8);
+  const Tensor o = empty_layout(1, rows, s.T, s.dv, q.options().dtype(type_of(o_dtype)), tf);
+  const Tensor sT = at::empty({nseg, rows, s.dk, s.dv}, q.options().dtype(at::kFloat));
+  lnx_scan_args a = base_args(1, rows, s.T, s.dk, s.dv, code_of(q.scalar_type()), (int)o_dtype, s.gate, false, in.number(6));
+  a.use_qk_l2norm = in.flag(7) && lnx_chunk_fuses_l2norm(&a);
+  if (in.flag(7) && !a.use_qk_l2norm) q = l2norm_fwd(q), k = l2norm_fwd(k);
+  a.token_first = tf, a.forward_only = 1;
+  a.q = ptr(q), a.k = ptr(k), a.v = ptr(v), a.beta = fptr(beta), a.g = fptr(g);
+  a.initial_state = fptr(s0), a.final_state = fptr(sT), a.o = ptr(o);
+  const uint64_t nbytes = lnx_chunk_fwd_segmented_bytes(&a, (int32_t)nseg);
+  const Tensor ws = at::empty({(int64_t)std::max<uint64_t>(nbytes, 1)}, q.options().dtype(at::kByte));
+  a.workspace = ptr(ws), a.workspace_bytes = nbytes;
+  check_status(lnx_chunk_fwd_segmented(&a, (int32_t)nseg, stream_of(q)), "lnx_chunk_fwd_segmented");
+  return pack(s.B == 1 ? o : o.reshape({s.B, s.H, s.T, s.dv}), sT.select(0, nseg - 1).view({s.B, s.H, s.dk, s.dv}));
+  LNX_END
+}
+
+// chunk(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu, forward_only, A_log, g_bias, threshold,
 //       scan_slab, out_slabs): (o or None, final state), in the graph unless forward_only
 PyObject* py_chunk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   LNX_BEGIN
-  Args in(args, nargs, 18, "chunk");
+  Args in(args, nargs, 16, "chunk");
   const Tensor q = in.tensor(0, "q"), k = in.tensor(1, "k"), v = in.tensor(2, "v"), g = in.maybe(3, "g"), s0 = in.maybe(5, "initial_state"),
-               A_log = in.maybe(13, "A_log"), g_bias = in.maybe(14, "g_bias");
+               A_log = in.maybe(11, "A_log"), g_bias = in.maybe(12, "g_bias");
   const Tensor beta = squeeze_beta(in.tensor(4, "beta"), 4);
   ChunkOptions o;
   o.cu = in.maybe(9, "cu_seqlens");
   o.scale = in.number(6), o.l2norm = in.flag(7), o.o_dtype = in.integer(8), o.forward_only = in.flag(10);
-  o.dv_total = in.integer(11), o.want_o = in.flag(12), o.threshold = in.number(15), o.scan_slab = in.integer(16), o.out_slabs = in.integer(17);
+  o.threshold = in.number(13), o.scan_slab = in.integer(14), o.out_slabs = in.integer(15);
   if (!o.forward_only) {
     const variable_list r = ChunkFn::apply(q, k, v, opt(g), beta, opt(s0), opt(A_log), opt(g_bias), o);
     return pack(r[0], r[1]);
@@ -949,7 +985,7 @@ PyObject* py_set_kernel_error(PyObject*, PyObject* const* args, Py_ssize_t nargs
 }
 
 #define LNX_FN(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_##name)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {LNX_FN(step),     LNX_FN(recurrent), LNX_FN(l2norm), LNX_FN(l2norm_bwd), LNX_FN(chunk),     LNX_FN(conv1d),           LNX_FN(rmsnorm_gated), LNX_FN(gdn_gate),
+PyMethodDef methods[] = {LNX_FN(step),     LNX_FN(recurrent), LNX_FN(l2norm), LNX_FN(l2norm_bwd), LNX_FN(chunk), LNX_FN(chunk_segmented),     LNX_FN(conv1d),           LNX_FN(rmsnorm_gated), LNX_FN(gdn_gate),
                          LNX_FN(kda_gate), LNX_FN(dplr),      LNX_FN(dplr_step), LNX_FN(set_kernel_error), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Host path of the linearnexus_amd ops.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

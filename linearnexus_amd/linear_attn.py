@@ -269,16 +269,14 @@ def _l2norm_rows_bwd(x: Tensor, dy: Tensor) -> Tensor:
 
 
 def _chunk_forward(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens, forward_only,
-                   dv_total=None, want_o=True, raw_gate=None):
+                   raw_gate=None):
     """One chunked scan, ``(o, final_state)``.  Without ``forward_only`` the call is a node of the autograd graph
-    whose backward is lnx_chunk_bwd; with it the kernels skip what only a backward pass reads.  ``dv_total`` > v's
-    columns: the state has dv_total value columns of which v holds the first ones and the others are zero
-    (``value_cols``); ``want_o=False``: final states only.  Both forward-only.  ``raw_gate = (A_log, g_bias or None,
+    whose backward is lnx_chunk_bwd; with it the kernels skip what only a backward pass reads.  ``raw_gate = (A_log, g_bias or None,
     threshold)``: ``g`` is the raw per-channel gate projection in q's dtype and the kernels apply kda_gate's
     activation themselves."""
     A_log, g_bias, threshold = raw_gate or (None, None, 0.0)
     return _lib.host().chunk(q, k, v, g, beta, initial_state, scale, l2norm, _DT[o_dtype], _packed_table(cu_seqlens, q),
-                             forward_only, dv_total or 0, want_o, A_log, g_bias, threshold,
+                             forward_only, A_log, g_bias, threshold,
                              _test_hooks["scan_slab"], _test_hooks["out_slabs"])
 
 
@@ -305,34 +303,11 @@ def _segmented_forward(q, k, v, g, beta, scale, initial_state, l2norm, o_dtype, 
     """Forward pass of a long sequence as nseg segments processed in parallel (no gradients).
 
     The scan is linear in the state: over a segment s, S_out = A_s S_in + B_s with A_s [dk, dk] the product of the
-    segment's token transitions and B_s [dk, dv] what the segment writes into a zero state.  One packed call with the
-    value columns extended to [v | 0] and every segment started from [0 | I] returns [B_s | A_s] as its final states;
-    a short loop chains the segments' entering states; a second packed call with those as initial states gives the
+    segment's token transitions and B_s [dk, dv] what the segment writes into a zero state.  One pass with the
+    value columns extended to [v | 0] and every segment started from [0 | I] leaves [B_s | A_s] as its final states;
+    a short kernel chains the segments' entering states; a second pass with those as initial states gives the
     outputs.  (The same (A_s, B_s) pair is what ranks would exchange if a sequence were split across GPUs.)"""
-    B, H, T, dk = q.shape
-    dv = v.shape[-1]
-    rows = B * H
-    seg = -(-(-(-T // CHUNK)) // nseg) * CHUNK                      # whole chunks per segment
-    bounds = list(range(0, T, seg)) + [T]
-    nseg = len(bounds) - 1
-    cu = torch.tensor(bounds, dtype=torch.int32, device=q.device)
-    fold = lambda t: None if t is None else t.reshape(1, rows, *t.shape[2:])   # batch rows become heads of a packed batch
-    q1, k1, v1, g1, beta1 = fold(q), fold(k), fold(v), fold(g), fold(_squeeze_beta(beta, 4))
-    s_ext = torch.zeros(nseg, rows, dk, dv + dk, dtype=torch.float32, device=q.device)
-    s_ext[..., dv:] = torch.eye(dk, dtype=torch.float32, device=q.device)
-    _, ab = _chunk_forward(q1, k1, v1, g1, beta1, s_ext, scale, l2norm, o_dtype, cu, forward_only=True,
-                                 dv_total=dv + dk, want_o=False)  # v's columns followed by dk zero columns
-    del s_ext
-    Bs, As = ab[..., :dv], ab[..., dv:]
-    s_in = torch.empty(nseg, rows, dk, dv, dtype=torch.float32, device=q.device)
-    cur = torch.zeros(rows, dk, dv, dtype=torch.float32, device=q.device) if initial_state is None \
-        else _f32(initial_state).reshape(rows, dk, dv)
-    for i in range(nseg):
-        s_in[i] = cur
-        if i + 1 < nseg:
-            cur = torch.baddbmm(Bs[i], As[i], cur)
-    o, sT = _chunk_forward(q1, k1, v1, g1, beta1, s_in, scale, l2norm, o_dtype, cu, forward_only=True)
-    return o.reshape(B, H, T, dv), sT[nseg - 1].reshape(B, H, dk, dv)
+    return _lib.host().chunk_segmented(q, k, v, g, _squeeze_beta(beta, 4), initial_state, scale, l2norm, _DT[o_dtype], nseg)
 
 
 def _chunk(q, k, v, g, beta, scale, initial_state, chunk_size, l2norm, o_dtype, need_mult16, cu_seqlens):
