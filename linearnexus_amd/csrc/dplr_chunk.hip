@@ -23,7 +23,7 @@
 // Kernels, each a workgroup per chunk but for the two sequential passes.  Measured at B8 H16 T4096 bf16 (8192 chunks):
 // see the table at the launch functions.
 #include "lnx_common.h"
-#include "mma_tiles.h"
+#include "chunk_common.h"
 
 namespace {
 
@@ -73,42 +73,12 @@ __device__ __forceinline__ float exp_f(float x) {
   return __builtin_amdgcn_exp2f(t) * (1.f + 0.69314718f * e);
 }
 
-// Eight consecutive elements as loaded
-template <typename T> struct Raw8;
-template <> struct Raw8<bf16_t> {
-  bf16x8 x;
-  __device__ __forceinline__ void load(const bf16_t* p, bool ok) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = (bf16_t)0.f;
-    if (ok) x = *reinterpret_cast<const bf16x8*>(p);
-  }
-  __device__ __forceinline__ float get(int i) const { return (float)x[i]; }
-};
-template <> struct Raw8<float> {
-  floatx4 x[2];
-  __device__ __forceinline__ void load(const float* p, bool ok) {
-    x[0] = x[1] = floatx4{0.f, 0.f, 0.f, 0.f};
-    if (ok) x[0] = load4(p), x[1] = load4(p + 4);
-  }
-  __device__ __forceinline__ float get(int i) const { return x[i >> 2][i & 3]; }
-};
-
-__device__ __forceinline__ void put8(float* p, const float (&v)[8]) {
-  store4(p, floatx4{v[0], v[1], v[2], v[3]});
-  store4(p + 4, floatx4{v[4], v[5], v[6], v[7]});
-}
-template <typename R> __device__ __forceinline__ void put8(float* p, const R& r) {
-  float v[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = r.get(i);
-  put8(p, v);
-}
-
-// ---- products of 16 x 16 tiles, operands in LDS --------------------------------------------------------------
+// ---- products of 16 x 16 tiles ------------------------------------------------------------------------------------
 // Result fragment: r-th element = row i0 + 4 g + r, column j0 + l16 (g = lane / 16, l16 = lane % 16).  The contraction
 // index of step r inside a block of 16 is 4 g + r in both operands, so an operand stored with the contraction along its
 // rows (ROW) is read as one 16-byte vector per block, the other way round as four single reads of 16 consecutive columns;
-// with rows 68 floats apart both touch every bank once.
+// with rows 68 floats apart both touch every bank once.  A result fragment is itself an operand whose contraction index is the
+// result's row -- with the result's column as its row or its column --, and so are four consecutive elements of a row per lane.
 template <bool ROW> __device__ __forceinline__ floatx4 frag(const float* t, int i, int k) {
   if (ROW) return load4(t + i * LD + k);
   return floatx4{t[k * LD + i], t[(k + 1) * LD + i], t[(k + 2) * LD + i], t[(k + 3) * LD + i]};
@@ -117,52 +87,86 @@ __device__ __forceinline__ void mfma4(floatx4& c, floatx4 a, floatx4 b) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
 }
-// c += A[rows i0..][k] B[k][columns j0..] over the blocks kb0 <= kb < kb1 of 16
-template <bool AR, bool BR>
-__device__ __forceinline__ void mm(floatx4& c, const float* A, int i0, const float* B, int j0, int kb0, int kb1, int l16, int g) {
-  for (int kb = kb0; kb < kb1; ++kb) mfma4(c, frag<AR>(A, i0 + l16, 16 * kb + 4 * g), frag<BR>(B, j0 + l16, 16 * kb + 4 * g));
-}
-// the same for two column tiles over one range
-template <bool AR, bool BR>
-__device__ __forceinline__ void mm2(floatx4 (&c)[2], const float* A, int i0, const float* B, int j0, int j1, int kb0, int kb1, int l16, int g) {
-  for (int kb = kb0; kb < kb1; ++kb) {
-    const floatx4 a = frag<AR>(A, i0 + l16, 16 * kb + 4 * g);
-    const floatx4 b0 = frag<BR>(B, j0 + l16, 16 * kb + 4 * g), b1 = frag<BR>(B, j1 + l16, 16 * kb + 4 * g);
-    mfma4(c[0], a, b0);
-    mfma4(c[1], a, b1);
-  }
-}
-template <bool AR, bool BR>
-__device__ __forceinline__ void mm2_full(floatx4 (&c)[2], const float* A, int i0, const float* B, int j0, int j1, int l16, int g) {
-#pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
-    const floatx4 a = frag<AR>(A, i0 + l16, 16 * kb + 4 * g);
-    const floatx4 b0 = frag<BR>(B, j0 + l16, 16 * kb + 4 * g), b1 = frag<BR>(B, j1 + l16, 16 * kb + 4 * g);
-    mfma4(c[0], a, b0);
-    mfma4(c[1], a, b1);
-  }
-}
-__device__ __forceinline__ void put_frag(float* t, int i0, int j0, floatx4 c, int l16, int g) {  // [row][column]
-#pragma unroll
-  for (int r = 0; r < 4; ++r) t[(i0 + 4 * g + r) * LD + j0 + l16] = c[r];
-}
 __device__ __forceinline__ floatx4 zero4() { return floatx4{0.f, 0.f, 0.f, 0.f}; }
 
-// Eight waves on the 4 x 4 tiles of a 64 x 64 result, two tiles each.  `row`: the wave's row block for results whose
-// contraction is cut by the row (waves w and w + 4, which share a SIMD, take complementary ones), columns c0, c1; `rowT`,
-// t0, t1: the same for results whose contraction is cut by the column.
-struct Role {
-  int wave, lane, l16, g, row, c0, c1, rowT, t0, t1;
-  __device__ __forceinline__ Role() {
-    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    lane = threadIdx.x & 63;
-    l16 = lane & 15, g = lane >> 4;
-    row = 16 * (wave < 4 ? wave : 7 - wave);
-    c0 = wave < 4 ? 0 : 32, c1 = c0 + 16;
-    rowT = 16 * (wave & 3);
-    t0 = wave < 4 ? 0 : 16, t1 = 48 - t0;
+// Four waves, each with a block of 16 tokens (of rows of the state tiles); the lane's token is t, its channels in block cb
+// are 16 cb + 4 g + 0..3.  Sums over earlier tokens make blocks 0 .. j work, sums over later ones j .. 3: the workgroups that
+// share a CU (256 apart at the start) take the blocks in opposite order.
+struct Lane {
+  int j, l16, g, t;
+  __device__ __forceinline__ Lane() {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    j = (blockIdx.x >> 8) & 1 ? 3 - wave : wave;
+    l16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    t = 16 * j + l16;
   }
 };
+
+// Blocks 0 .. j, or 3 .. j, as constants: the accumulators stay where they are when a wave leaves early (a branch around each
+// block's products made the compiler copy them, 1000 moves among 850 products)
+template <int B> struct Int {
+  static constexpr int value = B;
+};
+template <typename F> __device__ __forceinline__ void upto(int j, F&& f) {
+  f(Int<0>{});
+  if (j == 0) return;
+  f(Int<1>{});
+  if (j == 1) return;
+  f(Int<2>{});
+  if (j == 2) return;
+  f(Int<3>{});
+}
+template <typename F> __device__ __forceinline__ void downto(int j, F&& f) {
+  f(Int<3>{});
+  if (j == 3) return;
+  f(Int<2>{});
+  if (j == 2) return;
+  f(Int<1>{});
+  if (j == 1) return;
+  f(Int<0>{});
+}
+
+// Four consecutive elements as loaded
+template <typename T> struct Raw4;
+template <> struct Raw4<bf16_t> {
+  bf16x4 x;
+  __device__ __forceinline__ void load(const bf16_t* p) { x = *reinterpret_cast<const bf16x4*>(p); }
+  __device__ __forceinline__ floatx4 get() const { return floatx4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]}; }
+};
+template <> struct Raw4<float> {
+  floatx4 x;
+  __device__ __forceinline__ void load(const float* p) { x = load4(p); }
+  __device__ __forceinline__ floatx4 get() const { return x; }
+};
+// This lane's share of a row of 64, zeros where there is no such token (no load behind a branch: `base` is readable anyway)
+template <typename T> struct Row {
+  Raw4<T> x[4];
+  bool ok;
+  __device__ __forceinline__ void load(const void* base, int64_t at, bool ok_ = true) {  // at: element of the lane's first channel
+    ok = ok_;
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) x[cb].load(static_cast<const T*>(base) + (ok ? at + 16 * cb : 0));
+  }
+  __device__ __forceinline__ floatx4 operator[](int cb) const { return ok ? x[cb].get() : zero4(); }
+};
+// ... into its row of a tile
+template <typename F> __device__ __forceinline__ void put_row(float* tile, const Lane& w, F&& value) {
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) store4(tile + w.t * LD + 16 * cb + 4 * w.g, value(cb));
+}
+// A result whose columns are the wave's tokens (column l16, rows 16 nb + 4 g ..) into rows = tokens
+__device__ __forceinline__ void put_cols(float* tile, const Lane& w, const floatx4 (&c)[4]) {
+  put_row(tile, w, [&](int cb) { return c[cb]; });
+}
+// A result whose rows are the wave's tokens (rows 4 g .., column 16 nb + l16) into rows = columns
+__device__ __forceinline__ void put_rows(float* tile, const Lane& w, const floatx4 (&c)[4]) {
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) store4(tile + (16 * nb + w.l16) * LD + 16 * w.j + 4 * w.g, c[nb]);
+}
+__device__ __forceinline__ void clear(floatx4 (&c)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c[i] = zero4();
+}
 
 // ---- decays --------------------------------------------------------------------------------------------------
 struct Gates {      // arrays of 64 floats in LDS
@@ -170,30 +174,30 @@ struct Gates {      // arrays of 64 floats in LDS
   int* wide;                 // some channel's range is too wide for the split: pairs one by one, em = ec = 1
 };
 
-// Gt: gk of the chunk on entry ([t][c], visible after the first barrier), its cumulative sum on return; scr: 1536 floats
+// Gt: gk of the chunk on entry ([t][c], visible after the first barrier), its cumulative sum on return; scr: 768 floats
 __device__ __forceinline__ void cumulate(float* Gt, float* scr, const Gates& s) {
   const int tid = threadIdx.x, c = tid & 63, seg = tid >> 6;
   lds_barrier();
-  float v[8], sum = 0.f;
+  float v[16], sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = (sum += Gt[(8 * seg + i) * LD + c]);
+  for (int i = 0; i < 16; ++i) v[i] = (sum += Gt[(16 * seg + i) * LD + c]);
   scr[64 * seg + c] = sum;
   lds_barrier();
   float pre = 0.f;
   for (int j = 0; j < seg; ++j) pre += scr[64 * j + c];
   float mx = 0.f, mn = 0.f;  // the token before the chunk has G = 0
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < 16; ++i) {
     const float x = pre + v[i];
-    Gt[(8 * seg + i) * LD + c] = x;
+    Gt[(16 * seg + i) * LD + c] = x;
     mx = fmaxf(mx, x), mn = fminf(mn, x);
   }
-  scr[512 + 64 * seg + c] = mx;
-  scr[1024 + 64 * seg + c] = mn;
+  scr[256 + 64 * seg + c] = mx;
+  scr[512 + 64 * seg + c] = mn;
   lds_barrier();
   if (seg == 0) {
 #pragma unroll
-    for (int j = 1; j < 8; ++j) mx = fmaxf(mx, scr[512 + 64 * j + c]), mn = fminf(mn, scr[1024 + 64 * j + c]);
+    for (int j = 1; j < 4; ++j) mx = fmaxf(mx, scr[256 + 64 * j + c]), mn = fminf(mn, scr[512 + 64 * j + c]);
     const bool wide = __ballot(!(mx - mn <= RANGE)) != 0;
     const float m = 0.5f * (mx + mn), last = Gt[(C - 1) * LD + c];
     s.gm[c] = m;
@@ -205,120 +209,113 @@ __device__ __forceinline__ void cumulate(float* Gt, float* scr, const Gates& s) 
   lds_barrier();
 }
 
-// The chunk's vectors with their factors (q also times scale) -- plain where the chunk is wide
-template <typename T> struct Vectors {
-  Raw8<T> q, k, a, b;
-  Raw8<float> g;
-  __device__ __forceinline__ void load(const ChunkParams& p, const Slot& s) {
-    const int t = threadIdx.x >> 3, c = (threadIdx.x & 7) * 8;
-    const bool ok = t < s.len;
-    const int64_t at = (s.tok + t) * D + c;
-    g.load(p.gk + at, ok);
-    q.load(static_cast<const T*>(p.q) + at, ok);
-    a.load(static_cast<const T*>(p.a) + at, ok);
-    b.load(static_cast<const T*>(p.b) + at, ok);
-    k.load(static_cast<const T*>(p.k) + at, ok);
+__device__ __forceinline__ floatx4 rcp4(floatx4 x) {  // of e^x, |x| <= RANGE / 2
+  return floatx4{__builtin_amdgcn_rcpf(x[0]), __builtin_amdgcn_rcpf(x[1]), __builtin_amdgcn_rcpf(x[2]), __builtin_amdgcn_rcpf(x[3])};
+}
+__device__ __forceinline__ floatx4 exp4(floatx4 x) { return floatx4{exp_f(x[0]), exp_f(x[1]), exp_f(x[2]), exp_f(x[3])}; }
+
+// The lane's row of q, k, a, b and of the cumulative gate
+template <typename T> struct Own {
+  Row<T> q, k, a, b;
+  floatx4 G[4];
+  __device__ __forceinline__ void load(const ChunkParams& p, const Slot& s, const Lane& w, float* Gt) {
+    const bool ok = w.t < s.len;
+    const int64_t at = (s.tok + w.t) * D + 4 * w.g;
+    Row<float> g;
+    g.load(p.gk, at, ok);
+    q.load(p.q, at, ok);
+    a.load(p.a, at, ok);
+    b.load(p.b, at, ok);
+    k.load(p.k, at, ok);
+    put_row(Gt, w, [&](int cb) { return g[cb]; });
   }
-  __device__ __forceinline__ void store(float* tq, float* ta, float* tb, float* tk, const float* Gt, const Gates& s, float scale) const {
-    const int t = threadIdx.x >> 3, c = (threadIdx.x & 7) * 8, at = t * LD + c;
-    float vq[8], va[8], vb[8], vk[8];
-    if (*s.wide) {
+  __device__ __forceinline__ void gates(const float* Gt, const Lane& w) {  // Gt: the cumulative sums
 #pragma unroll
-      for (int i = 0; i < 8; ++i) vq[i] = scale * q.get(i), va[i] = a.get(i), vb[i] = b.get(i), vk[i] = k.get(i);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float m = s.gm[c + i], G = Gt[at + i], Gp = t ? Gt[at - LD + i] : 0.f;
-        const float eb = exp_f(m - G);
-        vq[i] = scale * q.get(i) * exp_f(G - m);
-        va[i] = a.get(i) * exp_f(Gp - m);
-        vb[i] = b.get(i) * eb;
-        vk[i] = k.get(i) * eb;
-      }
+    for (int cb = 0; cb < 4; ++cb) {
+      G[cb] = load4(Gt + w.t * LD + 16 * cb + 4 * w.g);
     }
-    put8(tq + at, vq);
-    put8(ta + at, va);
-    put8(tb + at, vb);
-    put8(tk + at, vk);
   }
 };
-
-// Wide chunk: the tiles' plain vectors become q e^G, a e^Gp, b e^(G_C - G), k e^(G_C - G) (no factor of either sign left over)
-__device__ __forceinline__ void rescale_wide(float* tq, float* ta, float* tb, float* tk, const float* Gt) {
-  const int t = threadIdx.x >> 3, c = (threadIdx.x & 7) * 8, at = t * LD + c;
+// e^(G - m), e^(Gp - m) and e^(m - G), or e^G, e^Gp and e^(G_C - G) in a wide chunk, of the lane's channels
+struct Decay {
+  floatx4 q[4], a[4], b[4];
+  __device__ __forceinline__ Decay(const floatx4 (&G)[4], const floatx4 (&Gp)[4], const float* last, const Gates& s, const Lane& w, bool wide) {
+    if (!wide) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float G = Gt[at + i], Gp = t ? Gt[at - LD + i] : 0.f, eb = exp_f(Gt[(C - 1) * LD + c + i] - G);
-    tq[at + i] *= exp_f(G);
-    ta[at + i] *= exp_f(Gp);
-    tb[at + i] *= eb;
-    tk[at + i] *= eb;
+      for (int cb = 0; cb < 4; ++cb) {
+        const floatx4 m = load4(s.gm + 16 * cb + 4 * w.g);
+        q[cb] = exp4(G[cb] - m), a[cb] = exp4(Gp[cb] - m), b[cb] = rcp4(q[cb]);
+      }
+    } else {
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) q[cb] = exp4(G[cb]), a[cb] = exp4(Gp[cb]), b[cb] = exp4(load4(last + 16 * cb + 4 * w.g) - G[cb]);
+    }
+  }
+};
+__device__ __forceinline__ void gates_before(floatx4 (&Gp)[4], const float* Gt, const Lane& w) {  // of the token before the lane's
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const floatx4 x = load4(Gt + max(w.t - 1, 0) * LD + 16 * cb + 4 * w.g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) Gp[cb][e] = w.t ? x[e] : 0.f;
   }
 }
 
-// -Aab, Pqb, Pqk, Aak into their tiles, zeros above the diagonal.  The tiles of a wide chunk hold the plain vectors.
-__device__ __forceinline__ void pair_matrices(const float* tq, const float* ta, const float* tb, const float* tk, const float* Gt, bool wide, const Role& w,
-                                              float* nAab, float* Pqb, float* Pqk, float* Aak) {
-  if (!wide) {
-    floatx4 ab[2], ak[2], qb[2], qk[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) ab[j] = ak[j] = qb[j] = qk[j] = zero4();
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = j ? w.c1 : w.c0;
-      if (col > w.row) continue;
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const int k = 16 * kb + 4 * w.g;
-        const floatx4 fa = frag<true>(ta, w.row + w.l16, k), fq = frag<true>(tq, w.row + w.l16, k);
-        const floatx4 fb = frag<true>(tb, col + w.l16, k), fk = frag<true>(tk, col + w.l16, k);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {  // four accumulators in turn: no product waits for the one before it
-          ab[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[r], fb[r], ab[j], 0, 0, 0);
-          ak[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[r], fk[r], ak[j], 0, 0, 0);
-          qb[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fq[r], fb[r], qb[j], 0, 0, 0);
-          qk[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fq[r], fk[r], qk[j], 0, 0, 0);
-        }
-      }
+// Wide chunk: the pair (t, s) of Aab, Aak, Pqb, Pqk from the difference of the gates, the vectors from memory
+struct Pair {
+  float ab, ak, qb, qk;
+};
+template <typename T> __device__ __forceinline__ Pair wide_pair(const ChunkParams& p, int64_t tok, int len, const float* Gt, int t, int s) {
+  Pair r{0.f, 0.f, 0.f, 0.f};
+  if (s > t || t >= len) return r;
+  const T *q = static_cast<const T*>(p.q) + (tok + t) * D, *a = static_cast<const T*>(p.a) + (tok + t) * D;
+  const T *b = static_cast<const T*>(p.b) + (tok + s) * D, *k = static_cast<const T*>(p.k) + (tok + s) * D;
+  for (int c = 0; c < D; ++c) {
+    const float G = Gt[s * LD + c], eq = p.scale * to_f32(q[c]) * exp_f(Gt[t * LD + c] - G), vb = to_f32(b[c]), vk = to_f32(k[c]);
+    r.qb += eq * vb;
+    r.qk += eq * vk;
+    if (s < t) {
+      const float ea = to_f32(a[c]) * exp_f(Gt[(t - 1) * LD + c] - G);
+      r.ab += ea * vb;
+      r.ak += ea * vk;
     }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = (j ? w.c1 : w.c0) + w.l16;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = w.row + 4 * w.g + r;
-        nAab[t * LD + col] = col < t ? -ab[j][r] : 0.f;
-        Aak[t * LD + col] = col < t ? ak[j][r] : 0.f;
-        Pqb[t * LD + col] = col <= t ? qb[j][r] : 0.f;
-        Pqk[t * LD + col] = col <= t ? qk[j][r] : 0.f;
-      }
-    }
-    return;
   }
-  const int t = threadIdx.x >> 3;
-  for (int s = threadIdx.x & 7; s < C; s += 8) {
-    float ab = 0.f, ak = 0.f, qb = 0.f, qk = 0.f;
-    if (s <= t) {
-      for (int c = 0; c < D; ++c) {
-        const float G = Gt[s * LD + c], eq = exp_f(Gt[t * LD + c] - G);
-        qb += tq[t * LD + c] * eq * tb[s * LD + c];
-        qk += tq[t * LD + c] * eq * tk[s * LD + c];
-        if (s < t) {
-          const float ea = exp_f(Gt[(t - 1) * LD + c] - G);
-          ab += ta[t * LD + c] * ea * tb[s * LD + c];
-          ak += ta[t * LD + c] * ea * tk[s * LD + c];
-        }
-      }
+  return r;
+}
+
+// What `pair(o, x)` gives of the lane's pairs with tokens o = 16 b + 4 g + r, through the lane's own places of N tiles
+template <int N, typename F> __device__ __forceinline__ void wide_pairs(floatx4 (*const (&m)[N])[4], float* const (&tile)[N], const Lane& w, F&& pair) {
+#pragma unroll 1
+  for (int e = 0; e < 16; ++e) {
+    const int o = 16 * (e >> 2) + 4 * w.g + (e & 3);
+    float x[N];
+    pair(o, x);
+#pragma unroll
+    for (int i = 0; i < N; ++i) tile[i][w.t * LD + o] = x[i];
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) (*m[i])[b] = load4(tile[i] + w.t * LD + 16 * b + 4 * w.g);
+}
+
+// Blocks of a lower-triangular pair matrix M[t][s].  `ByT`: tile sb <= j holds rows s, columns t = the wave's tokens; ByS: tile
+// tb >= j rows t, columns s = the wave's tokens.  Entries above the diagonal (STRICT: on it, too) are cleared.
+template <bool BY_T, bool STRICT> __device__ __forceinline__ void mask(floatx4 (&m)[4], const Lane& w) {
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const bool diagonal = b == w.j;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 4 * w.g + r, t = BY_T ? w.l16 : row, s = BY_T ? row : w.l16;
+      m[b][r] = (diagonal && (STRICT ? s >= t : s > t)) ? 0.f : m[b][r];
     }
-    nAab[t * LD + s] = -ab;
-    Aak[t * LD + s] = ak;
-    Pqb[t * LD + s] = qb;
-    Pqk[t * LD + s] = qk;
   }
 }
 
-constexpr int LDS_TILES = 9;
+constexpr int LDS_TILES = 4;
 constexpr unsigned LDS_BYTES = (LDS_TILES * TS + 4 * 64 + 4 + 32 * 36) * sizeof(float);
+static_assert(LDS_BYTES <= 80 * 1024, "two workgroups per CU");
 struct Lds {
   float* base;
   Gates gate;
@@ -334,166 +331,214 @@ struct Lds {
 
 // ---- forward: M, X, N^T, Y of a chunk ------------------------------------------------------------------------
 template <typename T>
-__global__ __launch_bounds__(512) void dplr_prepare_kernel(ChunkParams p) {
+__global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
   extern __shared__ __align__(16) char smem[];
   const Lds L(smem);
   const Slot s = slot_of(p);
-  const Role w;
-  float *tq = L.tile(0), *ta = L.tile(1), *tb = L.tile(2), *tk = L.tile(3), *Tm = L.tile(4), *Pqb = L.tile(5), *Pqk = L.tile(6), *Aak = L.tile(7), *tv = L.tile(8);
-  const int t = threadIdx.x >> 3, c8 = (threadIdx.x & 7) * 8;
-  Vectors<T> x;
-  x.load(p, s);
-  Raw8<T> v;
-  v.load(static_cast<const T*>(p.v) + (s.tok + t) * D + c8, t < s.len);
-  put8(tv + t * LD + c8, x.g);  // G until the pairs are done
-  cumulate(tv, Pqb, L.gate);
-  x.store(tq, ta, tb, tk, tv, L.gate, p.scale);
-  lds_barrier();
+  const Lane w;
+  const int l16 = w.l16, g = w.g, g4 = 4 * w.g;
+  float *tb = L.tile(0), *tk = L.tile(1), *ta = L.tile(2), *tx = L.tile(3);
+  Own<T> x;
+  x.load(p, s, w, tx);
+  Row<T> v;
+  v.load(p.v, (s.tok + w.t) * D + g4, w.t < s.len);
+  cumulate(tx, L.sx, L.gate);
+  x.gates(tx, w);
   const bool wide = *L.gate.wide;
-  pair_matrices(tq, ta, tb, tk, tv, wide, w, Tm, Pqb, Pqk, Aak);
-  lds_barrier();
-  if (wide) {
-    rescale_wide(tq, ta, tb, tk, tv);
-    lds_barrier();
-  }
-  put8(tv + t * LD + c8, v);
-  lds_barrier();
-  floatx4 z[2] = {zero4(), zero4()};
-  mm2<true, false>(z, Aak, w.row, tv, w.c0, w.c1, 0, w.row / 16 + 1, w.l16, w.g);  // Aak v
-  tri_inverse_64<true, 512>(Tm, Tm, L.sx, threadIdx.x);
-  put_frag(Aak, w.row, w.c0, z[0], w.l16, w.g);  // every wave has passed a barrier since its last read of Aak
-  put_frag(Aak, w.row, w.c1, z[1], w.l16, w.g);
-  lds_barrier();
-  floatx4 W[2] = {zero4(), zero4()}, u[2] = {zero4(), zero4()};
-  mm2<true, false>(W, Tm, w.row, ta, w.c0, w.c1, 0, w.row / 16 + 1, w.l16, w.g);
-  mm2<true, false>(u, Tm, w.row, Aak, w.c0, w.c1, 0, w.row / 16 + 1, w.l16, w.g);
-  lds_barrier();
-  float *tW = ta, *tU = Aak;
-  put_frag(tW, w.row, w.c0, W[0], w.l16, w.g);
-  put_frag(tW, w.row, w.c1, W[1], w.l16, w.g);
-  put_frag(tU, w.row, w.c0, u[0], w.l16, w.g);
-  put_frag(tU, w.row, w.c1, u[1], w.l16, w.g);
-  lds_barrier();
-  // Results as [column][4 consecutive rows]: 16-byte stores
-  const int i0 = w.rowT, ch = i0 + 4 * w.g;  // this lane's four channels (of M's columns, X's columns, N^T's columns, Y's)
+  floatx4 xx[4];  // q with its factor, then X^T: rows = channels, columns = tokens
+  floatx4 ab[4], ak[4], qb[4], qk[4];
+  clear(ab), clear(ak), clear(qb), clear(qk);
   {
-    floatx4 m[2] = {zero4(), zero4()}, nt[2] = {zero4(), zero4()};
-    mm2_full<false, false>(m, tW, i0, tb, w.t0, w.t1, w.l16, w.g);    // M[i][c] at rows c, columns i
-    mm2_full<false, false>(nt, tb, i0, tU, w.t0, w.t1, w.l16, w.g);   // N[i][n] at rows i, columns n
-    mm2_full<false, false>(nt, tk, i0, tv, w.t0, w.t1, w.l16, w.g);
-    const floatx4 em = load4(L.gate.em + ch), ec4 = load4(L.gate.ec + ch);
+    floatx4 fa[4], fb[4], fk[4];
+    {
+      floatx4 Gp[4];
+      gates_before(Gp, tx, w);
+      const Decay e(x.G, Gp, tx + (C - 1) * LD, L.gate, w, wide);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = (j ? w.t1 : w.t0) + w.l16;
-      floatx4 r = m[j] * em * L.gate.ec[col];
+      for (int cb = 0; cb < 4; ++cb) xx[cb] = p.scale * x.q[cb] * e.q[cb], fa[cb] = x.a[cb] * e.a[cb], fb[cb] = x.b[cb] * e.b[cb], fk[cb] = x.k[cb] * e.b[cb];
+    }
+    if (wide) {
+      wide_pairs<2>({&ab, &ak}, {tb, tk}, w, [&](int o, float* r) { const Pair y = wide_pair<T>(p, s.tok, s.len, tx, w.t, o); r[0] = y.ab, r[1] = y.ak; });
+      wide_pairs<2>({&qb, &qk}, {tb, tk}, w, [&](int o, float* r) { const Pair y = wide_pair<T>(p, s.tok, s.len, tx, w.t, o); r[0] = y.qb, r[1] = y.qk; });
+    }
+    put_cols(ta, w, fa), put_cols(tb, w, fb), put_cols(tk, w, fk);
+    lds_barrier();
+    if (!wide) {
+      upto(w.j, [&](auto sb_) {
+        constexpr int sb = decltype(sb_)::value;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (ch + e == col) r[e] += L.gate.eC[col];
-      store4(p.M + s.kept * TG + col * D + ch, r);
-      store4(p.s1 + s.win * TG + col * D + ch, nt[j] * ec4);
+        for (int kb = 0; kb < 4; ++kb) {
+          const floatx4 rb = frag<true>(tb, 16 * sb + l16, 16 * kb + g4), rk = frag<true>(tk, 16 * sb + l16, 16 * kb + g4);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {  // four accumulators in turn: no product waits for the one before it
+            ab[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb[r], fa[kb][r], ab[sb], 0, 0, 0);
+            ak[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(rk[r], fa[kb][r], ak[sb], 0, 0, 0);
+            qb[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb[r], xx[kb][r], qb[sb], 0, 0, 0);
+            qk[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(rk[r], xx[kb][r], qk[sb], 0, 0, 0);
+          }
+        }
+      });
+      mask<true, true>(ab, w), mask<true, true>(ak, w), mask<true, false>(qb, w), mask<true, false>(qk, w);
     }
   }
+  lds_barrier();  // the gates have been read
+  put_row(tx, w, [&](int cb) { return v[cb]; });
+  lds_barrier();
+  floatx4 nt[4], z[4], y[4];  // N (rows i, columns n), Aak v (rows t, columns n), Y^T (rows n, columns t)
+  clear(nt), clear(z), clear(y);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int col = j ? w.t1 : w.t0, tt = col + w.l16;  // this lane's token
-    floatx4 xx = zero4(), y = zero4();
-    mm<false, true>(xx, tW, i0, Pqb, col, 0, col / 16 + 1, w.l16, w.g);
-    mm<false, true>(y, tU, i0, Pqb, col, 0, col / 16 + 1, w.l16, w.g);
-    mm<false, true>(y, tv, i0, Pqk, col, 0, col / 16 + 1, w.l16, w.g);
-    store4(p.X + s.kept * TG + tt * D + ch, (xx + load4(tq + tt * LD + ch)) * load4(L.gate.em + ch));
-    store4(p.s2 + s.win * TG + tt * D + ch, y);
+  for (int sb = 0; sb < 4; ++sb) {
+    const floatx4 kf = frag<false>(tk, 16 * w.j + l16, 16 * sb + g4);
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) mfma4(nt[nb], kf, frag<false>(tx, 16 * nb + l16, 16 * sb + g4));
+  }
+  upto(w.j, [&](auto sb_) {
+    constexpr int sb = decltype(sb_)::value;
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+      const floatx4 vf = frag<false>(tx, 16 * nb + l16, 16 * sb + g4);
+      mfma4(z[nb], ak[sb], vf);
+      mfma4(y[nb], vf, qk[sb]);
+    }
+  });
+  lds_barrier();
+#pragma unroll
+  for (int sb = 0; sb < 4; ++sb) store4(tx + w.t * LD + 16 * sb + g4, sb <= w.j ? -ab[sb] : zero4());
+  put_rows(tk, w, z);
+  lds_barrier();
+  tri_inverse_64<true>(tx, tx, L.sx, threadIdx.x);
+  {
+    floatx4 W[4], u[4];
+    clear(W), clear(u);
+    upto(w.j, [&](auto sb_) {
+      constexpr int sb = decltype(sb_)::value;
+      const floatx4 tf = frag<true>(tx, w.t, 16 * sb + g4);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) {
+        mfma4(W[cb], tf, frag<false>(ta, 16 * cb + l16, 16 * sb + g4));
+        mfma4(u[cb], tf, frag<true>(tk, 16 * cb + l16, 16 * sb + g4));
+      }
+    });
+    lds_barrier();
+    put_rows(ta, w, W);
+    put_rows(tk, w, u);
+  }
+  lds_barrier();
+  floatx4 m[4];  // M[i][c]: rows c, columns i
+  clear(m);
+#pragma unroll
+  for (int sb = 0; sb < 4; ++sb) {
+    const floatx4 bf = frag<false>(tb, 16 * w.j + l16, 16 * sb + g4);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) {
+      const floatx4 wf = frag<true>(ta, 16 * cb + l16, 16 * sb + g4), uf = frag<true>(tk, 16 * cb + l16, 16 * sb + g4);
+      mfma4(m[cb], wf, bf);
+      mfma4(nt[cb], bf, uf);
+    }
+  }
+  upto(w.j, [&](auto sb_) {
+    constexpr int sb = decltype(sb_)::value;
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) {
+      mfma4(xx[cb], frag<true>(ta, 16 * cb + l16, 16 * sb + g4), qb[sb]);
+      mfma4(y[cb], frag<true>(tk, 16 * cb + l16, 16 * sb + g4), qb[sb]);
+    }
+  });
+  const float eci = L.gate.ec[w.t], eCi = L.gate.eC[w.t];
+  const floatx4 ec4 = load4(L.gate.ec + 16 * w.j + g4);
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const floatx4 em = load4(L.gate.em + 16 * cb + g4);
+    floatx4 r = m[cb] * em * eci;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (16 * cb + g4 + e == w.t) r[e] += eCi;
+    const int at = w.t * D + 16 * cb + g4;
+    store4(p.M + s.kept * TG + at, r);
+    store4(p.X + s.kept * TG + at, xx[cb] * em);
+    store4(p.s2 + s.win * TG + at, y[cb]);
+    store4(p.s1 + s.win * TG + (16 * cb + l16) * D + 16 * w.j + g4, nt[cb] * ec4);
   }
 }
 
 // ---- the sequential pass: h <- M h + N (forward), D <- M^T D + R (backward) ------------------------------------
-// One workgroup per row; wave w owns 16 of the 64 value columns, whose part of the state stays in four accumulator
-// fragments: an accumulator fragment is the B operand of the next product as it stands (its rows 16 b + 4 g + r are the
-// contraction indices that step r of block b wants in lane group g), so the state never leaves the wave.  M arrives
-// through registers two chunks ahead and one LDS tile ahead; one LDS barrier per chunk.  64 products of 32 cycles on the
-// chain of a chunk, 0.9 us.
+// One workgroup per row and 16 of the 64 value columns; wave w forms 16 rows of the new state, sixteen products of 32 cycles, from its
+// rows of M, which come straight into its registers three chunks ahead, and the old state, which the waves exchange
+// through LDS (transposed), one LDS barrier per chunk.  A whole chain on one wave per 16 columns took four times the products and
+// M through LDS: 1.85 us per chunk.
 struct ScanParams {
   const float* M;    // kept tiles [rows][KN]
   const float* add;  // window tiles: N^T or R^T
   float* st;         // the state entering (forward: kept [rows][KN + 1]) or the gradient leaving (backward: window) each chunk, transposed
   const float* s_in; // [dk][dv] per row, or NULL
   float* s_out;      // [dk][dv] per row, or NULL
+  int64_t rows;
   int KN, at, nw;    // the window is chunks [at, at + nw) of the kept tensors
 };
 
 template <bool BWD>
 __global__ __launch_bounds__(256) void dplr_chunk_scan_kernel(ScanParams p) {
-  __shared__ __align__(16) float buf[2][TS];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
-  const int64_t row = blockIdx.x;
-  const int col = 16 * wave + l16;
-  const float* Mrow = p.M + (row * p.KN + p.at) * TG;
-  const float* Arow = p.add + row * p.nw * TG + col * D + 4 * g;
-  float* Srow = p.st + (BWD ? row * p.nw : row * (p.KN + 1) + p.at) * TG + col * D + 4 * g;
+  __shared__ __align__(16) float buf[2][16 * LD];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  int64_t row;
+  int part;
+  if (!xcd_slot_part(p.rows, 4, row, part)) return;  // the four parts read the same M: one XCD
+  const int col = 16 * part + l16, r0 = 16 * wave + 4 * g;  // this lane's column and its first row of the state
+  const float* Mrow = p.M + (row * p.KN + p.at) * TG + (BWD ? 4 * g * D + 16 * wave + l16 : (16 * wave + l16) * D + 4 * g);
+  const float* Arow = p.add + row * p.nw * TG + col * D + r0;
+  float* Srow = p.st + (BWD ? row * p.nw : row * (p.KN + 1) + p.at) * TG + col * D + r0;
   auto chunk = [&](int i) { return (int64_t)(BWD ? p.nw - 1 - i : i); };
-  floatx4 h[4];
+  floatx4 h;
 #pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) h[b][r] = p.s_in ? p.s_in[row * TG + (16 * b + 4 * g + r) * D + col] : 0.f;
+  for (int r = 0; r < 4; ++r) h[r] = p.s_in ? p.s_in[row * TG + (r0 + r) * D + col] : 0.f;
   struct Ahead {
-    floatx4 m[4], a[4];
-  } r0, r1;
-  const int lr = tid >> 2, lc = (tid & 3) * 4;  // this thread's row of M and its first column in each quarter
+    floatx4 m[4], a;
+  } x0, x1, x2, x3;
   auto fetch = [&](Ahead& x, int i) {
-    const int64_t n = chunk(min(i, p.nw - 1));
-#pragma unroll
-    for (int q = 0; q < 4; ++q) x.m[q] = load4(Mrow + n * TG + lr * D + 16 * q + lc);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) x.a[q] = load4(Arow + n * TG + 16 * q);
-  };
-  auto stage = [&](const Ahead& x, float* dst) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) store4(dst + lr * LD + 16 * q + lc, x.m[q]);
-  };
-  auto step = [&](const Ahead& x, const float* M, int i) {
-    floatx4 y[4];
-    float* out = Srow + chunk(i) * TG;
+    const float* M = Mrow + chunk(min(i, p.nw - 1)) * TG;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      store4(out + 16 * b, h[b]);
-      y[b] = x.a[b];
+      if (BWD) x.m[b] = floatx4{M[16 * b * D], M[(16 * b + 1) * D], M[(16 * b + 2) * D], M[(16 * b + 3) * D]};
+      else x.m[b] = load4(M + 16 * b);
     }
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {  // contraction block
-      floatx4 f[4];
-#pragma unroll
-      for (int ib = 0; ib < 4; ++ib) f[ib] = frag<!BWD>(M, 16 * ib + l16, 16 * b + 4 * g);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int ib = 0; ib < 4; ++ib) y[ib] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[ib][r], h[b][r], y[ib], 0, 0, 0);
-    }
-#pragma unroll
-    for (int b = 0; b < 4; ++b) h[b] = y[b];
+    x.a = load4(Arow + chunk(min(i, p.nw - 1)) * TG);
   };
-  fetch(r0, 0);
-  fetch(r1, 1);
-  stage(r0, buf[0]);
-  for (int i = 0; i < p.nw; i += 2) {
+  auto step = [&](Ahead& x, Ahead& next, int i) {  // next: the set that chunk i - 1 has used
     lds_barrier();
-    step(r0, buf[0], i);
-    stage(r1, buf[1]);
-    fetch(r0, i + 2);
-    if (i + 1 >= p.nw) break;
-    lds_barrier();
-    step(r1, buf[1], i + 1);
-    stage(r0, buf[0]);
-    fetch(r1, i + 3);
-  }
-  if (!BWD && p.at + p.nw == p.KN) {
+    const float* cur = buf[i & 1] + l16 * LD + 4 * g;
+    floatx4 f[4];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) store4(Srow + (int64_t)p.nw * TG + 16 * b, h[b]);
+    for (int b = 0; b < 4; ++b) f[b] = load4(cur + 16 * b);
+    fetch(next, i + 3);
+    store4(Srow + chunk(i) * TG, h);
+    floatx4 y0 = x.a, y1 = zero4();
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[2 * b][r], f[2 * b][r], y0, 0, 0, 0);
+        y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[2 * b + 1][r], f[2 * b + 1][r], y1, 0, 0, 0);
+      }
+    h = y0 + y1;
+    store4(buf[(i + 1) & 1] + l16 * LD + r0, h);
+  };
+  fetch(x0, 0);
+  fetch(x1, 1);
+  fetch(x2, 2);
+  store4(buf[0] + l16 * LD + r0, h);
+  for (int i = 0; i < p.nw; i += 4) {
+    step(x0, x3, i);
+    if (i + 1 >= p.nw) break;
+    step(x1, x0, i + 1);
+    if (i + 2 >= p.nw) break;
+    step(x2, x1, i + 2);
+    if (i + 3 >= p.nw) break;
+    step(x3, x2, i + 3);
   }
+  if (!BWD && p.at + p.nw == p.KN) store4(Srow + (int64_t)p.nw * TG, h);
   if (p.s_out) {
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) p.s_out[row * TG + (16 * b + 4 * g + r) * D + col] = h[b][r];
+    for (int r = 0; r < 4; ++r) p.s_out[row * TG + (r0 + r) * D + col] = h[r];
   }
 }
 
@@ -527,295 +572,375 @@ template <typename T>
 __global__ __launch_bounds__(256) void dplr_r_kernel(ChunkParams p) {
   __shared__ __align__(16) float tX[TS], tO[TS];
   const Slot s = slot_of(p);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int t = (threadIdx.x >> 3) + 32 * h, c = (threadIdx.x & 7) * 8;
-    Raw8<float> x;
-    Raw8<T> d;
-    x.load(p.X + s.kept * TG + t * D + c, true);
-    d.load(static_cast<const T*>(p.d_o) + (s.tok + t) * D + c, t < s.len);
-    put8(tX + t * LD + c, x);
-    put8(tO + t * LD + c, d);
-  }
+  const Lane w;
+  const int l16 = w.l16, g4 = 4 * w.g;
+  Row<float> x;
+  Row<T> d;
+  x.load(p.X, s.kept * TG + w.t * D + g4);
+  d.load(p.d_o, (s.tok + w.t) * D + g4, w.t < s.len);
+  put_row(tX, w, [&](int cb) { return x[cb]; });
+  put_row(tO, w, [&](int cb) { return d[cb]; });
   lds_barrier();
-  floatx4 acc[4] = {zero4(), zero4(), zero4(), zero4()};
+  floatx4 acc[4];
+  clear(acc);
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
-    const floatx4 a = frag<false>(tX, 16 * wave + l16, 16 * kb + 4 * g);
+    const floatx4 a = frag<false>(tX, w.t, 16 * kb + g4);
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) mfma4(acc[nb], a, frag<false>(tO, 16 * nb + l16, 16 * kb + 4 * g));
+    for (int nb = 0; nb < 4; ++nb) mfma4(acc[nb], a, frag<false>(tO, 16 * nb + l16, 16 * kb + g4));
   }
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) store4(p.s2 + s.win * TG + (16 * nb + l16) * D + 16 * wave + 4 * g, acc[nb]);
+  for (int nb = 0; nb < 4; ++nb) store4(p.s2 + s.win * TG + (16 * nb + l16) * D + 16 * w.j + g4, acc[nb]);
 }
 
 // ---- backward: u, dU and dv of a chunk -----------------------------------------------------------------------
 // The pair matrices and the inverse are formed again: keeping them would move 128 KB per chunk through memory.
 template <typename T>
-__global__ __launch_bounds__(512) void dplr_u_kernel(ChunkParams p) {
+__global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   extern __shared__ __align__(16) char smem[];
   const Lds L(smem);
   const Slot s = slot_of(p);
-  const Role w;
-  float *tq = L.tile(0), *ta = L.tile(1), *tb = L.tile(2), *tk = L.tile(3), *Tm = L.tile(4), *Pqb = L.tile(5), *Pqk = L.tile(6), *Aak = L.tile(7), *tv = L.tile(8);
-  const int t = threadIdx.x >> 3, c8 = (threadIdx.x & 7) * 8, at = t * LD + c8;
-  Vectors<T> x;
-  x.load(p, s);
-  Raw8<T> v, d_o;
-  v.load(static_cast<const T*>(p.v) + (s.tok + t) * D + c8, t < s.len);
-  d_o.load(static_cast<const T*>(p.d_o) + (s.tok + t) * D + c8, t < s.len);
-  Raw8<float> h0, dC;
-  h0.load(p.hT + s.st * TG + t * D + c8, true);
-  dC.load(p.s1 + s.win * TG + t * D + c8, true);
-  put8(tv + at, x.g);
-  cumulate(tv, Pqb, L.gate);
-  x.store(tq, ta, tb, tk, tv, L.gate, p.scale);
-  lds_barrier();
+  const Lane w;
+  const int l16 = w.l16, g4 = 4 * w.g;
+  float *tb = L.tile(0), *tk = L.tile(1), *ta = L.tile(2), *tx = L.tile(3);
+  Own<T> x;
+  x.load(p, s, w, tx);
+  Row<T> v, d_o;
+  v.load(p.v, (s.tok + w.t) * D + g4, w.t < s.len);
+  d_o.load(p.d_o, (s.tok + w.t) * D + g4, w.t < s.len);
+  Row<float> h0, dC;
+  h0.load(p.hT, s.st * TG + w.t * D + g4);
+  dC.load(p.s1, s.win * TG + w.t * D + g4);
+  cumulate(tx, L.sx, L.gate);
+  x.gates(tx, w);
   const bool wide = *L.gate.wide;
-  pair_matrices(tq, ta, tb, tk, tv, wide, w, Tm, Pqb, Pqk, Aak);
-  lds_barrier();
-  if (wide) {
-    rescale_wide(tq, ta, tb, tk, tv);
-    lds_barrier();
-  }
-  put8(tv + at, v);
+  floatx4 fa[4], fb[4], fk[4];  // the lane's row with its factors
+  floatx4 ab[4], akT[4];        // Aab, Aak by t
+  floatx4 ak[4], qb[4], qk[4];  // Aak, Pqb, Pqk by s
+  clear(ab), clear(akT), clear(ak), clear(qb), clear(qk);
   {
-    float y[8];
+    floatx4 fq[4];
+    {
+      floatx4 Gp[4];
+      gates_before(Gp, tx, w);
+      const Decay e(x.G, Gp, tx + (C - 1) * LD, L.gate, w, wide);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = h0.get(i) * L.gate.em[c8 + i];
-    put8(tq + at, y);  // e^m h, [value column][channel]; q is not needed any more
+      for (int cb = 0; cb < 4; ++cb) fq[cb] = p.scale * x.q[cb] * e.q[cb], fa[cb] = x.a[cb] * e.a[cb], fb[cb] = x.b[cb] * e.b[cb], fk[cb] = x.k[cb] * e.b[cb];
+    }
+    if (!wide) {
+      put_cols(ta, w, fa), put_cols(tb, w, fb), put_cols(tk, w, fk);
+      lds_barrier();  // the gates have been read
+      put_cols(tx, w, fq);
+      lds_barrier();
+    }
+  }
+  if (!wide) {
+    upto(w.j, [&](auto b_) {
+      constexpr int b = decltype(b_)::value;
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        const floatx4 rb = frag<true>(tb, 16 * b + l16, 16 * kb + g4), rk = frag<true>(tk, 16 * b + l16, 16 * kb + g4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          ab[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb[r], fa[kb][r], ab[b], 0, 0, 0);
+          akT[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(rk[r], fa[kb][r], akT[b], 0, 0, 0);
+        }
+      }
+    });
+    downto(w.j, [&](auto b_) {
+      constexpr int b = decltype(b_)::value;
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        const floatx4 ra = frag<true>(ta, 16 * b + l16, 16 * kb + g4), rq = frag<true>(tx, 16 * b + l16, 16 * kb + g4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          ak[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[r], fk[kb][r], ak[b], 0, 0, 0);
+          qb[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(rq[r], fb[kb][r], qb[b], 0, 0, 0);
+          qk[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(rq[r], fk[kb][r], qk[b], 0, 0, 0);
+        }
+      }
+    });
+    mask<true, true>(ab, w), mask<true, true>(akT, w), mask<false, true>(ak, w), mask<false, false>(qb, w), mask<false, false>(qk, w);
+  } else {
+    wide_pairs<2>({&ab, &akT}, {tb, tk}, w, [&](int o, float* r) { const Pair y = wide_pair<T>(p, s.tok, s.len, tx, w.t, o); r[0] = y.ab, r[1] = y.ak; });
+    wide_pairs<3>({&ak, &qb, &qk}, {tb, tk, ta}, w, [&](int o, float* r) { const Pair y = wide_pair<T>(p, s.tok, s.len, tx, o, w.t); r[0] = y.ak, r[1] = y.qb, r[2] = y.qk; });
   }
   lds_barrier();
-  floatx4 z[2] = {zero4(), zero4()};
-  mm2_full<true, true>(z, ta, w.row, tq, w.c0, w.c1, w.l16, w.g);                   // a h
-  mm2<true, false>(z, Aak, w.row, tv, w.c0, w.c1, 0, w.row / 16 + 1, w.l16, w.g);   // + Aak v
-  tri_inverse_64<true, 512>(Tm, Tm, L.sx, threadIdx.x);
-  put_frag(ta, w.row, w.c0, z[0], w.l16, w.g);
-  put_frag(ta, w.row, w.c1, z[1], w.l16, w.g);
-  put8(tv + at, d_o);
-  {
-    float y[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = dC.get(i) * L.gate.ec[c8 + i];
-    put8(tq + at, y);  // e^(G_C - m) D, [value column][channel]
-  }
+  float *th = ta, *tO = tb, *tD = tk, *tv = tx;
+  put_row(tv, w, [&](int cb) { return v[cb]; });
+  put_row(tO, w, [&](int cb) { return d_o[cb]; });
+  put_row(th, w, [&](int cb) { return h0[cb] * load4(L.gate.em + 16 * cb + g4); });  // e^m h, [value column][channel]
+  put_row(tD, w, [&](int cb) { return dC[cb] * load4(L.gate.ec + 16 * cb + g4); });  // e^(G_C - m) D, [value column][channel]
   lds_barrier();
-  // u = Tm z: rows = value columns, columns = tokens
+  floatx4 z[4], y[4], dv[4];  // a h + Aak v, Bg D + Pqb^T dO (rows t, columns n), dv (rows n, columns t)
+  clear(z), clear(y), clear(dv);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int col = j ? w.t1 : w.t0;
-    floatx4 u = zero4();
-    mm<false, true>(u, ta, w.rowT, Tm, col, 0, col / 16 + 1, w.l16, w.g);
-    store4(p.s3 + s.win * TG + (col + w.l16) * D + w.rowT + 4 * w.g, u);
-  }
-  floatx4 y[2] = {zero4(), zero4()};
-  mm2_full<true, true>(y, tb, w.row, tq, w.c0, w.c1, w.l16, w.g);                        // Bg D
-  mm2<false, false>(y, Pqb, w.row, tv, w.c0, w.c1, w.row / 16, 4, w.l16, w.g);           // + Pqb^T dO
-  floatx4 dv[2] = {zero4(), zero4()};
+  for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {  // rows = value columns, columns = tokens
-    const int col = j ? w.t1 : w.t0;
-    mm<true, true>(dv[j], tq, w.rowT, tk, col, 0, 4, w.l16, w.g);                        // Kg D
-    mm<false, false>(dv[j], tv, w.rowT, Pqk, col, col / 16, 4, w.l16, w.g);              // + Pqk^T dO
-  }
-  lds_barrier();
-  put_frag(ta, w.row, w.c0, y[0], w.l16, w.g);
-  put_frag(ta, w.row, w.c1, y[1], w.l16, w.g);
-  lds_barrier();
-  floatx4 du[2] = {zero4(), zero4()};
-  mm2<false, false>(du, Tm, w.row, ta, w.c0, w.c1, w.row / 16, 4, w.l16, w.g);
-  put_frag(tb, w.row, w.c0, du[0], w.l16, w.g);  // b was last read before two barriers
-  put_frag(tb, w.row, w.c1, du[1], w.l16, w.g);
-  lds_barrier();
+    for (int nb = 0; nb < 4; ++nb) {
+      const floatx4 hf = frag<true>(th, 16 * nb + l16, 16 * kb + g4), df = frag<true>(tD, 16 * nb + l16, 16 * kb + g4);
+      mfma4(z[nb], fa[kb], hf);
+      mfma4(y[nb], fb[kb], df);
+      mfma4(dv[nb], df, fk[kb]);
+    }
+  upto(w.j, [&](auto b_) {
+    constexpr int b = decltype(b_)::value;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int col = j ? w.t1 : w.t0, tt = col + w.l16;
-    mm<false, false>(dv[j], tb, w.rowT, Aak, col, col / 16, 4, w.l16, w.g);              // + Aak^T dU
-    if (tt < s.len) store_row4<T>(p.dv, (s.tok + tt) * D + w.rowT + 4 * w.g, dv[j]);
+    for (int nb = 0; nb < 4; ++nb) mfma4(z[nb], akT[b], frag<false>(tv, 16 * nb + l16, 16 * b + g4));
+  });
+  downto(w.j, [&](auto b_) {
+    constexpr int b = decltype(b_)::value;
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+      const floatx4 of = frag<false>(tO, 16 * nb + l16, 16 * b + g4);
+      mfma4(y[nb], qb[b], of);
+      mfma4(dv[nb], of, qk[b]);
+    }
+  });
+  lds_barrier();
+  float *Tm = tx, *tz = ta, *ty = tk, *tdu = tb;
+#pragma unroll
+  for (int sb = 0; sb < 4; ++sb) store4(Tm + w.t * LD + 16 * sb + g4, sb <= w.j ? -ab[sb] : zero4());
+  put_rows(tz, w, z);
+  put_rows(ty, w, y);
+  lds_barrier();
+  tri_inverse_64<true>(Tm, Tm, L.sx, threadIdx.x);
+  floatx4 u[4], du[4];  // rows n, columns t
+  clear(u), clear(du);
+  upto(w.j, [&](auto b_) {
+    constexpr int b = decltype(b_)::value;
+    const floatx4 tf = frag<true>(Tm, w.t, 16 * b + g4);
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) mfma4(u[nb], frag<true>(tz, 16 * nb + l16, 16 * b + g4), tf);
+  });
+  downto(w.j, [&](auto b_) {
+    constexpr int b = decltype(b_)::value;
+    const floatx4 tf = frag<false>(Tm, w.t, 16 * b + g4);
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) mfma4(du[nb], frag<true>(ty, 16 * nb + l16, 16 * b + g4), tf);
+  });
+  const int64_t wt = s.win * TG + w.t * D + g4;
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    store4(p.s3 + wt + 16 * nb, u[nb]);
+    store4(p.s4 + wt + 16 * nb, du[nb]);
   }
-  store4(p.s4 + s.win * TG + t * D + c8, load4(tb + at));
-  store4(p.s4 + s.win * TG + t * D + c8 + 4, load4(tb + at + 4));
+  put_cols(tdu, w, du);
+  lds_barrier();
+  downto(w.j, [&](auto b_) {
+    constexpr int b = decltype(b_)::value;
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) mfma4(dv[nb], frag<false>(tdu, 16 * nb + l16, 16 * b + g4), ak[b]);
+  });
+  if (w.t < s.len) {
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) store_row4<T>(p.dv, (s.tok + w.t) * D + 16 * nb + g4, dv[nb]);
+  }
 }
 
 // ---- backward: dq, dk, da, db, dgk of a chunk ----------------------------------------------------------------
+// Wide chunk: what the matrices Mb, Mk (which pair b and k with q: LAG 0, or with a, whose decay lags by its own token: LAG 1) add to
+// the gradients of the lane's token: d1 (q or a), db, dk, four channels from ch.
+template <typename T, int LAG>
+__device__ __forceinline__ void wide_grads(const ChunkParams& p, int64_t tok, int len, const float* Mb, const float* Mk, const float* Gt, int t, int ch,
+                                                     floatx4& d1, floatx4& db, floatx4& dk) {
+  auto row = [&](const void* base, int i) { Raw4<T> x; x.load(static_cast<const T*>(base) + (tok + min(i, len - 1)) * D + ch); return i < len ? x.get() : zero4(); };
+  auto gate = [&](int i) { return i < 0 ? zero4() : load4(Gt + i * LD + ch); };
+  const floatx4 G = gate(t), Gl = gate(t - LAG);
+  for (int i = 0; i <= t - LAG; ++i) d1 += exp4(Gl - gate(i)) * (Mb[t * LD + i] * row(p.b, i) + Mk[t * LD + i] * row(p.k, i));
+  for (int i = t + LAG; i < C; ++i) {
+    const floatx4 e = exp4(gate(i - LAG) - G) * (LAG ? row(p.a, i) : p.scale * row(p.q, i));
+    db += e * Mb[i * LD + t];
+    dk += e * Mk[i * LD + t];
+  }
+}
+
 template <typename T>
-__global__ __launch_bounds__(512) void dplr_grad_kernel(ChunkParams p) {
+__global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
   extern __shared__ __align__(16) char smem[];
   const Lds L(smem);
   const Slot s = slot_of(p);
-  const Role w;
-  const int tid = threadIdx.x, t = tid >> 3, c8 = (tid & 7) * 8, at = t * LD + c8;
-  float *Gt = L.tile(8), *prod = L.tile(6);
-  float* red = L.sx;  // [8][64]: partial sums of <D, h'> per channel
-  Vectors<T> x;
-  x.load(p, s);
+  const Lane w;
+  const int tid = threadIdx.x, l16 = w.l16, g4 = 4 * w.g;
+  float *t0 = L.tile(0), *t1 = L.tile(1), *t2 = L.tile(2), *t3 = L.tile(3);
+  float* red = L.sx + 768;  // [4][64]: partial sums of <D, h'> per channel
+  const int64_t at = (s.tok + w.t) * D + g4, wt = s.win * TG + w.t * D + g4, ht = s.st * TG + w.t * D + g4;
+  const bool ok = w.t < s.len;
+  Own<T> x;
+  Row<T> v, d_o;
+  Row<float> u, du;
   {
-    Raw8<T> v, d_o;
-    Raw8<float> u, du, h0, dC, hC;
-    v.load(static_cast<const T*>(p.v) + (s.tok + t) * D + c8, t < s.len);
-    d_o.load(static_cast<const T*>(p.d_o) + (s.tok + t) * D + c8, t < s.len);
-    const int64_t wt = s.win * TG + t * D + c8, ht = s.st * TG + t * D + c8;
-    u.load(p.s3 + wt, true);
-    du.load(p.s4 + wt, true);
-    h0.load(p.hT + ht, true);
-    hC.load(p.hT + ht + TG, true);
-    dC.load(p.s1 + wt, true);
-    put8(Gt + at, x.g);
-    cumulate(Gt, L.tile(7), L.gate);
-    put8(L.tile(0) + at, v);
-    put8(L.tile(1) + at, d_o);
-    put8(L.tile(2) + at, u);
-    put8(L.tile(3) + at, du);
-    float y[8], z[8], r[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      y[i] = h0.get(i) * L.gate.em[c8 + i];
-      z[i] = dC.get(i) * L.gate.ec[c8 + i];
-      r[i] = dC.get(i) * hC.get(i);
-    }
-    put8(L.tile(4) + at, y);
-    put8(L.tile(5) + at, z);
-    put8(prod + at, r);
+    Row<float> hC, dC;
+    hC.load(p.hT, ht + TG);
+    dC.load(p.s1, wt);
+    x.load(p, s, w, t3);
+    v.load(p.v, at, ok);
+    d_o.load(p.d_o, at, ok);
+    u.load(p.s3, wt);
+    du.load(p.s4, wt);
+    put_row(t0, w, [&](int cb) { return dC[cb] * hC[cb]; });
   }
-  lds_barrier();
-  const float *tv = L.tile(0), *tO = L.tile(1), *tu = L.tile(2), *tdu = L.tile(3), *th = L.tile(4), *tD = L.tile(5);
+  cumulate(t3, L.sx, L.gate);
+  x.gates(t3, w);
   {
     const int c = tid & 63, seg = tid >> 6;
     float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) sum += prod[(8 * seg + i) * LD + c];
+    for (int i = 0; i < 16; ++i) sum += t0[(16 * seg + i) * LD + c];
     red[64 * seg + c] = sum;
   }
-  floatx4 pb[2], pk[2], ab[2], ak[2];  // dPqb, dPqk, dAab, dAak
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    pb[j] = pk[j] = ab[j] = ak[j] = zero4();
-    const int col = j ? w.c1 : w.c0;
-    if (col > w.row) continue;
+  const bool wide = *L.gate.wide;
+  float* edge = L.sx;  // G of the blocks' last tokens
+  edge[tid] = t3[(16 * (tid >> 6) + 15) * LD + (tid & 63)];
+  lds_barrier();
+  put_row(t0, w, [&](int cb) { return v[cb]; });
+  put_row(t2, w, [&](int cb) { return u[cb]; });
+  lds_barrier();
+  floatx4 pb[4], pk[4], nb_[4], nk[4];  // dPqb, dPqk, dAab, dAak by t
+  clear(pb), clear(pk), clear(nb_), clear(nk);
+  upto(w.j, [&](auto sb_) {
+    constexpr int sb = decltype(sb_)::value;
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
-      const int k = 16 * kb + 4 * w.g;
-      const floatx4 fo = frag<true>(tO, w.row + w.l16, k), fd = frag<true>(tdu, w.row + w.l16, k);
-      const floatx4 fu = frag<true>(tu, col + w.l16, k), fv = frag<true>(tv, col + w.l16, k);
+      const floatx4 fu = frag<true>(t2, 16 * sb + l16, 16 * kb + g4), fv = frag<true>(t0, 16 * sb + l16, 16 * kb + g4);
+      const floatx4 fo = d_o[kb], fd = du[kb];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        pb[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fo[r], fu[r], pb[j], 0, 0, 0);
-        pk[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fo[r], fv[r], pk[j], 0, 0, 0);
-        ab[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fd[r], fu[r], ab[j], 0, 0, 0);
-        ak[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fd[r], fv[r], ak[j], 0, 0, 0);
+        pb[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(fu[r], fo[r], pb[sb], 0, 0, 0);
+        pk[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(fv[r], fo[r], pk[sb], 0, 0, 0);
+        nb_[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(fu[r], fd[r], nb_[sb], 0, 0, 0);
+        nk[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(fv[r], fd[r], nk[sb], 0, 0, 0);
       }
     }
+  });
+  mask<true, false>(pb, w), mask<true, false>(pk, w), mask<true, true>(nb_, w), mask<true, true>(nk, w);
+  {
+    Row<float> h0, dC;
+    h0.load(p.hT, ht);
+    dC.load(p.s1, wt);
+    // t1 and t3 are free since the gates were read
+    put_row(t1, w, [&](int cb) { return h0[cb] * load4(L.gate.em + 16 * cb + g4); });
+    put_row(t3, w, [&](int cb) { return dC[cb] * load4(L.gate.ec + 16 * cb + g4); });
   }
-  // rows = channels, columns = tokens from here on
-  floatx4 dq[2] = {zero4(), zero4()}, da[2] = {zero4(), zero4()}, db[2] = {zero4(), zero4()}, dk[2] = {zero4(), zero4()};
-  mm2_full<false, true>(dq, th, w.rowT, tO, w.t0, w.t1, w.l16, w.g);
-  mm2_full<false, true>(da, th, w.rowT, tdu, w.t0, w.t1, w.l16, w.g);
-  mm2_full<false, true>(db, tD, w.rowT, tu, w.t0, w.t1, w.l16, w.g);
-  mm2_full<false, true>(dk, tD, w.rowT, tv, w.t0, w.t1, w.l16, w.g);
   lds_barrier();
-  float *Mb = L.tile(0), *Mk = L.tile(1), *Nb = L.tile(2), *Nk = L.tile(3), *tq = L.tile(4), *ta = L.tile(5), *tb = L.tile(6), *tk = L.tile(7);
+  floatx4 dq[4], da[4], db[4], dk[4];  // rows = channels, columns = tokens
+  clear(dq), clear(da), clear(db), clear(dk);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int col = (j ? w.c1 : w.c0) + w.l16;
+  for (int kb = 0; kb < 4; ++kb) {
+    const floatx4 fo = d_o[kb], fd = du[kb], fu = u[kb], fv = v[kb];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tt = w.row + 4 * w.g + r, o = tt * LD + col;
-      Mb[o] = col <= tt ? pb[j][r] : 0.f;
-      Mk[o] = col <= tt ? pk[j][r] : 0.f;
-      Nb[o] = col < tt ? ab[j][r] : 0.f;
-      Nk[o] = col < tt ? ak[j][r] : 0.f;
+    for (int cb = 0; cb < 4; ++cb) {
+      const floatx4 hf = frag<false>(t1, 16 * cb + l16, 16 * kb + g4), df = frag<false>(t3, 16 * cb + l16, 16 * kb + g4);
+      mfma4(dq[cb], hf, fo);
+      mfma4(da[cb], hf, fd);
+      mfma4(db[cb], df, fu);
+      mfma4(dk[cb], df, fv);
     }
   }
-  x.store(tq, ta, tb, tk, Gt, L.gate, p.scale);
-  lds_barrier();
-  const bool wide = *L.gate.wide;
-  const int ch = w.rowT + 4 * w.g;
-  floatx4 xs[2], as[2];  // q dq + a da - b db - k dk and a da
+  floatx4 Gp[4];  // from the lane before
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int col = j ? w.t1 : w.t0, tt = col + w.l16, cb = col / 16;
-    if (!wide) {
-      mm<false, true>(dq[j], tb, w.rowT, Mb, col, 0, cb + 1, w.l16, w.g);
-      mm<false, true>(dq[j], tk, w.rowT, Mk, col, 0, cb + 1, w.l16, w.g);
-      mm<false, true>(da[j], tb, w.rowT, Nb, col, 0, cb + 1, w.l16, w.g);
-      mm<false, true>(da[j], tk, w.rowT, Nk, col, 0, cb + 1, w.l16, w.g);
-      mm<false, false>(db[j], tq, w.rowT, Mb, col, cb, 4, w.l16, w.g);
-      mm<false, false>(db[j], ta, w.rowT, Nb, col, cb, 4, w.l16, w.g);
-      mm<false, false>(dk[j], tq, w.rowT, Mk, col, cb, 4, w.l16, w.g);
-      mm<false, false>(dk[j], ta, w.rowT, Nk, col, cb, 4, w.l16, w.g);
+  for (int cb = 0; cb < 4; ++cb) {
+    const floatx4 G = load4(edge + 64 * max(w.j - 1, 0) + 16 * cb + g4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float prev = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x.G[cb][e]), 0x111, 0xF, 0xF, true));  // row_shr:1
+      Gp[cb][e] = l16 ? prev : w.j ? G[e] : 0.f;
     }
-    const floatx4 G = load4(Gt + tt * LD + ch), Gp = tt ? load4(Gt + (tt - 1) * LD + ch) : zero4(), gl = load4(Gt + (C - 1) * LD + ch);
-    const floatx4 q4 = load4(tq + tt * LD + ch), a4 = load4(ta + tt * LD + ch), b4 = load4(tb + tt * LD + ch), k4 = load4(tk + tt * LD + ch);
-    if (!wide) {
-      const floatx4 m = load4(L.gate.gm + ch);
-      as[j] = a4 * da[j];
-      xs[j] = q4 * dq[j] + as[j] - b4 * db[j] - k4 * dk[j];
+  }
+  const Decay e(x.G, Gp, edge + 192, L.gate, w, wide);
+  auto put_tri = [&](float* tile, const floatx4 (&m)[4]) {  // [t][s]
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float eb = exp_f(m[e] - G[e]);
-        dq[j][e] *= exp_f(G[e] - m[e]);
-        da[j][e] *= exp_f(Gp[e] - m[e]);
-        db[j][e] *= eb;
-        dk[j][e] *= eb;
+    for (int sb = 0; sb < 4; ++sb)
+      if (sb <= w.j) store4(tile + w.t * LD + 16 * sb + g4, m[sb]);
+  };
+  floatx4 xs[4], as[4];  // q dq + a da - b db - k dk and a da
+  if (!wide) {
+    put_row(t0, w, [&](int cb) { return x.b[cb] * e.b[cb]; });
+    put_row(t2, w, [&](int cb) { return x.k[cb] * e.b[cb]; });  // v and u were last read before a barrier
+    lds_barrier();
+    upto(w.j, [&](auto sb_) {
+      constexpr int sb = decltype(sb_)::value;
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) {
+        const floatx4 bf = frag<false>(t0, 16 * cb + l16, 16 * sb + g4), kf = frag<false>(t2, 16 * cb + l16, 16 * sb + g4);
+        mfma4(dq[cb], bf, pb[sb]);
+        mfma4(da[cb], bf, nb_[sb]);
+        mfma4(dq[cb], kf, pk[sb]);
+        mfma4(da[cb], kf, nk[sb]);
       }
-    } else {
+    });
+    lds_barrier();
+    // db, dk: the matrices with the contraction along t, first those of q, then those of a
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int c = ch + e;
-        const float eb = exp_f(gl[e] - G[e]);
-        float rq = exp_f(G[e]) * dq[j][e], ra = exp_f(Gp[e]) * da[j][e], rb = eb * db[j][e], rk = eb * dk[j][e];
-        for (int i = 0; i <= tt; ++i) {
-          const float eq = exp_f(G[e] - Gt[i * LD + c]);
-          rq += eq * (Mb[tt * LD + i] * tb[i * LD + c] + Mk[tt * LD + i] * tk[i * LD + c]);
-          if (i < tt) ra += exp_f(Gp[e] - Gt[i * LD + c]) * (Nb[tt * LD + i] * tb[i * LD + c] + Nk[tt * LD + i] * tk[i * LD + c]);
+    for (int half = 0; half < 2; ++half) {
+      if (half) lds_barrier();
+      put_tri(t1, half ? nb_ : pb), put_tri(t2, half ? nk : pk);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) {
+        if (half) store4(t0 + w.t * LD + 16 * cb + g4, x.a[cb] * e.a[cb]);
+        else store4(t0 + w.t * LD + 16 * cb + g4, p.scale * x.q[cb] * e.q[cb]);
+      }
+      lds_barrier();
+      downto(w.j, [&](auto tb_) {
+        constexpr int tb = decltype(tb_)::value;
+        const floatx4 mb = frag<false>(t1, w.t, 16 * tb + g4), mk = frag<false>(t2, w.t, 16 * tb + g4);
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+          const floatx4 xf = frag<false>(t0, 16 * cb + l16, 16 * tb + g4);
+          mfma4(db[cb], xf, mb);
+          mfma4(dk[cb], xf, mk);
         }
-        for (int i = tt; i < C; ++i) {
-          const float eq = exp_f(Gt[i * LD + c] - G[e]) * tq[i * LD + c];
-          rb += eq * Mb[i * LD + tt];
-          rk += eq * Mk[i * LD + tt];
-          if (i > tt) {
-            const float ea = exp_f(Gt[(i - 1) * LD + c] - G[e]) * ta[i * LD + c];
-            rb += ea * Nb[i * LD + tt];
-            rk += ea * Nk[i * LD + tt];
-          }
-        }
-        dq[j][e] = rq, da[j][e] = ra, db[j][e] = rb, dk[j][e] = rk;
-      }
-      as[j] = a4 * da[j];
-      xs[j] = q4 * dq[j] + as[j] - b4 * db[j] - k4 * dk[j];
-    }
-    if (tt < s.len) {
-      const int64_t o = (s.tok + tt) * D + ch;
-      store_row4<T>(p.dq, o, dq[j] * p.scale);
-      store_row4<T>(p.da, o, da[j]);
-      store_row4<T>(p.db, o, db[j]);
-      store_row4<T>(p.dk, o, dk[j]);
+      });
     }
   }
-  lds_barrier();
-  float *tx = L.tile(0), *tas = L.tile(1), *scr = L.tile(2);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int tt = (j ? w.t1 : w.t0) + w.l16;
-    store4(tx + tt * LD + ch, xs[j]);
-    store4(tas + tt * LD + ch, as[j]);
+  for (int cb = 0; cb < 4; ++cb) dq[cb] *= e.q[cb], da[cb] *= e.a[cb], db[cb] *= e.b[cb], dk[cb] *= e.b[cb];
+  if (wide) {
+    put_tri(t0, pb), put_tri(t2, pk);
+    lds_barrier();
+    put_cols(t1, w, x.G);
+    lds_barrier();
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) wide_grads<T, 0>(p, s.tok, s.len, t0, t2, t1, w.t, 16 * cb + g4, dq[cb], db[cb], dk[cb]);
+    lds_barrier();
+    put_tri(t0, nb_), put_tri(t2, nk);
+    lds_barrier();
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) wide_grads<T, 1>(p, s.tok, s.len, t0, t2, t1, w.t, 16 * cb + g4, da[cb], db[cb], dk[cb]);
   }
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    as[cb] = x.a[cb] * da[cb];
+    xs[cb] = p.scale * x.q[cb] * dq[cb] + as[cb] - x.b[cb] * db[cb] - x.k[cb] * dk[cb];
+  }
+  if (ok) {
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) {
+      store_row4<T>(p.dq, at + 16 * cb, dq[cb] * p.scale);
+      store_row4<T>(p.da, at + 16 * cb, da[cb]);
+      store_row4<T>(p.db, at + 16 * cb, db[cb]);
+      store_row4<T>(p.dk, at + 16 * cb, dk[cb]);
+    }
+  }
+  float *tx = t3, *tas = wide ? t1 : t0, *scr = L.sx;  // tas: read by nobody since the last barrier but in the products above
+  lds_barrier();
+  put_cols(tx, w, xs);
+  put_cols(tas, w, as);
   lds_barrier();
   {
     const int c = tid & 63, seg = tid >> 6;
-    float v[8], sum = 0.f;
+    float val[16], sum = 0.f;
 #pragma unroll
-    for (int i = 7; i >= 0; --i) v[i] = (sum += tx[(8 * seg + i) * LD + c]);
+    for (int i = 15; i >= 0; --i) val[i] = (sum += tx[(16 * seg + i) * LD + c]);
     scr[64 * seg + c] = sum;
     lds_barrier();
     float after = 0.f;
-    for (int j = seg + 1; j < 8; ++j) after += scr[64 * j + c];
+    for (int j = seg + 1; j < 4; ++j) after += scr[64 * j + c];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) after += red[64 * j + c];
+    for (int j = 0; j < 4; ++j) after += red[64 * j + c];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (8 * seg + i < s.len) p.dgk[(s.tok + 8 * seg + i) * D + c] = v[i] + after - tas[(8 * seg + i) * LD + c];
+    for (int i = 0; i < 16; ++i)
+      if (16 * seg + i < s.len) p.dgk[(s.tok + 16 * seg + i) * D + c] = val[i] + after - tas[(16 * seg + i) * LD + c];
   }
 }
 
@@ -869,10 +994,10 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
     else set_kept(p, scratch + 2 * rows * W * TG, rows, n0, p.nw);
     const unsigned grid = (unsigned)(rows * p.nw);
     lnx_profile_mark("dplr_prepare", st);
-    hipLaunchKernelGGL(dplr_prepare_kernel<T>, dim3(grid), dim3(512), LDS_BYTES, st, p);
+    hipLaunchKernelGGL(dplr_prepare_kernel<T>, dim3(grid), dim3(256), LDS_BYTES, st, p);
     lnx_profile_mark("dplr_chunk_scan", st);
-    const ScanParams sp{p.M, p.s1, p.hT, n0 ? a->final_state : a->initial_state, a->final_state, p.KN, n0 - p.k0, p.nw};
-    hipLaunchKernelGGL(dplr_chunk_scan_kernel<false>, dim3((unsigned)rows), dim3(256), 0, st, sp);
+    const ScanParams sp{p.M, p.s1, p.hT, n0 ? a->final_state : a->initial_state, a->final_state, rows, p.KN, n0 - p.k0, p.nw};
+    hipLaunchKernelGGL(dplr_chunk_scan_kernel<false>, dim3(lnx_xcd_grid(rows, 4)), dim3(256), 0, st, sp);
     lnx_profile_mark("dplr_out", st);
     hipLaunchKernelGGL(dplr_out_kernel<T>, dim3(grid), dim3(256), 0, st, p);
   }
@@ -897,12 +1022,12 @@ template <typename T> int backward(const lnx_dplr_chunk_grads* g, const lnx_dplr
     lnx_profile_mark("dplr_r", st);
     hipLaunchKernelGGL(dplr_r_kernel<T>, dim3(grid), dim3(256), 0, st, p);
     lnx_profile_mark("dplr_chunk_scan_bwd", st);
-    const ScanParams sp{p.M, p.s2, p.s1, i == nwin - 1 ? g->d_final_state : carry, i ? carry : g->d_initial_state, p.KN, p.n0, p.nw};
-    hipLaunchKernelGGL(dplr_chunk_scan_kernel<true>, dim3((unsigned)rows), dim3(256), 0, st, sp);
+    const ScanParams sp{p.M, p.s2, p.s1, i == nwin - 1 ? g->d_final_state : carry, i ? carry : g->d_initial_state, rows, p.KN, p.n0, p.nw};
+    hipLaunchKernelGGL(dplr_chunk_scan_kernel<true>, dim3(lnx_xcd_grid(rows, 4)), dim3(256), 0, st, sp);
     lnx_profile_mark("dplr_u", st);
-    hipLaunchKernelGGL(dplr_u_kernel<T>, dim3(grid), dim3(512), LDS_BYTES, st, p);
+    hipLaunchKernelGGL(dplr_u_kernel<T>, dim3(grid), dim3(256), LDS_BYTES, st, p);
     lnx_profile_mark("dplr_grad", st);
-    hipLaunchKernelGGL(dplr_grad_kernel<T>, dim3(grid), dim3(512), LDS_BYTES, st, p);
+    hipLaunchKernelGGL(dplr_grad_kernel<T>, dim3(grid), dim3(256), LDS_BYTES, st, p);
   }
   return LNX_OK;
 }
