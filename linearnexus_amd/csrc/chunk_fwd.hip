@@ -1376,10 +1376,32 @@ template <typename T, int DK> struct PrepSelect<T, DK, LNX_GATE_VECTOR> {
   static auto kernel(bool raw_gate) { return raw_gate ? kda_prepare_kernel<T, DK, true> : kda_prepare_kernel<T, DK, false>; }
 };
 
+// What the scans of chunk_direct.hip and chunk_wide.hip take
+DirectParams direct_params(const FwdParams& p, int gate) {
+  DirectParams d = {};
+  d.geom = p.geom;
+  d.q = reinterpret_cast<const bf16_t*>(p.q); d.k = reinterpret_cast<const bf16_t*>(p.k);
+  d.v = reinterpret_cast<const bf16_t*>(p.v); d.beta = p.beta; d.s0 = p.s0; d.sT_out = p.sT_out;
+  d.o = p.o; d.dv = p.dv; d.o_dtype = p.o_dtype; d.save = p.save; d.vcols = p.vcols; d.gate = gate;
+  d.l2norm = p.l2norm; d.slab = p.slab;
+  d.scale = p.scale; d.ws = p.ws; d.off = p.off;
+  return d;
+}
+
 template <typename T, int DK, int GATE>
 int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   const int64_t slots = (int64_t)p.geom.rows * p.geom.N;
   auto k1 = PrepSelect<T, DK, GATE>::kernel(p.graw != nullptr);
+  const size_t b1 = PrepSelect<T, DK, GATE>::bytes;
+  if (const hipError_t e = hipFuncSetAttribute((const void*)k1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b1); e != hipSuccess)
+    return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  lnx_profile_mark("chunk_prepare", st);
+  hipLaunchKernelGGL(k1, dim3((unsigned)slots), dim3(256), b1, st, p);
+  if constexpr (sizeof(T) == 2 && DK == 256 && GATE != LNX_GATE_VECTOR) {
+    const int rc = lnx_wide_scan(false, direct_params(p, GATE), nstate, st);
+    lnx_profile_mark(nullptr, st);
+    return rc;
+  } else {
   // 32-column slabs when 64-column ones would occupy at most half of the chip (256 CUs); always for 4-byte inputs
   // with dk = 256, whose tiles leave no room in LDS for a wider slab
   constexpr bool can_narrow = (DK >= 128 && sizeof(T) == 2) || (DK == 128 && sizeof(T) == 4);
@@ -1388,15 +1410,12 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   auto k2 = narrow ? chunk_scan_kernel<T, DK, GATE, NARROW> : chunk_scan_kernel<T, DK, GATE, WIDE>;
   auto k3 = chunk_output_kernel<T, DK, GATE>;
   const int bv = narrow ? NARROW : WIDE;
-  const size_t b1 = PrepSelect<T, DK, GATE>::bytes, b3 = OutSmem<T, DK>::bytes;
+  const size_t b3 = OutSmem<T, DK>::bytes;
   const size_t b2 = narrow ? ScanSmem<T, DK, NARROW>::bytes : ScanSmem<T, DK, WIDE>::bytes;
   hipError_t e;
-  if ((e = hipFuncSetAttribute((const void*)k1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b1)) != hipSuccess ||
-      (e = hipFuncSetAttribute((const void*)k2, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b2)) != hipSuccess ||
+  if ((e = hipFuncSetAttribute((const void*)k2, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b2)) != hipSuccess ||
       (e = hipFuncSetAttribute((const void*)k3, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b3)) != hipSuccess)
     return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-  lnx_profile_mark("chunk_prepare", st);
-  hipLaunchKernelGGL(k1, dim3((unsigned)slots), dim3(256), b1, st, p);
   lnx_profile_mark("chunk_scan", st);
   hipLaunchKernelGGL(k2, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(512), b2, st, p);
   if (!ScanSmem<T, DK>::FUSE_OUT && p.o) {  // otherwise the scan has written the outputs
@@ -1410,6 +1429,7 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   }
   lnx_profile_mark(nullptr, st);
   return LNX_OK;
+  }
 }
 
 template <typename T, int DK>
@@ -1491,13 +1511,7 @@ int launch_direct_fwd(const lnx_scan_args* a, const FwdParams& p, int nstate, bo
     if (a->gate == LNX_GATE_SCALAR) launch_prepare_lite<64, LNX_GATE_SCALAR>(p, st);
     else launch_prepare_lite<64, LNX_GATE_NONE>(p, st);
   }
-  DirectParams d = {};
-  d.geom = p.geom;
-  d.q = reinterpret_cast<const bf16_t*>(a->q); d.k = reinterpret_cast<const bf16_t*>(a->k);
-  d.v = reinterpret_cast<const bf16_t*>(a->v); d.beta = a->beta; d.s0 = a->initial_state; d.sT_out = a->final_state;
-  d.o = a->o; d.dv = a->dv; d.o_dtype = a->o_dtype; d.save = !a->forward_only; d.vcols = p.vcols; d.gate = a->gate;
-  d.l2norm = a->use_qk_l2norm; d.slab = a->test_scan_slab;
-  d.scale = a->scale; d.ws = p.ws; d.off = p.off;
+  const DirectParams d = direct_params(p, a->gate);
   int rc = lnx_direct_scan_fwd(d, a->dk, a->gate, nstate, st);
   if (rc != LNX_OK) return rc;
   hipError_t e = hipGetLastError();
