@@ -235,6 +235,14 @@ int lnx_conv1d_packed_fwd(const void* x, const float* weight, const float* bias,
 int lnx_conv1d_packed_bwd(const void* x, const float* weight, const float* bias, const int32_t* cu_seqlens, int32_t nseq,
                           const void* dy, void* dx, float* d_weight, float* d_bias, int32_t T, int32_t D, int32_t K,
                           int32_t dtype, int32_t activation, void* hip_stream);
+/* The same pair without the backward pass's fill kernel: the forward kernel clears `nzeroed` floats on its way, and
+ * lnx_conv1d_bwd_add adds to a d_weight and d_bias cleared like that.  cu_seqlens NULL: a dense batch. */
+int lnx_conv1d_fwd_zero(const void* x, const float* weight, const float* bias, const void* cache, const int32_t* cu_seqlens, int32_t nseq,
+                        void* y, void* new_cache, float* zeroed, int64_t nzeroed, int32_t B, int32_t T, int32_t D, int32_t K,
+                        int32_t dtype, int32_t activation, void* hip_stream);
+int lnx_conv1d_bwd_add(const void* x, const float* weight, const float* bias, const void* cache, const int32_t* cu_seqlens, int32_t nseq,
+                       const void* dy, void* dx, float* d_weight, float* d_bias, int32_t B, int32_t T, int32_t D, int32_t K,
+                       int32_t dtype, int32_t activation, void* hip_stream);
 
 /*
  * RWKV-7's diagonal-plus-low-rank delta rule (linearnexus/modules/linear_attn/rwkv7.py:114-265), the sibling

@@ -28,6 +28,7 @@ struct ConvParams {
   int B, T, D, K, act, gx, seg;  // seg: tokens per thread
   const int32_t* cu; int nseq;  // packed batch (B = 1): the taps stop at the start of each token's sequence
   void* dcache;                 // conv1d_dcache_kernel only
+  float* zero; int64_t nzero;   // forward: cleared on the way, the sums that the backward pass will add to; backward: zero means they are clear
 };
 
 // Packed batches: [lo, hi) is the sequence that holds token t (bisection over the table; entries clamped to [0, T]).
@@ -98,6 +99,10 @@ __device__ __forceinline__ void load_taps(const ConvParams& p, int c, float (&w)
 
 template <typename T, int N, bool PACKED>
 __global__ __launch_bounds__(256) void conv1d_fwd_kernel(ConvParams p) {
+  if (p.zero) {
+    const int64_t threads = (int64_t)gridDim.x * gridDim.y * gridDim.z * 256;
+    for (int64_t i = (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * 256 + threadIdx.x; i < p.nzero; i += threads) p.zero[i] = 0.f;
+  }
   const int c = (blockIdx.x * p.gx + (threadIdx.x & (p.gx - 1))) * N;
   const int seg = blockIdx.y * (256 / p.gx) + threadIdx.x / p.gx;
   const int b = blockIdx.z;
@@ -417,6 +422,7 @@ int conv_fwd(ConvParams p, int dtype, hipStream_t st) {
   if (K == 1) p.new_cache = nullptr, p.cache = nullptr;  // a width-1 kernel carries nothing
   const int n = dtype == LNX_BF16 ? 8 : 4;
   if ((size_t)B * T == 0) {
+    if (p.zero) fill_zero_kernel<<<(unsigned)((p.nzero + 255) / 256), 256, 0, st>>>(p.zero, (int)p.nzero, nullptr, 0);
     // nothing to convolve: the carry passes through unchanged (zeros without one, like the reference's zero cache)
     if (p.new_cache && p.new_cache != p.cache && B > 0) {
       const size_t bytes = (size_t)B * (K - 1) * D * (dtype == LNX_BF16 ? 2 : 4);
@@ -449,7 +455,7 @@ int conv_bwd(ConvParams p, int dtype, hipStream_t st) {
   if (int rc = check(p, dtype, true)) return rc;
   if (p.dbias && !p.dw) return lnx_set_error(LNX_ERR_NULL, "conv1d_bwd: d_bias needs d_weight");
   const int B = p.B, T = p.T, D = p.D, K = p.K;
-  if (p.dw) {
+  if (p.dw && !p.nzero) {
     lnx_profile_mark("conv1d_fill", st);
     fill_zero_kernel<<<(K * D + 255) / 256, 256, 0, st>>>(p.dw, K * D, p.dbias, D);
   }
@@ -482,14 +488,14 @@ int check_packed(const int32_t* cu, int nseq) {
 extern "C" int lnx_conv1d_fwd(const void* x, const float* weight, const float* bias, const void* cache, void* y,
                               void* new_cache, int32_t B, int32_t T, int32_t D, int32_t K, int32_t dtype,
                               int32_t activation, void* hip_stream) {
-  ConvParams p{x, weight, bias, cache, y, new_cache, nullptr, nullptr, nullptr, nullptr, B, T, D, K, activation, 64, SEG_FWD, nullptr, 0, nullptr};
+  ConvParams p{x, weight, bias, cache, y, new_cache, nullptr, nullptr, nullptr, nullptr, B, T, D, K, activation, 64, SEG_FWD, nullptr, 0, nullptr, nullptr, 0};
   return conv_fwd(p, dtype, static_cast<hipStream_t>(hip_stream));
 }
 
 extern "C" int lnx_conv1d_bwd(const void* x, const float* weight, const float* bias, const void* cache, const void* dy,
                               void* dx, float* d_weight, float* d_bias, int32_t B, int32_t T, int32_t D, int32_t K,
                               int32_t dtype, int32_t activation, void* hip_stream) {
-  ConvParams p{x, weight, bias, cache, nullptr, nullptr, dy, dx, d_weight, d_bias, B, T, D, K, activation, 64, SEG_FWD, nullptr, 0, nullptr};
+  ConvParams p{x, weight, bias, cache, nullptr, nullptr, dy, dx, d_weight, d_bias, B, T, D, K, activation, 64, SEG_FWD, nullptr, 0, nullptr, nullptr, 0};
   return conv_bwd(p, dtype, static_cast<hipStream_t>(hip_stream));
 }
 
@@ -497,7 +503,7 @@ extern "C" int lnx_conv1d_packed_fwd(const void* x, const float* weight, const f
                                      int32_t nseq, void* y, void* new_cache, int32_t T, int32_t D, int32_t K, int32_t dtype,
                                      int32_t activation, void* hip_stream) {
   if (int rc = check_packed(cu_seqlens, nseq)) return rc;
-  ConvParams p{x, weight, bias, nullptr, y, new_cache, nullptr, nullptr, nullptr, nullptr, 1, T, D, K, activation, 64, SEG_FWD, cu_seqlens, nseq, nullptr};
+  ConvParams p{x, weight, bias, nullptr, y, new_cache, nullptr, nullptr, nullptr, nullptr, 1, T, D, K, activation, 64, SEG_FWD, cu_seqlens, nseq, nullptr, nullptr, 0};
   return conv_fwd(p, dtype, static_cast<hipStream_t>(hip_stream));
 }
 
@@ -505,14 +511,33 @@ extern "C" int lnx_conv1d_packed_bwd(const void* x, const float* weight, const f
                                      int32_t nseq, const void* dy, void* dx, float* d_weight, float* d_bias, int32_t T,
                                      int32_t D, int32_t K, int32_t dtype, int32_t activation, void* hip_stream) {
   if (int rc = check_packed(cu_seqlens, nseq)) return rc;
-  ConvParams p{x, weight, bias, nullptr, nullptr, nullptr, dy, dx, d_weight, d_bias, 1, T, D, K, activation, 64, SEG_FWD, cu_seqlens, nseq, nullptr};
+  ConvParams p{x, weight, bias, nullptr, nullptr, nullptr, dy, dx, d_weight, d_bias, 1, T, D, K, activation, 64, SEG_FWD, cu_seqlens, nseq, nullptr, nullptr, 0};
+  return conv_bwd(p, dtype, static_cast<hipStream_t>(hip_stream));
+}
+
+extern "C" int lnx_conv1d_fwd_zero(const void* x, const float* weight, const float* bias, const void* cache, const int32_t* cu_seqlens, int32_t nseq,
+                                   void* y, void* new_cache, float* zeroed, int64_t nzeroed, int32_t B, int32_t T, int32_t D, int32_t K, int32_t dtype,
+                                   int32_t activation, void* hip_stream) {
+  if (cu_seqlens && (B != 1 || cache)) return lnx_set_error(LNX_ERR_SHAPE, "conv1d: a packed batch has B == 1 (B=%d) and no cache", B);
+  if (cu_seqlens) if (int rc = check_packed(cu_seqlens, nseq)) return rc;
+  if (!zeroed || nzeroed <= 0 || nzeroed >= (1ll << 31)) return lnx_set_error(LNX_ERR_NULL, "conv1d_fwd_zero: nothing to clear");
+  ConvParams p{x, weight, bias, cache, y, new_cache, nullptr, nullptr, nullptr, nullptr, B, T, D, K, activation, 64, SEG_FWD, cu_seqlens, nseq, nullptr, zeroed, nzeroed};
+  return conv_fwd(p, dtype, static_cast<hipStream_t>(hip_stream));
+}
+
+extern "C" int lnx_conv1d_bwd_add(const void* x, const float* weight, const float* bias, const void* cache, const int32_t* cu_seqlens, int32_t nseq,
+                                  const void* dy, void* dx, float* d_weight, float* d_bias, int32_t B, int32_t T, int32_t D, int32_t K, int32_t dtype,
+                                  int32_t activation, void* hip_stream) {
+  if (cu_seqlens && (B != 1 || cache)) return lnx_set_error(LNX_ERR_SHAPE, "conv1d: a packed batch has B == 1 (B=%d) and no cache", B);
+  if (cu_seqlens) if (int rc = check_packed(cu_seqlens, nseq)) return rc;
+  ConvParams p{x, weight, bias, cache, nullptr, nullptr, dy, dx, d_weight, d_bias, B, T, D, K, activation, 64, SEG_FWD, cu_seqlens, nseq, nullptr, nullptr, 1};
   return conv_bwd(p, dtype, static_cast<hipStream_t>(hip_stream));
 }
 
 extern "C" int lnx_conv1d_cache_bwd(const void* x, const float* weight, const float* bias, const void* cache, const void* dy,
                                     void* d_cache, int32_t B, int32_t T, int32_t D, int32_t K, int32_t dtype,
                                     int32_t activation, void* hip_stream) {
-  ConvParams p{x, weight, bias, cache, nullptr, nullptr, dy, d_cache, nullptr, nullptr, B, T, D, K, activation, 64, SEG_FWD, nullptr, 0, d_cache};
+  ConvParams p{x, weight, bias, cache, nullptr, nullptr, dy, d_cache, nullptr, nullptr, B, T, D, K, activation, 64, SEG_FWD, nullptr, 0, d_cache, nullptr, 0};
   if (int rc = check(p, dtype, true)) return rc;
   if (K == 1 || B == 0) return 0;  // no carry to differentiate
   if (!d_cache) return lnx_set_error(LNX_ERR_NULL, "conv1d_cache_bwd: d_cache is required");

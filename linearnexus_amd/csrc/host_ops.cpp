@@ -13,6 +13,7 @@
 
 #include <c10/hip/HIPStream.h>
 
+#include <atomic>
 #include <optional>
 #include <stdexcept>
 #include <string>
@@ -542,11 +543,21 @@ struct ConvSide {
   Tensor x, cin, cout, cu;
 };
 
-Tensor conv_forward(const Tensor& w, const Tensor& bias, const ConvSide& side, int64_t act) {
+// A buffer that the forward kernel has cleared, for the first backward pass of its node.
+struct Cleared : torch::CustomClassHolder {
+  Tensor buffer;
+  std::atomic<bool> taken{false};
+};
+
+// zeroed: cleared by the kernel on its way, or undefined
+Tensor conv_forward(const Tensor& w, const Tensor& bias, const ConvSide& side, int64_t act, const Tensor& zeroed = Tensor()) {
   const Tensor &x = side.x, &cin = side.cin, &cout = side.cout, &cu = side.cu;
   const int32_t B = (int32_t)x.size(0), T = (int32_t)x.size(1), D = (int32_t)x.size(2), K = (int32_t)w.size(0), dt = code_of(x.scalar_type());
   Tensor y = at::empty_like(x);
-  if (cu.defined())
+  if (zeroed.defined())
+    check_status(lnx_conv1d_fwd_zero(ptr(x), fptr(w), fptr(bias), ptr(cin), static_cast<const int32_t*>(ptr(cu)), cu.defined() ? (int32_t)cu.numel() - 1 : 0, ptr(y),
+                                     ptr(cout), fptr(zeroed), zeroed.numel(), B, T, D, K, dt, (int32_t)act, stream_of(x)), "lnx_conv1d_fwd_zero");
+  else if (cu.defined())
     check_status(lnx_conv1d_packed_fwd(ptr(x), fptr(w), fptr(bias), static_cast<const int32_t*>(ptr(cu)), (int32_t)cu.numel() - 1, ptr(y), ptr(cout), T, D, K,
                                        dt, (int32_t)act, stream_of(x)), "lnx_conv1d_packed_fwd");
   else
@@ -559,7 +570,11 @@ struct ConvFn : Function<ConvFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const OptT& bias, const OptT& cache, const ConvSide& side,
                         int64_t act, bool lost_cache) {
     const Tensor w = f32(weight), b = f32(undef(bias));
-    Tensor y = conv_forward(w, b, side, act);
+    // the parameters' gradients are sums that start from zero: this kernel clears them, the backward pass saves a launch
+    auto cleared = c10::make_intrusive<Cleared>();
+    cleared->buffer = at::empty({w.size(0) + (b.defined() ? 1 : 0), w.size(1)}, w.options());
+    Tensor y = conv_forward(w, b, side, act, cleared->buffer);
+    ctx->saved_data["cleared"] = c10::IValue::make_capsule(cleared);
     ctx->save_for_backward({x.is_contiguous() ? x : side.x, w, b, lost_cache ? Tensor() : side.cin, side.cu});
     ctx->saved_data["i"] = std::vector<int64_t>{act, (int64_t)weight.scalar_type(), (int64_t)(bias.has_value() ? bias->scalar_type() : at::kFloat),
                                                 (int64_t)(cache.has_value() ? cache->scalar_type() : at::kFloat), lost_cache,
@@ -573,8 +588,15 @@ struct ConvFn : Function<ConvFn> {
     const Tensor &x = s[0], &w = s[1], &b = s[2], &cin = s[3], &cu = s[4];
     const int32_t B = (int32_t)x.size(0), T = (int32_t)x.size(1), D = (int32_t)x.size(2), K = (int32_t)w.size(0), dt = code_of(x.scalar_type()), act = (int32_t)m[0];
     const Tensor dy = grads[0].to(x.scalar_type()).contiguous();
-    Tensor dx = at::empty_like(x), dw = at::empty_like(w), db = b.defined() ? at::empty_like(b) : Tensor(), dc;
-    if (cu.defined())
+    Tensor dx = at::empty_like(x), dw, db, dc;
+    auto cleared = c10::static_intrusive_pointer_cast<Cleared>(ctx->saved_data["cleared"].toCapsule());
+    if (!cleared->taken.exchange(true)) {
+      const Tensor buffer = std::move(cleared->buffer);
+      dw = b.defined() ? buffer.narrow(0, 0, K) : buffer;
+      if (b.defined()) db = buffer.select(0, K);
+      check_status(lnx_conv1d_bwd_add(ptr(x), fptr(w), fptr(b), ptr(cin), static_cast<const int32_t*>(ptr(cu)), cu.defined() ? (int32_t)cu.numel() - 1 : 0, ptr(dy),
+                                      ptr(dx), fptr(dw), fptr(db), B, T, D, K, dt, act, stream_of(x)), "lnx_conv1d_bwd_add");
+    } else if (dw = at::empty_like(w), db = b.defined() ? at::empty_like(b) : Tensor(); cu.defined())
       check_status(lnx_conv1d_packed_bwd(ptr(x), fptr(w), fptr(b), static_cast<const int32_t*>(ptr(cu)), (int32_t)cu.numel() - 1, ptr(dy), ptr(dx), fptr(dw),
                                          fptr(db), T, D, K, dt, act, stream_of(x)), "lnx_conv1d_packed_bwd");
     else
