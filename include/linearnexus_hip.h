@@ -204,6 +204,10 @@ int lnx_chunk_bwd(const lnx_scan_args* a, void* hip_stream);
 int lnx_l2norm_fwd(const void* x, void* y, int64_t rows, int32_t d, int32_t dtype, void* hip_stream);
 int lnx_l2norm_bwd(const void* x, const void* dy, void* dx, int64_t rows, int32_t d, int32_t dtype,
                    void* hip_stream);
+/* Two tensors of one shape in one launch. */
+int lnx_l2norm_pair_fwd(const void* x0, const void* x1, void* y0, void* y1, int64_t rows, int32_t d, int32_t dtype, void* hip_stream);
+int lnx_l2norm_pair_bwd(const void* x0, const void* x1, const void* dy0, const void* dy1, void* dx0, void* dx1, int64_t rows, int32_t d,
+                        int32_t dtype, void* hip_stream);
 
 /*
  * Short causal depthwise convolution over [B, T, D] activations, kernel width K <= 4, with the SiLU the

@@ -116,7 +116,9 @@ __global__ __launch_bounds__(256) void l2norm_bwd_kernel(const T* x, const T* dy
 // wavefront covers 64 / LPR rows per pass and four passes per step (all loads of a step issued
 // before the first reduction), so the kernels run at streaming bandwidth.
 template <typename T, int LPR>
-__global__ __launch_bounds__(256) void l2norm_fwd_vec_kernel(const T* x, T* y, int64_t rows) {
+__global__ __launch_bounds__(256) void l2norm_fwd_vec_kernel(const T* x0, const T* x1, T* y0, T* y1, int64_t rows) {
+  const T* x = blockIdx.y ? x1 : x0;
+  T* y = blockIdx.y ? y1 : y0;
   typedef typename Vec16<T>::V V;
   constexpr int VN = Vec16<T>::N, RPW = 64 / LPR, UNR = 4, D = LPR * VN;
   const int lane = threadIdx.x & 63, sub = lane / LPR, li = lane % LPR;
@@ -146,7 +148,9 @@ __global__ __launch_bounds__(256) void l2norm_fwd_vec_kernel(const T* x, T* y, i
 }
 
 template <typename T, int LPR>
-__global__ __launch_bounds__(256) void l2norm_bwd_vec_kernel(const T* x, const T* dy, T* dx, int64_t rows) {
+__global__ __launch_bounds__(256) void l2norm_bwd_vec_kernel(const T* x0, const T* x1, const T* dy0, const T* dy1, T* dx0, T* dx1, int64_t rows) {
+  const T *x = blockIdx.y ? x1 : x0, *dy = blockIdx.y ? dy1 : dy0;
+  T* dx = blockIdx.y ? dx1 : dx0;
   typedef typename Vec16<T>::V V;
   constexpr int VN = Vec16<T>::N, RPW = 64 / LPR, UNR = 4, D = LPR * VN;
   const int lane = threadIdx.x & 63, sub = lane / LPR, li = lane % LPR;
@@ -196,33 +200,33 @@ template <typename T> int norm_lanes(int d) {
 }
 
 template <typename T>
-bool launch_norm_fwd(const T* x, T* y, int64_t rows, int d, hipStream_t st) {
+bool launch_norm_fwd(const T* x, T* y, int64_t rows, int d, hipStream_t st, const T* x1 = nullptr, T* y1 = nullptr) {
   const int l = norm_lanes<T>(d);
   if (!l) return false;
   const int64_t waves = (rows + (64 / l) * 4 - 1) / ((64 / l) * 4);
-  dim3 grid((unsigned)((waves + 3) / 4));
+  dim3 grid((unsigned)((waves + 3) / 4), x1 ? 2 : 1);  // the second tensor of a pair: blockIdx.y
   switch (l) {
-    case 4: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 4>), grid, dim3(256), 0, st, x, y, rows); break;
-    case 8: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 8>), grid, dim3(256), 0, st, x, y, rows); break;
-    case 16: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 16>), grid, dim3(256), 0, st, x, y, rows); break;
-    case 32: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 32>), grid, dim3(256), 0, st, x, y, rows); break;
-    default: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 64>), grid, dim3(256), 0, st, x, y, rows); break;
+    case 4: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 4>), grid, dim3(256), 0, st, x, x1, y, y1, rows); break;
+    case 8: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 8>), grid, dim3(256), 0, st, x, x1, y, y1, rows); break;
+    case 16: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 16>), grid, dim3(256), 0, st, x, x1, y, y1, rows); break;
+    case 32: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 32>), grid, dim3(256), 0, st, x, x1, y, y1, rows); break;
+    default: hipLaunchKernelGGL((l2norm_fwd_vec_kernel<T, 64>), grid, dim3(256), 0, st, x, x1, y, y1, rows); break;
   }
   return true;
 }
 
 template <typename T>
-bool launch_norm_bwd(const T* x, const T* dy, T* dx, int64_t rows, int d, hipStream_t st) {
+bool launch_norm_bwd(const T* x, const T* dy, T* dx, int64_t rows, int d, hipStream_t st, const T* x1 = nullptr, const T* dy1 = nullptr, T* dx1 = nullptr) {
   const int l = norm_lanes<T>(d);
   if (!l) return false;
   const int64_t waves = (rows + (64 / l) * 4 - 1) / ((64 / l) * 4);
-  dim3 grid((unsigned)((waves + 3) / 4));
+  dim3 grid((unsigned)((waves + 3) / 4), x1 ? 2 : 1);  // the second tensor of a pair: blockIdx.y
   switch (l) {
-    case 4: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 4>), grid, dim3(256), 0, st, x, dy, dx, rows); break;
-    case 8: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 8>), grid, dim3(256), 0, st, x, dy, dx, rows); break;
-    case 16: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 16>), grid, dim3(256), 0, st, x, dy, dx, rows); break;
-    case 32: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 32>), grid, dim3(256), 0, st, x, dy, dx, rows); break;
-    default: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 64>), grid, dim3(256), 0, st, x, dy, dx, rows); break;
+    case 4: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 4>), grid, dim3(256), 0, st, x, x1, dy, dy1, dx, dx1, rows); break;
+    case 8: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 8>), grid, dim3(256), 0, st, x, x1, dy, dy1, dx, dx1, rows); break;
+    case 16: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 16>), grid, dim3(256), 0, st, x, x1, dy, dy1, dx, dx1, rows); break;
+    case 32: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 32>), grid, dim3(256), 0, st, x, x1, dy, dy1, dx, dx1, rows); break;
+    default: hipLaunchKernelGGL((l2norm_bwd_vec_kernel<T, 64>), grid, dim3(256), 0, st, x, x1, dy, dy1, dx, dx1, rows); break;
   }
   return true;
 }
@@ -258,6 +262,33 @@ extern "C" int lnx_l2norm_fwd(const void* x, void* y, int64_t rows, int32_t d, i
   return finish("l2norm_fwd");
 }
 
+extern "C" int lnx_l2norm_pair_fwd(const void* x0, const void* x1, void* y0, void* y1, int64_t rows, int32_t d, int32_t dtype, void* stream) {
+  int rc = check_norm_args(x0, y0, rows, d, dtype);
+  if (rc == LNX_OK) rc = check_norm_args(x1, y1, rows, d, dtype);
+  if (rc != LNX_OK || rows == 0) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  const bool vec = (dtype == LNX_BF16) ? launch_norm_fwd<bf16_t>((const bf16_t*)x0, (bf16_t*)y0, rows, d, st, (const bf16_t*)x1, (bf16_t*)y1)
+                                       : launch_norm_fwd<float>((const float*)x0, (float*)y0, rows, d, st, (const float*)x1, (float*)y1);
+  if (vec) return finish("l2norm_pair_fwd");
+  rc = lnx_l2norm_fwd(x0, y0, rows, d, dtype, stream);
+  return rc != LNX_OK ? rc : lnx_l2norm_fwd(x1, y1, rows, d, dtype, stream);
+}
+
+extern "C" int lnx_l2norm_pair_bwd(const void* x0, const void* x1, const void* dy0, const void* dy1, void* dx0, void* dx1, int64_t rows, int32_t d,
+                                   int32_t dtype, void* stream) {
+  int rc = check_norm_args(x0, dy0, rows, d, dtype);
+  if (rc == LNX_OK) rc = check_norm_args(x1, dy1, rows, d, dtype);
+  if (rc != LNX_OK || rows == 0) return rc;
+  if (!dx0 || !dx1) return lnx_set_error(LNX_ERR_NULL, "l2norm_pair_bwd: dx is NULL");
+  hipStream_t st = (hipStream_t)stream;
+  const bool vec = (dtype == LNX_BF16)
+                       ? launch_norm_bwd<bf16_t>((const bf16_t*)x0, (const bf16_t*)dy0, (bf16_t*)dx0, rows, d, st, (const bf16_t*)x1, (const bf16_t*)dy1, (bf16_t*)dx1)
+                       : launch_norm_bwd<float>((const float*)x0, (const float*)dy0, (float*)dx0, rows, d, st, (const float*)x1, (const float*)dy1, (float*)dx1);
+  if (vec) return finish("l2norm_pair_bwd");
+  rc = lnx_l2norm_bwd(x0, dy0, dx0, rows, d, dtype, stream);
+  return rc != LNX_OK ? rc : lnx_l2norm_bwd(x1, dy1, dx1, rows, d, dtype, stream);
+}
+
 extern "C" int lnx_l2norm_bwd(const void* x, const void* dy, void* dx, int64_t rows, int32_t d, int32_t dtype,
                               void* stream) {
   int rc = check_norm_args(x, dy, rows, d, dtype);
@@ -276,4 +307,22 @@ extern "C" int lnx_l2norm_bwd(const void* x, const void* dy, void* dx, int64_t r
       hipLaunchKernelGGL(l2norm_bwd_kernel<float>, grid, dim3(256), 0, st, (const float*)x, (const float*)dy, (float*)dx, rows, d);
   }
   return finish("l2norm_bwd");
+}
+
+// The dynamic LDS limit of a kernel on the current device, set when this thread first needs it: the runtime call costs a launch
+// path of several kernels about a microsecond each time.
+int lnx_lds_limit(const void* kernel, size_t bytes) {
+  struct Seen {
+    const void* kernel;
+    int device, bytes;
+  };
+  static thread_local Seen seen[256] = {};
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  Seen& s = seen[(reinterpret_cast<uintptr_t>(kernel) >> 4 ^ (uintptr_t)device * 31) & 255];
+  if (e == hipSuccess && s.kernel == kernel && s.device == device && s.bytes >= (int)bytes) return LNX_OK;
+  if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (e != hipSuccess) return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  s = Seen{kernel, device, (int)bytes};
+  return LNX_OK;
 }

@@ -1449,10 +1449,8 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
   auto k2 = bwd_dqk_kernel<T, DK, GATE>;
   auto k3 = (GATE == LNX_GATE_VECTOR && p.graw) ? bwd_wy2_kernel<T, DK, GATE, GATE == LNX_GATE_VECTOR> : bwd_wy2_kernel<T, DK, GATE>;
   const size_t b2 = DqkCfg<T, DK, GATE>::bytes, b3 = Wy2Cfg<T, DK, GATE>::bytes;
-  hipError_t e;
-  if ((e = hipFuncSetAttribute((const void*)k2, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b2)) != hipSuccess ||
-      (e = hipFuncSetAttribute((const void*)k3, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b3)) != hipSuccess)
-    return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  int rc;
+  if ((rc = lnx_lds_limit((const void*)k2, b2)) != LNX_OK || (rc = lnx_lds_limit((const void*)k3, b3)) != LNX_OK) return rc;
   if (!BScanCfg<T, DK>::FUSE_LOCAL) {  // otherwise bwd_scan forms the chunk-local part itself
     lnx_profile_mark("bwd_local", st);
     hipLaunchKernelGGL(bwd_local_kernel<T>, dim3(lnx_xcd_grid(slots, p.dv / 64)), dim3(256), 0, st, p);
@@ -1463,13 +1461,12 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
     d.q = reinterpret_cast<const bf16_t*>(p.q); d.k = reinterpret_cast<const bf16_t*>(p.k);
     d.dv = p.dv; d.gate = GATE; d.slab = p.slab; d.scale = p.scale; d.ws = p.ws; d.off = p.off;
     d.d_o = reinterpret_cast<const bf16_t*>(p.d_o); d.d_sT = p.d_sT; d.ds0 = p.ds0;
-    if (const int rc = lnx_wide_scan(true, d, nstate, st); rc != LNX_OK) return rc;
+    if ((rc = lnx_wide_scan(true, d, nstate, st)) != LNX_OK) return rc;
   } else {
     auto k1 = narrow ? bwd_scan_kernel<T, DK, GATE, NARROW> : bwd_scan_kernel<T, DK, GATE, WIDE>;
     const int bv = narrow ? BScanCfg<T, DK, NARROW>::BV : BScanCfg<T, DK, WIDE>::BV;
     const size_t b1 = narrow ? BScanCfg<T, DK, NARROW>::bytes : BScanCfg<T, DK, WIDE>::bytes;
-    if ((e = hipFuncSetAttribute((const void*)k1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b1)) != hipSuccess)
-      return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+    if ((rc = lnx_lds_limit((const void*)k1, b1)) != LNX_OK) return rc;
     lnx_profile_mark("bwd_scan", st);
     hipLaunchKernelGGL(k1, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(512), b1, st, p);
   }

@@ -427,8 +427,7 @@ int launch_scan_fwd(const DirectParams& p, int nstate, hipStream_t st) {
   auto k = narrow ? scan_fwd_kernel<DK, GATE, 32, OT> : scan_fwd_kernel<DK, GATE, 64, OT>;
   const size_t b = narrow ? FScanL<DK, 32>::bytes : FScanL<DK, 64>::bytes;
   const int bv = narrow ? 32 : 64, threads = narrow ? FScanL<DK, 32>::threads : FScanL<DK, 64>::threads;
-  hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
-  if (e != hipSuccess) return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  if (const int rc = lnx_lds_limit((const void*)k, b); rc != LNX_OK) return rc;
   lnx_profile_mark("chunk_scan", st);
   hipLaunchKernelGGL(k, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(threads), b, st, p);
   lnx_profile_mark(nullptr, st);
@@ -746,8 +745,7 @@ int launch_scan_bwd(const DirectParams& p, int nstate, hipStream_t st) {
   auto k = narrow ? scan_bwd_kernel<DK, GATE, 32> : scan_bwd_kernel<DK, GATE, 64>;
   const size_t b = narrow ? BScanL<DK, 32>::bytes : BScanL<DK, 64>::bytes;
   const int bv = narrow ? 32 : 64, threads = narrow ? BScanL<DK, 32>::threads : BScanL<DK, 64>::threads;
-  hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
-  if (e != hipSuccess) return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  if (const int rc = lnx_lds_limit((const void*)k, b); rc != LNX_OK) return rc;
   lnx_profile_mark("bwd_scan", st);
   hipLaunchKernelGGL(k, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(threads), b, st, p);
   return LNX_OK;
@@ -1116,8 +1114,7 @@ template <int DK, int GATE>
 int launch_bwd_chunk(const DirectParams& p, hipStream_t st) {
   auto k = bwd_chunk_kernel<DK, GATE>;
   const size_t b = BChunkL<DK>::bytes;
-  hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
-  if (e != hipSuccess) return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  if (const int rc = lnx_lds_limit((const void*)k, b); rc != LNX_OK) return rc;
   lnx_profile_mark("bwd_chunk", st);
   hipLaunchKernelGGL(k, dim3((unsigned)((int64_t)p.geom.rows * p.geom.N)), dim3(256), b, st, p);
   lnx_profile_mark(nullptr, st);

@@ -1393,8 +1393,7 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   const int64_t slots = (int64_t)p.geom.rows * p.geom.N;
   auto k1 = PrepSelect<T, DK, GATE>::kernel(p.graw != nullptr);
   const size_t b1 = PrepSelect<T, DK, GATE>::bytes;
-  if (const hipError_t e = hipFuncSetAttribute((const void*)k1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b1); e != hipSuccess)
-    return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  if (const int rc = lnx_lds_limit((const void*)k1, b1); rc != LNX_OK) return rc;
   lnx_profile_mark("chunk_prepare", st);
   hipLaunchKernelGGL(k1, dim3((unsigned)slots), dim3(256), b1, st, p);
   if constexpr (sizeof(T) == 2 && DK == 256 && GATE != LNX_GATE_VECTOR) {
@@ -1412,10 +1411,8 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   const int bv = narrow ? NARROW : WIDE;
   const size_t b3 = OutSmem<T, DK>::bytes;
   const size_t b2 = narrow ? ScanSmem<T, DK, NARROW>::bytes : ScanSmem<T, DK, WIDE>::bytes;
-  hipError_t e;
-  if ((e = hipFuncSetAttribute((const void*)k2, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b2)) != hipSuccess ||
-      (e = hipFuncSetAttribute((const void*)k3, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b3)) != hipSuccess)
-    return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  int rc;
+  if ((rc = lnx_lds_limit((const void*)k2, b2)) != LNX_OK || (rc = lnx_lds_limit((const void*)k3, b3)) != LNX_OK) return rc;
   lnx_profile_mark("chunk_scan", st);
   hipLaunchKernelGGL(k2, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(512), b2, st, p);
   if (!ScanSmem<T, DK>::FUSE_OUT && p.o) {  // otherwise the scan has written the outputs

@@ -487,8 +487,7 @@ int slab_width(const DirectParams& p, int nstate) {
 }
 
 template <typename K> int launch(K k, size_t bytes, int bv, int threads, const char* name, const DirectParams& p, int nstate, hipStream_t st) {
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  if (e != hipSuccess) return lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  if (const int rc = lnx_lds_limit(reinterpret_cast<const void*>(k), bytes); rc != LNX_OK) return rc;
   lnx_profile_mark(name, st);
   hipLaunchKernelGGL(k, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(threads), bytes, st, p);
   return LNX_OK;

@@ -978,10 +978,7 @@ void set_kept(ChunkParams& p, float* kept, int64_t rows, int k0, int KN) {
 }
 constexpr int64_t kept_tiles(int64_t n) { return 3 * n + 1; }  // of a row that keeps n chunks
 
-template <typename K> int lds_limit(K* k) {
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES);
-  return e == hipSuccess ? LNX_OK : lnx_set_error(LNX_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-}
+template <typename K> int lds_limit(K* k) { return lnx_lds_limit(reinterpret_cast<const void*>(k), LDS_BYTES); }
 
 template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;

@@ -17,6 +17,7 @@
 #include <optional>
 #include <stdexcept>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/linearnexus_hip.h"
@@ -317,6 +318,26 @@ Tensor l2norm_bwd(const Tensor& x0, const Tensor& dy0) {
   return turned ? dx.transpose(1, 2) : dx;
 }
 
+// q and k of a chunk call (one shape, dense in the call's layout), one launch for both
+std::pair<Tensor, Tensor> l2norm_pair_fwd(const Tensor& q0, const Tensor& k0) {
+  bool turned_q, turned_k;
+  const Tensor q = dense(q0, turned_q), k = dense(k0, turned_k);
+  Tensor qn = at::empty_like(q), kn = at::empty_like(k);
+  const int64_t d = q.size(-1);
+  check_status(lnx_l2norm_pair_fwd(ptr(q), ptr(k), ptr(qn), ptr(kn), d ? q.numel() / d : 0, (int32_t)d, code_of(q.scalar_type()), stream_of(q)), "lnx_l2norm_pair_fwd");
+  return {turned_q ? qn.transpose(1, 2) : qn, turned_k ? kn.transpose(1, 2) : kn};
+}
+std::pair<Tensor, Tensor> l2norm_pair_bwd(const Tensor& q0, const Tensor& k0, const Tensor& dq0, const Tensor& dk0) {
+  bool turned_q, turned_k;
+  const Tensor q = dense(q0, turned_q), k = dense(k0, turned_k);
+  const Tensor gq = (turned_q ? dq0.transpose(1, 2) : dq0).contiguous(), gk = (turned_k ? dk0.transpose(1, 2) : dk0).contiguous();
+  Tensor dq = at::empty_like(q), dk = at::empty_like(k);
+  const int64_t d = q.size(-1);
+  check_status(lnx_l2norm_pair_bwd(ptr(q), ptr(k), ptr(gq), ptr(gk), ptr(dq), ptr(dk), d ? q.numel() / d : 0, (int32_t)d, code_of(q.scalar_type()), stream_of(q)),
+               "lnx_l2norm_pair_bwd");
+  return {turned_q ? dq.transpose(1, 2) : dq, turned_k ? dk.transpose(1, 2) : dk};
+}
+
 struct L2NormFn : Function<L2NormFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x) {
     ctx->save_for_backward({x});
@@ -396,8 +417,8 @@ std::pair<Tensor, Tensor> chunk_forward(const Tensor& q, const Tensor& k, const 
   const bool fused = opt_.l2norm && lnx_chunk_fuses_l2norm(&a);
   a.use_qk_l2norm = fused;
   c.norm_outside = opt_.l2norm && !fused;
-  c.qn = c.norm_outside ? l2norm_fwd(c.q_in) : c.q_in;
-  c.kn = c.norm_outside ? l2norm_fwd(c.k_in) : c.k_in;
+  if (c.norm_outside) std::tie(c.qn, c.kn) = l2norm_pair_fwd(c.q_in, c.k_in);
+  else c.qn = c.q_in, c.kn = c.k_in;
   a.nseq = (int32_t)s.nseq;
   a.token_first = tf;
   a.forward_only = opt_.forward_only;
@@ -463,10 +484,7 @@ struct ChunkFn : Function<ChunkFn> {
       a.d_gate_raw = ptr(dg), a.d_gate_A_log = fptr(dA), a.d_gate_bias = fptr(dbias);
     }
     check_status(lnx_chunk_bwd(&a, stream_of(c.qn)), "lnx_chunk_bwd");
-    if (c.norm_outside) {
-      dq = l2norm_bwd(c.q_in, dq);
-      dk = l2norm_bwd(c.k_in, dk);
-    }
+    if (c.norm_outside) std::tie(dq, dk) = l2norm_pair_bwd(c.q_in, c.k_in, dq, dk);
     auto to = [](const Tensor& t, int64_t type) { return t.defined() ? t.to((at::ScalarType)type) : t; };
     return {dq, dk, dv, to(dg, m[14]), to(dbeta, m[13]), to(ds0, m[15]), to(dA, m[16]), to(dbias, m[17]), Tensor()};
   }
@@ -498,7 +516,7 @@ PyObject* py_chunk_segmented(PyObject*, PyObject* const* args, Py_ssize_t nargs)
   const Tensor sT = at::empty({nseg, rows, s.dk, s.dv}, q.options().dtype(at::kFloat));
   lnx_scan_args a = base_args(1, rows, s.T, s.dk, s.dv, code_of(q.scalar_type()), (int)o_dtype, s.gate, false, in.number(6));
   a.use_qk_l2norm = in.flag(7) && lnx_chunk_fuses_l2norm(&a);
-  if (in.flag(7) && !a.use_qk_l2norm) q = l2norm_fwd(q), k = l2norm_fwd(k);
+  if (in.flag(7) && !a.use_qk_l2norm) std::tie(q, k) = l2norm_pair_fwd(q, k);
   a.token_first = tf, a.forward_only = 1;
   a.q = ptr(q), a.k = ptr(k), a.v = ptr(v), a.beta = fptr(beta), a.g = fptr(g);
   a.initial_state = fptr(s0), a.final_state = fptr(sT), a.o = ptr(o);

@@ -20,6 +20,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 // Host side: records a message for lnx_last_error() and returns `code`.
 int lnx_set_error(int code, const char* fmt, ...);
+int lnx_lds_limit(const void* kernel, size_t bytes);  // raises the kernel's dynamic LDS limit to `bytes`; LNX_OK or an error status
 
 // Host side: when per-kernel timing is enabled (lnx_profile_enable), records a HIP event on
 // `st` before the kernel named `kernel_name`; a NULL name closes the current entry point.
