@@ -81,8 +81,9 @@ struct Scal {
 // operands (K, Q, Tm, Pm rows) come from LDS.  Strips of 16 columns put a slab's chain on twice as many SIMDs as strips of 32:
 // B2 H16 T2007 d128 (32 chunks in a row, 128 workgroups) 65 -> 57 us forward and 74 -> 59 us in reverse, one prompt of 1000
 // tokens 34 -> 29 us, B8 H16 T4096 204 -> 198 and 217 -> 207 us; the bits are those of 32-column strips (Mma16).  What is left of
-// a chunk's 1.7 us there: a SIMD takes 1 KB of LDS reads in about 16 cycles, and a strip reads 60 KB of operands whatever its
-// width; then the movers' conversions of K and Q rows.
+// a chunk's 1.5 us there: a SIMD takes 1 KB of LDS reads in about 16 cycles, and a strip reads 60 KB of operands whatever its
+// width.  The movers convert K and Q rows, 2.5 VALU instructions an element: with eight waves of them instead of four 57 -> 51 us and
+// 29 -> 25 us; in reverse the third wave of each SIMD leaves too few registers (59 -> 59 - 68 us), it keeps four.
 //  All five input tiles are double-buffered, so the movers write chunk
 // n + 1 while chunk n is being read and two barriers per chunk are enough:
 //   B1    buffers of chunk n complete           compute: S^T -> LDS (saved states), Y, Q S, R, D (-> LDS, transposed), O -> LDS
@@ -94,13 +95,13 @@ template <int DK, int BVW> struct FScanL {
   // chain: operand tiles in chain order, rows 32 bytes off a multiple of 64 (Mma16).  64-column slabs are bound by what the
   // movers carry.
   static constexpr bool CHAIN = BVW == 32;
-  static constexpr int BV = BVW, PAD = M::PAD, OPAD = CHAIN ? 16 : 8, LDK = DK + OPAD, LDC = LNX_C + OPAD, LDV = BV + PAD, NCW = BV / 16;
+  static constexpr int BV = BVW, PAD = M::PAD, OPAD = CHAIN ? 16 : 8, LDK = DK + OPAD, LDC = LNX_C + OPAD, LDV = BV + PAD, NCW = BV / 16, MT = CHAIN && DK == 128 ? 512 : 256;
   static constexpr int LDS = DK + PAD, LDD = LNX_C + PAD;  // of the tiles on their way out: states, D or dR
   static constexpr int kK = 64 * LDK, kST = BV * LDS, kV = 64 * LDV, kC = 64 * LDC;
   static constexpr int kDT = BV * LDD;
   // [2] x (K, Q, V, Tm, Pm) | O | S^T | D^T | scalars [2]
   static constexpr size_t bytes = sizeof(T) * (2 * (2 * kK + kV + 2 * kC) + kV + kST + kDT) + sizeof(float) * 2 * Scal::SIZE;
-  static constexpr int threads = 64 * NCW + 256;
+  static constexpr int threads = 64 * NCW + MT;
 };
 
 template <int DK, int GATE, int BVW, typename OT>
@@ -108,6 +109,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
   typedef FScanL<DK, BVW> L;
   constexpr int LDK = L::LDK, LDC = L::LDC, BV = L::BV, LDV = L::LDV, NCW = L::NCW, LDS = L::LDS, LDD = L::LDD;
   constexpr bool CHAIN = L::CHAIN;
+  constexpr int MT = L::MT;  // mover threads
   constexpr int KT = DK / 16;  // row tiles of the state strip
   static_assert(DK == 64 || DK == 128, "dk = 64 or 128");
   extern __shared__ __align__(16) char smem[];
@@ -137,12 +139,12 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
   if (wave >= NCW) {
     // ---------------- movers ----------------
     const int mt = tid - 64 * NCW;
-    typedef TileRegs<T, 64, DK> RowTile;
-    typedef TileRegs<T, 64, BV> ValTile;
+    typedef TileRegs<T, 64, DK, MT> RowTile;
+    typedef TileRegs<T, 64, BV, MT> ValTile;
     struct Tiles {
       RowTile K, Q;
       ValTile V;
-      TriRegs<T, CHAIN> Tm, P;  // lower-triangular tiles, packed in the workspace
+      TriRegs<T, CHAIN, MT> Tm, P;  // lower-triangular tiles, packed in the workspace
       float g, gc, b;  // per-token scalars of token mt % 64
       float fq[RowTile::IT], nk[RowTile::IT];  // factors of the token each of this thread's Q / K vectors belongs to
       float bv[ValTile::IT];  // beta of the token each of its V vectors belongs to
@@ -178,19 +180,19 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
       }
 #pragma unroll
       for (int it = 0; it < RowTile::IT; ++it) {
-        R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
-        R.nk[it] = at<const float>(p.ws, p.off.Nk)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
+        R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + MT * it) / RowTile::VPR];
+        R.nk[it] = at<const float>(p.ws, p.off.Nk)[slot * 64 + (mt + MT * it) / RowTile::VPR];
       }
       R.b = p.beta[tbase + (int64_t)min(t, R.len - 1) * p.geom.ts];
 #pragma unroll
       for (int it = 0; it < ValTile::IT; ++it)
-        R.bv[it] = p.beta[tbase + (int64_t)min(min((mt + 256 * it) / ValTile::VPR, 63), R.len - 1) * p.geom.ts];
+        R.bv[it] = p.beta[tbase + (int64_t)min(min((mt + MT * it) / ValTile::VPR, 63), R.len - 1) * p.geom.ts];
     };
     // K rows normalised (their own bits where nothing is to be normalised), Q rows normalised and scaled by scale e^{G_i}
     auto commit = [&](const Tiles& R, int pb, int part = -1) {
 #pragma unroll
       for (int it = 0; it < RowTile::IT; ++it) {
-        const int idx = mt + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
+        const int idx = mt + MT * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
         if (part < 0 || part == 0)
           S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), p.l2norm ? scaled(R.K.x[it], R.nk[it]) : R.K.x[it]);
         if (part < 0 || part == 1)
@@ -201,7 +203,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
         T* dst = sV + pb * L::kV;
 #pragma unroll
         for (int it = 0; it < ValTile::IT; ++it) {
-          const int idx = mt + 256 * it, r = idx / ValTile::VPR, c = (idx - r * ValTile::VPR) * ValTile::N;
+          const int idx = mt + MT * it, r = idx / ValTile::VPR, c = (idx - r * ValTile::VPR) * ValTile::N;
           typename Vec16<T>::V x = R.V.x[it];
 #pragma unroll
           for (int e = 0; e < ValTile::N; ++e) x[e] = (bf16_t)((float)x[e] * R.bv[it]);
@@ -240,16 +242,19 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
       lds_barrier();  // Bmid
       int tok0, len;
       chunk_span(span, n, tok0, len);
-      if (p.o) {
+      // with 512 movers: O and D are 256 vectors each, one half of the movers takes each
+      const bool lower = MT == 256 || mt < 256, upper = MT == 256 || mt >= 256;
+      const int ot = mt & 255;
+      if (p.o && lower) {
         if constexpr (std::is_same<OT, float>::value)
-          unstage_tile_checked_widen<64, BV>(reinterpret_cast<float*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + v0, tso, sO, LDV, len, mt);
+          unstage_tile_checked_widen<64, BV>(reinterpret_cast<float*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + v0, tso, sO, LDV, len, ot);
         else
-          unstage_tile_checked<bf16_t, 64, BV>(reinterpret_cast<bf16_t*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + v0, tso, sO, LDV, len, mt);
+          unstage_tile_checked<bf16_t, 64, BV>(reinterpret_cast<bf16_t*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + v0, tso, sO, LDV, len, ot);
       }
       if (p.save) {
         const int64_t slot = (int64_t)row * N + n;
-        unstage_tile<T, BV, DK, true>(at<T>(p.ws, p.off.SnT) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sST, LDS, BV, mt);
-        unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT, LDD, BV, mt);
+        unstage_tile<T, BV, DK, true, MT>(at<T>(p.ws, p.off.SnT) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sST, LDS, BV, mt);
+        if (upper) unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT, LDD, BV, ot);
       }
       lds_barrier();  // B1 of the next chunk
     };
@@ -448,13 +453,13 @@ template <int DK, int BVW> struct BScanL {
   // chain: operand tiles in chain order, rows 32 bytes off a multiple of 64 (Mma16).  64-column slabs are bound by what the
   // movers carry.
   static constexpr bool CHAIN = BVW == 32;
-  static constexpr int BV = BVW, PAD = M::PAD, OPAD = CHAIN ? 16 : 8, LDK = DK + OPAD, LDC = LNX_C + OPAD, LDV = BV + PAD, NCW = BV / 16;
+  static constexpr int BV = BVW, PAD = M::PAD, OPAD = CHAIN ? 16 : 8, LDK = DK + OPAD, LDC = LNX_C + OPAD, LDV = BV + PAD, NCW = BV / 16, MT = 256;
   static constexpr int LDS = DK + PAD, LDD = LNX_C + PAD;  // of the tiles on their way out: states, D or dR
   static constexpr int kK = 64 * LDK, kST = BV * LDS, kV = 64 * LDV, kC = 64 * LDC;
   static constexpr int kDT = BV * LDD;
   // [2] x (K, scaled Q, dO, Tm, Pm) | dS'^T | dR^T | dv | scalars [2]
   static constexpr size_t bytes = sizeof(T) * (2 * (2 * kK + kV + 2 * kC) + kST + kDT + kV) + sizeof(float) * 2 * Scal::SIZE;
-  static constexpr int threads = 64 * NCW + 256;
+  static constexpr int threads = 64 * NCW + MT;
 };
 
 template <int DK, int GATE, int BVW>
@@ -462,6 +467,7 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
   typedef BScanL<DK, BVW> L;
   constexpr int LDK = L::LDK, LDC = L::LDC, BV = L::BV, LDV = L::LDV, NCW = L::NCW, LDS = L::LDS, LDD = L::LDD;
   constexpr bool CHAIN = L::CHAIN;
+  constexpr int MT = L::MT;  // mover threads
   constexpr int KT = DK / 16;
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);  // [2][64][LDK]
@@ -490,11 +496,11 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
   if (wave >= NCW) {
     // ---------------- movers ----------------
     const int mt = tid - 64 * NCW;
-    typedef TileRegs<T, 64, DK> RowTile;
+    typedef TileRegs<T, 64, DK, MT> RowTile;
     struct Tiles {
       RowTile K, Q;
-      TileRegs<T, 64, BV> dO;
-      TriRegs<T, CHAIN> Tm, P;  // lower-triangular tiles, packed in the workspace
+      TileRegs<T, 64, BV, MT> dO;
+      TriRegs<T, CHAIN, MT> Tm, P;  // lower-triangular tiles, packed in the workspace
       float g, gc, b;  // per-token scalars of token mt % 64
       float fq[RowTile::IT], nk[RowTile::IT];  // factors of the token each of this thread's Q / K vectors belongs to
       int len;
@@ -525,8 +531,8 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
       }
 #pragma unroll
       for (int it = 0; it < RowTile::IT; ++it) {
-        R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
-        R.nk[it] = at<const float>(p.ws, p.off.Nk)[slot * 64 + (mt + 256 * it) / RowTile::VPR];
+        R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + MT * it) / RowTile::VPR];
+        R.nk[it] = at<const float>(p.ws, p.off.Nk)[slot * 64 + (mt + MT * it) / RowTile::VPR];
       }
       R.b = p.beta[tbase + (int64_t)min(t, R.len - 1) * p.geom.ts];
     };
@@ -534,7 +540,7 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
     auto commit = [&](const Tiles& R, int pb, int part = -1) {
 #pragma unroll
       for (int it = 0; it < RowTile::IT; ++it) {
-        const int idx = mt + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
+        const int idx = mt + MT * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
         if (part < 0 || part == 0)
           S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), p.l2norm ? scaled(R.K.x[it], R.nk[it]) : R.K.x[it]);
         if (part < 0 || part == 1)
@@ -571,7 +577,7 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
       }
       lds_barrier();  // Bmid
       const int64_t slot = (int64_t)row * N + n;
-      unstage_tile<T, BV, DK, true>(at<T>(p.ws, p.off.dSn) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sdST, LDS, BV, mt);
+      unstage_tile<T, BV, DK, true, MT>(at<T>(p.ws, p.off.dSn) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sdST, LDS, BV, mt);
       unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.dD) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sdRT, LDD, BV, mt);
       int tok0, len;
       chunk_span(span, n, tok0, len);

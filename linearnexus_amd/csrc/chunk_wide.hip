@@ -86,13 +86,6 @@ template <int BV> __device__ __forceinline__ bool chain_of(const DirectParams& p
   return true;
 }
 
-// The lane's number again, of unknown origin: what is computed from it is computed where it is used.  Addresses formed outside
-// the loop over the chunks went to scratch memory, and a reload waits for every store issued before it.
-__device__ __forceinline__ int fresh(int lane) {
-  asm volatile("" : "+v"(lane));
-  return lane;
-}
-
 // the gate's scalars of a chunk, by 64 threads
 template <int GATE> __device__ __forceinline__ void put_scalars(float* sc, float g, float gl, float scale, int t) {
   sc[Sc::R + t] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(gl - g, 0.f)) : 1.f;

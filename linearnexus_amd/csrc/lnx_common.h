@@ -75,6 +75,13 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// The lane's number again, of unknown origin: what is computed from it is computed where it is used.  Addresses formed outside
+// the loop over the chunks went to scratch memory, and a reload waits for every store issued before it.
+__device__ __forceinline__ int fresh(int lane) {
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
 // Sum over all 64 lanes; every lane gets the total.
 // Sum over the four lanes of a quad (lanes 4q .. 4q+3), in every lane: two DPP quad permutes, no LDS crossbar.
 __device__ __forceinline__ float quad_sum(float x) {

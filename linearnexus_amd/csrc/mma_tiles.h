@@ -363,8 +363,8 @@ __device__ __forceinline__ typename Vec16<T>::V vec_zero() {
 // registers per load), and no load sits behind a branch or a select -- either would keep the compiler from
 // counting the loads in flight exactly, and it would then make the next tile store wait for (nearly) all of
 // them, younger prefetches included.
-template <typename T, int ROWS, int COLS> struct TileRegs {
-  static constexpr int N = Vec16<T>::N, VPR = COLS / N, TOTAL = ROWS * VPR, IT = (TOTAL + 255) / 256;
+template <typename T, int ROWS, int COLS, int THREADS = 256> struct TileRegs {
+  static constexpr int N = Vec16<T>::N, VPR = COLS / N, TOTAL = ROWS * VPR, IT = (TOTAL + THREADS - 1) / THREADS;
   typename Vec16<T>::V x[IT];
   __device__ __forceinline__ void load(const T* src, int64_t stride, int valid, int tid) {
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -373,7 +373,7 @@ template <typename T, int ROWS, int COLS> struct TileRegs {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(src), 0, bytes, 0x00020000);
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int idx = tid + 256 * it, r = idx / VPR, c = (idx - r * VPR) * N;
+      const int idx = tid + THREADS * it, r = idx / VPR, c = (idx - r * VPR) * N;
       const u32x4 raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)((r * stride + c) * (int64_t)sizeof(T)), 0, 0);
       x[it] = __builtin_bit_cast(typename Vec16<T>::V, raw);
     }
@@ -386,7 +386,7 @@ template <typename T, int ROWS, int COLS> struct TileRegs {
   __device__ __forceinline__ void store(T* dst, int ld, int tid) const {
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int idx = tid + 256 * it, r = idx / VPR, c = (idx - r * VPR) * N;
+      const int idx = tid + THREADS * it, r = idx / VPR, c = (idx - r * VPR) * N;
       if (idx < TOTAL) *reinterpret_cast<typename Vec16<T>::V*>(dst + r * ld + c) = x[it];
     }
   }
@@ -406,30 +406,33 @@ __device__ __forceinline__ void tri_vec_pos(int idx, int& r, int& c) {  // idx <
   r = 8 * g + q;
   c = o - q * (g + 1);
 }
-// The packed tile in the registers of 256 threads (vector tid, and vector 256 + tid for tid < 32) between its global
+// The packed tile in the registers of 256 or 512 threads (vector tid, with 256 also vector 256 + tid for tid < 32) between its global
 // loads and its LDS stores (columns in the order CHAIN of Mma16), like TileRegs; the LDS tile's upper part is zeroed once by the caller and never written.
-template <typename T, bool CHAIN> struct TriRegs {
+template <typename T, bool CHAIN, int THREADS = 256> struct TriRegs {
   static_assert(sizeof(T) == 2, "packed triangles are a 2-byte format");
+  static constexpr bool TWO = THREADS < LNX_TRI_VECS;
   typename Vec16<T>::V x[2];
   int o0, o1;  // LDS element offsets of this thread's two vectors for a leading dimension fixed at init
-  bool second;
+  bool first, second;
   __device__ __forceinline__ void init(int ld, int tid) {
     int r, c;
-    tri_vec_pos(tid, r, c);
+    first = TWO || tid < LNX_TRI_VECS;
+    tri_vec_pos(first ? tid : LNX_TRI_VECS - 1, r, c);
     o0 = r * ld + Mma16::pos<CHAIN>(8 * c);
-    second = tid < LNX_TRI_VECS - 256;
+    second = TWO && tid < LNX_TRI_VECS - 256;
+    if (!TWO) return;
     tri_vec_pos(second ? 256 + tid : LNX_TRI_VECS - 1, r, c);
     o1 = r * ld + Mma16::pos<CHAIN>(8 * c);
   }
   __device__ __forceinline__ void load(const T* src, int tid) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(src), 0, LNX_TRI_VECS * 16, 0x00020000);
+    // threads without a (second) vector read past the end: the range check returns zeros, nothing sits behind a branch
     x[0] = __builtin_bit_cast(typename Vec16<T>::V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * tid, 0, 0));
-    // threads without a second vector read past the end: the range check returns zeros, nothing sits behind a branch
-    x[1] = __builtin_bit_cast(typename Vec16<T>::V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * (256 + tid), 0, 0));
+    if (TWO) x[1] = __builtin_bit_cast(typename Vec16<T>::V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * (256 + tid), 0, 0));
   }
   __device__ __forceinline__ void store(T* dst) const {
-    Mma16::put<CHAIN>(dst + o0, x[0]);
-    if (second) Mma16::put<CHAIN>(dst + o1, x[1]);
+    if (first) Mma16::put<CHAIN>(dst + o0, x[0]);
+    if (TWO && second) Mma16::put<CHAIN>(dst + o1, x[1]);
   }
 };
 
@@ -444,27 +447,27 @@ __device__ __forceinline__ void stage_tile(T* dst, int ld, const T* src, int64_t
 // LDS tile [ROWS][COLS] (leading dimension ld) -> global, 16-byte vectors, rows < valid only.
 // FULL: every row is written and the tile is a whole number of 256-thread passes, so the loads
 // and stores are unconditional and issued as two batches.
-template <typename T, int ROWS, int COLS, bool FULL = false>
+template <typename T, int ROWS, int COLS, bool FULL = false, int THREADS = 256>
 __device__ __forceinline__ void unstage_tile(T* dst, int64_t stride, const T* src, int ld, int valid, int tid) {
   typedef typename Vec16<T>::V V;
-  constexpr int N = Vec16<T>::N, VPR = COLS / N, TOTAL = ROWS * VPR, IT = (TOTAL + 255) / 256;
+  constexpr int N = Vec16<T>::N, VPR = COLS / N, TOTAL = ROWS * VPR, IT = (TOTAL + THREADS - 1) / THREADS;
   if constexpr (FULL) {
-    static_assert(TOTAL % 256 == 0, "whole passes only");
+    static_assert(TOTAL % THREADS == 0, "whole passes only");
     V x[IT];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int idx = tid + 256 * it, r = idx / VPR, c = (idx - r * VPR) * N;
+      const int idx = tid + THREADS * it, r = idx / VPR, c = (idx - r * VPR) * N;
       x[it] = *reinterpret_cast<const V*>(src + r * ld + c);
     }
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int idx = tid + 256 * it, r = idx / VPR, c = (idx - r * VPR) * N;
+      const int idx = tid + THREADS * it, r = idx / VPR, c = (idx - r * VPR) * N;
       *reinterpret_cast<V*>(dst + r * stride + c) = x[it];
     }
   } else {
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int idx = tid + 256 * it, r = idx / VPR, c = (idx - r * VPR) * N;
+      const int idx = tid + THREADS * it, r = idx / VPR, c = (idx - r * VPR) * N;
       if (idx < TOTAL && r < valid) *reinterpret_cast<V*>(dst + r * stride + c) = *reinterpret_cast<const V*>(src + r * ld + c);
     }
   }
