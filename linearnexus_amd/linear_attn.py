@@ -283,20 +283,35 @@ def _chunk_forward(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_s
 _CHUNK_DK = (64, 128, 256)  # key head dimensions the chunk kernels are built for
 
 
-def _prefill_segments(B: int, H: int, T: int, dv: int) -> int:
+def _prefill_segments(B: int, H: int, T: int, dv: int, dk: int = 256, two_byte: bool = True, vector_gate: bool = False) -> int:
     """How many segments a forward-only call is cut into (1: not at all).  The sequential kernels have one workgroup
-    per (batch, head, 64 value columns); a single long prompt leaves most of the 256 CUs without one.  Segments are run
-    as independent sequences -- see _segmented_forward -- for three times the scan work spread over nseg times the
-    workgroups, so it pays when at most an eighth of the CUs would be busy and every segment keeps >= 64 chunks:
-    measured 2.11 -> 0.84 ms for one 65536-token prompt with 4 heads of 128, 4.64 -> 3.36 ms for 131072 tokens with
-    16 heads.  LNX_PREFILL_SEGMENTS forces a count (0 or 1: never)."""
+    per (batch, head, 32 or 64 value columns); a few long prompts leave most of the 256 CUs without one.  Segments are run
+    as independent sequences -- see _segmented_forward -- which is three times the scan work over nseg times the
+    workgroups and one short step per segment.  LNX_PREFILL_SEGMENTS forces a count (0 or 1: never).
+
+    dk <= 128: the first pass has w = B H (dk + dv) / 64 workgroups per segment, so 256 / w segments fill the chip once.
+    Segments of 16 chunks or more, but eight of them where the chip has room (a segment's step costs as much as two chunks).
+    The lines are where the measured gain starts, bf16 d128 unless said: 4 heads of 4096 tokens 90 -> 74 us (2048: 52 -> 62),
+    8 heads of 16384 332 -> 168, 16 heads (w = 64) of 8192 182 -> 158 (4096: 98 -> 101), 32 heads never.  The kernels that form
+    W and U prepare both passes: no gain at w = 64; fp32 4 heads of 4096 284 -> 194 us, bf16 per-channel gate 4 heads
+    of 8192 237 -> 163 (4096: 131 -> 133).  From 512 chunks on, w = 64 gains from a second round (32768 tokens: 541 -> 508).
+
+    dk = 256: at most an eighth of the CUs busy and every segment keeps >= 64 chunks (fewer heads of 512 values gain
+    less than their longer preparation costs: 16 workgroups of 4096 tokens 196 -> 216 us)."""
     forced = os.environ.get("LNX_PREFILL_SEGMENTS")
+    chunks = -(-T // CHUNK)
     if forced is not None:
-        return max(1, min(int(forced), -(-T // CHUNK)))
-    wide = B * H * -(-dv // 64)
-    if wide > 32 or T < 16384 * max(1, wide // 16):  # measured: no gain at 32 workgroups x 16384 tokens, loss at 64
+        return max(1, min(int(forced), chunks))
+    if dk > 128:
+        wide = B * H * -(-dv // 64)
+        if wide > 32 or T < 16384 * max(1, wide // 16):  # measured: no gain at 32 workgroups x 16384 tokens, loss at 64
+            return 1
+        return max(1, min(256 // wide, T // 4096))
+    direct = two_byte and not vector_gate
+    w = B * H * (-(-dk // 64) + -(-dv // 64))
+    if w > (64 if direct else 32) or chunks < (64 if (direct and w <= 32) or not two_byte else 128):
         return 1
-    return max(1, min(256 // wide, T // 4096))
+    return min((512 if w > 32 and chunks >= 512 else 256) // w, max(8, chunks // 16))
 
 
 def _segmented_forward(q, k, v, g, beta, scale, initial_state, l2norm, o_dtype, nseg):
@@ -328,7 +343,10 @@ def _chunk(q, k, v, g, beta, scale, initial_state, chunk_size, l2norm, o_dtype, 
     forward_only = not _wants_grad(q, k, v, g, beta, initial_state)
     if dkp is None or q.dim() != 4 or (dkp, dvp) == (dk, dv):
         if forward_only and dkp is not None and q.dim() == 4 and cu_seqlens is None:
-            nseg = _prefill_segments(q.shape[0], q.shape[1], q.shape[2], dv)
+            # batch rows become heads: free for contiguous tensors, a copy of the token-first views of several rows
+            folds = q.shape[0] == 1 or (q.is_contiguous() and k.is_contiguous() and v.is_contiguous())
+            nseg = _prefill_segments(q.shape[0], q.shape[1], q.shape[2], dv, dk if folds else 256, q.element_size() == 2,
+                                     g is not None and g.dim() == 4 and g.shape[-1] == dk)
             if nseg > 1:
                 return _segmented_forward(q, k, v, g, beta, scale, initial_state, l2norm, o_dtype, nseg)
         return _chunk_forward(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens, forward_only=forward_only)[:2]
