@@ -3,25 +3,35 @@
 // The token-by-token scan (dplr.hip) is one dependent step of some 270 wave instructions per token on the one or two waves
 // that a (batch, head) row has.  Over a chunk the recurrence is a linear map of the state, so everything but a 64 x 64
 // product per chunk can be done for all chunks at once, on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands and
-// accumulation, nothing is rounded below the token kernels' precision).
+// accumulation, no operand is rounded to less).
 //
-// Per chunk, G = cumulative gk, Gp the same before the token's own decay, E_ts = exp(G_t - G_s) per channel:
-//   Aab = stril(<a_t e^Gp_t, b_s e^-G_s>)  Aak = stril(<a_t e^Gp_t, k_s e^-G_s>)  Pqb, Pqk = tril(<q_t e^G_t, b_s / k_s e^-G_s>)
-//   Tm = (I - Aab)^-1     u = Tm (a e^Gp h + Aak v)     o = q e^G h + Pqb u + Pqk v     h' = e^G_C h + (b e^(G_C-G))^T u + (k e^(G_C-G))^T v
-// and with W = Tm (a e^Gp), U0 = Tm Aak v:
-//   o = X h + Y,  X = q e^G + Pqb W,  Y = Pqb U0 + Pqk v          h' = M h + N,  M = e^G_C + Bg^T W,  N = Bg^T U0 + Kg^T v
+// Per chunk, w = e^gk, E_ts = product of w over the tokens after s up to and with t, per channel; e_t = E from the chunk's start, r_s = E
+// to its end, and t- the token before t (a token's own decay comes after its a):
+//   Aab = stril(<a_t E_t-s, b_s>)  Aak = stril(<a_t E_t-s, k_s>)  Pqb, Pqk = tril(<q_t E_ts, b_s / k_s>)
+//   Tm = (I - Aab)^-1     u = Tm (a e_t- h + Aak v)     o = q e_t h + Pqb u + Pqk v     h' = e_C h + (b r)^T u + (k r)^T v
+// and with W = Tm (a e_t-), U0 = Tm Aak v:
+//   o = X h + Y,  X = q e + Pqb W,  Y = Pqb U0 + Pqk v          h' = M h + N,  M = e_C + (b r)^T W,  N = (b r)^T U0 + (k r)^T v
 // Backward: D = gradient of the state leaving the chunk, R = X^T dO; the gradient of the state entering it is M^T D + R, and
-//   dU = Tm^T (Pqb^T dO + Bg D)      dv = Pqk^T dO + Kg D + Aak^T dU
+//   dU = Tm^T (Pqb^T dO + b r D)      dv = Pqk^T dO + k r D + Aak^T dU
 //   dPqb = tril(dO u^T)  dPqk = tril(dO v^T)  dAab = stril(dU u^T)  dAak = stril(dU v^T), and from these the vectors' gradients;
-//   dgk_t = <D, h'>_c + sum_{t' >= t} (q dq + a da - b db - k dk)_t' - (a da)_t   (how each exponential depends on G).
+//   dgk_t = <D, h'>_c + sum_{t' >= t} (q dq + a da - b db - k dk)_t' - (a da)_t   (how each decay depends on gk).
 //
-// The factors e^(G_t - G_s) <= 1 are split as e^(G_t - m) e^(m - G_s) around the middle m of the chunk's range of G, one m
-// per channel.  RWKV-7's decays are above exp(-0.607) per token, so |G - m| <= 20 and both factors are harmless; a chunk in
-// which any channel's range exceeds LNX_DPLR_RANGE evaluates its pairs one by one from the difference instead (a uniform
-// branch per chunk: exact for any decay, and some 20 us per workgroup slower).
+// Decays are products and never differences of rounded sums: a float sum of gates over 64 tokens is rounded to its own size, which costs
+// the decays of later tokens 4e-7 of their value inside RWKV-7's range and all of it behind a large negative gate (a caller without
+// cu_seqlens ends a document inside a row that way).  A block of 16 tokens is a row of 16 lanes; it has P_t, the decay from before the
+// block's first token to token t, and S_s, that of the tokens after s.  A pair in two blocks has E = P_t (whole blocks between) S_s:
+// factors of the path from s to t, so any decay down to 0 (gk = -inf) gives what the token kernels give.  A pair inside a block has
+// E = P_t / P_s.  P, S and 1 / P come from sums in fixed point, which are exact; a block whose P leave 2^+-60 (RWKV-7's decays are above
+// exp(-0.607), 2^-14 over a block) multiplies its decays up as floats and takes its 120 pairs one by one (a uniform branch per wave, DIRECT
+// below: B8 H16 T4096 forward and backward 2.2 ms without such blocks, 6.4 ms where all are).
 //
-// Kernels, each a workgroup per chunk but for the two sequential passes.  Measured at B8 H16 T4096 bf16 (8192 chunks):
-// see the table at the launch functions.
+// Sums that carry the recent tokens' large terms take the far ones first, and a sum of two products is added up from two chains: what
+// comes second on one chain would be rounded at the size of the whole, 64 times.  Errors against fp64, relative 2-norms, one row of 512
+// tokens with RWKV-7's decays (behind a reset of any size the same), in brackets the token kernels: o 1.2e-7 (1.0), h 0.7e-7 (0.6), dq,
+// dk, dv 1.7, 1.8, 1.2e-7 (0.9), da, db 2.2e-7 (1.3), dgk 5.5e-7 (1.2), dh0 1.1e-7 (0.8); with gates a hundredth of that o 2.5e-7 (4.7),
+// gradients 2.3 - 4.4e-7 (4.7 - 7.4): there the token kernels round the state at every token.
+//
+// Kernels, each a workgroup per chunk but for the two sequential passes: the launch functions name them with their times.
 #include "lnx_common.h"
 #include "chunk_common.h"
 
@@ -31,7 +41,7 @@ constexpr int C = 64, D = 64;       // tokens of a chunk, channels of a head
 constexpr int LD = LNX_LDA;         // leading dimension of the fp32 tiles in LDS: 68 floats, rows 4 banks apart
 constexpr int TS = C * LD;          // floats of a tile in LDS
 constexpr int TG = C * D;           // floats of a tile in the workspace
-constexpr float RANGE = 80.f;       // widest range of G that the split around its middle may span: e^40 e^-40 in each factor
+constexpr int RANGE = 60;           // products of decays of a block's first tokens lie within 2^+-RANGE, or the block is DIRECT
 
 struct ChunkParams {
   const void *q, *k, *v, *a, *b;
@@ -64,13 +74,19 @@ __device__ __forceinline__ Slot slot_of(const ChunkParams& p) {
   return s;
 }
 
-// e^x with the rounding of x log2(e) carried along: the factors' exponents reach 40, where the plain product's rounding is
-// already 2e-6 of the result.
+// e^x with the rounding of x log2(e) carried along, 0 for -inf and whatever underflows.  The correction is that of a clamped x: of x
+// near the lowest float or -inf its own would be inf - inf.
 __device__ __forceinline__ float exp_f(float x) {
   float t = x * 1.44269504f;
-  asm volatile("" : "+v"(t));  // -ffast-math must not see that the next line is a rounding error
-  const float e = __builtin_fmaf(x, 1.44269504f, -t) + x * 1.92596299e-8f;
+  const float y = fmaxf(x, -128.f);
+  float ty = y * 1.44269504f;
+  asm volatile("" : "+v"(t), "+v"(ty));  // -ffast-math must not see that the next line is a rounding error
+  const float e = __builtin_fmaf(y, 1.44269504f, -ty) + y * 1.92596299e-8f;
   return __builtin_amdgcn_exp2f(t) * (1.f + 0.69314718f * e);
+}
+__device__ __forceinline__ float rcp_f(float x) {  // one Newton step on the instruction's estimate
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.f), r, r);
 }
 
 // ---- products of 16 x 16 tiles ------------------------------------------------------------------------------------
@@ -88,6 +104,24 @@ __device__ __forceinline__ void mfma4(floatx4& c, floatx4 a, floatx4 b) {
   for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
 }
 __device__ __forceinline__ floatx4 zero4() { return floatx4{0.f, 0.f, 0.f, 0.f}; }
+// c[i] += a_i b_i over a block of 16 of the contraction, N sums in turn so that no product waits for the one before it
+template <int N, typename F, typename G> __device__ __forceinline__ void mfma4_each(floatx4* const (&c)[N], F&& a, G&& b) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int i = 0; i < N; ++i) *c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a(i)[r], b(i)[r], *c[i], 0, 0, 0);
+}
+// ... the block summed from zero: for the pairs' sums over channels, where one chain of 64 additions rounds the outputs by 1.5e-7 at RWKV-7's
+// decays and four chains of 16 by 1.1e-7 (all else exact).  Not in dplr_grad, whose registers are full: 775 -> 980 us for dq 1.7 -> 1.25e-7.
+template <int N, typename F, typename G> __device__ __forceinline__ void mfma_block(floatx4* const (&c)[N], F&& a, G&& b) {
+  floatx4 t[N];
+  floatx4* pt[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) t[i] = zero4(), pt[i] = &t[i];
+  mfma4_each<N>(pt, a, b);
+#pragma unroll
+  for (int i = 0; i < N; ++i) *c[i] += t[i];
+}
 
 // Four waves, each with a block of 16 tokens (of rows of the state tiles); the lane's token is t, its channels in block cb
 // are 16 cb + 4 g + 0..3.  Sums over earlier tokens make blocks 0 .. j work, sums over later ones j .. 3: the workgroups that
@@ -102,8 +136,8 @@ struct Lane {
   }
 };
 
-// Blocks 0 .. j, or 3 .. j, as constants: the accumulators stay where they are when a wave leaves early (a branch around each
-// block's products made the compiler copy them, 1000 moves among 850 products)
+// Blocks 0 .. j, 3 .. j, and those without j, as constants: the accumulators stay where they are when a wave leaves early (a branch
+// around each block's products made the compiler copy them, 1000 moves among 850 products)
 template <int B> struct Int {
   static constexpr int value = B;
 };
@@ -124,6 +158,22 @@ template <typename F> __device__ __forceinline__ void downto(int j, F&& f) {
   f(Int<1>{});
   if (j == 1) return;
   f(Int<0>{});
+}
+template <typename F> __device__ __forceinline__ void before(int j, F&& f) {
+  if (j == 0) return;
+  f(Int<0>{});
+  if (j == 1) return;
+  f(Int<1>{});
+  if (j == 2) return;
+  f(Int<2>{});
+}
+template <typename F> __device__ __forceinline__ void after(int j, F&& f) {
+  if (j == 3) return;
+  f(Int<3>{});
+  if (j == 2) return;
+  f(Int<2>{});
+  if (j == 1) return;
+  f(Int<1>{});
 }
 
 // Four consecutive elements as loaded
@@ -169,165 +219,231 @@ __device__ __forceinline__ void clear(floatx4 (&c)[4]) {
 }
 
 // ---- decays --------------------------------------------------------------------------------------------------
-struct Gates {      // arrays of 64 floats in LDS
-  float *em, *ec, *eC, *gm;  // e^m, e^(G_C - m), e^G_C, m
-  int* wide;                 // some channel's range is too wide for the split: pairs one by one, em = ec = 1
+// of another lane in the row of 16 (CTRL: a DPP control), 1 where there is none
+template <int CTRL> __device__ __forceinline__ floatx4 neighbour(floatx4 x) {
+  floatx4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = __int_as_float(__builtin_amdgcn_update_dpp(0x3f800000, __float_as_int(x[e]), CTRL, 0xF, 0xF, false));
+  return r;
+}
+__device__ __forceinline__ floatx4 token_before(floatx4 x) { return neighbour<0x111>(x); }
+__device__ __forceinline__ floatx4 token_after(floatx4 x) { return neighbour<0x101>(x); }
+// Products over the row of 16 lanes up to and with the lane's own, and from it on
+__device__ __forceinline__ floatx4 product_upto(floatx4 x) {  // row_shr 1, 2, 4, 8
+  x *= neighbour<0x111>(x);
+  x *= neighbour<0x112>(x);
+  x *= neighbour<0x114>(x);
+  return x * neighbour<0x118>(x);
+}
+__device__ __forceinline__ floatx4 product_from(floatx4 x) {  // row_shl
+  x *= neighbour<0x101>(x);
+  x *= neighbour<0x102>(x);
+  x *= neighbour<0x104>(x);
+  return x * neighbour<0x108>(x);
+}
+
+constexpr int LDS_TILES = 4;
+constexpr unsigned LDS_BYTES = (LDS_TILES * TS + 5 * 64 + 32 * 36) * sizeof(float);
+static_assert(LDS_BYTES <= 80 * 1024, "two workgroups per CU");
+struct Lds {
+  float *base, *total, *one;  // total: [4][64], decays of the whole blocks; one: 64 ones
+  float* sx;                  // 32 x 36 floats
+  __device__ __forceinline__ Lds(char* smem) {
+    base = reinterpret_cast<float*>(smem);
+    total = base + LDS_TILES * TS, one = total + 256, sx = one + 64;
+  }
+  __device__ __forceinline__ float* tile(int i) const { return base + i * TS; }
+  // Decays of the whole blocks between two, e < l: blocks 1 and 2 are the only ones that can lie between others.  One of the two is a
+  // constant; `at`: channel.  No branch: a block that is not in between reads ones.
+  template <int E> __device__ __forceinline__ floatx4 from(int l, int at) const { return between4(E, l, at, E < 1, E < 2); }
+  template <int L> __device__ __forceinline__ floatx4 to(int e, int at) const { return between4(e, L, at, L > 1, L > 2); }
+  template <int E> __device__ __forceinline__ float from1(int l, int at) const { return between1(E, l, at, E < 1, E < 2); }
+  template <int L> __device__ __forceinline__ float to1(int e, int at) const { return between1(e, L, at, L > 1, L > 2); }
+  __device__ __forceinline__ const float* if_between(int e, int m, int l) const { return e < m && m < l ? total + 64 * m : one; }
+  __device__ __forceinline__ floatx4 between4(int e, int l, int at, bool m1, bool m2) const {
+    floatx4 x = {1.f, 1.f, 1.f, 1.f};
+    if (m1) x = load4(if_between(e, 1, l) + at);
+    if (m2) x *= load4(if_between(e, 2, l) + at);
+    return x;
+  }
+  __device__ __forceinline__ float between1(int e, int l, int at, bool m1, bool m2) const {
+    float x = 1.f;
+    if (m1) x = if_between(e, 1, l)[at];
+    if (m2) x *= if_between(e, 2, l)[at];
+    return x;
+  }
+  // Decays from the chunk's start to block j, and from its end to the chunk's
+  __device__ __forceinline__ floatx4 start_to(int j, int at) const { return load4((j > 0 ? total : one) + at) * load4(if_between(0, 1, j) + at) * load4(if_between(0, 2, j) + at); }
+  __device__ __forceinline__ floatx4 end_from(int j, int at) const { return load4(if_between(j, 1, 3) + at) * load4(if_between(j, 2, 3) + at) * load4((j < 3 ? total + 192 : one) + at); }
+  __device__ __forceinline__ float start_to1(int j, int c) const { return (j > 0 ? total : one)[c] * if_between(0, 1, j)[c] * if_between(0, 2, j)[c]; }
+  __device__ __forceinline__ float end_from1(int j, int c) const { return if_between(j, 1, 3)[c] * if_between(j, 2, 3)[c] * (j < 3 ? total + 192 : one)[c]; }
+  // ... from the end of each block, of one channel, and of the whole chunk
+  __device__ __forceinline__ void ends(int c, float (&r)[4], float& chunk) const {
+    r[3] = 1.f, r[2] = total[192 + c], r[1] = r[2] * total[128 + c], r[0] = r[1] * total[64 + c], chunk = r[0] * total[c];
+  }
 };
 
-// Gt: gk of the chunk on entry ([t][c], visible after the first barrier), its cumulative sum on return; scr: 768 floats
-__device__ __forceinline__ void cumulate(float* Gt, float* scr, const Gates& s) {
-  const int tid = threadIdx.x, c = tid & 63, seg = tid >> 6;
-  lds_barrier();
-  float v[16], sum = 0.f;
+// The gates of the lane's block.  Sums of gates in fixed point (2^-24 in units of log 2) are exact: P and S carry the rounding of one
+// exponential each, whatever the sums' sizes.  A gate or a sum that the format does not hold, or NaN, makes the block DIRECT.
+constexpr int ONE = 1 << 24;
+__device__ __forceinline__ int fixed_gate(float g, float& size) {
+  const float c = 1.44269504f * ONE;
+  float t = g * c;
+  asm volatile("" : "+v"(t));  // -ffast-math must not see that the next line is a rounding error
+  const float e = __builtin_fmaf(g, 1.92596299e-8f * ONE, __builtin_fmaf(g, c, -t));
+  size = fabsf(t);
+  return (int)__builtin_rintf(t + e);
+}
+__device__ __forceinline__ float exp2_fixed(int x) { return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((float)(x & (ONE - 1)) * (1.f / ONE)), x >> 24); }
+template <int CTRL> __device__ __forceinline__ int dpp_of(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, true); }
+struct Gates {
+  int sum[4][4];  // from the block's first token up to and with the lane's
+  bool direct;
+  __device__ __forceinline__ explicit Gates(const Row<float>& gk) {
+    bool fits = true;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) v[i] = (sum += Gt[(16 * seg + i) * LD + c]);
-  scr[64 * seg + c] = sum;
-  lds_barrier();
-  float pre = 0.f;
-  for (int j = 0; j < seg; ++j) pre += scr[64 * j + c];
-  float mx = 0.f, mn = 0.f;  // the token before the chunk has G = 0
+    for (int cb = 0; cb < 4; ++cb) {
+      const floatx4 g = gk[cb];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const float x = pre + v[i];
-    Gt[(16 * seg + i) * LD + c] = x;
-    mx = fmaxf(mx, x), mn = fminf(mn, x);
+      for (int e = 0; e < 4; ++e) {
+        float size;
+        int x = fixed_gate(g[e], size);
+        fits = fits && size <= 8.f * ONE;  // sixteen of them stay below 2^31
+        x += dpp_of<0x111>(x), x += dpp_of<0x112>(x), x += dpp_of<0x114>(x), x += dpp_of<0x118>(x);  // row_shr 1, 2, 4, 8
+        fits = fits && abs(x) <= RANGE * ONE;
+        sum[cb][e] = x;
+      }
+    }
+    direct = __ballot(!fits) != 0;
   }
-  scr[256 + 64 * seg + c] = mx;
-  scr[512 + 64 * seg + c] = mn;
-  lds_barrier();
-  if (seg == 0) {
+  __device__ __forceinline__ floatx4 upto(int cb) const {  // P
+    floatx4 r;
 #pragma unroll
-    for (int j = 1; j < 4; ++j) mx = fmaxf(mx, scr[256 + 64 * j + c]), mn = fminf(mn, scr[512 + 64 * j + c]);
-    const bool wide = __ballot(!(mx - mn <= RANGE)) != 0;
-    const float m = 0.5f * (mx + mn), last = Gt[(C - 1) * LD + c];
-    s.gm[c] = m;
-    s.em[c] = wide ? 1.f : exp_f(m);
-    s.ec[c] = wide ? 1.f : exp_f(last - m);
-    s.eC[c] = exp_f(last);
-    if (c == 0) *s.wide = wide;
+    for (int e = 0; e < 4; ++e) r[e] = exp2_fixed(sum[cb][e]);
+    return r;
   }
-  lds_barrier();
+  __device__ __forceinline__ floatx4 upto_inverse(int cb) const {  // 1 / P
+    floatx4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = exp2_fixed(-sum[cb][e]);
+    return r;
+  }
+  __device__ __forceinline__ floatx4 behind(int cb) const {  // S
+    floatx4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = exp2_fixed(dpp_of<0x15F>(sum[cb][e]) - sum[cb][e]);  // row_newbcast:15
+    return r;
+  }
+};
+// The decays of a DIRECT block's tokens, one by one
+__device__ __forceinline__ void token_decays(const ChunkParams& p, const Slot& s, const Lane& w, floatx4 (&x)[4]) {
+  Row<float> gk;
+  gk.load(p.gk, (s.tok + w.t) * D + 4 * w.g, w.t < s.len);
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const floatx4 g = gk[cb];
+    x[cb] = floatx4{exp_f(g[0]), exp_f(g[1]), exp_f(g[2]), exp_f(g[3])};
+  }
+}
+struct Decay {
+  floatx4 p[4], s[4];
+  __device__ __forceinline__ Decay(const Gates& g, const ChunkParams& c, const Slot& sl, const Lane& w) {
+    if (!g.direct) {
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) p[cb] = g.upto(cb), s[cb] = g.behind(cb);
+    } else {
+      floatx4 x[4];
+      token_decays(c, sl, w, x);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) p[cb] = product_upto(x[cb]), s[cb] = product_from(token_after(x[cb]));
+    }
+  }
+};
+// The whole block's, for the other waves (visible after a barrier)
+__device__ __forceinline__ void put_total(const Lds& L, const Lane& w, int cb, floatx4 p) {
+  if (w.l16 == 15) store4(L.total + 64 * w.j + 16 * cb + 4 * w.g, p);
 }
 
-__device__ __forceinline__ floatx4 rcp4(floatx4 x) {  // of e^x, |x| <= RANGE / 2
-  return floatx4{__builtin_amdgcn_rcpf(x[0]), __builtin_amdgcn_rcpf(x[1]), __builtin_amdgcn_rcpf(x[2]), __builtin_amdgcn_rcpf(x[3])};
-}
-__device__ __forceinline__ floatx4 exp4(floatx4 x) { return floatx4{exp_f(x[0]), exp_f(x[1]), exp_f(x[2]), exp_f(x[3])}; }
-
-// The lane's row of q, k, a, b and of the cumulative gate
+// The lane's row of q, k, a, b and its gates
 template <typename T> struct Own {
   Row<T> q, k, a, b;
-  floatx4 G[4];
-  __device__ __forceinline__ void load(const ChunkParams& p, const Slot& s, const Lane& w, float* Gt) {
+  Row<float> gk;
+  __device__ __forceinline__ void load(const ChunkParams& p, const Slot& s, const Lane& w) { load_gates(p, s, w), load_rows(p, s, w); }
+  __device__ __forceinline__ void load_gates(const ChunkParams& p, const Slot& s, const Lane& w) { gk.load(p.gk, (s.tok + w.t) * D + 4 * w.g, w.t < s.len); }
+  __device__ __forceinline__ void load_rows(const ChunkParams& p, const Slot& s, const Lane& w) {
     const bool ok = w.t < s.len;
     const int64_t at = (s.tok + w.t) * D + 4 * w.g;
-    Row<float> g;
-    g.load(p.gk, at, ok);
     q.load(p.q, at, ok);
     a.load(p.a, at, ok);
     b.load(p.b, at, ok);
     k.load(p.k, at, ok);
-    put_row(Gt, w, [&](int cb) { return g[cb]; });
-  }
-  __device__ __forceinline__ void gates(const float* Gt, const Lane& w) {  // Gt: the cumulative sums
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-      G[cb] = load4(Gt + w.t * LD + 16 * cb + 4 * w.g);
-    }
   }
 };
-// e^(G - m), e^(Gp - m) and e^(m - G), or e^G, e^Gp and e^(G_C - G) in a wide chunk, of the lane's channels
-struct Decay {
-  floatx4 q[4], a[4], b[4];
-  __device__ __forceinline__ Decay(const floatx4 (&G)[4], const floatx4 (&Gp)[4], const float* last, const Gates& s, const Lane& w, bool wide) {
-    if (!wide) {
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        const floatx4 m = load4(s.gm + 16 * cb + 4 * w.g);
-        q[cb] = exp4(G[cb] - m), a[cb] = exp4(Gp[cb] - m), b[cb] = rcp4(q[cb]);
-      }
-    } else {
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) q[cb] = exp4(G[cb]), a[cb] = exp4(Gp[cb]), b[cb] = exp4(load4(last + 16 * cb + 4 * w.g) - G[cb]);
-    }
-  }
-};
-__device__ __forceinline__ void gates_before(floatx4 (&Gp)[4], const float* Gt, const Lane& w) {  // of the token before the lane's
-#pragma unroll
-  for (int cb = 0; cb < 4; ++cb) {
-    const floatx4 x = load4(Gt + max(w.t - 1, 0) * LD + 16 * cb + 4 * w.g);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) Gp[cb][e] = w.t ? x[e] : 0.f;
-  }
-}
 
-// Wide chunk: the pair (t, s) of Aab, Aak, Pqb, Pqk from the difference of the gates, the vectors from memory
-struct Pair {
-  float ab, ak, qb, qk;
+// DIRECT block: its pairs one by one.  The lane has four pairs, of tokens l16 and 4 g + r; BY_T: l16 is the later one.  The vectors come
+// from memory, the decays w from the wave's rows of `own`.
+struct Pairs {
+  floatx4 ab, ak, qb, qk;
 };
-template <typename T> __device__ __forceinline__ Pair wide_pair(const ChunkParams& p, int64_t tok, int len, const float* Gt, int t, int s) {
-  Pair r{0.f, 0.f, 0.f, 0.f};
-  if (s > t || t >= len) return r;
-  const T *q = static_cast<const T*>(p.q) + (tok + t) * D, *a = static_cast<const T*>(p.a) + (tok + t) * D;
-  const T *b = static_cast<const T*>(p.b) + (tok + s) * D, *k = static_cast<const T*>(p.k) + (tok + s) * D;
-  for (int c = 0; c < D; ++c) {
-    const float G = Gt[s * LD + c], eq = p.scale * to_f32(q[c]) * exp_f(Gt[t * LD + c] - G), vb = to_f32(b[c]), vk = to_f32(k[c]);
-    r.qb += eq * vb;
-    r.qk += eq * vk;
-    if (s < t) {
-      const float ea = to_f32(a[c]) * exp_f(Gt[(t - 1) * LD + c] - G);
-      r.ab += ea * vb;
-      r.ak += ea * vk;
-    }
-  }
-  return r;
-}
-
-// What `pair(o, x)` gives of the lane's pairs with tokens o = 16 b + 4 g + r, through the lane's own places of N tiles
-template <int N, typename F> __device__ __forceinline__ void wide_pairs(floatx4 (*const (&m)[N])[4], float* const (&tile)[N], const Lane& w, F&& pair) {
+template <typename T, bool BY_T> __device__ __forceinline__ Pairs direct_pairs(const ChunkParams& p, const Slot& sl, const Lane& w, const float* own) {
+  auto row = [&](const void* base, int i, int c) {
+    Raw4<T> x;
+    const bool ok = 16 * w.j + i < sl.len;
+    x.load(static_cast<const T*>(base) + (ok ? (sl.tok + 16 * w.j + i) * D + c : 0));
+    return ok ? x.get() : zero4();
+  };
+  auto dot = [](floatx4 x, floatx4 y) { return x[0] * y[0] + x[1] * y[1] + x[2] * y[2] + x[3] * y[3]; };
+  Pairs m{zero4(), zero4(), zero4(), zero4()};
 #pragma unroll 1
-  for (int e = 0; e < 16; ++e) {
-    const int o = 16 * (e >> 2) + 4 * w.g + (e & 3);
-    float x[N];
-    pair(o, x);
+  for (int c = 0; c < D; c += 4) {
+    floatx4 e[4], el[4];  // E of the later token and of the one before it
 #pragma unroll
-    for (int i = 0; i < N; ++i) tile[i][w.t * LD + o] = x[i];
-  }
+    for (int r = 0; r < 4; ++r) e[r] = el[r] = floatx4{1.f, 1.f, 1.f, 1.f};
+#pragma unroll 1
+    for (int i = 1; i < 16; ++i) {
+      const floatx4 x = load4(own + (16 * w.j + i) * LD + c);
 #pragma unroll
-  for (int i = 0; i < N; ++i)
+      for (int r = 0; r < 4; ++r) {
+        const int t = BY_T ? w.l16 : 4 * w.g + r, s = BY_T ? 4 * w.g + r : w.l16;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) (*m[i])[b] = load4(tile[i] + w.t * LD + 16 * b + 4 * w.g);
-}
-
-// Blocks of a lower-triangular pair matrix M[t][s].  `ByT`: tile sb <= j holds rows s, columns t = the wave's tokens; ByS: tile
-// tb >= j rows t, columns s = the wave's tokens.  Entries above the diagonal (STRICT: on it, too) are cleared.
-template <bool BY_T, bool STRICT> __device__ __forceinline__ void mask(floatx4 (&m)[4], const Lane& w) {
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const bool diagonal = b == w.j;
+        for (int n = 0; n < 4; ++n) {
+          e[r][n] *= i > s && i <= t ? x[n] : 1.f;
+          el[r][n] *= i > s && i < t ? x[n] : 1.f;
+        }
+      }
+    }
+    const floatx4 f1 = row(BY_T ? p.a : p.b, w.l16, c), f2 = row(BY_T ? p.q : p.k, w.l16, c);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = 4 * w.g + r, t = BY_T ? w.l16 : row, s = BY_T ? row : w.l16;
-      m[b][r] = (diagonal && (STRICT ? s >= t : s > t)) ? 0.f : m[b][r];
+      const int o = 4 * w.g + r;
+      const floatx4 h1 = row(BY_T ? p.b : p.a, o, c), h2 = row(BY_T ? p.k : p.q, o, c);
+      const floatx4 a = BY_T ? f1 : h1, q = p.scale * (BY_T ? f2 : h2), b = BY_T ? h1 : f1, k = BY_T ? h2 : f2;
+      const int t = BY_T ? w.l16 : o, s = BY_T ? o : w.l16;
+      if (s < t) m.ab[r] += dot(a * el[r], b), m.ak[r] += dot(a * el[r], k);
+      if (s <= t) m.qb[r] += dot(q * e[r], b), m.qk[r] += dot(q * e[r], k);
     }
   }
+  return m;
 }
 
-constexpr int LDS_TILES = 4;
-constexpr unsigned LDS_BYTES = (LDS_TILES * TS + 4 * 64 + 4 + 32 * 36) * sizeof(float);
-static_assert(LDS_BYTES <= 80 * 1024, "two workgroups per CU");
-struct Lds {
-  float* base;
-  Gates gate;
-  float* sx;  // 32 x 36 floats
-  __device__ __forceinline__ Lds(char* smem) {
-    base = reinterpret_cast<float*>(smem);
-    float* x = base + LDS_TILES * TS;
-    gate = Gates{x, x + 64, x + 128, x + 192, reinterpret_cast<int*>(x + 256)};
-    sx = x + 260;
+// A block of a lower-triangular pair matrix M[t][s] on the diagonal.  BY_T: rows s, columns t, else rows t, columns s.  Entries above the
+// diagonal (STRICT: on it, too) are cleared.
+template <bool BY_T, bool STRICT> __device__ __forceinline__ void mask(floatx4& m, const Lane& w) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = 4 * w.g + r, t = BY_T ? w.l16 : row, s = BY_T ? row : w.l16;
+    m[r] = (STRICT ? s >= t : s > t) ? 0.f : m[r];
   }
-  __device__ __forceinline__ float* tile(int i) const { return base + i * TS; }
-};
+}
+// The wave's rows of a lower-triangular matrix: what lies before block j, the block itself, zeros
+template <typename F> __device__ __forceinline__ void put_tri(float* tile, const Lane& w, const floatx4 (&x)[3], floatx4 d, F&& value) {
+#pragma unroll
+  for (int sb = 0; sb < 4; ++sb) {
+    floatx4 y = sb == w.j ? d : zero4();
+    if (sb < 3) y = sb < w.j ? x[sb < 3 ? sb : 0] : y;
+    store4(tile + w.t * LD + 16 * sb + 4 * w.g, value(y));
+  }
+}
 
 // ---- forward: M, X, N^T, Y of a chunk ------------------------------------------------------------------------
 template <typename T>
@@ -339,60 +455,69 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
   const int l16 = w.l16, g = w.g, g4 = 4 * w.g;
   float *tb = L.tile(0), *tk = L.tile(1), *ta = L.tile(2), *tx = L.tile(3);
   Own<T> x;
-  x.load(p, s, w, tx);
+  x.load(p, s, w);
   Row<T> v;
   v.load(p.v, (s.tok + w.t) * D + g4, w.t < s.len);
-  cumulate(tx, L.sx, L.gate);
-  x.gates(tx, w);
-  const bool wide = *L.gate.wide;
-  floatx4 xx[4];  // q with its factor, then X^T: rows = channels, columns = tokens
-  floatx4 ab[4], ak[4], qb[4], qk[4];
-  clear(ab), clear(ak), clear(qb), clear(qk);
+  floatx4 fq[4], fa[4];                // q P, a P of the token before
+  floatx4 ab[3], ak[3], qb[3], qk[3];  // pairs with tokens of earlier blocks, by t
+  Pairs m{zero4(), zero4(), zero4(), zero4()};  // and of the lane's own
+#pragma unroll
+  for (int i = 0; i < 3; ++i) ab[i] = ak[i] = qb[i] = qk[i] = zero4();
   {
-    floatx4 fa[4], fb[4], fk[4];
-    {
-      floatx4 Gp[4];
-      gates_before(Gp, tx, w);
-      const Decay e(x.G, Gp, tx + (C - 1) * LD, L.gate, w, wide);
+    const Gates gates(x.gk);
+    const Decay e(gates, p, s, w);
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) xx[cb] = p.scale * x.q[cb] * e.q[cb], fa[cb] = x.a[cb] * e.a[cb], fb[cb] = x.b[cb] * e.b[cb], fk[cb] = x.k[cb] * e.b[cb];
-    }
-    if (wide) {
-      wide_pairs<2>({&ab, &ak}, {tb, tk}, w, [&](int o, float* r) { const Pair y = wide_pair<T>(p, s.tok, s.len, tx, w.t, o); r[0] = y.ab, r[1] = y.ak; });
-      wide_pairs<2>({&qb, &qk}, {tb, tk}, w, [&](int o, float* r) { const Pair y = wide_pair<T>(p, s.tok, s.len, tx, w.t, o); r[0] = y.qb, r[1] = y.qk; });
-    }
-    put_cols(ta, w, fa), put_cols(tb, w, fb), put_cols(tk, w, fk);
-    lds_barrier();
-    if (!wide) {
-      upto(w.j, [&](auto sb_) {
-        constexpr int sb = decltype(sb_)::value;
+    for (int cb = 0; cb < 4; ++cb) put_total(L, w, cb, e.p[cb]);
+    if (threadIdx.x < 64) L.one[threadIdx.x] = 1.f;
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-          const floatx4 rb = frag<true>(tb, 16 * sb + l16, 16 * kb + g4), rk = frag<true>(tk, 16 * sb + l16, 16 * kb + g4);
+    for (int cb = 0; cb < 4; ++cb) fq[cb] = p.scale * x.q[cb] * e.p[cb], fa[cb] = x.a[cb] * token_before(e.p[cb]);
+    if (!gates.direct) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {  // four accumulators in turn: no product waits for the one before it
-            ab[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb[r], fa[kb][r], ab[sb], 0, 0, 0);
-            ak[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(rk[r], fa[kb][r], ak[sb], 0, 0, 0);
-            qb[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb[r], xx[kb][r], qb[sb], 0, 0, 0);
-            qk[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(rk[r], xx[kb][r], qk[sb], 0, 0, 0);
-          }
-        }
-      });
-      mask<true, true>(ab, w), mask<true, true>(ak, w), mask<true, false>(qb, w), mask<true, false>(qk, w);
+      for (int cb = 0; cb < 4; ++cb) {
+        const floatx4 r = gates.upto_inverse(cb), b = x.b[cb] * r, k = x.k[cb] * r;
+        mfma_block<4>({&m.ab, &m.ak, &m.qb, &m.qk}, [&](int i) { return i & 1 ? k : b; }, [&](int i) { return i & 2 ? fq[cb] : fa[cb]; });
+      }
+      mask<true, true>(m.ab, w), mask<true, true>(m.ak, w), mask<true, false>(m.qb, w), mask<true, false>(m.qk, w);
+    } else {
+      floatx4 decays[4];
+      token_decays(p, s, w, decays);
+      put_cols(tx, w, decays);
+      __builtin_amdgcn_wave_barrier();
+      m = direct_pairs<T, true>(p, s, w, tx);
+      __builtin_amdgcn_wave_barrier();
     }
+    put_row(tb, w, [&](int cb) { return x.b[cb] * e.s[cb]; });
+    put_row(tk, w, [&](int cb) { return x.k[cb] * e.s[cb]; });
+    put_row(tx, w, [&](int cb) { return v[cb]; });
   }
-  lds_barrier();  // the gates have been read
-  put_row(tx, w, [&](int cb) { return v[cb]; });
   lds_barrier();
+  before(w.j, [&](auto sb_) {
+    constexpr int sb = decltype(sb_)::value;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      const floatx4 rb = frag<true>(tb, 16 * sb + l16, 16 * kb + g4), rk = frag<true>(tk, 16 * sb + l16, 16 * kb + g4), gap = L.from<sb>(w.j, 16 * kb + g4);
+      const floatx4 ra = fa[kb] * gap, rq = fq[kb] * gap;
+      mfma_block<4>({&ab[sb], &ak[sb], &qb[sb], &qk[sb]}, [&](int i) { return i & 1 ? rk : rb; }, [&](int i) { return i & 2 ? rq : ra; });
+    }
+  });
+  floatx4 xx[4];  // q e, then X^T: rows = channels, columns = tokens
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const floatx4 st = L.start_to(w.j, 16 * cb + g4);
+    xx[cb] = fq[cb] * st;
+    store4(ta + w.t * LD + 16 * cb + g4, fa[cb] * st);  // a e of the token before
+  }
+  float end[4], chunk;  // decays of channel w.t from the end of each block
+  L.ends(w.t, end, chunk);
   floatx4 nt[4], z[4], y[4];  // N (rows i, columns n), Aak v (rows t, columns n), Y^T (rows n, columns t)
   clear(nt), clear(z), clear(y);
 #pragma unroll
   for (int sb = 0; sb < 4; ++sb) {
-    const floatx4 kf = frag<false>(tk, 16 * w.j + l16, 16 * sb + g4);
+    const floatx4 kf = frag<false>(tk, 16 * w.j + l16, 16 * sb + g4) * end[sb];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) mfma4(nt[nb], kf, frag<false>(tx, 16 * nb + l16, 16 * sb + g4));
   }
-  upto(w.j, [&](auto sb_) {
+  before(w.j, [&](auto sb_) {
     constexpr int sb = decltype(sb_)::value;
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
@@ -401,9 +526,14 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
       mfma4(y[nb], vf, qk[sb]);
     }
   });
-  lds_barrier();
 #pragma unroll
-  for (int sb = 0; sb < 4; ++sb) store4(tx + w.t * LD + 16 * sb + g4, sb <= w.j ? -ab[sb] : zero4());
+  for (int nb = 0; nb < 4; ++nb) {
+    const floatx4 vf = frag<false>(tx, 16 * nb + l16, 16 * w.j + g4);
+    mfma4(z[nb], m.ak, vf);
+    mfma4(y[nb], vf, m.qk);
+  }
+  lds_barrier();
+  put_tri(tx, w, ab, m.ab, [](floatx4 y_) { return -y_; });
   put_rows(tk, w, z);
   lds_barrier();
   tri_inverse_64<true>(tx, tx, L.sx, threadIdx.x);
@@ -424,40 +554,40 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
     put_rows(tk, w, u);
   }
   lds_barrier();
-  floatx4 m[4];  // M[i][c]: rows c, columns i
-  clear(m);
+  floatx4 mm[4];  // M[i][c]: rows c, columns i
+  floatx4 ntu[4], xw[4], yu[4];  // what W and U0 add to N, X and Y
+  clear(mm), clear(ntu), clear(xw), clear(yu);
 #pragma unroll
   for (int sb = 0; sb < 4; ++sb) {
-    const floatx4 bf = frag<false>(tb, 16 * w.j + l16, 16 * sb + g4);
+    const floatx4 bf = frag<false>(tb, 16 * w.j + l16, 16 * sb + g4) * end[sb];
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {
       const floatx4 wf = frag<true>(ta, 16 * cb + l16, 16 * sb + g4), uf = frag<true>(tk, 16 * cb + l16, 16 * sb + g4);
-      mfma4(m[cb], wf, bf);
-      mfma4(nt[cb], bf, uf);
+      mfma4(mm[cb], wf, bf);
+      mfma4(ntu[cb], bf, uf);
     }
   }
-  upto(w.j, [&](auto sb_) {
+  before(w.j, [&](auto sb_) {
     constexpr int sb = decltype(sb_)::value;
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {
-      mfma4(xx[cb], frag<true>(ta, 16 * cb + l16, 16 * sb + g4), qb[sb]);
-      mfma4(y[cb], frag<true>(tk, 16 * cb + l16, 16 * sb + g4), qb[sb]);
+      mfma4(xw[cb], frag<true>(ta, 16 * cb + l16, 16 * sb + g4), qb[sb]);
+      mfma4(yu[cb], frag<true>(tk, 16 * cb + l16, 16 * sb + g4), qb[sb]);
     }
   });
-  const float eci = L.gate.ec[w.t], eCi = L.gate.eC[w.t];
-  const floatx4 ec4 = load4(L.gate.ec + 16 * w.j + g4);
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) {
-    const floatx4 em = load4(L.gate.em + 16 * cb + g4);
-    floatx4 r = m[cb] * em * eci;
+    mfma4(xw[cb], frag<true>(ta, 16 * cb + l16, 16 * w.j + g4), m.qb);
+    mfma4(yu[cb], frag<true>(tk, 16 * cb + l16, 16 * w.j + g4), m.qb);
+    floatx4 r = mm[cb];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (16 * cb + g4 + e == w.t) r[e] += eCi;
+      if (16 * cb + g4 + e == w.t) r[e] += chunk;
     const int at = w.t * D + 16 * cb + g4;
     store4(p.M + s.kept * TG + at, r);
-    store4(p.X + s.kept * TG + at, xx[cb] * em);
-    store4(p.s2 + s.win * TG + at, y[cb]);
-    store4(p.s1 + s.win * TG + (16 * cb + l16) * D + 16 * w.j + g4, nt[cb] * ec4);
+    store4(p.X + s.kept * TG + at, xx[cb] + xw[cb]);
+    store4(p.s2 + s.win * TG + at, y[cb] + yu[cb]);
+    store4(p.s1 + s.win * TG + (16 * cb + l16) * D + 16 * w.j + g4, nt[cb] + ntu[cb]);
   }
 }
 
@@ -511,7 +641,7 @@ __global__ __launch_bounds__(256) void dplr_chunk_scan_kernel(ScanParams p) {
     for (int b = 0; b < 4; ++b) f[b] = load4(cur + 16 * b);
     fetch(next, i + 3);
     store4(Srow + chunk(i) * TG, h);
-    floatx4 y0 = x.a, y1 = zero4();
+    floatx4 y0 = zero4(), y1 = zero4();
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
@@ -519,7 +649,7 @@ __global__ __launch_bounds__(256) void dplr_chunk_scan_kernel(ScanParams p) {
         y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[2 * b][r], f[2 * b][r], y0, 0, 0, 0);
         y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[2 * b + 1][r], f[2 * b + 1][r], y1, 0, 0, 0);
       }
-    h = y0 + y1;
+    h = (y0 + y1) + x.a;
     store4(buf[(i + 1) & 1] + l16 * LD + r0, h);
   };
   fetch(x0, 0);
@@ -554,16 +684,16 @@ __global__ __launch_bounds__(256) void dplr_out_kernel(ChunkParams p) {
   const float* Y = p.s2 + s.win * TG + t * D + 4 * g;
   const float* h = p.hT + s.st * TG + l16 * D + 4 * g;
   if (16 * wave >= s.len) return;
-  floatx4 x[4], acc[4];
+  floatx4 x[4], y[4], acc[4];
 #pragma unroll
-  for (int b = 0; b < 4; ++b) x[b] = load4(X + 16 * b), acc[b] = load4(Y + 16 * b);
+  for (int b = 0; b < 4; ++b) x[b] = load4(X + 16 * b), y[b] = load4(Y + 16 * b), acc[b] = zero4();
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) mfma4(acc[nb], load4(h + 16 * nb * D + 16 * kb), x[kb]);
   if (t < s.len) {
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) store_row4<T>(p.o, (s.tok + t) * D + 16 * nb + 4 * g, acc[nb]);
+    for (int nb = 0; nb < 4; ++nb) store_row4<T>(p.o, (s.tok + t) * D + 16 * nb + 4 * g, acc[nb] + y[nb]);
   }
 }
 
@@ -584,7 +714,7 @@ __global__ __launch_bounds__(256) void dplr_r_kernel(ChunkParams p) {
   floatx4 acc[4];
   clear(acc);
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
+  for (int kb = 3; kb >= 0; --kb) {  // the chunk's first tokens, whose share is the largest, last
     const floatx4 a = frag<false>(tX, w.t, 16 * kb + g4);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) mfma4(acc[nb], a, frag<false>(tO, 16 * nb + l16, 16 * kb + g4));
@@ -604,75 +734,79 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   const int l16 = w.l16, g4 = 4 * w.g;
   float *tb = L.tile(0), *tk = L.tile(1), *ta = L.tile(2), *tx = L.tile(3);
   Own<T> x;
-  x.load(p, s, w, tx);
+  x.load(p, s, w);
   Row<T> v, d_o;
   v.load(p.v, (s.tok + w.t) * D + g4, w.t < s.len);
   d_o.load(p.d_o, (s.tok + w.t) * D + g4, w.t < s.len);
   Row<float> h0, dC;
   h0.load(p.hT, s.st * TG + w.t * D + g4);
   dC.load(p.s1, s.win * TG + w.t * D + g4);
-  cumulate(tx, L.sx, L.gate);
-  x.gates(tx, w);
-  const bool wide = *L.gate.wide;
-  floatx4 fa[4], fb[4], fk[4];  // the lane's row with its factors
-  floatx4 ab[4], akT[4];        // Aab, Aak by t
-  floatx4 ak[4], qb[4], qk[4];  // Aak, Pqb, Pqk by s
-  clear(ab), clear(akT), clear(ak), clear(qb), clear(qk);
+  floatx4 fa[4], fb[4], fk[4];  // the lane's row: a P of the token before, b S, k S
+  floatx4 ab[3], akT[3];        // Aab, Aak by t, with earlier blocks
+  floatx4 ak[3], qb[3], qk[3];  // Aak, Pqb, Pqk by s, with later blocks (of block i + 1)
+  floatx4 abd = zero4(), akTd = zero4(), akd = zero4(), qbd = zero4(), qkd = zero4();  // the lane's own block
+#pragma unroll
+  for (int i = 0; i < 3; ++i) ab[i] = akT[i] = ak[i] = qb[i] = qk[i] = zero4();
   {
+    const Gates gates(x.gk);
+    const Decay e(gates, p, s, w);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) put_total(L, w, cb, e.p[cb]);
+    if (threadIdx.x < 64) L.one[threadIdx.x] = 1.f;
     floatx4 fq[4];
-    {
-      floatx4 Gp[4];
-      gates_before(Gp, tx, w);
-      const Decay e(x.G, Gp, tx + (C - 1) * LD, L.gate, w, wide);
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) fq[cb] = p.scale * x.q[cb] * e.q[cb], fa[cb] = x.a[cb] * e.a[cb], fb[cb] = x.b[cb] * e.b[cb], fk[cb] = x.k[cb] * e.b[cb];
+    for (int cb = 0; cb < 4; ++cb)
+      fq[cb] = p.scale * x.q[cb] * e.p[cb], fa[cb] = x.a[cb] * token_before(e.p[cb]), fb[cb] = x.b[cb] * e.s[cb], fk[cb] = x.k[cb] * e.s[cb];
+    if (!gates.direct) {
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) {
+        const floatx4 r = gates.upto_inverse(cb), b = x.b[cb] * r, k = x.k[cb] * r;
+        mfma_block<5>({&abd, &akTd, &akd, &qbd, &qkd}, [&](int i) { return i == 0 ? b : i == 1 ? k : i == 2 ? fa[cb] : fq[cb]; },
+                      [&](int i) { return i < 2 ? fa[cb] : i == 3 ? b : k; });
+      }
+      mask<true, true>(abd, w), mask<true, true>(akTd, w), mask<false, true>(akd, w), mask<false, false>(qbd, w), mask<false, false>(qkd, w);
+    } else {
+      floatx4 decays[4];
+      token_decays(p, s, w, decays);
+      put_cols(tx, w, decays);
+      __builtin_amdgcn_wave_barrier();
+      const Pairs byt = direct_pairs<T, true>(p, s, w, tx), bys = direct_pairs<T, false>(p, s, w, tx);
+      abd = byt.ab, akTd = byt.ak, akd = bys.ak, qbd = bys.qb, qkd = bys.qk;
+      __builtin_amdgcn_wave_barrier();
     }
-    if (!wide) {
-      put_cols(ta, w, fa), put_cols(tb, w, fb), put_cols(tk, w, fk);
-      lds_barrier();  // the gates have been read
-      put_cols(tx, w, fq);
-      lds_barrier();
-    }
+    put_cols(ta, w, fa), put_cols(tb, w, fb), put_cols(tk, w, fk), put_cols(tx, w, fq);
   }
-  if (!wide) {
-    upto(w.j, [&](auto b_) {
-      constexpr int b = decltype(b_)::value;
+  lds_barrier();
+  before(w.j, [&](auto b_) {
+    constexpr int b = decltype(b_)::value;
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const floatx4 rb = frag<true>(tb, 16 * b + l16, 16 * kb + g4), rk = frag<true>(tk, 16 * b + l16, 16 * kb + g4);
+    for (int kb = 0; kb < 4; ++kb) {
+      const floatx4 rb = frag<true>(tb, 16 * b + l16, 16 * kb + g4), rk = frag<true>(tk, 16 * b + l16, 16 * kb + g4), ra = fa[kb] * L.from<b>(w.j, 16 * kb + g4);
+      mfma_block<2>({&ab[b], &akT[b]}, [&](int i) { return i ? rk : rb; }, [&](int) { return ra; });
+    }
+  });
+  after(w.j, [&](auto b_) {
+    constexpr int b = decltype(b_)::value;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          ab[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb[r], fa[kb][r], ab[b], 0, 0, 0);
-          akT[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(rk[r], fa[kb][r], akT[b], 0, 0, 0);
-        }
-      }
-    });
-    downto(w.j, [&](auto b_) {
-      constexpr int b = decltype(b_)::value;
+    for (int kb = 0; kb < 4; ++kb) {
+      const floatx4 ra = frag<true>(ta, 16 * b + l16, 16 * kb + g4), rq = frag<true>(tx, 16 * b + l16, 16 * kb + g4), gap = L.to<b>(w.j, 16 * kb + g4);
+      const floatx4 rk = fk[kb] * gap, rb = fb[kb] * gap;
+      mfma_block<3>({&ak[b - 1], &qb[b - 1], &qk[b - 1]}, [&](int i) { return i ? rq : ra; }, [&](int i) { return i == 1 ? rb : rk; });
+    }
+  });
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const floatx4 ra = frag<true>(ta, 16 * b + l16, 16 * kb + g4), rq = frag<true>(tx, 16 * b + l16, 16 * kb + g4);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          ak[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[r], fk[kb][r], ak[b], 0, 0, 0);
-          qb[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(rq[r], fb[kb][r], qb[b], 0, 0, 0);
-          qk[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(rq[r], fk[kb][r], qk[b], 0, 0, 0);
-        }
-      }
-    });
-    mask<true, true>(ab, w), mask<true, true>(akT, w), mask<false, true>(ak, w), mask<false, false>(qb, w), mask<false, false>(qk, w);
-  } else {
-    wide_pairs<2>({&ab, &akT}, {tb, tk}, w, [&](int o, float* r) { const Pair y = wide_pair<T>(p, s.tok, s.len, tx, w.t, o); r[0] = y.ab, r[1] = y.ak; });
-    wide_pairs<3>({&ak, &qb, &qk}, {tb, tk, ta}, w, [&](int o, float* r) { const Pair y = wide_pair<T>(p, s.tok, s.len, tx, o, w.t); r[0] = y.ak, r[1] = y.qb, r[2] = y.qk; });
+  for (int cb = 0; cb < 4; ++cb) {  // from here on relative to the chunk's start and end
+    const floatx4 en = L.end_from(w.j, 16 * cb + g4);
+    fa[cb] *= L.start_to(w.j, 16 * cb + g4), fb[cb] *= en, fk[cb] *= en;
   }
   lds_barrier();
   float *th = ta, *tO = tb, *tD = tk, *tv = tx;
   put_row(tv, w, [&](int cb) { return v[cb]; });
   put_row(tO, w, [&](int cb) { return d_o[cb]; });
-  put_row(th, w, [&](int cb) { return h0[cb] * load4(L.gate.em + 16 * cb + g4); });  // e^m h, [value column][channel]
-  put_row(tD, w, [&](int cb) { return dC[cb] * load4(L.gate.ec + 16 * cb + g4); });  // e^(G_C - m) D, [value column][channel]
+  put_row(th, w, [&](int cb) { return h0[cb]; });  // [value column][channel]
+  put_row(tD, w, [&](int cb) { return dC[cb]; });
   lds_barrier();
-  floatx4 z[4], y[4], dv[4];  // a h + Aak v, Bg D + Pqb^T dO (rows t, columns n), dv (rows n, columns t)
+  floatx4 z[4], y[4], dv[4];  // a h + Aak v, b r D + Pqb^T dO (rows t, columns n), dv (rows n, columns t)
   clear(z), clear(y), clear(dv);
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb)
@@ -683,24 +817,30 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
       mfma4(y[nb], fb[kb], df);
       mfma4(dv[nb], df, fk[kb]);
     }
-  upto(w.j, [&](auto b_) {
+  before(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) mfma4(z[nb], akT[b], frag<false>(tv, 16 * nb + l16, 16 * b + g4));
   });
-  downto(w.j, [&](auto b_) {
+  after(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       const floatx4 of = frag<false>(tO, 16 * nb + l16, 16 * b + g4);
-      mfma4(y[nb], qb[b], of);
-      mfma4(dv[nb], of, qk[b]);
+      mfma4(y[nb], qb[b - 1], of);
+      mfma4(dv[nb], of, qk[b - 1]);
     }
   });
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    const floatx4 of = frag<false>(tO, 16 * nb + l16, 16 * w.j + g4);
+    mfma4(z[nb], akTd, frag<false>(tv, 16 * nb + l16, 16 * w.j + g4));
+    mfma4(y[nb], qbd, of);
+    mfma4(dv[nb], of, qkd);
+  }
   lds_barrier();
   float *Tm = tx, *tz = ta, *ty = tk, *tdu = tb;
-#pragma unroll
-  for (int sb = 0; sb < 4; ++sb) store4(Tm + w.t * LD + 16 * sb + g4, sb <= w.j ? -ab[sb] : zero4());
+  put_tri(Tm, w, ab, abd, [](floatx4 x_) { return -x_; });
   put_rows(tz, w, z);
   put_rows(ty, w, y);
   lds_barrier();
@@ -727,220 +867,306 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   }
   put_cols(tdu, w, du);
   lds_barrier();
-  downto(w.j, [&](auto b_) {
+  floatx4 dva[4];  // Aak^T dU
+  clear(dva);
+  after(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) mfma4(dv[nb], frag<false>(tdu, 16 * nb + l16, 16 * b + g4), ak[b]);
+    for (int nb = 0; nb < 4; ++nb) mfma4(dva[nb], frag<false>(tdu, 16 * nb + l16, 16 * b + g4), ak[b - 1]);
   });
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) mfma4(dva[nb], frag<false>(tdu, 16 * nb + l16, 16 * w.j + g4), akd);
   if (w.t < s.len) {
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) store_row4<T>(p.dv, (s.tok + w.t) * D + 16 * nb + g4, dv[nb]);
+    for (int nb = 0; nb < 4; ++nb) store_row4<T>(p.dv, (s.tok + w.t) * D + 16 * nb + g4, dv[nb] + dva[nb]);
   }
 }
 
 // ---- backward: dq, dk, da, db, dgk of a chunk ----------------------------------------------------------------
-// Wide chunk: what the matrices Mb, Mk (which pair b and k with q: LAG 0, or with a, whose decay lags by its own token: LAG 1) add to
-// the gradients of the lane's token: d1 (q or a), db, dk, four channels from ch.
-template <typename T, int LAG>
-__device__ __forceinline__ void wide_grads(const ChunkParams& p, int64_t tok, int len, const float* Mb, const float* Mk, const float* Gt, int t, int ch,
-                                                     floatx4& d1, floatx4& db, floatx4& dk) {
-  auto row = [&](const void* base, int i) { Raw4<T> x; x.load(static_cast<const T*>(base) + (tok + min(i, len - 1)) * D + ch); return i < len ? x.get() : zero4(); };
-  auto gate = [&](int i) { return i < 0 ? zero4() : load4(Gt + i * LD + ch); };
-  const floatx4 G = gate(t), Gl = gate(t - LAG);
-  for (int i = 0; i <= t - LAG; ++i) d1 += exp4(Gl - gate(i)) * (Mb[t * LD + i] * row(p.b, i) + Mk[t * LD + i] * row(p.k, i));
-  for (int i = t + LAG; i < C; ++i) {
-    const floatx4 e = exp4(gate(i - LAG) - G) * (LAG ? row(p.a, i) : p.scale * row(p.q, i));
-    db += e * Mb[i * LD + t];
-    dk += e * Mk[i * LD + t];
+// DIRECT block: what the pairs of the block add to the gradients of the lane's token, four channels from ch.  The matrices lie in LDS rows
+// of the wave ([t][s]); E of consecutive partners is a running product of decays, which are formed again from the gates.
+template <typename T> struct DirectRows {
+  const ChunkParams& p;
+  const Slot& sl;
+  const Lane& w;
+  __device__ __forceinline__ floatx4 operator()(const void* base, int i, int ch) const {
+    Raw4<T> x;
+    const bool ok = 16 * w.j + i < sl.len;
+    x.load(static_cast<const T*>(base) + (ok ? (sl.tok + 16 * w.j + i) * D + ch : 0));
+    return ok ? x.get() : zero4();
+  }
+  __device__ __forceinline__ floatx4 decay(int i, int ch) const {
+    const bool ok = 16 * w.j + i < sl.len;
+    const floatx4 g = load4(p.gk + (ok ? (sl.tok + 16 * w.j + i) * D + ch : 0));
+    return ok ? floatx4{exp_f(g[0]), exp_f(g[1]), exp_f(g[2]), exp_f(g[3])} : floatx4{1.f, 1.f, 1.f, 1.f};
+  }
+};
+// of earlier tokens to dq and da; m: the lane's row with dPqb, dPqk, dAab, dAak at columns 0, 16, 32, 48
+template <typename T> __device__ __forceinline__ void direct_sinks(const DirectRows<T>& row, const float* m, int ch, floatx4& dq, floatx4& da) {
+  const int t = row.w.l16;
+  floatx4 e = {1.f, 1.f, 1.f, 1.f}, el = e;
+#pragma unroll 1
+  for (int s = 15; s >= 0; --s) {
+    const floatx4 b = row(row.p.b, s, ch), k = row(row.p.k, s, ch), x = row.decay(s, ch);
+    if (s <= t) {
+      dq += e * (m[s] * b + m[16 + s] * k);
+      e *= x;
+    }
+    if (s < t) {
+      da += el * (m[32 + s] * b + m[48 + s] * k);
+      el *= x;
+    }
+  }
+}
+// of later tokens to db and dk; m: the lane's column of the block's matrices, which lie at columns 0, 16, 32, 48
+template <typename T> __device__ __forceinline__ void direct_sources(const DirectRows<T>& row, const float* m, int ch, floatx4& db, floatx4& dk) {
+  const int s = row.w.l16;
+  floatx4 e = {1.f, 1.f, 1.f, 1.f}, el = e;
+#pragma unroll 1
+  for (int t = 0; t < 16; ++t) {
+    const floatx4 q = row.p.scale * row(row.p.q, t, ch), a = row(row.p.a, t, ch), x = row.decay(t, ch);
+    const float* mt = m + t * LD;
+    if (t > s) {
+      e *= x;
+      db += el * a * mt[32], dk += el * a * mt[48];
+      el *= x;
+    }
+    if (t >= s) db += e * q * mt[0], dk += e * q * mt[16];
   }
 }
 
+// Over the tokens of the lane's block, from its own on (inclusive) / before its own: each step is one addition with a DPP operand
+template <int CTRL> __device__ __forceinline__ floatx4 dpp_add(floatx4 x) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x[e]), CTRL, 0xF, 0xF, true));
+  return x;
+}
+__device__ __forceinline__ floatx4 sum_from(floatx4 x) { return dpp_add<0x108>(dpp_add<0x104>(dpp_add<0x102>(dpp_add<0x101>(x)))); }  // row_shl 1, 2, 4, 8
+__device__ __forceinline__ floatx4 sum_upto(floatx4 x) { return dpp_add<0x118>(dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(x)))); }  // row_shr
+__device__ __forceinline__ floatx4 sum_block(floatx4 x) { return dpp_add<0x128>(dpp_add<0x124>(dpp_add<0x122>(dpp_add<0x121>(x)))); }  // row_ror
+
+// dgk_t is what flows through the decay of token t: pairs of a source (b or k of a token before t, the state entering) and a sink (q of t or
+// later, a of a later token, the state's gradient).  The formula at the top takes it from sums over the rest of the chunk, where a pair
+// behind t is added at its sink and taken away at its source, and all of their roundings stay (8.8e-7 of dgk against 7.4e-7, the rest as it
+// was then).  Here only pairs inside a block of 16 are treated that way; pairs of two blocks are sums of sinks from t on and of sources
+// before t, and what passes a whole block is <D, h'> less the sources and plus the sinks of the blocks behind it.
 template <typename T>
 __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
   extern __shared__ __align__(16) char smem[];
   const Lds L(smem);
   const Slot s = slot_of(p);
   const Lane w;
-  const int tid = threadIdx.x, l16 = w.l16, g4 = 4 * w.g;
+  const int l16 = w.l16, g4 = 4 * w.g;
   float *t0 = L.tile(0), *t1 = L.tile(1), *t2 = L.tile(2), *t3 = L.tile(3);
-  float* red = L.sx + 768;  // [4][64]: partial sums of <D, h'> per channel
+  float *tin = L.sx, *tout = L.sx + 256, *red = L.sx + 512;  // [4][64] per channel: the blocks' sinks and sources, parts of <D, h'>
   const int64_t at = (s.tok + w.t) * D + g4, wt = s.win * TG + w.t * D + g4, ht = s.st * TG + w.t * D + g4;
   const bool ok = w.t < s.len;
   Own<T> x;
   Row<T> v, d_o;
   Row<float> u, du;
   {
-    Row<float> hC, dC;
+    Row<float> h0, hC, dC;
     hC.load(p.hT, ht + TG);
     dC.load(p.s1, wt);
-    x.load(p, s, w, t3);
+    x.load(p, s, w);
     v.load(p.v, at, ok);
     d_o.load(p.d_o, at, ok);
     u.load(p.s3, wt);
     du.load(p.s4, wt);
-    put_row(t0, w, [&](int cb) { return dC[cb] * hC[cb]; });
-  }
-  cumulate(t3, L.sx, L.gate);
-  x.gates(t3, w);
-  {
-    const int c = tid & 63, seg = tid >> 6;
-    float sum = 0.f;
+    h0.load(p.hT, ht);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) sum += t0[(16 * seg + i) * LD + c];
-    red[64 * seg + c] = sum;
+    for (int cb = 0; cb < 4; ++cb) {  // the wave's sixteen value columns
+      const floatx4 y = sum_block(dC[cb] * hC[cb]);
+      if (l16 == 0) store4(red + 64 * w.j + 16 * cb + g4, y);
+    }
+    put_row(t0, w, [&](int cb) { return v[cb]; });
+    put_row(t2, w, [&](int cb) { return u[cb]; });
+    put_row(t1, w, [&](int cb) { return h0[cb]; });  // states: [value column][channel]
+    put_row(t3, w, [&](int cb) { return dC[cb]; });
   }
-  const bool wide = *L.gate.wide;
-  float* edge = L.sx;  // G of the blocks' last tokens
-  edge[tid] = t3[(16 * (tid >> 6) + 15) * LD + (tid & 63)];
+  Gates gates(x.gk);
+  if (!gates.direct) {
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) put_total(L, w, cb, gates.upto(cb));
+  } else {
+    floatx4 y[4];
+    token_decays(p, s, w, y);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) put_total(L, w, cb, product_upto(y[cb]));
+  }
+  if (threadIdx.x < 64) L.one[threadIdx.x] = 1.f;
   lds_barrier();
-  put_row(t0, w, [&](int cb) { return v[cb]; });
-  put_row(t2, w, [&](int cb) { return u[cb]; });
-  lds_barrier();
-  floatx4 pb[4], pk[4], nb_[4], nk[4];  // dPqb, dPqk, dAab, dAak by t
-  clear(pb), clear(pk), clear(nb_), clear(nk);
-  upto(w.j, [&](auto sb_) {
+  floatx4 pb[3], pk[3], nb_[3], nk[3];          // dPqb, dPqk, dAab, dAak by t, with earlier blocks
+  Pairs m{zero4(), zero4(), zero4(), zero4()};  // of the lane's own block
+#pragma unroll
+  for (int i = 0; i < 3; ++i) pb[i] = pk[i] = nb_[i] = nk[i] = zero4();
+  before(w.j, [&](auto sb_) {
     constexpr int sb = decltype(sb_)::value;
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
-      const floatx4 fu = frag<true>(t2, 16 * sb + l16, 16 * kb + g4), fv = frag<true>(t0, 16 * sb + l16, 16 * kb + g4);
-      const floatx4 fo = d_o[kb], fd = du[kb];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        pb[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(fu[r], fo[r], pb[sb], 0, 0, 0);
-        pk[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(fv[r], fo[r], pk[sb], 0, 0, 0);
-        nb_[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(fu[r], fd[r], nb_[sb], 0, 0, 0);
-        nk[sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(fv[r], fd[r], nk[sb], 0, 0, 0);
-      }
+      const floatx4 fu = frag<true>(t2, 16 * sb + l16, 16 * kb + g4), fv = frag<true>(t0, 16 * sb + l16, 16 * kb + g4), fo = d_o[kb], fd = du[kb];
+      mfma4_each<4>({&pb[sb], &pk[sb], &nb_[sb], &nk[sb]}, [&](int i) { return i & 1 ? fv : fu; }, [&](int i) { return i & 2 ? fd : fo; });
     }
   });
-  mask<true, false>(pb, w), mask<true, false>(pk, w), mask<true, true>(nb_, w), mask<true, true>(nk, w);
-  {
-    Row<float> h0, dC;
-    h0.load(p.hT, ht);
-    dC.load(p.s1, wt);
-    // t1 and t3 are free since the gates were read
-    put_row(t1, w, [&](int cb) { return h0[cb] * load4(L.gate.em + 16 * cb + g4); });
-    put_row(t3, w, [&](int cb) { return dC[cb] * load4(L.gate.ec + 16 * cb + g4); });
-  }
-  lds_barrier();
-  floatx4 dq[4], da[4], db[4], dk[4];  // rows = channels, columns = tokens
-  clear(dq), clear(da), clear(db), clear(dk);
+  floatx4 dq[4], da[4];  // rows = channels, columns = tokens
+  clear(dq), clear(da);
+  float st[4];  // decays from the chunk's start to the lane's block, channels 16 cb + l16
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) st[cb] = L.start_to1(w.j, 16 * cb + l16);
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
     const floatx4 fo = d_o[kb], fd = du[kb], fu = u[kb], fv = v[kb];
+    mfma4_each<4>({&m.qb, &m.qk, &m.ab, &m.ak}, [&](int i) { return i & 1 ? fv : fu; }, [&](int i) { return i & 2 ? fd : fo; });
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {
-      const floatx4 hf = frag<false>(t1, 16 * cb + l16, 16 * kb + g4), df = frag<false>(t3, 16 * cb + l16, 16 * kb + g4);
+      const floatx4 hf = frag<false>(t1, 16 * cb + l16, 16 * kb + g4) * st[cb];
       mfma4(dq[cb], hf, fo);
       mfma4(da[cb], hf, fd);
-      mfma4(db[cb], df, fu);
-      mfma4(dk[cb], df, fv);
     }
   }
-  floatx4 Gp[4];  // from the lane before
+  mask<true, false>(m.qb, w), mask<true, false>(m.qk, w), mask<true, true>(m.ab, w), mask<true, true>(m.ak, w);
 #pragma unroll
-  for (int cb = 0; cb < 4; ++cb) {
-    const floatx4 G = load4(edge + 64 * max(w.j - 1, 0) + 16 * cb + g4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float prev = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x.G[cb][e]), 0x111, 0xF, 0xF, true));  // row_shr:1
-      Gp[cb][e] = l16 ? prev : w.j ? G[e] : 0.f;
-    }
-  }
-  const Decay e(x.G, Gp, edge + 192, L.gate, w, wide);
-  auto put_tri = [&](float* tile, const floatx4 (&m)[4]) {  // [t][s]
-#pragma unroll
-    for (int sb = 0; sb < 4; ++sb)
-      if (sb <= w.j) store4(tile + w.t * LD + 16 * sb + g4, m[sb]);
-  };
-  floatx4 xs[4], as[4];  // q dq + a da - b db - k dk and a da
-  if (!wide) {
-    put_row(t0, w, [&](int cb) { return x.b[cb] * e.b[cb]; });
-    put_row(t2, w, [&](int cb) { return x.k[cb] * e.b[cb]; });  // v and u were last read before a barrier
-    lds_barrier();
-    upto(w.j, [&](auto sb_) {
-      constexpr int sb = decltype(sb_)::value;
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        const floatx4 bf = frag<false>(t0, 16 * cb + l16, 16 * sb + g4), kf = frag<false>(t2, 16 * cb + l16, 16 * sb + g4);
-        mfma4(dq[cb], bf, pb[sb]);
-        mfma4(da[cb], bf, nb_[sb]);
-        mfma4(dq[cb], kf, pk[sb]);
-        mfma4(da[cb], kf, nk[sb]);
-      }
-    });
-    lds_barrier();
-    // db, dk: the matrices with the contraction along t, first those of q, then those of a
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      if (half) lds_barrier();
-      put_tri(t1, half ? nb_ : pb), put_tri(t2, half ? nk : pk);
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        if (half) store4(t0 + w.t * LD + 16 * cb + g4, x.a[cb] * e.a[cb]);
-        else store4(t0 + w.t * LD + 16 * cb + g4, p.scale * x.q[cb] * e.q[cb]);
-      }
-      lds_barrier();
-      downto(w.j, [&](auto tb_) {
-        constexpr int tb = decltype(tb_)::value;
-        const floatx4 mb = frag<false>(t1, w.t, 16 * tb + g4), mk = frag<false>(t2, w.t, 16 * tb + g4);
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb) {
-          const floatx4 xf = frag<false>(t0, 16 * cb + l16, 16 * tb + g4);
-          mfma4(db[cb], xf, mb);
-          mfma4(dk[cb], xf, mk);
-        }
-      });
-    }
-  }
-#pragma unroll
-  for (int cb = 0; cb < 4; ++cb) dq[cb] *= e.q[cb], da[cb] *= e.a[cb], db[cb] *= e.b[cb], dk[cb] *= e.b[cb];
-  if (wide) {
-    put_tri(t0, pb), put_tri(t2, pk);
-    lds_barrier();
-    put_cols(t1, w, x.G);
-    lds_barrier();
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb) wide_grads<T, 0>(p, s.tok, s.len, t0, t2, t1, w.t, 16 * cb + g4, dq[cb], db[cb], dk[cb]);
-    lds_barrier();
-    put_tri(t0, nb_), put_tri(t2, nk);
-    lds_barrier();
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb) wide_grads<T, 1>(p, s.tok, s.len, t0, t2, t1, w.t, 16 * cb + g4, da[cb], db[cb], dk[cb]);
-  }
-#pragma unroll
-  for (int cb = 0; cb < 4; ++cb) {
-    as[cb] = x.a[cb] * da[cb];
-    xs[cb] = p.scale * x.q[cb] * dq[cb] + as[cb] - x.b[cb] * db[cb] - x.k[cb] * dk[cb];
-  }
-  if (ok) {
+  for (int cb = 0; cb < 4; ++cb) asm volatile("" : "+v"(gates.sum[cb][0]), "+v"(gates.sum[cb][1]), "+v"(gates.sum[cb][2]), "+v"(gates.sum[cb][3]));
+  const Decay e(gates, p, s, w);  // formed here, not kept from the totals on: the registers are full in between
+  lds_barrier();
+  put_row(t0, w, [&](int cb) { return x.b[cb] * e.s[cb]; });
+  put_row(t2, w, [&](int cb) { return x.k[cb] * e.s[cb]; });
+  lds_barrier();
+  before(w.j, [&](auto sb_) {
+    constexpr int sb = decltype(sb_)::value;
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {
+      const float gap = L.from1<sb>(w.j, 16 * cb + l16);
+      const floatx4 bf = frag<false>(t0, 16 * cb + l16, 16 * sb + g4) * gap, kf = frag<false>(t2, 16 * cb + l16, 16 * sb + g4) * gap;
+      mfma4(dq[cb], bf, pb[sb]);
+      mfma4(da[cb], bf, nb_[sb]);
+      mfma4(dq[cb], kf, pk[sb]);
+      mfma4(da[cb], kf, nk[sb]);
+    }
+  });
+  float rt[4];  // 1 / decays of the whole block, channels 16 cb + l16: turns S of the block into 1 / P
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) rt[cb] = rcp_f(L.total[64 * w.j + 16 * cb + l16]);
+  if (gates.direct) {
+    float* own = t1 + w.t * LD;  // the state was last read before a barrier
+    store4(own + g4, m.qb), store4(own + 16 + g4, m.qk), store4(own + 32 + g4, m.ab), store4(own + 48 + g4, m.ak);
+    __builtin_amdgcn_wave_barrier();
+  }
+  const DirectRows<T> rows{p, s, w};
+  floatx4 flow[4];  // dgk so far: of sinks from the lane's token on, less a da of the token itself
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const floatx4 pl = token_before(e.p[cb]), q = p.scale * x.q[cb];
+    floatx4 dqo = zero4(), dao = zero4();  // of the block's own pairs
+    if (!gates.direct) {
+      const floatx4 bf = frag<false>(t0, 16 * cb + l16, 16 * w.j + g4) * rt[cb], kf = frag<false>(t2, 16 * cb + l16, 16 * w.j + g4) * rt[cb];
+      mfma4(dqo, bf, m.qb);
+      mfma4(dao, bf, m.ab);
+      mfma4(dqo, kf, m.qk);
+      mfma4(dao, kf, m.ak);
+      dqo *= e.p[cb], dao *= pl;
+    } else {
+      direct_sinks<T>(rows, t1 + w.t * LD, 16 * cb + g4, dqo, dao);
+    }
+    dq[cb] *= e.p[cb], da[cb] *= pl;
+    const floatx4 sink = q * dq[cb] + x.a[cb] * da[cb];  // of earlier blocks' sources
+    const floatx4 in = sum_block(sink);
+    if (l16 == 0) store4(tin + 64 * w.j + 16 * cb + g4, in);
+    flow[cb] = sum_from(sink + q * dqo + x.a[cb] * dao);
+    dq[cb] += dqo, da[cb] += dao;
+    flow[cb] -= x.a[cb] * da[cb];
+    if (ok) {
       store_row4<T>(p.dq, at + 16 * cb, dq[cb] * p.scale);
       store_row4<T>(p.da, at + 16 * cb, da[cb]);
+    }
+  }
+  lds_barrier();
+  // db, dk, relative to the end of the lane's block: the matrices with the contraction along t, first those of q, then those of a
+  floatx4 db[4], dk[4], own[4];  // own: b db + k dk of the block's own pairs
+  clear(db), clear(dk), clear(own);
+  auto same = [](floatx4 y) { return y; };
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    if (half) lds_barrier();
+    put_tri(t1, w, half ? nb_ : pb, half ? m.ab : m.qb, same), put_tri(t2, w, half ? nk : pk, half ? m.ak : m.qk, same);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) store4(t0 + w.t * LD + 16 * cb + g4, half ? x.a[cb] * token_before(e.p[cb]) : p.scale * x.q[cb] * e.p[cb]);
+    lds_barrier();
+    if (!half) {
+      float en[4];
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) en[cb] = L.end_from1(w.j, 16 * cb + l16);
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        const floatx4 fu = u[kb], fv = v[kb];
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+          const floatx4 df = frag<false>(t3, 16 * cb + l16, 16 * kb + g4) * en[cb];
+          mfma4(db[cb], df, fu);
+          mfma4(dk[cb], df, fv);
+        }
+      }
+    }
+    floatx4 dbh[4], dkh[4];  // apart from the other half's sums
+    clear(dbh), clear(dkh);
+    after(w.j, [&](auto tb_) {
+      constexpr int tb = decltype(tb_)::value;
+      const floatx4 mb = frag<false>(t1, w.t, 16 * tb + g4), mk = frag<false>(t2, w.t, 16 * tb + g4);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) {
+        const floatx4 xf = frag<false>(t0, 16 * cb + l16, 16 * tb + g4) * L.to1<tb>(w.j, 16 * cb + l16);
+        mfma4(dbh[cb], xf, mb);
+        mfma4(dkh[cb], xf, mk);
+      }
+    });
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) db[cb] += dbh[cb], dk[cb] += dkh[cb];
+    if (!gates.direct) {
+      const floatx4 mb = frag<false>(t1, w.t, 16 * w.j + g4), mk = frag<false>(t2, w.t, 16 * w.j + g4);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) {
+        const floatx4 xf = frag<false>(t0, 16 * cb + l16, 16 * w.j + g4) * rt[cb];
+        floatx4 ob = zero4(), ok_ = zero4();
+        mfma4(ob, xf, mb);
+        mfma4(ok_, xf, mk);
+        db[cb] += ob, dk[cb] += ok_;
+        own[cb] += (x.b[cb] * ob + x.k[cb] * ok_) * e.s[cb];
+      }
+    }
+  }
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) db[cb] *= e.s[cb], dk[cb] *= e.s[cb];
+  lds_barrier();
+  if (gates.direct) {
+    float* mine = t1 + w.t * LD;
+    store4(mine + g4, m.qb), store4(mine + 16 + g4, m.qk), store4(mine + 32 + g4, m.ab), store4(mine + 48 + g4, m.ak);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) {
+      floatx4 ob = zero4(), ok_ = zero4();
+      direct_sources<T>(rows, t1 + 16 * w.j * LD + l16, 16 * cb + g4, ob, ok_);
+      db[cb] += ob, dk[cb] += ok_;
+      own[cb] = x.b[cb] * ob + x.k[cb] * ok_;
+    }
+  }
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const floatx4 source = x.b[cb] * db[cb] + x.k[cb] * dk[cb] - own[cb], out = sum_upto(source);  // of later blocks' sinks
+    flow[cb] += out - source - sum_from(own[cb]);
+    if (l16 == 15) store4(tout + 64 * w.j + 16 * cb + g4, out);
+    if (ok) {
       store_row4<T>(p.db, at + 16 * cb, db[cb]);
       store_row4<T>(p.dk, at + 16 * cb, dk[cb]);
     }
   }
-  float *tx = t3, *tas = wide ? t1 : t0, *scr = L.sx;  // tas: read by nobody since the last barrier but in the products above
   lds_barrier();
-  put_cols(tx, w, xs);
-  put_cols(tas, w, as);
-  lds_barrier();
-  {
-    const int c = tid & 63, seg = tid >> 6;
-    float val[16], sum = 0.f;
 #pragma unroll
-    for (int i = 15; i >= 0; --i) val[i] = (sum += tx[(16 * seg + i) * LD + c]);
-    scr[64 * seg + c] = sum;
-    lds_barrier();
-    float after = 0.f;
-    for (int j = seg + 1; j < 4; ++j) after += scr[64 * j + c];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) after += red[64 * j + c];
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (16 * seg + i < s.len) p.dgk[(s.tok + 16 * seg + i) * D + c] = val[i] + after - tas[(16 * seg + i) * LD + c];
+  for (int cb = 0; cb < 4; ++cb) {
+    const int c = 16 * cb + g4;
+    floatx4 pass = (load4(red + c) + load4(red + 64 + c)) + (load4(red + 128 + c) + load4(red + 192 + c));
+    for (int j = 3; j > w.j; --j) pass += load4(tin + 64 * j + c) - load4(tout + 64 * j + c);
+    pass -= load4(tout + 64 * w.j + c);
+    if (ok) store4(p.dgk + at + 16 * cb, flow[cb] + pass);
   }
 }
 
@@ -980,6 +1206,7 @@ constexpr int64_t kept_tiles(int64_t n) { return 3 * n + 1; }  // of a row that 
 
 template <typename K> int lds_limit(K* k) { return lnx_lds_limit(reinterpret_cast<const void*>(k), LDS_BYTES); }
 
+// B8 H16 T4096 bf16 (8192 chunks), us: dplr_prepare 512, dplr_chunk_scan 111, dplr_out 112 (48 KB of reads and 8 of writes per chunk: 4.1 TB/s)
 template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
   if (int rc = lds_limit(dplr_prepare_kernel<T>)) return rc;
@@ -1001,6 +1228,8 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
   return LNX_OK;
 }
 
+// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 497, dplr_grad 773 (66 registers spilled: everything a chunk's token needs is
+// live between the pair sums and the last products)
 template <typename T> int backward(const lnx_dplr_chunk_grads* g, const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
   set_kept(p, kept, rows, 0, p.N);

@@ -1,5 +1,5 @@
 """The chunked RWKV-7 scan (heads of 64 x 64) against the fp64 oracle and its adjoint: lengths around one chunk, decays of
-RWKV-7's range, decays so strong that a chunk's pairs are evaluated one by one, both in one sequence, and growth; 1e-4
+RWKV-7's range, decays so strong that a block's pairs are evaluated one by one, both in one sequence, and growth; 1e-4
 (fp32) / 2e-2 (bf16) of max|ref|.  Windows: a call whose work areas are cut into windows of chunks returns the bits of a
 call on some of its rows alone."""
 import numpy as np
@@ -23,7 +23,7 @@ def _data(seed, B, H, T, decay, bf16):
     kk /= np.linalg.norm(kk, axis=-1, keepdims=True)
     rate = r.random((B, H, T, d)).astype(np.float32)
     gk = {"rwkv": -0.6065 * rate, "none": 0 * rate, "strong": -6 * rate, "growth": 0.01 * rate}.get(decay)
-    if decay == "mixed":  # wide chunks only where a few channels decay strongly, from the second chunk on
+    if decay == "mixed":  # such blocks only where a few channels decay strongly, from the second chunk on
         gk = -0.3 * rate
         gk[:, :, 64:, ::17] -= 9.0
     x = dict(q=n(B, H, T, d), k=n(B, H, T, d) * 0.5, v=n(B, H, T, d), a=-kk, b=kk * r.random((B, H, T, d)).astype(np.float32), gk=gk.astype(np.float32),
