@@ -66,6 +66,17 @@ bool wants_grad(std::initializer_list<const Tensor*> ts) {
   return false;
 }
 
+// The kernels read values only: an input that carries a tangent would give a result without one, so it is refused, whether a gradient
+// is wanted or not.
+void refuse_tangents(const char* op, std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(/*level=*/0).defined(), op, " has no forward-mode derivative (jvp)");
+}
+
+void refuse_tangents(const char* op, const variable_list& ts) {
+  for (const Tensor& t : ts) refuse_tangents(op, {&t});
+}
+
 std::string shape_text(const Tensor& t) {
   std::string s = "(";
   for (int64_t i = 0; i < t.dim(); ++i) s += (i ? ", " : "") + std::to_string(t.size(i));
@@ -223,6 +234,7 @@ PyObject* py_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     else Py_RETURN_NONE;
   }
   if (wants_grad({&q, &k, &v, &g, &beta, &state})) Py_RETURN_NONE;
+  refuse_tangents("step", {&q, &k, &v, &g, &beta, &state});
   const bool l2norm = in.flag(7), o_f32 = in.flag(8), inplace = in.flag(9);
   const double scale = in.is_none(6) ? 1.0 / std::sqrt((double)dk) : in.number(6);
   const Tensor s_out = inplace ? state : at::empty_like(state);
@@ -272,6 +284,7 @@ PyObject* py_recurrent(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Tensor q0 = in.tensor(0, "q"), k0 = in.tensor(1, "k"), v0 = in.tensor(2, "v"), g0 = in.maybe(3, "g"), s0 = in.maybe(5, "initial_state"),
                cu = in.maybe(8, "cu_seqlens");
   const Tensor b0 = squeeze_beta(in.tensor(4, "beta"), 4);
+  refuse_tangents("recurrent", {&q0, &k0, &v0, &g0, &b0, &s0});
   const SeqShape s = seq_shape(q0, k0, v0, g0, b0, cu);
   check_state(s0, s, s.dv);
   const bool tf = is_token_first(q0) && is_token_first(k0) && is_token_first(v0);
@@ -344,6 +357,7 @@ struct L2NormFn : Function<L2NormFn> {
     return l2norm_fwd(x);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    refuse_tangents("the gradient of l2norm_rows", grads);
     const Tensor x = ctx->get_saved_variables()[0];
     return {l2norm_bwd(x, grads[0].to(x.scalar_type()))};
   }
@@ -355,6 +369,7 @@ PyObject* py_l2norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Tensor x = in.tensor(0, "x");
   TORCH_CHECK(x.is_cuda() && x.dim() > 0 && known_dtype(x.scalar_type()), "l2norm_rows takes float32 or bfloat16 rows on the GPU, got ", shape_text(x), " ",
               x.scalar_type(), " on ", x.device().str());
+  refuse_tangents("l2norm_rows", {&x});
   return THPVariable_Wrap(wants_grad({&x}) ? L2NormFn::apply(x) : l2norm_fwd(x));
   LNX_END
 }
@@ -453,6 +468,7 @@ struct ChunkFn : Function<ChunkFn> {
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    refuse_tangents("the gradient of chunkwise", grads);
     const variable_list s = ctx->get_saved_variables();
     const std::vector<int64_t> m = ctx->saved_data["i"].toIntVector();
     const std::vector<double> d = ctx->saved_data["d"].toDoubleVector();
@@ -498,6 +514,7 @@ PyObject* py_chunk_segmented(PyObject*, PyObject* const* args, Py_ssize_t nargs)
   at::NoGradGuard no_grad;
   const Tensor q0 = in.tensor(0, "q"), k0 = in.tensor(1, "k"), v0 = in.tensor(2, "v"), g0 = in.maybe(3, "g"), s00 = in.maybe(5, "initial_state");
   const Tensor beta0 = squeeze_beta(in.tensor(4, "beta"), 4);
+  refuse_tangents("chunkwise", {&q0, &k0, &v0, &g0, &beta0, &s00});
   const SeqShape s = seq_shape(q0, k0, v0, g0, beta0, Tensor());
   check_state(s00, s, s.dv);
   const int64_t rows = s.B * s.H, chunks = (s.T + 63) / 64, per = (chunks + in.integer(9) - 1) / in.integer(9), nseg = (chunks + per - 1) / per;
@@ -536,6 +553,7 @@ PyObject* py_chunk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Tensor q = in.tensor(0, "q"), k = in.tensor(1, "k"), v = in.tensor(2, "v"), g = in.maybe(3, "g"), s0 = in.maybe(5, "initial_state"),
                A_log = in.maybe(11, "A_log"), g_bias = in.maybe(12, "g_bias");
   const Tensor beta = squeeze_beta(in.tensor(4, "beta"), 4);
+  refuse_tangents("chunkwise", {&q, &k, &v, &g, &beta, &s0, &A_log, &g_bias});
   ChunkOptions o;
   o.cu = in.maybe(9, "cu_seqlens");
   o.scale = in.number(6), o.l2norm = in.flag(7), o.o_dtype = in.integer(8), o.forward_only = in.flag(10);
@@ -600,6 +618,7 @@ struct ConvFn : Function<ConvFn> {
     return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    refuse_tangents("the gradient of depthwise_conv1d_causal", grads);
     const variable_list s = ctx->get_saved_variables();
     const std::vector<int64_t> m = ctx->saved_data["i"].toIntVector();
     TORCH_CHECK(!m[4], "cannot differentiate through a convolution whose cache was updated in place");
@@ -634,6 +653,7 @@ PyObject* py_conv1d(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Args in(args, nargs, 7, "conv1d");
   TORCH_CHECK(in.is_tensor(0) && THPVariable_Unpack(args[0]).is_cuda(), "inputs must be a torch.Tensor on the GPU; the convolution runs on the GPU only");
   const Tensor x = in.tensor(0, "inputs"), weight = in.tensor(1, "weight"), bias = in.maybe(2, "bias"), cache = in.maybe(3, "cache"), cu = in.maybe(6, "cu_seqlens");
+  refuse_tangents("depthwise_conv1d_causal", {&x, &weight, &bias, &cache});
   const int64_t act = in.integer(4);
   const bool inplace = in.flag(5);
   TORCH_CHECK(x.dim() == 3, "inputs must be [batch, seq, channels], got ", shape_text(x));
@@ -690,6 +710,7 @@ struct RmsFn : Function<RmsFn> {
     return rms_forward(x, gate, w, eps);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    refuse_tangents("the gradient of rmsnorm_gated", grads);
     const variable_list s = ctx->get_saved_variables();
     const std::vector<int64_t> m = ctx->saved_data["i"].toIntVector();
     const Tensor &x = s[0], &gate = s[1], &w = s[2];
@@ -715,6 +736,7 @@ PyObject* py_rmsnorm_gated(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   TORCH_CHECK(known_dtype(x.scalar_type()), "unsupported dtype ", x.scalar_type(), ": use float32 or bfloat16");
   TORCH_CHECK(!gate.defined() || gate.sizes() == x.sizes(), "gate shape ", gate.defined() ? shape_text(gate) : "", " != x shape ", shape_text(x));
   TORCH_CHECK(x.dim() > 0 && weight.dim() == 1 && weight.size(0) == x.size(-1), "weight must be [", x.dim() ? x.size(-1) : 0, "], got ", shape_text(weight));
+  refuse_tangents("rmsnorm_gated", {&x, &gate, &weight});
   if (wants_grad({&x, &gate, &weight})) return THPVariable_Wrap(RmsFn::apply(x, opt(gate), weight, eps));
   return THPVariable_Wrap(rms_forward(x.contiguous(), gate.defined() ? gate.to(x.scalar_type()).contiguous() : gate, f32(weight), eps));
   LNX_END
@@ -746,6 +768,7 @@ struct GdnGateFn : Function<GdnGateFn> {
     return {g, beta};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    refuse_tangents("the gradient of gated_deltanet_gate", grads);
     const variable_list s = ctx->get_saved_variables();
     const std::vector<int64_t> m = ctx->saved_data["i"].toIntVector();
     const Tensor &a = s[0], &b = s[1], &A = s[2], &bias = s[3];
@@ -772,6 +795,7 @@ PyObject* py_gdn_gate(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   TORCH_CHECK(A_log.dim() == 1 && a.dim() >= 1 && a.size(-1) == A_log.size(0), "a ", shape_text(a), " must end in the heads of A_log ", shape_text(A_log));
   TORCH_CHECK(!dt_bias.defined() || dt_bias.sizes() == A_log.sizes(), "dt_bias must be [", A_log.size(0), "], got ", dt_bias.defined() ? shape_text(dt_bias) : "");
   TORCH_CHECK(!b.defined() || b.sizes() == a.sizes(), "b ", b.defined() ? shape_text(b) : "", " must have a's shape ", shape_text(a));
+  refuse_tangents("gated_deltanet_gate", {&a, &A_log, &dt_bias, &b});
   if (wants_grad({&a, &A_log, &dt_bias, &b})) {
     const variable_list r = GdnGateFn::apply(a, opt(b), A_log, opt(dt_bias), beta_scale);
     return pack(r[0], r.size() > 1 ? r[1] : Tensor());
@@ -798,6 +822,7 @@ struct KdaGateFn : Function<KdaGateFn> {
     return kda_gate_forward(g, A, bias, dk, threshold, out_dtype);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    refuse_tangents("the gradient of kda_gate", grads);
     const variable_list s = ctx->get_saved_variables();
     const std::vector<int64_t> m = ctx->saved_data["i"].toIntVector();
     const Tensor &g = s[0], &A = s[1], &bias = s[2];
@@ -826,6 +851,7 @@ struct SigmoidFn : Function<SigmoidFn> {
     return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    refuse_tangents("the gradient of kda_gate", grads);
     const Tensor y = ctx->get_saved_variables()[0], dy = f32(grads[0]);
     Tensor dx = at::empty_like(y);
     check_status(lnx_sigmoid_bwd(fptr(y), fptr(dy), fptr(dx), y.numel(), stream_of(y)), "lnx_sigmoid_bwd");
@@ -845,6 +871,7 @@ PyObject* py_kda_gate(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   TORCH_CHECK(g.dim() == 3 && A_log.dim() == 1 && g.size(2) == A_log.size(0) * dk, "g ", shape_text(g), " must be [batch, seq, heads of A_log ", shape_text(A_log),
               " * ", dk, "]");
   TORCH_CHECK(!g_bias.defined() || (g_bias.dim() == 1 && g_bias.size(0) == g.size(2)), "g_bias must be [", g.size(2), "], got ", g_bias.defined() ? shape_text(g_bias) : "");
+  refuse_tangents("kda_gate", {&g, &A_log, &g_bias, &beta});
   const int64_t out_dtype = in.is_none(6) ? code_of(g.scalar_type()) : in.integer(6);
   const Tensor out = wants_grad({&g, &A_log, &g_bias}) ? KdaGateFn::apply(g, A_log, opt(g_bias), dk, threshold, out_dtype)
                                                        : kda_gate_forward(g.contiguous(), f32(A_log), f32(g_bias), dk, threshold, out_dtype);
@@ -935,6 +962,7 @@ struct DplrFn : Function<DplrFn> {
     return {o, s_out};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    refuse_tangents("the gradient of dplr_delta_rule_recurrent", grads);
     const variable_list s = ctx->get_saved_variables();
     const std::vector<int64_t> m = ctx->saved_data["i"].toIntVector();
     const Tensor &q = s[0], &k = s[1], &v = s[2], &a = s[3], &b = s[4], &gk = s[5], &s_in = s[6];
@@ -983,6 +1011,7 @@ PyObject* py_dplr(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Args in(args, nargs, 8, "dplr");
   const Tensor q = in.tensor(0, "q"), k = in.tensor(1, "k"), v = in.tensor(2, "v"), a = in.tensor(3, "a"), b = in.tensor(4, "b"), gk = in.tensor(5, "gk"),
                s0 = in.maybe(7, "initial_state");
+  refuse_tangents("dplr_delta_rule_recurrent", {&q, &k, &v, &a, &b, &gk, &s0});
   check_dplr(q, k, v, a, b, gk, 4);
   TORCH_CHECK(!s0.defined() || s0.sizes() == at::IntArrayRef({q.size(0), q.size(1), q.size(3), v.size(3)}), "initial_state shape ",
               s0.defined() ? shape_text(s0) : "", " != (", q.size(0), ", ", q.size(1), ", ", q.size(3), ", ", v.size(3), ")");
@@ -999,6 +1028,7 @@ PyObject* py_dplr_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                state = in.tensor(6, "state");
   const double scale = in.number(7);
   const bool inplace = in.flag(8);
+  refuse_tangents("dplr_delta_rule_step", {&q, &k, &v, &a, &b, &gk, &state});
   check_dplr(q, k, v, a, b, gk, 3);
   TORCH_CHECK(state.sizes() == at::IntArrayRef({q.size(0), q.size(1), q.size(2), v.size(2)}), "state shape ", shape_text(state), " != (", q.size(0), ", ", q.size(1), ", ",
               q.size(2), ", ", v.size(2), ")");
