@@ -48,6 +48,12 @@ void check_status(int status, const char* what) {
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
+bool capturing(const Tensor& t) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  TORCH_CHECK(hipStreamIsCapturing(c10::hip::getCurrentHIPStream(t.get_device()).stream(), &status) == hipSuccess, "hipStreamIsCapturing failed");
+  return status != hipStreamCaptureStatusNone;
+}
+
 void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 float* fptr(const Tensor& t) { return static_cast<float*>(ptr(t)); }
 OptT opt(const Tensor& t) { return t.defined() ? OptT(t) : OptT(); }
@@ -579,7 +585,9 @@ struct ConvSide {
   Tensor x, cin, cout, cu;
 };
 
-// A buffer that the forward kernel has cleared, for the first backward pass of its node.
+// A buffer that the forward kernel has cleared, for the first backward pass of its node.  Only between eager passes: a captured
+// backward pass is replayed and would find its own sums, and a captured forward pass clears the buffer at every replay, when it has long
+// been somebody's gradient.
 struct Cleared : torch::CustomClassHolder {
   Tensor buffer;
   std::atomic<bool> taken{false};
@@ -608,7 +616,8 @@ struct ConvFn : Function<ConvFn> {
     const Tensor w = f32(weight), b = f32(undef(bias));
     // the parameters' gradients are sums that start from zero: this kernel clears them, the backward pass saves a launch
     auto cleared = c10::make_intrusive<Cleared>();
-    cleared->buffer = at::empty({w.size(0) + (b.defined() ? 1 : 0), w.size(1)}, w.options());
+    if (capturing(x)) cleared->taken = true;
+    else cleared->buffer = at::empty({w.size(0) + (b.defined() ? 1 : 0), w.size(1)}, w.options());
     Tensor y = conv_forward(w, b, side, act, cleared->buffer);
     ctx->saved_data["cleared"] = c10::IValue::make_capsule(cleared);
     ctx->save_for_backward({x.is_contiguous() ? x : side.x, w, b, lost_cache ? Tensor() : side.cin, side.cu});
@@ -627,7 +636,7 @@ struct ConvFn : Function<ConvFn> {
     const Tensor dy = grads[0].to(x.scalar_type()).contiguous();
     Tensor dx = at::empty_like(x), dw, db, dc;
     auto cleared = c10::static_intrusive_pointer_cast<Cleared>(ctx->saved_data["cleared"].toCapsule());
-    if (!cleared->taken.exchange(true)) {
+    if (!capturing(x) && !cleared->taken.exchange(true)) {
       const Tensor buffer = std::move(cleared->buffer);
       dw = b.defined() ? buffer.narrow(0, 0, K) : buffer;
       if (b.defined()) db = buffer.select(0, K);
