@@ -189,6 +189,19 @@ PyObject* pack(const Tensor& x, const Tensor& y) {
   return t;
 }
 
+// What an op does between reading its arguments and wrapping its results: allocations and launches, which can wait for the driver or for
+// a full queue.  Other Python threads run meanwhile.  0.1 us a call.
+struct NoLock {
+  PyThreadState* state = PyEval_SaveThread();
+  NoLock() = default;
+  NoLock(const NoLock&) = delete;
+  ~NoLock() { PyEval_RestoreThread(state); }
+};
+template <typename F> auto without_lock(F&& f) {
+  const NoLock released;
+  return f();
+}
+
 // Every entry point: C++ exceptions become Python ones (a failed C-ABI call: HipKernelError).
 #define LNX_BEGIN HANDLE_TH_ERRORS try {
 #define LNX_END                                      \
@@ -221,9 +234,9 @@ PyObject* py_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Args in(args, nargs, 10, "step");
   for (int i = 0; i < 6; ++i)
     if (!in.is_tensor(i) && !(i == 3 && in.is_none(i))) Py_RETURN_NONE;
-  const Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]);
+  const Tensor q = THPVariable_Unpack(args[0]), k = THPVariable_Unpack(args[1]), v = THPVariable_Unpack(args[2]);
   const Tensor g = in.is_none(3) ? Tensor() : THPVariable_Unpack(args[3]);
-  const Tensor &beta = THPVariable_Unpack(args[4]), &state = THPVariable_Unpack(args[5]);
+  const Tensor beta = THPVariable_Unpack(args[4]), state = THPVariable_Unpack(args[5]);
   const auto dt = q.scalar_type();
   if (q.dim() != 3 || v.dim() != 3 || !q.is_cuda() || !k.is_cuda() || !v.is_cuda() || !known_dtype(dt) || k.scalar_type() != dt || v.scalar_type() != dt) Py_RETURN_NONE;
   const int64_t B = q.size(0), H = q.size(1), dk = q.size(2), dv = v.size(2);
@@ -243,13 +256,16 @@ PyObject* py_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   refuse_tangents("step", {&q, &k, &v, &g, &beta, &state});
   const bool l2norm = in.flag(7), o_f32 = in.flag(8), inplace = in.flag(9);
   const double scale = in.is_none(6) ? 1.0 / std::sqrt((double)dk) : in.number(6);
-  const Tensor s_out = inplace ? state : at::empty_like(state);
-  const Tensor o = at::empty({B, H, dv}, q.options().dtype(o_f32 ? at::kFloat : dt));
-  lnx_scan_args a = base_args(B, H, 1, dk, dv, code_of(dt), code_of(o.scalar_type()), gate, l2norm, scale);
-  a.q = ptr(q), a.k = ptr(k), a.v = ptr(v), a.beta = fptr(beta), a.g = fptr(g);
-  a.initial_state = fptr(state), a.final_state = fptr(s_out), a.o = ptr(o);
-  check_status(lnx_decode_step(&a, stream_of(q)), "lnx_decode_step");
-  return pack(o, s_out);
+  const auto r = without_lock([&] {
+    const Tensor s_out = inplace ? state : at::empty_like(state);
+    const Tensor o = at::empty({B, H, dv}, q.options().dtype(o_f32 ? at::kFloat : dt));
+    lnx_scan_args a = base_args(B, H, 1, dk, dv, code_of(dt), code_of(o.scalar_type()), gate, l2norm, scale);
+    a.q = ptr(q), a.k = ptr(k), a.v = ptr(v), a.beta = fptr(beta), a.g = fptr(g);
+    a.initial_state = fptr(state), a.final_state = fptr(s_out), a.o = ptr(o);
+    check_status(lnx_decode_step(&a, stream_of(q)), "lnx_decode_step");
+    return std::make_pair(o, s_out);
+  });
+  return pack(r.first, r.second);
   LNX_END
 }
 
@@ -293,19 +309,24 @@ PyObject* py_recurrent(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   refuse_tangents("recurrent", {&q0, &k0, &v0, &g0, &b0, &s0});
   const SeqShape s = seq_shape(q0, k0, v0, g0, b0, cu);
   check_state(s0, s, s.dv);
-  const bool tf = is_token_first(q0) && is_token_first(k0) && is_token_first(v0);
-  const Tensor q = as_layout(q0, tf), k = as_layout(k0, tf), v = as_layout(v0, tf), beta = as_layout(b0.to(at::kFloat), tf);
-  const Tensor g = g0.defined() ? as_layout(g0.to(at::kFloat), tf) : g0, si = f32(s0);
-  const Tensor o = empty_layout(s.B, s.H, s.T, s.dv, q.options(), tf);
-  const Tensor sT = at::empty({s.nstate, s.H, s.dk, s.dv}, q.options().dtype(at::kFloat));
-  const int dt = code_of(q.scalar_type());
-  lnx_scan_args a = base_args(s.B, s.H, s.T, s.dk, s.dv, dt, dt, s.gate, in.flag(7), in.is_none(6) ? 1.0 / std::sqrt((double)s.dk) : in.number(6));
-  a.nseq = (int32_t)s.nseq;
-  a.token_first = tf;
-  a.q = ptr(q), a.k = ptr(k), a.v = ptr(v), a.beta = fptr(beta), a.g = fptr(g);
-  a.initial_state = fptr(si), a.final_state = fptr(sT), a.o = ptr(o), a.cu_seqlens = static_cast<const int32_t*>(ptr(cu));
-  check_status(lnx_recurrent_fwd(&a, stream_of(q)), "lnx_recurrent_fwd");
-  return pack(o, sT);
+  const bool l2norm = in.flag(7);
+  const double scale = in.is_none(6) ? 1.0 / std::sqrt((double)s.dk) : in.number(6);
+  const auto r = without_lock([&] {
+    const bool tf = is_token_first(q0) && is_token_first(k0) && is_token_first(v0);
+    const Tensor q = as_layout(q0, tf), k = as_layout(k0, tf), v = as_layout(v0, tf), beta = as_layout(b0.to(at::kFloat), tf);
+    const Tensor g = g0.defined() ? as_layout(g0.to(at::kFloat), tf) : g0, si = f32(s0);
+    const Tensor o = empty_layout(s.B, s.H, s.T, s.dv, q.options(), tf);
+    const Tensor sT = at::empty({s.nstate, s.H, s.dk, s.dv}, q.options().dtype(at::kFloat));
+    const int dt = code_of(q.scalar_type());
+    lnx_scan_args a = base_args(s.B, s.H, s.T, s.dk, s.dv, dt, dt, s.gate, l2norm, scale);
+    a.nseq = (int32_t)s.nseq;
+    a.token_first = tf;
+    a.q = ptr(q), a.k = ptr(k), a.v = ptr(v), a.beta = fptr(beta), a.g = fptr(g);
+    a.initial_state = fptr(si), a.final_state = fptr(sT), a.o = ptr(o), a.cu_seqlens = static_cast<const int32_t*>(ptr(cu));
+    check_status(lnx_recurrent_fwd(&a, stream_of(q)), "lnx_recurrent_fwd");
+    return std::make_pair(o, sT);
+  });
+  return pack(r.first, r.second);
   LNX_END
 }
 
@@ -376,7 +397,7 @@ PyObject* py_l2norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   TORCH_CHECK(x.is_cuda() && x.dim() > 0 && known_dtype(x.scalar_type()), "l2norm_rows takes float32 or bfloat16 rows on the GPU, got ", shape_text(x), " ",
               x.scalar_type(), " on ", x.device().str());
   refuse_tangents("l2norm_rows", {&x});
-  return THPVariable_Wrap(wants_grad({&x}) ? L2NormFn::apply(x) : l2norm_fwd(x));
+  return THPVariable_Wrap(without_lock([&] { return wants_grad({&x}) ? L2NormFn::apply(x) : l2norm_fwd(x); }));
   LNX_END
 }
 
@@ -384,7 +405,8 @@ PyObject* py_l2norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 PyObject* py_l2norm_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   LNX_BEGIN
   Args in(args, nargs, 2, "l2norm_bwd");
-  return THPVariable_Wrap(l2norm_bwd(in.tensor(0, "x"), in.tensor(1, "dy")));
+  const Tensor x = in.tensor(0, "x"), dy = in.tensor(1, "dy");
+  return THPVariable_Wrap(without_lock([&] { return l2norm_bwd(x, dy); }));
   LNX_END
 }
 
@@ -512,18 +534,12 @@ struct ChunkFn : Function<ChunkFn> {
   }
 };
 
-// chunk_segmented(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, nseg): (o, final state) of a forward-only call on dense
-// sequences, cut into about nseg segments that run in parallel (lnx_chunk_fwd_segmented); batch rows become heads.
-PyObject* py_chunk_segmented(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  LNX_BEGIN
-  Args in(args, nargs, 10, "chunk_segmented");
+std::pair<Tensor, Tensor> chunk_segmented(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor& g0, const Tensor& beta0, const Tensor& s00, double scale,
+                                          bool l2norm, int64_t o_dtype, int64_t wanted) {
   at::NoGradGuard no_grad;
-  const Tensor q0 = in.tensor(0, "q"), k0 = in.tensor(1, "k"), v0 = in.tensor(2, "v"), g0 = in.maybe(3, "g"), s00 = in.maybe(5, "initial_state");
-  const Tensor beta0 = squeeze_beta(in.tensor(4, "beta"), 4);
-  refuse_tangents("chunkwise", {&q0, &k0, &v0, &g0, &beta0, &s00});
   const SeqShape s = seq_shape(q0, k0, v0, g0, beta0, Tensor());
   check_state(s00, s, s.dv);
-  const int64_t rows = s.B * s.H, chunks = (s.T + 63) / 64, per = (chunks + in.integer(9) - 1) / in.integer(9), nseg = (chunks + per - 1) / per;
+  const int64_t rows = s.B * s.H, chunks = (s.T + 63) / 64, per = (chunks + wanted - 1) / wanted, nseg = (chunks + per - 1) / per;
   auto fold = [&](const Tensor& t) {
     if (!t.defined() || s.B == 1) return t;
     std::vector<int64_t> sizes = t.sizes().vec();
@@ -534,12 +550,11 @@ PyObject* py_chunk_segmented(PyObject*, PyObject* const* args, Py_ssize_t nargs)
   const bool tf = is_token_first(q1) && is_token_first(k1) && is_token_first(v1);
   Tensor q = as_layout(q1, tf), k = as_layout(k1, tf);
   const Tensor v = as_layout(v1, tf), beta = as_layout(fold(beta0).to(at::kFloat), tf), g = g0.defined() ? as_layout(fold(g0).to(at::kFloat), tf) : g0, s0 = f32(s00);
-  const int64_t o_dtype = in.integer(8);
   const Tensor o = empty_layout(1, rows, s.T, s.dv, q.options().dtype(type_of(o_dtype)), tf);
   const Tensor sT = at::empty({nseg, rows, s.dk, s.dv}, q.options().dtype(at::kFloat));
-  lnx_scan_args a = base_args(1, rows, s.T, s.dk, s.dv, code_of(q.scalar_type()), (int)o_dtype, s.gate, false, in.number(6));
-  a.use_qk_l2norm = in.flag(7) && lnx_chunk_fuses_l2norm(&a);
-  if (in.flag(7) && !a.use_qk_l2norm) std::tie(q, k) = l2norm_pair_fwd(q, k);
+  lnx_scan_args a = base_args(1, rows, s.T, s.dk, s.dv, code_of(q.scalar_type()), (int)o_dtype, s.gate, false, scale);
+  a.use_qk_l2norm = l2norm && lnx_chunk_fuses_l2norm(&a);
+  if (l2norm && !a.use_qk_l2norm) std::tie(q, k) = l2norm_pair_fwd(q, k);
   a.token_first = tf, a.forward_only = 1;
   a.q = ptr(q), a.k = ptr(k), a.v = ptr(v), a.beta = fptr(beta), a.g = fptr(g);
   a.initial_state = fptr(s0), a.final_state = fptr(sT), a.o = ptr(o);
@@ -547,7 +562,22 @@ PyObject* py_chunk_segmented(PyObject*, PyObject* const* args, Py_ssize_t nargs)
   const Tensor ws = at::empty({(int64_t)std::max<uint64_t>(nbytes, 1)}, q.options().dtype(at::kByte));
   a.workspace = ptr(ws), a.workspace_bytes = nbytes;
   check_status(lnx_chunk_fwd_segmented(&a, (int32_t)nseg, stream_of(q)), "lnx_chunk_fwd_segmented");
-  return pack(s.B == 1 ? o : o.reshape({s.B, s.H, s.T, s.dv}), sT.select(0, nseg - 1).view({s.B, s.H, s.dk, s.dv}));
+  return {s.B == 1 ? o : o.reshape({s.B, s.H, s.T, s.dv}), sT.select(0, nseg - 1).view({s.B, s.H, s.dk, s.dv})};
+}
+
+// chunk_segmented(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, nseg): (o, final state) of a forward-only call on dense
+// sequences, cut into about nseg segments that run in parallel (lnx_chunk_fwd_segmented); batch rows become heads.
+PyObject* py_chunk_segmented(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  LNX_BEGIN
+  Args in(args, nargs, 10, "chunk_segmented");
+  const Tensor q = in.tensor(0, "q"), k = in.tensor(1, "k"), v = in.tensor(2, "v"), g = in.maybe(3, "g"), s0 = in.maybe(5, "initial_state");
+  const Tensor beta = squeeze_beta(in.tensor(4, "beta"), 4);
+  refuse_tangents("chunkwise", {&q, &k, &v, &g, &beta, &s0});
+  const double scale = in.number(6);
+  const bool l2norm = in.flag(7);
+  const int64_t o_dtype = in.integer(8), nseg = in.integer(9);
+  const auto r = without_lock([&] { return chunk_segmented(q, k, v, g, beta, s0, scale, l2norm, o_dtype, nseg); });
+  return pack(r.first, r.second);
   LNX_END
 }
 
@@ -564,13 +594,15 @@ PyObject* py_chunk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   o.cu = in.maybe(9, "cu_seqlens");
   o.scale = in.number(6), o.l2norm = in.flag(7), o.o_dtype = in.integer(8), o.forward_only = in.flag(10);
   o.threshold = in.number(13), o.scan_slab = in.integer(14), o.out_slabs = in.integer(15);
-  if (!o.forward_only) {
-    const variable_list r = ChunkFn::apply(q, k, v, opt(g), beta, opt(s0), opt(A_log), opt(g_bias), o);
-    return pack(r[0], r[1]);
-  }
-  at::NoGradGuard no_grad;
-  ChunkCall c;
-  const auto r = chunk_forward(q, k, v, g, beta, s0, A_log, g_bias, o, c);
+  const auto r = without_lock([&]() -> std::pair<Tensor, Tensor> {
+    if (!o.forward_only) {
+      const variable_list r = ChunkFn::apply(q, k, v, opt(g), beta, opt(s0), opt(A_log), opt(g_bias), o);
+      return {r[0], r[1]};
+    }
+    at::NoGradGuard no_grad;
+    ChunkCall c;
+    return chunk_forward(q, k, v, g, beta, s0, A_log, g_bias, o, c);
+  });
   return pack(r.first, r.second);
   LNX_END
 }
@@ -679,21 +711,23 @@ PyObject* py_conv1d(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     TORCH_CHECK(B == 1, "cu_seqlens needs a packed batch with B == 1");
     TORCH_CHECK(!cache.defined(), "a packed batch starts every sequence from a zero cache: pass cache=None");
   }
-  const Tensor xc = x.is_contiguous() ? x : x.detach().contiguous();
   Tensor cin, cout;  // cache before and after
   const bool kept = cache.defined() && K > 1, own = kept && inplace;
-  if (own) {
-    TORCH_CHECK(cache.scalar_type() == x.scalar_type() && cache.is_contiguous(), "inplace_cache=True needs a contiguous cache of the inputs' dtype");
-    cin = cout = cache.detach();
-  } else if (kept) {
-    cin = cache.detach().to(x.scalar_type()).contiguous();
-    cout = at::empty_like(cin);
-  } else {
-    cout = at::empty({B, K - 1, D}, x.options());
-  }
-  const ConvSide side{xc, cin, cout, cu};
-  const Tensor y = wants_grad({&x, &weight, &bias, &cache}) ? ConvFn::apply(x, weight, opt(bias), opt(cache), side, act, own)
-                                                            : conv_forward(f32(weight), f32(bias), side, act);
+  TORCH_CHECK(!own || (cache.scalar_type() == x.scalar_type() && cache.is_contiguous()), "inplace_cache=True needs a contiguous cache of the inputs' dtype");
+  const Tensor y = without_lock([&] {
+    const Tensor xc = x.is_contiguous() ? x : x.detach().contiguous();
+    if (own) {
+      cin = cout = cache.detach();
+    } else if (kept) {
+      cin = cache.detach().to(x.scalar_type()).contiguous();
+      cout = at::empty_like(cin);
+    } else {
+      cout = at::empty({B, K - 1, D}, x.options());
+    }
+    const ConvSide side{xc, cin, cout, cu};
+    return wants_grad({&x, &weight, &bias, &cache}) ? ConvFn::apply(x, weight, opt(bias), opt(cache), side, act, own)
+                                                    : conv_forward(f32(weight), f32(bias), side, act);
+  });
   return pack(y, own ? cache : cout);
   LNX_END
 }
@@ -746,8 +780,10 @@ PyObject* py_rmsnorm_gated(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   TORCH_CHECK(!gate.defined() || gate.sizes() == x.sizes(), "gate shape ", gate.defined() ? shape_text(gate) : "", " != x shape ", shape_text(x));
   TORCH_CHECK(x.dim() > 0 && weight.dim() == 1 && weight.size(0) == x.size(-1), "weight must be [", x.dim() ? x.size(-1) : 0, "], got ", shape_text(weight));
   refuse_tangents("rmsnorm_gated", {&x, &gate, &weight});
-  if (wants_grad({&x, &gate, &weight})) return THPVariable_Wrap(RmsFn::apply(x, opt(gate), weight, eps));
-  return THPVariable_Wrap(rms_forward(x.contiguous(), gate.defined() ? gate.to(x.scalar_type()).contiguous() : gate, f32(weight), eps));
+  return THPVariable_Wrap(without_lock([&] {
+    if (wants_grad({&x, &gate, &weight})) return RmsFn::apply(x, opt(gate), weight, eps);
+    return rms_forward(x.contiguous(), gate.defined() ? gate.to(x.scalar_type()).contiguous() : gate, f32(weight), eps);
+  }));
   LNX_END
 }
 
@@ -805,11 +841,13 @@ PyObject* py_gdn_gate(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   TORCH_CHECK(!dt_bias.defined() || dt_bias.sizes() == A_log.sizes(), "dt_bias must be [", A_log.size(0), "], got ", dt_bias.defined() ? shape_text(dt_bias) : "");
   TORCH_CHECK(!b.defined() || b.sizes() == a.sizes(), "b ", b.defined() ? shape_text(b) : "", " must have a's shape ", shape_text(a));
   refuse_tangents("gated_deltanet_gate", {&a, &A_log, &dt_bias, &b});
-  if (wants_grad({&a, &A_log, &dt_bias, &b})) {
-    const variable_list r = GdnGateFn::apply(a, opt(b), A_log, opt(dt_bias), beta_scale);
-    return pack(r[0], r.size() > 1 ? r[1] : Tensor());
-  }
-  const auto r = gdn_forward(a.contiguous(), b.defined() ? b.to(a.scalar_type()).contiguous() : b, f32(A_log), f32(dt_bias), beta_scale);
+  const auto r = without_lock([&]() -> std::pair<Tensor, Tensor> {
+    if (wants_grad({&a, &A_log, &dt_bias, &b})) {
+      const variable_list r = GdnGateFn::apply(a, opt(b), A_log, opt(dt_bias), beta_scale);
+      return {r[0], r.size() > 1 ? r[1] : Tensor()};
+    }
+    return gdn_forward(a.contiguous(), b.defined() ? b.to(a.scalar_type()).contiguous() : b, f32(A_log), f32(dt_bias), beta_scale);
+  });
   return pack(r.first, r.second);
   LNX_END
 }
@@ -882,14 +920,14 @@ PyObject* py_kda_gate(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   TORCH_CHECK(!g_bias.defined() || (g_bias.dim() == 1 && g_bias.size(0) == g.size(2)), "g_bias must be [", g.size(2), "], got ", g_bias.defined() ? shape_text(g_bias) : "");
   refuse_tangents("kda_gate", {&g, &A_log, &g_bias, &beta});
   const int64_t out_dtype = in.is_none(6) ? code_of(g.scalar_type()) : in.integer(6);
-  const Tensor out = wants_grad({&g, &A_log, &g_bias}) ? KdaGateFn::apply(g, A_log, opt(g_bias), dk, threshold, out_dtype)
-                                                       : kda_gate_forward(g.contiguous(), f32(A_log), f32(g_bias), dk, threshold, out_dtype);
-  Tensor b;
-  if (beta.defined()) {
-    TORCH_CHECK(beta.is_cuda(), "beta is on ", beta.device().str(), "; the op runs on the GPU only");
-    b = wants_grad({&beta}) ? SigmoidFn::apply(beta) : sigmoid_forward(f32(beta));
-  }
-  return pack(out, b);
+  TORCH_CHECK(!beta.defined() || beta.is_cuda(), "beta is on ", beta.defined() ? beta.device().str() : "", "; the op runs on the GPU only");
+  const auto r = without_lock([&]() -> std::pair<Tensor, Tensor> {
+    const Tensor out = wants_grad({&g, &A_log, &g_bias}) ? KdaGateFn::apply(g, A_log, opt(g_bias), dk, threshold, out_dtype)
+                                                         : kda_gate_forward(g.contiguous(), f32(A_log), f32(g_bias), dk, threshold, out_dtype);
+    if (!beta.defined()) return {out, Tensor()};
+    return {out, wants_grad({&beta}) ? SigmoidFn::apply(beta) : sigmoid_forward(f32(beta))};
+  });
+  return pack(r.first, r.second);
   LNX_END
 }
 
@@ -1024,7 +1062,8 @@ PyObject* py_dplr(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   check_dplr(q, k, v, a, b, gk, 4);
   TORCH_CHECK(!s0.defined() || s0.sizes() == at::IntArrayRef({q.size(0), q.size(1), q.size(3), v.size(3)}), "initial_state shape ",
               s0.defined() ? shape_text(s0) : "", " != (", q.size(0), ", ", q.size(1), ", ", q.size(3), ", ", v.size(3), ")");
-  const auto r = dplr_scan(q, k, v, a, b, gk, s0, in.number(6));
+  const double scale = in.number(6);
+  const auto r = without_lock([&] { return dplr_scan(q, k, v, a, b, gk, s0, scale); });
   return pack(r.first, r.second);
   LNX_END
 }
@@ -1041,14 +1080,18 @@ PyObject* py_dplr_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   check_dplr(q, k, v, a, b, gk, 3);
   TORCH_CHECK(state.sizes() == at::IntArrayRef({q.size(0), q.size(1), q.size(2), v.size(2)}), "state shape ", shape_text(state), " != (", q.size(0), ", ", q.size(1), ", ",
               q.size(2), ", ", v.size(2), ")");
-  if (wants_grad({&q, &k, &v, &a, &b, &gk, &state})) {
-    TORCH_CHECK(!inplace, "cannot differentiate through a step that updates its state in place");
-    const auto r = dplr_scan(q.unsqueeze(2), k.unsqueeze(2), v.unsqueeze(2), a.unsqueeze(2), b.unsqueeze(2), gk.unsqueeze(2), state, scale);
-    return pack(r.first.squeeze(2), r.second);
-  }
+  const bool grad = wants_grad({&q, &k, &v, &a, &b, &gk, &state});
+  TORCH_CHECK(!grad || !inplace, "cannot differentiate through a step that updates its state in place");
   TORCH_CHECK(!inplace || (state.scalar_type() == at::kFloat && state.is_contiguous()), "inplace=True needs a contiguous float32 state");
-  const Tensor s_in = f32(state), s_out = inplace ? state : at::empty_like(s_in);
-  return pack(dplr_call(true, q.contiguous(), k.contiguous(), v.contiguous(), a.contiguous(), b.contiguous(), f32(gk), s_in, s_out, scale), s_out);
+  const auto r = without_lock([&]() -> std::pair<Tensor, Tensor> {
+    if (grad) {
+      const auto r = dplr_scan(q.unsqueeze(2), k.unsqueeze(2), v.unsqueeze(2), a.unsqueeze(2), b.unsqueeze(2), gk.unsqueeze(2), state, scale);
+      return {r.first.squeeze(2), r.second};
+    }
+    const Tensor s_in = f32(state), s_out = inplace ? state : at::empty_like(s_in);
+    return {dplr_call(true, q.contiguous(), k.contiguous(), v.contiguous(), a.contiguous(), b.contiguous(), f32(gk), s_in, s_out, scale), s_out};
+  });
+  return pack(r.first, r.second);
   LNX_END
 }
 
