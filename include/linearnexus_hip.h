@@ -154,11 +154,13 @@ int lnx_chunk_fwd(const lnx_scan_args* a, void* hip_stream);
  * parallel, for calls with too few (head, value slab) chains to fill the GPU.  The scan is linear in the state: a first pass
  * from [0 | I] leaves [B_i | A_i] with S_out = A_i S_in + B_i per segment, these are chained, and a second pass from the
  * chained states gives the outputs.  nseg must be the number of segments of ceil(ceil(T / 64) / nseg) chunks that T tokens
- * make.  final_state is [nseg, H, dk, dv] here: the states at the end of every segment, the last one being the final state.
+ * make.  final_state is [nseg, H, dk, dv] here: the states at the end of every segment, the last one being the final state;
+ * for lnx_chunk_fwd_segmented_final it is [H, dk, dv], the final state alone.
  * The workspace takes lnx_chunk_fwd_segmented_bytes(a, nseg).
  */
 uint64_t lnx_chunk_fwd_segmented_bytes(const lnx_scan_args* a, int32_t nseg);
 int lnx_chunk_fwd_segmented(const lnx_scan_args* a, int32_t nseg, void* hip_stream);
+int lnx_chunk_fwd_segmented_final(const lnx_scan_args* a, int32_t nseg, void* hip_stream);
 /*
  * 1 when lnx_chunk_fwd / lnx_chunk_bwd apply the in-op normalisation of q and k themselves for these arguments
  * (use_qk_l2norm = 1: gated_deltanet.py:273-275, kda.py:379-381 normalise inside the op, and it is their default):

@@ -188,6 +188,14 @@ inline bool lnx_narrow_slabs(int64_t wide_workgroups, int forced) {
   return wide_workgroups <= 128;
 }
 
+// Where the final states go: state i (of dk x dv floats) to all + i, but from state `from` on to last + i - from.
+struct FinalStates {
+  float* all;
+  float* last;
+  int from;
+  __device__ __forceinline__ float* at(int sidx, int64_t size) const { return sidx < from ? all + sidx * size : last + (sidx - from) * size; }
+};
+
 // Arguments of the kernels of chunk_direct.hip (2-byte inputs).
 struct DirectParams {
   ChunkGeom geom;
@@ -196,7 +204,7 @@ struct DirectParams {
   const bf16_t* v;
   const float* beta;
   const float* s0;
-  float* sT_out;
+  FinalStates sT_out;
   void* o;
   int dv, o_dtype;
   int save;   // forward scan: write the state entering every chunk (the backward pass reads it)

@@ -418,7 +418,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     for (int ci = 0; ci < KT; ++ci) S16::mma(S[ci], fu[1][ci], bu1);
     lds_barrier();  // B1 of the next chunk
   }
-  float* out = p.sT_out + (int64_t)sidx * DK * p.dv + v0 + vs + l16;
+  float* out = p.sT_out.at(sidx, (int64_t)DK * p.dv) + v0 + vs + l16;
 #pragma unroll
   for (int ci = 0; ci < KT; ++ci)
 #pragma unroll

@@ -14,6 +14,7 @@
 // (delta_net.py:296-330 without a gate, kda.py:569-648 with a vector gate); E_ij =
 // exp(G_i - G_j) with G the cumulative log-decay inside the chunk.
 
+#include <climits>
 #include <algorithm>
 #include <cstdlib>
 #include <mutex>
@@ -31,7 +32,7 @@ struct FwdParams {
   const float* beta;
   const float* g;
   const float* s0;
-  float* sT_out;
+  FinalStates sT_out;
   void* o;
   int dv, o_dtype;
   int save;  // write the per-chunk tensors the backward pass (or the separate output kernel) reads
@@ -1211,7 +1212,7 @@ __global__ __launch_bounds__(512) void chunk_scan_kernel(FwdParams p) {
     lds_barrier();  // B1 of the next chunk
   }
 
-  float* out = p.sT_out + (int64_t)sidx * DK * p.dv + v0;
+  float* out = p.sT_out.at(sidx, (int64_t)DK * p.dv) + v0;
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
@@ -1517,8 +1518,9 @@ int launch_direct_fwd(const lnx_scan_args* a, const FwdParams& p, int nstate, bo
 }
 
 // The forward pass on a caller-chosen workspace (a->workspace is not looked at).  `prepared`: the same call but for v, dv and
-// the states has just used this workspace, whose sequence table and value-independent tensors are taken over.
-int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_bytes, hipStream_t st, bool prepared = false) {
+// the states has just used this workspace, whose sequence table and value-independent tensors are taken over.  `last`: where the last
+// sequence's final states go instead of into a->final_state.
+int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_bytes, hipStream_t st, bool prepared = false, float* last = nullptr) {
   const bool packed = a->cu_seqlens != nullptr;
   const int nstate = packed ? a->nseq : a->B;
   if (nstate == 0) return LNX_OK;
@@ -1544,7 +1546,8 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
   p.geom.cu = a->cu_seqlens;
   p.geom.tab = packed ? reinterpret_cast<const int32_t*>(ws + w.tab) : nullptr;
   p.q = a->q; p.k = a->k; p.v = a->v; p.beta = a->beta; p.g = a->g; p.s0 = a->initial_state;
-  p.sT_out = a->final_state; p.o = a->o; p.dv = a->dv; p.o_dtype = a->o_dtype; p.scale = a->scale;
+  p.sT_out = last ? FinalStates{a->final_state, last, (nstate - 1) * a->H} : FinalStates{a->final_state, nullptr, INT_MAX};
+  p.o = a->o; p.dv = a->dv; p.o_dtype = a->o_dtype; p.scale = a->scale;
   // 4-byte inputs form the outputs in a separate kernel that reads the state and D back
   p.save = !(a->forward_only && a->dtype == LNX_BF16);
   p.out_spw = a->test_out_slabs;
@@ -1714,7 +1717,7 @@ extern "C" uint64_t lnx_chunk_fwd_segmented_bytes(const lnx_scan_args* a, int32_
   return Segmented(a, nseg).total;
 }
 
-extern "C" int lnx_chunk_fwd_segmented(const lnx_scan_args* a, int32_t nseg, void* stream) {
+static int fwd_segmented(const lnx_scan_args* a, int32_t nseg, bool every_state, void* stream) {
   int rc = lnx_chunk_check(a, false);
   if (rc != LNX_OK) return rc;
   if (a->B != 1 || a->T <= 0 || a->cu_seqlens || !a->forward_only || !a->o || a->value_cols != 0 || nseg <= 0)
@@ -1736,8 +1739,13 @@ extern "C" int lnx_chunk_fwd_segmented(const lnx_scan_args* a, int32_t nseg, voi
   auto chain = a->dk == 256 ? segment_chain_kernel<256> : a->dk == 128 ? segment_chain_kernel<128> : segment_chain_kernel<64>;
   lnx_profile_mark("segment_chain", st);
   hipLaunchKernelGGL(chain, dim3(a->H, a->dv / 16), dim3(a->dk == 64 ? 256 : 512), 0, st, ab, a->initial_state, s_in, g.n, a->H, a->dv);
-  return chunk_fwd_on(&g.second, ws, g.ws_bytes, st, lnx_chunk_direct(a));
+  if (every_state) return chunk_fwd_on(&g.second, ws, g.ws_bytes, st, lnx_chunk_direct(a));
+  g.second.final_state = s_in;  // the states at the other segments' ends: nobody reads them
+  return chunk_fwd_on(&g.second, ws, g.ws_bytes, st, lnx_chunk_direct(a), a->final_state);
 }
+
+extern "C" int lnx_chunk_fwd_segmented(const lnx_scan_args* a, int32_t nseg, void* stream) { return fwd_segmented(a, nseg, true, stream); }
+extern "C" int lnx_chunk_fwd_segmented_final(const lnx_scan_args* a, int32_t nseg, void* stream) { return fwd_segmented(a, nseg, false, stream); }
 
 extern "C" int lnx_chunk_fwd_static_init(void) {
   void* ws = nullptr;

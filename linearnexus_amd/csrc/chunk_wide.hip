@@ -319,7 +319,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
     if (n + 1 < c1) save(n + 1);
     lds_barrier();  // B1 of the next chunk
   }
-  S.store(p.sT_out + (int64_t)ch.sidx * DK * p.dv + v0 + vs, p.dv, fresh(tid & 63));
+  S.store(p.sT_out.at(ch.sidx, (int64_t)DK * p.dv) + v0 + vs, p.dv, fresh(tid & 63));
 }
 
 template <int GATE, int NC, int NCW>

@@ -551,7 +551,7 @@ std::pair<Tensor, Tensor> chunk_segmented(const Tensor& q0, const Tensor& k0, co
   Tensor q = as_layout(q1, tf), k = as_layout(k1, tf);
   const Tensor v = as_layout(v1, tf), beta = as_layout(fold(beta0).to(at::kFloat), tf), g = g0.defined() ? as_layout(fold(g0).to(at::kFloat), tf) : g0, s0 = f32(s00);
   const Tensor o = empty_layout(1, rows, s.T, s.dv, q.options().dtype(type_of(o_dtype)), tf);
-  const Tensor sT = at::empty({nseg, rows, s.dk, s.dv}, q.options().dtype(at::kFloat));
+  const Tensor sT = at::empty({s.B, s.H, s.dk, s.dv}, q.options().dtype(at::kFloat));
   lnx_scan_args a = base_args(1, rows, s.T, s.dk, s.dv, code_of(q.scalar_type()), (int)o_dtype, s.gate, false, scale);
   a.use_qk_l2norm = l2norm && lnx_chunk_fuses_l2norm(&a);
   if (l2norm && !a.use_qk_l2norm) std::tie(q, k) = l2norm_pair_fwd(q, k);
@@ -561,12 +561,12 @@ std::pair<Tensor, Tensor> chunk_segmented(const Tensor& q0, const Tensor& k0, co
   const uint64_t nbytes = lnx_chunk_fwd_segmented_bytes(&a, (int32_t)nseg);
   const Tensor ws = at::empty({(int64_t)std::max<uint64_t>(nbytes, 1)}, q.options().dtype(at::kByte));
   a.workspace = ptr(ws), a.workspace_bytes = nbytes;
-  check_status(lnx_chunk_fwd_segmented(&a, (int32_t)nseg, stream_of(q)), "lnx_chunk_fwd_segmented");
-  return {s.B == 1 ? o : o.reshape({s.B, s.H, s.T, s.dv}), sT.select(0, nseg - 1).view({s.B, s.H, s.dk, s.dv})};
+  check_status(lnx_chunk_fwd_segmented_final(&a, (int32_t)nseg, stream_of(q)), "lnx_chunk_fwd_segmented_final");
+  return {s.B == 1 ? o : o.reshape({s.B, s.H, s.T, s.dv}), sT};
 }
 
 // chunk_segmented(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, nseg): (o, final state) of a forward-only call on dense
-// sequences, cut into about nseg segments that run in parallel (lnx_chunk_fwd_segmented); batch rows become heads.
+// sequences, cut into about nseg segments that run in parallel (lnx_chunk_fwd_segmented_final); batch rows become heads.
 PyObject* py_chunk_segmented(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   LNX_BEGIN
   Args in(args, nargs, 10, "chunk_segmented");
