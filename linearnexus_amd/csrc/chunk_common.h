@@ -229,7 +229,6 @@ int lnx_direct_scan_fwd(const DirectParams& p, int dk, int gate, int nstate, hip
 int lnx_direct_bwd(const DirectParams& p, int dk, int gate, int nstate, hipStream_t st);
 // The sequential passes of the WY-split kernels for 2-byte inputs with dk = 256 and no / a scalar gate (chunk_wide.hip).
 int lnx_wide_scan(bool backward, const DirectParams& p, int nstate, hipStream_t st);
-inline bool lnx_wide_scans(int dtype, int dk, int gate) { return dtype == LNX_BF16 && dk == 256 && gate != LNX_GATE_VECTOR; }
 
 // Shared argument validation of the chunk entry points; returns LNX_OK or an error status.
 int lnx_chunk_check(const lnx_scan_args* a, bool backward);
