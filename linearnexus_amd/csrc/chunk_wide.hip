@@ -1,6 +1,8 @@
 // The two sequential passes of the WY-split chunk kernels for 2-byte inputs with dk = 256 and no / a scalar gate (the head shape of
-// the Gated DeltaNet presets).  Same products, roundings and order of sums as chunk_scan (chunk_fwd.hip) and bwd_scan
-// (chunk_bwd.hip), which serve the other shapes:
+// the Gated DeltaNet presets).  Same products and roundings as chunk_scan (chunk_fwd.hip) and bwd_scan (chunk_bwd.hip), which serve
+// the other shapes.  The forward sums have their order, too; in reverse Q^T dO is added before W^T dD, as bwd_scan does up to dk = 128 --
+// its 64-column slabs of dk = 256 added W^T dD first, because Q shared a tile with K -- so that gradients differ from that form's by the
+// rounding of one sum (1.2e-4 of the 2-norm in bf16):
 //
 //   forward   D = U - W S       O = scale diag(e^G) (Q S) + Pm D       S' = e^{G_C} S + (diag(e^{G_C - G}) K)^T D
 //   reverse   dD = Pm^T dO + diag(e^{G_C - G}) K dS'                   dS = e^{G_C} dS' + (scale diag(e^G) Q)^T dO - W^T dD
