@@ -78,12 +78,13 @@ struct Scal {
 // scan_fwd.  A compute wave owns a 16-column strip of the value slab: its [dk x 16] part of the state stays in MFMA
 // accumulators for the whole sequence, and the chain  S -> Y = K S -> R -> D = Tm R -> S'  never leaves the wave's
 // registers -- two accumulator tiles are the B operand of the next product as they are (Mma16::from_acc), only the A
-// operands (K, Q, Tm, Pm rows) come from LDS.  Strips of 16 columns put a slab's chain on twice as many SIMDs as strips of 32:
-// B2 H16 T2007 d128 (32 chunks in a row, 128 workgroups) 65 -> 57 us forward and 74 -> 59 us in reverse, one prompt of 1000
-// tokens 34 -> 29 us, B8 H16 T4096 204 -> 198 and 217 -> 207 us; the bits are those of 32-column strips (Mma16).  What is left of
-// a chunk's 1.5 us there: a SIMD takes 1 KB of LDS reads in about 16 cycles, and a strip reads 60 KB of operands whatever its
-// width.  The movers convert K and Q rows, 2.5 VALU instructions an element: with eight waves of them instead of four 57 -> 51 us and
-// 29 -> 25 us; in reverse the third wave of each SIMD leaves too few registers (59 -> 59 - 68 us), it keeps four.
+// operands (K, Q, Tm, Pm rows) come from LDS.  Strips of 16 columns put a slab's chain on twice as many SIMDs as strips of 32, which counts
+// where there are fewer workgroups than CUs: B2 H16 T2007 d128 (32 chunks in a row, 128 workgroups) 66 -> 57 us forward and 74 -> 60 us
+// in reverse, one prompt of 1000 tokens 34 -> 29 us.  With 256 workgroups of 64-column slabs, bound by what the movers carry, it changes
+// nothing: B8 H16 T4096 184 and 200 us before and after.  The bits are those of 32-column strips (Mma16).  What is left of a chunk's
+// 1.5 us in the short calls: a SIMD takes 1 KB of LDS reads in about 16 cycles, and a strip reads 60 KB of operands whatever its
+// width.  The movers convert K and Q rows, 2.5 VALU instructions an element: with eight waves of them instead of four 57 -> 52 us and
+// 29 -> 27 us; in reverse the third wave of each SIMD leaves too few registers (59 -> 59 - 68 us), it keeps four.
 //  All five input tiles are double-buffered, so the movers write chunk
 // n + 1 while chunk n is being read and two barriers per chunk are enough:
 //   B1    buffers of chunk n complete           compute: S^T -> LDS (saved states), Y, Q S, R, D (-> LDS, transposed), O -> LDS
