@@ -112,7 +112,7 @@ template <int N, typename F, typename G> __device__ __forceinline__ void mfma4_e
     for (int i = 0; i < N; ++i) *c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a(i)[r], b(i)[r], *c[i], 0, 0, 0);
 }
 // ... the block summed from zero: for the pairs' sums over channels, where one chain of 64 additions rounds the outputs by 1.5e-7 at RWKV-7's
-// decays and four chains of 16 by 1.1e-7 (all else exact).  Not in dplr_grad, whose registers are full: 775 -> 980 us for dq 1.7 -> 1.25e-7.
+// decays and four chains of 16 by 1.1e-7 (all else exact).  Not in dplr_grad, whose registers are full: 725 -> 866 us for dq 1.7 -> 1.25e-7.
 template <int N, typename F, typename G> __device__ __forceinline__ void mfma_block(floatx4* const (&c)[N], F&& a, G&& b) {
   floatx4 t[N];
   floatx4* pt[N];
@@ -968,7 +968,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
     Row<float> h0, hC, dC;
     hC.load(p.hT, ht + TG);
     dC.load(p.s1, wt);
-    x.load(p, s, w);
+    x.load_gates(p, s, w);
     v.load(p.v, at, ok);
     d_o.load(p.d_o, at, ok);
     u.load(p.s3, wt);
@@ -1015,7 +1015,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
   for (int cb = 0; cb < 4; ++cb) st[cb] = L.start_to1(w.j, 16 * cb + l16);
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
-    const floatx4 fo = d_o[kb], fd = du[kb], fu = u[kb], fv = v[kb];
+    const floatx4 fo = d_o[kb], fd = du[kb], fu = frag<true>(t2, w.t, 16 * kb + g4), fv = frag<true>(t0, w.t, 16 * kb + g4);
     mfma4_each<4>({&m.qb, &m.qk, &m.ab, &m.ak}, [&](int i) { return i & 1 ? fv : fu; }, [&](int i) { return i & 2 ? fd : fo; });
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {
@@ -1024,6 +1024,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
       mfma4(da[cb], hf, fd);
     }
   }
+  x.load_rows(p, s, w);  // not before: the registers are full up to here
   mask<true, false>(m.qb, w), mask<true, false>(m.qk, w), mask<true, true>(m.ab, w), mask<true, true>(m.ak, w);
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) asm volatile("" : "+v"(gates.sum[cb][0]), "+v"(gates.sum[cb][1]), "+v"(gates.sum[cb][2]), "+v"(gates.sum[cb][3]));
@@ -1076,10 +1077,12 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
     dq[cb] += dqo, da[cb] += dao;
     flow[cb] -= x.a[cb] * da[cb];
     if (ok) {
+      store4(p.dgk + at + 16 * cb, flow[cb]);  // read back at the end
       store_row4<T>(p.dq, at + 16 * cb, dq[cb] * p.scale);
       store_row4<T>(p.da, at + 16 * cb, da[cb]);
     }
   }
+  u.load(p.s3, wt), v.load(p.v, at, ok);  // again, ahead of their use: in between the registers are full
   lds_barrier();
   // db, dk, relative to the end of the lane's block: the matrices with the contraction along t, first those of q, then those of a
   floatx4 db[4], dk[4], own[4];  // own: b db + k dk of the block's own pairs
@@ -1130,12 +1133,14 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
         mfma4(ob, xf, mb);
         mfma4(ok_, xf, mk);
         db[cb] += ob, dk[cb] += ok_;
-        own[cb] += (x.b[cb] * ob + x.k[cb] * ok_) * e.s[cb];
+        own[cb] += x.b[cb] * ob + x.k[cb] * ok_;
       }
     }
   }
 #pragma unroll
-  for (int cb = 0; cb < 4; ++cb) db[cb] *= e.s[cb], dk[cb] *= e.s[cb];
+  for (int cb = 0; cb < 4; ++cb) db[cb] *= e.s[cb], dk[cb] *= e.s[cb], own[cb] *= e.s[cb];
+  Row<float> fl;
+  fl.load(p.dgk, at, ok);
   lds_barrier();
   if (gates.direct) {
     float* mine = t1 + w.t * LD;
@@ -1152,7 +1157,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) {
     const floatx4 source = x.b[cb] * db[cb] + x.k[cb] * dk[cb] - own[cb], out = sum_upto(source);  // of later blocks' sinks
-    flow[cb] += out - source - sum_from(own[cb]);
+    flow[cb] = fl[cb] + (out - source - sum_from(own[cb]));
     if (l16 == 15) store4(tout + 64 * w.j + 16 * cb + g4, out);
     if (ok) {
       store_row4<T>(p.db, at + 16 * cb, db[cb]);
@@ -1228,8 +1233,8 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
   return LNX_OK;
 }
 
-// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 497, dplr_grad 773 (66 registers spilled: everything a chunk's token needs is
-// live between the pair sums and the last products)
+// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 497, dplr_grad 725 (two workgroups per CU leave 256 registers, and what a
+// token needs between the pair sums and the last products is more: 24 are spilled, three rows are loaded twice)
 template <typename T> int backward(const lnx_dplr_chunk_grads* g, const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
   set_kept(p, kept, rows, 0, p.N);
