@@ -286,13 +286,13 @@ struct Lds {
 // The gates of the lane's block.  Sums of gates in fixed point (2^-24 in units of log 2) are exact: P and S carry the rounding of one
 // exponential each, whatever the sums' sizes.  A gate or a sum that the format does not hold, or NaN, makes the block DIRECT.
 constexpr int ONE = 1 << 24;
-__device__ __forceinline__ int fixed_gate(float g, float& size) {
+__device__ __forceinline__ int fixed_gate(float g, bool& ok) {
   const float c = 1.44269504f * ONE;
   float t = g * c;
   asm volatile("" : "+v"(t));  // -ffast-math must not see that the next line is a rounding error
   const float e = __builtin_fmaf(g, 1.92596299e-8f * ONE, __builtin_fmaf(g, c, -t));
-  size = fabsf(t);
-  return (int)__builtin_rintf(t + e);
+  ok = fabsf(t) <= 7.f * ONE;  // sixteen of them stay below 2^31
+  return ok ? (int)__builtin_rintf(t + e) : 0;
 }
 __device__ __forceinline__ float exp2_fixed(int x) { return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((float)(x & (ONE - 1)) * (1.f / ONE)), x >> 24); }
 template <int CTRL> __device__ __forceinline__ int dpp_of(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, true); }
@@ -306,9 +306,9 @@ struct Gates {
       const floatx4 g = gk[cb];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float size;
-        int x = fixed_gate(g[e], size);
-        fits = fits && size <= 8.f * ONE;  // sixteen of them stay below 2^31
+        bool ok;
+        int x = fixed_gate(g[e], ok);
+        fits = fits && ok;
         x += dpp_of<0x111>(x), x += dpp_of<0x112>(x), x += dpp_of<0x114>(x), x += dpp_of<0x118>(x);  // row_shr 1, 2, 4, 8
         fits = fits && abs(x) <= RANGE * ONE;
         sum[cb][e] = x;

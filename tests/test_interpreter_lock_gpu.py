@@ -58,3 +58,34 @@ def test_other_threads_run_during_an_op(name):
     torch.cuda.synchronize()
     print(f"the other thread ran after {calls} calls" if seen else f"not during {calls} calls")
     assert seen
+
+
+@pytest.mark.parametrize("anomaly", [False, True])
+def test_python_hooks_run_inside_the_ops(anomaly):
+    """Saved-tensor hooks and the anomaly mode call into the interpreter while a node is made: they take the lock themselves."""
+    import linearnexus_amd as la
+    torch.manual_seed(0)
+    r = lambda *s: torch.randn(*s, device=DEV).requires_grad_(True)
+    B, T, H, d = 1, 70, 2, 64
+    leaves = [r(B, T, H * d), r(4, H * d), r(B, T, H), r(H), r(B, T, H, d), r(d)]
+
+    def loss():
+        x, w, a, A_log, gate, norm = leaves
+        y = la.depthwise_conv1d_causal(x, w, None, activation="silu")[0].view(B, T, H, d).transpose(1, 2)
+        g, beta = la.gated_deltanet_gate(a, A_log, None, a)
+        o, S = la.gated_delta_rule_chunkwise(y, y, y, g.transpose(1, 2), beta.transpose(1, 2))
+        p, _ = la.dplr_delta_rule_recurrent(y, y, y, -y * 0.1, y * 0.1, -y.abs())
+        return la.rmsnorm_gated((o + p).transpose(1, 2), gate, norm).square().sum() + S.square().sum()
+
+    want = torch.autograd.grad(loss(), leaves)
+    packed = []
+
+    def pack(t):
+        packed.append(t.shape)
+        return t.clone()
+
+    with torch.autograd.set_detect_anomaly(anomaly), torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        got = torch.autograd.grad(loss(), leaves)
+    assert len(packed) > 20
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4)
