@@ -473,9 +473,9 @@ def bench_dplr_step(torch, la, _lib, steps):
 
 def bench_dplr_train(torch, la, _lib, steps, warmup):
     """RWKV-7 DPLR scan forward + backward at B8 H16 T4096 dk=dv=64 bf16 (the block's head size 64): tokens/s, and the
-    backward kernel against the HBM roofline.  Algorithmic bytes of the backward: every token's starting state is written
-    to the segment tape and read back once (2 * 4 B per state element and token; the checkpoints add 1/64 of that), the
-    token vectors are read three times (checkpoint sweep, tape sweep, reverse sweep), six fp32 gradients leave."""
+    largest kernel (dplr_grad) against the fp32 matrix peak: per chunk of 64 tokens the four pair matrices over 64 value columns
+    and the eight products of them with token rows, each on the ten 16 x 16 blocks of the lower triangle, and four full
+    64 x 64 x 64 products with the state and its gradient."""
     B, H, T, d = 8, 16, 4096, 64
     gen = torch.Generator(device="cpu").manual_seed(9)
     rn = lambda *s: torch.randn(*s, generator=gen, dtype=torch.float32)
@@ -505,16 +505,16 @@ def bench_dplr_train(torch, la, _lib, steps, warmup):
         acc.setdefault(n, []).append(ms)
     _lib.profile_enable(False)
     avg = {n: sum(x) / len(x) for n, x in acc.items()}
-    tok = B * H * T
-    nbytes = tok * d * d * 4 * (2 + 1 / 64) + 3 * tok * (5 * d * 2 + d * 4 + d * 2) + tok * d * 2 + 6 * tok * d * 4
-    ach = nbytes / (avg["dplr_bwd"] * 1e-3) / 1e9
+    flops = B * H * (T // 64) * 2 * (10 * 16 * 16 * d * (4 + 8) + 4 * 64 * d * d)
+    ach = flops / (avg["dplr_grad"] * 1e-3) / 1e12
+    tr, tr_src = measured_traffic("dplr_train", "dplr_grad")
     return {"metric": "DPLR scan fwd+bwd tokens/s", "value": B * T / dt, "unit": "tokens/s", "n_gpus": 1, "steps": steps,
             "warmup": warmup, "ms_per_step": dt * 1e3, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
             "dtype": "f32", "data": "synthetic",
             "config": {"workload": "rwkv7_dplr_scan_fwd_bwd", "B": B, "H": H, "T": T, "dk": d, "dv": d, "inputs": "bf16, fp32 gk"},
             "kernel_ms": {n: round(x, 4) for n, x in avg.items()},
-            "roofline": {"bound": "hbm", "kernel": "dplr_bwd", "achieved": ach, "peak": PEAK_HBM, "unit": "GB/s",
-                         "frac": ach / PEAK_HBM, "traffic": None}}
+            "roofline": {"bound": "mfma", "kernel": "dplr_grad", "achieved": ach, "peak": PEAK_FP32_MFMA, "unit": "TFLOP/s",
+                         "frac": ach / PEAK_FP32_MFMA, "traffic": tr, "traffic_source": tr_src}}
 
 
 def bench_rmsnorm_gated(torch, la, _lib, steps, warmup):
