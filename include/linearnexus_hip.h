@@ -242,7 +242,8 @@ int lnx_conv1d_packed_bwd(const void* x, const float* weight, const float* bias,
                           const void* dy, void* dx, float* d_weight, float* d_bias, int32_t T, int32_t D, int32_t K,
                           int32_t dtype, int32_t activation, void* hip_stream);
 /* The same pair without the backward pass's fill kernel: the forward kernel clears `nzeroed` floats on its way, and
- * lnx_conv1d_bwd_add adds to a d_weight and d_bias cleared like that.  cu_seqlens NULL: a dense batch. */
+ * lnx_conv1d_bwd_add adds to a d_weight and d_bias cleared like that -- once: a backward call that is captured in a graph of
+ * its own and replayed would add to its own sums (use lnx_conv1d_bwd there).  cu_seqlens NULL: a dense batch. */
 int lnx_conv1d_fwd_zero(const void* x, const float* weight, const float* bias, const void* cache, const int32_t* cu_seqlens, int32_t nseq,
                         void* y, void* new_cache, float* zeroed, int64_t nzeroed, int32_t B, int32_t T, int32_t D, int32_t K,
                         int32_t dtype, int32_t activation, void* hip_stream);
@@ -309,9 +310,10 @@ int lnx_dplr_recurrent_bwd(const lnx_dplr_bwd_args* a, void* hip_stream);
  * lnx_dplr_recurrent_fwd with o_dtype == dtype and 16-byte aligned tensors; the forward call leaves what the backward call
  * needs in `kept` (NULL: no backward pass will follow).  lnx_dplr_chunk_bytes gives the bytes of `kept` (LNX_DPLR_KEPT, both
  * calls) and of the scratch areas (forward with kept, forward without, backward), which hold nothing between calls and are
- * bounded (about 1 GiB) however long the sequence is.  The token gradients dq,
- * dk, dv, da, db have args->dtype; dgk and d_initial_state (may be NULL) are fp32; d_final_state may be NULL (zero).  No
- * atomics: the result is the same from run to run.
+ * bounded (about 1 GiB) however long the sequence is.  `kept` is 48 KB per chunk of a row; the token kernels keep nothing between
+ * the passes.  The token gradients dq, dk, dv, da, db have args->dtype; dgk (read back within the call) and d_initial_state
+ * (may be NULL) are fp32; d_final_state may be NULL (zero).  Gates may be anything that the token kernels take, down to -inf.
+ * No atomics: the result is the same from run to run.
  */
 enum { LNX_DPLR_KEPT = 0, LNX_DPLR_FWD_SCRATCH = 1, LNX_DPLR_BWD_SCRATCH = 2, LNX_DPLR_ONLY_SCRATCH = 3 };
 typedef struct lnx_dplr_chunk_grads {
