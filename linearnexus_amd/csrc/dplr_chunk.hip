@@ -28,8 +28,8 @@
 // Sums that carry the recent tokens' large terms take the far ones first, and a sum of two products is added up from two chains: what
 // comes second on one chain would be rounded at the size of the whole, 64 times.  Errors against fp64, relative 2-norms, one row of 512
 // tokens with RWKV-7's decays (behind a reset of any size the same), in brackets the token kernels: o 1.2e-7 (1.0), h 0.7e-7 (0.6), dq,
-// dk, dv 1.7, 1.8, 1.2e-7 (0.9), da, db 2.2e-7 (1.3), dgk 5.5e-7 (1.2), dh0 1.1e-7 (0.8); with gates a hundredth of that o 2.5e-7 (4.7),
-// gradients 2.3 - 4.4e-7 (4.7 - 7.4): there the token kernels round the state at every token.
+// dk, dv 1.2e-7 (0.9), da, db 1.8, 1.7e-7 (1.3), dgk 2.4e-7 (1.2), dh0 1.1e-7 (0.8); with gates a hundredth of that o 2.5e-7 (4.7),
+// gradients 2.3 - 4.1e-7 (4.7 - 7.4): there the token kernels round the state at every token.
 //
 // Kernels, each a workgroup per chunk but for the two sequential passes: the launch functions name them with their times.
 #include "lnx_common.h"
@@ -112,7 +112,8 @@ template <int N, typename F, typename G> __device__ __forceinline__ void mfma4_e
     for (int i = 0; i < N; ++i) *c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a(i)[r], b(i)[r], *c[i], 0, 0, 0);
 }
 // ... the block summed from zero: for the pairs' sums over channels, where one chain of 64 additions rounds the outputs by 1.5e-7 at RWKV-7's
-// decays and four chains of 16 by 1.1e-7 (all else exact).  Not in dplr_grad, whose registers are full: 725 -> 866 us for dq 1.7 -> 1.25e-7.
+// decays and four chains of 16 by 1.1e-7 (all else exact).  In dplr_grad it costs four spilled registers, 750 -> 771 us, for dq 1.62 -> 1.15e-7,
+// dk 1.65 -> 1.19, da 2.2 -> 1.8, db 2.1 -> 1.7, dgk 2.7 -> 2.4.
 template <int N, typename F, typename G> __device__ __forceinline__ void mfma_block(floatx4* const (&c)[N], F&& a, G&& b) {
   floatx4 t[N];
   floatx4* pt[N];
@@ -199,6 +200,11 @@ template <typename T> struct Row {
   }
   __device__ __forceinline__ floatx4 operator[](int cb) const { return ok ? x[cb].get() : zero4(); }
 };
+// What was read, not what it was converted to, is what a kernel short of registers keeps from here on
+template <typename T> __device__ __forceinline__ void keep_as_read(Row<T>& r) {
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) asm volatile("" : "+v"(r.x[cb].x));
+}
 // ... into its row of a tile
 template <typename F> __device__ __forceinline__ void put_row(float* tile, const Lane& w, F&& value) {
 #pragma unroll
@@ -901,7 +907,7 @@ template <typename T> struct DirectRows {
     return ok ? floatx4{exp_f(g[0]), exp_f(g[1]), exp_f(g[2]), exp_f(g[3])} : floatx4{1.f, 1.f, 1.f, 1.f};
   }
 };
-// of earlier tokens to dq and da; m: the lane's row with dPqb, dPqk, dAab, dAak at columns 0, 16, 32, 48
+// of earlier tokens to dq and da (a token's own b and k apart); m: the lane's row with dPqb, dPqk, dAab, dAak at columns 0, 16, 32, 48
 template <typename T> __device__ __forceinline__ void direct_sinks(const DirectRows<T>& row, const float* m, int ch, floatx4& dq, floatx4& da) {
   const int t = row.w.l16;
   floatx4 e = {1.f, 1.f, 1.f, 1.f}, el = e;
@@ -945,11 +951,31 @@ __device__ __forceinline__ floatx4 sum_from(floatx4 x) { return dpp_add<0x108>(d
 __device__ __forceinline__ floatx4 sum_upto(floatx4 x) { return dpp_add<0x118>(dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(x)))); }  // row_shr
 __device__ __forceinline__ floatx4 sum_block(floatx4 x) { return dpp_add<0x128>(dpp_add<0x124>(dpp_add<0x122>(dpp_add<0x121>(x)))); }  // row_ror
 
+// Of another lane in the row of 16, 0 where there is none
+template <int CTRL> __device__ __forceinline__ floatx4 dpp_move(floatx4 x) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = __int_as_float(dpp_of<CTRL>(__float_as_int(x[e])));
+  return x;
+}
+// Of two rows whose difference sums up to 0 over the block, the difference from the lane on: from lane 8 on that sum, below minus what lies
+// before, half as many terms (without bank masks, which keep the additions from taking a DPP operand: 760 us against 750)
+__device__ __forceinline__ floatx4 to_middle(floatx4 x) {
+  const floatx4 from = dpp_add<0x104>(dpp_add<0x102>(dpp_add<0x101>(x)));                   // right in lanes 8 to 15
+  const floatx4 upto = dpp_move<0x111>(dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(x))));  // right in lanes 0 to 7
+  return threadIdx.x & 8 ? from : -upto;
+}
+
 // dgk_t is what flows through the decay of token t: pairs of a source (b or k of a token before t, the state entering) and a sink (q of t or
 // later, a of a later token, the state's gradient).  The formula at the top takes it from sums over the rest of the chunk, where a pair
-// behind t is added at its sink and taken away at its source, and all of their roundings stay (8.8e-7 of dgk against 7.4e-7, the rest as it
-// was then).  Here only pairs inside a block of 16 are treated that way; pairs of two blocks are sums of sinks from t on and of sources
-// before t, and what passes a whole block is <D, h'> less the sources and plus the sinks of the blocks behind it.
+// behind t is added at its sink and taken away at its source, and their roundings stay: what does not flow through t is left out here.
+//   in t's block   sinks from t on of sources in earlier blocks, sources before t of sinks in later ones: nothing to take away
+//   past the block sinks in later blocks of sources in earlier ones: a later block adds up its sinks before each earlier block's sources are
+//                  added (`over`), the state's gradient takes sources block by block (`out_of`) and the state entering as <D, e_C h> (`through`)
+//   pairs inside   both, over the half of the block that has fewer of them (to_middle).  A q with its own token's b and k passes no decay: dPqb
+//                  and dPqk lose their diagonals, which go to dq, db and dk by themselves.
+// dgk's error against fp64, 1e-7 of its 2-norm, with RWKV-7's decays, a hundredth of those, ten times those: 5.7, 4.4, 26 with sums over the
+// block and <D, h'> less what does not pass, 4.6, 4.3, 5.0 (21 in the last chunk under a state's gradient) with the diagonals apart, 3.3,
+// 3.6, 4.1 with `over` and `out_of`, 2.7, 3.6, 3.1 with to_middle, 2.4, 3.5, 2.9 as it is (mfma_block); dplr_grad 725, 714, 735, 750, 771 us.
 template <typename T>
 __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
   extern __shared__ __align__(16) char smem[];
@@ -958,15 +984,17 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
   const Lane w;
   const int l16 = w.l16, g4 = 4 * w.g;
   float *t0 = L.tile(0), *t1 = L.tile(1), *t2 = L.tile(2), *t3 = L.tile(3);
-  float *tin = L.sx, *tout = L.sx + 256, *red = L.sx + 512;  // [4][64] per channel: the blocks' sinks and sources, parts of <D, h'>
+  float* through = L.sx;                             // [4][64] per channel: parts of <D, h>
+  float* over = L.sx + 256;                          // [6][64]: row l (l - 1) / 2 + m has what flows into block l from before block m
+  float* out_of = L.sx + 640;                        // [3][64]: from block j to D
+  float *same_b = L.sx + 832, *same_k = L.sx + 896;  // [64]: the diagonals of dPqb and dPqk
   const int64_t at = (s.tok + w.t) * D + g4, wt = s.win * TG + w.t * D + g4, ht = s.st * TG + w.t * D + g4;
   const bool ok = w.t < s.len;
   Own<T> x;
   Row<T> v, d_o;
   Row<float> u, du;
   {
-    Row<float> h0, hC, dC;
-    hC.load(p.hT, ht + TG);
+    Row<float> h0, dC;
     dC.load(p.s1, wt);
     x.load_gates(p, s, w);
     v.load(p.v, at, ok);
@@ -976,8 +1004,8 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
     h0.load(p.hT, ht);
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {  // the wave's sixteen value columns
-      const floatx4 y = sum_block(dC[cb] * hC[cb]);
-      if (l16 == 0) store4(red + 64 * w.j + 16 * cb + g4, y);
+      const floatx4 y = sum_block(dC[cb] * h0[cb]);
+      if (l16 == 0) store4(through + 64 * w.j + 16 * cb + g4, y);
     }
     put_row(t0, w, [&](int cb) { return v[cb]; });
     put_row(t2, w, [&](int cb) { return u[cb]; });
@@ -1005,7 +1033,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
       const floatx4 fu = frag<true>(t2, 16 * sb + l16, 16 * kb + g4), fv = frag<true>(t0, 16 * sb + l16, 16 * kb + g4), fo = d_o[kb], fd = du[kb];
-      mfma4_each<4>({&pb[sb], &pk[sb], &nb_[sb], &nk[sb]}, [&](int i) { return i & 1 ? fv : fu; }, [&](int i) { return i & 2 ? fd : fo; });
+      mfma_block<4>({&pb[sb], &pk[sb], &nb_[sb], &nk[sb]}, [&](int i) { return i & 1 ? fv : fu; }, [&](int i) { return i & 2 ? fd : fo; });
     }
   });
   floatx4 dq[4], da[4];  // rows = channels, columns = tokens
@@ -1016,7 +1044,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
     const floatx4 fo = d_o[kb], fd = du[kb], fu = frag<true>(t2, w.t, 16 * kb + g4), fv = frag<true>(t0, w.t, 16 * kb + g4);
-    mfma4_each<4>({&m.qb, &m.qk, &m.ab, &m.ak}, [&](int i) { return i & 1 ? fv : fu; }, [&](int i) { return i & 2 ? fd : fo; });
+    mfma_block<4>({&m.qb, &m.qk, &m.ab, &m.ak}, [&](int i) { return i & 1 ? fv : fu; }, [&](int i) { return i & 2 ? fd : fo; });
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {
       const floatx4 hf = frag<false>(t1, 16 * cb + l16, 16 * kb + g4) * st[cb];
@@ -1025,16 +1053,26 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
     }
   }
   x.load_rows(p, s, w);  // not before: the registers are full up to here
-  mask<true, false>(m.qb, w), mask<true, false>(m.qk, w), mask<true, true>(m.ab, w), mask<true, true>(m.ak, w);
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (g4 + r == l16) same_b[w.t] = m.qb[r], same_k[w.t] = m.qk[r];  // read by this wave alone, behind barriers
+  mask<true, true>(m.qb, w), mask<true, true>(m.qk, w), mask<true, true>(m.ab, w), mask<true, true>(m.ak, w);
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) asm volatile("" : "+v"(gates.sum[cb][0]), "+v"(gates.sum[cb][1]), "+v"(gates.sum[cb][2]), "+v"(gates.sum[cb][3]));
   const Decay e(gates, p, s, w);  // formed here, not kept from the totals on: the registers are full in between
   lds_barrier();
   put_row(t0, w, [&](int cb) { return x.b[cb] * e.s[cb]; });
   put_row(t2, w, [&](int cb) { return x.k[cb] * e.s[cb]; });
+  keep_as_read(x.b), keep_as_read(x.k);
   lds_barrier();
   before(w.j, [&](auto sb_) {
     constexpr int sb = decltype(sb_)::value;
+    keep_as_read(x.q), keep_as_read(x.a);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) {
+      const floatx4 y = sum_block(p.scale * x.q[cb] * e.p[cb] * dq[cb] + x.a[cb] * token_before(e.p[cb]) * da[cb]);
+      if (l16 == 0) store4(over + 64 * (w.j * (w.j - 1) / 2 + sb) + 16 * cb + g4, y);
+    }
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {
       const float gap = L.from1<sb>(w.j, 16 * cb + l16);
@@ -1054,7 +1092,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
     __builtin_amdgcn_wave_barrier();
   }
   const DirectRows<T> rows{p, s, w};
-  floatx4 flow[4];  // dgk so far: of sinks from the lane's token on, less a da of the token itself
+  floatx4 flow[4];  // dgk so far: of the q from the lane's token on and the a behind it
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) {
     const floatx4 pl = token_before(e.p[cb]), q = p.scale * x.q[cb];
@@ -1070,18 +1108,15 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
       direct_sinks<T>(rows, t1 + w.t * LD, 16 * cb + g4, dqo, dao);
     }
     dq[cb] *= e.p[cb], da[cb] *= pl;
-    const floatx4 sink = q * dq[cb] + x.a[cb] * da[cb];  // of earlier blocks' sources
-    const floatx4 in = sum_block(sink);
-    if (l16 == 0) store4(tin + 64 * w.j + 16 * cb + g4, in);
-    flow[cb] = sum_from(sink + q * dqo + x.a[cb] * dao);
-    dq[cb] += dqo, da[cb] += dao;
-    flow[cb] -= x.a[cb] * da[cb];
+    flow[cb] = sum_from(q * dq[cb] + dpp_move<0x101>(x.a[cb] * da[cb])) + (to_middle(q * dqo + x.a[cb] * dao) - x.a[cb] * dao);  // row_shl:1
+    dq[cb] += dqo + (same_b[w.t] * x.b[cb] + same_k[w.t] * x.k[cb]), da[cb] += dao;
     if (ok) {
       store4(p.dgk + at + 16 * cb, flow[cb]);  // read back at the end
       store_row4<T>(p.dq, at + 16 * cb, dq[cb] * p.scale);
       store_row4<T>(p.da, at + 16 * cb, da[cb]);
     }
   }
+  keep_as_read(x.b), keep_as_read(x.k), keep_as_read(x.q), keep_as_read(x.a);
   u.load(p.s3, wt), v.load(p.v, at, ok);  // again, ahead of their use: in between the registers are full
   lds_barrier();
   // db, dk, relative to the end of the lane's block: the matrices with the contraction along t, first those of q, then those of a
@@ -1109,6 +1144,15 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
           mfma4(dk[cb], df, fv);
         }
       }
+    }
+    if (!half && w.j < 3) {
+      keep_as_read(x.b), keep_as_read(x.k);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) {
+        const floatx4 y = sum_block((x.b[cb] * db[cb] + x.k[cb] * dk[cb]) * e.s[cb]);
+        if (l16 == 0) store4(out_of + 64 * w.j + 16 * cb + g4, y);
+      }
+      keep_as_read(x.b), keep_as_read(x.k);
     }
     floatx4 dbh[4], dkh[4];  // apart from the other half's sums
     clear(dbh), clear(dkh);
@@ -1141,6 +1185,9 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
   for (int cb = 0; cb < 4; ++cb) db[cb] *= e.s[cb], dk[cb] *= e.s[cb], own[cb] *= e.s[cb];
   Row<float> fl;
   fl.load(p.dgk, at, ok);
+  int64_t again = at;
+  asm volatile("" : "+v"(again));  // its addresses are formed here
+  x.q.load(p.q, again, ok);
   lds_barrier();
   if (gates.direct) {
     float* mine = t1 + w.t * LD;
@@ -1157,8 +1204,9 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) {
     const floatx4 source = x.b[cb] * db[cb] + x.k[cb] * dk[cb] - own[cb], out = sum_upto(source);  // of later blocks' sinks
-    flow[cb] = fl[cb] + (out - source - sum_from(own[cb]));
-    if (l16 == 15) store4(tout + 64 * w.j + 16 * cb + g4, out);
+    flow[cb] = fl[cb] + (dpp_move<0x111>(out) - to_middle(own[cb]));  // row_shr:1
+    const floatx4 q = p.scale * x.q[cb];
+    db[cb] += same_b[w.t] * q, dk[cb] += same_k[w.t] * q;
     if (ok) {
       store_row4<T>(p.db, at + 16 * cb, db[cb]);
       store_row4<T>(p.dk, at + 16 * cb, dk[cb]);
@@ -1168,9 +1216,10 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) {
     const int c = 16 * cb + g4;
-    floatx4 pass = (load4(red + c) + load4(red + 64 + c)) + (load4(red + 128 + c) + load4(red + 192 + c));
-    for (int j = 3; j > w.j; --j) pass += load4(tin + 64 * j + c) - load4(tout + 64 * j + c);
-    pass -= load4(tout + 64 * w.j + c);
+    floatx4 pass = (load4(through + c) + load4(through + 64 + c)) + (load4(through + 128 + c) + load4(through + 192 + c));
+    pass *= load4(L.total + c) * load4(L.total + 64 + c) * (load4(L.total + 128 + c) * load4(L.total + 192 + c));
+    for (int l = 3; l > w.j; --l) pass += load4(over + 64 * (l * (l - 1) / 2 + w.j) + c);
+    for (int j = 0; j < w.j; ++j) pass += load4(out_of + 64 * j + c);
     if (ok) store4(p.dgk + at + 16 * cb, flow[cb] + pass);
   }
 }
@@ -1233,8 +1282,8 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
   return LNX_OK;
 }
 
-// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 497, dplr_grad 725 (two workgroups per CU leave 256 registers, and what a
-// token needs between the pair sums and the last products is more: 24 are spilled, three rows are loaded twice)
+// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 497, dplr_grad 771 (two workgroups per CU leave 256 registers, and what a
+// token needs between the pair sums and the last products is more: rows stay as they were read, and three are loaded twice)
 template <typename T> int backward(const lnx_dplr_chunk_grads* g, const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
   set_kept(p, kept, rows, 0, p.N);

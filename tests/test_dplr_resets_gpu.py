@@ -100,3 +100,25 @@ def test_relative_error(decay, reset):
     err = {n: float(np.linalg.norm(u.detach().cpu().numpy() - r) / np.linalg.norm(r)) for n, u, r in pairs}
     print({n: f"{e:.1e}" for n, e in err.items()})
     assert all(e < 1e-6 for e in err.values()), err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("decay", [4.0, 10.0])
+def test_gate_gradient_behind_strong_decays(decay, dtype):
+    """What flows through a strong decay is small next to what a token gives its own output: the gates' gradients must not carry the
+    rounding of that, 2-norm, fp32 gates and their gradients in both types.  A block's sums have at most 16 terms of the flow's size on
+    each side, every one rounded in a product of 64 terms (1.9e-7 of itself): sqrt(2 * 16) * 1.9e-7 = 1.1e-6 if all were as large as the
+    sum; the mean of the token's place in the block halves their number, 7.5e-7."""
+    import linearnexus_amd as la
+    x = _data(22, 1, 2, 300)
+    x["gk"] *= np.float32(decay)
+    t = {n: torch.from_numpy(x[n]).to(DEV).to(dtype if n in NAMES[:5] else torch.float32).requires_grad_(True) for n in NAMES + ("h0",)}
+    y = {n: u.detach().float().cpu().numpy() for n, u in t.items()}
+    o, h = la.dplr_delta_rule_recurrent(*(t[n] for n in NAMES), 0.125, t["h0"])
+    d_o = torch.from_numpy(x["dO"]).to(DEV).to(dtype)
+    dgk, = torch.autograd.grad([o, h], [t["gk"]], [d_o, torch.from_numpy(x["dS"]).to(DEV)])
+    ref = od.dplr_delta_rule_adjoint(*(y[n] for n in NAMES), d_o.float().cpu().numpy(), x["dS"], 0.125, y["h0"])["dgk"]
+    err = float(np.linalg.norm(dgk.cpu().numpy() - ref) / np.linalg.norm(ref))
+    print(f"{err:.1e}")
+    assert err < 7.5e-7, err
