@@ -21,7 +21,7 @@
 // cu_seqlens ends a document inside a row that way).  A block of 16 tokens is a row of 16 lanes; it has P_t, the decay from before the
 // block's first token to token t, and S_s, that of the tokens after s.  A pair in two blocks has E = P_t (whole blocks between) S_s:
 // factors of the path from s to t, so any decay down to 0 (gk = -inf) gives what the token kernels give.  A pair inside a block has
-// E = P_t / P_s.  P, S and 1 / P come from sums in fixed point, which are exact; a block whose P leave 2^+-60 (RWKV-7's decays are above
+// E = P_t / P_s.  P and S come from sums in fixed point, which are exact; a block whose P leave 2^+-60 (RWKV-7's decays are above
 // exp(-0.607), 2^-14 over a block) multiplies its decays up as floats and takes its 120 pairs one by one (a uniform branch per wave, DIRECT
 // below: B8 H16 T4096 forward and backward 2.2 ms without such blocks, 6.4 ms where all are).
 //
@@ -88,6 +88,7 @@ __device__ __forceinline__ float rcp_f(float x) {  // one Newton step on the ins
   const float r = __builtin_amdgcn_rcpf(x);
   return __builtin_fmaf(__builtin_fmaf(-x, r, 1.f), r, r);
 }
+__device__ __forceinline__ floatx4 rcp4(floatx4 x) { return floatx4{rcp_f(x[0]), rcp_f(x[1]), rcp_f(x[2]), rcp_f(x[3])}; }
 
 // ---- products of 16 x 16 tiles ------------------------------------------------------------------------------------
 // Result fragment: r-th element = row i0 + 4 g + r, column j0 + l16 (g = lane / 16, l16 = lane % 16).  The contraction
@@ -328,12 +329,6 @@ struct Gates {
     for (int e = 0; e < 4; ++e) r[e] = exp2_fixed(sum[cb][e]);
     return r;
   }
-  __device__ __forceinline__ floatx4 upto_inverse(int cb) const {  // 1 / P
-    floatx4 r;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) r[e] = exp2_fixed(-sum[cb][e]);
-    return r;
-  }
   __device__ __forceinline__ floatx4 behind(int cb) const {  // S
     floatx4 r;
 #pragma unroll
@@ -480,7 +475,7 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
     if (!gates.direct) {
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
-        const floatx4 r = gates.upto_inverse(cb), b = x.b[cb] * r, k = x.k[cb] * r;
+        const floatx4 r = rcp4(e.p[cb]), b = x.b[cb] * r, k = x.k[cb] * r;
         mfma_block<4>({&m.ab, &m.ak, &m.qb, &m.qk}, [&](int i) { return i & 1 ? k : b; }, [&](int i) { return i & 2 ? fq[cb] : fa[cb]; });
       }
       mask<true, true>(m.ab, w), mask<true, true>(m.ak, w), mask<true, false>(m.qb, w), mask<true, false>(m.qk, w);
@@ -766,7 +761,7 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
     if (!gates.direct) {
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
-        const floatx4 r = gates.upto_inverse(cb), b = x.b[cb] * r, k = x.k[cb] * r;
+        const floatx4 r = rcp4(e.p[cb]), b = x.b[cb] * r, k = x.k[cb] * r;
         mfma_block<5>({&abd, &akTd, &akd, &qbd, &qkd}, [&](int i) { return i == 0 ? b : i == 1 ? k : i == 2 ? fa[cb] : fq[cb]; },
                       [&](int i) { return i < 2 ? fa[cb] : i == 3 ? b : k; });
       }
@@ -1260,7 +1255,7 @@ constexpr int64_t kept_tiles(int64_t n) { return 3 * n + 1; }  // of a row that 
 
 template <typename K> int lds_limit(K* k) { return lnx_lds_limit(reinterpret_cast<const void*>(k), LDS_BYTES); }
 
-// B8 H16 T4096 bf16 (8192 chunks), us: dplr_prepare 512, dplr_chunk_scan 111, dplr_out 112 (48 KB of reads and 8 of writes per chunk: 4.1 TB/s)
+// B8 H16 T4096 bf16 (8192 chunks), us: dplr_prepare 507, dplr_chunk_scan 111, dplr_out 112 (48 KB of reads and 8 of writes per chunk: 4.1 TB/s)
 template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
   if (int rc = lds_limit(dplr_prepare_kernel<T>)) return rc;
@@ -1282,7 +1277,7 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
   return LNX_OK;
 }
 
-// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 497, dplr_grad 771 (two workgroups per CU leave 256 registers, and what a
+// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 490, dplr_grad 771 (two workgroups per CU leave 256 registers, and what a
 // token needs between the pair sums and the last products is more: rows stay as they were read, and three are loaded twice)
 template <typename T> int backward(const lnx_dplr_chunk_grads* g, const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
