@@ -23,7 +23,7 @@
 // factors of the path from s to t, so any decay down to 0 (gk = -inf) gives what the token kernels give.  A pair inside a block has
 // E = P_t / P_s.  P and S come from sums in fixed point, which are exact; a block whose P leave 2^+-60 (RWKV-7's decays are above
 // exp(-0.607), 2^-14 over a block) multiplies its decays up as floats and takes its 120 pairs one by one (a uniform branch per wave, DIRECT
-// below: B8 H16 T4096 forward and backward 2.2 ms without such blocks, 6.4 ms where all are).
+// below: B8 H16 T4096 forward and backward 2.2 ms without such blocks, 6.2 ms where all are).
 //
 // Sums that carry the recent tokens' large terms take the far ones first, and a sum of two products is added up from two chains: what
 // comes second on one chain would be rounded at the size of the whole, 64 times.  Errors against fp64, relative 2-norms, one row of 512
