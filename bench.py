@@ -90,7 +90,7 @@ def measured_traffic(workload, kernel):
 def chunk_flops(dk, dv, direct=False):
     """Dense-product FLOPs per (batch, head, chunk) that each kernel performs.  In the WY split the forward
     terms add up to F_chunk = 2C^2(3dk+2dv) + 6C*dk*dv and the backward terms to 2*F_chunk; `direct` is the split of
-    the kernels for 2-byte inputs with dk <= 128 and no per-channel gate."""
+    the kernels for 2-byte inputs without a per-channel gate."""
     cc, cd = 2 * C * C, 2 * C * dk * dv
     if direct:
         return {

@@ -164,7 +164,7 @@ int lnx_chunk_fwd_segmented_final(const lnx_scan_args* a, int32_t nseg, void* hi
 /*
  * 1 when lnx_chunk_fwd / lnx_chunk_bwd apply the in-op normalisation of q and k themselves for these arguments
  * (use_qk_l2norm = 1: gated_deltanet.py:273-275, kda.py:379-381 normalise inside the op, and it is their default):
- * q, k, v in bf16, dk <= 128, no per-channel gate.  The rows are scaled where the kernels stage them and the
+ * q, k, v in bf16, no per-channel gate.  The rows are scaled where the kernels stage them and the
  * backward pass carries d_q, d_k through the normalisation, so no normalised copies of q and k exist.  0: the chunk
  * entry points refuse use_qk_l2norm for these arguments; normalise with lnx_l2norm_fwd first.
  */
@@ -179,7 +179,7 @@ int lnx_chunk_fuses_l2norm(const lnx_scan_args* a);
  * or other allocating routine.  All calls on one GPU share that GPU's array: calls that overlap in time on one GPU
  * (two streams, two threads) race and must be serialised by the caller.  No counterpart in the reference, whose
  * JAX ops leave allocation to XLA.
- * For bf16 inputs with dk <= 128 and no per-channel gate the scratch takes 17 KiB per 64-token chunk of every
+ * For bf16 inputs without a per-channel gate the scratch takes 17 KiB per 64-token chunk of every
  * (batch, head) row, so B * H * ceil(T / 64) <= 3855 chunks fit (8 heads of 30720 tokens; a packed batch counts
  * T / 64 + nseq chunks per head); the other shapes also keep W and U there, (dk + dv) * 128 bytes more per chunk (twice
  * that for fp32); lnx_chunk_workspace_bytes with forward_only = 1 gives the exact figure.  The address of the array on the current device is looked up on the first call on

@@ -599,7 +599,8 @@ template <typename T, int DK, int GATE> struct DqkCfg {
   static constexpr int kLoop = (64 * LDSV > SV * LDC) ? 64 * LDSV : SV * LDC;
   // 2-byte inputs: NBUF buffers of dO | D | dD ([64][SV], read by rows) | S_n | dS_n ([SV][64], transposing reads)
   static constexpr bool DMA = sizeof(T) == 2;
-  static constexpr int NBUF = GATE == LNX_GATE_VECTOR ? 3 : 2;  // what two / three workgroups per CU leave room for
+  static_assert(!DMA || GATE == LNX_GATE_VECTOR, "2-byte inputs without a per-channel gate take bwd_chunk");
+  static constexpr int NBUF = 3;  // what two workgroups per CU leave room for
   static constexpr int slab_bytes = 5 * 64 * SV * 2;
   static constexpr size_t loop_bytes = DMA ? (size_t)NBUF * slab_bytes : sizeof(T) * 5 * kLoop;
   // scalar epilogue: dPe, K rows, Q rows and one staging tile (dW, then dk), four [64][64] tiles
@@ -610,11 +611,11 @@ template <typename T, int DK, int GATE> struct DqkCfg {
   static constexpr size_t big = epi_bytes > loop_bytes ? epi_bytes : loop_bytes;
   static constexpr int kSmall = 64 * 4 + (GATE == LNX_GATE_VECTOR ? 64 * LNX_LDA : 0);  // floats
   static constexpr size_t bytes = sizeof(float) * kSmall + big;
-  static_assert(!DMA || bytes * (GATE == LNX_GATE_VECTOR ? 2 : 3) <= 160 * 1024, "workgroups per CU");
+  static_assert(!DMA || bytes * 2 <= 160 * 1024, "workgroups per CU");
 };
 
 template <typename T, int DK, int GATE>
-__global__ __launch_bounds__(256, (GATE == LNX_GATE_VECTOR ? (sizeof(T) == 2 ? 2 : 1) : sizeof(T) == 2 ? 3 : 2)) void bwd_dqk_kernel(BwdParams p) {
+__global__ __launch_bounds__(256, GATE == LNX_GATE_VECTOR && sizeof(T) == 4 ? 1 : 2) void bwd_dqk_kernel(BwdParams p) {
   typedef DqkCfg<T, DK, GATE> L;
   constexpr int LDC = L::LDC, LDF = L::LDF;
   extern __shared__ __align__(16) char smem[];
@@ -969,8 +970,8 @@ template <typename T, int DK, int GATE> struct Wy2Cfg {
   static constexpr size_t vec_bytes = sizeof(float) * 2 * 64 * LDF + sizeof(T) * kTile;
   static_assert(GATE != LNX_GATE_VECTOR || vec_bytes <= sizeof(T) * 5 * kTile, "epilogue tiles overlay the loop tiles");
   // tiles: Tm^T, dW/dD slab, dB slab, K/V slab, and the W/U slab (vector gate) or all K slabs but the last kept
-  // for the epilogue (other gates; 4-byte inputs with dk <= 128 read K again instead, so that two workgroups fit a CU)
-  static constexpr bool KEEP_K = GATE != LNX_GATE_VECTOR && (sizeof(T) == 2 || DK > 128);
+  // for the epilogue (other gates with dk = 256; with dk <= 128 K is read again instead, so that two workgroups fit a CU)
+  static constexpr bool KEEP_K = GATE != LNX_GATE_VECTOR && DK > 128;
   static constexpr int ntile = (GATE == LNX_GATE_VECTOR) ? 5 : KEEP_K ? 4 + (DK / 64 - 1) : 4;
   // vector gate, 2-byte inputs, dk = 128: the second half's dBw fragments wait in LDS while the first half's pair sums
   // run (one value per thread and fragment element; in registers they went to scratch memory)
@@ -982,7 +983,7 @@ template <typename T, int DK, int GATE> struct Wy2Cfg {
 // GRAW (per-channel gate only): the gate was activated inside the op from the raw projection; dg goes on through the
 // activation to d_gate_raw and to the per-chunk partial sums of the parameter gradients.
 template <typename T, int DK, int GATE, bool GRAW = false>
-__global__ __launch_bounds__(256, (sizeof(T) == 2 ? (GATE == LNX_GATE_VECTOR || DK > 128 ? 2 : 3) : (GATE == LNX_GATE_VECTOR || DK > 128 ? 1 : 2))) void bwd_wy2_kernel(BwdParams p) {
+__global__ __launch_bounds__(256, sizeof(T) == 4 && (GATE == LNX_GATE_VECTOR || DK > 128) ? 1 : 2) void bwd_wy2_kernel(BwdParams p) {
   typedef Wy2Cfg<T, DK, GATE> L;
   constexpr int LDC = L::LDC, LDF = L::LDF, NKS = DK / 64;
   extern __shared__ __align__(16) char smem[];
@@ -1445,7 +1446,6 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
   constexpr bool can_narrow = (DK >= 128 && sizeof(T) == 2) || (DK == 128 && sizeof(T) == 4);
   constexpr int WIDE = 64, NARROW = can_narrow ? 32 : WIDE;
   const bool narrow = can_narrow && lnx_narrow_slabs((int64_t)nstate * p.geom.H * (p.dv / 64), p.slab);
-  constexpr bool wide_scan = sizeof(T) == 2 && DK == 256 && GATE != LNX_GATE_VECTOR;  // chunk_wide.hip
   auto k2 = bwd_dqk_kernel<T, DK, GATE>;
   auto k3 = (GATE == LNX_GATE_VECTOR && p.graw) ? bwd_wy2_kernel<T, DK, GATE, GATE == LNX_GATE_VECTOR> : bwd_wy2_kernel<T, DK, GATE>;
   const size_t b2 = DqkCfg<T, DK, GATE>::bytes, b3 = Wy2Cfg<T, DK, GATE>::bytes;
@@ -1455,21 +1455,12 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
     lnx_profile_mark("bwd_local", st);
     hipLaunchKernelGGL(bwd_local_kernel<T>, dim3(lnx_xcd_grid(slots, p.dv / 64)), dim3(256), 0, st, p);
   }
-  if constexpr (wide_scan) {
-    DirectParams d = {};
-    d.geom = p.geom;
-    d.q = reinterpret_cast<const bf16_t*>(p.q); d.k = reinterpret_cast<const bf16_t*>(p.k);
-    d.dv = p.dv; d.gate = GATE; d.slab = p.slab; d.scale = p.scale; d.ws = p.ws; d.off = p.off;
-    d.d_o = reinterpret_cast<const bf16_t*>(p.d_o); d.d_sT = p.d_sT; d.ds0 = p.ds0;
-    if ((rc = lnx_wide_scan(true, d, nstate, st)) != LNX_OK) return rc;
-  } else {
-    auto k1 = narrow ? bwd_scan_kernel<T, DK, GATE, NARROW> : bwd_scan_kernel<T, DK, GATE, WIDE>;
-    const int bv = narrow ? BScanCfg<T, DK, NARROW>::BV : BScanCfg<T, DK, WIDE>::BV;
-    const size_t b1 = narrow ? BScanCfg<T, DK, NARROW>::bytes : BScanCfg<T, DK, WIDE>::bytes;
-    if ((rc = lnx_lds_limit((const void*)k1, b1)) != LNX_OK) return rc;
-    lnx_profile_mark("bwd_scan", st);
-    hipLaunchKernelGGL(k1, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(512), b1, st, p);
-  }
+  auto k1 = narrow ? bwd_scan_kernel<T, DK, GATE, NARROW> : bwd_scan_kernel<T, DK, GATE, WIDE>;
+  const int bv = narrow ? BScanCfg<T, DK, NARROW>::BV : BScanCfg<T, DK, WIDE>::BV;
+  const size_t b1 = narrow ? BScanCfg<T, DK, NARROW>::bytes : BScanCfg<T, DK, WIDE>::bytes;
+  if ((rc = lnx_lds_limit((const void*)k1, b1)) != LNX_OK) return rc;
+  lnx_profile_mark("bwd_scan", st);
+  hipLaunchKernelGGL(k1, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(512), b1, st, p);
   lnx_profile_mark("bwd_dqk", st);
   hipLaunchKernelGGL(k2, dim3(lnx_xcd_grid(slots, DK / 64)), dim3(256), b2, st, p);
   lnx_profile_mark("bwd_wy", st);
@@ -1547,8 +1538,8 @@ extern "C" int lnx_chunk_bwd(const lnx_scan_args* a, void* stream) {
     if (e != hipSuccess) return lnx_set_error(LNX_ERR_LAUNCH, "chunk backward launch: %s", hipGetErrorString(e));
     return LNX_OK;
   }
-  if (a->dtype == LNX_BF16)  // dk <= 128 without a per-channel gate went to the direct-solve kernels above
-    rc = (a->dk == 256)   ? launch_bwd_gate<bf16_t, 256>(a->gate, p, nstate, st)
+  if (a->dtype == LNX_BF16)  // calls without a per-channel gate went to the direct-solve kernels above
+    rc = (a->dk == 256)   ? launch_bwd<bf16_t, 256, LNX_GATE_VECTOR>(p, nstate, st)
          : (a->dk == 128) ? launch_bwd<bf16_t, 128, LNX_GATE_VECTOR>(p, nstate, st)
                           : launch_bwd<bf16_t, 64, LNX_GATE_VECTOR>(p, nstate, st);
   else

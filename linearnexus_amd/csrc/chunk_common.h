@@ -115,12 +115,12 @@ __device__ __forceinline__ float lnx_softplus_thr(float x, float thr) {
   return x > thr ? x : fmaxf(x, 0.f) + __logf(1.f + __expf(-fabsf(x)));
 }
 
-// 2-byte inputs with dk <= 128 and no per-channel gate take the kernels of chunk_direct.hip, which keep G, Pm, Tm, the
+// 2-byte inputs without a per-channel gate take the kernels of chunk_direct.hip (dk = 256: the scans of chunk_wide.hip), which keep G, Pm, Tm, the
 // per-chunk states and state gradients, D and dR in the workspace (no W, U, dW); every other shape takes the WY-split
 // kernels.  The choice reads only fields that the forward and the backward call of one step necessarily share (element
 // type, dk, gate kind), so both calls lay the workspace out the same way; there is one set of kernels per shape.
 inline bool lnx_chunk_direct(const lnx_scan_args* a) {
-  return a->dtype == LNX_BF16 && a->dk <= 128 && a->gate != LNX_GATE_VECTOR;
+  return a->dtype == LNX_BF16 && a->gate != LNX_GATE_VECTOR;
 }
 
 inline uint64_t lnx_align256(uint64_t x) { return (x + 255) & ~uint64_t(255); }
@@ -227,7 +227,7 @@ struct DirectParams {
 };
 int lnx_direct_scan_fwd(const DirectParams& p, int dk, int gate, int nstate, hipStream_t st);
 int lnx_direct_bwd(const DirectParams& p, int dk, int gate, int nstate, hipStream_t st);
-// The sequential passes of the WY-split kernels for 2-byte inputs with dk = 256 and no / a scalar gate (chunk_wide.hip).
+// The sequential passes for dk = 256 (chunk_wide.hip).
 int lnx_wide_scan(bool backward, const DirectParams& p, int nstate, hipStream_t st);
 
 // Shared argument validation of the chunk entry points; returns LNX_OK or an error status.

@@ -1,5 +1,5 @@
-// Chunked delta-rule forward and backward for 2-byte inputs with dk <= 128 and no / a scalar gate, in the
-// "direct solve" split: the only per-chunk tensors that cross kernels are Tm = (I + A)^-1, Pm = scale tril(E * Q K^T)
+// Chunked delta-rule forward and backward for 2-byte inputs with no / a scalar gate, in the
+// "direct solve" split (dk = 256: the scans are those of chunk_wide.hip): the only per-chunk tensors that cross kernels are Tm = (I + A)^-1, Pm = scale tril(E * Q K^T)
 // and the cumulative gate G from the chunk-parallel prepare kernel, the states entering the chunks and D (forward scan
 // -> chunk-local backward) and the state gradients leaving them and dR (reverse scan -> chunk-local backward).  W, U,
 // dD, dW of the WY form are never materialised: with S the state entering a chunk,
@@ -51,14 +51,12 @@ __device__ __forceinline__ void store_frag_t(const floatx16& a, T* dst, int ld, 
   }
 }
 
-// Zeroes the 224 vectors above the diagonal (row r, columns 8 c .. 8 c + 7 with 8 c > r) of `ntile` consecutive
-// [64][ld] tiles of `stride` elements, columns in the order CHAIN; 256 threads.  Group g of eight rows has 7 - g such vectors per row.
+// Zeroes the vectors above the diagonal of `ntile` consecutive [64][ld] tiles of `stride` elements, columns in the order CHAIN; 256 threads
+// or more.
 template <bool CHAIN> __device__ __forceinline__ void zero_upper_triangles(T* tiles, int ntile, int stride, int ld, int tid) {
   if (tid >= 512 - LNX_TRI_VECS) return;
-  int g = 0;
-  while (56 * (g + 1) - 4 * (g + 1) * g <= tid) ++g;  // vectors of the groups before g + 1
-  const int o = tid - (56 * g - 4 * g * (g - 1)), per = 7 - g;
-  const int r = 8 * g + o / per, c = g + 1 + (o - (o / per) * per);
+  int r, c;
+  upper_vec_pos(tid, r, c);
   for (int t = 0; t < ntile; ++t) S16::put<CHAIN>(tiles + t * stride + r * ld + S16::pos<CHAIN>(8 * c), vec_zero<T>());
 }
 
@@ -776,42 +774,51 @@ int launch_scan_bwd(const DirectParams& p, int nstate, hipStream_t st) {
 // Measured per workgroup at B8 H16 T4096 d128 (wall clock of wave 0, 2 workgroups per CU): 4.3 us until the first slab
 // is there, 6.2 us for the loop, 2.1 us staging K, Q and the four small tiles, 1.8 us for the epilogue's products and
 // 3.4 us until dq, dk have left -- memory latency at every step; the kernel moves 4.9 TB/s.
+// dk = 256: 896 KB a chunk at dv = 512, most of it the two states; B8 H8 T4096 790 us, 4.6 TB/s.
 // ---------------------------------------------------------------------------------------
 template <int DK> struct BChunkL {
+  // dk = 256: eight waves, one workgroup per CU -- the [64 x dk] accumulators of four would take 192 registers, the slabs of two
+  // workgroups more LDS than there is -- and a third slab buffer, for nobody else's loads are in flight while this workgroup multiplies
+  static constexpr int NW = DK == 256 ? 8 : 4, THREADS = 64 * NW, NBUF = DK == 256 ? 3 : 2;
   static constexpr int SV = 32;
+  static constexpr int SC = DK < 128 ? DK : 128, NH = DK / SC;  // a state slab is NH tiles of SC columns
   typedef SwzTile<64, SV> TokT;            // dO, V slabs [64][SV], read by rows
   typedef SwzTile<SV, 64, false> TrT;      // D^T, dR^T slabs [SV][64], transposing reads only
-  typedef SwzTile<SV, DK, false> StT;      // S^T, dS'^T slabs [SV][DK], transposing reads only
+  typedef SwzTile<SV, SC, false> StT;      // S^T, dS'^T slabs [SV][SC], transposing reads only
   static constexpr int LDKT = DK + 32;     // the epilogue's K, Q tiles [64][DK], transposing reads
   static constexpr int LDC = 64 + 8;       // dPe, dPe^T, dXa, dXe^T [64][64], read by rows
   static constexpr int LDK = DK + 8;       // staging tile for dq, dk [64][DK]
-  static constexpr int kC = 64 * LDC, kRow = 64 * LDKT;
-  // one slab of the loop: dO | V | D^T | dR^T | S^T | dS'^T, unpadded; two of them, filled by LDS-direct loads in turn
-  static constexpr int oV = TokT::BYTES, oDT = 2 * TokT::BYTES, odRT = oDT + TrT::BYTES, oSn = odRT + TrT::BYTES, odSn = oSn + StT::BYTES;
-  static constexpr int slab_bytes = odSn + StT::BYTES;
-  static constexpr size_t loop_bytes = 2 * slab_bytes;
-  static constexpr size_t epi_bytes = sizeof(T) * (2 * kRow + 4 * kC);
-  static_assert(64 * LDK <= 2 * kC, "the staging tile overlays dPe and dPe^T");
-  static constexpr int nfloat = 64 * 8;
+  static constexpr int kC = 64 * LDC, kRow = 64 * LDKT, kSt = 64 * LDK;
+  // one slab of the loop: dO | V | D^T | dR^T | S^T | dS'^T, unpadded; NBUF of them, filled by LDS-direct loads in turn
+  static constexpr int oV = TokT::BYTES, oDT = 2 * TokT::BYTES, odRT = oDT + TrT::BYTES, oSn = odRT + TrT::BYTES, odSn = oSn + NH * StT::BYTES;
+  static constexpr int slab_bytes = odSn + NH * StT::BYTES;
+  static constexpr size_t loop_bytes = NBUF * slab_bytes;
+  // the staging tiles of dq and dk: over dPe and dPe^T, over dXa and dXe^T; dk = 256: dq over all four, dk's behind the Q tile
+  static constexpr bool OVER2 = DK <= 128;
+  static constexpr size_t epi_bytes = sizeof(T) * (2 * kRow + 4 * kC + (OVER2 ? 0 : kSt));
+  static_assert(kSt <= (OVER2 ? 2 : 4) * kC, "the staging tile overlays the small tiles");
+  static constexpr int nfloat = 64 * 10;
   static constexpr size_t bytes = sizeof(float) * nfloat + (epi_bytes > loop_bytes ? epi_bytes : loop_bytes);
-  static_assert(bytes <= 80 * 1024, "two workgroups per CU");
+  static_assert(bytes <= (NW == 4 ? 80 : 160) * 1024, "two workgroups of four waves per CU, one of eight");
 };
 
 template <int DK, int GATE>
-__global__ __launch_bounds__(256, 2) void bwd_chunk_kernel(DirectParams p) {
+__global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(DirectParams p) {
   typedef BChunkL<DK> L;
-  constexpr int SV = L::SV, LDKT = L::LDKT, LDC = L::LDC, LDK = L::LDK;
+  constexpr int SV = L::SV, LDKT = L::LDKT, LDC = L::LDC, LDK = L::LDK, NW = L::NW, THREADS = L::THREADS, NBUF = L::NBUF, SC = L::SC, NH = L::NH;
   typedef typename L::TokT TokT;
   typedef typename L::TrT TrT;
   typedef typename L::StT StT;
-  constexpr int NKT = DK / 64;  // key-column tiles per wave
+  constexpr int NKT = DK / (16 * NW);  // key-column tiles per wave
+  constexpr int NPA = 8 / NW;          // of dPm's and dAm's eight tiles: one of each per wave, or one of either
+  constexpr int TPT = THREADS / 64;    // threads per token where rows are summed
   extern __shared__ __align__(16) char smem[];
   float* sG = reinterpret_cast<float*>(smem);
   float* sBeta = sG + 64;
   float* sRdv = sBeta + 64;   // <dR_t, v_t>
-  float* sM = sRdv + 64;      // m_t
-  float* sdG = sM + 64;
-  float* sMisc = sdG + 64;    // [4 + wave] = the wave's share of sum_t r_t <k_t, dK2_t>, [8 + wave] = of <dS', S>
+  float* sM = sRdv + 64;      // [2]: m_t is the sum of the two
+  float* sdG = sM + 128;      // [2]: <q_t, dq_t> - <k_t, dk_t> is the sum of the two
+  float* sMisc = sdG + 128;    // [8 + wave] = the wave's share of sum_t r_t <k_t, dK2_t>, [16 + wave] = of <dS', S>
   float* sNq = sMisc + 64;    // normalisation factors of the q and k rows (1 when the inputs come normalised)
   float* sNk = sNq + 64;
   T* tiles = reinterpret_cast<T*>(smem + sizeof(float) * L::nfloat);
@@ -823,10 +830,10 @@ __global__ __launch_bounds__(256, 2) void bwd_chunk_kernel(DirectParams p) {
   T* sXeT = sXa + L::kC;      // [j][i]
   T* sK = sXeT + L::kC;       // [token][dk]
   T* sQ = sK + L::kRow;
-  T* sSt = tiles;             // staging for dq (over dPe, dPe^T) and dk (over dXa, dXe^T), once the four small tiles are dead
-  T* sSt2 = sXa;
+  T* sSt = tiles;             // staging for dq and dk, once the four small tiles are dead
+  T* sSt2 = L::OVER2 ? sXa : sQ + L::kRow;
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = NW == 4 ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int N = p.geom.N;
   const int64_t slot = blockIdx.x;
   const int row = (int)(slot / N), n = (int)(slot % N);
@@ -835,26 +842,39 @@ __global__ __launch_bounds__(256, 2) void bwd_chunk_kernel(DirectParams p) {
   if (len <= 0) return;
   const int64_t tbase = tok_index(p.geom, row, tok0);
   const int64_t ts = p.geom.ts, tsk = ts * DK, tsv = ts * p.dv;
-  const int wi = wave >> 1, wj = wave & 1;
+  const int wi = wave / (NW / 2), wj = wave % (NW / 2);
   const int fr = lane & 31, kg8 = 8 * (lane >> 5);
+  // the wave's tiles of dPm (all waves, or those of wj < 2) and dAm: token-row tile wi, columns 32 jt ..
+  const int jt = wj & 1;
+  const bool has_p = NPA == 2 || wj < 2, has_a = NPA == 2 || wj >= 2;
 
-  TileRegs<T, 64, DK> rK, rQ;  // the epilogue's tiles, requested during the last slab
-  floatx16 aP[1][1], aA[1][1], aQ[1][NKT], aK1[1][NKT], aK2[1][NKT];
+  TileRegs<T, 64, DK, THREADS> rK, rQ;  // the epilogue's tiles, requested during the last slab
+  floatx16 aPA[NPA][1][1], aQ[1][NKT], aK1[1][NKT], aK2[1][NKT];
+  auto& aP = aPA[0];
+  auto& aA = aPA[NPA - 1];
   frag_zero(aP);
   frag_zero(aA);
   frag_zero(aQ);
   frag_zero(aK1);
   frag_zero(aK2);
   float ss = 0.f, rdv = 0.f;
+  auto token_sum = [](float x) {  // over the TPT threads of a token
+    x = quad_sum(x);
+    return TPT == 8 ? x + __shfl_xor(x, 4, LNX_WAVE) : x;
+  };
+  auto waves_sum = [](const float* x) {
+    const float lo = (x[0] + x[1]) + (x[2] + x[3]);
+    return NW == 8 ? lo + ((x[4] + x[5]) + (x[6] + x[7])) : lo;
+  };
   if (tid < 64) {
     sG[tid] = (GATE == LNX_GATE_SCALAR) ? at<const float>(p.ws, p.off.G)[slot * 64 + tid] : 0.f;
     sBeta[tid] = (tid < len) ? p.beta[tbase + tid * ts] : 0.f;
-    sM[tid] = 0.f;
+    sM[tid] = sM[64 + tid] = sdG[tid] = sdG[64 + tid] = 0.f;
     sMisc[tid] = 0.f;
     sNq[tid] = at<const float>(p.ws, p.off.Nq)[slot * 64 + tid];
     sNk[tid] = at<const float>(p.ws, p.off.Nk)[slot * 64 + tid];
   }
-  // ---- the slab loads: 32 one-KB instructions per slab, eight per wave, straight into LDS buffer `b` ----
+  // ---- the slab loads: one-KB instructions, PER_WAVE of them per wave and slab, straight into LDS buffer `b` ----
   // Token rows past the chunk's end fetch the chunk's last row instead of zeros: whatever they hold only reaches rows of
   // dq, dk, dbeta, dg that are not stored (q, k and beta of those rows are zero).
   const unsigned slab0 = lds_byte_addr(sSlab);
@@ -867,37 +887,39 @@ __global__ __launch_bounds__(256, 2) void bwd_chunk_kernel(DirectParams p) {
   auto issue = [&](int v0, int b) {
     const unsigned dst = slab0 + b * L::slab_bytes;
     int r, c;
-    // wave w: instructions w, w + 4, ... of each tile
+    // wave w: instructions w, w + NW, ... of the states; of the four small tiles one each, or with eight waves one of two
 #pragma unroll
-    for (int j = wave; j < StT::NINSTR; j += 4) {
+    for (int u = 0; u < NH * StT::NINSTR / NW; ++u) {
+      const int i = wave + NW * u, h = i / StT::NINSTR, j = i % StT::NINSTR;
       StT::src(j, lane, r, c);
-      dma16(gSn + (int64_t)(v0 + r) * DK + c, dst + L::oSn + 1024 * j);
-      dma16(gdSn + (int64_t)(v0 + r) * DK + c, dst + L::odSn + 1024 * j);
+      dma16(gSn + (int64_t)(v0 + r) * DK + SC * h + c, dst + L::oSn + 1024 * i);
+      dma16(gdSn + (int64_t)(v0 + r) * DK + SC * h + c, dst + L::odSn + 1024 * i);
     }
-#pragma unroll
-    for (int j = wave; j < TokT::NINSTR; j += 4) {
+    const int j = wave & 3;
+    if (NW == 4 || wave < 4) {
       TokT::src(j, lane, r, c);
       r = min(r, len - 1);
       dma16(gdO + (int64_t)r * tsv + v0 + c, dst + 1024 * j);
       dma16(gV + (int64_t)r * tsv + v0 + c, dst + L::oV + 1024 * j);
     }
-#pragma unroll
-    for (int j = wave; j < TrT::NINSTR; j += 4) {
+    if (NW == 4 || wave >= 4) {
       TrT::src(j, lane, r, c);
       dma16(gDT + (int64_t)(v0 + r) * 64 + c, dst + L::oDT + 1024 * j);
       dma16(gdRT + (int64_t)(v0 + r) * 64 + c, dst + L::odRT + 1024 * j);
     }
   };
-  constexpr int PER_WAVE = (2 * StT::NINSTR + 2 * TokT::NINSTR + 2 * TrT::NINSTR) / 4;  // loads per wave and slab
-  static_assert(StT::NINSTR % 4 == 0 && TokT::NINSTR % 4 == 0 && TrT::NINSTR % 4 == 0, "the same count for every wave");
+  constexpr int PER_WAVE = 2 * NH * StT::NINSTR / NW + 16 / NW;  // loads per wave and slab
+  static_assert(NH * StT::NINSTR % NW == 0 && TokT::NINSTR == 4 && TrT::NINSTR == 4, "the same count for every wave");
   __builtin_amdgcn_s_waitcnt(0);  // the small loads above are behind us: from here on this wave's vmcnt counts slab loads only
-  issue(0, 0);
-  if (SV < p.dv) issue(SV, 1);
+#pragma unroll
+  for (int u = 0; u < NBUF; ++u)
+    if (u * SV < p.dv) issue(u * SV, u);
   int b = 0;
 #pragma unroll 1
-  for (int v0 = 0; v0 < p.dv; v0 += SV, b ^= 1) {
-    // this slab has landed: all but the next slab's loads of this wave, then every wave's
-    if (v0 + SV < p.dv) dma_wait<PER_WAVE>();
+  for (int v0 = 0; v0 < p.dv; v0 += SV, b = b + 1 == NBUF ? 0 : b + 1) {
+    // this slab has landed: all but this wave's loads of the slabs behind it, then every wave's
+    if (NBUF > 2 && v0 + 2 * SV < p.dv) dma_wait<2 * PER_WAVE>();
+    else if (v0 + SV < p.dv) dma_wait<PER_WAVE>();
     else dma_wait<0>();
     lds_barrier();
     const T* sdO = reinterpret_cast<const T*>(sSlab + b * L::slab_bytes);
@@ -916,53 +938,54 @@ __global__ __launch_bounds__(256, 2) void bwd_chunk_kernel(DirectParams p) {
       const M::Frag fdO = TokT::load(sdO, 32 * wi + fr, k0 + kg8);
       const M::Frag fdR = TrT::load_t(sdRT, k0, 32 * wi, lane);
       const M::Frag fDi = TrT::load_t(sDT, k0, 32 * wi, lane);
-      const M::Frag fDj = TrT::load_t(sDT, k0, 32 * wj, lane);
-      M::mma(aP[0][0], fdO, fDj);
-      M::mma(aA[0][0], fdR, fDj);
+      const M::Frag fDj = TrT::load_t(sDT, k0, 32 * jt, lane);
+      if (has_p) M::mma(aP[0][0], fdO, fDj);
+      if (has_a) M::mma(aA[0][0], fdR, fDj);
 #pragma unroll
       for (int c = 0; c < NKT; ++c) {
-        const M::Frag fS = StT::load_t(sSn, k0, 32 * (NKT * wj + c), lane);
-        const M::Frag fdS = StT::load_t(sdSn, k0, 32 * (NKT * wj + c), lane);
+        const int col = 32 * (NKT * wj + c), st = NH == 1 ? 0 : (col / SC) * (StT::BYTES / 2);
+        const M::Frag fS = StT::load_t(sSn + st, k0, NH == 1 ? col : col % SC, lane);
+        const M::Frag fdS = StT::load_t(sdSn + st, k0, NH == 1 ? col : col % SC, lane);
         M::mma(aQ[0][c], fdO, fS);
         M::mma(aK1[0][c], fdR, fS);
         M::mma(aK2[0][c], fDi, fdS);
       }
     }
-    {  // <dR_t, v_t> over this slab: thread = (token tid / 4, eight value columns)
-      const int t = tid >> 2, c0 = 8 * (tid & 3);
-      const M::Frag vv = TokT::load(sV, t, c0);
+    {  // <dR_t, v_t> over this slab: thread = (token tid / TPT, SV / TPT value columns)
+      typedef bf16_t VecV __attribute__((ext_vector_type(SV / TPT)));
+      const int t = tid / TPT, c0 = (SV / TPT) * (tid % TPT);
+      const VecV vv = *reinterpret_cast<const VecV*>(sV + TokT::at(t, c0));
 #pragma unroll
-      for (int e = 0; e < 8; ++e) rdv += (float)vv[e] * (float)sdRT[TrT::at(c0 + e, t)];
+      for (int e = 0; e < SV / TPT; ++e) rdv += (float)vv[e] * (float)sdRT[TrT::at(c0 + e, t)];
     }
     if (GATE == LNX_GATE_SCALAR) {  // <dS', S> over this slab: the two tiles share one layout, so granule by granule
 #pragma unroll
-      for (int u = 0; u < StT::BYTES / 16 / 256; ++u) {
-        const M::Frag a = *reinterpret_cast<const M::Frag*>(sSn + 8 * (tid + 256 * u));
-        const M::Frag b2 = *reinterpret_cast<const M::Frag*>(sdSn + 8 * (tid + 256 * u));
+      for (int u = 0; u < NH * StT::BYTES / 16 / THREADS; ++u) {
+        const M::Frag a = *reinterpret_cast<const M::Frag*>(sSn + 8 * (tid + THREADS * u));
+        const M::Frag b2 = *reinterpret_cast<const M::Frag*>(sdSn + 8 * (tid + THREADS * u));
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += (float)a[e] * (float)b2[e];
       }
     }
-    if (v0 + 2 * SV < p.dv) {  // this buffer takes the slab after the next, once every wave has read it
+    if (v0 + NBUF * SV < p.dv) {  // this buffer takes the slab NBUF ahead, once every wave has read it
       lds_barrier();
-      issue(v0 + 2 * SV, b);
+      issue(v0 + NBUF * SV, b);
     }
   }
-  rdv += __shfl_xor(rdv, 1, LNX_WAVE);
-  rdv += __shfl_xor(rdv, 2, LNX_WAVE);
-  if ((tid & 3) == 0) sRdv[tid >> 2] = rdv;
+  rdv = token_sum(rdv);
+  if (tid % TPT == 0) sRdv[tid / TPT] = rdv;
   if (GATE == LNX_GATE_SCALAR) {
     ss = wave_sum(ss);
-    if (lane == 0) sMisc[8 + wave] = ss;  // one slot per wave, added in a fixed order below
+    if (lane == 0) sMisc[16 + wave] = ss;  // one slot per wave, added in a fixed order below
   }
   lds_barrier();  // slab tiles are dead from here on
 
   // ---- epilogue ----
   {  // K and Q rows, normalised
-    typedef TileRegs<T, 64, DK> RowTile;
+    typedef TileRegs<T, 64, DK, THREADS> RowTile;
 #pragma unroll
     for (int it = 0; it < RowTile::IT; ++it) {
-      const int idx = tid + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
+      const int idx = tid + THREADS * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
       const float fk = sNk[r], fq = sNq[r];
       typename Vec16<T>::V x = rK.x[it], y = rQ.x[it];
 #pragma unroll
@@ -982,22 +1005,26 @@ __global__ __launch_bounds__(256, 2) void bwd_chunk_kernel(DirectParams p) {
   }
   const float gC = sG[63];
   {
-    floatx16 pe[1][1];
-    const int j = 32 * wj + frag_col(lane);
+    float dec[16];
+    const int j = 32 * jt + frag_col(lane);
     const float gj = sG[j];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int i = 32 * wi + frag_row(e, lane);
-      const float dec = (GATE == LNX_GATE_NONE) ? 1.f : __expf(fminf(gi[e >> 2][e & 3] - gj, 0.f));
-      pe[0][0][e] = (i >= j) ? p.scale * dec * aP[0][0][e] : 0.f;
-      aA[0][0][e] = (i > j) ? -dec * aA[0][0][e] : 0.f;  // dXa
-    }
-    frag_store<T, 1, 1>(pe, sPe + 32 * wi * LDC + 32 * wj, LDC, lane);
-    frag_store_t<T, 1, 1>(pe, sPeT + 32 * wj * LDC + 32 * wi, LDC, lane);
-    frag_store<T, 1, 1>(aA, sXa + 32 * wi * LDC + 32 * wj, LDC, lane);
+    for (int e = 0; e < 16; ++e) dec[e] = (GATE == LNX_GATE_NONE) ? 1.f : __expf(fminf(gi[e >> 2][e & 3] - gj, 0.f));
+    if (has_p) {
+      floatx16 pe[1][1];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) aA[0][0][e] *= bi[e >> 2][e & 3];  // dXe
-    frag_store_t<T, 1, 1>(aA, sXeT + 32 * wj * LDC + 32 * wi, LDC, lane);
+      for (int e = 0; e < 16; ++e) pe[0][0][e] = (32 * wi + frag_row(e, lane) >= j) ? p.scale * dec[e] * aP[0][0][e] : 0.f;
+      frag_store<T, 1, 1>(pe, sPe + 32 * wi * LDC + 32 * jt, LDC, lane);
+      frag_store_t<T, 1, 1>(pe, sPeT + 32 * jt * LDC + 32 * wi, LDC, lane);
+    }
+    if (has_a) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) aA[0][0][e] = (32 * wi + frag_row(e, lane) > j) ? -dec[e] * aA[0][0][e] : 0.f;  // dXa
+      frag_store<T, 1, 1>(aA, sXa + 32 * wi * LDC + 32 * jt, LDC, lane);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) aA[0][0][e] *= bi[e >> 2][e & 3];  // dXe
+      frag_store_t<T, 1, 1>(aA, sXeT + 32 * jt * LDC + 32 * wi, LDC, lane);
+    }
   }
   lds_barrier();
   // dq = scale e^G dQa + dPe K;   row = dXa K - e^G dK1 (in aK1)
@@ -1043,10 +1070,10 @@ __global__ __launch_bounds__(256, 2) void bwd_chunk_kernel(DirectParams p) {
         aK2[0][c][e] += bt * aK1[0][c][e];
       }
     }
-    rows_reduce_add<1>(mv, 32 * wi, lane, sM);  // two waves (wj = 0, 1) add to a zeroed entry: order-independent
+    rows_reduce_add<1>(mv, 32 * wi, lane, sM + 64 * (wj >> 1));  // two waves (wj even, odd) add to a zeroed entry: order-independent
     if (GATE == LNX_GATE_SCALAR) {
       tot = wave_sum(tot);
-      if (lane == 0) sMisc[4 + wave] = tot;
+      if (lane == 0) sMisc[8 + wave] = tot;
     }
   }
   // dk += dPe^T Q + dXe^T K
@@ -1060,27 +1087,43 @@ __global__ __launch_bounds__(256, 2) void bwd_chunk_kernel(DirectParams p) {
       M::mma(aK2[0][c], fXt, M::load_t(sK, LDKT, k0, 32 * (NKT * wj + c), lane));
     }
   }
-  lds_barrier();  // the four small tiles are dead; sM and sMisc are complete
-  // dq and dk through their staging tiles.  Thread = (token tid / 4, the 8-column groups tid % 4, tid % 4 + 4, ...): the
-  // row dots <q_t, dq_t> and <k_t, dk_t> give the gate gradient and carry the gradients through the normalisation,
+  if (GATE == LNX_GATE_SCALAR) {  // <q_t, dq_t> - <k_t, dk_t> before anything is rounded: what one pair gives to both cancels along the chunk
+    float x[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) x[e] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NKT; ++c)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const floatx4 k4 = M::load_acc_rows(sK, LDKT, 32 * wi, q, 32 * (NKT * wj + c), lane);
+        const floatx4 q4 = M::load_acc_rows(sQ, LDKT, 32 * wi, q, 32 * (NKT * wj + c), lane);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[4 * q + u] += q4[u] * aQ[0][c][4 * q + u] - k4[u] * aK2[0][c][4 * q + u];
+      }
+    rows_reduce_add<1>(x, 32 * wi, lane, sdG + 64 * (wj >> 1));
+  }
+  lds_barrier();  // the four small tiles are dead; sM, sdG and sMisc are complete
+  // dq and dk through their staging tiles.  Thread = (token tid / TPT, the 8-column groups tid % TPT, tid % TPT + TPT, ...): the
+  // row dots <q_t, dq_t> and <k_t, dk_t> carry the gradients through the normalisation,
   //   d/dx of x / (|x| + eps) applied to dy:  dy / (|x| + eps) - y <y, dy> / |x|.
-  const int tr = tid >> 2, tq = 8 * (tid & 3);
-  float dgp = 0.f;
-  auto emit = [&](const T* sSt, const T* sIn, float fac, T* out, float sign) {
-    float dot = 0.f;
+  const int tr = tid / TPT, tq = 8 * (tid % TPT);
+  auto emit = [&](const T* sSt, const T* sIn, float fac, T* out) {
+    float cf = 0.f;
+    if (p.l2norm) {
+      float dot = 0.f;
 #pragma unroll
-    for (int u = 0; u < DK; u += 32) {
-      const M::Frag a = M::load(sSt + tr * LDK + tq + u), b = M::load(sIn + tr * LDKT + tq + u);
+      for (int u = 0; u < DK; u += 8 * TPT) {
+        const M::Frag a = M::load(sSt + tr * LDK + tq + u), b = M::load(sIn + tr * LDKT + tq + u);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) dot += (float)a[e] * (float)b[e];
+        for (int e = 0; e < 8; ++e) dot += (float)a[e] * (float)b[e];
+      }
+      dot = token_sum(dot);
+      const float nrm = 1.f / fac - LNX_L2_EPS;
+      cf = nrm > 0.f ? dot / nrm : 0.f;
     }
-    dot = quad_sum(dot);
-    dgp += sign * dot;
-    const float nrm = 1.f / fac - LNX_L2_EPS;
-    const float cf = (p.l2norm && nrm > 0.f) ? dot / nrm : 0.f;
     if (tr < len) {
 #pragma unroll
-      for (int u = 0; u < DK; u += 32) {
+      for (int u = 0; u < DK; u += 8 * TPT) {
         M::Frag a = M::load(sSt + tr * LDK + tq + u);
         const M::Frag b = M::load(sIn + tr * LDKT + tq + u);
 #pragma unroll
@@ -1092,21 +1135,14 @@ __global__ __launch_bounds__(256, 2) void bwd_chunk_kernel(DirectParams p) {
   frag_store<T, 1, NKT>(aQ, sSt + 32 * wi * LDK + 32 * NKT * wj, LDK, lane);
   frag_store<T, 1, NKT>(aK2, sSt2 + 32 * wi * LDK + 32 * NKT * wj, LDK, lane);
   lds_barrier();
-  emit(sSt, sQ, sNq[tr], p.dq, 1.f);
-  emit(sSt2, sK, sNk[tr], p.dk, -1.f);
-  if (GATE == LNX_GATE_SCALAR) {
-    if ((tid & 3) == 0) {
-      float d = dgp + 2.f * sBeta[tr] * sM[tr];
-      if (tr == 63) d += ((sMisc[4] + sMisc[5]) + (sMisc[6] + sMisc[7])) + __expf(gC) * ((sMisc[8] + sMisc[9]) + (sMisc[10] + sMisc[11]));
-      sdG[tr] = d;
-    }
-    lds_barrier();
-  }
+  emit(sSt, sQ, sNq[tr], p.dq);
+  emit(sSt2, sK, sNk[tr], p.dk);
   if (wave == 0) {
     const int t = lane;
-    if (t < len) p.dbeta[tbase + t * ts] = sRdv[t] + sM[t];
+    if (t < len) p.dbeta[tbase + t * ts] = sRdv[t] + (sM[t] + sM[64 + t]);
     if (GATE == LNX_GATE_SCALAR) {  // dg = reverse cumulative sum of dG over the chunk
-      float d = sdG[t];
+      float d = sdG[t] + sdG[64 + t] + 2.f * sBeta[t] * (sM[t] + sM[64 + t]);
+      if (t == 63) d += waves_sum(sMisc + 8) + __expf(gC) * waves_sum(sMisc + 16);
 #pragma unroll
       for (int s_ = 1; s_ < 64; s_ <<= 1) {
         const float y = __shfl_down(d, s_, LNX_WAVE);
@@ -1123,14 +1159,16 @@ int launch_bwd_chunk(const DirectParams& p, hipStream_t st) {
   const size_t b = BChunkL<DK>::bytes;
   if (const int rc = lnx_lds_limit((const void*)k, b); rc != LNX_OK) return rc;
   lnx_profile_mark("bwd_chunk", st);
-  hipLaunchKernelGGL(k, dim3((unsigned)((int64_t)p.geom.rows * p.geom.N)), dim3(256), b, st, p);
+  hipLaunchKernelGGL(k, dim3((unsigned)((int64_t)p.geom.rows * p.geom.N)), dim3(BChunkL<DK>::THREADS), b, st, p);
   lnx_profile_mark(nullptr, st);
   return LNX_OK;
 }
 
 template <int DK, int GATE>
 int launch_bwd(const DirectParams& p, int nstate, hipStream_t st) {
-  int rc = launch_scan_bwd<DK, GATE>(p, nstate, st);
+  int rc;
+  if constexpr (DK == 256) rc = lnx_wide_scan(true, p, nstate, st);
+  else rc = launch_scan_bwd<DK, GATE>(p, nstate, st);
   if (rc != LNX_OK) return rc;
   return launch_bwd_chunk<DK, GATE>(p, st);
 }
@@ -1147,11 +1185,20 @@ int scan_fwd_by_shape(const DirectParams& p, int dk, int gate, int nstate, hipSt
 }  // namespace
 
 int lnx_direct_scan_fwd(const DirectParams& p, int dk, int gate, int nstate, hipStream_t st) {
+  if (dk == 256) {
+    const int rc = lnx_wide_scan(false, p, nstate, st);
+    lnx_profile_mark(nullptr, st);
+    return rc;
+  }
   return p.o_dtype == LNX_F32 ? scan_fwd_by_shape<float>(p, dk, gate, nstate, st) : scan_fwd_by_shape<bf16_t>(p, dk, gate, nstate, st);
 }
 
+namespace {
+template <int DK> int bwd_by_gate(const DirectParams& p, int gate, int nstate, hipStream_t st) {
+  return gate == LNX_GATE_SCALAR ? launch_bwd<DK, LNX_GATE_SCALAR>(p, nstate, st) : launch_bwd<DK, LNX_GATE_NONE>(p, nstate, st);
+}
+}  // namespace
+
 int lnx_direct_bwd(const DirectParams& p, int dk, int gate, int nstate, hipStream_t st) {
-  if (dk == 128)
-    return gate == LNX_GATE_SCALAR ? launch_bwd<128, LNX_GATE_SCALAR>(p, nstate, st) : launch_bwd<128, LNX_GATE_NONE>(p, nstate, st);
-  return gate == LNX_GATE_SCALAR ? launch_bwd<64, LNX_GATE_SCALAR>(p, nstate, st) : launch_bwd<64, LNX_GATE_NONE>(p, nstate, st);
+  return dk == 256 ? bwd_by_gate<256>(p, gate, nstate, st) : dk == 128 ? bwd_by_gate<128>(p, gate, nstate, st) : bwd_by_gate<64>(p, gate, nstate, st);
 }

@@ -1397,11 +1397,6 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   if (const int rc = lnx_lds_limit((const void*)k1, b1); rc != LNX_OK) return rc;
   lnx_profile_mark("chunk_prepare", st);
   hipLaunchKernelGGL(k1, dim3((unsigned)slots), dim3(256), b1, st, p);
-  if constexpr (sizeof(T) == 2 && DK == 256 && GATE != LNX_GATE_VECTOR) {
-    const int rc = lnx_wide_scan(false, direct_params(p, GATE), nstate, st);
-    lnx_profile_mark(nullptr, st);
-    return rc;
-  } else {
   // 32-column slabs when 64-column ones would occupy at most half of the chip (256 CUs); always for 4-byte inputs
   // with dk = 256, whose tiles leave no room in LDS for a wider slab
   constexpr bool can_narrow = (DK >= 128 && sizeof(T) == 2) || (DK == 128 && sizeof(T) == 4);
@@ -1427,7 +1422,6 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   }
   lnx_profile_mark(nullptr, st);
   return LNX_OK;
-  }
 }
 
 template <typename T, int DK>
@@ -1468,7 +1462,7 @@ int lnx_chunk_check(const lnx_scan_args* a, bool backward) {
   if (a->dtype != LNX_F32 && a->dtype != LNX_BF16) return lnx_set_error(LNX_ERR_DTYPE, "dtype %d", a->dtype);
   if (a->o_dtype != LNX_F32 && a->o_dtype != LNX_BF16) return lnx_set_error(LNX_ERR_DTYPE, "o_dtype %d", a->o_dtype);
   if (a->use_qk_l2norm && !lnx_chunk_direct(a))
-    return lnx_set_error(LNX_ERR_SHAPE, "use_qk_l2norm inside the chunk kernels needs 2-byte inputs, dk <= 128 and no per-channel gate; "
+    return lnx_set_error(LNX_ERR_SHAPE, "use_qk_l2norm inside the chunk kernels needs 2-byte inputs and no per-channel gate; "
                                         "normalise with lnx_l2norm_fwd first");
   if (a->token_first != 0 && a->token_first != 1) return lnx_set_error(LNX_ERR_SHAPE, "token_first must be 0 or 1");
   if ((a->test_scan_slab != 0 && a->test_scan_slab != 32 && a->test_scan_slab != 64) || a->test_out_slabs < 0)
@@ -1489,8 +1483,8 @@ int lnx_chunk_check(const lnx_scan_args* a, bool backward) {
 
 namespace {
 
-// 2-byte inputs with dk <= 128 and no per-channel gate: the prepare kernel stops at Tm, Pm and G, the scan of
-// chunk_direct.hip does the rest.
+// 2-byte inputs without a per-channel gate: the prepare kernel stops at Tm, Pm and G, the scans of chunk_direct.hip and
+// chunk_wide.hip do the rest.
 template <int DK, int GATE>
 void launch_prepare_lite(const FwdParams& p, hipStream_t st) {
   auto k = chunk_prepare2_kernel<bf16_t, DK, GATE, true>;
@@ -1502,12 +1496,10 @@ void launch_prepare_lite(const FwdParams& p, hipStream_t st) {
 int launch_direct_fwd(const lnx_scan_args* a, const FwdParams& p, int nstate, bool prepared, hipStream_t st) {
   if (prepared) {
     // Tm, Pm, G and the row factors do not depend on the values or the states
-  } else if (a->dk == 128) {
-    if (a->gate == LNX_GATE_SCALAR) launch_prepare_lite<128, LNX_GATE_SCALAR>(p, st);
-    else launch_prepare_lite<128, LNX_GATE_NONE>(p, st);
+  } else if (a->gate == LNX_GATE_SCALAR) {
+    (a->dk == 256 ? launch_prepare_lite<256, LNX_GATE_SCALAR> : a->dk == 128 ? launch_prepare_lite<128, LNX_GATE_SCALAR> : launch_prepare_lite<64, LNX_GATE_SCALAR>)(p, st);
   } else {
-    if (a->gate == LNX_GATE_SCALAR) launch_prepare_lite<64, LNX_GATE_SCALAR>(p, st);
-    else launch_prepare_lite<64, LNX_GATE_NONE>(p, st);
+    (a->dk == 256 ? launch_prepare_lite<256, LNX_GATE_NONE> : a->dk == 128 ? launch_prepare_lite<128, LNX_GATE_NONE> : launch_prepare_lite<64, LNX_GATE_NONE>)(p, st);
   }
   const DirectParams d = direct_params(p, a->gate);
   int rc = lnx_direct_scan_fwd(d, a->dk, a->gate, nstate, st);
@@ -1558,8 +1550,8 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
   p.ws = ws; p.off = w;
   int rc;
   if (lnx_chunk_direct(a)) return launch_direct_fwd(a, p, nstate, prepared, st);
-  if (a->dtype == LNX_BF16)  // dk <= 128 without a per-channel gate went to the direct-solve kernels above
-    rc = (a->dk == 256)   ? launch_fwd_gate<bf16_t, 256>(a->gate, p, nstate, st)
+  if (a->dtype == LNX_BF16)  // calls without a per-channel gate went to the direct-solve kernels above
+    rc = (a->dk == 256)   ? launch_fwd<bf16_t, 256, LNX_GATE_VECTOR>(p, nstate, st)
          : (a->dk == 128) ? launch_fwd<bf16_t, 128, LNX_GATE_VECTOR>(p, nstate, st)
                           : launch_fwd<bf16_t, 64, LNX_GATE_VECTOR>(p, nstate, st);
   else

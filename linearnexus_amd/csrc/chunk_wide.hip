@@ -1,24 +1,25 @@
-// The two sequential passes of the WY-split chunk kernels for 2-byte inputs with dk = 256 and no / a scalar gate (the head shape of
-// the Gated DeltaNet presets).  Same products and roundings as chunk_scan (chunk_fwd.hip) and bwd_scan (chunk_bwd.hip), which serve
-// the other shapes.  The forward sums have their order, too; in reverse Q^T dO is added before W^T dD, as bwd_scan does up to dk = 128 --
-// its 64-column slabs of dk = 256 added W^T dD first, because Q shared a tile with K -- so that gradients differ from that form's by the
-// rounding of one sum (1.2e-4 of the 2-norm in bf16):
+// The two sequential passes of the direct-solve split (chunk_direct.hip has the algebra) for 2-byte inputs with dk = 256 and no / a
+// scalar gate (the head shape of the Gated DeltaNet presets):
 //
-//   forward   D = U - W S       O = scale diag(e^G) (Q S) + Pm D       S' = e^{G_C} S + (diag(e^{G_C - G}) K)^T D
-//   reverse   dD = Pm^T dO + diag(e^{G_C - G}) K dS'                   dS = e^{G_C} dS' + (scale diag(e^G) Q)^T dO - W^T dD
+//   forward   Y = K S    R = diag(beta) (V - diag(e^G) Y)    D = Tm R    O = scale diag(e^G) (Q S) + Pm D
+//             S' = e^{G_C} S + (diag(e^{G_C - G}) K)^T D
+//   reverse   dD = Pm^T dO + diag(e^{G_C - G}) K dS'    dR = Tm^T dD    dv = diag(beta) dR    dY = -diag(beta e^G) dR
+//             dS = e^{G_C} dS' + (scale diag(e^G) Q)^T dO + K^T dY
 //
-// What bounds them: with dk = 256 a chunk's K, Q and W rows are 96 KB, which every workgroup of a (state, head) loads again for
-// its slab of value columns, and LDS holds them once.  So a slab is as wide as the registers allow: a compute wave owns 16 NC value
+// What bounds them: with dk = 256 a chunk's K and Q rows are 64 KB, which every workgroup of a (state, head) loads again for
+// its slab of value columns.  So a slab is as wide as the registers allow: a compute wave owns 16 NC value
 // columns, whose [256 x 16 NC] part of the state stays in accumulators for the whole sequence and is the operand of the next
-// products as it stands (a column of tiles as Mma16 describes, in natural order); only K, Q, W and Pm come from LDS.  The state also
+// products as it stands (a column of tiles as Mma16 describes, in natural order); only K, Q, Tm and Pm come from LDS.  The state also
 // leaves from there: an operand fragment is 16 bytes of a row of the saved tensor.  Four mover waves hold the next chunk
 // in registers.  Per chunk:
 //   B1   tiles of chunk n in LDS               compute: everything but the last product     movers: loads of the next chunk
-//   B2   its K (forward) / W (reverse) is left   compute: the last product    movers: results -> global, the other tiles -> LDS
-//   B3                                         compute: state -> global     movers: the last tile -> LDS
-// Measured at B8 H8 T4096 dv512 (128-column slabs, 256 workgroups): forward 750 -> 551 us, reverse 658 -> 464 us against the
-// passes with 64-column slabs.  A chunk takes 7 - 8.6 us there, of which 216 KB through the CU's memory path are most: 64 KB of
-// state per chunk and slab leave for the backward kernels.  State stores among the products of the first phase instead of
+//   B2   its K is left                         compute: the last product    movers: results -> global, the other tiles -> LDS
+//   B3                                         compute: state -> global     movers: K -> LDS
+// Measured at B8 H8 T4096 dv512 (128-column slabs, 256 workgroups): forward 511 us, reverse 470 us, 8 and 7.4 us a chunk, of which
+// 185 KB through the CU's memory path (64 KB of state per chunk and slab leave for the backward kernels) are most.  The WY split's
+// passes, which read W and U instead of Tm and V, took 521 and 435 us behind 205 us of preparation (now 68) and 221 us of normalisation
+// outside the kernels (now none), and before two more kernels of 804 and 289 us (now one of 806): the step 2478 -> 1827 us.
+// State stores among the products of the first phase instead of
 // behind the last barrier: 551 -> 587 and 464 -> 521 us (a wave whose store waits for a slot multiplies nothing).
 
 #include <type_traits>
@@ -51,26 +52,92 @@ __device__ __forceinline__ Frag load_cols(const T* tile, int ld, int s, int ci, 
   return S16::join(__builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((S16::lds_short4*)(p))),
                    __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((S16::lds_short4*)(p + 16 * ld))));
 }
-// a fetched tile to LDS, its rows at their places
-template <int COLS> __device__ __forceinline__ void store_placed(const TileRegs<T, 64, COLS>& R, T* dst, int ld, int tid) {
-  typedef TileRegs<T, 64, COLS> Tile;
-#pragma unroll
-  for (int it = 0; it < Tile::IT; ++it) {
-    const int idx = tid + 256 * it, r = idx / Tile::VPR, c = (idx - r * Tile::VPR) * Tile::N;
-    *reinterpret_cast<bf16x8*>(dst + place(r) * ld + c) = R.x[it];
-  }
-}
-
 template <int NC, int NCW> struct WideL {
-  static constexpr int BV = 16 * NC * NCW, LDK = DK + 16, LDC = LNX_C + 16, LDV = BV + 8;
-  static constexpr int kRow = 64 * LDK, kC = 64 * LDC, kV = 64 * LDV;
-  // K | Q | W | Pm | U, replaced by D (reverse: dO) | O on its way out (reverse: dD) | scalars
-  static constexpr size_t bytes = sizeof(T) * (3 * kRow + kC + 2 * kV) + sizeof(float) * 192;
+  static constexpr int BV = 16 * NC * NCW, LDK = DK + 16, LDC = LNX_C + 16, LDV = BV + 8, LDT = LNX_C + 8;
+  static constexpr int kRow = 64 * LDK, kC = 64 * LDC, kV = 64 * LDV, kT = BV * LDT;
+  // K | Q | Tm | Pm | V (reverse: dO) | O (reverse: dv) on its way out | D^T (reverse: dR^T) on its way out | scalars
+  static constexpr size_t bytes = sizeof(T) * (2 * kRow + 2 * kC + 2 * kV + kT) + sizeof(float) * 272;
   static constexpr int threads = 64 * NCW + 256;
   static_assert(bytes <= 160 * 1024, "LDS");
 };
 struct Sc {
-  enum { R = 0, Q = 64, DEC = 128 };  // e^{G_C - G}, scale e^G, e^{G_C}
+  enum { R = 0, Q = 64, BETA = 128, GAM = 192, DEC = 256 };  // e^{G_C - G}, scale e^G, beta, beta e^G, e^{G_C}
+};
+
+// Tm or Pm, lower-triangular and packed in the workspace, between its loads and its LDS stores: 288 vectors for 256 threads, rows at
+// their places.  The vectors above the diagonal are zeroed once ...
+struct PlacedTri {
+  bf16x8 x[2];
+  int o[2];
+  bool second;
+  __device__ __forceinline__ void init(int ld, int tid) {
+    second = tid < LNX_TRI_VECS - 256;
+    int r, c;
+    tri_vec_pos(tid, r, c);
+    o[0] = place(r) * ld + 8 * c;
+    tri_vec_pos(second ? 256 + tid : 0, r, c);
+    o[1] = place(r) * ld + 8 * c;
+  }
+  __device__ __forceinline__ void load(const T* src, int tid) {  // threads without a second vector read past the end: zeros
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(src), 0, LNX_TRI_VECS * 16, 0x00020000);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) x[u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * (256 * u + tid), 0, 0));
+  }
+  __device__ __forceinline__ void store(T* dst) const {
+    *reinterpret_cast<bf16x8*>(dst + o[0]) = x[0];
+    if (second) *reinterpret_cast<bf16x8*>(dst + o[1]) = x[1];
+  }
+};
+// ... of both, one behind the other
+__device__ __forceinline__ void zero_upper(T* tiles, int ld, int stride, int tid) {
+  if (tid >= 512 - LNX_TRI_VECS) return;
+  int r, c;
+  upper_vec_pos(tid, r, c);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) *reinterpret_cast<bf16x8*>(tiles + t * stride + place(r) * ld + 8 * c) = vec_zero<T>();
+}
+// Row factors of a [64][DK] tile's vectors (1 / (|x| + eps) where the op normalises), and the tile's rows times them to LDS
+struct RowFactors {
+  float f[64 * DK / 8 / 256];
+  __device__ __forceinline__ void load(const float* src, int tid) {
+#pragma unroll
+    for (int it = 0; it < 64 * DK / 8 / 256; ++it) f[it] = src[(tid + 256 * it) / (DK / 8)];
+  }
+};
+__device__ __forceinline__ void store_rows(const TileRegs<T, 64, DK>& R, const RowFactors& F, bool scaled, T* dst, int ld, int tid) {
+#pragma unroll
+  for (int it = 0; it < TileRegs<T, 64, DK>::IT; ++it) {
+    const int idx = tid + 256 * it, r = idx / (DK / 8), c = (idx - r * (DK / 8)) * 8;
+    bf16x8 x = R.x[it];
+    if (scaled) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = (bf16_t)((float)x[e] * F.f[it]);
+    }
+    *reinterpret_cast<bf16x8*>(dst + place(r) * ld + c) = x;
+  }
+}
+// What the movers read per chunk besides the row and value tiles
+template <int GATE> struct Scalars {
+  float g = 0.f, gl = 0.f, b = 0.f;
+  __device__ __forceinline__ void load(const DirectParams& p, int64_t slot, int64_t tbase, int len, int mt) {
+    const int t = mt & 63;
+    if (GATE == LNX_GATE_SCALAR) {
+      const float* G = at<const float>(p.ws, p.off.G) + slot * 64;
+      g = G[t];
+      gl = G[63];
+    }
+    b = p.beta[tbase + (int64_t)min(t, len - 1) * p.geom.ts];
+    if (t >= len) b = 0.f;
+  }
+  __device__ __forceinline__ void put(float* sc, float scale, int mt) const {  // by the first 64 movers
+    if (mt >= 64) return;
+    const float eg = (GATE == LNX_GATE_SCALAR) ? __expf(g) : 1.f;
+    sc[Sc::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(gl - g, 0.f)) : 1.f;
+    sc[Sc::Q + mt] = scale * eg;
+    sc[Sc::BETA + mt] = b;
+    sc[Sc::GAM + mt] = b * eg;
+    if (mt == 0) sc[Sc::DEC] = (GATE == LNX_GATE_SCALAR) ? __expf(gl) : 1.f;
+  }
 };
 
 struct Chain {
@@ -88,13 +155,6 @@ template <int BV> __device__ __forceinline__ bool chain_of(const DirectParams& p
   return true;
 }
 
-// the gate's scalars of a chunk, by 64 threads
-template <int GATE> __device__ __forceinline__ void put_scalars(float* sc, float g, float gl, float scale, int t) {
-  sc[Sc::R + t] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(gl - g, 0.f)) : 1.f;
-  sc[Sc::Q + t] = (GATE == LNX_GATE_SCALAR) ? scale * __expf(g) : scale;
-  if (t == 0) sc[Sc::DEC] = (GATE == LNX_GATE_SCALAR) ? __expf(gl) : 1.f;
-}
-
 // The strip's state: column l16 of column tile c, rows by tiles.
 template <int NC> struct Strip {
   floatx4 x[NC][KT];
@@ -104,7 +164,14 @@ template <int NC> struct Strip {
 #pragma unroll
       for (int ci = 0; ci < KT; ++ci)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[c][ci][e] = src ? src[(int64_t)(row0(ci) + grp(lane) + e) * dv + 16 * c + (lane & 15)] : 0.f;
+        for (int e = 0; e < 4; ++e) x[c][ci][e] = 0.f;
+    if (!src) return;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int ci = 0; ci < KT; ++ci)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[c][ci][e] = src[(int64_t)(row0(ci) + grp(lane) + e) * dv + 16 * c + (lane & 15)];
     // the loads complete here: left pending into the loop, every iteration would count them down again
 #pragma unroll
     for (int c = 0; c < NC; ++c)
@@ -147,18 +214,25 @@ template <int NC> struct Strip {
   }
 };
 
+// D (dR) of a column tile as operands, transposed to LDS: 16 bytes are eight tokens of a value column
+__device__ __forceinline__ void put_t(T* sT, int ld, int col, const Frag (&b)[2], int lane) {
+#pragma unroll
+  for (int s = 0; s < 2; ++s) *reinterpret_cast<bf16x8*>(sT + (col + (lane & 15)) * ld + 32 * s + grp(lane)) = b[s];
+}
+
 template <int GATE, int NC, int NCW, typename OT>
 __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kernel(DirectParams p) {
   typedef WideL<NC, NCW> L;
-  constexpr int BV = L::BV, LDK = L::LDK, LDC = L::LDC, LDV = L::LDV;
+  constexpr int BV = L::BV, LDK = L::LDK, LDC = L::LDC, LDV = L::LDV, LDT = L::LDT;
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);
   T* sQ = sK + L::kRow;
-  T* sW = sQ + L::kRow;
-  T* sP = sW + L::kRow;
-  T* sU = sP + L::kC;
-  T* sO = sU + L::kV;
-  float* sc = reinterpret_cast<float*>(sO + L::kV);
+  T* sTm = sQ + L::kRow;
+  T* sP = sTm + L::kC;
+  T* sV = sP + L::kC;
+  T* sO = sV + L::kV;
+  T* sDT = sO + L::kV;
+  float* sc = reinterpret_cast<float*>(sDT + L::kT);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   Chain ch;
   if (!chain_of<BV>(p, ch)) return;
@@ -168,36 +242,37 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
   if (wave >= NCW) {
     // ---------------- movers ----------------
     const int mt = tid - 64 * NCW;
-    TileRegs<T, 64, DK> rK, rQ, rW;
-    TileRegs<T, 64, BV> rU;
-    TileRegs<T, 64, 64> rP;
-    float g = 0.f, gl = 0.f;
-    const int64_t tsk = (int64_t)p.geom.ts * DK;
+    TileRegs<T, 64, DK> rK, rQ;
+    TileRegs<T, 64, BV> rV;
+    PlacedTri rTm, rP;
+    RowFactors fk, fq;
+    Scalars<GATE> rs;
+    rTm.init(LDC, mt), rP.init(LDC, mt);
+    zero_upper(sTm, LDC, L::kC, mt);
+    const int64_t tsk = (int64_t)p.geom.ts * DK, tsv = (int64_t)p.geom.ts * p.vcols;
     auto fetch = [&](int n) {
       const int64_t slot = (int64_t)ch.row * N + n;
       int tok0, len;
       chunk_span(ch.span, n, tok0, len);
       const int64_t tbase = tok_index(p.geom, ch.row, tok0);
-      rW.load(at<const T>(p.ws, p.off.W) + slot * 64 * DK, DK, 64, mt);
       rQ.load(p.q + tbase * DK, tsk, len, mt);
-      rU.load(at<const T>(p.ws, p.off.U) + slot * 64 * p.dv + v0, p.dv, 64, mt);
-      rP.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, 64, 64, mt);
-      if (GATE == LNX_GATE_SCALAR) {
-        const float* G = at<const float>(p.ws, p.off.G) + slot * 64;
-        g = G[mt & 63];
-        gl = G[63];
-      }
+      fq.load(at<const float>(p.ws, p.off.Nq) + slot * 64, mt);
+      rV.load(p.v + tbase * p.vcols + v0, tsv, (v0 < p.vcols) ? len : 0, mt);  // columns v does not hold read as zero
+      rTm.load(at<const T>(p.ws, p.off.Tm) + slot * 64 * 64, mt);
+      rP.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
+      rs.load(p, slot, tbase, len, mt);
       rK.load(p.k + tbase * DK, tsk, len, mt);
+      fk.load(at<const float>(p.ws, p.off.Nk) + slot * 64, mt);
     };
     auto commit = [&]() {
-      store_placed<DK>(rW, sW, LDK, mt);
-      store_placed<DK>(rQ, sQ, LDK, mt);
-      rU.store(sU, LDV, mt);
-      store_placed<64>(rP, sP, LDC, mt);
+      store_rows(rQ, fq, p.l2norm, sQ, LDK, mt);
+      rV.store(sV, LDV, mt);
+      rTm.store(sTm);
+      rP.store(sP);
     };
     auto commit_k = [&]() {  // the scalars with it: the last product's decay is read until here
-      store_placed<DK>(rK, sK, LDK, mt);
-      if (mt < 64) put_scalars<GATE>(sc, g, gl, p.scale, mt);
+      store_rows(rK, fk, p.l2norm, sK, LDK, mt);
+      rs.put(sc, p.scale, mt);
     };
     if (c0 < c1) {
       fetch(c0);
@@ -213,8 +288,8 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
       chunk_span(ch.span, n, tok0, len);
       if (std::is_same<OT, T>::value && p.o)
         unstage_tile_checked<T, 64, BV>(reinterpret_cast<T*>(p.o) + tok_index(p.geom, ch.row, tok0) * p.dv + v0, tso, sO, LDV, len, mt);
-      if (p.save) unstage_tile<T, 64, BV, true>(at<T>(p.ws, p.off.D) + slot * 64 * p.dv + v0, p.dv, sU, LDV, 64, mt);
-      commit();  // U over D: every thread writes the vectors that it has just read
+      if (p.save) unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT, LDT, BV, mt);
+      commit();
       lds_barrier();  // B3
       commit_k();
       lds_barrier();  // B1 of the next chunk
@@ -232,8 +307,8 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
   if (c0 < c1) save(c0);
   lds_barrier();  // B1 of the first chunk
   for (int n = c0; n < c1; ++n) {
-    const int lane = fresh(tid & 63), l16 = lane & 15, g8 = grp(lane);
-    // ---- D = U - W S: rows = tokens ----
+    const int lane = fresh(tid & 63), g8 = grp(lane);
+    // ---- Y = K S: rows = tokens ----
     floatx4 y[NC][4];
 #pragma unroll
     for (int c = 0; c < NC; ++c)
@@ -246,29 +321,56 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
       for (int c = 0; c < NC; ++c) b[c] = S.operand(c, ks);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const Frag a = load_rows(sW, LDK, i, ks, lane);
+        const Frag a = load_rows(sK, LDK, i, ks, lane);
 #pragma unroll
         for (int c = 0; c < NC; ++c) S16::mma(y[c][i], a, b[c]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    Frag bd[NC][2], bu[NC][2];  // D, and D with its rows scaled by e^{G_C - G}, as operands
+    // ---- R = beta V - beta e^G Y, in place of Y ----
+    Frag br[NC][2];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      floatx4 d[4], e[4];
+    for (int s = 0; s < 2; ++s) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const bf16x4 u = S16::rows4(sU, LDV, row0(i) + g8, vs + 16 * c, lane);
-        d[i] = floatx4{(float)u[0], (float)u[1], (float)u[2], (float)u[3]} - y[c][i];
-        e[i] = d[i] * load4(sc + Sc::R + row0(i) + g8);
+      for (int i = 2 * s; i < 2 * s + 2; ++i) {
+        const floatx4 bt = load4(sc + Sc::BETA + row0(i) + g8), gm = load4(sc + Sc::GAM + row0(i) + g8);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const bf16x4 u = S16::rows4(sV, LDV, row0(i) + g8, vs + 16 * c, lane);
+          y[c][i] = bt * floatx4{(float)u[0], (float)u[1], (float)u[2], (float)u[3]} - gm * y[c][i];
+        }
       }
 #pragma unroll
-      for (int s = 0; s < 2; ++s) bd[c][s] = S16::from_acc(d[2 * s], d[2 * s + 1]), bu[c][s] = S16::from_acc(e[2 * s], e[2 * s + 1]);
-#pragma unroll
-      for (int s = 0; s < 2; ++s)  // D replaces U
-#pragma unroll
-        for (int r = 0; r < 8; ++r) sU[(32 * s + g8 + r) * LDV + vs + 16 * c + l16] = bd[c][s][r];
+      for (int c = 0; c < NC; ++c) br[c][s] = S16::from_acc(y[c][2 * s], y[c][2 * s + 1]);
     }
+    // ---- D = Tm R (Tm is lower-triangular: the first 32 tokens take the first step only) ----
+    Frag bd[NC][2], bu[NC][2];  // D, and D with its rows scaled by e^{G_C - G}, as operands
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      bf16x4 d0[NC], u0[NC];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int i = 2 * s + h;
+        floatx4 d[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) d[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k <= s; ++k) {
+          const Frag f = load_rows(sTm, LDC, i, k, lane);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) S16::mma(d[c], f, br[c][k]);
+        }
+        const floatx4 r = load4(sc + Sc::R + row0(i) + g8);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const bf16x4 x = pack_bf16x4(d[c]), u = pack_bf16x4(d[c] * r);
+          if (h == 0) d0[c] = x, u0[c] = u;
+          else bd[c][s] = S16::join(d0[c], x), bu[c][s] = S16::join(u0[c], u);
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) put_t(sDT, LDT, vs + 16 * c, bd[c], lane);
     __builtin_amdgcn_sched_barrier(0);
     // ---- O^T = scale e^G (Q S)^T + D^T Pm^T: columns = tokens, 32 of them at a time ----
 #pragma unroll
@@ -298,7 +400,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
 #pragma unroll
         for (int c = 0; c < NC; ++c) o[c][i] *= f;
 #pragma unroll
-        for (int k = 0; k <= h; ++k) {  // Pm is lower-triangular: the first 32 tokens take the first step only
+        for (int k = 0; k <= h; ++k) {  // Pm is lower-triangular, too
           const Frag f = load_rows(sP, LDC, 2 * h + i, k, lane);
 #pragma unroll
           for (int c = 0; c < NC; ++c) S16::mma(o[c][i], bd[c][k], f);
@@ -327,15 +429,16 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
 template <int GATE, int NC, int NCW>
 __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kernel(DirectParams p) {
   typedef WideL<NC, NCW> L;
-  constexpr int BV = L::BV, LDK = L::LDK, LDC = L::LDC, LDV = L::LDV;
+  constexpr int BV = L::BV, LDK = L::LDK, LDC = L::LDC, LDV = L::LDV, LDT = L::LDT;
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);
   T* sQ = sK + L::kRow;
-  T* sW = sQ + L::kRow;
-  T* sP = sW + L::kRow;
+  T* sTm = sQ + L::kRow;
+  T* sP = sTm + L::kC;
   T* sdO = sP + L::kC;
-  T* sdD = sdO + L::kV;
-  float* sc = reinterpret_cast<float*>(sdD + L::kV);
+  T* sdV = sdO + L::kV;
+  T* sdRT = sdV + L::kV;
+  float* sc = reinterpret_cast<float*>(sdRT + L::kT);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   Chain ch;
   if (!chain_of<BV>(p, ch)) return;
@@ -344,47 +447,51 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
   if (wave >= NCW) {
     // ---------------- movers ----------------
     const int mt = tid - 64 * NCW;
-    TileRegs<T, 64, DK> rK, rQ, rW;
+    TileRegs<T, 64, DK> rK, rQ;
     TileRegs<T, 64, BV> rdO;
-    TileRegs<T, 64, 64> rP;
-    float g = 0.f, gl = 0.f;
+    PlacedTri rTm, rP;
+    RowFactors fk, fq;
+    Scalars<GATE> rs;
+    rTm.init(LDC, mt), rP.init(LDC, mt);
+    zero_upper(sTm, LDC, L::kC, mt);
     const int64_t tsk = (int64_t)p.geom.ts * DK, tsv = (int64_t)p.geom.ts * p.dv;
     auto fetch = [&](int n) {
       const int64_t slot = (int64_t)ch.row * N + n;
       int tok0, len;
       chunk_span(ch.span, n, tok0, len);
       const int64_t tbase = tok_index(p.geom, ch.row, tok0);
-      rK.load(p.k + tbase * DK, tsk, len, mt);
       rdO.load(p.d_o + tbase * p.dv + v0, tsv, len, mt);
-      rP.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, 64, 64, mt);
+      rP.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
+      rTm.load(at<const T>(p.ws, p.off.Tm) + slot * 64 * 64, mt);
+      rs.load(p, slot, tbase, len, mt);
       rQ.load(p.q + tbase * DK, tsk, len, mt);
-      if (GATE == LNX_GATE_SCALAR) {
-        const float* G = at<const float>(p.ws, p.off.G) + slot * 64;
-        g = G[mt & 63];
-        gl = G[63];
-      }
-      rW.load(at<const T>(p.ws, p.off.W) + slot * 64 * DK, DK, 64, mt);
+      fq.load(at<const float>(p.ws, p.off.Nq) + slot * 64, mt);
+      rK.load(p.k + tbase * DK, tsk, len, mt);
+      fk.load(at<const float>(p.ws, p.off.Nk) + slot * 64, mt);
     };
     auto commit = [&]() {
-      store_placed<DK>(rK, sK, LDK, mt);
       rdO.store(sdO, LDV, mt);
-      store_placed<64>(rP, sP, LDC, mt);
-      store_placed<DK>(rQ, sQ, LDK, mt);
-      if (mt < 64) put_scalars<GATE>(sc, g, gl, p.scale, mt);
+      rP.store(sP);
+      rTm.store(sTm);
+      rs.put(sc, p.scale, mt);
+      store_rows(rQ, fq, p.l2norm, sQ, LDK, mt);
     };
     if (c0 < c1) {
       fetch(c1 - 1);
       commit();
-      store_placed<DK>(rW, sW, LDK, mt);
+      store_rows(rK, fk, p.l2norm, sK, LDK, mt);
     }
     lds_barrier();  // B1 of the first chunk
     for (int n = c1 - 1; n >= c0; --n) {
       fetch(max(n - 1, c0));
       lds_barrier();  // B2
-      unstage_tile<T, 64, BV, true>(at<T>(p.ws, p.off.dD) + ((int64_t)ch.row * N + n) * 64 * p.dv + v0, p.dv, sdD, LDV, 64, mt);
+      int tok0, len;
+      chunk_span(ch.span, n, tok0, len);
+      unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.dD) + ((int64_t)ch.row * N + n) * p.dv * 64 + (int64_t)v0 * 64, 64, sdRT, LDT, BV, mt);
+      unstage_tile_checked<T, 64, BV>(p.dv_out + tok_index(p.geom, ch.row, tok0) * p.dv + v0, tsv, sdV, LDV, len, mt);
       commit();
       lds_barrier();  // B3
-      store_placed<DK>(rW, sW, LDK, mt);
+      store_rows(rK, fk, p.l2norm, sK, LDK, mt);
       lds_barrier();  // B1 of the next chunk
     }
     return;
@@ -398,7 +505,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
   if (c0 < c1) save(c1 - 1);
   lds_barrier();  // B1 of the first chunk
   for (int n = c1 - 1; n >= c0; --n) {
-    const int lane = fresh(tid & 63), l16 = lane & 15, g8 = grp(lane);
+    const int lane = fresh(tid & 63), g8 = grp(lane);
     // ---- Z = K dS' ----
     floatx4 z[NC][4];
 #pragma unroll
@@ -431,7 +538,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
       }
     }
     // ---- dD = Pm^T dO + e^{G_C - G} Z; Pm^T is upper-triangular ----
-    Frag bd[NC][2];  // -dD
+    Frag bd[NC][2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       floatx4 d[NC][2];
@@ -451,19 +558,44 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
         for (int c = 0; c < NC; ++c) d[c][h] += r * z[c][i];
       }
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const Frag x = S16::from_acc(d[c][0], d[c][1]);
+      for (int c = 0; c < NC; ++c) bd[c][s] = S16::from_acc(d[c][0], d[c][1]);
+    }
+    // ---- dR = Tm^T dD (rows = tokens), and once more with the operands exchanged (columns = tokens), the orientation that dv leaves in;
+    //      Tm^T is upper-triangular ----
+    Frag by[NC][2];  // dY
 #pragma unroll
-        for (int r = 0; r < 8; ++r) sdD[(32 * s + g8 + r) * LDV + vs + 16 * c + l16] = x[r];
-        bd[c][s] = S16::from_acc(-d[c][0], -d[c][1]);
+    for (int s = 0; s < 2; ++s) {
+      floatx4 x[NC][2], gm[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int i = 2 * s + h;
+        floatx4 w[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) x[c][h] = w[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = s; k < 2; ++k) {
+          const Frag f = load_cols(sTm, LDC, k, i, lane);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) S16::mma(x[c][h], f, bd[c][k]), S16::mma(w[c], bd[c][k], f);
+        }
+        gm[h] = load4(sc + Sc::GAM + row0(i) + g8);
+        const int t = row0(i) + row_of(lane);
+        const float bt = sc[Sc::BETA + t];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) store4(sdV + t * LDV + vs + 16 * c + 4 * (lane >> 4), w[c] * bt);
+      }
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        *reinterpret_cast<bf16x8*>(sdRT + (vs + 16 * c + (lane & 15)) * LDT + 32 * s + g8) = S16::from_acc(x[c][0], x[c][1]);
+        by[c][s] = S16::from_acc(-gm[0] * x[c][0], -gm[1] * x[c][1]);
       }
     }
     // ---- dS <- e^{G_C} dS' + (scale e^G Q)^T dO ----
     if (GATE == LNX_GATE_SCALAR) dS.scale(sc[Sc::DEC]);
     dS.add(sQ, LDK, foq, lane);
     lds_barrier();  // B2
-    // ---- dS -= W^T dD ----
-    dS.add(sW, LDK, bd, lane);
+    // ---- dS += K^T dY ----
+    dS.add(sK, LDK, by, lane);
     lds_barrier();  // B3
     if (n > c0) save(n - 1);
     lds_barrier();  // B1 of the next chunk

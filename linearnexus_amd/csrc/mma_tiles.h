@@ -406,6 +406,14 @@ __device__ __forceinline__ void tri_vec_pos(int idx, int& r, int& c) {  // idx <
   r = 8 * g + q;
   c = o - q * (g + 1);
 }
+// The vectors above the diagonal (8 c > r) in turn, idx < 512 - LNX_TRI_VECS: group g of eight rows has 7 - g of them per row.
+__device__ __forceinline__ void upper_vec_pos(int idx, int& r, int& c) {
+  int g = 0;
+  while (56 * (g + 1) - 4 * (g + 1) * g <= idx) ++g;  // vectors of the groups before g + 1
+  const int o = idx - (56 * g - 4 * g * (g - 1)), per = 7 - g;
+  r = 8 * g + o / per;
+  c = g + 1 + (o - (o / per) * per);
+}
 // The packed tile in the registers of 256 or 512 threads (vector tid, with 256 also vector 256 + tid for tid < 32) between its global
 // loads and its LDS stores (columns in the order CHAIN of Mma16), like TileRegs; the LDS tile's upper part is zeroed once by the caller and never written.
 template <typename T, bool CHAIN, int THREADS = 256> struct TriRegs {

@@ -296,8 +296,8 @@ def _prefill_segments(B: int, H: int, T: int, dv: int, dk: int = 256, two_byte: 
     W and U prepare both passes: no gain at w = 64; fp32 4 heads of 4096 284 -> 194 us, bf16 per-channel gate 4 heads
     of 8192 237 -> 163 (4096: 131 -> 133).  From 512 chunks on, w = 64 gains from a second round (32768 tokens: 541 -> 508).
 
-    dk = 256: at most an eighth of the CUs busy and every segment keeps >= 64 chunks (fewer heads of 512 values gain
-    less than their longer preparation costs: 16 workgroups of 4096 tokens 196 -> 216 us)."""
+    dk = 256, and rows that would have to be copied to become heads: at most an eighth of the CUs busy and every segment keeps >= 64 chunks
+    (fewer heads of 512 values gain less than their longer preparation costs: 16 workgroups of 4096 tokens 196 -> 216 us)."""
     forced = os.environ.get("LNX_PREFILL_SEGMENTS")
     chunks = -(-T // CHUNK)
     if forced is not None:
@@ -312,6 +312,20 @@ def _prefill_segments(B: int, H: int, T: int, dv: int, dk: int = 256, two_byte: 
     if w > (64 if direct else 32) or chunks < (64 if (direct and w <= 32) or not two_byte else 128):
         return 1
     return min((512 if w > 32 and chunks >= 512 else 256) // w, max(8, chunks // 16))
+
+
+def _prefill_segments_256(B: int, H: int, T: int, dv: int) -> int:
+    """The same for dk = 256 in bf16 without a per-channel gate, where the second pass finds everything prepared.  A chain takes 3.3 - 6.5 us
+    a chunk and cutting about two of them more work, so it pays from 64 chunks on while w <= 64 and from 128 on while w <= 128 (H4 dv 512,
+    w = 48: 2048 tokens 115 -> 134 us, 4096 216 -> 185, 8192 419 -> 274; H8 dv 512, w = 96: 4096 219 -> 236, 8192 427 -> 384).  Eight segments;
+    four where w or a short prompt leaves them too little (w = 48, 4096 tokens: 185 against 199 us; w = 96, 16384: 687 against 715), sixteen
+    of few heads and long prompts (w = 12, 16384: 297 against 314; w = 24, 32768: 496 against 540)."""
+    chunks, w = -(-T // CHUNK), B * H * (4 + -(-dv // 64))
+    if os.environ.get("LNX_PREFILL_SEGMENTS") is not None:
+        return _prefill_segments(B, H, T, dv)
+    if w > 128 or chunks < (64 if w <= 64 else 128):
+        return 1
+    return 4 if w > 64 or (w > 24 and chunks < 128) else 16 if 3 * chunks >= 64 * w else 8
 
 
 def _segmented_forward(q, k, v, g, beta, scale, initial_state, l2norm, o_dtype, nseg):
@@ -345,8 +359,11 @@ def _chunk(q, k, v, g, beta, scale, initial_state, chunk_size, l2norm, o_dtype, 
         if forward_only and dkp is not None and q.dim() == 4 and cu_seqlens is None:
             # batch rows become heads: free for contiguous tensors, a copy of the token-first views of several rows
             folds = q.shape[0] == 1 or (q.is_contiguous() and k.is_contiguous() and v.is_contiguous())
-            nseg = _prefill_segments(q.shape[0], q.shape[1], q.shape[2], dv, dk if folds else 256, q.element_size() == 2,
-                                     g is not None and g.dim() == 4 and g.shape[-1] == dk)
+            two_byte, vector_gate = q.element_size() == 2, g is not None and g.dim() == 4 and g.shape[-1] == dk
+            if folds and dk > 128 and two_byte and not vector_gate:
+                nseg = _prefill_segments_256(q.shape[0], q.shape[1], q.shape[2], dv)
+            else:
+                nseg = _prefill_segments(q.shape[0], q.shape[1], q.shape[2], dv, dk if folds else 256, two_byte, vector_gate)
             if nseg > 1:
                 return _segmented_forward(q, k, v, g, beta, scale, initial_state, l2norm, o_dtype, nseg)
         return _chunk_forward(q, k, v, g, beta, initial_state, scale, l2norm, o_dtype, cu_seqlens, forward_only=forward_only)[:2]
