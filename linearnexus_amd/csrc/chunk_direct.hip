@@ -797,6 +797,10 @@ template <int DK> struct BChunkL {
   static constexpr bool OVER2 = DK <= 128;
   static constexpr size_t epi_bytes = sizeof(T) * (2 * kRow + 4 * kC + (OVER2 ? 0 : kSt));
   static_assert(kSt <= (OVER2 ? 2 : 4) * kC, "the staging tile overlays the small tiles");
+  // The gate gradient's row dots <q_t, dq_t> - <k_t, dk_t> from the accumulators, before anything is rounded (what one pair of tokens gives
+  // to both cancels along the chunk): dg is 4.0e-3 off instead of 6.5e-3.  dk <= 128 takes them from the staged rows, which its
+  // emit reads anyway: 7.0e-3.
+  static constexpr bool DOTS = DK == 256;
   static constexpr int nfloat = 64 * 10;
   static constexpr size_t bytes = sizeof(float) * nfloat + (epi_bytes > loop_bytes ? epi_bytes : loop_bytes);
   static_assert(bytes <= (NW == 4 ? 80 : 160) * 1024, "two workgroups of four waves per CU, one of eight");
@@ -1087,7 +1091,7 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
       M::mma(aK2[0][c], fXt, M::load_t(sK, LDKT, k0, 32 * (NKT * wj + c), lane));
     }
   }
-  if (GATE == LNX_GATE_SCALAR) {  // <q_t, dq_t> - <k_t, dk_t> before anything is rounded: what one pair gives to both cancels along the chunk
+  if constexpr (GATE == LNX_GATE_SCALAR && L::DOTS) {
     float x[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) x[e] = 0.f;
@@ -1107,9 +1111,10 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
   // row dots <q_t, dq_t> and <k_t, dk_t> carry the gradients through the normalisation,
   //   d/dx of x / (|x| + eps) applied to dy:  dy / (|x| + eps) - y <y, dy> / |x|.
   const int tr = tid / TPT, tq = 8 * (tid % TPT);
-  auto emit = [&](const T* sSt, const T* sIn, float fac, T* out) {
+  float dgp = 0.f;
+  auto emit = [&](const T* sSt, const T* sIn, float fac, T* out, float sign) {
     float cf = 0.f;
-    if (p.l2norm) {
+    if (!L::DOTS || p.l2norm) {
       float dot = 0.f;
 #pragma unroll
       for (int u = 0; u < DK; u += 8 * TPT) {
@@ -1118,8 +1123,9 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
         for (int e = 0; e < 8; ++e) dot += (float)a[e] * (float)b[e];
       }
       dot = token_sum(dot);
+      dgp += sign * dot;
       const float nrm = 1.f / fac - LNX_L2_EPS;
-      cf = nrm > 0.f ? dot / nrm : 0.f;
+      cf = (p.l2norm && nrm > 0.f) ? dot / nrm : 0.f;
     }
     if (tr < len) {
 #pragma unroll
@@ -1135,13 +1141,17 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
   frag_store<T, 1, NKT>(aQ, sSt + 32 * wi * LDK + 32 * NKT * wj, LDK, lane);
   frag_store<T, 1, NKT>(aK2, sSt2 + 32 * wi * LDK + 32 * NKT * wj, LDK, lane);
   lds_barrier();
-  emit(sSt, sQ, sNq[tr], p.dq);
-  emit(sSt2, sK, sNk[tr], p.dk);
+  emit(sSt, sQ, sNq[tr], p.dq, 1.f);
+  emit(sSt2, sK, sNk[tr], p.dk, -1.f);
+  if (GATE == LNX_GATE_SCALAR && !L::DOTS) {
+    if (tid % TPT == 0) sdG[tr] = dgp;
+    lds_barrier();
+  }
   if (wave == 0) {
     const int t = lane;
     if (t < len) p.dbeta[tbase + t * ts] = sRdv[t] + (sM[t] + sM[64 + t]);
     if (GATE == LNX_GATE_SCALAR) {  // dg = reverse cumulative sum of dG over the chunk
-      float d = sdG[t] + sdG[64 + t] + 2.f * sBeta[t] * (sM[t] + sM[64 + t]);
+      float d = (L::DOTS ? sdG[t] + sdG[64 + t] : sdG[t]) + 2.f * sBeta[t] * (sM[t] + sM[64 + t]);
       if (t == 63) d += waves_sum(sMisc + 8) + __expf(gC) * waves_sum(sMisc + 16);
 #pragma unroll
       for (int s_ = 1; s_ < 64; s_ <<= 1) {
