@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liblinearnexus_hip.so")
 HOST = os.path.join(HERE, "_host.so")
-SOURCES = ["c_api.hip", "recurrent.hip", "chunk_fwd.hip", "chunk_bwd.hip", "chunk_direct.hip", "chunk_wide.hip", "conv1d.hip", "dplr.hip", "dplr_chunk.hip", "rmsnorm_gated.hip", "kda_gate.hip", "gdn_gate.hip"]
+SOURCES = ["c_api.hip", "recurrent.hip", "chunk_fwd.hip", "chunk_bwd.hip", "chunk_direct.hip", "chunk_wide.hip", "chunk_kda.hip", "conv1d.hip", "dplr.hip", "dplr_chunk.hip", "rmsnorm_gated.hip", "kda_gate.hip", "gdn_gate.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffast-math", "-fno-finite-math-only",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -1446,11 +1446,7 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
   constexpr bool can_narrow = (DK >= 128 && sizeof(T) == 2) || (DK == 128 && sizeof(T) == 4);
   constexpr int WIDE = 64, NARROW = can_narrow ? 32 : WIDE;
   const bool narrow = can_narrow && lnx_narrow_slabs((int64_t)nstate * p.geom.H * (p.dv / 64), p.slab);
-  auto k2 = bwd_dqk_kernel<T, DK, GATE>;
-  auto k3 = (GATE == LNX_GATE_VECTOR && p.graw) ? bwd_wy2_kernel<T, DK, GATE, GATE == LNX_GATE_VECTOR> : bwd_wy2_kernel<T, DK, GATE>;
-  const size_t b2 = DqkCfg<T, DK, GATE>::bytes, b3 = Wy2Cfg<T, DK, GATE>::bytes;
   int rc;
-  if ((rc = lnx_lds_limit((const void*)k2, b2)) != LNX_OK || (rc = lnx_lds_limit((const void*)k3, b3)) != LNX_OK) return rc;
   if (!BScanCfg<T, DK>::FUSE_LOCAL) {  // otherwise bwd_scan forms the chunk-local part itself
     lnx_profile_mark("bwd_local", st);
     hipLaunchKernelGGL(bwd_local_kernel<T>, dim3(lnx_xcd_grid(slots, p.dv / 64)), dim3(256), 0, st, p);
@@ -1461,12 +1457,28 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
   if ((rc = lnx_lds_limit((const void*)k1, b1)) != LNX_OK) return rc;
   lnx_profile_mark("bwd_scan", st);
   hipLaunchKernelGGL(k1, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(512), b1, st, p);
+  if constexpr (sizeof(T) == 2 && DK <= 128) {
+    KdaBwdParams k = {};
+    k.geom = p.geom;
+    k.q = reinterpret_cast<const bf16_t*>(p.q); k.k = reinterpret_cast<const bf16_t*>(p.k); k.v = reinterpret_cast<const bf16_t*>(p.v);
+    k.beta = p.beta; k.dv = p.dv; k.scale = p.scale; k.ws = p.ws; k.off = p.off;
+    k.d_o = reinterpret_cast<const bf16_t*>(p.d_o); k.dq = reinterpret_cast<bf16_t*>(p.dq); k.dk = reinterpret_cast<bf16_t*>(p.dk);
+    k.dv_out = reinterpret_cast<bf16_t*>(p.dv_out); k.dbeta = p.dbeta; k.dg = p.dg;
+    k.graw = reinterpret_cast<const bf16_t*>(p.graw); k.gA = p.gA; k.gbias = p.gbias; k.gthr = p.gthr; k.gband = p.gband;
+    k.dgraw = reinterpret_cast<bf16_t*>(p.dgraw); k.gpart = p.gpart; k.gprows = p.gprows;
+    return lnx_kda_bwd_chunk(k, DK, st);
+  } else {
+  auto k2 = bwd_dqk_kernel<T, DK, GATE>;
+  auto k3 = (GATE == LNX_GATE_VECTOR && p.graw) ? bwd_wy2_kernel<T, DK, GATE, GATE == LNX_GATE_VECTOR> : bwd_wy2_kernel<T, DK, GATE>;
+  const size_t b2 = DqkCfg<T, DK, GATE>::bytes, b3 = Wy2Cfg<T, DK, GATE>::bytes;
+  if ((rc = lnx_lds_limit((const void*)k2, b2)) != LNX_OK || (rc = lnx_lds_limit((const void*)k3, b3)) != LNX_OK) return rc;
   lnx_profile_mark("bwd_dqk", st);
   hipLaunchKernelGGL(k2, dim3(lnx_xcd_grid(slots, DK / 64)), dim3(256), b2, st, p);
   lnx_profile_mark("bwd_wy", st);
   hipLaunchKernelGGL(k3, dim3((unsigned)slots), dim3(256), b3, st, p);
   lnx_profile_mark(nullptr, st);
   return LNX_OK;
+  }
 }
 
 template <typename T, int DK>

@@ -123,6 +123,9 @@ inline bool lnx_chunk_direct(const lnx_scan_args* a) {
   return a->dtype == LNX_BF16 && a->gate != LNX_GATE_VECTOR;
 }
 
+// 2-byte inputs with a per-channel gate and dk <= 128: the scans of the WY split, then the one gradient kernel of chunk_kda.hip.
+inline bool lnx_chunk_kda(const lnx_scan_args* a) { return a->dtype == LNX_BF16 && a->dk <= 128 && a->gate == LNX_GATE_VECTOR; }
+
 inline uint64_t lnx_align256(uint64_t x) { return (x + 255) & ~uint64_t(255); }
 
 inline int lnx_chunk_slots(const lnx_scan_args* a) {
@@ -161,7 +164,8 @@ inline ChunkWs lnx_chunk_ws_layout(const lnx_scan_args* a) {
   w.Tm = w.Nq = w.Nk = w.Fq = 0;
   w.G = take(vec ? slots * C * dk * 4 : slots * C * 4);
   w.P = take(slots * C * C * es);
-  w.X = take(vec && saved ? slots * C * C * es : 0);
+  const bool kda = lnx_chunk_kda(a);
+  w.X = take(vec && saved && !kda ? slots * C * C * es : 0);
   w.W = take(slots * C * dk * es);
   w.U = take(slots * C * dv * es);
   w.Kr = take(vec ? slots * C * dk * es : 0);
@@ -171,8 +175,8 @@ inline ChunkWs lnx_chunk_ws_layout(const lnx_scan_args* a) {
   w.SnT = take(saved ? slots * dv * dk * es : 0);
   w.dD = take(bwd ? slots * C * dv * es : 0);
   w.dSn = take(bwd ? slots * dk * dv * es : 0);
-  w.dW = take(bwd ? slots * C * dk * es : 0);
-  w.dG = take(bwd ? (vec ? slots * C * dk * 4 : slots * C * 4 * (dk / 64)) : 0);  // scalar gate: one slot per 64-channel part
+  w.dW = take(bwd && !kda ? slots * C * dk * es : 0);
+  w.dG = take(bwd && !kda ? (vec ? slots * C * dk * 4 : slots * C * 4 * (dk / 64)) : 0);  // scalar gate: one slot per 64-channel part
   // fused gate activation: one partial row of its parameter gradients per chunk slot of a (batch element, head)
   w.gpart = take(bwd && vec && a->gate_raw ? lnx_gate_part_bytes((int64_t)(slots / a->H), a->H * a->dk) : 0);
   w.total = off;
@@ -225,6 +229,18 @@ struct DirectParams {
   float* dg;
   float* ds0;
 };
+// ... and of the chunk-local gradients of the per-channel gate (chunk_kda.hip): what a gate activated inside the op adds
+struct KdaBwdParams : DirectParams {
+  const bf16_t* graw;  // raw gate projection, or NULL
+  const float* gA;
+  const float* gbias;
+  float gthr;
+  int gband;
+  bf16_t* dgraw;
+  float* gpart;
+  int64_t gprows;
+};
+int lnx_kda_bwd_chunk(const KdaBwdParams& p, int dk, hipStream_t st);
 int lnx_direct_scan_fwd(const DirectParams& p, int dk, int gate, int nstate, hipStream_t st);
 int lnx_direct_bwd(const DirectParams& p, int dk, int gate, int nstate, hipStream_t st);
 // The sequential passes for dk = 256 (chunk_wide.hip).

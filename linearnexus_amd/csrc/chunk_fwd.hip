@@ -669,7 +669,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
         x[e] = (j0 + e < i) ? x[e] : 0.f;
         pp[e] = (j0 + e <= i) ? p.scale * pp[e] : 0.f;
       }
-      if (p.save) store4(Xg + i * 64 + j0, x);
+      if (p.save && !(sizeof(T) == 2 && DK <= 128)) store4(Xg + i * 64 + j0, x);  // chunk_kda.hip does without
       store4(Pg + i * 64 + j0, pp);
       store4(sA + i * LNX_LDA + j0, x * sBeta[i]);
     }
