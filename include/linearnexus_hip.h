@@ -54,7 +54,7 @@ typedef struct lnx_scan_args {
   int32_t o_dtype;          /* lnx_dtype of o */
   int32_t gate;             /* lnx_gate */
   int32_t use_qk_l2norm;    /* normalise q, k rows as x / (|x|_2 + 1e-6) inside the op: always honoured by the decode step
-                               and the token-by-token scan; by the chunk entry points where lnx_chunk_fuses_l2norm
+                               and the token-by-token scan; by the chunk entry points where lnx_chunk_normalises_qk
                                says so (ABI version 6), d_q and d_k are then the gradients of the raw q and k */
   int32_t nseq;             /* number of packed sequences; 0 for a dense batch */
   float scale;              /* multiplies q (after normalisation) */
@@ -164,10 +164,12 @@ int lnx_chunk_fwd_segmented_final(const lnx_scan_args* a, int32_t nseg, void* hi
 /*
  * 1 when lnx_chunk_fwd / lnx_chunk_bwd apply the in-op normalisation of q and k themselves for these arguments
  * (use_qk_l2norm = 1: gated_deltanet.py:273-275, kda.py:379-381 normalise inside the op, and it is their default):
- * q, k, v in bf16, no per-channel gate.  The rows are scaled where the kernels stage them and the
+ * q, k, v in bf16, and dk <= 128 with a per-channel gate.  The rows are scaled where the kernels stage them and the
  * backward pass carries d_q, d_k through the normalisation, so no normalised copies of q and k exist.  0: the chunk
  * entry points refuse use_qk_l2norm for these arguments; normalise with lnx_l2norm_fwd first.
  */
+int lnx_chunk_normalises_qk(const lnx_scan_args* a);
+/* The same for calls without a per-channel gate only (0 with one). */
 int lnx_chunk_fuses_l2norm(const lnx_scan_args* a);
 
 /*

@@ -30,7 +30,7 @@ struct BwdParams {
   float* dbeta;
   float* dg;
   float* ds0;
-  int dv, gate;
+  int dv, gate, l2norm;
   int slab;  // lnx_scan_args.test_scan_slab
   // per-channel gate activated inside the op (lnx_scan_args.gate_raw): bwd_wy2 carries dg through the activation
   const void* graw;
@@ -1461,7 +1461,7 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
     KdaBwdParams k = {};
     k.geom = p.geom;
     k.q = reinterpret_cast<const bf16_t*>(p.q); k.k = reinterpret_cast<const bf16_t*>(p.k); k.v = reinterpret_cast<const bf16_t*>(p.v);
-    k.beta = p.beta; k.dv = p.dv; k.scale = p.scale; k.ws = p.ws; k.off = p.off;
+    k.beta = p.beta; k.dv = p.dv; k.l2norm = p.l2norm; k.scale = p.scale; k.ws = p.ws; k.off = p.off;
     k.d_o = reinterpret_cast<const bf16_t*>(p.d_o); k.dq = reinterpret_cast<bf16_t*>(p.dq); k.dk = reinterpret_cast<bf16_t*>(p.dk);
     k.dv_out = reinterpret_cast<bf16_t*>(p.dv_out); k.dbeta = p.dbeta; k.dg = p.dg;
     k.graw = reinterpret_cast<const bf16_t*>(p.graw); k.gA = p.gA; k.gbias = p.gbias; k.gthr = p.gthr; k.gband = p.gband;
@@ -1526,7 +1526,7 @@ extern "C" int lnx_chunk_bwd(const lnx_scan_args* a, void* stream) {
   p.geom.tab = packed ? reinterpret_cast<const int32_t*>(reinterpret_cast<char*>(a->workspace) + w.tab) : nullptr;
   p.q = a->q; p.k = a->k; p.v = a->v; p.beta = a->beta; p.d_o = a->d_o; p.d_sT = a->d_final_state;
   p.dq = a->d_q; p.dk = a->d_k; p.dv_out = a->d_v; p.dbeta = a->d_beta; p.dg = a->d_g; p.ds0 = a->d_initial_state;
-  p.dv = a->dv; p.gate = a->gate; p.scale = a->scale; p.slab = a->test_scan_slab;
+  p.dv = a->dv; p.gate = a->gate; p.l2norm = a->use_qk_l2norm; p.scale = a->scale; p.slab = a->test_scan_slab;
   const bool raw_gate = a->gate == LNX_GATE_VECTOR && a->gate_raw != nullptr;
   p.graw = raw_gate ? a->gate_raw : nullptr; p.gA = a->gate_A_log; p.gbias = a->gate_bias; p.gthr = a->gate_threshold;
   p.gband = a->gate_threshold + log1pf(expf(-a->gate_threshold)) != a->gate_threshold;

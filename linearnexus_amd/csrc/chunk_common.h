@@ -161,10 +161,12 @@ inline ChunkWs lnx_chunk_ws_layout(const lnx_scan_args* a) {
     w.total = off;
     return w;
   }
-  w.Tm = w.Nq = w.Nk = w.Fq = 0;
+  const bool kda = lnx_chunk_kda(a);
+  w.Tm = w.Fq = 0;
+  w.Nq = take(bwd && kda ? slots * C * 4 : 0);  // of the rows that the op normalises, as above
+  w.Nk = take(bwd && kda ? slots * C * 4 : 0);
   w.G = take(vec ? slots * C * dk * 4 : slots * C * 4);
   w.P = take(slots * C * C * es);
-  const bool kda = lnx_chunk_kda(a);
   w.X = take(vec && saved && !kda ? slots * C * C * es : 0);
   w.W = take(slots * C * dk * es);
   w.U = take(slots * C * dv * es);

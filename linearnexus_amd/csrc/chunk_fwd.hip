@@ -38,7 +38,7 @@ struct FwdParams {
   int save;  // write the per-chunk tensors the backward pass (or the separate output kernel) reads
   int out_spw;  // chunk_output: value slabs per workgroup
   int vcols;    // leading value columns present in v (its row length); the rest of the dv columns are zero
-  int l2norm;   // chunk_prepare2<LITE>: q and k rows are normalised as x / (|x| + 1e-6) inside the kernels
+  int l2norm;   // chunk_prepare2<LITE>, kda_prepare: q and k rows are normalised as x / (|x| + 1e-6) inside the kernels
   int slab;     // lnx_scan_args.test_scan_slab
   // per-channel gate formed inside kda_prepare from the raw projection (lnx_scan_args.gate_raw): element type of q
   const void* graw;
@@ -433,8 +433,9 @@ template <typename T, int DK> struct KdaPrepSmem {
   static constexpr int LDC = LNX_C + PAD, LDF = 64 + 4;
   static constexpr int kTile = 64 * LDC;
   // K half (later Tm), Q half (later Tm diag(beta)); gate half (later the staged slab); A (later the
-  // output staging); the P accumulator / inverse; inverse scratch; beta
-  static constexpr size_t bytes = sizeof(T) * 2 * kTile + sizeof(float) * (64 * LDF + 2 * 64 * LNX_LDA + 32 * 36 + 64);
+  // output staging); the P accumulator / inverse; inverse scratch; beta, and where the rows are normalised inside their factors
+  static constexpr bool NORM = sizeof(T) == 2 && DK <= 128;
+  static constexpr size_t bytes = sizeof(T) * 2 * kTile + sizeof(float) * (64 * LDF + 2 * 64 * LNX_LDA + 32 * 36 + (NORM ? 192 : 64));
 };
 
 // GRAW: the gate arrives as the block's raw projection and is activated here, g = -exp(A_log[h]) softplus(raw + bias)
@@ -451,6 +452,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   float* sT = sA + 64 * LNX_LDA;
   float* sX = sT + 64 * LNX_LDA;
   float* sBeta = sX + 32 * 36;
+  float* sNk = sBeta + 64;  // NORM: 1 / (|x| + eps) of the k and q rows
+  float* sNq = sNk + 64;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int N = p.geom.N;
@@ -506,6 +509,53 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   };
   fetch_half(0);
   if (tid < 64) sBeta[tid] = (tid < len) ? p.beta[tbase + (int64_t)tid * p.geom.ts] : 0.f;
+  // The op's normalisation of q and k inside (kda.py:379-381): the second half is read once more for the row norms, the rows are rounded to
+  // T behind it as the stand-alone kernel rounds them, and the factors stay for the backward pass.  Normalised copies of q and k and a pass
+  // over their gradients took 84 + 133 us of 2150 at B4 H16 T8192 d128.
+  const bool norm = L::NORM && p.l2norm;
+  if constexpr (L::NORM) {
+    if (norm) {
+      float k2[GT::IT], q2[GT::IT];
+#pragma unroll
+      for (int it = 0; it < GT::IT; ++it) k2[it] = q2[it] = 0.f;
+      auto squares = [&](const GT& a, const GT& b) {
+#pragma unroll
+        for (int it = 0; it < GT::IT; ++it)
+#pragma unroll
+          for (int e = 0; e < GT::N; ++e) k2[it] += to_f32(a.x[it][e]) * to_f32(a.x[it][e]), q2[it] += to_f32(b.x[it][e]) * to_f32(b.x[it][e]);
+      };
+      if constexpr (NH == 2) {
+        GT k1, q1;
+        k1.load(kg + 64, tsk, len, tid);
+        q1.load(qg + 64, tsk, len, tid);
+        squares(rK, rQ);
+        squares(k1, q1);
+      } else {
+        squares(rK, rQ);
+      }
+      static_assert(GT::VPR == 8, "eight threads per row");
+#pragma unroll
+      for (int it = 0; it < GT::IT; ++it) {
+        k2[it] = quad_sum(k2[it]), q2[it] = quad_sum(q2[it]);
+        k2[it] += __shfl_xor(k2[it], 4, LNX_WAVE), q2[it] += __shfl_xor(q2[it], 4, LNX_WAVE);
+        if ((tid & 7) == 0) {
+          const int r = (tid + 256 * it) / 8;
+          const float fk = 1.f / (sqrtf(k2[it]) + LNX_L2_EPS), fq = 1.f / (sqrtf(q2[it]) + LNX_L2_EPS);
+          sNk[r] = fk, sNq[r] = fq;
+          if (p.save) {
+            ws_ptr<float>(p, p.off.Nk)[slot * 64 + r] = fk;
+            ws_ptr<float>(p, p.off.Nq)[slot * 64 + r] = fq;
+          }
+        }
+      }
+    }
+  }
+  auto scale_rows = [&](GT& a, const float* f) {
+#pragma unroll
+    for (int it = 0; it < GT::IT; ++it)
+#pragma unroll
+      for (int e = 0; e < GT::N; ++e) a.x[it][e] = from_f32<T>(to_f32(a.x[it][e]) * f[(tid + 256 * it) / GT::VPR]);
+  };
   floatx4 acc[3];  // this wave's three below-diagonal tasks (block, product), summed over the halves
 #pragma unroll
   for (int u = 0; u < 3; ++u) acc[u] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -525,7 +575,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
 
 #pragma unroll 1
   for (int h = 0; h < NH; ++h) {
-    lds_barrier();  // the previous half's tiles are dead
+    lds_barrier();  // the previous half's tiles are dead (and the row factors are there)
+    if (norm) scale_rows(rK, sNk), scale_rows(rQ, sNq);
     rK.store(sK, LDC, tid);
     rQ.store(sQ, LDC, tid);
     store_gate(h);
@@ -729,6 +780,10 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       for (int it = 0; it < Slab::IT; ++it) {
         const int idx = tid + 256 * it, r = idx / Slab::VPR, c = (idx - r * Slab::VPR) * VN;
         typename Vec16<T>::V x = rIn.x[it];
+        if (norm) {
+#pragma unroll
+          for (int e = 0; e < VN; ++e) x[e] = from_f32<T>(to_f32(x[e]) * sNk[r]);
+        }
 #pragma unroll
         for (int e = 0; e < VN; ++e) x[e] = from_f32<T>(to_f32(x[e]) * sBeta[r] * __expf(rGs[it][e / 4][e % 4]));
         *reinterpret_cast<typename Vec16<T>::V*>(sIn + r * LDC + c) = x;
@@ -1461,8 +1516,8 @@ int lnx_chunk_check(const lnx_scan_args* a, bool backward) {
   if (a->chunk != LNX_C) return lnx_set_error(LNX_ERR_SHAPE, "chunk length must be %d, got %d", LNX_C, a->chunk);
   if (a->dtype != LNX_F32 && a->dtype != LNX_BF16) return lnx_set_error(LNX_ERR_DTYPE, "dtype %d", a->dtype);
   if (a->o_dtype != LNX_F32 && a->o_dtype != LNX_BF16) return lnx_set_error(LNX_ERR_DTYPE, "o_dtype %d", a->o_dtype);
-  if (a->use_qk_l2norm && !lnx_chunk_direct(a))
-    return lnx_set_error(LNX_ERR_SHAPE, "use_qk_l2norm inside the chunk kernels needs 2-byte inputs and no per-channel gate; "
+  if (a->use_qk_l2norm && !lnx_chunk_normalises_qk(a))
+    return lnx_set_error(LNX_ERR_SHAPE, "use_qk_l2norm inside the chunk kernels needs 2-byte inputs, and dk <= 128 with a per-channel gate; "
                                         "normalise with lnx_l2norm_fwd first");
   if (a->token_first != 0 && a->token_first != 1) return lnx_set_error(LNX_ERR_SHAPE, "token_first must be 0 or 1");
   if ((a->test_scan_slab != 0 && a->test_scan_slab != 32 && a->test_scan_slab != 64) || a->test_out_slabs < 0)
@@ -1694,6 +1749,8 @@ extern "C" uint64_t lnx_chunk_workspace_bytes(const lnx_scan_args* a) {
     return 0;
   return lnx_chunk_ws_layout(a).total;
 }
+
+extern "C" int lnx_chunk_normalises_qk(const lnx_scan_args* a) { return a && (lnx_chunk_direct(a) || lnx_chunk_kda(a)) ? 1 : 0; }
 
 extern "C" int lnx_chunk_fuses_l2norm(const lnx_scan_args* a) { return a && lnx_chunk_direct(a) ? 1 : 0; }
 

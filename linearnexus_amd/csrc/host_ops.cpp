@@ -457,7 +457,7 @@ std::pair<Tensor, Tensor> chunk_forward(const Tensor& q, const Tensor& k, const 
   // The reference's chunk path normalises in the input dtype before anything else (gated_deltanet.py:273-275,
   // kda.py:379-381).  Where the kernels scale the rows themselves (no normalised copies, gradients carried through the
   // normalisation inside lnx_chunk_bwd) they get the raw q and k; otherwise the rows are normalised first.
-  const bool fused = opt_.l2norm && lnx_chunk_fuses_l2norm(&a);
+  const bool fused = opt_.l2norm && lnx_chunk_normalises_qk(&a);
   a.use_qk_l2norm = fused;
   c.norm_outside = opt_.l2norm && !fused;
   if (c.norm_outside) std::tie(c.qn, c.kn) = l2norm_pair_fwd(c.q_in, c.k_in);
@@ -553,7 +553,7 @@ std::pair<Tensor, Tensor> chunk_segmented(const Tensor& q0, const Tensor& k0, co
   const Tensor o = empty_layout(1, rows, s.T, s.dv, q.options().dtype(type_of(o_dtype)), tf);
   const Tensor sT = at::empty({s.B, s.H, s.dk, s.dv}, q.options().dtype(at::kFloat));
   lnx_scan_args a = base_args(1, rows, s.T, s.dk, s.dv, code_of(q.scalar_type()), (int)o_dtype, s.gate, false, scale);
-  a.use_qk_l2norm = l2norm && lnx_chunk_fuses_l2norm(&a);
+  a.use_qk_l2norm = l2norm && lnx_chunk_normalises_qk(&a);
   if (l2norm && !a.use_qk_l2norm) std::tie(q, k) = l2norm_pair_fwd(q, k);
   a.token_first = tf, a.forward_only = 1;
   a.q = ptr(q), a.k = ptr(k), a.v = ptr(v), a.beta = fptr(beta), a.g = fptr(g);
