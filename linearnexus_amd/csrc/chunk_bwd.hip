@@ -825,7 +825,7 @@ __global__ __launch_bounds__(256, GATE == LNX_GATE_VECTOR && sizeof(T) == 4 ? 1 
     float pr[16], pc[16];
     const int pch = 16 * wave + (lane & 15), ptok = 4 * (lane >> 4);  // this lane's channel; its tokens are 16 t + ptok + e
     if constexpr (sizeof(T) == 2) {
-      pair_levels<false>(pr, pc, sR, sAl, LDF, sKr, LDC, sQr, LDC, tid);
+      pair_levels(pr, pc, sR, sAl, LDF, sKr, LDC, sQr, LDC, tid);
 #pragma unroll
       for (int x = 0; x < 16; ++x) sOut[(16 * (x >> 2) + ptok + (x & 3)) * LDF + pch] += p.scale * pr[x];
     } else {
@@ -973,11 +973,7 @@ template <typename T, int DK, int GATE> struct Wy2Cfg {
   // for the epilogue (other gates with dk = 256; with dk <= 128 K is read again instead, so that two workgroups fit a CU)
   static constexpr bool KEEP_K = GATE != LNX_GATE_VECTOR && DK > 128;
   static constexpr int ntile = (GATE == LNX_GATE_VECTOR) ? 5 : KEEP_K ? 4 + (DK / 64 - 1) : 4;
-  // vector gate, 2-byte inputs, dk = 128: the second half's dBw fragments wait in LDS while the first half's pair sums
-  // run (one value per thread and fragment element; in registers they went to scratch memory)
-  static constexpr bool STASH = GATE == LNX_GATE_VECTOR && sizeof(T) == 2 && DK == 128;
-  static constexpr size_t stash_off = sizeof(T) * ntile * kTile + sizeof(float) * nfloat;
-  static constexpr size_t bytes = stash_off + (STASH ? sizeof(float) * 16 * 256 : 0);
+  static constexpr size_t bytes = sizeof(T) * ntile * kTile + sizeof(float) * nfloat;
 };
 
 // GRAW (per-channel gate only): the gate was activated inside the op from the raw projection; dg goes on through the
@@ -1140,11 +1136,6 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && (GATE == LNX_GATE_VECTOR || 
       const int i = 32 * wi + frag_row(e, lane), j = 32 * wj + frag_col(lane);
       sR[i * LNX_LDA + j] = (i > j) ? -aM[0][0][e] : 0.f;  // dA
     }
-    float* sStash = reinterpret_cast<float*>(smem + L::stash_off);
-    if constexpr (L::STASH) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) sStash[e * 256 + tid] = aBw[NKS - 1][0][0][e];
-    }
     lds_barrier();
     {  // dbeta += sum_j dA_ij X_ij, then dX = beta_i dA_ij in place; thread = (row, quarter of the columns)
       const int r = tid >> 2, j0 = (tid & 3) * 16;
@@ -1186,23 +1177,15 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && (GATE == LNX_GATE_VECTOR || 
         store4(sGc + r * LDF + c, up[it]);
       }
       lds_barrier();
-      if (L::STASH && h == NKS - 1) {  // out = e^G dBw
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int r = 32 * wi + frag_row(e, lane), c = 32 * wj + frag_col(lane);
-          sOut[r * LDF + c] = sStash[e * 256 + tid] * __expf(sGc[r * LDF + c]);
-        }
-      } else {
+      for (int u = 0; u < NKS; ++u)
+        if (u == h) {  // out = e^G dBw
 #pragma unroll
-        for (int u = 0; u < NKS; ++u)
-          if (u == h) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-              const int r = 32 * wi + frag_row(e, lane), c = 32 * wj + frag_col(lane);
-              sOut[r * LDF + c] = aBw[u][0][0][e] * __expf(sGc[r * LDF + c]);
-            }
+          for (int e = 0; e < 16; ++e) {
+            const int r = 32 * wi + frag_row(e, lane), c = 32 * wj + frag_col(lane);
+            sOut[r * LDF + c] = aBw[u][0][0][e] * __expf(sGc[r * LDF + c]);
           }
-      }
+        }
       lds_barrier();
       {  // dbeta += <e^G dBw, k>;  out = beta e^G dBw; thread = (row, quarter of the channels)
         const int r = tid >> 2, q0 = (tid & 3) * 16;
@@ -1219,30 +1202,17 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && (GATE == LNX_GATE_VECTOR || 
         if ((tid & 3) == 0) sdB[r] += t;
       }
       lds_barrier();
-      float pr[16], pc[16];
-      const int pch = 16 * wave + (lane & 15), ptok = 4 * (lane >> 4);  // this lane's channel; its tokens are 16 t + ptok + e
-      constexpr bool LEVELS = DK <= 128;  // beyond that the live accumulators leave too few registers for it
-      if constexpr (sizeof(T) == 2 && LEVELS) {  // both pair sums of dA together on the bf16 MFMA
-        pair_levels<true>(pr, pc, sR, sGc, LDF, sKr, LDC, sKr, LDC, tid);
-#pragma unroll
-        for (int x = 0; x < 16; ++x) sOut[(16 * (x >> 2) + ptok + (x & 3)) * LDF + pch] += pr[x];
-      } else {
-        pair_row<T, 64, true>(sOut, sR, sGc, LDF, sKr, LDC, 1.f, tid);
-      }
+      // (pair_levels needs more registers than the live accumulators of dk = 256 leave, and dk <= 128 in bf16 is chunk_kda.hip's)
+      pair_row<T, 64, true>(sOut, sR, sGc, LDF, sKr, LDC, 1.f, tid);
       lds_barrier();
 #pragma unroll
       for (int it = 0; it < 4; ++it) {  // row-type part to registers, out restarts from zero
         const int idx = tid + 256 * it, r = idx >> 4, c = (idx & 15) * 4;
         up[it] = load4(sOut + r * LDF + c);
-        if (!(sizeof(T) == 2 && LEVELS)) store4(sOut + r * LDF + c, floatx4{0.f, 0.f, 0.f, 0.f});
+        store4(sOut + r * LDF + c, floatx4{0.f, 0.f, 0.f, 0.f});
       }
       lds_barrier();
-      if constexpr (sizeof(T) == 2 && LEVELS) {
-#pragma unroll
-        for (int x = 0; x < 16; ++x) sOut[(16 * (x >> 2) + ptok + (x & 3)) * LDF + pch] = pc[x];
-      } else {
-        pair_col<T, 64, true>(sOut, sR, sGc, LDF, sKr, LDC, 1.f, tid);
-      }
+      pair_col<T, 64, true>(sOut, sR, sGc, LDF, sKr, LDC, 1.f, tid);
       lds_barrier();
 #pragma unroll
       for (int it = 0; it < 4; ++it) {

@@ -410,7 +410,7 @@ __device__ __forceinline__ void pair_col(float* out, const float* M, const float
 // blocks for h = 4, 2, 1.  Wave w owns channels 16 w .. 16 w + 15; lane (c = lane % 16, kq = lane / 16) holds the
 // sixteen tokens 16 t + 4 kq + e (t, e = 0..3) of its channel, which is at once the k-slot order of the scaled B
 // operands of v_mfma_f32_16x16x16_bf16 and the accumulator rows of its results, so factors, operands and results
-// never leave the lane.  Not STRICT: the diagonal X[i][i] (E = 1) is added to both sums.
+// never leave the lane.  The diagonal X[i][i] (E = 1) is added to both sums.
 // X [64][LNX_LDA] fp32, G [64][ldf] fp32, b / a [64][ld] bf16, all in LDS; results are per lane, index 4 t + e.
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ floatx4 mfma16_bf16(bf16x4 a, bf16x4 b, floatx4 c) {
@@ -527,7 +527,6 @@ __device__ __forceinline__ void pair_diag(floatx4& ro, floatx4& co, const floatx
   }
 }
 
-template <bool STRICT>
 __device__ __forceinline__ void pair_levels(float (&ro)[16], float (&co)[16], const float* __restrict__ X,
                                             const float* __restrict__ G, int ldf, const bf16_t* __restrict__ b, int ldb,
                                             const bf16_t* __restrict__ a, int lda, int tid) {
@@ -542,7 +541,7 @@ __device__ __forceinline__ void pair_levels(float (&ro)[16], float (&co)[16], co
       g[x] = 1.4426950408889634f * G[tok * ldf + c];
       bv[x] = (float)b[tok * ldb + c];
       av[x] = (float)a[tok * lda + c];
-      const float d = STRICT ? 0.f : X[tok * LNX_LDA + tok];
+      const float d = X[tok * LNX_LDA + tok];
       ro[x] = d * bv[x];
       co[x] = d * av[x];
     }

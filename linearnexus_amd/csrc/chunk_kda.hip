@@ -11,12 +11,15 @@
 // the adjoint of linearnexus/modules/linear_attn/kda.py:569-648 in the form of chunk_direct.hip: neither dW = -dD S^T nor W, U and the
 // forward pass's X are needed, nor partial sums of dk and dG in memory between two kernels.
 //
-// One workgroup per chunk, four waves per 64 channels.  A loop over 32-column slabs of the value dimension (LDS-direct loads, NBUF slabs
-// in flight) forms dR and accumulates what contracts over value columns on 16x16x32 products: wave w of a team owns the 16 channels
-// 16 w .. of its 64 and all tokens, so that an accumulator element is at the place where pair_levels wants its channel and token:
+// One workgroup of four waves per chunk, two of them per CU: what one loads, the other covers with the pair sums, which take about as
+// long on the VALU as the loads on the memory path.  A loop over 32-column slabs of the value dimension (LDS-direct loads, two slabs in
+// flight) forms dR and accumulates what contracts over value columns on 16x16x32 products: wave w owns the channels 64 s + 16 w .. of every
+// set s of 64 and all tokens, so that an accumulator element is at the place where pair_levels wants its channel and token:
 // lane (c = lane % 16, kq = lane / 16) holds the tokens 16 t + 4 kq + e of channel c, and everything between the loop and the
 // tiles on their way out happens in registers.  The four pair sums share their factors (pair_sums).
-//@@MEASURED@@
+// Measured at B4 H16 T8192 d128 (8192 chunks): 560 us for 280 KB a chunk, 4.1 TB/s; bwd_dqk and bwd_wy2, which passed dW, a partial dk and an
+// fp32 partial gradient of the gate through memory, 402 + 497 us behind and before 217 us of normalisation outside.  With eight waves and one
+// workgroup per CU 650 us: of 20.6 us a chunk 8.5 were pair sums with nothing in flight.
 
 #include "chunk_common.h"
 #include "reduce_rows.h"
@@ -27,35 +30,47 @@ using T = bf16_t;
 typedef Mma16 S16;
 typedef S16::Frag Frag;
 template <typename X> __device__ __forceinline__ X* at(char* ws, uint64_t off) { return reinterpret_cast<X*>(ws + off); }
-constexpr float LOG2E = 1.4426950408889634f;
-constexpr int LDX = LNX_C + 8, LDF = 64 + 4;  // bf16 and fp32 [64][64] tiles
+constexpr int LDX = LNX_C + 8;  // dPm, dXa: bf16 [64][64] tiles
 
-// The four tokens 16 t + 4 kq + e of column c0 + l16 of a bf16 [64][LDX] tile: one transposing read
-__device__ __forceinline__ bf16x4 column4(const T* tile, int t, int c0, int lane) { return S16::rows4(tile, LDX, 16 * t + 4 * (lane >> 4), c0, lane); }
 // A operands of the 16x16x16 products from such a tile: block (ti, t), lane = (row l16, k-slots 4 kq + e); transposed: (column l16, rows)
 __device__ __forceinline__ bf16x4 block_rows(const T* X, int ti, int t, int lane) {
   return *reinterpret_cast<const bf16x4*>(X + (16 * ti + (lane & 15)) * LDX + 16 * t + 4 * (lane >> 4));
 }
-__device__ __forceinline__ bf16x4 block_cols(const T* X, int ti, int t, int lane) { return column4(X, ti, 16 * t, lane); }
+__device__ __forceinline__ bf16x4 block_cols(const T* X, int ti, int t, int lane) { return S16::rows4(X, LDX, 16 * ti + 4 * (lane >> 4), 16 * t, lane); }
 
 // pair_levels (chunk_common.h) for two matrices at once.  Per level every token has one factor, and P and A share it and the column
 // tokens' operand F k:
 //   rp[i] += sum_{j < i} P_ij E_ij k_j     ra[i] += sum_{j < i} A_ij E_ij k_j     co[j] += sum_{i > j} E_ij (P_ij q_i + A_ij (beta k)_i)
-// Lane, index 4 t + e and levels as there; g = G log2(e).  P and A: bf16 [64][LDX].
+// Lane, index 4 t + e and levels as there; g = G, whose reference tokens are values of the other lane groups of the channel.
+// P and A: bf16 [64][LDX].
+// the value of lane group 0, and of group 2, in every group; of the odd group of a pair, in both
+__device__ __forceinline__ float of_group0(float x) {
+  const unsigned u = __float_as_uint(x), v = __builtin_amdgcn_permlane32_swap(u, u, false, false)[0];
+  return __uint_as_float(__builtin_amdgcn_permlane16_swap(v, v, false, false)[0]);
+}
+__device__ __forceinline__ float of_group2(float x) {
+  const unsigned u = __float_as_uint(x), v = __builtin_amdgcn_permlane32_swap(u, u, false, false)[1];
+  return __uint_as_float(__builtin_amdgcn_permlane16_swap(v, v, false, false)[0]);
+}
+__device__ __forceinline__ float of_odd_group(float x) {
+  const unsigned u = __float_as_uint(x);
+  return __uint_as_float(__builtin_amdgcn_permlane16_swap(u, u, false, false)[1]);
+}
+// Everything these depend on is computed here: arithmetic may pass a scheduling barrier, loads may not, and what had been loaded for sums
+// that were put off went to scratch memory.
+__device__ __forceinline__ void settle16(float (&x)[16]) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(x[i]));
+}
 struct PairSums {
   float rp[16], ra[16], co[16];
-  // Everything so far is computed here: arithmetic may pass a scheduling barrier, loads may not, and what had been loaded for sums that were
-  // put off went to scratch memory.
-  __device__ __forceinline__ void settle() {
-#pragma unroll
-    for (int x = 0; x < 16; ++x) asm volatile("" : "+v"(rp[x]), "+v"(ra[x]), "+v"(co[x]));
-  }
+  __device__ __forceinline__ void settle() { settle16(rp), settle16(ra), settle16(co); }
 };
 template <int H>
 __device__ __forceinline__ void sums_cross(PairSums& s, const float (&g)[16], const float (&dec)[16], const bf16x4 (&k4)[4], const bf16x4 (&q4)[4],
-                                           const float* __restrict__ beta, const T* __restrict__ P, const T* __restrict__ A, const float* __restrict__ G, int c, int lane_) {
+                                           const float* __restrict__ beta, const T* __restrict__ P, const T* __restrict__ A, int lane_) {
   const int lane = fresh(lane_);  // the matrices' blocks are read where they are used
-  const float m0 = LOG2E * G[H * LDF + c], m1 = H == 32 ? m0 : LOG2E * G[48 * LDF + c];
+  const float m0 = of_group0(g[H / 4]), m1 = H == 32 ? m0 : of_group0(g[12]);  // G of token H, and of token 48
   float F[16];
   bf16x4 B[4], Bk[4];  // a column block's F k; a row block's F q and F beta k
 #pragma unroll
@@ -64,11 +79,11 @@ __device__ __forceinline__ void sums_cross(PairSums& s, const float (&g)[16], co
     const float ref = (H == 32 || t < 2) ? m0 : m1;
     // one exponential per four tokens, the others by the single-step decays: away from the reference the factors shrink
     if (up) {
-      F[4 * t] = __builtin_amdgcn_exp2f(fminf(g[4 * t] - ref, 0.f));
+      F[4 * t] = __expf(fminf(g[4 * t] - ref, 0.f));
 #pragma unroll
       for (int e = 1; e < 4; ++e) F[4 * t + e] = F[4 * t + e - 1] * dec[4 * t + e];
     } else {
-      F[4 * t + 3] = __builtin_amdgcn_exp2f(fminf(ref - g[4 * t + 3], 0.f));
+      F[4 * t + 3] = __expf(fminf(ref - g[4 * t + 3], 0.f));
 #pragma unroll
       for (int e = 2; e >= 0; --e) F[4 * t + e] = F[4 * t + e + 1] * dec[4 * t + e + 1];
     }
@@ -114,7 +129,7 @@ __device__ __forceinline__ void sums_cross(PairSums& s, const float (&g)[16], co
 
 // Levels 8, 4, 2, 1 of the diagonal 16x16 block t
 __device__ __forceinline__ void sums_diag(PairSums& s, const float (&g)[16], const float (&dec)[16], const bf16x4 (&kb)[4], const bf16x4 (&qb)[4],
-                                          const float* __restrict__ beta, const T* __restrict__ P, const T* __restrict__ A, const float* __restrict__ G, int c, int t, int lane_) {
+                                          const float* __restrict__ beta, const T* __restrict__ P, const T* __restrict__ A, int t, int lane_) {
   const int lane = fresh(lane_);
   typedef unsigned uint2_ __attribute__((ext_vector_type(2)));
   const int l16 = lane & 15, kq = lane >> 4;
@@ -129,8 +144,8 @@ __device__ __forceinline__ void sums_diag(PairSums& s, const float (&g)[16], con
     floatx4 fu, fl;  // the factor of each token in its role at this level (row token: fu, column token: fl), 0 in the other
     if (H >= 4) {  // all four tokens share the role and the reference: one exponential, the rest by the single-step decays
       const bool up = H == 8 ? (kq & 2) != 0 : (kq & 1) != 0;
-      const float ref = LOG2E * G[(16 * t + (H == 8 ? 8 : 8 * (kq >> 1) + 4)) * LDF + c];
-      const float f = __builtin_amdgcn_exp2f(fminf(up ? g[4 * t] - ref : ref - g[4 * t + 3], 0.f));
+      const float ref = H == 8 ? of_group2(g[4 * t]) : of_odd_group(g[4 * t]);  // G of token 16 t + 8, or of the half block's fifth
+      const float f = __expf(fminf(up ? g[4 * t] - ref : ref - g[4 * t + 3], 0.f));
       floatx4 F;
       F[0] = up ? f : f * d3 * d2 * d1;
       F[1] = up ? f * d1 : f * d3 * d2;
@@ -166,60 +181,67 @@ __device__ __forceinline__ void sums_diag(PairSums& s, const float (&g)[16], con
 
 // Adds to what s holds; the diagonal's part of P (E = 1) is the caller's.
 __device__ __forceinline__ void pair_sums(PairSums& s, const float (&g)[16], const bf16x4 (&k4)[4], const bf16x4 (&q4)[4], const float* __restrict__ beta,
-                                          const T* __restrict__ P, const T* __restrict__ A, const float* __restrict__ G, int c, int lane) {
+                                          const T* __restrict__ P, const T* __restrict__ A, int lane) {
   float dec[16];  // single-step decays exp(G_tok - G_{tok-1}) inside each group of four (the first entry of a group is unused)
 #pragma unroll
-  for (int x = 0; x < 16; ++x) dec[x] = (x & 3) ? __builtin_amdgcn_exp2f(fminf(g[x] - g[x - 1], 0.f)) : 1.f;
+  for (int x = 0; x < 16; ++x) dec[x] = (x & 3) ? __expf(fminf(g[x] - g[x - 1], 0.f)) : 1.f;
   // one part at a time: interleaving them multiplies the live factors
   s.settle();
-  sums_cross<32>(s, g, dec, k4, q4, beta, P, A, G, c, lane);
+  sums_cross<32>(s, g, dec, k4, q4, beta, P, A, lane);
   s.settle();
-  sums_cross<16>(s, g, dec, k4, q4, beta, P, A, G, c, lane);
+  sums_cross<16>(s, g, dec, k4, q4, beta, P, A, lane);
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     s.settle();
-    sums_diag(s, g, dec, k4, q4, beta, P, A, G, c, t, lane);
+    sums_diag(s, g, dec, k4, q4, beta, P, A, t, lane);
   }
   s.settle();
 }
 
+// One step of sixteen sums over sixteen lanes: of 2 M values a lane keeps M, adding what its partner sends
+template <int M> __device__ __forceinline__ void exchange(float (&v)[16], int l16) {
+  const bool hi = (l16 & M) != 0;
+#pragma unroll
+  for (int x = 0; x < M; ++x) {
+    const float lo = v[x], up = v[x + M];
+    v[x] = (hi ? up : lo) + __shfl_xor(hi ? lo : up, M, LNX_WAVE);
+  }
+}
+
 template <int DK> struct KdaL {
-  static constexpr int NT = DK / 64, THREADS = 256 * NT, NW = 4 * NT, SV = 32;  // teams of four waves
-  static constexpr int NBUF = NT == 2 ? 3 : 2;  // one workgroup per CU, or two
+  static constexpr int NS = DK / 64, SV = 32, NBUF = 2;  // sets of 64 channels
   typedef SwzTile<64, SV> TokT;         // dO, D, dD, V slabs, and dR
   typedef SwzTile<SV, DK, false> StT;   // S^T, dS'^T slabs, transposing reads only
+  typedef SwzTile<64, 64> TmT;          // Tm^T, read by rows
+  typedef SwzTile<64, DK> RowT;         // K and Q rows; dq and dk on their way out
   static constexpr int oD = TokT::BYTES, odD = 2 * oD, oV = 3 * oD, oS = 4 * oD, odS = oS + StT::BYTES, slab_bytes = odS + StT::BYTES;
-  static constexpr int tile = 64 * LDX * 2, ftile = 64 * LDF * 4;
-  static constexpr int odR = NBUF * slab_bytes, oTm = odR + TokT::BYTES;
-  static constexpr size_t loop_bytes = oTm + tile;
-  // epilogue: dPm, dXa | per team G (fp32), K, Q, dq and dk on their way out (then dg, fp32)
-  static constexpr int team_bytes = ftile + 4 * tile;
-  static constexpr size_t epi_bytes = 2 * tile + NT * team_bytes;
-  static_assert(ftile <= 2 * tile, "dg leaves over dq and dk");
-  static constexpr int nfloat = 64 * (6 + NW);
-  static constexpr size_t bytes = sizeof(float) * nfloat + (epi_bytes > loop_bytes ? epi_bytes : loop_bytes);
-  static_assert(bytes <= (NT == 2 ? 160 : 80) * 1024, "LDS");
+  static constexpr int odR = NBUF * slab_bytes, oTm = odR + TokT::BYTES, loop_bytes = oTm + TmT::BYTES;
+  // epilogue: K | Q (then dq | dk, then the gate's gradient) | dPm | dXa | diagonal of dPm, <dR, v>, factors of the normalisation [2], shares of
+  // m, <q, dq>, <k, dk> [3][set, wave]
+  static constexpr int tile = 64 * LDX * 2, oP = 2 * RowT::BYTES, oF = oP + 2 * tile, epi_bytes = oF + 4 * 64 * (4 + 12 * NS);
+  static constexpr int LDO = DK + 4;    // fp32 rows of the gate's gradient
+  static_assert(64 * LDO * 4 <= oF, "the gate's gradient leaves over the tiles");
+  static constexpr size_t bytes = sizeof(float) * 192 + (epi_bytes > loop_bytes ? epi_bytes : loop_bytes);
+  static_assert(bytes <= 80 * 1024, "two workgroups per CU");
 };
 
 template <int DK, bool GRAW>
-__global__ __launch_bounds__(KdaL<DK>::THREADS, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
+__global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
   typedef KdaL<DK> L;
-  constexpr int NT = L::NT, THREADS = L::THREADS, NW = L::NW, NBUF = L::NBUF, SV = L::SV;
+  constexpr int NS = L::NS, SV = L::SV;
   typedef typename L::TokT TokT;
   typedef typename L::StT StT;
+  typedef typename L::TmT TmT;
+  typedef typename L::RowT RowT;
   extern __shared__ __align__(16) char smem[];
   float* sBeta = reinterpret_cast<float*>(smem);
-  float* sDiag = sBeta + 64;      // scale dPm_tt
-  float* sRdv = sDiag + 64;       // [2] <dR_t, v_t> over the even and the odd slabs
-  float* sNq = sRdv + 128;        // normalisation factors of the q and k rows (1 when the inputs come normalised)
+  float* sNq = sBeta + 64;        // normalisation factors of the q and k rows
   float* sNk = sNq + 64;
-  float* sM = sNk + 64;           // [wave] the wave's share of m_t
-  char* region = smem + sizeof(float) * L::nfloat;
+  char* region = smem + sizeof(float) * 192;
   T* sdR = reinterpret_cast<T*>(region + L::odR);
   T* sTm = reinterpret_cast<T*>(region + L::oTm);  // Tm^T
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, kq = lane >> 4;
-  const int team = wave >> 2, w4 = wave & 3;
   const int N = p.geom.N;
   const int64_t slot = blockIdx.x;
   const int row = (int)(slot / N), n = (int)(slot % N);
@@ -232,7 +254,7 @@ __global__ __launch_bounds__(KdaL<DK>::THREADS, 2) void kda_bwd_chunk_kernel(Kda
   };
   if (len <= 0) {  // an unused slot of a packed batch: its partial sums are zero
     if constexpr (GRAW)
-      for (int c = tid; c < DK; c += THREADS) gate_part(0)[c] = gate_part(1)[c] = 0.f;
+      for (int c = tid; c < DK; c += 256) gate_part(0)[c] = gate_part(1)[c] = 0.f;
     return;
   }
   const int64_t tbase = tok_index(p.geom, row, tok0);
@@ -241,18 +263,21 @@ __global__ __launch_bounds__(KdaL<DK>::THREADS, 2) void kda_bwd_chunk_kernel(Kda
   float gna = 0.f;
   if constexpr (GRAW) gna = -__expf(p.gA[row % p.geom.H]);
 
-  if (tid < 64) {
-    sBeta[tid] = (tid < len) ? p.beta[tbase + tid * ts] : 0.f;
-    sRdv[tid] = sRdv[64 + tid] = 0.f;
-    sNq[tid] = p.l2norm ? at<const float>(p.ws, p.off.Nq)[slot * 64 + tid] : 1.f;
-    sNk[tid] = p.l2norm ? at<const float>(p.ws, p.off.Nk)[slot * 64 + tid] : 1.f;
-  }
-  if (NT == 1 || team == 0) stage_tile<T, 64, 64>(sTm, LDX, at<const T>(p.ws, p.off.TmT) + slot * 64 * 64, 64, 64, tid);
-  __builtin_amdgcn_s_waitcnt(0);  // the small loads are behind us: this wave's vmcnt now counts slab loads and the stores of dv
-
   // ---- the slab loads: one-KB instructions, PER_WAVE of them per wave and slab.  Token rows past the chunk's end fetch the chunk's last
-  // row instead of zeros: they only reach rows that are not stored and products with rows of q and k that are zero.
+  // row instead of zeros: they only reach rows that are not stored and products with rows of q and k that are zero.  The small loads go the
+  // same way ahead of them.
   const unsigned slab0 = lds_byte_addr(region);
+  if (wave == 0) dma4(p.beta + tbase + (int64_t)min(lane, len - 1) * ts, lds_byte_addr(sBeta));
+  if (p.l2norm) {
+    if (wave == 1) dma4(at<const float>(p.ws, p.off.Nq) + slot * 64 + lane, lds_byte_addr(sNq));
+    if (wave == 2) dma4(at<const float>(p.ws, p.off.Nk) + slot * 64 + lane, lds_byte_addr(sNk));
+  }
+#pragma unroll
+  for (int u = 0; u < TmT::NINSTR / 4; ++u) {
+    int r, c;
+    TmT::src(wave + 4 * u, lane, r, c);
+    dma16(at<const T>(p.ws, p.off.TmT) + slot * 64 * 64 + r * 64 + c, slab0 + L::oTm + 1024 * (wave + 4 * u));
+  }
   const T* gdO = p.d_o + tbase * p.dv;
   const T* gV = p.v + tbase * p.dv;
   const T* gD = at<const T>(p.ws, p.off.D) + slot * 64 * p.dv;
@@ -261,102 +286,98 @@ __global__ __launch_bounds__(KdaL<DK>::THREADS, 2) void kda_bwd_chunk_kernel(Kda
   const T* gdS = at<const T>(p.ws, p.off.dSn) + slot * p.dv * DK;
   auto issue = [&](int s) {
     const int v0 = SV * s;
-    const unsigned dst = slab0 + (s % NBUF) * L::slab_bytes;
+    const unsigned dst = slab0 + (s & 1) * L::slab_bytes;
     int r, c;
-    StT::src(wave, lane, r, c);
-    dma16(gS + (int64_t)(v0 + r) * DK + c, dst + L::oS + 1024 * wave);
-    dma16(gdS + (int64_t)(v0 + r) * DK + c, dst + L::odS + 1024 * wave);
-    TokT::src(w4, lane, r, c);
+#pragma unroll
+    for (int u = 0; u < StT::NINSTR / 4; ++u) {
+      StT::src(wave + 4 * u, lane, r, c);
+      dma16(gS + (int64_t)(v0 + r) * DK + c, dst + L::oS + 1024 * (wave + 4 * u));
+      dma16(gdS + (int64_t)(v0 + r) * DK + c, dst + L::odS + 1024 * (wave + 4 * u));
+    }
+    TokT::src(wave, lane, r, c);
     const int64_t rc = (int64_t)min(r, len - 1) * tsv + v0 + c, rw = (int64_t)r * p.dv + v0 + c;
-    if (NT == 1 || team == 0) {
-      dma16(gdO + rc, dst + 1024 * w4);
-      dma16(gD + rw, dst + L::oD + 1024 * w4);
-    }
-    if (NT == 1 || team == 1) {
-      dma16(gdD + rw, dst + L::odD + 1024 * w4);
-      dma16(gV + rc, dst + L::oV + 1024 * w4);
-    }
+    dma16(gdO + rc, dst + 1024 * wave);
+    dma16(gD + rw, dst + L::oD + 1024 * wave);
+    dma16(gdD + rw, dst + L::odD + 1024 * wave);
+    dma16(gV + rc, dst + L::oV + 1024 * wave);
   };
-  constexpr int PER_WAVE = NT == 1 ? 6 : 4;
-  static_assert(StT::NINSTR == NW && TokT::NINSTR == 4, "the same count for every wave");
+  constexpr int PER_WAVE = StT::NINSTR / 2 + 4;
+  static_assert(StT::NINSTR % 4 == 0 && TokT::NINSTR == 4 && TmT::NINSTR % 4 == 0, "the same count for every wave");
   const int nslab = p.dv / SV;  // two or more
-#pragma unroll
-  for (int s = 0; s < NBUF; ++s)
-    if (s < nslab) issue(s);
+  issue(0);
+  issue(1);
 
-  const int ch = 64 * team + 16 * w4;  // the wave's first channel
-  floatx4 aQ[4], aK1[4], aK2[4], aP[4], aA[4];  // dO S^T, dR S^T, D dS'^T: [token tile]; row tile w4 of dO D^T (team 0) and dR D^T (last team)
+  floatx4 aQ[NS][4], aK1[NS][4], aK2[NS][4], aP[4], aA[4];  // dO S^T, dR S^T, D dS'^T: [set][token tile]; row tile `wave` of dO D^T and dR D^T
 #pragma unroll
-  for (int i = 0; i < 4; ++i) aQ[i] = aK1[i] = aK2[i] = aP[i] = aA[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const bool has_p = team == 0, has_a = team == NT - 1;
-  float ss = 0.f, rdv = 0.f;
-  TileRegs<T, 64, 64> rK, rQ;  // the epilogue's tiles of this team's channels, requested during the last slab
-  TileRegs<float, 64, 64> rG;
-  const int tt = tid & 255;
+  for (int i = 0; i < 4; ++i) {
+    aP[i] = aA[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < NS; ++u) aQ[u][i] = aK1[u][i] = aK2[u][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  float ss[NS] = {}, rdv = 0.f;
 #pragma unroll 1
   for (int s = 0; s < nslab; ++s) {
-    // this slab has landed: all but this wave's loads of the slabs behind it, then every wave's
-    if (NBUF == 3 && s == 0 && nslab > 2) dma_wait<2 * PER_WAVE>();
-    else if (s + 1 < nslab) dma_wait<PER_WAVE>();
+    // this slab has landed: all but this wave's loads of the next one, then every wave's
+    if (s + 1 < nslab) dma_wait<PER_WAVE>();
     else dma_wait<0>();
-    lds_barrier();  // and every wave is done with the slab before, whose buffer takes the next one but one
-    if (NBUF == 3 && s > 0 && s + 2 < nslab) issue(s + 2);
-    if (s + 1 == nslab) {
-      rK.load(p.k + tbase * DK + 64 * team, tsk, len, tt);
-      rQ.load(p.q + tbase * DK + 64 * team, tsk, len, tt);
-      rG.load(at<const float>(p.ws, p.off.G) + slot * 64 * DK + 64 * team, DK, 64, tt);
-    }
-    const char* slab = region + (s % NBUF) * L::slab_bytes;
+    lds_barrier();
+    const char* slab = region + (s & 1) * L::slab_bytes;
     const T* tdO = reinterpret_cast<const T*>(slab);
     const T* tD = reinterpret_cast<const T*>(slab + L::oD);
     const T* tdD = reinterpret_cast<const T*>(slab + L::odD);
     const T* tV = reinterpret_cast<const T*>(slab + L::oV);
     const T* tS = reinterpret_cast<const T*>(slab + L::oS);
     const T* tdS = reinterpret_cast<const T*>(slab + L::odS);
-    // ---- dR = Tm^T dD, transposed products: lane = token 16 w4 + l16, four value columns; Tm^T is upper-triangular ----
+    // ---- dR = Tm^T dD, transposed products: lane = token 16 wave + l16, four value columns; Tm^T is upper-triangular ----
 #pragma unroll
-    for (int u = 0; u < 2 / NT; ++u) {
-      const int vt = NT == 1 ? u : team;
+    for (int vt = 0; vt < 2; ++vt) {
       floatx4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        if (k == 0 && w4 >= 2) continue;
+        if (k == 0 && wave >= 2) continue;
         const Frag fa = S16::join(__builtin_bit_cast(bf16x4, TokT::tr4(tdD, 32 * k + 8 * kq, 16 * vt, lane)),
                                   __builtin_bit_cast(bf16x4, TokT::tr4(tdD, 32 * k + 8 * kq + 4, 16 * vt, lane)));
-        S16::mma(x, fa, *reinterpret_cast<const Frag*>(sTm + (16 * w4 + l16) * LDX + 32 * k + 8 * kq));
+        S16::mma(x, fa, TmT::load(sTm, 16 * wave + l16, 32 * k + 8 * kq));
       }
-      store4(sdR + TokT::at(16 * w4 + l16, 16 * vt + 4 * kq), x);
+      store4(sdR + TokT::at(16 * wave + l16, 16 * vt + 4 * kq), x);
     }
     // ---- what does not need dR ----
-    Frag fD[4];
+    Frag fD[4], fS[NS], fdS[NS];
 #pragma unroll
     for (int i = 0; i < 4; ++i) fD[i] = TokT::load(tD, 16 * i + l16, 8 * kq);
-    const Frag fS = S16::join(__builtin_bit_cast(bf16x4, StT::tr4(tS, 8 * kq, ch, lane)), __builtin_bit_cast(bf16x4, StT::tr4(tS, 8 * kq + 4, ch, lane)));
-    const Frag fdS = S16::join(__builtin_bit_cast(bf16x4, StT::tr4(tdS, 8 * kq, ch, lane)), __builtin_bit_cast(bf16x4, StT::tr4(tdS, 8 * kq + 4, ch, lane)));
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      const int ch = 64 * u + 16 * wave;
+      fS[u] = S16::join(__builtin_bit_cast(bf16x4, StT::tr4(tS, 8 * kq, ch, lane)), __builtin_bit_cast(bf16x4, StT::tr4(tS, 8 * kq + 4, ch, lane)));
+      fdS[u] = S16::join(__builtin_bit_cast(bf16x4, StT::tr4(tdS, 8 * kq, ch, lane)), __builtin_bit_cast(bf16x4, StT::tr4(tdS, 8 * kq + 4, ch, lane)));
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const Frag f = TokT::load(tdO, 16 * i + l16, 8 * kq);
-      S16::mma(aQ[i], f, fS);
-      S16::mma(aK2[i], fD[i], fdS);
-      if (has_p && i == w4) {
+#pragma unroll
+      for (int u = 0; u < NS; ++u) S16::mma(aQ[u][i], f, fS[u]), S16::mma(aK2[u][i], fD[i], fdS[u]);
+      if (i == wave) {
 #pragma unroll
         for (int j = 0; j <= i; ++j) S16::mma(aP[j], f, fD[j]);
       }
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ss += (float)fS[e] * (float)fdS[e];  // <dS', S> of channel ch + l16
+    for (int u = 0; u < NS; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss[u] += (float)fS[u][e] * (float)fdS[u][e];  // <dS', S> of channel 64 u + 16 wave + l16
     lds_barrier();  // dR is there
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const Frag f = TokT::load(sdR, 16 * i + l16, 8 * kq);
-      S16::mma(aK1[i], f, fS);
-      if (has_a && i == w4) {
+#pragma unroll
+      for (int u = 0; u < NS; ++u) S16::mma(aK1[u][i], f, fS[u]);
+      if (i == wave) {
 #pragma unroll
         for (int j = 0; j <= i; ++j) S16::mma(aA[j], f, fD[j]);
       }
     }
-    if (NT == 1 || team == (s & 1)) {  // <dR_t, v_t> and dv = beta dR: thread = (token tt / 4, eight value columns); the teams take turns
-      const int t = tt >> 2, c0 = 8 * (tt & 3);
+    {  // <dR_t, v_t> and dv = beta dR: thread = (token tid / 4, eight value columns)
+      const int t = tid >> 2, c0 = 8 * (tid & 3);
       Frag x = TokT::load(sdR, t, c0);
       const Frag vv = TokT::load(tV, t, c0);
       const float bt = sBeta[t];
@@ -367,228 +388,235 @@ __global__ __launch_bounds__(KdaL<DK>::THREADS, 2) void kda_bwd_chunk_kernel(Kda
       }
       if (t < len) *reinterpret_cast<Frag*>(p.dv_out + tbase * p.dv + (int64_t)t * tsv + SV * s + c0) = x;
     }
-    if (NBUF == 2 && s + 2 < nslab) {  // this buffer takes the slab after the next, once every wave has read it
+    if (s + 2 < nslab) {  // this buffer takes the slab after the next, once every wave has read it
       lds_barrier();
       issue(s + 2);
     }
   }
-  rdv = quad_sum(rdv);
-  if ((lane & 3) == 0) sRdv[64 * team + (tt >> 2)] = rdv;
   lds_barrier();  // slab tiles are dead from here on
 
   // ---- epilogue ----
-  T* sP = reinterpret_cast<T*>(region);
+  T* sK = reinterpret_cast<T*>(region);
+  T* sQ = reinterpret_cast<T*>(region + RowT::BYTES);
+  T* sP = reinterpret_cast<T*>(region + L::oP);
   T* sA = sP + 64 * LDX;
-  char* mine = region + 2 * L::tile + team * L::team_bytes;
-  float* sG = reinterpret_cast<float*>(mine);
-  T* sK = reinterpret_cast<T*>(mine + L::ftile);
-  T* sQ = sK + 64 * LDX;
-  T* sdQ = sQ + 64 * LDX;
-  T* sdK = sdQ + 64 * LDX;
-  float* sOut = reinterpret_cast<float*>(sdQ);  // dg, once dq and dk have left
+  float* sDiag = reinterpret_cast<float*>(region + L::oF);  // scale dPm_tt
+  float* sRdv = sDiag + 64;
+  float* sC = sRdv + 64;   // [2] <q, dq> / |q|, <k, dk> / |k|
+  float* sM = sC + 128;    // [3][set, wave]
+#pragma unroll
+  for (int u = 0; u < RowT::NINSTR / 4; ++u) {
+    int r, c;
+    RowT::src(wave + 4 * u, lane, r, c);
+    r = min(r, len - 1);
+    dma16(p.k + (tbase + (int64_t)r * ts) * DK + c, slab0 + 1024 * (wave + 4 * u));
+    dma16(p.q + (tbase + (int64_t)r * ts) * DK + c, slab0 + RowT::BYTES + 1024 * (wave + 4 * u));
+  }
+  float G[NS][16];  // the cumulative gate of this lane's channels and tokens
+#pragma unroll
+  for (int u = 0; u < NS; ++u)
+#pragma unroll
+    for (int x = 0; x < 16; ++x)
+      G[u][x] = at<const float>(p.ws, p.off.G)[(slot * 64 + 16 * (x >> 2) + 4 * kq + (x & 3)) * DK + 64 * u + 16 * wave + l16];
+  rdv = quad_sum(rdv);
+  if ((tid & 3) == 0) sRdv[tid >> 2] = rdv;
+  if (!p.l2norm && tid < 64) sNq[tid] = sNk[tid] = 1.f;
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    if (j <= w4) {
+    if (j <= wave) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int i = 16 * w4 + 4 * kq + e, col = 16 * j + l16;
-        if (has_p) {
-          const float x = p.scale * aP[j][e];
-          sP[i * LDX + col] = (bf16_t)(i > col ? x : 0.f);
-          if (i == col) sDiag[i] = x;
-        }
-        if (has_a) sA[i * LDX + col] = (bf16_t)(i > col ? -aA[j][e] : 0.f);
+        const int i = 16 * wave + 4 * kq + e, col = 16 * j + l16;
+        const float x = p.scale * aP[j][e];
+        sP[i * LDX + col] = (bf16_t)(i > col ? x : 0.f);
+        sA[i * LDX + col] = (bf16_t)(i > col ? -aA[j][e] : 0.f);
+        if (i == col) sDiag[i] = x;
       }
     }
-  {
-    typedef TileRegs<T, 64, 64> RowTile;
-#pragma unroll
-    for (int it = 0; it < RowTile::IT; ++it) {
-      const int idx = tt + 256 * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
-      Frag x = rK.x[it], y = rQ.x[it];
-      if (p.l2norm) {
-        const float fk = sNk[r], fq = sNq[r];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = (bf16_t)((float)x[e] * fk), y[e] = (bf16_t)((float)y[e] * fq);
-      }
-      *reinterpret_cast<Frag*>(sK + r * LDX + c) = x;
-      *reinterpret_cast<Frag*>(sQ + r * LDX + c) = y;
-    }
-    rG.store(sG, LDF, tt);
-  }
+  dma_wait<0>();
   lds_barrier();
-  const int c = 16 * w4 + l16;  // this lane's channel of the team's 64
-  float dG[16];
-  {
-    float g[16], tot = 0.f;
-    bf16x4 k4[4], q4[4];
+  float dq[NS][16], dk[NS][16], dG[NS][16];
+  bf16x4 k4[NS][4], q4[NS][4];
+  // Sums over the wave's sixteen channels of a set; lane l16 ends with value l16
+  auto channel_sum = [&](float (&v)[16], int which, int u) {
+    exchange<8>(v, l16), exchange<4>(v, l16), exchange<2>(v, l16), exchange<1>(v, l16);
+    sM[64 * (4 * (NS * which + u) + wave) + 16 * (l16 >> 2) + 4 * kq + (l16 & 3)] = v[0];
+  };
+#pragma unroll
+  for (int u = 0; u < NS; ++u) {
+    const int lane = fresh(tid & 63), c0 = 64 * u + 16 * wave;
+    // K and Q at this lane's channel and tokens, normalised (rounded as the op rounds the normalised rows), zero past the chunk's end
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bf16x4 k = __builtin_bit_cast(bf16x4, RowT::tr4(sK, 16 * t + 4 * kq, c0, lane)), q = __builtin_bit_cast(bf16x4, RowT::tr4(sQ, 16 * t + 4 * kq, c0, lane));
+      const floatx4 fk = load4(sNk + 16 * t + 4 * kq), fq = load4(sNq + 16 * t + 4 * kq);
+      floatx4 kf, qf;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool on = 16 * t + 4 * kq + e < len;
+        kf[e] = on ? (float)k[e] * fk[e] : 0.f;
+        qf[e] = on ? (float)q[e] * fq[e] : 0.f;
+      }
+      k4[u][t] = pack_bf16x4(kf), q4[u][t] = pack_bf16x4(qf);
+    }
     PairSums s;
-    const float gC = LOG2E * sG[63 * LDF + c];
+    float tot = 0.f;
+    const float gC = __shfl(G[u][15], 48 + l16, LNX_WAVE);
     // what the loop left, and the diagonal of dPm; rp becomes dq, ra row, co dk without beta row
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      k4[t] = column4(sK, t, 16 * w4, lane), q4[t] = column4(sQ, t, 16 * w4, lane);
       const floatx4 d4 = load4(sDiag + 16 * t + 4 * kq);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int x = 4 * t + e;
-        g[x] = LOG2E * sG[(16 * t + 4 * kq + e) * LDF + c];
-        const float eg = __builtin_amdgcn_exp2f(g[x]), k2 = __builtin_amdgcn_exp2f(fminf(gC - g[x], 0.f)) * aK2[t][e], kv = (float)k4[t][e];
-        s.rp[x] = p.scale * eg * aQ[t][e] + d4[e] * kv;
-        s.ra[x] = -eg * aK1[t][e];
-        s.co[x] = k2 + d4[e] * (float)q4[t][e];
+        const float eg = __expf(G[u][x]), k2 = __expf(fminf(gC - G[u][x], 0.f)) * aK2[u][t][e], kv = (float)k4[u][t][e];
+        s.rp[x] = p.scale * eg * aQ[u][t][e] + d4[e] * kv;
+        s.ra[x] = -eg * aK1[u][t][e];
+        s.co[x] = k2 + d4[e] * (float)q4[u][t][e];
         tot += kv * k2;
       }
     }
-    pair_sums(s, g, k4, q4, sBeta, sP, sA, sG, c, lane);
+    pair_sums(s, G[u], k4[u], q4[u], sBeta, sP, sA, lane);
     float mv[16];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const floatx4 bt = load4(sBeta + 16 * t + 4 * kq);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int x = 4 * t + e, tok = 16 * t + 4 * kq + e;
-        const float kv = (float)k4[t][e], dk = bt[e] * s.ra[x] + s.co[x];
+        const int x = 4 * t + e;
+        const float kv = (float)k4[u][t][e];
         mv[x] = kv * s.ra[x];
-        dG[x] = (float)q4[t][e] * s.rp[x] - kv * dk + 2.f * bt[e] * mv[x];
-        sdQ[tok * LDX + c] = (bf16_t)s.rp[x];
-        sdK[tok * LDX + c] = (bf16_t)dk;
+        dq[u][x] = s.rp[x];
+        dk[u][x] = bt[e] * s.ra[x] + s.co[x];
+        dG[u][x] = (float)q4[u][t][e] * dq[u][x] - kv * dk[u][x] + 2.f * bt[e] * mv[x];
       }
     }
-    tot = xor32_sum(xor16_sum(tot + __builtin_amdgcn_exp2f(gC) * ss));  // over the tokens (ss: over its value columns) of this channel
-    if (kq == 3) dG[15] += tot;
-    // m_t over the wave's sixteen channels: sixteen values over sixteen lanes, halving the values with each exchange
+    channel_sum(mv, 0, u);
+    if (p.l2norm) {
 #pragma unroll
-    for (int m = 8; m >= 1; m >>= 1) {
-      const bool hi = (l16 & m) != 0;
+      for (int x = 0; x < 16; ++x) mv[x] = (float)q4[u][x >> 2][x & 3] * dq[u][x];
+      channel_sum(mv, 1, u);
 #pragma unroll
-      for (int x = 0; x < m; ++x) {
-        const float send = hi ? mv[x] : mv[x + m], keep = hi ? mv[x + m] : mv[x];
-        mv[x] = keep + __shfl_xor(send, m, LNX_WAVE);
-      }
+      for (int x = 0; x < 16; ++x) mv[x] = (float)k4[u][x >> 2][x & 3] * dk[u][x];
+      channel_sum(mv, 2, u);
     }
-    sM[64 * wave + 16 * (l16 >> 2) + 4 * kq + (l16 & 3)] = mv[0];  // lane l16 ends with value l16 = 4 t + e
-  }
-  // ---- dg: reverse cumulative sum over the chunk's tokens of this channel ----
-  {
+    tot = xor32_sum(xor16_sum(tot + __expf(gC) * ss[u]));  // over the tokens (ss: over its value columns) of this channel
+    if (kq == 3) dG[u][15] += tot;
+    // dg: reverse cumulative sum over the chunk's tokens of this channel
     float after = 0.f;  // what later blocks of sixteen tokens add
 #pragma unroll
     for (int t = 3; t >= 0; --t) {
 #pragma unroll
-      for (int e = 2; e >= 0; --e) dG[4 * t + e] += dG[4 * t + e + 1];
-      const float own = dG[4 * t];
-      const float y1 = __shfl_down(own, 16, LNX_WAVE), y2 = __shfl_down(own, 32, LNX_WAVE), y3 = __shfl_down(own, 48, LNX_WAVE);
-      float add = after;
-      if (kq < 3) add += y1;
-      if (kq < 2) add += y2;
-      if (kq < 1) add += y3;
+      for (int e = 2; e >= 0; --e) dG[u][4 * t + e] += dG[u][4 * t + e + 1];
+      // the four lane groups' totals on the VALU (xor16_sum in lnx_common.h): a group adds its odd neighbour's and the upper pair's
+      const unsigned own = __float_as_uint(dG[u][4 * t]);
+      const auto p16 = __builtin_amdgcn_permlane16_swap(own, own, false, false);
+      const unsigned pair = __float_as_uint(__uint_as_float(p16[0]) + __uint_as_float(p16[1]));
+      const auto p32 = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
+      const float add = after + ((kq & 1) ? 0.f : __uint_as_float(p16[1])) + ((kq & 2) ? 0.f : __uint_as_float(p32[1]));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dG[4 * t + e] += add;
-      after = __shfl(dG[4 * t], l16, LNX_WAVE);  // the block's first token holds the sum of everything from it on
+      for (int e = 0; e < 4; ++e) dG[u][4 * t + e] += add;
+      after += __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
+    }
+    // With the gate activated inside the op, g = -e^{A_log} softplus(x), x = raw + bias (kda.py:153-165), the gradient goes on to the raw
+    // projection as bwd_wy2 (chunk_bwd.hip) explains: the activated gate is the difference of two rows of the cumulative gate, its derivative
+    // 1 - e^{-softplus}; x itself is read again only where the threshold is so low that it does not follow from softplus(x) (gband).
+    if constexpr (GRAW) {
+      const int c = c0 + l16;
+      const float inv_na = 1.f / gna, gb = (p.gband && p.gbias) ? p.gbias[(row % p.geom.H) * DK + c] : 0.f;
+      float sb = 0.f, sa = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        // the token before this lane's four: the last of the group below, of the block below for group 0
+        const float below = __shfl(G[u][4 * t + 3], (lane - 16) & 63, LNX_WAVE), under = t ? __shfl(G[u][t ? 4 * t - 1 : 0], 48 + l16, LNX_WAVE) : 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int x = 4 * t + e, r = 16 * t + 4 * kq + e;
+          const float gv = G[u][x] - (e ? G[u][x - (e ? 1 : 0)] : kq ? below : under);
+          const float sp = gv * inv_na;
+          bool lin = sp > p.gthr;
+          if (p.gband) lin = (float)p.graw[(tbase + (int64_t)min(r, len - 1) * ts) * DK + c] + gb > p.gthr;  // the unusual case may wait
+          const float ds = lin ? 1.f : 1.f - __expf(-sp);
+          sa += r < len ? dG[u][x] * gv : 0.f;
+          dG[u][x] = r < len ? dG[u][x] * gna * ds : 0.f;
+          sb += dG[u][x];
+        }
+      }
+      sb = xor32_sum(xor16_sum(sb)), sa = xor32_sum(xor16_sum(sa));
+      if (kq == 0) gate_part(0)[c] = sb, gate_part(1)[c] = sa;
+    }
+    settle16(dq[u]), settle16(dk[u]), settle16(dG[u]);  // one set at a time
+  }
+  lds_barrier();  // the shares are there; K, Q, dPm and dXa are dead
+  auto shares = [&](int which, int t) {
+    float x = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4 * NS; ++w) x += sM[64 * (4 * NS * which + w) + t];
+    return x;
+  };
+  if (tid < 64) {
+    if (tid < len) p.dbeta[tbase + tid * ts] = sRdv[tid] + shares(0, tid);
+  } else if (p.l2norm && tid < 192) {  // through the normalisation: d/dx of x / (|x| + eps) applied to dy is dy / (|x| + eps) - y <y, dy> / |x|
+    const int t = tid & 63, w = (tid >> 6) - 1;
+    const float nrm = 1.f / (w ? sNk : sNq)[t] - LNX_L2_EPS;
+    sC[64 * w + t] = nrm > 0.f ? shares(1 + w, t) / nrm : 0.f;
+  }
+  if (p.l2norm) {
+    lds_barrier();
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const floatx4 fq = load4(sNq + 16 * t + 4 * kq), fk = load4(sNk + 16 * t + 4 * kq), cq = load4(sC + 16 * t + 4 * kq), ck = load4(sC + 64 + 16 * t + 4 * kq);
+#pragma unroll
+      for (int u = 0; u < NS; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          dq[u][4 * t + e] = fq[e] * dq[u][4 * t + e] - cq[e] * (float)q4[u][t][e];
+          dk[u][4 * t + e] = fk[e] * dk[u][4 * t + e] - ck[e] * (float)k4[u][t][e];
+        }
     }
   }
-  lds_barrier();  // dq, dk and the shares of m are in LDS
-  // ---- dq, dk out: thread = (token, the 8-channel groups tq, tq + TPT, ...); the row dots carry them through the normalisation,
-  //      d/dx of x / (|x| + eps) applied to dy:  dy / (|x| + eps) - y <y, dy> / |x| ----
-  {
-    constexpr int TPT = THREADS / 64;
-    const int tr = tid / TPT, tq = tid % TPT;
-    auto emit = [&](int from, int own, const float* fac, T* out) {  // tiles `from` (gradient) and `own` (the row) of a team's 64-channel block
-      auto rows = [&](int tile, int u) {
-        return *reinterpret_cast<const Frag*>(region + 2 * L::tile + (u >> 3) * L::team_bytes + L::ftile + tile * L::tile + (tr * LDX + 8 * (u & 7)) * 2);
-      };
-      const float f = fac[tr];
-      float cf = 0.f;
-      if (p.l2norm) {
-        float dot = 0.f;
+  // ---- dq, dk out over the K and Q tiles, by rows ----
 #pragma unroll
-        for (int u = 0; u < DK / 8; u += TPT) {
-          const Frag a = rows(from, tq + u), b = rows(own, tq + u);
+  for (int u = 0; u < NS; ++u)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) dot += (float)a[e] * (float)b[e];
-        }
-        dot = quad_sum(dot);
-        if (TPT == 8) dot += __shfl_xor(dot, 4, LNX_WAVE);
-        const float nrm = 1.f / f - LNX_L2_EPS;
-        cf = nrm > 0.f ? dot / nrm : 0.f;
-      }
-      if (tr < len) {
+    for (int x = 0; x < 16; ++x) {
+      const int o = RowT::at(16 * (x >> 2) + 4 * kq + (x & 3), 64 * u + 16 * wave + l16);
+      sK[o] = (bf16_t)dk[u][x];
+      sQ[o] = (bf16_t)dq[u][x];
+    }
+  lds_barrier();
 #pragma unroll
-        for (int u = 0; u < DK / 8; u += TPT) {
-          Frag a = rows(from, tq + u);
-          if (p.l2norm) {
-            const Frag b = rows(own, tq + u);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) a[e] = (bf16_t)(f * (float)a[e] - cf * (float)b[e]);
-          }
-          *reinterpret_cast<Frag*>(out + tbase * DK + (int64_t)tr * tsk + 8 * (tq + u)) = a;
-        }
-      }
-    };
-    emit(2, 1, sNq, p.dq);
-    emit(3, 0, sNk, p.dk);
-  }
-  if (tid < 64 && tid < len) {
-    float m = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) m += sM[64 * w + tid];
-    p.dbeta[tbase + tid * ts] = sRdv[tid] + (NT == 2 ? sRdv[64 + tid] : 0.f) + m;
+  for (int u = 0; u < 64 * DK / 8 / 256; ++u) {
+    const int idx = tid + 256 * u, r = idx / (DK / 8), c = 8 * (idx % (DK / 8));
+    if (r < len) {
+      *reinterpret_cast<Frag*>(p.dq + tbase * DK + (int64_t)r * tsk + c) = RowT::load(sQ, r, c);
+      *reinterpret_cast<Frag*>(p.dk + tbase * DK + (int64_t)r * tsk + c) = RowT::load(sK, r, c);
+    }
   }
   lds_barrier();  // dq and dk have left
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) sOut[(16 * t + 4 * kq + e) * LDF + c] = dG[4 * t + e];
-  lds_barrier();
-  // dg leaves by rows: thread = (row tt / 16 + 16 it, four channels), 16-byte accesses.  With the gate activated inside the op,
-  // g = -e^{A_log} softplus(x), x = raw + bias (kda.py:153-165), the gradient goes on to the raw projection as bwd_wy2 (chunk_bwd.hip)
-  // explains: the activated gate is the difference of two rows of the cumulative gate, its derivative 1 - e^{-softplus}; x itself
-  // is read again only where the threshold is so low that it does not follow from softplus(x) (gband).
+  // ---- dg, or the raw projection's gradient, by rows ----
+  float* sOut = reinterpret_cast<float*>(region);  // dg, fp32 [64][LDO]
   if constexpr (!GRAW) {
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int idx = tt + 256 * it, r = idx >> 4, c4 = (idx & 15) * 4;
-      if (r < len) store4(p.dg + (tbase + (int64_t)r * ts) * DK + 64 * team + c4, load4(sOut + r * LDF + c4));
+    for (int u = 0; u < NS; ++u)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) sOut[(16 * (x >> 2) + 4 * kq + (x & 3)) * L::LDO + 64 * u + 16 * wave + l16] = dG[u][x];
+    lds_barrier();
+#pragma unroll
+    for (int u = 0; u < 64 * DK / 4 / 256; ++u) {
+      const int idx = tid + 256 * u, r = idx / (DK / 4), c = 4 * (idx % (DK / 4));
+      if (r < len) store4(p.dg + (tbase + (int64_t)r * ts) * DK + c, load4(sOut + r * L::LDO + c));
     }
   } else {
-    const int c4 = (tt & 15) * 4, r0 = tt >> 4;
-    const float na = gna, inv_na = 1.f / na;
-    floatx4 sb = {0.f, 0.f, 0.f, 0.f}, sa = sb;
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int r = r0 + 16 * it;
-      const floatx4 dgv = load4(sOut + r * LDF + c4);
-      floatx4 gv = load4(sG + r * LDF + c4);
-      if (r > 0) gv = gv - load4(sG + (r - 1) * LDF + c4);
-      floatx4 xv = {0.f, 0.f, 0.f, 0.f};  // x = raw + bias, fetched where it is used: the unusual case may wait
-      if (p.gband) {
-        if (p.gbias) xv = load4(p.gbias + (row % p.geom.H) * DK + 64 * team + c4);
-        const bf16x4 rq = *reinterpret_cast<const bf16x4*>(p.graw + (tbase + (int64_t)min(r, len - 1) * ts) * DK + 64 * team + c4);
+    for (int u = 0; u < NS; ++u)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) xv[e] += (float)rq[e];
-      }
-      floatx4 dr;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float sp = gv[e] * inv_na;
-        const bool lin = p.gband ? xv[e] > p.gthr : sp > p.gthr;
-        const float ds = lin ? 1.f : 1.f - __expf(-sp);
-        dr[e] = r < len ? dgv[e] * na * ds : 0.f;
-        sb[e] += dr[e];
-        sa[e] += r < len ? dgv[e] * gv[e] : 0.f;
-      }
-      if (r < len) store4(p.dgraw + (tbase + (int64_t)r * ts) * DK + 64 * team + c4, dr);
-    }
-    float* sPart = reinterpret_cast<float*>(sK);  // [2][16 row groups][64]: the K and Q tiles are dead
-    store4(sPart + r0 * 64 + c4, sb);
-    store4(sPart + 1024 + r0 * 64 + c4, sa);
+      for (int x = 0; x < 16; ++x) sQ[RowT::at(16 * (x >> 2) + 4 * kq + (x & 3), 64 * u + 16 * wave + l16)] = (bf16_t)dG[u][x];
     lds_barrier();
-    if (tt < 128) {  // the sixteen row groups in a fixed order
-      const float* src = sPart + (tt >> 6) * 1024 + (tt & 63);
-      float t = 0.f;
 #pragma unroll
-      for (int q = 0; q < 16; ++q) t += src[64 * q];
-      gate_part(tt >> 6)[64 * team + (tt & 63)] = t;
+    for (int u = 0; u < 64 * DK / 8 / 256; ++u) {
+      const int idx = tid + 256 * u, r = idx / (DK / 8), c = 8 * (idx % (DK / 8));
+      if (r < len) *reinterpret_cast<Frag*>(p.dgraw + (tbase + (int64_t)r * ts) * DK + c) = RowT::load(sQ, r, c);
     }
   }
 }
@@ -599,7 +627,7 @@ int launch(const KdaBwdParams& p, hipStream_t st) {
   const size_t b = KdaL<DK>::bytes;
   if (const int rc = lnx_lds_limit((const void*)k, b); rc != LNX_OK) return rc;
   lnx_profile_mark("bwd_chunk", st);
-  hipLaunchKernelGGL(k, dim3((unsigned)((int64_t)p.geom.rows * p.geom.N)), dim3(KdaL<DK>::THREADS), b, st, p);
+  hipLaunchKernelGGL(k, dim3((unsigned)((int64_t)p.geom.rows * p.geom.N)), dim3(256), b, st, p);
   lnx_profile_mark(nullptr, st);
   return LNX_OK;
 }

@@ -255,6 +255,10 @@ __device__ __forceinline__ unsigned lds_byte_addr(const void* p) { return (unsig
 __device__ __forceinline__ void dma16(const void* src, unsigned dst) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
 }
+// The same with four bytes per lane: 256 consecutive bytes of LDS
+__device__ __forceinline__ void dma4(const void* src, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
+}
 template <int N> __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 // A [ROWS][COLS] bf16 tile in LDS without padding, COLS * 2 bytes per row, granule g (16 bytes) of row r at granule
