@@ -870,13 +870,15 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
     const float lo = (x[0] + x[1]) + (x[2] + x[3]);
     return NW == 8 ? lo + ((x[4] + x[5]) + (x[6] + x[7])) : lo;
   };
+  // the small loads go straight to LDS, ahead of the slabs: nothing waits for them before the first slab is requested
+  if (wave == 0) dma4(p.beta + tbase + (int64_t)min(lane, len - 1) * ts, lds_byte_addr(sBeta));  // (past the end k and q are zero)
+  if (GATE == LNX_GATE_SCALAR && wave == 1) dma4(at<const float>(p.ws, p.off.G) + slot * 64 + lane, lds_byte_addr(sG));
+  if (wave == 2) dma4(at<const float>(p.ws, p.off.Nq) + slot * 64 + lane, lds_byte_addr(sNq));
+  if (wave == 3) dma4(at<const float>(p.ws, p.off.Nk) + slot * 64 + lane, lds_byte_addr(sNk));
   if (tid < 64) {
-    sG[tid] = (GATE == LNX_GATE_SCALAR) ? at<const float>(p.ws, p.off.G)[slot * 64 + tid] : 0.f;
-    sBeta[tid] = (tid < len) ? p.beta[tbase + tid * ts] : 0.f;
+    if (GATE == LNX_GATE_NONE) sG[tid] = 0.f;
     sM[tid] = sM[64 + tid] = sdG[tid] = sdG[64 + tid] = 0.f;
     sMisc[tid] = 0.f;
-    sNq[tid] = at<const float>(p.ws, p.off.Nq)[slot * 64 + tid];
-    sNk[tid] = at<const float>(p.ws, p.off.Nk)[slot * 64 + tid];
   }
   // ---- the slab loads: one-KB instructions, PER_WAVE of them per wave and slab, straight into LDS buffer `b` ----
   // Token rows past the chunk's end fetch the chunk's last row instead of zeros: whatever they hold only reaches rows of
@@ -914,7 +916,6 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
   };
   constexpr int PER_WAVE = 2 * NH * StT::NINSTR / NW + 16 / NW;  // loads per wave and slab
   static_assert(NH * StT::NINSTR % NW == 0 && TokT::NINSTR == 4 && TrT::NINSTR == 4, "the same count for every wave");
-  __builtin_amdgcn_s_waitcnt(0);  // the small loads above are behind us: from here on this wave's vmcnt counts slab loads only
 #pragma unroll
   for (int u = 0; u < NBUF; ++u)
     if (u * SV < p.dv) issue(u * SV, u);
