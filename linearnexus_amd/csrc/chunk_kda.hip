@@ -17,7 +17,7 @@
 // set s of 64 and all tokens, so that an accumulator element is at the place where pair_levels wants its channel and token:
 // lane (c = lane % 16, kq = lane / 16) holds the tokens 16 t + 4 kq + e of channel c, and everything between the loop and the
 // tiles on their way out happens in registers.  The four pair sums share their factors (pair_sums).
-// Measured at B4 H16 T8192 d128 (8192 chunks): 560 us for 280 KB a chunk, 4.1 TB/s; bwd_dqk and bwd_wy2, which passed dW, a partial dk and an
+// Measured at B4 H16 T8192 d128 (8192 chunks): 461 us for 280 KB a chunk, 5.0 TB/s (with the normalisation about 500); bwd_dqk and bwd_wy2, which passed dW, a partial dk and an
 // fp32 partial gradient of the gate through memory, 402 + 497 us behind and before 217 us of normalisation outside.  With eight waves and one
 // workgroup per CU 650 us: of 20.6 us a chunk 8.5 were pair sums with nothing in flight.
 
@@ -219,9 +219,10 @@ template <int DK> struct KdaL {
   // epilogue: K | Q (then dq | dk, then the gate's gradient) | dPm | dXa | diagonal of dPm, <dR, v>, factors of the normalisation [2], shares of
   // m, <q, dq>, <k, dk> [3][set, wave]
   static constexpr int tile = 64 * LDX * 2, oP = 2 * RowT::BYTES, oF = oP + 2 * tile, epi_bytes = oF + 4 * 64 * (4 + 12 * NS);
-  static constexpr int LDO = DK + 4;    // fp32 rows of the gate's gradient
-  static_assert(64 * LDO * 4 <= oF, "the gate's gradient leaves over the tiles");
-  static constexpr size_t bytes = sizeof(float) * 192 + (epi_bytes > loop_bytes ? epi_bytes : loop_bytes);
+  // the gate's gradient, fp32 [64][LDF] per set: the last set's over K and Q, the one before it waits behind everything else
+  static constexpr int LDF = 64 + 4, oG0 = epi_bytes, all_bytes = epi_bytes + (NS - 1) * 64 * LDF * 4;
+  static_assert(NS <= 2 && 64 * LDF * 4 <= oF, "the gate's gradient leaves over the tiles");
+  static constexpr size_t bytes = sizeof(float) * 192 + (all_bytes > loop_bytes ? all_bytes : loop_bytes);
   static_assert(bytes <= 80 * 1024, "two workgroups per CU");
 };
 
@@ -435,20 +436,14 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
     }
   dma_wait<0>();
   lds_barrier();
-  float dq[NS][16], dk[NS][16], dG[NS][16];
-  bf16x4 k4[NS][4], q4[NS][4];
-  // Sums over the wave's sixteen channels of a set; lane l16 ends with value l16
-  auto channel_sum = [&](float (&v)[16], int which, int u) {
-    exchange<8>(v, l16), exchange<4>(v, l16), exchange<2>(v, l16), exchange<1>(v, l16);
-    sM[64 * (4 * (NS * which + u) + wave) + 16 * (l16 >> 2) + 4 * kq + (l16 & 3)] = v[0];
-  };
-#pragma unroll
-  for (int u = 0; u < NS; ++u) {
-    const int lane = fresh(tid & 63), c0 = 64 * u + 16 * wave;
-    // K and Q at this lane's channel and tokens, normalised (rounded as the op rounds the normalised rows), zero past the chunk's end
+  float dq[NS][16], dk[NS][16], dG[16];
+  // K and Q at this lane's channel and tokens, normalised (rounded as the op rounds the normalised rows), zero past the chunk's end
+  auto rows = [&](int u, bf16x4 (&k4)[4], bf16x4 (&q4)[4]) {
+    const int lane = fresh(tid & 63);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const bf16x4 k = __builtin_bit_cast(bf16x4, RowT::tr4(sK, 16 * t + 4 * kq, c0, lane)), q = __builtin_bit_cast(bf16x4, RowT::tr4(sQ, 16 * t + 4 * kq, c0, lane));
+      const bf16x4 k = __builtin_bit_cast(bf16x4, RowT::tr4(sK, 16 * t + 4 * kq, 64 * u + 16 * wave, lane));
+      const bf16x4 q = __builtin_bit_cast(bf16x4, RowT::tr4(sQ, 16 * t + 4 * kq, 64 * u + 16 * wave, lane));
       const floatx4 fk = load4(sNk + 16 * t + 4 * kq), fq = load4(sNq + 16 * t + 4 * kq);
       floatx4 kf, qf;
 #pragma unroll
@@ -457,8 +452,19 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
         kf[e] = on ? (float)k[e] * fk[e] : 0.f;
         qf[e] = on ? (float)q[e] * fq[e] : 0.f;
       }
-      k4[u][t] = pack_bf16x4(kf), q4[u][t] = pack_bf16x4(qf);
+      k4[t] = pack_bf16x4(kf), q4[t] = pack_bf16x4(qf);
     }
+  };
+  // Sums over the wave's sixteen channels of a set; lane l16 ends with value l16
+  auto channel_sum = [&](float (&v)[16], int which, int u) {
+    exchange<8>(v, l16), exchange<4>(v, l16), exchange<2>(v, l16), exchange<1>(v, l16);
+    sM[64 * (4 * (NS * which + u) + wave) + 16 * (l16 >> 2) + 4 * kq + (l16 & 3)] = v[0];
+  };
+#pragma unroll
+  for (int u = 0; u < NS; ++u) {
+    const int lane = fresh(tid & 63);
+    bf16x4 k4[4], q4[4];
+    rows(u, k4, q4);
     PairSums s;
     float tot = 0.f;
     const float gC = __shfl(G[u][15], 48 + l16, LNX_WAVE);
@@ -469,14 +475,14 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int x = 4 * t + e;
-        const float eg = __expf(G[u][x]), k2 = __expf(fminf(gC - G[u][x], 0.f)) * aK2[u][t][e], kv = (float)k4[u][t][e];
+        const float eg = __expf(G[u][x]), k2 = __expf(fminf(gC - G[u][x], 0.f)) * aK2[u][t][e], kv = (float)k4[t][e];
         s.rp[x] = p.scale * eg * aQ[u][t][e] + d4[e] * kv;
         s.ra[x] = -eg * aK1[u][t][e];
-        s.co[x] = k2 + d4[e] * (float)q4[u][t][e];
+        s.co[x] = k2 + d4[e] * (float)q4[t][e];
         tot += kv * k2;
       }
     }
-    pair_sums(s, G[u], k4[u], q4[u], sBeta, sP, sA, lane);
+    pair_sums(s, G[u], k4, q4, sBeta, sP, sA, lane);
     float mv[16];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -484,47 +490,58 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int x = 4 * t + e;
-        const float kv = (float)k4[u][t][e];
+        const float kv = (float)k4[t][e];
         mv[x] = kv * s.ra[x];
         dq[u][x] = s.rp[x];
         dk[u][x] = bt[e] * s.ra[x] + s.co[x];
-        dG[u][x] = (float)q4[u][t][e] * dq[u][x] - kv * dk[u][x] + 2.f * bt[e] * mv[x];
+        dG[x] = (float)q4[t][e] * dq[u][x] - kv * dk[u][x] + 2.f * bt[e] * mv[x];
       }
     }
+    settle16(dq[u]), settle16(dk[u]), settle16(dG);
     channel_sum(mv, 0, u);
     if (p.l2norm) {
 #pragma unroll
-      for (int x = 0; x < 16; ++x) mv[x] = (float)q4[u][x >> 2][x & 3] * dq[u][x];
+      for (int x = 0; x < 16; ++x) mv[x] = (float)q4[x >> 2][x & 3] * dq[u][x];
       channel_sum(mv, 1, u);
 #pragma unroll
-      for (int x = 0; x < 16; ++x) mv[x] = (float)k4[u][x >> 2][x & 3] * dk[u][x];
+      for (int x = 0; x < 16; ++x) mv[x] = (float)k4[x >> 2][x & 3] * dk[u][x];
       channel_sum(mv, 2, u);
     }
     tot = xor32_sum(xor16_sum(tot + __expf(gC) * ss[u]));  // over the tokens (ss: over its value columns) of this channel
-    if (kq == 3) dG[u][15] += tot;
+    if (kq == 3) dG[15] += tot;
     // dg: reverse cumulative sum over the chunk's tokens of this channel
     float after = 0.f;  // what later blocks of sixteen tokens add
 #pragma unroll
     for (int t = 3; t >= 0; --t) {
 #pragma unroll
-      for (int e = 2; e >= 0; --e) dG[u][4 * t + e] += dG[u][4 * t + e + 1];
+      for (int e = 2; e >= 0; --e) dG[4 * t + e] += dG[4 * t + e + 1];
       // the four lane groups' totals on the VALU (xor16_sum in lnx_common.h): a group adds its odd neighbour's and the upper pair's
-      const unsigned own = __float_as_uint(dG[u][4 * t]);
+      const unsigned own = __float_as_uint(dG[4 * t]);
       const auto p16 = __builtin_amdgcn_permlane16_swap(own, own, false, false);
       const unsigned pair = __float_as_uint(__uint_as_float(p16[0]) + __uint_as_float(p16[1]));
       const auto p32 = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
       const float add = after + ((kq & 1) ? 0.f : __uint_as_float(p16[1])) + ((kq & 2) ? 0.f : __uint_as_float(p32[1]));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dG[u][4 * t + e] += add;
+      for (int e = 0; e < 4; ++e) dG[4 * t + e] += add;
       after += __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
     }
     // With the gate activated inside the op, g = -e^{A_log} softplus(x), x = raw + bias (kda.py:153-165), the gradient goes on to the raw
     // projection as bwd_wy2 (chunk_bwd.hip) explains: the activated gate is the difference of two rows of the cumulative gate, its derivative
     // 1 - e^{-softplus}; x itself is read again only where the threshold is so low that it does not follow from softplus(x) (gband).
+    settle16(dG);
     if constexpr (GRAW) {
-      const int c = c0 + l16;
-      const float inv_na = 1.f / gna, gb = (p.gband && p.gbias) ? p.gbias[(row % p.geom.H) * DK + c] : 0.f;
+      const int c = 64 * u + 16 * wave + l16;
+      const float inv_na = 1.f / gna;
       float sb = 0.f, sa = 0.f;
+      unsigned above = 0;  // bit x: x beyond the threshold, read where it is used: the unusual case may wait
+      if (p.gband) {
+        const float gb = p.gbias ? p.gbias[(row % p.geom.H) * DK + c] : 0.f;
+#pragma unroll 1
+        for (int x = 0; x < 16; ++x) {
+          const int r = min(16 * (x >> 2) + 4 * kq + (x & 3), len - 1);
+          above |= (float)p.graw[(tbase + (int64_t)r * ts) * DK + c] + gb > p.gthr ? 1u << x : 0u;
+        }
+      }
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         // the token before this lane's four: the last of the group below, of the block below for group 0
@@ -534,20 +551,24 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
           const int x = 4 * t + e, r = 16 * t + 4 * kq + e;
           const float gv = G[u][x] - (e ? G[u][x - (e ? 1 : 0)] : kq ? below : under);
           const float sp = gv * inv_na;
-          bool lin = sp > p.gthr;
-          if (p.gband) lin = (float)p.graw[(tbase + (int64_t)min(r, len - 1) * ts) * DK + c] + gb > p.gthr;  // the unusual case may wait
+          const bool lin = p.gband ? (above >> x & 1) != 0 : sp > p.gthr;
           const float ds = lin ? 1.f : 1.f - __expf(-sp);
-          sa += r < len ? dG[u][x] * gv : 0.f;
-          dG[u][x] = r < len ? dG[u][x] * gna * ds : 0.f;
-          sb += dG[u][x];
+          sa += r < len ? dG[x] * gv : 0.f;
+          dG[x] = r < len ? dG[x] * gna * ds : 0.f;
+          sb += dG[x];
         }
       }
       sb = xor32_sum(xor16_sum(sb)), sa = xor32_sum(xor16_sum(sa));
       if (kq == 0) gate_part(0)[c] = sb, gate_part(1)[c] = sa;
     }
-    settle16(dq[u]), settle16(dk[u]), settle16(dG[u]);  // one set at a time
+    if (u + 1 < NS) {
+      float* sG0 = reinterpret_cast<float*>(region + L::oG0);
+#pragma unroll
+      for (int x = 0; x < 16; ++x) sG0[(16 * (x >> 2) + 4 * kq + (x & 3)) * L::LDF + 16 * wave + l16] = dG[x];
+    }
+    settle16(dq[u]), settle16(dk[u]), settle16(dG);  // one set at a time
   }
-  lds_barrier();  // the shares are there; K, Q, dPm and dXa are dead
+  lds_barrier();  // the shares are there; dPm and dXa are dead, a wave's channels of K and Q are its own
   auto shares = [&](int which, int t) {
     float x = 0.f;
 #pragma unroll
@@ -564,15 +585,18 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
   if (p.l2norm) {
     lds_barrier();
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const floatx4 fq = load4(sNq + 16 * t + 4 * kq), fk = load4(sNk + 16 * t + 4 * kq), cq = load4(sC + 16 * t + 4 * kq), ck = load4(sC + 64 + 16 * t + 4 * kq);
+    for (int u = 0; u < NS; ++u) {
+      bf16x4 k4[4], q4[4];
+      rows(u, k4, q4);
 #pragma unroll
-      for (int u = 0; u < NS; ++u)
+      for (int t = 0; t < 4; ++t) {
+        const floatx4 fq = load4(sNq + 16 * t + 4 * kq), fk = load4(sNk + 16 * t + 4 * kq), cq = load4(sC + 16 * t + 4 * kq), ck = load4(sC + 64 + 16 * t + 4 * kq);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          dq[u][4 * t + e] = fq[e] * dq[u][4 * t + e] - cq[e] * (float)q4[u][t][e];
-          dk[u][4 * t + e] = fk[e] * dk[u][4 * t + e] - ck[e] * (float)k4[u][t][e];
+          dq[u][4 * t + e] = fq[e] * dq[u][4 * t + e] - cq[e] * (float)q4[t][e];
+          dk[u][4 * t + e] = fk[e] * dk[u][4 * t + e] - ck[e] * (float)k4[t][e];
         }
+      }
     }
   }
   // ---- dq, dk out over the K and Q tiles, by rows ----
@@ -595,28 +619,20 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
   }
   lds_barrier();  // dq and dk have left
   // ---- dg, or the raw projection's gradient, by rows ----
-  float* sOut = reinterpret_cast<float*>(region);  // dg, fp32 [64][LDO]
-  if constexpr (!GRAW) {
+  float* sOut = reinterpret_cast<float*>(region);
 #pragma unroll
-    for (int u = 0; u < NS; ++u)
+  for (int x = 0; x < 16; ++x) sOut[(16 * (x >> 2) + 4 * kq + (x & 3)) * L::LDF + 16 * wave + l16] = dG[x];
+  lds_barrier();
 #pragma unroll
-      for (int x = 0; x < 16; ++x) sOut[(16 * (x >> 2) + 4 * kq + (x & 3)) * L::LDO + 64 * u + 16 * wave + l16] = dG[u][x];
-    lds_barrier();
+  for (int u = 0; u < NS; ++u) {
+    const float* src = u + 1 < NS ? reinterpret_cast<const float*>(region + L::oG0) : sOut;
 #pragma unroll
-    for (int u = 0; u < 64 * DK / 4 / 256; ++u) {
-      const int idx = tid + 256 * u, r = idx / (DK / 4), c = 4 * (idx % (DK / 4));
-      if (r < len) store4(p.dg + (tbase + (int64_t)r * ts) * DK + c, load4(sOut + r * L::LDO + c));
-    }
-  } else {
-#pragma unroll
-    for (int u = 0; u < NS; ++u)
-#pragma unroll
-      for (int x = 0; x < 16; ++x) sQ[RowT::at(16 * (x >> 2) + 4 * kq + (x & 3), 64 * u + 16 * wave + l16)] = (bf16_t)dG[u][x];
-    lds_barrier();
-#pragma unroll
-    for (int u = 0; u < 64 * DK / 8 / 256; ++u) {
-      const int idx = tid + 256 * u, r = idx / (DK / 8), c = 8 * (idx % (DK / 8));
-      if (r < len) *reinterpret_cast<Frag*>(p.dgraw + (tbase + (int64_t)r * ts) * DK + c) = RowT::load(sQ, r, c);
+    for (int it = 0; it < 4; ++it) {
+      const int idx = tid + 256 * it, r = idx >> 4, c = 4 * (idx & 15);
+      if (r < len) {
+        if constexpr (GRAW) store4(p.dgraw + (tbase + (int64_t)r * ts) * DK + 64 * u + c, load4(src + r * L::LDF + c));
+        else store4(p.dg + (tbase + (int64_t)r * ts) * DK + 64 * u + c, load4(src + r * L::LDF + c));
+      }
     }
   }
 }
