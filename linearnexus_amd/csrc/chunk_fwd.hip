@@ -1564,10 +1564,11 @@ int launch_direct_fwd(const lnx_scan_args* a, const FwdParams& p, int nstate, bo
   return LNX_OK;
 }
 
-// The forward pass on a caller-chosen workspace (a->workspace is not looked at).  `prepared`: the same call but for v, dv and
-// the states has just used this workspace, whose sequence table and value-independent tensors are taken over.  `last`: where the last
+// The forward pass on a caller-chosen workspace (a->workspace is not looked at).  `reuse`: what the workspace already
+// holds, the sequence table, or after the same call but for v, dv and the states the value-independent tensors too.  `last`: where the last
 // sequence's final states go instead of into a->final_state.
-int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_bytes, hipStream_t st, bool prepared = false, float* last = nullptr) {
+enum Reuse { REUSE_NOTHING, REUSE_TABLE, REUSE_PREPARED };
+int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_bytes, hipStream_t st, Reuse reuse = REUSE_NOTHING, float* last = nullptr) {
   const bool packed = a->cu_seqlens != nullptr;
   const int nstate = packed ? a->nseq : a->B;
   if (nstate == 0) return LNX_OK;
@@ -1583,7 +1584,7 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
     return lnx_set_error(LNX_ERR_WORKSPACE, "workspace of %llu bytes needed, %llu given", (unsigned long long)w.total,
                          (unsigned long long)workspace_bytes);
   char* ws = reinterpret_cast<char*>(workspace);
-  if (packed && !prepared)
+  if (packed && reuse == REUSE_NOTHING)
     hipLaunchKernelGGL(build_table_kernel, dim3(1), dim3(1024), 0, st, a->cu_seqlens, a->nseq, lnx_chunk_slots(a), a->T,
                        reinterpret_cast<int32_t*>(ws + w.tab));
   FwdParams p;
@@ -1604,7 +1605,7 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
   p.l2norm = a->use_qk_l2norm;
   p.ws = ws; p.off = w;
   int rc;
-  if (lnx_chunk_direct(a)) return launch_direct_fwd(a, p, nstate, prepared, st);
+  if (lnx_chunk_direct(a)) return launch_direct_fwd(a, p, nstate, reuse == REUSE_PREPARED, st);
   if (a->dtype == LNX_BF16)  // calls without a per-channel gate went to the direct-solve kernels above
     rc = (a->dk == 256)   ? launch_fwd<bf16_t, 256, LNX_GATE_VECTOR>(p, nstate, st)
          : (a->dk == 128) ? launch_fwd<bf16_t, 128, LNX_GATE_VECTOR>(p, nstate, st)
@@ -1620,16 +1621,25 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
 }
 
 // ---------------------------------------------------------------------------------------
-// A long sequence in segments (lnx_chunk_fwd_segmented).  setup: cu_seqlens of the segments and their states [0 | I].
+// A long sequence in segments (lnx_chunk_fwd_segmented).  setup: cu_seqlens of the segments, the slot table that build_table_kernel
+// would make of it (one launch of 4.5 us less) and their states [0 | I].
 // chain: s_in[0] = s0, s_in[i + 1] = B_i + A_i s_in[i], where segment i left [B_i | A_i] in ab [n, H, dk, dv + dk].
 // One workgroup per (head, 16 value columns): the columns stay in LDS (transposed) for all segments, wave w forms rows
-// 16 w .. on the fp32 matrix cores (16x16x4) with its rows of the next A_i on their way meanwhile.  A step waits for 64 KB
-// of A_i from L2 and 4 products of 32 in a row: 16 segments of 4 heads d128 21 us, where a batched library product and
-// two copies per step took 310 us.
+// 16 w .. on the fp32 matrix cores (16x16x4).  A step is a serial chain: barrier, the columns from LDS, 32 products a wave with two waves
+// on a matrix core (0.85 us of the step's 2), the sums back into LDS.  So its operands from LDS are requested at once, and the rows of
+// A_i two steps on (one at dk = 256) go out one by one between the products, each into the registers that have just been used: in front
+// of them they held the first product up.  16 segments of 4 heads d128 43.8 -> 37.3 us (with four sets in flight but in front 43.8, with
+// four waves of two row tiles 40.4), where a batched library product and two copies per step took 310.
 // ---------------------------------------------------------------------------------------
-__global__ void segment_setup_kernel(int32_t* cu, int n, int seg, int T, float* ab, int dk, int dv, int64_t total) {
+__global__ void segment_setup_kernel(int32_t* cu, int32_t* tab, int N, int n, int seg, int T, float* ab, int dk, int dv, int64_t total) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i <= n) cu[i] = min((int)i * seg, T);
+  if (i <= n) cu[i] = min((int)i * seg, T), tab[2 * N + i] = (cu[i] + LNX_C - 1) / LNX_C;
+  if (i < n) tab[2 * N + n + 1 + i] = (int)i;  // no segment is longer than one before it
+  for (int64_t c = i; c < N; c += (int64_t)gridDim.x * 256) {  // segments are whole chunks: slot c is chunk c of the sequence
+    const int t0 = (int)min(c * LNX_C, (int64_t)T);
+    tab[2 * c] = t0 < T ? t0 : 0;
+    tab[2 * c + 1] = min(LNX_C, T - t0);
+  }
   const int w = (dk + dv) / 4;
   if (i >= total / 4) return;
   const int c = 4 * (int)(i % w), r = (int)((i / w) % dk);
@@ -1652,45 +1662,69 @@ __global__ __launch_bounds__(segment_chain_threads<DK>) void segment_chain_kerne
   struct Rows {
     floatx4 a[PW][NT], b[PW];
   };
+  auto fetch_a = [&](Rows& r, int i, int s) {
+    const float* m = ab + ((int64_t)i * H + h) * DK * ldab + dv + 16 * s + 4 * kq;
+#pragma unroll
+    for (int t = 0; t < PW; ++t) r.a[t][s] = load4(m + (int64_t)(16 * tile(t) + l16) * ldab);
+  };
+  auto fetch_b = [&](Rows& r, int i) {
+    const float* m = ab + ((int64_t)i * H + h) * DK * ldab + v0 + l16;
+#pragma unroll
+    for (int t = 0; t < PW; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r.b[t][e] = m[(int64_t)(16 * tile(t) + 4 * kq + e) * ldab];
+  };
   auto fetch = [&](Rows& r, int i) {
-    const float* m = ab + ((int64_t)i * H + h) * DK * ldab;
 #pragma unroll
-    for (int t = 0; t < PW; ++t) {
-#pragma unroll
-      for (int s = 0; s < NT; ++s) r.a[t][s] = load4(m + (int64_t)(16 * tile(t) + l16) * ldab + dv + 16 * s + 4 * kq);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) r.b[t][e] = m[(int64_t)(16 * tile(t) + 4 * kq + e) * ldab + v0 + l16];
-    }
+    for (int s = 0; s < NT; ++s) fetch_a(r, i, s);
+    fetch_b(r, i);
   };
   for (int i = tid; i < DK * 16; i += THREADS) sS[0][(i & 15) * LD + (i >> 4)] = s0 ? s0[((int64_t)h * DK + (i >> 4)) * dv + v0 + (i & 15)] : 0.f;
-  constexpr bool AHEAD = DK <= 128;  // two sets of registers: the next rows are requested before this step's products
-  Rows ra, rb;
-  fetch(ra, 0);
-  // no load behind a branch, where its wait could not be counted: the last steps fetch and multiply what nobody reads
-  auto step = [&](Rows& r, Rows& next, int i) {
+  constexpr int RING = DK <= 128 ? 2 : 1;
+  Rows r[RING];
+#pragma unroll
+  for (int i = 0; i < RING; ++i) {
+    fetch(r[i], min(i, n - 1));
+    __builtin_amdgcn_sched_barrier(0);  // the sets' loads stay in order: the wait for one leaves the other in flight
+  }
+  auto step = [&](Rows& r, int i) {
     lds_barrier();
     const float* cur = sS[i & 1];
-    if (AHEAD) fetch(next, min(i + 1, n - 1));
-    float* out = s_in + ((int64_t)i * H + h) * DK * dv + v0;
-    for (int j = tid; j < DK * 16; j += THREADS) out[(int64_t)(j >> 4) * dv + (j & 15)] = cur[(j & 15) * LD + (j >> 4)];
-    floatx4 acc[PW][2];
+    // no load behind a branch, where its wait could not be counted: the last steps fetch and multiply what nobody reads
+    const int ahead = min(i + RING, n - 1);
+    constexpr int XS = DK <= 128 ? NT : 2;
+    floatx4 acc[PW][2], x[NT];
 #pragma unroll
-    for (int t = 0; t < PW; ++t) acc[t][0] = r.b[t], acc[t][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < XS; ++s) x[s] = load4(cur + l16 * LD + 16 * s + 4 * kq);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < PW; ++t) acc[t][0] = acc[t][1] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < NT; ++s) {
-      const floatx4 x = load4(cur + l16 * LD + 16 * s + 4 * kq);
 #pragma unroll
       for (int t = 0; t < PW; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[t][s & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.a[t][s][e], x[e], acc[t][s & 1], 0, 0, 0);
+        for (int e = 0; e < 4; ++e) acc[t][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.a[t][s][e], x[s][e], acc[t][e & 1], 0, 0, 0);
+      // these registers take the rows RING steps on: a step's loads go out between its products and not in front of them
+      fetch_a(r, ahead, s);
+      if (s + XS < NT) x[s + XS] = load4(cur + l16 * LD + 16 * (s + XS) + 4 * kq);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (!AHEAD) fetch(r, min(i + 1, n - 1));
 #pragma unroll
-    for (int t = 0; t < PW; ++t) store4(sS[(i + 1) & 1] + l16 * LD + 16 * tile(t) + 4 * kq, acc[t][0] + acc[t][1]);
+    for (int t = 0; t < PW; ++t) store4(sS[(i + 1) & 1] + l16 * LD + 16 * tile(t) + 4 * kq, r.b[t] + (acc[t][0] + acc[t][1]));
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_b(r, ahead);
+    if (i >= n) return;
+    float* out = s_in + ((int64_t)i * H + h) * DK * dv + v0;
+#pragma unroll
+    for (int u = 0; u < DK * 16 / THREADS; ++u) {
+      const int j = tid + u * THREADS;
+      out[(int64_t)(j >> 4) * dv + (j & 15)] = cur[(j & 15) * LD + (j >> 4)];
+    }
   };
-  for (int i = 0; i < n; i += 2) {
-    step(ra, AHEAD ? rb : ra, i);
-    if (i + 1 < n) step(AHEAD ? rb : ra, ra, i + 1);
+  for (int i = 0; i < n; i += RING) {  // one exit: a way out between two steps would join the others' count of loads in flight
+#pragma unroll
+    for (int e = 0; e < RING; ++e) step(r[e], i + e);
   }
 }
 
@@ -1780,17 +1814,19 @@ static int fwd_segmented(const lnx_scan_args* a, int32_t nseg, bool every_state,
   int32_t* cu = reinterpret_cast<int32_t*>(ws + g.cu);
   float *ab = reinterpret_cast<float*>(ws + g.ab), *s_in = reinterpret_cast<float*>(ws + g.s_in);
   const int64_t total = (int64_t)g.n * a->H * a->dk * (a->dv + a->dk);
-  hipLaunchKernelGGL(segment_setup_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, st, cu, g.n, g.seg, a->T, ab, a->dk, a->dv, total);
+  hipLaunchKernelGGL(segment_setup_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, st, cu,
+                     reinterpret_cast<int32_t*>(ws + lnx_chunk_ws_layout(&g.first).tab), lnx_chunk_slots(&g.first), g.n, g.seg, a->T, ab, a->dk, a->dv, total);
   g.first.cu_seqlens = g.second.cu_seqlens = cu;
   g.first.initial_state = ab, g.first.final_state = ab;  // every workgroup of the scan reads its columns before it writes them
   g.second.initial_state = s_in;
-  if ((rc = chunk_fwd_on(&g.first, ws, g.ws_bytes, st)) != LNX_OK) return rc;
+  if ((rc = chunk_fwd_on(&g.first, ws, g.ws_bytes, st, REUSE_TABLE)) != LNX_OK) return rc;
   auto chain = a->dk == 256 ? segment_chain_kernel<256> : a->dk == 128 ? segment_chain_kernel<128> : segment_chain_kernel<64>;
   lnx_profile_mark("segment_chain", st);
   hipLaunchKernelGGL(chain, dim3(a->H, a->dv / 16), dim3(a->dk == 64 ? 256 : 512), 0, st, ab, a->initial_state, s_in, g.n, a->H, a->dv);
-  if (every_state) return chunk_fwd_on(&g.second, ws, g.ws_bytes, st, lnx_chunk_direct(a));
+  const Reuse reuse = lnx_chunk_direct(a) ? REUSE_PREPARED : REUSE_TABLE;
+  if (every_state) return chunk_fwd_on(&g.second, ws, g.ws_bytes, st, reuse);
   g.second.final_state = s_in;  // the states at the other segments' ends: nobody reads them
-  return chunk_fwd_on(&g.second, ws, g.ws_bytes, st, lnx_chunk_direct(a), a->final_state);
+  return chunk_fwd_on(&g.second, ws, g.ws_bytes, st, reuse, a->final_state);
 }
 
 extern "C" int lnx_chunk_fwd_segmented(const lnx_scan_args* a, int32_t nseg, void* stream) { return fwd_segmented(a, nseg, true, stream); }

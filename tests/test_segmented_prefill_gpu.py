@@ -80,3 +80,16 @@ def test_long_prompt_agrees_with_the_sequential_kernels(monkeypatch):
     eo = (o1.float() - o2.float()).abs().max() / o1.float().abs().max()
     eS = (S1 - S2).abs().max() / S1.abs().max()
     assert eo < 2e-2 and eS < 2e-2, (float(eo), float(eS))
+
+
+@pytest.mark.parametrize("dk", [64, 128, 256])
+@pytest.mark.parametrize("nseg", ["3", "4", "7", "8", "9"])
+def test_chain_of_any_length(dk, nseg, monkeypatch):
+    """The chain of the segments' states keeps two sets of rows in flight (one at dk = 256): odd and even numbers of segments."""
+    monkeypatch.setenv("LNX_PREFILL_SEGMENTS", nseg)
+    x, dt = _prep(make_inputs(103, 1, 2, 64 * int(nseg) - 5, dk, 64, gate="scalar", with_state=True), False)
+    o_ref, S_ref = oracle_fwd(x, "scalar")
+    with torch.no_grad():
+        o, S = gpu_chunk_fwd(x, "scalar", dt)
+    eo, eS = max_rel(o.float().cpu().numpy(), o_ref), max_rel(S.cpu().numpy(), S_ref)
+    assert eo < 1e-4 and eS < 1e-4, (eo, eS)
