@@ -142,6 +142,7 @@ int lnx_recurrent_fwd(const lnx_scan_args* a, void* hip_stream);
  * workspace, unchanged, to lnx_chunk_bwd (unless forward_only was set), with the same shape, dtype, gate, nseq,
  * token_first, scale and use_qk_l2norm fields: the layout of the workspace follows from B, H, T, dk, dv, dtype, gate
  * and nseq alone (o_dtype does not enter it), and there is exactly one set of kernels per such shape.
+ * q, k, v, beta and a per-channel gate (g or gate_raw) are read again by lnx_chunk_bwd and must hold the same values.
  * Shapes: dk in {64, 128, 256} (256 is the head_dim of the reference's Gated DeltaNet presets,
  * models.py:142-143), dv a multiple of 64.  q, k, v, o, a per-channel gate (g or gate_raw), the states, the workspace
  * and the gradients of all of these must be 16-byte aligned (the kernels move their rows as 16-byte vectors);

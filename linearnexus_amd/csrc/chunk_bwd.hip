@@ -22,6 +22,7 @@ struct BwdParams {
   const void* k;
   const void* v;
   const float* beta;
+  const float* g;  // read again by chunk_kda.hip alone
   const void* d_o;
   const float* d_sT;
   void* dq;
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
         rdO.load(reinterpret_cast<const T*>(p.d_o) + tbase * p.dv + v0, (int64_t)p.geom.ts * p.dv, len, mt);
         rdD.load(wsp<T>(p, p.off.dD) + slot * 64 * p.dv + v0, p.dv, 64, mt);
         if (GATE == LNX_GATE_SCALAR && mt < 64) rG = wsp<float>(p, p.off.G)[slot * 64 + mt];
-        if (GATE == LNX_GATE_VECTOR && mt < DK) rG = wsp<float>(p, p.off.G)[(slot * 64 + 63) * DK + mt];
+        if (GATE == LNX_GATE_VECTOR && mt < DK) rG = wsp<float>(p, p.off.G)[gate_last<T, DK>(slot) + mt];
 #pragma unroll
         for (int it = 0; it < Slab::IT; ++it) {
           const int r = min((mt + 256 * it) / Slab::VPR, 63);
@@ -266,7 +267,7 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
         if (FUSE) rP.load(wsp<T>(p, p.off.P) + slot * 64 * 64, 64, 64, mt);
         else rdD.load(wsp<T>(p, p.off.dD) + slot * 64 * p.dv + v0, p.dv, 64, mt);
         if (GATE == LNX_GATE_SCALAR && mt < 64) rG = wsp<float>(p, p.off.G)[slot * 64 + mt];
-        if (GATE == LNX_GATE_VECTOR && mt < DK) rG = wsp<float>(p, p.off.G)[(slot * 64 + 63) * DK + mt];
+        if (GATE == LNX_GATE_VECTOR && mt < DK) rG = wsp<float>(p, p.off.G)[gate_last<T, DK>(slot) + mt];
 #pragma unroll
         for (int it = 0; it < Slab::IT; ++it) {
           const int r = min((mt + 256 * it) / Slab::VPR, 63);
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
         else R.dD.load(wsp<T>(p, p.off.dD) + slot * 64 * p.dv + v0, p.dv, 64, mt);
         // every thread loads (clamped index): a load behind a branch cannot be counted
         if (GATE == LNX_GATE_SCALAR) R.G = wsp<float>(p, p.off.G)[slot * 64 + (mt & 63)];
-        if (GATE == LNX_GATE_VECTOR) R.G = wsp<float>(p, p.off.G)[(slot * 64 + 63) * DK + min(mt, DK - 1)];
+        if (GATE == LNX_GATE_VECTOR) R.G = wsp<float>(p, p.off.G)[gate_last<T, DK>(slot) + min(mt, DK - 1)];
       }
       if (part < 0 || part == 2) {
         if (GATE == LNX_GATE_VECTOR) R.Q.load(wsp<T>(p, p.off.Qg) + slot * 64 * DK, DK, 64, mt);
@@ -1434,7 +1435,7 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
     k.beta = p.beta; k.dv = p.dv; k.l2norm = p.l2norm; k.scale = p.scale; k.ws = p.ws; k.off = p.off;
     k.d_o = reinterpret_cast<const bf16_t*>(p.d_o); k.dq = reinterpret_cast<bf16_t*>(p.dq); k.dk = reinterpret_cast<bf16_t*>(p.dk);
     k.dv_out = reinterpret_cast<bf16_t*>(p.dv_out); k.dbeta = p.dbeta; k.dg = p.dg;
-    k.graw = reinterpret_cast<const bf16_t*>(p.graw); k.gA = p.gA; k.gbias = p.gbias; k.gthr = p.gthr; k.gband = p.gband;
+    k.g = p.g, k.graw = reinterpret_cast<const bf16_t*>(p.graw); k.gA = p.gA; k.gbias = p.gbias; k.gthr = p.gthr; k.gband = p.gband;
     k.dgraw = reinterpret_cast<bf16_t*>(p.dgraw); k.gpart = p.gpart; k.gprows = p.gprows;
     return lnx_kda_bwd_chunk(k, DK, st);
   } else {
@@ -1494,7 +1495,7 @@ extern "C" int lnx_chunk_bwd(const lnx_scan_args* a, void* stream) {
   p.geom.rows = packed ? a->H : a->B * a->H;
   p.geom.cu = a->cu_seqlens;
   p.geom.tab = packed ? reinterpret_cast<const int32_t*>(reinterpret_cast<char*>(a->workspace) + w.tab) : nullptr;
-  p.q = a->q; p.k = a->k; p.v = a->v; p.beta = a->beta; p.d_o = a->d_o; p.d_sT = a->d_final_state;
+  p.q = a->q; p.k = a->k; p.v = a->v; p.beta = a->beta; p.g = a->g; p.d_o = a->d_o; p.d_sT = a->d_final_state;
   p.dq = a->d_q; p.dk = a->d_k; p.dv_out = a->d_v; p.dbeta = a->d_beta; p.dg = a->d_g; p.ds0 = a->d_initial_state;
   p.dv = a->dv; p.gate = a->gate; p.l2norm = a->use_qk_l2norm; p.scale = a->scale; p.slab = a->test_scan_slab;
   const bool raw_gate = a->gate == LNX_GATE_VECTOR && a->gate_raw != nullptr;

@@ -124,6 +124,9 @@ inline bool lnx_chunk_direct(const lnx_scan_args* a) {
 }
 
 // 2-byte inputs with a per-channel gate and dk <= 128: the scans of the WY split, then the one gradient kernel of chunk_kda.hip.
+// G then holds the chunks' last rows alone, [slot][dk]: the scans want e^{G_C}, and the gradient kernel sums the gate up itself.
+template <typename T, int DK> constexpr bool lnx_gate_last_only = sizeof(T) == 2 && DK <= 128;
+template <typename T, int DK> __device__ __forceinline__ int64_t gate_last(int64_t slot) { return lnx_gate_last_only<T, DK> ? slot * DK : (slot * LNX_C + LNX_C - 1) * DK; }
 inline bool lnx_chunk_kda(const lnx_scan_args* a) { return a->dtype == LNX_BF16 && a->dk <= 128 && a->gate == LNX_GATE_VECTOR; }
 
 inline uint64_t lnx_align256(uint64_t x) { return (x + 255) & ~uint64_t(255); }
@@ -165,7 +168,7 @@ inline ChunkWs lnx_chunk_ws_layout(const lnx_scan_args* a) {
   w.Tm = w.Fq = 0;
   w.Nq = take(bwd && kda ? slots * C * 4 : 0);  // of the rows that the op normalises, as above
   w.Nk = take(bwd && kda ? slots * C * 4 : 0);
-  w.G = take(vec ? slots * C * dk * 4 : slots * C * 4);
+  w.G = take(!vec ? slots * C * 4 : kda ? slots * dk * 4 : slots * C * dk * 4);
   w.P = take(slots * C * C * es);
   w.X = take(vec && saved && !kda ? slots * C * C * es : 0);
   w.W = take(slots * C * dk * es);
@@ -233,7 +236,8 @@ struct DirectParams {
 };
 // ... and of the chunk-local gradients of the per-channel gate (chunk_kda.hip): what a gate activated inside the op adds
 struct KdaBwdParams : DirectParams {
-  const bf16_t* graw;  // raw gate projection, or NULL
+  const float* g;      // the per-channel gate, or
+  const bf16_t* graw;  // its raw projection
   const float* gA;
   const float* gbias;
   float gthr;

@@ -467,7 +467,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   const T* qg = reinterpret_cast<const T*>(p.q) + tbase * DK;
   const T* kg = reinterpret_cast<const T*>(p.k) + tbase * DK;
   const T* vg = reinterpret_cast<const T*>(p.v) + tbase * p.vcols;
-  float* Gg = ws_ptr<float>(p, p.off.G) + slot * 64 * DK;
+  constexpr bool LAST = lnx_gate_last_only<T, DK>;
+  float* Gg = ws_ptr<float>(p, p.off.G) + (LAST ? gate_last<T, DK>(slot) : slot * 64 * DK);
   const int l16 = lane & 15, kq = lane >> 4;
 
   // ---- phase A: per 64-channel half ----
@@ -598,7 +599,11 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       for (int i = 0; i < 16; ++i) sG[(16 * seg + i) * LDF + c] = gs[i] + off;
     }
     lds_barrier();
-    {  // G, K e^{G_last - G}, scale Q e^G of this half -> workspace
+    // G, K e^{G_last - G}, scale Q e^G of this half -> workspace.  LAST: of G only the last row, but beta K e^G, into the place of W, where
+    // phase D finds it: the rows of G were 32 KB written a chunk, and a second exponential of all of them in phase D (B4 H16 T8192 d128, forward
+    // and backward: 1568 -> 1528 us).
+    {
+      T* Kbg = ws_ptr<T>(p, p.off.W) + slot * 64 * DK + 64 * h;
       T* Krg = ws_ptr<T>(p, p.off.Kr) + slot * 64 * DK + 64 * h;
       T* Qgg = ws_ptr<T>(p, p.off.Qg) + slot * 64 * DK + 64 * h;
 #pragma unroll
@@ -606,16 +611,21 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
         const int idx = tid + 256 * it, r = idx >> 4, c = (idx & 15) * 4;
         const floatx4 gr = load4(sG + r * LDF + c), gl = load4(sG + 63 * LDF + c);
         const floatx4 kk = load4(sK + r * LDC + c), qq = load4(sQ + r * LDC + c);
-        floatx4 kr, qgv;
+        const float bt = sBeta[r];
+        floatx4 kr, qgv, kb;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
+          const float eg = __expf(gr[e]);
           kr[e] = kk[e] * __expf(fminf(gl[e] - gr[e], 0.f));
-          qgv[e] = qq[e] * p.scale * __expf(gr[e]);
+          qgv[e] = qq[e] * p.scale * eg;
+          kb[e] = kk[e] * bt * eg;
         }
-        store4(Gg + r * DK + 64 * h + c, gr);
+        if constexpr (LAST) store4(Kbg + r * DK + c, kb);
+        else store4(Gg + r * DK + 64 * h + c, gr);
         store4(Krg + r * DK + c, kr);
         store4(Qgg + r * DK + c, qgv);
       }
+      if (LAST && tid < 16) store4(Gg + 64 * h + 4 * tid, load4(sG + 63 * LDF + 4 * tid));
     }
     if constexpr (LEVELS) {
       kda_pair_half(a32, a16, aD, reinterpret_cast<const bf16_t*>(sK), reinterpret_cast<const bf16_t*>(sQ), LDC, sG, LDF, wave, lane);
@@ -754,9 +764,11 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   typedef TileRegs<T, 64, 64> Slab;
   constexpr int VN = Slab::N;
   Slab rIn;
-  floatx4 rGs[Slab::IT][VN / 4];  // K slabs: the gate values of exactly the elements this thread holds
+  floatx4 rGs[LAST ? 1 : Slab::IT][VN / 4];  // K slabs: the gate values of exactly the elements this thread holds
   auto fetch_slab = [&](int s_) {
-    if (s_ < NH) {
+    if (LAST && s_ < NH) {
+      rIn.load(ws_ptr<T>(p, p.off.W) + slot * 64 * DK + 64 * s_, DK, 64, tid);
+    } else if (s_ < NH) {
       rIn.load(kg + 64 * s_, tsk, len, tid);
 #pragma unroll
       for (int it = 0; it < Slab::IT; ++it) {
@@ -769,21 +781,17 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       else rIn.zero();  // value columns that v does not hold
     }
   };
-  __syncthreads();  // G is read back from the workspace by other threads than wrote it: global memory must be ordered too
+  __syncthreads();  // G, or beta K e^G, is read back from the workspace by other threads than wrote it: global memory must be ordered too
   fetch_slab(0);
 #pragma unroll 1
   for (int s_ = 0; s_ < nslab; ++s_) {
     const bool is_k = s_ < NH;
     lds_barrier();  // the previous slab's tiles (first pass: the inverse, the gate tile) are dead
-    if (is_k) {     // K slab scaled by beta_t e^{G_t[c]} on its way into LDS
+    if (is_k && !LAST) {  // K slab scaled by beta_t e^{G_t[c]} on its way into LDS
 #pragma unroll
       for (int it = 0; it < Slab::IT; ++it) {
         const int idx = tid + 256 * it, r = idx / Slab::VPR, c = (idx - r * Slab::VPR) * VN;
         typename Vec16<T>::V x = rIn.x[it];
-        if (norm) {
-#pragma unroll
-          for (int e = 0; e < VN; ++e) x[e] = from_f32<T>(to_f32(x[e]) * sNk[r]);
-        }
 #pragma unroll
         for (int e = 0; e < VN; ++e) x[e] = from_f32<T>(to_f32(x[e]) * sBeta[r] * __expf(rGs[it][e / 4][e % 4]));
         *reinterpret_cast<typename Vec16<T>::V*>(sIn + r * LDC + c) = x;
@@ -908,7 +916,7 @@ __global__ __launch_bounds__(512) void chunk_scan_kernel(FwdParams p) {
         rW.load(ws_ptr<T>(p, p.off.W) + slot * 64 * DK, DK, 64, mt);
         rU.load(ws_ptr<T>(p, p.off.U) + slot * 64 * p.dv + v0, p.dv, 64, mt);
         if (GATE == LNX_GATE_SCALAR && mt < 64) rG = ws_ptr<float>(p, p.off.G)[slot * 64 + mt];
-        if (GATE == LNX_GATE_VECTOR && mt < DK) rG = ws_ptr<float>(p, p.off.G)[(slot * 64 + 63) * DK + mt];
+        if (GATE == LNX_GATE_VECTOR && mt < DK) rG = ws_ptr<float>(p, p.off.G)[gate_last<T, DK>(slot) + mt];
       };
       auto fetch_k = [&](int n) {
         const int64_t slot = (int64_t)row * N + n;
@@ -963,7 +971,7 @@ __global__ __launch_bounds__(512) void chunk_scan_kernel(FwdParams p) {
         rU.load(ws_ptr<T>(p, p.off.U) + slot * 64 * p.dv + v0, p.dv, 64, mt);
         rP.load(ws_ptr<T>(p, p.off.P) + slot * 64 * 64, 64, 64, mt);
         if (GATE == LNX_GATE_SCALAR && mt < 64) rG = ws_ptr<float>(p, p.off.G)[slot * 64 + mt];
-        if (GATE == LNX_GATE_VECTOR && mt < DK) rG = ws_ptr<float>(p, p.off.G)[(slot * 64 + 63) * DK + mt];
+        if (GATE == LNX_GATE_VECTOR && mt < DK) rG = ws_ptr<float>(p, p.off.G)[gate_last<T, DK>(slot) + mt];
       };
       auto fetch_q = [&](int n) {
         const int64_t slot = (int64_t)row * N + n;
@@ -1044,7 +1052,7 @@ __global__ __launch_bounds__(512) void chunk_scan_kernel(FwdParams p) {
       if (FUSE) R.P.load(ws_ptr<T>(p, p.off.P) + slot * 64 * 64, 64, 64, mt);
       // every thread loads (clamped index): a load behind a branch cannot be counted
       if (GATE == LNX_GATE_SCALAR) R.G = ws_ptr<float>(p, p.off.G)[slot * 64 + (mt & 63)];
-      if (GATE == LNX_GATE_VECTOR) R.G = ws_ptr<float>(p, p.off.G)[(slot * 64 + 63) * DK + min(mt, DK - 1)];  // G_last[c]
+      if (GATE == LNX_GATE_VECTOR) R.G = ws_ptr<float>(p, p.off.G)[gate_last<T, DK>(slot) + min(mt, DK - 1)];  // G_last[c]
     };
     auto commit_rest = [&](const Tiles& R, int pb, int part = -1) {  // parts as in fetch (W is written by the caller)
       if (part < 0 || part == 1) R.K.store(sK + pb * L::kKT, LDK, mt);

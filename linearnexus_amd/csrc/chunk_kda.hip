@@ -17,8 +17,9 @@
 // set s of 64 and all tokens, so that an accumulator element is at the place where pair_levels wants its channel and token:
 // lane (c = lane % 16, kq = lane / 16) holds the tokens 16 t + 4 kq + e of channel c, and everything between the loop and the
 // tiles on their way out happens in registers.  The four pair sums share their factors (pair_sums).
-// Measured at B4 H16 T8192 d128 (8192 chunks): 461 us for 280 KB a chunk, 5.0 TB/s (with the normalisation about 500); bwd_dqk and bwd_wy2, which passed dW, a partial dk and an
-// fp32 partial gradient of the gate through memory, 402 + 497 us behind and before 217 us of normalisation outside.  With eight waves and one
+// Measured at B4 H16 T8192 d128 (8192 chunks): 470 us for 280 KB a chunk, 4.9 TB/s (with the normalisation about 500); bwd_dqk and bwd_wy2,
+// which passed dW, a partial dk and an fp32 partial gradient of the gate through memory, 402 + 497 us behind and before 217 us of
+// normalisation outside.  The cumulative gate is summed up again from the gate: 461 -> 470 us here, 25 less where the prepare kernel wrote it.  With eight waves and one
 // workgroup per CU 650 us: of 20.6 us a chunk 8.5 were pair sums with nothing in flight.
 
 #include "chunk_common.h"
@@ -413,12 +414,16 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
     dma16(p.k + (tbase + (int64_t)r * ts) * DK + c, slab0 + 1024 * (wave + 4 * u));
     dma16(p.q + (tbase + (int64_t)r * ts) * DK + c, slab0 + RowT::BYTES + 1024 * (wave + 4 * u));
   }
-  float G[NS][16];  // the cumulative gate of this lane's channels and tokens
+  float G[NS][16];  // the gate of this lane's channels and tokens, later its cumulative sum
 #pragma unroll
   for (int u = 0; u < NS; ++u)
 #pragma unroll
-    for (int x = 0; x < 16; ++x)
-      G[u][x] = at<const float>(p.ws, p.off.G)[(slot * 64 + 16 * (x >> 2) + 4 * kq + (x & 3)) * DK + 64 * u + 16 * wave + l16];
+    for (int x = 0; x < 16; ++x) {
+      const int r = min(16 * (x >> 2) + 4 * kq + (x & 3), len - 1);
+      const int64_t o = (tbase + (int64_t)r * ts) * DK + 64 * u + 16 * wave + l16;
+      if constexpr (GRAW) G[u][x] = (float)p.graw[o];
+      else G[u][x] = p.g[o];
+    }
   rdv = quad_sum(rdv);
   if ((tid & 3) == 0) sRdv[tid >> 2] = rdv;
   if (!p.l2norm && tid < 64) sNq[tid] = sNk[tid] = 1.f;
@@ -436,6 +441,32 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
     }
   dma_wait<0>();
   lds_barrier();
+#pragma unroll
+  for (int u = 0; u < NS; ++u) {
+    float gb = 0.f;
+    if constexpr (GRAW) gb = p.gbias ? p.gbias[(row % p.geom.H) * DK + 64 * u + 16 * wave + l16] : 0.f;
+    float before = 0.f;  // what the blocks of sixteen tokens before add
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int x = 4 * t + e;
+        if constexpr (GRAW) G[u][x] = gna * lnx_softplus_thr(G[u][x] + gb, p.gthr);
+        G[u][x] = 16 * t + 4 * kq + e < len ? G[u][x] : 0.f;
+        if (e) G[u][x] += G[u][x - (e ? 1 : 0)];
+      }
+      // as the reverse sum of its gradient below
+      const unsigned own = __float_as_uint(G[u][4 * t + 3]);
+      const auto p16 = __builtin_amdgcn_permlane16_swap(own, own, false, false);
+      const unsigned pair = __float_as_uint(__uint_as_float(p16[0]) + __uint_as_float(p16[1]));
+      const auto p32 = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
+      const float add = before + (((kq & 1) ? __uint_as_float(p16[0]) : 0.f) + ((kq & 2) ? __uint_as_float(p32[0]) : 0.f));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) G[u][4 * t + e] += add;
+      before += __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
+    }
+    settle16(G[u]);
+  }
   float dq[NS][16], dk[NS][16], dG[16];
   // K and Q at this lane's channel and tokens, normalised (rounded as the op rounds the normalised rows), zero past the chunk's end
   auto rows = [&](int u, bf16x4 (&k4)[4], bf16x4 (&q4)[4]) {
