@@ -21,10 +21,10 @@
 //   bwd_chunk  (one workgroup per chunk, all in parallel)                         dq, dk, dbeta, dg from q, k, v, dO, the
 //              two saved states and D, dR as the scans left them (dv leaves the reverse scan)
 //
-// Both scans split their waves into one compute wave per 16 value columns of the slab (matrix work on the tiles in LDS, the fp32 state in MFMA accumulators for the whole sequence) and four mover waves
-// (global loads two chunks ahead into registers, the next chunk's tiles into LDS, LDS -> global copies of results as
-// whole rows); all five input tiles and the per-token scalars are double-buffered in LDS, so two LDS-only barriers per
-// chunk suffice.  bwd_chunk brings its slabs in with loads that go straight to LDS (mma_tiles.h).
+// Both scans split their waves into one compute wave per 16 value columns of the slab (matrix work on the tiles in LDS, the fp32 state in MFMA
+// accumulators for the whole sequence) and four or eight mover waves (global loads two chunks ahead into registers, the next chunk's tiles into
+// LDS, LDS -> global copies of results as whole rows), scan_fwd's narrow form into output waves as well; all five input tiles are
+// double-buffered in LDS, so one or two LDS-only barriers per chunk suffice.  bwd_chunk brings its slabs in with loads that go straight to LDS (mma_tiles.h).
 
 #include <type_traits>
 
@@ -69,8 +69,15 @@ __device__ __forceinline__ typename Vec16<T>::V scaled(typename Vec16<T>::V x, f
 
 // Per-token scalars of one chunk in LDS, written by the movers when they commit a chunk
 struct Scal {
-  enum { BETA = 0, GAM = 64, R = 128, DEC = 192, SIZE = 256 };  // beta, beta e^G, e^{G_C - G}, e^{G_C}
+  enum { BETA = 0, GAM = 64, R = 128, DEC = 192, SIZE = 256, NK = 256, FQ = 320, SIZE_FACTORS = 384 };  // beta, beta e^G, e^{G_C - G}, e^{G_C}, factors of the K and Q rows
 };
+template <int GATE> __device__ __forceinline__ void put_scalars(float* sc, int t, float b, float g, float gc) {
+  const float gam = (GATE == LNX_GATE_SCALAR) ? __expf(g) : 1.f;
+  sc[Scal::BETA + t] = b;
+  sc[Scal::GAM + t] = b * gam;
+  sc[Scal::R + t] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(gc - g, 0.f)) : 1.f;
+  if (t == 0) sc[Scal::DEC] = (GATE == LNX_GATE_SCALAR) ? __expf(gc) : 1.f;
+}
 
 // ---------------------------------------------------------------------------------------
 // scan_fwd.  A compute wave owns a 16-column strip of the value slab: its [dk x 16] part of the state stays in MFMA
@@ -83,13 +90,25 @@ struct Scal {
 // 1.5 us in the short calls: a SIMD takes 1 KB of LDS reads in about 16 cycles, and a strip reads 60 KB of operands whatever its
 // width.  The movers convert K and Q rows, 2.5 VALU instructions an element: with eight waves of them instead of four 57 -> 52 us and
 // 29 -> 27 us; in reverse the third wave of each SIMD leaves too few registers (59 -> 59 - 68 us), it keeps four.
-//  All five input tiles are double-buffered, so the movers write chunk
-// n + 1 while chunk n is being read and two barriers per chunk are enough:
+// All five input tiles are double-buffered, so the movers write chunk n + 1 while chunk n is being read.  64-column slabs with outputs:
 //   B1    buffers of chunk n complete           compute: S^T -> LDS (saved states), Y, Q S, R, D (-> LDS, transposed), O -> LDS
 //                                               movers:  loads of chunk n + 2; chunk n + 1 -> the other buffers
 //   Bmid  O, S^T and D^T are in LDS             compute: state update        movers: O, S^T, D^T -> global
+// 32-column slabs, where the chain of one chunk is what a call waits for: O hangs on S and D but nothing on O, so it has waves of its own, a
+// chunk behind, and one barrier per chunk is enough:
+//   B1    K, V, Tm of chunk n, Q, Pm of n - 1   compute: Y, R, D, state update; S^T and D^T -> LDS [n mod 2]
+//                                               output:  O of chunk n - 1 from S^T and D^T as the compute wave has them in registers -> global;
+//                                                        the per-token scalars of chunk n + 2
+//                                               movers:  S^T, D^T of n - 1 -> global; loads and writes as above, Q and Pm of the chunk before
+// A chunk of one prompt of 1000 tokens: 1.43 us with everything in the compute waves (Y and Q S 0.5, R and D 0.2, the rest of O 0.2, update 0.3,
+// movers 0.7 between B1 and Bmid), 1.23 so (compute 1.0, movers 1.15, output 0.8); the call 33.3 -> 32.1 us, the scan of B2 H16 T2007 53 -> 48.
+// Output waves beside two barriers: 35.4 us, the movers' 0.85 us then stood between B1 and Bmid alone.  One barrier with the row factors from
+// memory, five small loads a mover: 33.0; every mover in the same order: 33.0, all of them load, convert and write at the same time, so half
+// write a tile ahead of the next loads and half behind them.  The same bits in all.
+// Final states alone (OUT false, the first pass over a segmented prompt): no Q, no Pm, no O, one barrier: 16 segments of 4 heads, 64 chunks
+// each, 111 -> 73 us.
 // ---------------------------------------------------------------------------------------
-template <int DK, int BVW> struct FScanL {
+template <int DK, int BVW, bool OUT> struct FScanL {
   // 32-column slabs are taken where the chip has room for more workgroups, so what counts there is the time of a chunk's
   // chain: operand tiles in chain order, rows 32 bytes off a multiple of 64 (Mma16).  64-column slabs are bound by what the
   // movers carry.
@@ -98,29 +117,35 @@ template <int DK, int BVW> struct FScanL {
   static constexpr int LDS = DK + PAD, LDD = LNX_C + PAD;  // of the tiles on their way out: states, D or dR
   static constexpr int kK = 64 * LDK, kST = BV * LDS, kV = 64 * LDV, kC = 64 * LDC;
   static constexpr int kDT = BV * LDD;
-  // [2] x (K, Q, V, Tm, Pm) | O | S^T | D^T | scalars [2]
-  static constexpr size_t bytes = sizeof(T) * (2 * (2 * kK + kV + 2 * kC) + kV + kST + kDT) + sizeof(float) * 2 * Scal::SIZE;
-  static constexpr int threads = 64 * NCW + MT;
+  static constexpr int NOW = OUT && CHAIN ? NCW : 0;  // output waves, one per strip
+  static constexpr int NST = NOW ? 2 : 1;             // buffers of S^T and D^T
+  static constexpr int NSC = NOW ? 4 : 2;             // ... of scalars
+  static constexpr int SCS = NOW ? Scal::SIZE_FACTORS : Scal::SIZE;
+  // [2] x (K, Q, V, Tm, Pm) | O, unless output waves store it | S^T [NST] | D^T [NST] | scalars [2]; without outputs [2] x (K, V, Tm) | scalars [2]
+  static constexpr size_t bytes = sizeof(T) * (OUT ? 2 * (2 * kK + kV + 2 * kC) + (NOW ? 0 : kV) + NST * (kST + kDT) : 2 * (kK + kV + kC)) + sizeof(float) * NSC * SCS;
+  static constexpr int threads = 64 * (NCW + NOW) + MT;
 };
 
 template <int DK, int GATE, int BVW, typename OT>
-__global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(DirectParams p) {
-  typedef FScanL<DK, BVW> L;
+__global__ __launch_bounds__((FScanL<DK, BVW, !std::is_void<OT>::value>::threads)) void scan_fwd_kernel(DirectParams p) {
+  constexpr bool OUT = !std::is_void<OT>::value;  // void: final states alone (forward only)
+  typedef FScanL<DK, BVW, OUT> L;
   constexpr int LDK = L::LDK, LDC = L::LDC, BV = L::BV, LDV = L::LDV, NCW = L::NCW, LDS = L::LDS, LDD = L::LDD;
   constexpr bool CHAIN = L::CHAIN;
   constexpr int MT = L::MT;  // mover threads
+  constexpr int NOW = L::NOW;
   constexpr int KT = DK / 16;  // row tiles of the state strip
   static_assert(DK == 64 || DK == 128, "dk = 64 or 128");
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);  // [2][64][LDK]
   T* sQ = sK + 2 * L::kK;
-  T* sV = sQ + 2 * L::kK;              // [2][64][LDV]
+  T* sV = sQ + (OUT ? 2 * L::kK : 0);  // [2][64][LDV]
   T* sTm = sV + 2 * L::kV;             // [2][64][LDC]
   T* sP = sTm + 2 * L::kC;
   T* sO = sP + 2 * L::kC;              // bf16 outputs on their way out [64][LDV]
-  T* sST = sO + L::kV;                 // entering state, transposed [v][dk], on its way to the workspace
-  T* sDT = sST + L::kST;               // D^T [v][token] on its way to the workspace
-  float* sSc = reinterpret_cast<float*>(sDT + L::kDT);  // [2][Scal::SIZE]
+  T* sST = sO + (NOW ? 0 : L::kV);                 // entering state, transposed [v][dk], for the output waves and on its way to the workspace
+  T* sDT = sST + L::NST * L::kST;      // D^T [v][token], likewise
+  float* sSc = reinterpret_cast<float*>(OUT ? sDT + L::NST * L::kDT : sP);  // [2][L::SCS]
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int N = p.geom.N;
@@ -135,9 +160,9 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
   const SeqSpan span = seq_span(p.geom, seq, c0);
   const int64_t tsk = (int64_t)p.geom.ts * DK, tsv = (int64_t)p.geom.ts * p.vcols, tso = (int64_t)p.geom.ts * p.dv;
 
-  if (wave >= NCW) {
+  if (wave >= NCW + NOW) {
     // ---------------- movers ----------------
-    const int mt = tid - 64 * NCW;
+    const int mt = tid - 64 * (NCW + NOW);
     typedef TileRegs<T, 64, DK, MT> RowTile;
     typedef TileRegs<T, 64, BV, MT> ValTile;
     struct Tiles {
@@ -152,24 +177,33 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     Tiles ta, tb;
     ta.g = ta.gc = ta.b = tb.g = tb.gc = tb.b = 0.f;
     ta.Tm.init(LDC, mt), ta.P.init(LDC, mt), tb.Tm.init(LDC, mt), tb.P.init(LDC, mt);
-    zero_upper_triangles<CHAIN>(sTm, 4, L::kC, LDC, mt);  // both buffers of Tm and Pm: the packed tiles never write there
+    zero_upper_triangles<CHAIN>(sTm, OUT ? 4 : 2, L::kC, LDC, mt);  // both buffers of Tm and Pm: the packed tiles never write there
     ta.len = tb.len = 0;
 #pragma unroll
     for (int it = 0; it < RowTile::IT; ++it) ta.fq[it] = tb.fq[it] = ta.nk[it] = tb.nk[it] = 0.f;
 #pragma unroll
     for (int it = 0; it < ValTile::IT; ++it) ta.bv[it] = tb.bv[it] = 0.f;
-    // part 0: K, 1: Q, 2: the rest; < 0: everything
-    auto fetch = [&](Tiles& R, int n, int part = -1) {
+    // part 0: K, 1: Q, 2: the rest; < 0: everything.  With output waves Q and Pm are those of the chunk before (part 1).
+    auto fetch = [&](Tiles& R, int n, int part = -1) __attribute__((always_inline)) {
+      if (NOW && part == 1) {
+        const int64_t slot = (int64_t)row * N + n - 1;
+        int tok0, len;
+        chunk_span(span, n - 1, tok0, len);
+        R.Q.load(p.q + tok_index(p.geom, row, tok0) * DK, tsk, len, mt);
+        R.P.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
+        return;
+      }
       const int64_t slot = (int64_t)row * N + n;
       int tok0;
       chunk_span(span, n, tok0, R.len);
       const int64_t tbase = tok_index(p.geom, row, tok0);
       if (part < 0 || part == 0) R.K.load(p.k + tbase * DK, tsk, R.len, mt);
-      if (part < 0 || part == 1) R.Q.load(p.q + tbase * DK, tsk, R.len, mt);
+      if (OUT && (part < 0 || part == 1)) R.Q.load(p.q + tbase * DK, tsk, R.len, mt);
       if (part == 0 || part == 1) return;
       R.V.load(p.v + tbase * p.vcols + v0, tsv, (v0 < p.vcols) ? R.len : 0, mt);  // columns v does not hold read as zero
       R.Tm.load(at<const T>(p.ws, p.off.Tm) + slot * 64 * 64, mt);
-      R.P.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
+      if (OUT && !NOW) R.P.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
+      if (NOW) return;
       // every thread loads the scalars of token mt % 64 (no load behind a branch); tokens past the end are masked below
       const int t = mt & 63;
       if (GATE == LNX_GATE_SCALAR) {
@@ -179,7 +213,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
       }
 #pragma unroll
       for (int it = 0; it < RowTile::IT; ++it) {
-        R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + MT * it) / RowTile::VPR];
+        if (OUT) R.fq[it] = at<const float>(p.ws, p.off.Fq)[slot * 64 + (mt + MT * it) / RowTile::VPR];
         R.nk[it] = at<const float>(p.ws, p.off.Nk)[slot * 64 + (mt + MT * it) / RowTile::VPR];
       }
       R.b = p.beta[tbase + (int64_t)min(t, R.len - 1) * p.geom.ts];
@@ -188,15 +222,19 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
         R.bv[it] = p.beta[tbase + (int64_t)min(min((mt + MT * it) / ValTile::VPR, 63), R.len - 1) * p.geom.ts];
     };
     // K rows normalised (their own bits where nothing is to be normalised), Q rows normalised and scaled by scale e^{G_i}
-    auto commit = [&](const Tiles& R, int pb, int part = -1) {
+    auto commit = [&](const Tiles& R, int n, int part = -1) __attribute__((always_inline)) {
+      const int pb = (n - c0) & 1;
+      const float* sc = sSc + ((n - c0) & (L::NSC - 1)) * L::SCS;               // NOW: the factors come from the output waves
+      const float* scq = sSc + ((n - 1 - c0) & (L::NSC - 1)) * L::SCS + Scal::FQ;
 #pragma unroll
       for (int it = 0; it < RowTile::IT; ++it) {
         const int idx = mt + MT * it, r = idx / RowTile::VPR, c = (idx - r * RowTile::VPR) * RowTile::N;
         if (part < 0 || part == 0)
-          S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), p.l2norm ? scaled(R.K.x[it], R.nk[it]) : R.K.x[it]);
-        if (part < 0 || part == 1)
-          S16::put<CHAIN>(sQ + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), scaled(R.Q.x[it], R.fq[it]));
+          S16::put<CHAIN>(sK + pb * L::kK + r * LDK + S16::pos<CHAIN>(c), p.l2norm ? scaled(R.K.x[it], NOW ? sc[Scal::NK + r] : R.nk[it]) : R.K.x[it]);
+        if (OUT && (part < 0 || part == 1))
+          S16::put<CHAIN>(sQ + (NOW ? pb ^ 1 : pb) * L::kK + r * LDK + S16::pos<CHAIN>(c), scaled(R.Q.x[it], NOW ? scq[r] : R.fq[it]));
       }
+      if (NOW && part == 1) R.P.store(sP + (pb ^ 1) * L::kC);
       if (part == 0 || part == 1) return;
       {  // V rows scaled by beta_i: R = beta V - (beta e^G) Y
         T* dst = sV + pb * L::kV;
@@ -204,20 +242,15 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
         for (int it = 0; it < ValTile::IT; ++it) {
           const int idx = mt + MT * it, r = idx / ValTile::VPR, c = (idx - r * ValTile::VPR) * ValTile::N;
           typename Vec16<T>::V x = R.V.x[it];
+          const float bt = NOW ? sc[Scal::BETA + min(r, 63)] : R.bv[it];
 #pragma unroll
-          for (int e = 0; e < ValTile::N; ++e) x[e] = (bf16_t)((float)x[e] * R.bv[it]);
+          for (int e = 0; e < ValTile::N; ++e) x[e] = (bf16_t)((float)x[e] * bt);
           if (idx < ValTile::TOTAL) *reinterpret_cast<typename Vec16<T>::V*>(dst + r * LDV + c) = x;
         }
       }
       R.Tm.store(sTm + pb * L::kC);
-      R.P.store(sP + pb * L::kC);
-      if (mt < 64) {
-        float* sc = sSc + pb * Scal::SIZE;
-        const float gam = (GATE == LNX_GATE_SCALAR) ? __expf(R.g) : 1.f;
-        sc[Scal::GAM + mt] = (mt < R.len) ? R.b * gam : 0.f;
-        sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) : 1.f;
-        if (mt == 0) sc[Scal::DEC] = (GATE == LNX_GATE_SCALAR) ? __expf(R.gc) : 1.f;
-      }
+      if (OUT && !NOW) R.P.store(sP + pb * L::kC);
+      if (!NOW && mt < 64) put_scalars<GATE>(sSc + pb * L::SCS, mt, mt < R.len ? R.b : 0.f, R.g, R.gc);
     };
     // cur: the register set that held chunk n (in LDS since the last step) and now takes chunk n + 2; nxt: chunk n + 1.
     // `steady` (a std::bool_constant): chunks n + 1 and n + 2 exist, so nothing below sits behind a branch -- behind a
@@ -225,60 +258,178 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     // The loads are admitted at the rate the memory path takes them, and a wave that has a load waiting for a slot
     // issues nothing else: so the tile writes of chunk n + 1 sit between the loads of chunk n + 2, a tile at a time, and
     // go out while the loads before them drain (issued one after the other: forward scan 237 -> 216 us).
-    auto step = [&](Tiles& cur, const Tiles& nxt, int n, auto steady) {
-      constexpr bool STEADY = decltype(steady)::value;
-      if constexpr (STEADY) {
-#pragma unroll
-        for (int part = 0; part < 3; ++part) {
-          fetch(cur, n + 2, part);
-          commit(nxt, (n + 1 - c0) & 1, part);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      } else {
-        if (n + 2 < c1) fetch(cur, n + 2);
-        if (n + 1 < c1) commit(nxt, (n + 1 - c0) & 1);
-      }
-      lds_barrier();  // Bmid
+    // with 512 movers: O and D are 256 vectors each, one half of the movers takes each
+    const bool lower = MT == 256 || mt < 256, upper = MT == 256 || mt >= 256;
+    auto out_o = [&](int n) {
       int tok0, len;
       chunk_span(span, n, tok0, len);
-      // with 512 movers: O and D are 256 vectors each, one half of the movers takes each
-      const bool lower = MT == 256 || mt < 256, upper = MT == 256 || mt >= 256;
-      const int ot = mt & 255;
-      if (p.o && lower) {
-        if constexpr (std::is_same<OT, float>::value)
-          unstage_tile_checked_widen<64, BV>(reinterpret_cast<float*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + v0, tso, sO, LDV, len, ot);
-        else
-          unstage_tile_checked<bf16_t, 64, BV>(reinterpret_cast<bf16_t*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + v0, tso, sO, LDV, len, ot);
-      }
-      if (p.save) {
-        const int64_t slot = (int64_t)row * N + n;
-        unstage_tile<T, BV, DK, true, MT>(at<T>(p.ws, p.off.SnT) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sST, LDS, BV, mt);
-        if (upper) unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT, LDD, BV, ot);
+      if constexpr (OUT && !NOW)
+        if (p.o && lower) {
+          const int ot = mt & 255;
+          if constexpr (std::is_same<OT, float>::value)
+            unstage_tile_checked_widen<64, BV>(reinterpret_cast<float*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + v0, tso, sO, LDV, len, ot);
+          else
+            unstage_tile_checked<bf16_t, 64, BV>(reinterpret_cast<bf16_t*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + v0, tso, sO, LDV, len, ot);
+        }
+    };
+    auto out_state = [&](int n) {
+      if constexpr (OUT)
+        if (p.save) {
+          const int64_t slot = (int64_t)row * N + n;
+          unstage_tile<T, BV, DK, true, MT>(at<T>(p.ws, p.off.SnT) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sST + (NOW ? ((n - c0) & 1) * L::kST : 0), LDS, BV, mt);
+          if (upper) unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT + (NOW ? ((n - c0) & 1) * L::kDT : 0), LDD, BV, mt & 255);
+        }
+    };
+    auto step = [&](Tiles& cur, const Tiles& nxt, int n, auto steady, auto write_first) __attribute__((always_inline)) {
+      constexpr bool STEADY = decltype(steady)::value, WRITE_FIRST = decltype(write_first)::value;
+      auto carry = [&](int part) __attribute__((always_inline)) {
+        const int lag = NOW && part == 1;
+        if (WRITE_FIRST && (STEADY || n + 1 - lag < c1)) commit(nxt, n + 1, part);
+        if (WRITE_FIRST) __builtin_amdgcn_sched_barrier(0);
+        if (STEADY || n + 2 - lag < c1) fetch(cur, n + 2, part);
+        if (!WRITE_FIRST && (STEADY || n + 1 - lag < c1)) commit(nxt, n + 1, part);
+        if (STEADY) __builtin_amdgcn_sched_barrier(0);
+      };
+      if (NOW && n > c0) out_state(n - 1);
+      carry(0);
+      if (OUT) carry(1);
+      carry(2);
+      if constexpr (OUT && !NOW) {
+        lds_barrier();  // Bmid
+        out_o(n);
+        out_state(n);
       }
       lds_barrier();  // B1 of the next chunk
     };
     // the register sets and the LDS double buffers alternate by position in the sequence (chunk c0: set a, buffer 0)
-    if (c0 < c1) {
-      fetch(ta, c0);
-      commit(ta, 0);
+    if constexpr (NOW || !OUT) {
+      if (c0 < c1) {
+        fetch(ta, c0, 0), fetch(ta, c0, 2);
+        if (NOW) lds_barrier();  // the first chunks' scalars are there
+        commit(ta, c0, 0), commit(ta, c0, 2);
+        if (OUT) fetch(tb, c0 + 1, 1);
+      }
+      if (c0 + 1 < c1) fetch(tb, c0 + 1, 0), fetch(tb, c0 + 1, 2);
+    } else {
+      if (c0 < c1) {
+        fetch(ta, c0);
+        commit(ta, c0);
+      }
+      if (c0 + 1 < c1) fetch(tb, c0 + 1);
     }
-    if (c0 + 1 < c1) fetch(tb, c0 + 1);
     lds_barrier();  // B1 of the first chunk
-    int n = c0;
-    for (; n + 3 < c1; n += 2) {  // chunks n + 2 and n + 3 exist
-      step(ta, tb, n, std::true_type{});
-      step(tb, ta, n + 1, std::true_type{});
-    }
-    for (; n < c1; n += 2) {
-      step(ta, tb, n, std::false_type{});
-      if (n + 1 < c1) step(tb, ta, n + 1, std::false_type{});
-    }
+    auto run = [&](auto write_first) __attribute__((always_inline)) {
+      int n = c0;
+      for (; n + 3 < c1; n += 2) {  // chunks n + 2 and n + 3 exist
+        step(ta, tb, n, std::true_type{}, write_first);
+        step(tb, ta, n + 1, std::true_type{}, write_first);
+      }
+      for (; n < c1; n += 2) {
+        step(ta, tb, n, std::false_type{}, write_first);
+        if (n + 1 < c1) step(tb, ta, n + 1, std::false_type{}, write_first);
+      }
+    };
+    // each SIMD has a wave of either order
+    if (NOW && MT == 512 && mt >= 256) run(std::true_type{});
+    else run(std::false_type{});
+    if (NOW && c0 < c1) out_state(c1 - 1);
     return;
   }
 
-  // ---------------- compute waves: wave w owns value columns [16 w, 16 w + 16) of the slab ----------------
-  const int vs = 16 * wave;
+  const int vs = 16 * (wave < NCW ? wave : wave - NCW);
   const int l16 = lane & 15, lr = S16::row(lane), g4 = S16::grp(lane);
+  constexpr int NK = DK / 32;  // 32-wide steps over dk
+  if constexpr (NOW > 0)
+    if (wave >= NCW) {
+      // ---------------- output waves: O^T = (Q~ S)^T + D^T Pm^T of a strip, lane = token ----------------
+      // S^T and D^T as the compute wave stored them are the operands that it has in registers.
+      auto acc_rows = [&](const T* tile, int ld, int ks) {
+        const T* r = tile + (vs + l16) * ld + 32 * ks + g4;
+        return S16::join(*reinterpret_cast<const bf16x4*>(r), *reinterpret_cast<const bf16x4*>(r + 8));
+      };
+      // They bring the scalars, too, the same from every output wave: those of chunk n + 2 go to LDS and those of chunk n + 3 are requested in
+      // chunk n.  No load behind a branch: past the end the last chunk's come again.
+      float b_ = 0.f, g_ = 0.f, gc_ = 0.f, nk_ = 0.f, fq_ = 0.f;  // beta (0 past the end), G, G_C, the factors of the K and Q rows
+      auto fetch_scalars = [&](int n) {
+        n = min(n, c1 - 1);
+        const int64_t slot = (int64_t)row * N + n;
+        int tok0, len;
+        chunk_span(span, n, tok0, len);
+        b_ = p.beta[tok_index(p.geom, row, tok0) + (int64_t)min(lane, len - 1) * p.geom.ts];
+        b_ = lane < len ? b_ : 0.f;
+        if (GATE == LNX_GATE_SCALAR) {
+          const float* G = at<const float>(p.ws, p.off.G) + slot * 64;
+          g_ = G[lane], gc_ = G[63];
+        }
+        nk_ = at<const float>(p.ws, p.off.Nk)[slot * 64 + lane];
+        fq_ = at<const float>(p.ws, p.off.Fq)[slot * 64 + lane];
+      };
+      auto commit_scalars = [&](int n) {
+        float* sc = sSc + ((n - c0) & (L::NSC - 1)) * L::SCS;
+        put_scalars<GATE>(sc, lane, b_, g_, gc_);
+        sc[Scal::NK + lane] = nk_, sc[Scal::FQ + lane] = fq_;
+      };
+      if (c0 < c1) {
+        fetch_scalars(c0), commit_scalars(c0);
+        fetch_scalars(c0 + 1), commit_scalars(c0 + 1);
+        fetch_scalars(c0 + 2);
+        lds_barrier();
+      }
+      lds_barrier();  // B1 of the first chunk
+      for (int n = c0; n < c1; ++n) {
+        commit_scalars(n + 2);
+        fetch_scalars(n + 3);
+        lds_barrier();  // B1 of the next chunk, or the end of the last
+        const int pb = (n - c0) & 1;
+        const T* sQc = sQ + pb * L::kK;
+        const T* sPc = sP + pb * L::kC;
+        int tok0, len;
+        chunk_span(span, n, tok0, len);
+        floatx4 o[4];
+        S16::Frag fq[2][4], pm[6];
+        auto load_q = [&](int ks) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) fq[ks & 1][i] = S16::load<CHAIN>(sQc + (16 * i + l16) * LDK + 32 * ks, lane);
+        };
+        S16::Frag b[NK];
+#pragma unroll
+        for (int ks = 0; ks < NK; ++ks) b[ks] = acc_rows(sST + pb * L::kST, LDS, ks);
+        load_q(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < NK; ++ks) {
+          if (ks + 1 < NK) {
+            load_q(ks + 1);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pm[i] = S16::load<CHAIN>(sPc + (16 * i + l16) * LDC, lane);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S16::mma(o[i], b[ks], fq[ks & 1][i]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 2; i < 4; ++i) pm[i + 2] = S16::load<CHAIN>(sPc + (16 * i + l16) * LDC + 32, lane);
+        const S16::Frag bd0 = acc_rows(sDT + pb * L::kDT, LDD, 0), bd1 = acc_rows(sDT + pb * L::kDT, LDD, 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S16::mma(o[i], bd0, pm[i]);
+        S16::mma(o[2], bd1, pm[4]);
+        S16::mma(o[3], bd1, pm[5]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int t = 16 * i + l16;
+          if constexpr (std::is_same<OT, float>::value) {  // fp32 outputs are rounded as the others and widened
+            const bf16x4 x = pack_bf16x4(o[i]);
+            o[i] = floatx4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+          }
+          if (t < len) store4(reinterpret_cast<OT*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + t * tso + v0 + vs + 4 * (lane >> 4), o[i]);
+        }
+      }
+      return;
+    }
+
+  // ---------------- compute waves: wave w owns value columns [16 w, 16 w + 16) of the slab ----------------
   floatx4 S[KT];
 #pragma unroll
   for (int ci = 0; ci < KT; ++ci) S[ci] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -294,11 +445,106 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
 #pragma unroll
       for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(S[ci][e]));
   }
+  auto store_state = [&](int n) {
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci) store_t(S[ci], sST + (NOW ? ((n - c0) & 1) * L::kST : 0) + vs * LDS + S16::row0(ci), LDS, lane);
+  };
+  if (NOW && c0 < c1) lds_barrier();
   lds_barrier();  // B1 of the first chunk
   // Every LDS read is issued well ahead of the product that consumes it (A fragments two steps ahead, the next
   // phase's first fragments and scalars during the current phase's last steps): a compute wave has nothing else to cover
   // the LDS latency with.  The scheduling fences pin that order.
-  constexpr int NK = DK / 32;  // 32-wide steps over dk
+  if constexpr (NOW || !OUT) {
+    for (int n = c0; n < c1; ++n) {
+      const int pb = (n - c0) & 1;
+      const T* sKc = sK + pb * L::kK;
+      const T* sVc = sV + pb * L::kV;
+      const T* sTc = sTm + pb * L::kC;
+      const float* sc = sSc + ((n - c0) & (L::NSC - 1)) * L::SCS;
+      // ---- Y = K S (lane = value column) ----
+      floatx4 y[4], d[4], sv[4];
+      S16::Frag fa[NK][4], tm[6];  // K rows; Tm as below
+      bf16x4 vr[4];
+      auto load_k = [&](int ks) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fa[ks][i] = S16::load<CHAIN>(sKc + (S16::row0(i) + lr) * LDK + 32 * ks, lane);
+      };
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = d[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      load_k(0), load_k(1);
+      if (NK > 2) load_k(NK > 2 ? 2 : 0);
+#pragma unroll
+      for (int ks = 0; ks < NK; ++ks) {
+        const S16::Frag b = S16::from_acc(S[2 * ks], S[2 * ks + 1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S16::mma(y[i], fa[ks][i], b);
+        if (ks == 0 && NK > 2) load_k(NK > 2 ? 3 : 0);
+        if (ks == (NK > 2 ? 1 : 0)) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) vr[i] = S16::rows4(sVc, LDV, S16::row0(i) + g4, vs, lane);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::GAM + S16::row0(i) + g4);
+        }
+        if (ks == (NK > 2 ? 2 : 1)) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) tm[i] = S16::load<CHAIN>(sTc + (S16::row0(i) + lr) * LDC, lane);
+#pragma unroll
+          for (int i = 2; i < 4; ++i) tm[i + 2] = S16::load<CHAIN>(sTc + (S16::row0(i) + lr) * LDC + 32, lane);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // ---- R = beta V - (beta e^G) Y, in place of Y; D = Tm R ----
+      auto form_r = [&](int i) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) y[i][u] = (float)vr[i][u] - sv[i][u] * y[i][u];
+      };
+      form_r(0), form_r(1);
+      const S16::Frag br0 = S16::from_acc(y[0], y[1]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S16::mma(d[i], tm[i], br0);
+      form_r(2), form_r(3);
+      const S16::Frag br1 = S16::from_acc(y[2], y[3]);
+      __builtin_amdgcn_sched_barrier(0);
+      S16::mma(d[2], tm[4], br1);
+      S16::mma(d[3], tm[5], br1);
+      if (NOW) store_state(n);  // read behind the next barrier: it fills the wait for D
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sv[i] = load4(sc + Scal::R + S16::row0(i) + g4);  // e^{G_C - G} for the state update
+      const float dec = (GATE == LNX_GATE_SCALAR) ? sc[Scal::DEC] : 1.f;
+      S16::Frag fu[2][KT];  // K^T fragments of the state update, [step][row tile of the state]
+      constexpr int AHEAD = KT < 6 ? KT : 6;
+#pragma unroll
+      for (int ci = 0; ci < AHEAD; ++ci) fu[0][ci] = S16::load_cols<CHAIN>(sKc, LDK, 0, ci, lane);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (OUT) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) store_t(d[i], sDT + pb * L::kDT + vs * LDD + S16::row0(i), LDD, lane);
+      }
+      const S16::Frag bu0 = S16::from_acc(d[0] * sv[0], d[1] * sv[1]), bu1 = S16::from_acc(d[2] * sv[2], d[3] * sv[3]);
+      if (GATE == LNX_GATE_SCALAR) {
+#pragma unroll
+        for (int ci = 0; ci < KT; ++ci) S[ci] *= dec;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // ---- S <- e^{G_C} S + K^T (e^{G_C - G} D) ----
+#pragma unroll
+      for (int ci = AHEAD; ci < KT; ++ci) fu[0][ci] = S16::load_cols<CHAIN>(sKc, LDK, 0, ci, lane);
+#pragma unroll
+      for (int ci = 0; ci < 4; ++ci) fu[1][ci] = S16::load_cols<CHAIN>(sKc, LDK, 32, ci, lane);
+#pragma unroll
+      for (int ci = 0; ci < 4; ++ci) S16::mma(S[ci], fu[0][ci], bu0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ci = 4; ci < KT; ++ci) fu[1][ci] = S16::load_cols<CHAIN>(sKc, LDK, 32, ci, lane);
+#pragma unroll
+      for (int ci = 4; ci < KT; ++ci) S16::mma(S[ci], fu[0][ci], bu0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ci = 0; ci < KT; ++ci) S16::mma(S[ci], fu[1][ci], bu1);
+      lds_barrier();  // B1 of the next chunk
+    }
+  } else {
   for (int n = c0; n < c1; ++n) {
     const int pb = (n - c0) & 1;
     const T* sKc = sK + pb * L::kK;
@@ -306,11 +552,8 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     const T* sVc = sV + pb * L::kV;
     const T* sTc = sTm + pb * L::kC;
     const T* sPc = sP + pb * L::kC;
-    const float* sc = sSc + pb * Scal::SIZE;
-    if (p.save) {
-#pragma unroll
-      for (int ci = 0; ci < KT; ++ci) store_t(S[ci], sST + vs * LDS + S16::row0(ci), LDS, lane);
-    }
+    const float* sc = sSc + pb * L::SCS;
+    if (p.save) store_state(n);
     // ---- Y = K S (lane = value column) and (Q~ S)^T (lane = token): the state fragments are the shared operand ----
     floatx4 y[4], o[4];
 #pragma unroll
@@ -417,6 +660,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
     for (int ci = 0; ci < KT; ++ci) S16::mma(S[ci], fu[1][ci], bu1);
     lds_barrier();  // B1 of the next chunk
   }
+  }
   float* out = p.sT_out.at(sidx, (int64_t)DK * p.dv) + v0 + vs + l16;
 #pragma unroll
   for (int ci = 0; ci < KT; ++ci)
@@ -426,11 +670,12 @@ __global__ __launch_bounds__((FScanL<DK, BVW>::threads)) void scan_fwd_kernel(Di
 
 template <int DK, int GATE, typename OT>
 int launch_scan_fwd(const DirectParams& p, int nstate, hipStream_t st) {
+  constexpr bool OUT = !std::is_void<OT>::value;
   // 32-column slabs (two compute waves) when 64-column ones would occupy at most half of the chip
   const bool narrow = lnx_narrow_slabs((int64_t)nstate * p.geom.H * (p.dv / 64), p.slab);
   auto k = narrow ? scan_fwd_kernel<DK, GATE, 32, OT> : scan_fwd_kernel<DK, GATE, 64, OT>;
-  const size_t b = narrow ? FScanL<DK, 32>::bytes : FScanL<DK, 64>::bytes;
-  const int bv = narrow ? 32 : 64, threads = narrow ? FScanL<DK, 32>::threads : FScanL<DK, 64>::threads;
+  const size_t b = narrow ? FScanL<DK, 32, OUT>::bytes : FScanL<DK, 64, OUT>::bytes;
+  const int bv = narrow ? 32 : 64, threads = narrow ? FScanL<DK, 32, OUT>::threads : FScanL<DK, 64, OUT>::threads;
   if (const int rc = lnx_lds_limit((const void*)k, b); rc != LNX_OK) return rc;
   lnx_profile_mark("chunk_scan", st);
   hipLaunchKernelGGL(k, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / bv)), dim3(threads), b, st, p);
@@ -1201,6 +1446,7 @@ int lnx_direct_scan_fwd(const DirectParams& p, int dk, int gate, int nstate, hip
     lnx_profile_mark(nullptr, st);
     return rc;
   }
+  if (!p.o && !p.save) return scan_fwd_by_shape<void>(p, dk, gate, nstate, st);
   return p.o_dtype == LNX_F32 ? scan_fwd_by_shape<float>(p, dk, gate, nstate, st) : scan_fwd_by_shape<bf16_t>(p, dk, gate, nstate, st);
 }
 

@@ -291,10 +291,11 @@ def _prefill_segments(B: int, H: int, T: int, dv: int, dk: int = 256, two_byte: 
 
     dk <= 128: the first pass has w = B H (dk + dv) / 64 workgroups per segment, so 256 / w segments fill the chip once.
     Segments of 16 chunks or more, but eight of them where the chip has room (a segment's step costs as much as two chunks).
-    The lines are where the measured gain starts, bf16 d128 unless said: 4 heads of 4096 tokens 90 -> 74 us (2048: 52 -> 62),
-    8 heads of 16384 332 -> 168, 16 heads (w = 64) of 8192 182 -> 158 (4096: 98 -> 101), 32 heads never.  The kernels that form
-    W and U prepare both passes: no gain at w = 64; fp32 4 heads of 4096 284 -> 194 us, bf16 per-channel gate 4 heads
-    of 8192 237 -> 163 (4096: 131 -> 133).  From 512 chunks on, w = 64 gains from a second round (32768 tokens: 541 -> 508).
+    The lines are where the gain starts, bf16 d128 unless said (both sides as they are now; where a call beside a line lost, as the line was
+    drawn): 4 heads of 4096 tokens 83 -> 62 us (2048: 52 -> 62), 4 heads of 16384 298 -> 107, 16 heads (w = 64) of 8192 170 -> 131 (4096:
+    98 -> 101), 32 heads never.  The kernels that form W and U prepare both passes: no gain at w = 64; fp32 4 heads of 4096
+    275 -> 175 us, bf16 per-channel gate 4 heads of 8192 228 -> 143 (4096: 131 -> 133).  From 512 chunks on, w = 64 gains from a second
+    round (32768 tokens: 806 -> 395).
 
     dk = 256, and rows that would have to be copied to become heads: at most an eighth of the CUs busy and every segment keeps >= 64 chunks
     (fewer heads of 512 values gain less than their longer preparation costs: 16 workgroups of 4096 tokens 196 -> 216 us)."""
