@@ -113,7 +113,7 @@ template <int N, typename F, typename G> __device__ __forceinline__ void mfma4_e
     for (int i = 0; i < N; ++i) *c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a(i)[r], b(i)[r], *c[i], 0, 0, 0);
 }
 // ... the block summed from zero: for the pairs' sums over channels, where one chain of 64 additions rounds the outputs by 1.5e-7 at RWKV-7's
-// decays and four chains of 16 by 1.1e-7 (all else exact).  In dplr_grad it costs four spilled registers, 750 -> 771 us, for dq 1.62 -> 1.15e-7,
+// decays and four chains of 16 by 1.1e-7 (all else exact).  In dplr_grad it took 750 -> 771 us, for dq 1.62 -> 1.15e-7,
 // dk 1.65 -> 1.19, da 2.2 -> 1.8, db 2.1 -> 1.7, dgk 2.7 -> 2.4.
 template <int N, typename F, typename G> __device__ __forceinline__ void mfma_block(floatx4* const (&c)[N], F&& a, G&& b) {
   floatx4 t[N];
@@ -183,23 +183,31 @@ template <typename T> struct Raw4;
 template <> struct Raw4<bf16_t> {
   bf16x4 x;
   __device__ __forceinline__ void load(const bf16_t* p) { x = *reinterpret_cast<const bf16x4*>(p); }
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int o) { x = __builtin_bit_cast(bf16x4, __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, 0)); }
   __device__ __forceinline__ floatx4 get() const { return floatx4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]}; }
 };
 template <> struct Raw4<float> {
   floatx4 x;
   __device__ __forceinline__ void load(const float* p) { x = load4(p); }
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int o) { x = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0)); }
   __device__ __forceinline__ floatx4 get() const { return x; }
 };
-// This lane's share of a row of 64, zeros where there is no such token (no load behind a branch: `base` is readable anyway)
+// This lane's share of a row of 64: of a tile, or of the token's row of a caller's tensor, zeros past the chunk's end.  Those go through a buffer
+// descriptor that ends there: as a choice at every use of a row the zeros were one VALU instruction in ten of dplr_grad and cost it its spilled
+// registers (B8 H16 T4096 forward and backward 2138 -> 2094 us).
 template <typename T> struct Row {
   Raw4<T> x[4];
-  bool ok;
-  __device__ __forceinline__ void load(const void* base, int64_t at, bool ok_ = true) {  // at: element of the lane's first channel
-    ok = ok_;
+  __device__ __forceinline__ void load(const void* base, int64_t at) {  // at: element of the lane's first channel
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb) x[cb].load(static_cast<const T*>(base) + (ok ? at + 16 * cb : 0));
+    for (int cb = 0; cb < 4; ++cb) x[cb].load(static_cast<const T*>(base) + at + 16 * cb);
   }
-  __device__ __forceinline__ floatx4 operator[](int cb) const { return ok ? x[cb].get() : zero4(); }
+  __device__ __forceinline__ void load(const void* base, const Slot& s, const Lane& w) {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(static_cast<const T*>(base) + s.tok * D), 0, s.len * D * (int)sizeof(T), 0x00020000);
+    const int o = (w.t * D + 4 * w.g) * (int)sizeof(T);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) x[cb].load(rsrc, o + 16 * cb * (int)sizeof(T));
+  }
+  __device__ __forceinline__ floatx4 operator[](int cb) const { return x[cb].get(); }
 };
 // What was read, not what it was converted to, is what a kernel short of registers keeps from here on
 template <typename T> __device__ __forceinline__ void keep_as_read(Row<T>& r) {
@@ -339,7 +347,7 @@ struct Gates {
 // The decays of a DIRECT block's tokens, one by one
 __device__ __forceinline__ void token_decays(const ChunkParams& p, const Slot& s, const Lane& w, floatx4 (&x)[4]) {
   Row<float> gk;
-  gk.load(p.gk, (s.tok + w.t) * D + 4 * w.g, w.t < s.len);
+  gk.load(p.gk, s, w);
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) {
     const floatx4 g = gk[cb];
@@ -370,14 +378,12 @@ template <typename T> struct Own {
   Row<T> q, k, a, b;
   Row<float> gk;
   __device__ __forceinline__ void load(const ChunkParams& p, const Slot& s, const Lane& w) { load_gates(p, s, w), load_rows(p, s, w); }
-  __device__ __forceinline__ void load_gates(const ChunkParams& p, const Slot& s, const Lane& w) { gk.load(p.gk, (s.tok + w.t) * D + 4 * w.g, w.t < s.len); }
+  __device__ __forceinline__ void load_gates(const ChunkParams& p, const Slot& s, const Lane& w) { gk.load(p.gk, s, w); }
   __device__ __forceinline__ void load_rows(const ChunkParams& p, const Slot& s, const Lane& w) {
-    const bool ok = w.t < s.len;
-    const int64_t at = (s.tok + w.t) * D + 4 * w.g;
-    q.load(p.q, at, ok);
-    a.load(p.a, at, ok);
-    b.load(p.b, at, ok);
-    k.load(p.k, at, ok);
+    q.load(p.q, s, w);
+    a.load(p.a, s, w);
+    b.load(p.b, s, w);
+    k.load(p.k, s, w);
   }
 };
 
@@ -458,7 +464,7 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
   Own<T> x;
   x.load(p, s, w);
   Row<T> v;
-  v.load(p.v, (s.tok + w.t) * D + g4, w.t < s.len);
+  v.load(p.v, s, w);
   floatx4 fq[4], fa[4];                // q P, a P of the token before
   floatx4 ab[3], ak[3], qb[3], qk[3];  // pairs with tokens of earlier blocks, by t
   Pairs m{zero4(), zero4(), zero4(), zero4()};  // and of the lane's own
@@ -708,7 +714,7 @@ __global__ __launch_bounds__(256) void dplr_r_kernel(ChunkParams p) {
   Row<float> x;
   Row<T> d;
   x.load(p.X, s.kept * TG + w.t * D + g4);
-  d.load(p.d_o, (s.tok + w.t) * D + g4, w.t < s.len);
+  d.load(p.d_o, s, w);
   put_row(tX, w, [&](int cb) { return x[cb]; });
   put_row(tO, w, [&](int cb) { return d[cb]; });
   lds_barrier();
@@ -737,8 +743,8 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   Own<T> x;
   x.load(p, s, w);
   Row<T> v, d_o;
-  v.load(p.v, (s.tok + w.t) * D + g4, w.t < s.len);
-  d_o.load(p.d_o, (s.tok + w.t) * D + g4, w.t < s.len);
+  v.load(p.v, s, w);
+  d_o.load(p.d_o, s, w);
   Row<float> h0, dC;
   h0.load(p.hT, s.st * TG + w.t * D + g4);
   dC.load(p.s1, s.win * TG + w.t * D + g4);
@@ -992,8 +998,8 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
     Row<float> h0, dC;
     dC.load(p.s1, wt);
     x.load_gates(p, s, w);
-    v.load(p.v, at, ok);
-    d_o.load(p.d_o, at, ok);
+    v.load(p.v, s, w);
+    d_o.load(p.d_o, s, w);
     u.load(p.s3, wt);
     du.load(p.s4, wt);
     h0.load(p.hT, ht);
@@ -1112,7 +1118,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
     }
   }
   keep_as_read(x.b), keep_as_read(x.k), keep_as_read(x.q), keep_as_read(x.a);
-  u.load(p.s3, wt), v.load(p.v, at, ok);  // again, ahead of their use: in between the registers are full
+  u.load(p.s3, wt), v.load(p.v, s, w);  // again, ahead of their use: in between the registers are full
   lds_barrier();
   // db, dk, relative to the end of the lane's block: the matrices with the contraction along t, first those of q, then those of a
   floatx4 db[4], dk[4], own[4];  // own: b db + k dk of the block's own pairs
@@ -1179,10 +1185,8 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) db[cb] *= e.s[cb], dk[cb] *= e.s[cb], own[cb] *= e.s[cb];
   Row<float> fl;
-  fl.load(p.dgk, at, ok);
-  int64_t again = at;
-  asm volatile("" : "+v"(again));  // its addresses are formed here
-  x.q.load(p.q, again, ok);
+  fl.load(p.dgk, ok ? at : 0);
+  x.q.load(p.q, s, w);
   lds_barrier();
   if (gates.direct) {
     float* mine = t1 + w.t * LD;
