@@ -221,6 +221,7 @@ struct DirectParams {
   int gate;
   int l2norm;  // q and k rows are normalised inside the kernels (factors from the prepare kernel in Nq, Nk)
   int slab;    // lnx_scan_args.test_scan_slab
+  int ident;   // forward scan: the states start as [0 | I], the identity from column vcols on (s0 is not read)
   float scale;
   char* ws;
   ChunkWs off;

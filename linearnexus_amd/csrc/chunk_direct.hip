@@ -433,7 +433,13 @@ __global__ __launch_bounds__((FScanL<DK, BVW, !std::is_void<OT>::value>::threads
   floatx4 S[KT];
 #pragma unroll
   for (int ci = 0; ci < KT; ++ci) S[ci] = floatx4{0.f, 0.f, 0.f, 0.f};
-  if (p.s0) {
+  if (!OUT && p.ident) {
+    const int r = v0 + vs + l16 - p.vcols;
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[ci][e] = S16::row0(ci) + g4 + e == r ? 1.f : 0.f;
+  } else if (p.s0) {
     const float* s0 = p.s0 + (int64_t)sidx * DK * p.dv + v0 + vs + l16;
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci)

@@ -40,6 +40,7 @@ struct FwdParams {
   int vcols;    // leading value columns present in v (its row length); the rest of the dv columns are zero
   int l2norm;   // chunk_prepare2<LITE>, kda_prepare: q and k rows are normalised as x / (|x| + 1e-6) inside the kernels
   int slab;     // lnx_scan_args.test_scan_slab
+  int ident;    // the states start as [0 | I], the identity from column vcols on (s0 is not read)
   // per-channel gate formed inside kda_prepare from the raw projection (lnx_scan_args.gate_raw): element type of q
   const void* graw;
   const float* gA;
@@ -1169,7 +1170,15 @@ __global__ __launch_bounds__(512) void chunk_scan_kernel(FwdParams p) {
 
   floatx16 S[RT][NT];
   frag_zero(S);
-  if (p.s0) {
+  if (p.ident) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          S[i][j][e] = srow + 32 * i + frag_row(e, lane) == v0 + scol + 32 * j + frag_col(lane) - p.vcols ? 1.f : 0.f;
+  } else if (p.s0) {
     const float* s0 = p.s0 + (int64_t)sidx * DK * p.dv + v0;
 #pragma unroll
     for (int i = 0; i < RT; ++i)
@@ -1218,7 +1227,7 @@ __global__ __launch_bounds__(512) void chunk_scan_kernel(FwdParams p) {
     lds_barrier();  // B2
 
     auto outputs = [&]() {
-      if (FUSE && has_tile) {
+      if (FUSE && has_tile && p.o) {
         // o = scale e^G (Q S) + P D for this slab
         floatx16 o[1][1];
         frag_zero(o);
@@ -1447,7 +1456,7 @@ DirectParams direct_params(const FwdParams& p, int gate) {
   d.q = reinterpret_cast<const bf16_t*>(p.q); d.k = reinterpret_cast<const bf16_t*>(p.k);
   d.v = reinterpret_cast<const bf16_t*>(p.v); d.beta = p.beta; d.s0 = p.s0; d.sT_out = p.sT_out;
   d.o = p.o; d.dv = p.dv; d.o_dtype = p.o_dtype; d.save = p.save; d.vcols = p.vcols; d.gate = gate;
-  d.l2norm = p.l2norm; d.slab = p.slab;
+  d.l2norm = p.l2norm; d.slab = p.slab; d.ident = p.ident;
   d.scale = p.scale; d.ws = p.ws; d.off = p.off;
   return d;
 }
@@ -1574,9 +1583,9 @@ int launch_direct_fwd(const lnx_scan_args* a, const FwdParams& p, int nstate, bo
 
 // The forward pass on a caller-chosen workspace (a->workspace is not looked at).  `reuse`: what the workspace already
 // holds, the sequence table, or after the same call but for v, dv and the states the value-independent tensors too.  `last`: where the last
-// sequence's final states go instead of into a->final_state.
+// sequence's final states go instead of into a->final_state.  `ident`: the states start as [0 | I], not as a->initial_state.
 enum Reuse { REUSE_NOTHING, REUSE_TABLE, REUSE_PREPARED };
-int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_bytes, hipStream_t st, Reuse reuse = REUSE_NOTHING, float* last = nullptr) {
+int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_bytes, hipStream_t st, Reuse reuse = REUSE_NOTHING, float* last = nullptr, bool ident = false) {
   const bool packed = a->cu_seqlens != nullptr;
   const int nstate = packed ? a->nseq : a->B;
   if (nstate == 0) return LNX_OK;
@@ -1608,6 +1617,7 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
   p.save = !(a->forward_only && a->dtype == LNX_BF16);
   p.out_spw = a->test_out_slabs;
   p.slab = a->test_scan_slab;
+  p.ident = ident;
   p.graw = a->gate == LNX_GATE_VECTOR ? a->gate_raw : nullptr; p.gA = a->gate_A_log; p.gbias = a->gate_bias; p.gthr = a->gate_threshold;
   p.vcols = a->value_cols ? a->value_cols : a->dv;
   p.l2norm = a->use_qk_l2norm;
@@ -1629,8 +1639,8 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
 }
 
 // ---------------------------------------------------------------------------------------
-// A long sequence in segments (lnx_chunk_fwd_segmented).  setup: cu_seqlens of the segments, the slot table that build_table_kernel
-// would make of it (one launch of 4.5 us less) and their states [0 | I].
+// A long sequence in segments (lnx_chunk_fwd_segmented).  setup: cu_seqlens of the segments and the slot table that
+// build_table_kernel would make of it (one launch of 4.5 us less).  The scans start from [0 | I] by themselves.
 // chain: s_in[0] = s0, s_in[i + 1] = B_i + A_i s_in[i], where segment i left [B_i | A_i] in ab [n, H, dk, dv + dk].
 // One workgroup per (head, 16 value columns): the columns stay in LDS (transposed) for all segments, wave w forms rows
 // 16 w .. on the fp32 matrix cores (16x16x4).  A step is a serial chain: barrier, the columns from LDS, 32 products a wave with two waves
@@ -1639,22 +1649,18 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
 // of them they held the first product up.  16 segments of 4 heads d128 43.8 -> 37.3 us (with four sets in flight but in front 43.8, with
 // four waves of two row tiles 40.4), where a batched library product and two copies per step took 310.
 // ---------------------------------------------------------------------------------------
-__global__ void segment_setup_kernel(int32_t* cu, int32_t* tab, int N, int n, int seg, int T, float* ab, int dk, int dv, int64_t total) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i <= n) cu[i] = min((int)i * seg, T), tab[2 * N + i] = (cu[i] + LNX_C - 1) / LNX_C;
-  if (i < n) tab[2 * N + n + 1 + i] = (int)i;  // no segment is longer than one before it
-  for (int64_t c = i; c < N; c += (int64_t)gridDim.x * 256) {  // segments are whole chunks: slot c is chunk c of the sequence
-    const int t0 = (int)min(c * LNX_C, (int64_t)T);
+__global__ void segment_setup_kernel(int32_t* cu, int32_t* tab, int N, int n, int seg, int T) {
+  const int first = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+  for (int i = first; i <= n; i += step) {
+    const int t = (int)min((int64_t)i * seg, (int64_t)T);
+    cu[i] = t, tab[2 * N + i] = (t + LNX_C - 1) / LNX_C;
+    if (i < n) tab[2 * N + n + 1 + i] = i;  // no segment is longer than one before it
+  }
+  for (int c = first; c < N; c += step) {  // segments are whole chunks: slot c is chunk c of the sequence
+    const int t0 = (int)min((int64_t)c * LNX_C, (int64_t)T);
     tab[2 * c] = t0 < T ? t0 : 0;
     tab[2 * c + 1] = min(LNX_C, T - t0);
   }
-  const int w = (dk + dv) / 4;
-  if (i >= total / 4) return;
-  const int c = 4 * (int)(i % w), r = (int)((i / w) % dk);
-  floatx4 x;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) x[e] = c + e - dv == r ? 1.f : 0.f;
-  store4(ab + 4 * i, x);
 }
 
 template <int DK> constexpr int segment_chain_threads = DK == 64 ? 256 : 512;
@@ -1821,13 +1827,13 @@ static int fwd_segmented(const lnx_scan_args* a, int32_t nseg, bool every_state,
   char* ws = reinterpret_cast<char*>(a->workspace);
   int32_t* cu = reinterpret_cast<int32_t*>(ws + g.cu);
   float *ab = reinterpret_cast<float*>(ws + g.ab), *s_in = reinterpret_cast<float*>(ws + g.s_in);
-  const int64_t total = (int64_t)g.n * a->H * a->dk * (a->dv + a->dk);
-  hipLaunchKernelGGL(segment_setup_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, st, cu,
-                     reinterpret_cast<int32_t*>(ws + lnx_chunk_ws_layout(&g.first).tab), lnx_chunk_slots(&g.first), g.n, g.seg, a->T, ab, a->dk, a->dv, total);
+  const int slots = lnx_chunk_slots(&g.first);
+  hipLaunchKernelGGL(segment_setup_kernel, dim3((unsigned)std::min((slots + 255) / 256, 64)), dim3(256), 0, st, cu, reinterpret_cast<int32_t*>(ws + lnx_chunk_ws_layout(&g.first).tab),
+                     slots, g.n, g.seg, a->T);
   g.first.cu_seqlens = g.second.cu_seqlens = cu;
-  g.first.initial_state = ab, g.first.final_state = ab;  // every workgroup of the scan reads its columns before it writes them
+  g.first.final_state = ab;
   g.second.initial_state = s_in;
-  if ((rc = chunk_fwd_on(&g.first, ws, g.ws_bytes, st, REUSE_TABLE)) != LNX_OK) return rc;
+  if ((rc = chunk_fwd_on(&g.first, ws, g.ws_bytes, st, REUSE_TABLE, nullptr, true)) != LNX_OK) return rc;
   auto chain = a->dk == 256 ? segment_chain_kernel<256> : a->dk == 128 ? segment_chain_kernel<128> : segment_chain_kernel<64>;
   lnx_profile_mark("segment_chain", st);
   hipLaunchKernelGGL(chain, dim3(a->H, a->dv / 16), dim3(a->dk == 64 ? 256 : 512), 0, st, ab, a->initial_state, s_in, g.n, a->H, a->dv);

@@ -180,6 +180,14 @@ template <int NC> struct Strip {
 #pragma unroll
         for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(x[c][ci][e]));
   }
+  __device__ __forceinline__ void identity(int first, int lane) {  // of the columns from `first` on, the strip's first one
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int ci = 0; ci < KT; ++ci)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[c][ci][e] = row0(ci) + grp(lane) + e == first + 16 * c + (lane & 15) ? 1.f : 0.f;
+  }
   __device__ __forceinline__ void store(float* dst, int dv, int lane) const {
 #pragma unroll
     for (int c = 0; c < NC; ++c)
@@ -223,6 +231,7 @@ __device__ __forceinline__ void put_t(T* sT, int ld, int col, const Frag (&b)[2]
 template <int GATE, int NC, int NCW, typename OT>
 __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kernel(DirectParams p) {
   typedef WideL<NC, NCW> L;
+  constexpr bool OUT = !std::is_void<OT>::value;  // void: final states alone (forward only): no Q, no Pm, nothing saved
   constexpr int BV = L::BV, LDK = L::LDK, LDC = L::LDC, LDV = L::LDV, LDT = L::LDT;
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);
@@ -255,20 +264,22 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
       int tok0, len;
       chunk_span(ch.span, n, tok0, len);
       const int64_t tbase = tok_index(p.geom, ch.row, tok0);
-      rQ.load(p.q + tbase * DK, tsk, len, mt);
-      fq.load(at<const float>(p.ws, p.off.Nq) + slot * 64, mt);
+      if constexpr (OUT) {
+        rQ.load(p.q + tbase * DK, tsk, len, mt);
+        fq.load(at<const float>(p.ws, p.off.Nq) + slot * 64, mt);
+      }
       rV.load(p.v + tbase * p.vcols + v0, tsv, (v0 < p.vcols) ? len : 0, mt);  // columns v does not hold read as zero
       rTm.load(at<const T>(p.ws, p.off.Tm) + slot * 64 * 64, mt);
-      rP.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
+      if constexpr (OUT) rP.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
       rs.load(p, slot, tbase, len, mt);
       rK.load(p.k + tbase * DK, tsk, len, mt);
       fk.load(at<const float>(p.ws, p.off.Nk) + slot * 64, mt);
     };
     auto commit = [&]() {
-      store_rows(rQ, fq, p.l2norm, sQ, LDK, mt);
+      if constexpr (OUT) store_rows(rQ, fq, p.l2norm, sQ, LDK, mt);
       rV.store(sV, LDV, mt);
       rTm.store(sTm);
-      rP.store(sP);
+      if constexpr (OUT) rP.store(sP);
     };
     auto commit_k = [&]() {  // the scalars with it: the last product's decay is read until here
       store_rows(rK, fk, p.l2norm, sK, LDK, mt);
@@ -288,7 +299,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
       chunk_span(ch.span, n, tok0, len);
       if (std::is_same<OT, T>::value && p.o)
         unstage_tile_checked<T, 64, BV>(reinterpret_cast<T*>(p.o) + tok_index(p.geom, ch.row, tok0) * p.dv + v0, tso, sO, LDV, len, mt);
-      if (p.save) unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT, LDT, BV, mt);
+      if (OUT && p.save) unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT, LDT, BV, mt);
       commit();
       lds_barrier();  // B3
       commit_k();
@@ -300,9 +311,10 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
   // ---------------- compute waves: wave w owns value columns [16 NC w, 16 NC (w + 1)) of the slab ----------------
   const int vs = 16 * NC * wave;
   Strip<NC> S;
-  S.load(p.s0 ? p.s0 + (int64_t)ch.sidx * DK * p.dv + v0 + vs : nullptr, p.dv, lane);
+  if (!OUT && p.ident) S.identity(v0 + vs - p.vcols, lane);
+  else S.load(p.s0 ? p.s0 + (int64_t)ch.sidx * DK * p.dv + v0 + vs : nullptr, p.dv, lane);
   auto save = [&](int n) {
-    if (p.save) S.save(at<T>(p.ws, p.off.SnT) + ((int64_t)ch.row * N + n) * p.dv * DK + (int64_t)(v0 + vs) * DK, fresh(tid & 63));
+    if (OUT && p.save) S.save(at<T>(p.ws, p.off.SnT) + ((int64_t)ch.row * N + n) * p.dv * DK + (int64_t)(v0 + vs) * DK, fresh(tid & 63));
   };
   if (c0 < c1) save(c0);
   lds_barrier();  // B1 of the first chunk
@@ -370,11 +382,11 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
       }
     }
 #pragma unroll
-    for (int c = 0; c < NC; ++c) put_t(sDT, LDT, vs + 16 * c, bd[c], lane);
+    for (int c = 0; c < (OUT ? NC : 0); ++c) put_t(sDT, LDT, vs + 16 * c, bd[c], lane);
     __builtin_amdgcn_sched_barrier(0);
     // ---- O^T = scale e^G (Q S)^T + D^T Pm^T: columns = tokens, 32 of them at a time ----
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < (OUT ? 2 : 0); ++h) {
       const int lane = fresh(tid & 63);
       floatx4 o[NC][2];
 #pragma unroll
@@ -408,10 +420,12 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
         if constexpr (std::is_same<OT, T>::value) {
 #pragma unroll
           for (int c = 0; c < NC; ++c) store4(sO + t * LDV + vs + 16 * c + 4 * (lane >> 4), o[c][i]);
-        } else if (p.o && t < len) {
+        } else if constexpr (OUT) {
+          if (p.o && t < len) {
 #pragma unroll
-          for (int c = 0; c < NC; ++c)
-            store4(reinterpret_cast<float*>(p.o) + (tok_index(p.geom, ch.row, tok0) + (int64_t)t * p.geom.ts) * p.dv + v0 + vs + 16 * c + 4 * (lane >> 4), o[c][i]);
+            for (int c = 0; c < NC; ++c)
+              store4(reinterpret_cast<float*>(p.o) + (tok_index(p.geom, ch.row, tok0) + (int64_t)t * p.geom.ts) * p.dv + v0 + vs + 16 * c + 4 * (lane >> 4), o[c][i]);
+          }
         }
       }
     }
@@ -622,6 +636,7 @@ template <typename K> int launch(K k, size_t bytes, int bv, int threads, const c
 template <int GATE, int NC, int NCW> int launch_width(bool bwd, const DirectParams& p, int nstate, hipStream_t st) {
   typedef WideL<NC, NCW> L;
   if (bwd) return launch(wide_scan_bwd_kernel<GATE, NC, NCW>, L::bytes, L::BV, L::threads, "bwd_scan", p, nstate, st);
+  if (!p.o && !p.save) return launch(wide_scan_fwd_kernel<GATE, NC, NCW, void>, L::bytes, L::BV, L::threads, "chunk_scan", p, nstate, st);
   if (p.o_dtype == LNX_BF16) return launch(wide_scan_fwd_kernel<GATE, NC, NCW, bf16_t>, L::bytes, L::BV, L::threads, "chunk_scan", p, nstate, st);
   return launch(wide_scan_fwd_kernel<GATE, NC, NCW, float>, L::bytes, L::BV, L::threads, "chunk_scan", p, nstate, st);
 }
