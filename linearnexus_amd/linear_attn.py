@@ -316,17 +316,19 @@ def _prefill_segments(B: int, H: int, T: int, dv: int, dk: int = 256, two_byte: 
 
 
 def _prefill_segments_256(B: int, H: int, T: int, dv: int) -> int:
-    """The same for dk = 256 in bf16 without a per-channel gate, where the second pass finds everything prepared.  A chain takes 3.3 - 6.5 us
-    a chunk and cutting about two of them more work, so it pays from 64 chunks on while w <= 64 and from 128 on while w <= 128 (H4 dv 512,
-    w = 48: 2048 tokens 115 -> 134 us, 4096 216 -> 185, 8192 419 -> 274; H8 dv 512, w = 96: 4096 219 -> 236, 8192 427 -> 384).  Eight segments;
-    four where w or a short prompt leaves them too little (w = 48, 4096 tokens: 185 against 199 us; w = 96, 16384: 687 against 715), sixteen
-    of few heads and long prompts (w = 12, 16384: 297 against 314; w = 24, 32768: 496 against 540)."""
+    """The same for dk = 256 in bf16 without a per-channel gate, where the first pass forms no outputs and the second finds everything prepared.
+    A chain takes 3.3 us a chunk, cutting costs a setup and a short step per segment, so it pays from 32 chunks on while w <= 64 (H4 dv 512,
+    w = 48: 2048 tokens 117 -> 110 us, 4096 217 -> 153, 8192 420 -> 206) and from 64 on while w <= 128 (H8 dv 512, w = 96: 2048 tokens
+    117 -> 122, 4096 221 -> 174, 8192 427 -> 278; H16 dv 256, w = 128: 4096 227 -> 181), never beyond (H12 dv 512, w = 144:
+    8192 tokens 437 -> 495).  Eight segments; four where w or a short prompt leaves
+    them too little (2048 tokens, w = 24: 108 against 120 us; w = 96, 8192: 278 against 307), sixteen of few heads and long prompts
+    (16384 tokens, w = 24: 265 against 274; w = 48: 367 against 309)."""
     chunks, w = -(-T // CHUNK), B * H * (4 + -(-dv // 64))
     if os.environ.get("LNX_PREFILL_SEGMENTS") is not None:
         return _prefill_segments(B, H, T, dv)
-    if w > 128 or chunks < (64 if w <= 64 else 128):
+    if w > 128 or chunks < (32 if w <= 64 else 64):
         return 1
-    return 4 if w > 64 or (w > 24 and chunks < 128) else 16 if 3 * chunks >= 64 * w else 8
+    return 4 if w > 64 or chunks < 64 else 16 if w <= 24 and chunks >= 256 else 8
 
 
 def _segmented_forward(q, k, v, g, beta, scale, initial_state, l2norm, o_dtype, nseg):

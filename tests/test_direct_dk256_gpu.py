@@ -14,8 +14,9 @@ from test_chunk_bwd_gpu import _prep, check, gpu_grads
 from test_chunk_fwd_gpu import gpu_chunk_fwd, oracle_fwd
 
 
-@pytest.mark.parametrize("H,T,dv,expected", [(4, 4032, 512, 1), (4, 4033, 512, 4), (2, 4096, 512, 8), (5, 4096, 512, 4), (5, 8192, 512, 8), (6, 4096, 512, 1),
-                                             (6, 8192, 512, 4), (10, 8192, 512, 4), (11, 65536, 512, 1), (1, 16384, 512, 16), (2, 16384, 512, 8), (2, 32768, 512, 16)])
+@pytest.mark.parametrize("H,T,dv,expected", [(4, 1984, 512, 1), (4, 1985, 512, 4), (4, 4032, 512, 4), (4, 4033, 512, 8), (5, 4096, 512, 8), (6, 4032, 512, 1),
+                                             (6, 4096, 512, 4), (10, 8192, 512, 4), (11, 65536, 512, 1), (1, 16320, 512, 8), (2, 16384, 512, 16),
+                                             (3, 32768, 512, 8)])
 def test_segment_rule(monkeypatch, H, T, dv, expected):
     monkeypatch.delenv("LNX_PREFILL_SEGMENTS", raising=False)
     assert _prefill_segments_256(1, H, T, dv) == expected
