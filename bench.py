@@ -90,7 +90,7 @@ def measured_traffic(workload, kernel):
 def chunk_flops(dk, dv, direct=False):
     """Dense-product FLOPs per (batch, head, chunk) that each kernel performs.  In the WY split the forward
     terms add up to F_chunk = 2C^2(3dk+2dv) + 6C*dk*dv and the backward terms to 2*F_chunk; `direct` is the split of
-    the kernels for 2-byte inputs without a per-channel gate."""
+    the kernels for 2-byte inputs without a per-channel gate ("bwd_chunk" without it: see there)."""
     cc, cd = 2 * C * C, 2 * C * dk * dv
     if direct:
         return {
@@ -107,6 +107,8 @@ def chunk_flops(dk, dv, direct=False):
         "bwd_scan": 3 * cd,                           # K dS, Q^T dO, W^T dD
         "bwd_dqk": cc * dv + 3 * cd + 2 * cc * dk,    # dO D^T, dO S^T, dD S^T, D dS^T, dPe K, dPe^T Q
         "bwd_wy": cc * (4 * dk + 2 * dv),             # Tm^T dW, Tm^T dD, dBw W^T + dBu U^T, K K^T, Y K
+        # per-channel gate, 2-byte inputs, dk <= 128: in place of the two above
+        "bwd_chunk": 3 * cd + cc * (3 * dv + 4 * dk),  # dO S^T, dR S^T, D dS^T, Tm^T dD, dO D^T, dR D^T, the four pair sums
     }
 
 
@@ -274,7 +276,7 @@ def bench_chunk(args, torch, la, _lib, name):
     else:
         nchunks = B * H * (-(-T // C))
     avg = {n: sum(v_) / len(v_) for n, v_ in per_kernel.items()}
-    fl = chunk_flops(d, dv, direct="bwd_chunk" in avg)
+    fl = chunk_flops(d, dv, direct="bwd_chunk" in avg and variant != "kda")
     if "chunk_output" not in avg and "chunk_output" in fl:  # 2-byte inputs: the scan kernel also forms the outputs
         fl["chunk_scan"] += fl.pop("chunk_output")
     if "bwd_local" not in avg and "bwd_local" in fl:     # ... and the backward scan the chunk-local part of dD

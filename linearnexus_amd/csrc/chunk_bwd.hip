@@ -2,14 +2,15 @@
 // to q, k, v, beta, g and S_0, from the tensors lnx_chunk_fwd left in the workspace.  The
 // reference has no backward code (its gradients come from JAX autodiff of the recurrent scan,
 // linearnexus/train/sft.py:126-127); this is the hand-derived adjoint of the chunk algorithm of
-// gated_deltanet.py:444-523.  Four kernels:
+// gated_deltanet.py:444-523, for 4-byte inputs and the per-channel gate (chunk_direct.hip has the others).  Four kernels:
 //
 //   bwd_local  (chunk x dv-slab parallel)   dD_loc = P^T dO
 //   bwd_scan   (sequential, reverse)        dD = dD_loc + (K r) dS;  dS <- e^{G_last} dS + (Q~ e^G)^T dO - W^T dD
 //   bwd_dqk    (chunk parallel)             dP, dq, the P/K^r parts of dk, dW = -dD S^T, gate terms
 //   bwd_wy     (chunk parallel)             through W = Tm B_w, U = Tm B_u and Tm = (I + A)^-1:
 //                                           dv, dbeta, the remaining parts of dk, dg (reverse cumsum)
-// with r_j = exp(G_last - G_j), G the cumulative log-decay inside the chunk.
+// with r_j = exp(G_last - G_j), G the cumulative log-decay inside the chunk.  2-byte inputs with a per-channel gate and dk <= 128 take the
+// kernel of chunk_kda.hip in place of the last two.
 
 #include "chunk_common.h"
 #include "reduce_rows.h"

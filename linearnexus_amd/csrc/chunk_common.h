@@ -9,7 +9,7 @@
 // Per-slot tensors kept in the workspace (element type T = bf16 or fp32 unless noted), all
 // row-major with the token index first; kernels that contract over tokens read them through
 // the transposing LDS loads of mma_tiles.h, so no transposed copies are stored:
-//   G    fp32 [64] or [64][dk]   cumulative gate inside the chunk
+//   G    fp32 [64] or [64][dk]   cumulative gate inside the chunk (per-channel gate, 2-byte inputs, dk <= 128: [dk], its last row)
 //   P    [64][64]   scale * <q_i, k_j> * exp(G_i - G_j), i >= j
 //   W    [64][dk]   (I + A)^-1 diag(beta) (K * exp(G))
 //   U    [64][dv]   (I + A)^-1 diag(beta) V

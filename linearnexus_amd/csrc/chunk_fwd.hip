@@ -1,4 +1,5 @@
-// Chunked (WY) delta-rule forward on gfx950 MFMA, three kernels per call:
+// Chunked (WY) delta-rule forward on gfx950 MFMA for 4-byte inputs and the per-channel gate, three kernels per call (the scans for 2-byte inputs
+// without one are those of chunk_direct.hip and chunk_wide.hip, behind chunk_prepare2<LITE>), and what cuts a prompt into segments:
 //
 //   chunk_prepare2 (one workgroup per 64-token chunk, all chunks in parallel; kda_prepare for a vector gate)
 //       A = tril(diag(beta) K K^T * E, -1);  Tm = (I + A)^-1 (fp32, block forward substitution +
