@@ -1436,7 +1436,7 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
     k.beta = p.beta; k.dv = p.dv; k.l2norm = p.l2norm; k.scale = p.scale; k.ws = p.ws; k.off = p.off;
     k.d_o = reinterpret_cast<const bf16_t*>(p.d_o); k.dq = reinterpret_cast<bf16_t*>(p.dq); k.dk = reinterpret_cast<bf16_t*>(p.dk);
     k.dv_out = reinterpret_cast<bf16_t*>(p.dv_out); k.dbeta = p.dbeta; k.dg = p.dg;
-    k.g = p.g, k.graw = reinterpret_cast<const bf16_t*>(p.graw); k.gA = p.gA; k.gbias = p.gbias; k.gthr = p.gthr; k.gband = p.gband;
+    k.g = p.g, k.graw = reinterpret_cast<const bf16_t*>(p.graw); k.gA = p.gA; k.gbias = p.gbias; k.gthr = p.gthr;
     k.dgraw = reinterpret_cast<bf16_t*>(p.dgraw); k.gpart = p.gpart; k.gprows = p.gprows;
     return lnx_kda_bwd_chunk(k, DK, st);
   } else {

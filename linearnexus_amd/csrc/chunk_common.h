@@ -242,7 +242,6 @@ struct KdaBwdParams : DirectParams {
   const float* gA;
   const float* gbias;
   float gthr;
-  int gband;
   bf16_t* dgraw;
   float* gpart;
   int64_t gprows;

@@ -556,42 +556,7 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
       for (int e = 0; e < 4; ++e) dG[4 * t + e] += add;
       after += __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
     }
-    // With the gate activated inside the op, g = -e^{A_log} softplus(x), x = raw + bias (kda.py:153-165), the gradient goes on to the raw
-    // projection as bwd_wy2 (chunk_bwd.hip) explains: the activated gate is the difference of two rows of the cumulative gate, its derivative
-    // 1 - e^{-softplus}; x itself is read again only where the threshold is so low that it does not follow from softplus(x) (gband).
     settle16(dG);
-    if constexpr (GRAW) {
-      const int c = 64 * u + 16 * wave + l16;
-      const float inv_na = 1.f / gna;
-      float sb = 0.f, sa = 0.f;
-      unsigned above = 0;  // bit x: x beyond the threshold, read where it is used: the unusual case may wait
-      if (p.gband) {
-        const float gb = p.gbias ? p.gbias[(row % p.geom.H) * DK + c] : 0.f;
-#pragma unroll 1
-        for (int x = 0; x < 16; ++x) {
-          const int r = min(16 * (x >> 2) + 4 * kq + (x & 3), len - 1);
-          above |= (float)p.graw[(tbase + (int64_t)r * ts) * DK + c] + gb > p.gthr ? 1u << x : 0u;
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        // the token before this lane's four: the last of the group below, of the block below for group 0
-        const float below = __shfl(G[u][4 * t + 3], (lane - 16) & 63, LNX_WAVE), under = t ? __shfl(G[u][t ? 4 * t - 1 : 0], 48 + l16, LNX_WAVE) : 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int x = 4 * t + e, r = 16 * t + 4 * kq + e;
-          const float gv = G[u][x] - (e ? G[u][x - (e ? 1 : 0)] : kq ? below : under);
-          const float sp = gv * inv_na;
-          const bool lin = p.gband ? (above >> x & 1) != 0 : sp > p.gthr;
-          const float ds = lin ? 1.f : 1.f - __expf(-sp);
-          sa += r < len ? dG[x] * gv : 0.f;
-          dG[x] = r < len ? dG[x] * gna * ds : 0.f;
-          sb += dG[x];
-        }
-      }
-      sb = xor32_sum(xor16_sum(sb)), sa = xor32_sum(xor16_sum(sa));
-      if (kq == 0) gate_part(0)[c] = sb, gate_part(1)[c] = sa;
-    }
     if (u + 1 < NS) {
       float* sG0 = reinterpret_cast<float*>(region + L::oG0);
 #pragma unroll
@@ -650,20 +615,62 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
   }
   lds_barrier();  // dq and dk have left
   // ---- dg, or the raw projection's gradient, by rows ----
+  // With the gate activated inside the op, g = -e^{A_log} softplus(x), x = raw + bias (kda.py:153-165), the gradient goes on to the raw
+  // projection: dg g for A_log, -e^{A_log} sigmoid(x) dg (softplus' derivative is 1 beyond the threshold) for it and the bias.  The projection
+  // is read again here, by rows: as the difference of two rows of the cumulative gate, in the registers of the loop above, the activated gate
+  // cost shuffles and 21 spilled registers (B4 H16 T8192 d128: 643 us, so 544; 470 without the activation).
   float* sOut = reinterpret_cast<float*>(region);
 #pragma unroll
   for (int x = 0; x < 16; ++x) sOut[(16 * (x >> 2) + 4 * kq + (x & 3)) * L::LDF + 16 * wave + l16] = dG[x];
   lds_barrier();
+  float* sPart = reinterpret_cast<float*>(region + L::oP);  // GRAW: [set][which][wave][64]
 #pragma unroll
   for (int u = 0; u < NS; ++u) {
     const float* src = u + 1 < NS ? reinterpret_cast<const float*>(region + L::oG0) : sOut;
+    const int c = 4 * (tid & 15);  // the thread's channels of the set, in all its rows
+    bf16x4 raw[4];
+    floatx4 gb = {0.f, 0.f, 0.f, 0.f}, sb = gb, sa = gb;
+    if constexpr (GRAW) {
+#pragma unroll
+      for (int it = 0; it < 4; ++it) raw[it] = *reinterpret_cast<const bf16x4*>(p.graw + (tbase + (int64_t)min((tid >> 4) + 16 * it, len - 1) * ts) * DK + 64 * u + c);
+      if (p.gbias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) gb[e] = p.gbias[(row % p.geom.H) * DK + 64 * u + c + e];
+      }
+    }
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
-      const int idx = tid + 256 * it, r = idx >> 4, c = 4 * (idx & 15);
-      if (r < len) {
-        if constexpr (GRAW) store4(p.dgraw + (tbase + (int64_t)r * ts) * DK + 64 * u + c, load4(src + r * L::LDF + c));
-        else store4(p.dg + (tbase + (int64_t)r * ts) * DK + 64 * u + c, load4(src + r * L::LDF + c));
+      const int r = (tid >> 4) + 16 * it;
+      const int64_t o = (tbase + (int64_t)r * ts) * DK + 64 * u + c;
+      floatx4 d = load4(src + r * L::LDF + c);
+      if constexpr (GRAW) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = (float)raw[it][e] + gb[e], ex = __expf(-fabsf(x)), q = 1.f + ex;
+          const bool lin = x > p.gthr;
+          const float sp = lin ? x : fmaxf(x, 0.f) + __logf(q), ds = lin ? 1.f : __fdividef(x > 0.f ? 1.f : ex, q);
+          const float dr = r < len ? d[e] * gna : 0.f;
+          sa[e] += dr * sp;
+          d[e] = dr * ds;
+          sb[e] += d[e];
+        }
+        if (r < len) store4(p.dgraw + o, d);
+      } else if (r < len) {
+        store4(p.dg + o, d);
       }
+    }
+    if constexpr (GRAW) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sb[e] = xor32_sum(xor16_sum(sb[e])), sa[e] = xor32_sum(xor16_sum(sa[e]));
+      if (lane < 16) store4(sPart + (2 * u * 4 + wave) * 64 + c, sb), store4(sPart + ((2 * u + 1) * 4 + wave) * 64 + c, sa);
+    }
+  }
+  if constexpr (GRAW) {
+    lds_barrier();
+    if (tid < 2 * DK) {
+      const int which = tid / DK, c = tid % DK;
+      const float* x = sPart + (2 * (c >> 6) + which) * 256 + (c & 63);
+      gate_part(which)[c] = (x[0] + x[64]) + (x[128] + x[192]);
     }
   }
 }
