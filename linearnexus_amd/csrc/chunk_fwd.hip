@@ -452,6 +452,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   float* sG = reinterpret_cast<float*>(sQ + L::kTile);  // [64][LDF] cumulative gate of the half
   float* sA = sG + 64 * LDF;
   float* sT = sA + 64 * LNX_LDA;
+  T* sKb = reinterpret_cast<T*>(sA);  // LAST: beta K e^G [64][LDKB] from phase A to D
+  constexpr int LDKB = DK + L::PAD;
   float* sX = sT + 64 * LNX_LDA;
   float* sBeta = sX + 32 * 36;
   float* sNk = sBeta + 64;  // NORM: 1 / (|x| + eps) of the k and q rows
@@ -470,6 +472,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   const T* kg = reinterpret_cast<const T*>(p.k) + tbase * DK;
   const T* vg = reinterpret_cast<const T*>(p.v) + tbase * p.vcols;
   constexpr bool LAST = lnx_gate_last_only<T, DK>;
+  static_assert(!LAST || (LDKB * sizeof(T) <= LNX_LDA * sizeof(float) && LDF >= LNX_LDA), "the tiles change places");
   float* Gg = ws_ptr<float>(p, p.off.G) + (LAST ? gate_last<T, DK>(slot) : slot * 64 * DK);
   const int l16 = lane & 15, kq = lane >> 4;
 
@@ -601,11 +604,10 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       for (int i = 0; i < 16; ++i) sG[(16 * seg + i) * LDF + c] = gs[i] + off;
     }
     lds_barrier();
-    // G, K e^{G_last - G}, scale Q e^G of this half -> workspace.  LAST: of G only the last row, but beta K e^G, into the place of W, where
-    // phase D finds it: the rows of G were 32 KB written a chunk, and a second exponential of all of them in phase D (B4 H16 T8192 d128, forward
-    // and backward: 1568 -> 1528 us).
+    // G, K e^{G_last - G}, scale Q e^G of this half -> workspace.  LAST: of G only the last row, but beta K e^G for phase D into the tile that
+    // later held A, which goes to the gate's instead.  The rows of G were 32 KB written a chunk, and a second exponential of all of them in
+    // phase D (B4 H16 T8192 d128, forward and backward: 1568 us; beta K e^G through the place of W 1528, 16 KB that left and came back).
     {
-      T* Kbg = ws_ptr<T>(p, p.off.W) + slot * 64 * DK + 64 * h;
       T* Krg = ws_ptr<T>(p, p.off.Kr) + slot * 64 * DK + 64 * h;
       T* Qgg = ws_ptr<T>(p, p.off.Qg) + slot * 64 * DK + 64 * h;
 #pragma unroll
@@ -622,7 +624,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
           qgv[e] = qq[e] * p.scale * eg;
           kb[e] = kk[e] * bt * eg;
         }
-        if constexpr (LAST) store4(Kbg + r * DK + c, kb);
+        if constexpr (LAST) store4(sKb + r * LDKB + 64 * h + c, kb);
         else store4(Gg + r * DK + 64 * h + c, gr);
         store4(Krg + r * DK + c, kr);
         store4(Qgg + r * DK + c, qgv);
@@ -684,7 +686,10 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   // earlier stores have been acknowledged (the memory counter retires in order).
   int tid_late = threadIdx.x;
   asm volatile("" : "+v"(tid_late));
+  if (LAST) lds_barrier();  // the gate tile is dead: A takes it
+  float* sA_late = LAST ? sG : sA;
   {
+  float* const sA = sA_late;
   const int tid = tid_late, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, kq = lane >> 4;
   // ---- phase B: assemble X and <q, k>_E in sA / sT, write X and P, A = beta X, inverse ----
   if constexpr (LEVELS) {
@@ -759,8 +764,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
     }
   }
   // ---- phase D: W = Tm (beta e^G K), U = Tu V, one 64-column slab at a time ----
-  T* sIn = reinterpret_cast<T*>(sG);    // staged slab [token][col]
-  T* sOut = reinterpret_cast<T*>(sA);   // result slab on its way to the workspace
+  T* sIn = LAST ? sKb : reinterpret_cast<T*>(sG);  // staged slab [token][col]
+  T* sOut = reinterpret_cast<T*>(sA);              // result slab on its way to the workspace
   const int wi = wave >> 1, wj = wave & 1;
   const int nslab = NH + p.dv / 64;
   typedef TileRegs<T, 64, 64> Slab;
@@ -768,9 +773,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   Slab rIn;
   floatx4 rGs[LAST ? 1 : Slab::IT][VN / 4];  // K slabs: the gate values of exactly the elements this thread holds
   auto fetch_slab = [&](int s_) {
-    if (LAST && s_ < NH) {
-      rIn.load(ws_ptr<T>(p, p.off.W) + slot * 64 * DK + 64 * s_, DK, 64, tid);
-    } else if (s_ < NH) {
+    if (s_ < NH) {
       rIn.load(kg + 64 * s_, tsk, len, tid);
 #pragma unroll
       for (int it = 0; it < Slab::IT; ++it) {
@@ -783,13 +786,14 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       else rIn.zero();  // value columns that v does not hold
     }
   };
-  __syncthreads();  // G, or beta K e^G, is read back from the workspace by other threads than wrote it: global memory must be ordered too
-  fetch_slab(0);
+  if (!LAST) __syncthreads();  // G is read back from the workspace by other threads than wrote it: global memory must be ordered too
+  fetch_slab(LAST ? NH : 0);
 #pragma unroll 1
   for (int s_ = 0; s_ < nslab; ++s_) {
     const bool is_k = s_ < NH;
     lds_barrier();  // the previous slab's tiles (first pass: the inverse, the gate tile) are dead
-    if (is_k && !LAST) {  // K slab scaled by beta_t e^{G_t[c]} on its way into LDS
+    if (LAST && is_k) {  // in LDS since phase A
+    } else if (is_k) {   // K slab scaled by beta_t e^{G_t[c]} on its way into LDS
 #pragma unroll
       for (int it = 0; it < Slab::IT; ++it) {
         const int idx = tid + 256 * it, r = idx / Slab::VPR, c = (idx - r * Slab::VPR) * VN;
@@ -801,11 +805,14 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
     } else {
       rIn.store(sIn, LDC, tid);
     }
-    lds_barrier();
-    if (s_ + 1 < nslab) fetch_slab(s_ + 1);
+    if (!(LAST && is_k)) {
+      lds_barrier();
+      if (s_ + 1 < nslab) fetch_slab(s_ + 1);
+    }
     floatx16 o[1][1];
     frag_zero(o);
-    mma_x<T, 1, 1, false, true>(o, (is_k ? sTm : sTu) + 32 * wi * LDC, LDC, sIn + 32 * wj, LDC, 64, lane);
+    if (LAST && is_k) mma_x<T, 1, 1, false, true>(o, sTm + 32 * wi * LDC, LDC, sKb + 64 * s_ + 32 * wj, LDKB, 64, lane);
+    else mma_x<T, 1, 1, false, true>(o, (is_k ? sTm : sTu) + 32 * wi * LDC, LDC, sIn + 32 * wj, LDC, 64, lane);
     frag_store<T, 1, 1>(o, sOut + 32 * wi * LDC + 32 * wj, LDC, lane);
     lds_barrier();
     if (is_k)
