@@ -356,13 +356,15 @@ __device__ __forceinline__ void pair_mma(floatx4& acc, const PairOp& a, const Pa
   acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.lo, b.lo, acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, b.hi, acc, 0, 0, 0);
 }
+// e^x of a gate in natural units, or (LOG2) in units of log 2
+template <bool LOG2> __device__ __forceinline__ float gate_exp(float x) { return LOG2 ? __builtin_amdgcn_exp2f(x) : __expf(x); }
 // factors exp(-(ga - gb)) clamped to <= 1 (ga >= gb up to rounding: the cumulative gate does not increase)
-__device__ __forceinline__ void pair_factors(float (&F)[16], const float (&ga)[16], const float (&gb)[16]) {
+template <bool LOG2> __device__ __forceinline__ void pair_factors(float (&F)[16], const float (&ga)[16], const float (&gb)[16]) {
 #pragma unroll
-  for (int x = 0; x < 16; ++x) F[x] = __expf(fminf(gb[x] - ga[x], 0.f));
+  for (int x = 0; x < 16; ++x) F[x] = gate_exp<LOG2>(fminf(gb[x] - ga[x], 0.f));
 }
 
-__device__ __forceinline__ void kda_pair_half(floatx4 (&a32)[2], floatx4& a16, floatx4 (&aD)[5][2], const bf16_t* __restrict__ K,
+template <bool LOG2> __device__ __forceinline__ void kda_pair_half(floatx4 (&a32)[2], floatx4& a16, floatx4 (&aD)[5][2], const bf16_t* __restrict__ K,
                                               const bf16_t* __restrict__ Q, int ldc, const float* __restrict__ G, int ldf,
                                               int wave, int lane) {
   const int l16 = lane & 15, kq = lane >> 4;
@@ -375,9 +377,9 @@ __device__ __forceinline__ void kda_pair_half(floatx4 (&a32)[2], floatx4& a16, f
     pair_row_f32(gm, Gc + 32 * ldf);
     pair_row_f32(gi, Gc + i * ldf);
     pair_row_f32(gj, Gc + j * ldf);
-    pair_factors(F, gm, gi);  // exp(G_i - G_32)
+    pair_factors<LOG2>(F, gm, gi);  // exp(G_i - G_32)
     const PairOp kr = pair_scaled(pair_row_raw(Kc + i * ldc), F), qr = pair_scaled(pair_row_raw(Qc + i * ldc), F);
-    pair_factors(F, gj, gm);  // exp(G_32 - G_j)
+    pair_factors<LOG2>(F, gj, gm);  // exp(G_32 - G_j)
     const PairOp kc = pair_scaled(pair_row_raw(Kc + j * ldc), F);
     pair_mma(a32[0], kr, kc);
     pair_mma(a32[1], qr, kc);
@@ -388,9 +390,9 @@ __device__ __forceinline__ void kda_pair_half(floatx4 (&a32)[2], floatx4& a16, f
     pair_row_f32(gm, Gc + m * ldf);
     pair_row_f32(gi, Gc + i * ldf);
     pair_row_f32(gj, Gc + j * ldf);
-    pair_factors(F, gm, gi);
+    pair_factors<LOG2>(F, gm, gi);
     const PairOp r = pair_scaled(pair_row_raw(((wave & 1) ? Qc : Kc) + i * ldc), F);
-    pair_factors(F, gj, gm);
+    pair_factors<LOG2>(F, gj, gm);
     const PairOp kc = pair_scaled(pair_row_raw(Kc + j * ldc), F);
     pair_mma(a16, r, kc);
   }
@@ -404,10 +406,11 @@ __device__ __forceinline__ void kda_pair_half(floatx4 (&a32)[2], floatx4& a16, f
     for (int lv = 0; lv < 4; ++lv) {
       const int H = 8 >> lv;
       const bool up = (l16 & H) != 0;
+      const float sign = up ? 1.f : -1.f;
       const int m = 16 * wave + ((l16 & ~(2 * H - 1)) | H);
       pair_row_f32(gm, Gc + m * ldf);
 #pragma unroll
-      for (int x = 0; x < 16; ++x) F[x] = __expf(fminf(up ? gi[x] - gm[x] : gm[x] - gi[x], 0.f));
+      for (int x = 0; x < 16; ++x) F[x] = gate_exp<LOG2>(fminf((gi[x] - gm[x]) * sign, 0.f));
       const PairOp pk = pair_scaled(kraw, F), pq = pair_scaled(qraw, F);
       const unsigned mu = up ? 0xffffffffu : 0u;
       const PairOp kb = pair_masked(pk, ~mu);
@@ -479,6 +482,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   // ---- phase A: per 64-channel half ----
   TileRegs<T, 64, 64> rK, rQ;
   TileRegs<typename std::conditional<GRAW, T, float>::type, 64, 64> rG;
+  // LAST: the gate is held in units of log 2 (one product per element and not one per exponential, of which there are ten)
+  constexpr float LOG2E = 1.44269504f, UNIT = LAST ? LOG2E : 1.f;
   const float gna = GRAW ? -__expf(p.gA[row % p.geom.H]) : 0.f;
   typedef TileRegs<T, 64, 64> GT;
   float gbias[GRAW ? GT::N : 1];  // the bias of this thread's channel group (256 % VPR == 0: the same group in every pass)
@@ -592,7 +597,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       const int c = tid & 63, seg = tid >> 6;
       float gs[16];  // the segment's sixteen values in registers: all loads in flight together, one write each
 #pragma unroll
-      for (int i = 0; i < 16; ++i) gs[i] = sG[(16 * seg + i) * LDF + c];
+      for (int i = 0; i < 16; ++i) gs[i] = sG[(16 * seg + i) * LDF + c] * UNIT;
 #pragma unroll
       for (int i = 1; i < 16; ++i) gs[i] += gs[i - 1];
       float* sSeg = sX;  // segment totals [4][64] (the inverse's scratch is free here)
@@ -619,8 +624,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
         floatx4 kr, qgv, kb;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float eg = __expf(gr[e]);
-          kr[e] = kk[e] * __expf(fminf(gl[e] - gr[e], 0.f));
+          const float eg = gate_exp<LAST>(gr[e]);
+          kr[e] = kk[e] * gate_exp<LAST>(fminf(gl[e] - gr[e], 0.f));
           qgv[e] = qq[e] * p.scale * eg;
           kb[e] = kk[e] * bt * eg;
         }
@@ -629,10 +634,10 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
         store4(Krg + r * DK + c, kr);
         store4(Qgg + r * DK + c, qgv);
       }
-      if (LAST && tid < 16) store4(Gg + 64 * h + 4 * tid, load4(sG + 63 * LDF + 4 * tid));
+      if (LAST && tid < 16) store4(Gg + 64 * h + 4 * tid, load4(sG + 63 * LDF + 4 * tid) * (1.f / LOG2E));
     }
     if constexpr (LEVELS) {
-      kda_pair_half(a32, a16, aD, reinterpret_cast<const bf16_t*>(sK), reinterpret_cast<const bf16_t*>(sQ), LDC, sG, LDF, wave, lane);
+      kda_pair_half<LAST>(a32, a16, aD, reinterpret_cast<const bf16_t*>(sK), reinterpret_cast<const bf16_t*>(sQ), LDC, sG, LDF, wave, lane);
     } else {
     // blocks below the diagonal: six blocks x two products = twelve tasks, three per wave
 #pragma unroll

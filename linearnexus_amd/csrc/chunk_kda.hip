@@ -80,11 +80,11 @@ __device__ __forceinline__ void sums_cross(PairSums& s, const float (&g)[16], co
     const float ref = (H == 32 || t < 2) ? m0 : m1;
     // one exponential per four tokens, the others by the single-step decays: away from the reference the factors shrink
     if (up) {
-      F[4 * t] = __expf(fminf(g[4 * t] - ref, 0.f));
+      F[4 * t] = __builtin_amdgcn_exp2f(fminf(g[4 * t] - ref, 0.f));
 #pragma unroll
       for (int e = 1; e < 4; ++e) F[4 * t + e] = F[4 * t + e - 1] * dec[4 * t + e];
     } else {
-      F[4 * t + 3] = __expf(fminf(ref - g[4 * t + 3], 0.f));
+      F[4 * t + 3] = __builtin_amdgcn_exp2f(fminf(ref - g[4 * t + 3], 0.f));
 #pragma unroll
       for (int e = 2; e >= 0; --e) F[4 * t + e] = F[4 * t + e + 1] * dec[4 * t + e + 1];
     }
@@ -146,7 +146,7 @@ __device__ __forceinline__ void sums_diag(PairSums& s, const float (&g)[16], con
     if (H >= 4) {  // all four tokens share the role and the reference: one exponential, the rest by the single-step decays
       const bool up = H == 8 ? (kq & 2) != 0 : (kq & 1) != 0;
       const float ref = H == 8 ? of_group2(g[4 * t]) : of_odd_group(g[4 * t]);  // G of token 16 t + 8, or of the half block's fifth
-      const float f = __expf(fminf(up ? g[4 * t] - ref : ref - g[4 * t + 3], 0.f));
+      const float f = __builtin_amdgcn_exp2f(fminf(up ? g[4 * t] - ref : ref - g[4 * t + 3], 0.f));
       floatx4 F;
       F[0] = up ? f : f * d3 * d2 * d1;
       F[1] = up ? f * d1 : f * d3 * d2;
@@ -185,7 +185,7 @@ __device__ __forceinline__ void pair_sums(PairSums& s, const float (&g)[16], con
                                           const T* __restrict__ P, const T* __restrict__ A, int lane) {
   float dec[16];  // single-step decays exp(G_tok - G_{tok-1}) inside each group of four (the first entry of a group is unused)
 #pragma unroll
-  for (int x = 0; x < 16; ++x) dec[x] = (x & 3) ? __expf(fminf(g[x] - g[x - 1], 0.f)) : 1.f;
+  for (int x = 0; x < 16; ++x) dec[x] = (x & 3) ? __builtin_amdgcn_exp2f(fminf(g[x] - g[x - 1], 0.f)) : 1.f;
   // one part at a time: interleaving them multiplies the live factors
   s.settle();
   sums_cross<32>(s, g, dec, k4, q4, beta, P, A, lane);
@@ -414,7 +414,8 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
     dma16(p.k + (tbase + (int64_t)r * ts) * DK + c, slab0 + 1024 * (wave + 4 * u));
     dma16(p.q + (tbase + (int64_t)r * ts) * DK + c, slab0 + RowT::BYTES + 1024 * (wave + 4 * u));
   }
-  float G[NS][16];  // the gate of this lane's channels and tokens, later its cumulative sum
+  constexpr float LOG2E = 1.44269504f;
+  float G[NS][16];  // the gate of this lane's channels and tokens, later its cumulative sum in units of log 2: it is read by exponentials alone
 #pragma unroll
   for (int u = 0; u < NS; ++u)
 #pragma unroll
@@ -452,6 +453,7 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
       for (int e = 0; e < 4; ++e) {
         const int x = 4 * t + e;
         if constexpr (GRAW) G[u][x] = gna * lnx_softplus_thr(G[u][x] + gb, p.gthr);
+        G[u][x] *= LOG2E;
         G[u][x] = 16 * t + 4 * kq + e < len ? G[u][x] : 0.f;
         if (e) G[u][x] += G[u][x - (e ? 1 : 0)];
       }
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int x = 4 * t + e;
-        const float eg = __expf(G[u][x]), k2 = __expf(fminf(gC - G[u][x], 0.f)) * aK2[u][t][e], kv = (float)k4[t][e];
+        const float eg = __builtin_amdgcn_exp2f(G[u][x]), k2 = __builtin_amdgcn_exp2f(fminf(gC - G[u][x], 0.f)) * aK2[u][t][e], kv = (float)k4[t][e];
         s.rp[x] = p.scale * eg * aQ[u][t][e] + d4[e] * kv;
         s.ra[x] = -eg * aK1[u][t][e];
         s.co[x] = k2 + d4[e] * (float)q4[t][e];
@@ -538,7 +540,7 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
       for (int x = 0; x < 16; ++x) mv[x] = (float)k4[x >> 2][x & 3] * dk[u][x];
       channel_sum(mv, 2, u);
     }
-    tot = xor32_sum(xor16_sum(tot + __expf(gC) * ss[u]));  // over the tokens (ss: over its value columns) of this channel
+    tot = xor32_sum(xor16_sum(tot + __builtin_amdgcn_exp2f(gC) * ss[u]));  // over the tokens (ss: over its value columns) of this channel
     if (kq == 3) dG[15] += tot;
     // dg: reverse cumulative sum over the chunk's tokens of this channel
     float after = 0.f;  // what later blocks of sixteen tokens add
