@@ -348,10 +348,6 @@ __device__ __forceinline__ PairOp pair_scaled(const PairOp& x, const float (&F)[
   }
   return PairOp{__builtin_bit_cast(bf16x8, lo), __builtin_bit_cast(bf16x8, hi)};
 }
-__device__ __forceinline__ PairOp pair_masked(const PairOp& x, unsigned m) {
-  typedef unsigned uint4_ __attribute__((ext_vector_type(4)));
-  return PairOp{__builtin_bit_cast(bf16x8, __builtin_bit_cast(uint4_, x.lo) & m), __builtin_bit_cast(bf16x8, __builtin_bit_cast(uint4_, x.hi) & m)};
-}
 __device__ __forceinline__ void pair_mma(floatx4& acc, const PairOp& a, const PairOp& b) {
   acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.lo, b.lo, acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, b.hi, acc, 0, 0, 0);
@@ -412,10 +408,9 @@ template <bool LOG2> __device__ __forceinline__ void kda_pair_half(floatx4 (&a32
 #pragma unroll
       for (int x = 0; x < 16; ++x) F[x] = gate_exp<LOG2>(fminf((gi[x] - gm[x]) * sign, 0.f));
       const PairOp pk = pair_scaled(kraw, F), pq = pair_scaled(qraw, F);
-      const unsigned mu = up ? 0xffffffffu : 0u;
-      const PairOp kb = pair_masked(pk, ~mu);
-      pair_mma(aD[lv][0], pair_masked(pk, mu), kb);
-      pair_mma(aD[lv][1], pair_masked(pq, mu), kb);
+      // every pair of the block: which of them are a row token and a column token of this level is looked at when the sums are taken
+      pair_mma(aD[lv][0], pk, pk);
+      pair_mma(aD[lv][1], pq, pk);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -706,16 +701,10 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       sA[(16 * ti + il) * LNX_LDA + 16 * tj + l16] = a32[0][e];
       sT[(16 * ti + il) * LNX_LDA + 16 * tj + l16] = a32[1][e];
       d16[(16 * t16 + il) * LNX_LDA + 16 * (t16 - 1) + l16] = a16[e];
-      // diagonal block: level H keeps the pairs inside one 2H-token segment (the roles are in the operands already)
+      // diagonal block: a pair i > j is that of level H, the highest bit in which they differ (above the diagonal nobody reads)
       const int x = il ^ l16;
-      float va = aD[0][0][e], vp = aD[0][1][e];
-      va += (x < 8) ? aD[1][0][e] : 0.f;
-      vp += (x < 8) ? aD[1][1][e] : 0.f;
-      va += (x < 4) ? aD[2][0][e] : 0.f;
-      vp += (x < 4) ? aD[2][1][e] : 0.f;
-      va += (x < 2) ? aD[3][0][e] : 0.f;
-      vp += (x < 2) ? aD[3][1][e] : 0.f;
-      vp += (x == 0) ? aD[4][1][e] : 0.f;
+      const float va = x >= 8 ? aD[0][0][e] : x >= 4 ? aD[1][0][e] : x >= 2 ? aD[2][0][e] : aD[3][0][e];
+      const float vp = x >= 8 ? aD[0][1][e] : x >= 4 ? aD[1][1][e] : x >= 2 ? aD[2][1][e] : x == 1 ? aD[3][1][e] : aD[4][1][e];
       sA[(16 * wave + il) * LNX_LDA + 16 * wave + l16] = va;
       sT[(16 * wave + il) * LNX_LDA + 16 * wave + l16] = vp;
     }
