@@ -147,16 +147,8 @@ __device__ __forceinline__ void sums_diag(PairSums& s, const float (&g)[16], con
       const bool up = H == 8 ? (kq & 2) != 0 : (kq & 1) != 0;
       const float ref = H == 8 ? of_group2(g[4 * t]) : of_odd_group(g[4 * t]);  // G of token 16 t + 8, or of the half block's fifth
       const float f = __builtin_amdgcn_exp2f(fminf(up ? g[4 * t] - ref : ref - g[4 * t + 3], 0.f));
-      floatx4 F;
-      F[0] = up ? f : f * d3 * d2 * d1;
-      F[1] = up ? f * d1 : f * d3 * d2;
-      F[2] = up ? F[1] * d2 : f * d3;
-      F[3] = up ? F[2] * d3 : f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        fu[e] = up ? F[e] : 0.f;
-        fl[e] = up ? 0.f : F[e];
-      }
+      fu[0] = up ? f : 0.f, fu[1] = fu[0] * d1, fu[2] = fu[1] * d2, fu[3] = fu[2] * d3;
+      fl[3] = up ? 0.f : f, fl[2] = fl[3] * d3, fl[1] = fl[2] * d2, fl[0] = fl[1] * d1;
     } else if (H == 2) {  // reference: token 2 of the four
       fl = floatx4{d1 * d2, d2, 0.f, 0.f};
       fu = floatx4{0.f, 0.f, 1.f, d3};
@@ -427,7 +419,7 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
     }
   rdv = quad_sum(rdv);
   if ((tid & 3) == 0) sRdv[tid >> 2] = rdv;
-  if (!p.l2norm && tid < 64) sNq[tid] = sNk[tid] = 1.f;
+  if (tid < 64 && (!p.l2norm || tid >= len)) sNq[tid] = sNk[tid] = tid < len ? 1.f : 0.f;  // rows past the chunk's end are zero by their factor
 #pragma unroll
   for (int j = 0; j < 4; ++j)
     if (j <= wave) {
@@ -480,11 +472,7 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
       const floatx4 fk = load4(sNk + 16 * t + 4 * kq), fq = load4(sNq + 16 * t + 4 * kq);
       floatx4 kf, qf;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool on = 16 * t + 4 * kq + e < len;
-        kf[e] = on ? (float)k[e] * fk[e] : 0.f;
-        qf[e] = on ? (float)q[e] * fq[e] : 0.f;
-      }
+      for (int e = 0; e < 4; ++e) kf[e] = (float)k[e] * fk[e], qf[e] = (float)q[e] * fq[e];
       k4[t] = pack_bf16x4(kf), q4[t] = pack_bf16x4(qf);
     }
   };
