@@ -247,6 +247,8 @@ struct KdaBwdParams : DirectParams {
   int64_t gprows;
 };
 int lnx_kda_bwd_chunk(const KdaBwdParams& p, int dk, hipStream_t st);
+// The forward pass over the chunks with the state in registers, 32-column slabs.
+int lnx_kda_scan_fwd(const DirectParams& p, int dk, int nstate, hipStream_t st);
 int lnx_direct_scan_fwd(const DirectParams& p, int dk, int gate, int nstate, hipStream_t st);
 int lnx_direct_bwd(const DirectParams& p, int dk, int gate, int nstate, hipStream_t st);
 // The sequential passes for dk = 256 (chunk_wide.hip).

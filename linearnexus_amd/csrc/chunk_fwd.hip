@@ -1471,6 +1471,15 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   if (const int rc = lnx_lds_limit((const void*)k1, b1); rc != LNX_OK) return rc;
   lnx_profile_mark("chunk_prepare", st);
   hipLaunchKernelGGL(k1, dim3((unsigned)slots), dim3(256), b1, st, p);
+  // The chain in registers (kda_scan_fwd) where there are few slabs: at 2048 tokens, microseconds with chunk_scan -> with it,
+  // forward only / states saved as well, by the number of its workgroups (two to a 64-column slab):
+  //   dk = 128   8 .. 128: 57.5 -> 45 / 58.5 -> 49    192: 59.6 -> 46.3 / 87 -> 72    224: 71 -> 53.8 / 89.8 -> 87.5    240: 71.2 -> 59.6 / 91.3 -> 102    256: 74 -> 73 .. 79 / 93 -> 108
+  //   dk = 64    8 .. 128: 64 -> 36 / 66 -> 38.5      192: 67.5 -> 40.2 / 90.8 -> 64.3    224: 70.8 -> 55.3 / 91.3 -> 78.9    256: 72.2 -> 68 / 95 -> 88.5
+  // On a full chip the tiles come at the rate of HBM, and at dk = 128 its one chunk in flight is too little.
+  if constexpr (sizeof(T) == 2 && DK <= 128) {
+    const int64_t wide = (int64_t)nstate * p.geom.H * (p.dv / 64);
+    if (p.slab ? p.slab == 32 : wide <= (DK == 128 ? 112 : 128)) return lnx_kda_scan_fwd(direct_params(p, GATE), DK, nstate, st);
+  }
   // 32-column slabs when 64-column ones would occupy at most half of the chip (256 CUs); always for 4-byte inputs
   // with dk = 256, whose tiles leave no room in LDS for a wider slab
   constexpr bool can_narrow = (DK >= 128 && sizeof(T) == 2) || (DK == 128 && sizeof(T) == 4);

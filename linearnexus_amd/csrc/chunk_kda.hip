@@ -666,6 +666,279 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
   }
 }
 
+// ---------------------------------------------------------------------------------------
+// kda_scan_fwd: the forward pass over the chunks of one (state, 32-column slab of dv) where there are few of them and the
+// chain of a chunk is what a call waits for:  D = U - W S,  S <- diag(e^{G_C}) S + Kr^T D,  O = Qg S + P D.  chunk_scan
+// (chunk_fwd.hip) takes the chain through LDS between every two products, three barriers a chunk; here, as in scan_fwd
+// (chunk_direct.hip), a compute wave owns sixteen value columns, their part of the state stays in accumulators and is, like
+// D, an operand as it stands, and O has waves of its own a chunk behind.  What prepare leaves is an operand as it is, so no
+// wave converts anything: four waves request the tiles straight into LDS, four others take the states and D away.
+// One chunk: dk = 128 1.80 -> 1.38 us, dk = 64 1.99 -> 1.12 us.  Fetching lines ahead into the L2 by the idle savers (three
+// chunks ahead, for the full chip) made it slower: a prompt of four heads 192 -> 197 us, a saving scan 378 -> 408.
+//   B1    W, Kr, U of chunk n,   compute: D, state update; S^T and D^T -> LDS [n mod 2]   loads:  W, Kr, U of n + 1, Qg, P of n
+//         Qg, P of n - 1         output:  O of chunk n - 1; e^{G_C} of n + 1              savers: S, D of n - 1 -> workspace
+// ---------------------------------------------------------------------------------------
+template <int DK> struct KdaScanL {
+  typedef SwzTile<64, DK> RowT;  // W, Kr, Qg
+  typedef SwzTile<64, 32> ValT;  // U
+  typedef SwzTile<64, 64> TriT;  // P
+  typedef SwzTile<32, DK> StT;   // S^T
+  typedef SwzTile<32, 64> DtT;   // D^T
+  static constexpr int oKr = RowT::BYTES, oU = 2 * RowT::BYTES, first = oU + ValT::BYTES;  // W | Kr | U
+  static constexpr int oP = RowT::BYTES, second = oP + TriT::BYTES;                        // Qg | P
+  static constexpr int oSecond = 2 * first, oS = oSecond + 2 * second, oD = oS + 2 * StT::BYTES, oE = oD + 2 * DtT::BYTES;
+  static constexpr size_t bytes = oE + 2 * DK * sizeof(float);
+  static_assert(bytes <= 160 * 1024, "LDS");
+  static constexpr int threads = 64 * 12;
+};
+
+template <int DK>
+__global__ __launch_bounds__((KdaScanL<DK>::threads)) void kda_scan_fwd_kernel(DirectParams p) {
+  typedef KdaScanL<DK> L;
+  typedef typename L::RowT RowT;
+  typedef typename L::ValT ValT;
+  typedef typename L::TriT TriT;
+  typedef typename L::StT StT;
+  typedef typename L::DtT DtT;
+  constexpr int KT = DK / 16, NK = DK / 32;
+  extern __shared__ __align__(16) char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, kq = lane >> 4;
+  const int N = p.geom.N;
+  int64_t chain;
+  int slab, sidx, row, seq, c0, c1;
+  if (!xcd_slot_part((int64_t)(p.geom.tab ? p.geom.nseq : p.geom.rows / p.geom.H) * p.geom.H, p.dv / 32, chain, slab)) return;
+  scan_state(p.geom, (int)chain, sidx, row, seq);
+  seq_chunks(p.geom, seq, c0, c1);
+  const SeqSpan span = seq_span(p.geom, seq, c0);
+  const int v0 = 32 * slab, vs = 16 * (wave & 1);
+  auto first = [&](int n) { return smem + ((n - c0) & 1) * L::first; };
+  auto second = [&](int n) { return smem + L::oSecond + ((n - c0) & 1) * L::second; };
+  auto state_t = [&](int n) { return reinterpret_cast<T*>(smem + L::oS + ((n - c0) & 1) * StT::BYTES); };
+  auto d_t = [&](int n) { return reinterpret_cast<T*>(smem + L::oD + ((n - c0) & 1) * DtT::BYTES); };
+  auto decay = [&](int n) { return reinterpret_cast<float*>(smem + L::oE) + ((n - c0) & 1) * DK; };
+
+  if (wave >= 8) {  // ---------------- savers ----------------
+    const int t = tid - 512;
+    auto save = [&](int n) {
+      const int64_t slot = (int64_t)row * N + n;
+      const T* st = state_t(n);
+      const T* dt = d_t(n);
+      T* S = at<T>(p.ws, p.off.SnT) + slot * p.dv * DK + (int64_t)v0 * DK;
+      T* D = at<T>(p.ws, p.off.D) + slot * 64 * p.dv + v0;
+#pragma unroll
+      for (int u = 0; u < 32 * DK / 8 / 256; ++u) {
+        const int i = t + 256 * u, r = i / (DK / 8), c = 8 * (i % (DK / 8));
+        *reinterpret_cast<Frag*>(S + r * DK + c) = StT::load(st, r, c);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {  // four value columns of a token: rows of D^T
+        const int b = 2 * (wave & 3) + u, v = 4 * (kq + 4 * (b & 1)), tok = 16 * (b >> 1);
+        *reinterpret_cast<bf16x4*>(D + (int64_t)(tok + l16) * p.dv + v) = __builtin_bit_cast(bf16x4, DtT::tr4(dt, v, tok, lane));
+      }
+    };
+    lds_barrier();
+    for (int n = c0; n < c1; ++n) {
+      if (p.save && n > c0) save(n - 1);
+      lds_barrier();
+    }
+    if (p.save && c0 < c1) save(c1 - 1);
+    return;
+  }
+  if (wave >= 4) {  // ---------------- loads ----------------
+    const int w = wave - 4;
+    auto rows = [&](uint64_t off, int64_t slot, char* dst) {
+#pragma unroll
+      for (int u = 0; u < RowT::NINSTR / 4; ++u) {
+        int r, c;
+        RowT::src(w + 4 * u, lane, r, c);
+        dma16(at<const T>(p.ws, off) + slot * 64 * DK + r * DK + c, lds_byte_addr(dst) + 1024 * (w + 4 * u));
+      }
+    };
+    auto load_first = [&](int n) {
+      const int64_t slot = (int64_t)row * N + n;
+      char* dst = first(n);
+      rows(p.off.W, slot, dst);
+      rows(p.off.Kr, slot, dst + L::oKr);
+      int r, c;
+      ValT::src(w, lane, r, c);
+      dma16(at<const T>(p.ws, p.off.U) + slot * 64 * p.dv + (int64_t)r * p.dv + v0 + c, lds_byte_addr(dst) + L::oU + 1024 * w);
+    };
+    auto load_second = [&](int n) {
+      const int64_t slot = (int64_t)row * N + n;
+      char* dst = second(n);
+      rows(p.off.Qg, slot, dst);
+#pragma unroll
+      for (int u = 0; u < TriT::NINSTR / 4; ++u) {
+        int r, c;
+        TriT::src(w + 4 * u, lane, r, c);
+        dma16(at<const T>(p.ws, p.off.P) + slot * 64 * 64 + r * 64 + c, lds_byte_addr(dst) + L::oP + 1024 * (w + 4 * u));
+      }
+    };
+    static_assert(ValT::NINSTR == 4 && RowT::NINSTR % 4 == 0 && TriT::NINSTR % 4 == 0, "the same count for every wave");
+    if (c0 < c1) load_first(c0);
+    dma_wait<0>();
+    lds_barrier();
+    for (int n = c0; n < c1; ++n) {
+      if (n + 1 < c1) load_first(n + 1);
+      if (p.o) load_second(n);
+      dma_wait<0>();
+      lds_barrier();
+    }
+    return;
+  }
+  if (wave >= 2) {  // ---------------- output waves: O^T of a strip, lane = token ----------------
+    const int ch = DK == 128 ? 64 * (wave & 1) + lane : lane;
+    float g = 0.f;
+    auto fetch = [&](int n) { g = at<const float>(p.ws, p.off.G)[((int64_t)row * N + min(n, c1 - 1)) * DK + ch]; };
+    auto commit = [&](int n) { decay(n)[ch] = __expf(g); };
+    if (c0 < c1) {
+      fetch(c0), commit(c0);
+      fetch(c0 + 1);
+    }
+    lds_barrier();
+    for (int n = c0; n < c1; ++n) {
+      commit(n + 1);
+      fetch(n + 2);
+      lds_barrier();  // chunk n + 1, or the end of the last
+      if (!p.o) continue;
+      const T* tQ = reinterpret_cast<const T*>(second(n));
+      const T* tP = reinterpret_cast<const T*>(second(n) + L::oP);
+      int tok0, len;
+      chunk_span(span, n, tok0, len);
+      floatx4 o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < NK; ++ks) {
+        const Frag b = StT::load(state_t(n), vs + l16, 32 * ks + 8 * kq);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S16::mma(o[i], b, RowT::load(tQ, 16 * i + l16, 32 * ks + 8 * kq));
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const Frag b = DtT::load(d_t(n), vs + l16, 32 * s + 8 * kq);
+#pragma unroll
+        for (int i = 2 * s; i < 4; ++i) S16::mma(o[i], b, TriT::load(tP, 16 * i + l16, 32 * s + 8 * kq));
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = 16 * i + l16;
+        const int64_t e = (tok_index(p.geom, row, tok0) + (int64_t)t * p.geom.ts) * p.dv + v0 + vs + 4 * kq;
+        if (t < len) {
+          if (p.o_dtype == LNX_F32) store4(reinterpret_cast<float*>(p.o) + e, o[i]);
+          else store4(reinterpret_cast<T*>(p.o) + e, o[i]);
+        }
+      }
+    }
+    return;
+  }
+
+  // ---------------- compute waves: value columns v0 + vs .. + 15, rows of tile i: row0(i) + 8 kq + e ----------------
+  auto row0 = [](int i) { return 32 * (i >> 1) + 4 * (i & 1); };
+  const int lr = 8 * ((lane >> 2) & 3) + (lane & 3);  // operand row l16 of such a tile
+  floatx4 S[KT];
+#pragma unroll
+  for (int ci = 0; ci < KT; ++ci)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S[ci][e] = p.ident && row0(ci) + 8 * kq + e == v0 + vs + l16 - p.vcols ? 1.f : 0.f;
+  if (!p.ident && p.s0) {
+    const float* s0 = p.s0 + (int64_t)sidx * DK * p.dv + v0 + vs + l16;
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[ci][e] = s0[(int64_t)(row0(ci) + 8 * kq + e) * p.dv];
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci) asm volatile("" : "+v"(S[ci]));
+  }
+  const bool keep = p.o || p.save;
+  lds_barrier();
+  for (int n = c0; n < c1; ++n) {
+    const T* tW = reinterpret_cast<const T*>(first(n));
+    const T* tK = reinterpret_cast<const T*>(first(n) + L::oKr);
+    const T* tU = reinterpret_cast<const T*>(first(n) + L::oU);
+    const float* eg = decay(n);
+    floatx4 y[4];
+    Frag fa[NK][4], b[NK], bd[2], fu[2][KT];
+    bf16x4 u4[4];
+    auto load_w = [&](int ks) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) fa[ks][i] = RowT::load(tW, row0(i) + lr, 32 * ks + 8 * kq);
+    };
+    // channels of state tile ci, tokens 32 s + 8 kq ..
+    auto load_k = [&](int s, int ci) {
+      const int q = lane & 15, c = 32 * (ci >> 1) + 4 * (ci & 1) + 8 * (q & 3), r = 32 * s + 8 * kq + (q >> 2);
+      return S16::join(__builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((S16::lds_short4*)(tK + RowT::at(r, c)))),
+                       __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((S16::lds_short4*)(tK + RowT::at(r + 4, c)))));
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    load_w(0), load_w(1);
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) {
+      b[ks] = S16::from_acc(S[2 * ks], S[2 * ks + 1]);
+      if (ks + 2 < NK) {
+        load_w(ks + 2);
+      } else if (ks + 2 == NK) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u4[i] = __builtin_bit_cast(bf16x4, ValT::tr4(tU, row0(i) + 8 * kq, vs, lane));
+      } else {
+#pragma unroll
+        for (int ci = 0; ci < KT / 2; ++ci) fu[0][ci] = load_k(0, ci);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S16::mma(y[i], fa[ks][i], b[ks]);
+    }
+    if (keep) {  // read behind the next barrier
+#pragma unroll
+      for (int ks = 0; ks < NK; ++ks) *reinterpret_cast<Frag*>(state_t(n) + StT::at(vs + l16, 32 * ks + 8 * kq)) = b[ks];
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 2 * s; i < 2 * s + 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[i][e] = (float)u4[i][e] - y[i][e];
+      bd[s] = S16::from_acc(y[2 * s], y[2 * s + 1]);
+    }
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci) S[ci] *= load4(eg + row0(ci) + 8 * kq);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ci = KT / 2; ci < KT; ++ci) fu[0][ci] = load_k(0, ci);
+#pragma unroll
+    for (int ci = 0; ci < KT / 2; ++ci) S16::mma(S[ci], fu[0][ci], bd[0]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci) fu[1][ci] = load_k(1, ci);
+#pragma unroll
+    for (int ci = KT / 2; ci < KT; ++ci) S16::mma(S[ci], fu[0][ci], bd[0]);
+    if (keep) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) *reinterpret_cast<Frag*>(d_t(n) + DtT::at(vs + l16, 32 * s + 8 * kq)) = bd[s];
+    }
+#pragma unroll
+    for (int ci = 0; ci < KT; ++ci) S16::mma(S[ci], fu[1][ci], bd[1]);
+    lds_barrier();
+  }
+  float* out = p.sT_out.at(sidx, (int64_t)DK * p.dv) + v0 + vs + l16;
+#pragma unroll
+  for (int ci = 0; ci < KT; ++ci)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[(int64_t)(row0(ci) + 8 * kq + e) * p.dv] = S[ci][e];
+}
+
+template <int DK>
+int launch_scan(const DirectParams& p, int nstate, hipStream_t st) {
+  auto k = kda_scan_fwd_kernel<DK>;
+  const size_t b = KdaScanL<DK>::bytes;
+  if (const int rc = lnx_lds_limit((const void*)k, b); rc != LNX_OK) return rc;
+  lnx_profile_mark("chunk_scan", st);
+  hipLaunchKernelGGL(k, dim3(lnx_xcd_grid((int64_t)nstate * p.geom.H, p.dv / 32)), dim3(KdaScanL<DK>::threads), b, st, p);
+  lnx_profile_mark(nullptr, st);
+  return LNX_OK;
+}
+
 template <int DK>
 int launch(const KdaBwdParams& p, hipStream_t st) {
   auto k = p.graw ? kda_bwd_chunk_kernel<DK, true> : kda_bwd_chunk_kernel<DK, false>;
@@ -680,3 +953,5 @@ int launch(const KdaBwdParams& p, hipStream_t st) {
 }  // namespace
 
 int lnx_kda_bwd_chunk(const KdaBwdParams& p, int dk, hipStream_t st) { return dk == 128 ? launch<128>(p, st) : launch<64>(p, st); }
+
+int lnx_kda_scan_fwd(const DirectParams& p, int dk, int nstate, hipStream_t st) { return dk == 128 ? launch_scan<128>(p, nstate, st) : launch_scan<64>(p, nstate, st); }

@@ -294,7 +294,7 @@ def _prefill_segments(B: int, H: int, T: int, dv: int, dk: int = 256, two_byte: 
     The lines are where the gain starts, bf16 d128 unless said (both sides as they are now; where a call beside a line lost, as the line was
     drawn): 4 heads of 4096 tokens 83 -> 62 us (2048: 52 -> 62), 4 heads of 16384 298 -> 107, 16 heads (w = 64) of 8192 170 -> 131 (4096:
     98 -> 101), 32 heads never.  The kernels that form W and U prepare both passes: no gain at w = 64; fp32 4 heads of 4096
-    275 -> 175 us, bf16 per-channel gate 4 heads of 8192 228 -> 143 (4096: 131 -> 133).  From 512 chunks on, w = 64 gains from a second
+    275 -> 175 us, bf16 per-channel gate 4 heads of 8192 185 -> 131 (4096: 104 -> 112).  From 512 chunks on, w = 64 gains from a second
     round (32768 tokens: 806 -> 395).
 
     dk = 256, and rows that would have to be copied to become heads: at most an eighth of the CUs busy and every segment keeps >= 64 chunks

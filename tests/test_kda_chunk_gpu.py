@@ -46,3 +46,33 @@ def test_gradients(dk, dv, T, cu, l2):
     ref = {n: np.concatenate([p[n] for p in parts if n in p], 2) for n in ("dq", "dk", "dv", "dbeta", "dg")}
     ref["dS0"] = np.concatenate([p["dS0"] for p in parts], 0)
     check(gpu_grads(x, "vector", dt, cu=None if cu is None else np.array(cu, np.int32), l2=l2), ref, 2e-2)
+
+
+@pytest.mark.parametrize("dk", [64, 128])
+@pytest.mark.parametrize("H,T,cu", [(3, 500, None), (3, 64, None), (2, 700, [0, 0, 1, 64, 129, 129, 500, 700]), (56, 130, None), (60, 330, None)])
+@pytest.mark.parametrize("f32_out", [False, True])
+def test_forward_forms(monkeypatch, dk, H, T, cu, f32_out):
+    """The chain in registers (32-column slabs) against the one through LDS (64-column slabs) and against the own choice, which at dk = 128 lies
+    between 56 and 60 heads.  Both round the state and D to bf16 at the same places; what differs is the order of fp32 sums, which can move such
+    a rounding by one step, 2^-8 of a value: 1e-2 of the largest."""
+    import linearnexus_amd as la
+    from linearnexus_amd import linear_attn
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    x = [(rnd(1, H, T, dk) * dk ** -0.5).bfloat16(), (rnd(1, H, T, dk) * dk ** -0.5).bfloat16(), rnd(1, H, T, 128).bfloat16(),
+         -0.3 * torch.rand(1, H, T, dk, generator=gen, device="cuda"), torch.rand(1, H, T, generator=gen, device="cuda")]
+    out = torch.float32 if f32_out else torch.bfloat16
+    monkeypatch.setenv("LNX_PREFILL_SEGMENTS", "1")
+    cu = None if cu is None else torch.tensor(cu, dtype=torch.int32, device="cuda")
+    results = []
+    for slab in (64, 32, 0):
+        monkeypatch.setitem(linear_attn._test_hooks, "scan_slab", slab)
+        y = [t.clone().requires_grad_() for t in x]
+        with torch.no_grad():
+            plain = la.kda_chunkwise(*y, cu_seqlens=cu, output_dtype=out)
+        o, S = la.kda_chunkwise(*y, cu_seqlens=cu, output_dtype=out)
+        assert torch.equal(plain[0], o) and torch.equal(plain[1], S)  # with and without saved states
+        results.append([o, S, *torch.autograd.grad((o.float() ** 2).sum() + S.sum(), y)])
+    for got in results[1:]:
+        for a, b in zip(results[0], got):
+            assert torch.isfinite(b).all() and max_rel(b.detach().float().cpu().numpy(), a.detach().float().cpu().numpy()) < 1e-2
