@@ -215,7 +215,10 @@ template <int DK> struct KdaL {
   static constexpr int tile = 64 * LDX * 2, oP = 2 * RowT::BYTES, oF = oP + 2 * tile, epi_bytes = oF + 4 * 64 * (4 + 12 * NS);
   // the gate's gradient, fp32 [64][LDF] per set: the last set's over K and Q, the one before it waits behind everything else
   static constexpr int LDF = 64 + 4, oG0 = epi_bytes, all_bytes = epi_bytes + (NS - 1) * 64 * LDF * 4;
-  static_assert(NS <= 2 && 64 * LDF * 4 <= oF, "the gate's gradient leaves over the tiles");
+  // a gate activated inside the op: its partial sums [set][which][wave][64], behind the gradient, which other waves still read when they are
+  // stored -- at dk = 64 its last rows lie over dPm
+  static constexpr int grad = 64 * LDF * 4, oPart = oP > grad ? oP : grad;
+  static_assert(NS <= 2 && oPart % 16 == 0 && grad <= oPart && oPart + NS * 2 * 4 * 64 * 4 <= oF, "gradient and partial sums leave over the tiles, side by side");
   static constexpr size_t bytes = sizeof(float) * 192 + (all_bytes > loop_bytes ? all_bytes : loop_bytes);
   static_assert(bytes <= 80 * 1024, "two workgroups per CU");
 };
@@ -614,7 +617,7 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
 #pragma unroll
   for (int x = 0; x < 16; ++x) sOut[(16 * (x >> 2) + 4 * kq + (x & 3)) * L::LDF + 16 * wave + l16] = dG[x];
   lds_barrier();
-  float* sPart = reinterpret_cast<float*>(region + L::oP);  // GRAW: [set][which][wave][64]
+  float* sPart = reinterpret_cast<float*>(region + L::oPart);  // GRAW: [set][which][wave][64]
 #pragma unroll
   for (int u = 0; u < NS; ++u) {
     const float* src = u + 1 < NS ? reinterpret_cast<const float*>(region + L::oG0) : sOut;

@@ -136,3 +136,49 @@ def test_raw_gate_equals_gate_kernel_then_scan_and_refuses_bad_arguments():
         la.kda_chunkwise_raw_gate(q, k, v, gv.float(), beta, A, gb)          # gate dtype differs from q's
     with pytest.raises(RuntimeError):
         la.kda_chunkwise_raw_gate(q, k, v, gv, beta, A[:1], gb)
+
+
+@pytest.mark.parametrize("l2", [False, True])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("B,H,T,dv,cu", [(2, 3, 256, 64, None), (2, 3, 253, 128, None), (8, 8, 637, 64, None), (1, 3, 317, 64, [0, 61, 61, 189, 317])])
+def test_raw_gate_gradients_dk64(B, H, T, dv, cu, bias, l2):
+    """bf16 with dk = 64, where the gate's gradient on its way out and its partial sums share the place of the tiles: full chunks, 61 and 62 tokens
+    left, more chunks than fit the GPU at once, a packed batch with an empty sequence; the chunks' last four tokens by themselves, and the
+    same bits twice."""
+    import linearnexus_amd as la
+    dk, thr = 64, 0.5
+    x = _case(104, B, H, T, dk, dv, True, bias, cu=cu)
+    if l2:
+        for n in "qk":
+            x[n] = to_bf16_grid(x[n] * np.exp(np.random.default_rng(105).standard_normal((B, H, T, 1))).astype(np.float32))
+    t = lambda a, dt=None: torch.from_numpy(np.ascontiguousarray(a)).to(DEV).to(dt or torch.float32).requires_grad_()
+    q, k, v = (t(x[n], torch.bfloat16) for n in "qkv")
+    raw = t(x["raw"].reshape(B, T, H, dk).transpose(0, 2, 1, 3), torch.bfloat16)
+    leaves = [q, k, v, raw, t(x["beta"]), t(x["A_log"])] + ([t(x["bias"])] if bias else [])
+    q, k, v, raw, beta, A = leaves[:6]
+    dO = torch.from_numpy(x["dO"]).to(DEV)
+    runs = []
+    for _ in range(2):
+        o, _ = la.kda_chunkwise_raw_gate(q, k, v, raw, beta, A, leaves[6] if bias else None, None, None, 64, l2, threshold=thr, cu_seqlens=cu)
+        runs.append(torch.autograd.grad((o * dO).sum(), leaves))
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
+    g = np.ascontiguousarray(og.kda_gate(x["raw"], x["A_log"], dk, x["bias"], None, thr)[0].transpose(0, 2, 1, 3))
+    spans = [(a, b) for a, b in zip(cu[:-1], cu[1:]) if a < b] if cu else [(0, T)]
+    parts = [delta_rule_adjoint(*(z[:, :, a:b] for z in (x["q"], x["k"], x["v"], x["beta"], x["dO"], g)), None, None, None, l2) for a, b in spans]
+    ref = {n: np.concatenate([r[n] for r in parts], 2) for n in ("dq", "dk", "dv", "dg", "dbeta")}
+    draw = og.kda_gate_grad(x["raw"], x["A_log"], dk, ref["dg"].transpose(0, 2, 1, 3), x["bias"], thr)[0].reshape(B, T, H, dk).transpose(0, 2, 1, 3)
+    got = [z.double().cpu().numpy() for z in runs[0]]
+    for a, b in zip(got, (ref["dq"], ref["dk"], ref["dv"], draw, ref["dbeta"])):
+        assert max_rel(a, b) < 2e-2
+    last = np.concatenate([np.arange(c + min(60, b - c), min(c + 64, b)) for a, b in spans for c in range(a, b, 64)])
+    assert max_rel(got[3][:, :, last], draw[:, :, last]) < 2e-2
+    # The parameters' gradients are sums of thousands of terms of either sign, so they are held to the op's own d_raw: its values are the summed
+    # ones rounded to bf16, an error of 2^-9 / sqrt(3) of a term at most in the mean (eight standard deviations), beside the fp32 sums.
+    z = x["raw"].astype(np.float64).reshape(B, T, H, dk).transpose(0, 2, 1, 3) + (x["bias"].reshape(H, 1, dk) if bias else 0.0)
+    lin = z > thr
+    to_A = np.where(lin, z, np.log1p(np.exp(np.minimum(z, thr)))) * np.where(lin, 1.0, 1.0 + np.exp(-z))  # softplus over its derivative
+    sums = [(got[5], got[3] * to_A, (0, 2, 3))] + ([(got[6].reshape(H, dk), got[3], (0, 2))] if bias else [])
+    for total, terms, axes in sums:
+        bound = 8 * 2.0 ** -9 / 3 ** 0.5 * np.sqrt((terms ** 2).sum(axes)) + 1e-5 * np.abs(terms).sum(axes)
+        assert (np.abs(total - terms.sum(axes)) <= bound).all()
