@@ -98,7 +98,7 @@ template <int GATE> __device__ __forceinline__ void put_scalars(float* sc, int t
 // chunk behind, and one barrier per chunk is enough:
 //   B1    K, V, Tm of chunk n, Q, Pm of n - 1   compute: Y, R, D, state update; S^T and D^T -> LDS [n mod 2]
 //                                               output:  O of chunk n - 1 from S^T and D^T as the compute wave has them in registers -> global;
-//                                                        the per-token scalars of chunk n + 2
+//                                                        behind it the per-token scalars of chunk n + 2
 //                                               movers:  S^T, D^T of n - 1 -> global; loads and writes as above, Q and Pm of the chunk before
 // A chunk of one prompt of 1000 tokens: 1.43 us with everything in the compute waves (Y and Q S 0.5, R and D 0.2, the rest of O 0.2, update 0.3,
 // movers 0.7 between B1 and Bmid), 1.23 so (compute 1.0, movers 1.15, output 0.8); the call 33.3 -> 32.1 us, the scan of B2 H16 T2007 53 -> 48.
@@ -352,16 +352,19 @@ __global__ __launch_bounds__((FScanL<DK, BVW, !std::is_void<OT>::value>::threads
         const T* r = tile + (vs + l16) * ld + 32 * ks + g4;
         return S16::join(*reinterpret_cast<const bf16x4*>(r), *reinterpret_cast<const bf16x4*>(r + 8));
       };
-      // They bring the scalars, too, the same from every output wave: those of chunk n + 2 go to LDS and those of chunk n + 3 are requested in
-      // chunk n.  No load behind a branch: past the end the last chunk's come again.
-      float b_ = 0.f, g_ = 0.f, gc_ = 0.f, nk_ = 0.f, fq_ = 0.f;  // beta (0 past the end), G, G_C, the factors of the K and Q rows
+      // They bring the scalars, too, the same from every output wave: those of chunk n + 3 go to LDS and those of chunk n + 4 are requested behind
+      // the outputs of chunk n.  No load behind a branch: past the end the last chunk's come again.  Nor may the barrier that every wave waits at
+      // stand behind a load just requested or a store: beta's choice waits until it is used, and the stores are range-checked instead of
+      // branched around, so that the scalars are waited for by count (before: calls that exceed the 256 MiB cache, 16384 tokens forward only,
+      // 32 heads 443 us, without a gate 450; so 398 and 378; without output waves 410 and 374).
+      float b_ = 0.f, g_ = 0.f, gc_ = 0.f, nk_ = 0.f, fq_ = 0.f;  // beta, G, G_C, the factors of the K and Q rows
+      int len_ = 0;                                               // past the end beta is 0
       auto fetch_scalars = [&](int n) {
         n = min(n, c1 - 1);
         const int64_t slot = (int64_t)row * N + n;
-        int tok0, len;
-        chunk_span(span, n, tok0, len);
-        b_ = p.beta[tok_index(p.geom, row, tok0) + (int64_t)min(lane, len - 1) * p.geom.ts];
-        b_ = lane < len ? b_ : 0.f;
+        int tok0;
+        chunk_span(span, n, tok0, len_);
+        b_ = p.beta[tok_index(p.geom, row, tok0) + (int64_t)min(lane, len_ - 1) * p.geom.ts];
         if (GATE == LNX_GATE_SCALAR) {
           const float* G = at<const float>(p.ws, p.off.G) + slot * 64;
           g_ = G[lane], gc_ = G[63];
@@ -371,7 +374,7 @@ __global__ __launch_bounds__((FScanL<DK, BVW, !std::is_void<OT>::value>::threads
       };
       auto commit_scalars = [&](int n) {
         float* sc = sSc + ((n - c0) & (L::NSC - 1)) * L::SCS;
-        put_scalars<GATE>(sc, lane, b_, g_, gc_);
+        put_scalars<GATE>(sc, lane, lane < len_ ? b_ : 0.f, g_, gc_);
         sc[Scal::NK + lane] = nk_, sc[Scal::FQ + lane] = fq_;
       };
       if (c0 < c1) {
@@ -381,9 +384,14 @@ __global__ __launch_bounds__((FScanL<DK, BVW, !std::is_void<OT>::value>::threads
         lds_barrier();
       }
       lds_barrier();  // B1 of the first chunk
+      if (c0 < c1) {
+        commit_scalars(c0 + 2);
+        fetch_scalars(c0 + 3);
+      }
+      int off[4];  // of the lane's pieces of O
+#pragma unroll
+      for (int i = 0; i < 4; ++i) off[i] = (int)(((16 * i + l16) * tso + vs + 4 * (lane >> 4)) * (int64_t)sizeof(OT));
       for (int n = c0; n < c1; ++n) {
-        commit_scalars(n + 2);
-        fetch_scalars(n + 3);
         lds_barrier();  // B1 of the next chunk, or the end of the last
         const int pb = (n - c0) & 1;
         const T* sQc = sQ + pb * L::kK;
@@ -421,15 +429,22 @@ __global__ __launch_bounds__((FScanL<DK, BVW, !std::is_void<OT>::value>::threads
         for (int i = 0; i < 4; ++i) S16::mma(o[i], bd0, pm[i]);
         S16::mma(o[2], bd1, pm[4]);
         S16::mma(o[3], bd1, pm[5]);
+        const __amdgpu_buffer_rsrc_t rsrc =
+            __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<OT*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + v0, 0, (int)(len * tso * (int64_t)sizeof(OT)), 0x00020000);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int t = 16 * i + l16;
+          const bf16x4 x = pack_bf16x4(o[i]);
           if constexpr (std::is_same<OT, float>::value) {  // fp32 outputs are rounded as the others and widened
-            const bf16x4 x = pack_bf16x4(o[i]);
-            o[i] = floatx4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+            typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+            const floatx4 y = {(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, y), rsrc, off[i], 0, 0);
+          } else {
+            typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), rsrc, off[i], 0, 0);
           }
-          if (t < len) store4(reinterpret_cast<OT*>(p.o) + tok_index(p.geom, row, tok0) * p.dv + t * tso + v0 + vs + 4 * (lane >> 4), o[i]);
         }
+        commit_scalars(n + 3);
+        fetch_scalars(n + 4);
       }
       return;
     }

@@ -55,3 +55,23 @@ def test_final_states_alone(monkeypatch, dk, H, chunks):
         o2, S2 = _run(monkeypatch, 0, x, False)
     for a, b in ((o1, o2), (S1, S2)):
         assert ((a - b).float().norm() / a.float().norm()).item() < 2e-2
+
+
+@pytest.mark.parametrize("dk", [64, 128])
+@pytest.mark.parametrize("T", [1, 61, 64, 333])
+@pytest.mark.parametrize("token_first", [False, True])
+@pytest.mark.parametrize("gated", [False, True])
+def test_output_forms(monkeypatch, dk, T, token_first, gated):
+    """Outputs in fp32 are the bf16 ones widened, in both forms and both layouts."""
+    from linearnexus_amd import linear_attn
+    q, k, v, g, beta = (t.transpose(1, 2).contiguous().transpose(1, 2) if token_first and t.dim() == 4 else t for t in _inputs(2, 3, T, dk, 64))
+    results = []
+    for slab in (64, 32):
+        monkeypatch.setitem(linear_attn._test_hooks, "scan_slab", slab)
+        for dtype in (torch.bfloat16, torch.float32):
+            with torch.no_grad():
+                o, S = linear_attn._chunk(q, k, v, g if gated else None, beta, dk ** -0.5, None, 64, gated, dtype, False, None)
+            assert o.dtype == dtype
+            results.append((o.float(), S))
+    for o, S in results[1:]:
+        assert torch.equal(o, results[0][0]) and torch.equal(S, results[0][1])
