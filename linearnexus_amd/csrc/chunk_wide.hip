@@ -15,10 +15,18 @@
 //   B1   tiles of chunk n in LDS               compute: everything but the last product     movers: loads of the next chunk
 //   B2   its K is left                         compute: the last product    movers: results -> global, the other tiles -> LDS
 //   B3                                         compute: state -> global     movers: K -> LDS
-// Measured at B8 H8 T4096 dv512 (128-column slabs, 256 workgroups): forward 511 us, reverse 470 us, 8 and 7.4 us a chunk, of which
+// Slabs of 32 and 64 columns are taken where a chunk's chain is what a call waits for.  Their compute waves leave registers and LDS for more:
+// the movers hold two chunks, so that rows which the op normalises are converted ahead of B2 without waiting for memory, and K has two tiles
+// and no barrier of its own (AHEAD):
+//   B1   compute: everything but the last product     movers: loads of chunk n + 2; of chunk n + 1 Q (in reverse behind B2) and K converted, K -> LDS
+//   B2   compute: the last product, state -> global   movers: results -> global, the other tiles -> LDS
+// With one chunk held and converted where it is stored, between the barriers, 4 heads dv 256 of 8192 tokens took 418 us forward only and 849
+// with gradients, more than the WY split's kernels (360 and 769, the normalisation ahead of them); so 331 and 743.  The movers' loads and
+// conversions in turn, a tile at a time, and Q's conversion behind B2 in reverse are 366 -> 349 and 368 -> 326 us of the scans.
+// Measured at B8 H8 T4096 dv512 (128-column slabs, 256 workgroups): forward 498 us, reverse 448 us, 7.8 and 7 us a chunk, of which
 // 185 KB through the CU's memory path (64 KB of state per chunk and slab leave for the backward kernels) are most.  The WY split's
 // passes, which read W and U instead of Tm and V, took 521 and 435 us behind 205 us of preparation (now 68) and 221 us of normalisation
-// outside the kernels (now none), and before two more kernels of 804 and 289 us (now one of 806): the step 2478 -> 1827 us.
+// outside the kernels (now none), and before two more kernels of 804 and 289 us (now one of 788): the step 2478 -> 1830 us.
 // State stores among the products of the first phase instead of
 // behind the last barrier: 551 -> 587 and 464 -> 521 us (a wave whose store waits for a slot multiplies nothing).
 
@@ -55,8 +63,10 @@ __device__ __forceinline__ Frag load_cols(const T* tile, int ld, int s, int ci, 
 template <int NC, int NCW> struct WideL {
   static constexpr int BV = 16 * NC * NCW, LDK = DK + 16, LDC = LNX_C + 16, LDV = BV + 8, LDT = LNX_C + 8;
   static constexpr int kRow = 64 * LDK, kC = 64 * LDC, kV = 64 * LDV, kT = BV * LDT;
-  // K | Q | Tm | Pm | V (reverse: dO) | O (reverse: dv) on its way out | D^T (reverse: dR^T) on its way out | scalars
-  static constexpr size_t bytes = sizeof(T) * (2 * kRow + 2 * kC + 2 * kV + kT) + sizeof(float) * 272;
+  static constexpr bool AHEAD = NC == 1;  // the movers hold two chunks, and LDS two K tiles
+  static constexpr int NK2 = AHEAD ? 2 : 1;
+  // K [NK2] | Q | Tm | Pm | V (reverse: dO) | O (reverse: dv) on its way out | D^T (reverse: dR^T) on its way out | scalars
+  static constexpr size_t bytes = sizeof(T) * ((NK2 + 1) * kRow + 2 * kC + 2 * kV + kT) + sizeof(float) * 272;
   static constexpr int threads = 64 * NCW + 256;
   static_assert(bytes <= 160 * 1024, "LDS");
 };
@@ -96,24 +106,36 @@ __device__ __forceinline__ void zero_upper(T* tiles, int ld, int stride, int tid
 #pragma unroll
   for (int t = 0; t < 2; ++t) *reinterpret_cast<bf16x8*>(tiles + t * stride + place(r) * ld + 8 * c) = vec_zero<T>();
 }
-// Row factors of a [64][DK] tile's vectors (1 / (|x| + eps) where the op normalises), and the tile's rows times them to LDS
-struct RowFactors {
-  float f[64 * DK / 8 / 256];
+// Row factors of a [64][DK] tile (1 / (|x| + eps) where the op normalises), and the tile's rows times them.  A thread's vectors lie in eight
+// rows: it loads their factors, or where two chunks in flight leave the memory counter no room for that (LANES) that of row `lane`, and takes
+// the wave's two rows of every eight out of the lanes (128-column slabs, forward only, 202 us with the loads, 206 so).
+template <bool LANES> struct RowFactors {
+  static constexpr int IT = 64 * DK / 8 / 256;
+  float f[LANES ? 1 : IT];
   __device__ __forceinline__ void load(const float* src, int tid) {
 #pragma unroll
-    for (int it = 0; it < 64 * DK / 8 / 256; ++it) f[it] = src[(tid + 256 * it) / (DK / 8)];
+    for (int it = 0; it < (LANES ? 1 : IT); ++it) f[it] = src[LANES ? tid & 63 : (tid + 256 * it) / (DK / 8)];
+  }
+  __device__ __forceinline__ float of(int it, int tid) const {
+    if constexpr (!LANES) return f[it];
+    const int r = 2 * __builtin_amdgcn_readfirstlane(tid >> 6) + 8 * it, x = __float_as_int(f[0]);
+    const int lo = __builtin_amdgcn_readlane(x, r), hi = __builtin_amdgcn_readlane(x, r + 1);
+    return __int_as_float(tid & 32 ? hi : lo);
   }
 };
-__device__ __forceinline__ void store_rows(const TileRegs<T, 64, DK>& R, const RowFactors& F, bool scaled, T* dst, int ld, int tid) {
+template <bool LANES> __device__ __forceinline__ void scale_rows(TileRegs<T, 64, DK>& R, const RowFactors<LANES>& F, int tid) {
+#pragma unroll
+  for (int it = 0; it < TileRegs<T, 64, DK>::IT; ++it) {
+    const float f = F.of(it, tid);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) R.x[it][e] = (bf16_t)((float)R.x[it][e] * f);
+  }
+}
+__device__ __forceinline__ void store_rows(const TileRegs<T, 64, DK>& R, T* dst, int ld, int tid) {
 #pragma unroll
   for (int it = 0; it < TileRegs<T, 64, DK>::IT; ++it) {
     const int idx = tid + 256 * it, r = idx / (DK / 8), c = (idx - r * (DK / 8)) * 8;
-    bf16x8 x = R.x[it];
-    if (scaled) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = (bf16_t)((float)x[e] * F.f[it]);
-    }
-    *reinterpret_cast<bf16x8*>(dst + place(r) * ld + c) = x;
+    *reinterpret_cast<bf16x8*>(dst + place(r) * ld + c) = R.x[it];
   }
 }
 // What the movers read per chunk besides the row and value tiles
@@ -235,7 +257,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
   constexpr int BV = L::BV, LDK = L::LDK, LDC = L::LDC, LDV = L::LDV, LDT = L::LDT;
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);
-  T* sQ = sK + L::kRow;
+  T* sQ = sK + L::NK2 * L::kRow;
   T* sTm = sQ + L::kRow;
   T* sP = sTm + L::kC;
   T* sV = sP + L::kC;
@@ -245,54 +267,75 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   Chain ch;
   if (!chain_of<BV>(p, ch)) return;
+  auto k_tile = [&](int n) { return sK + (L::AHEAD ? (n & 1) * L::kRow : 0); };
   const int N = p.geom.N, c0 = ch.c0, c1 = ch.c1, v0 = ch.v0;
   const int64_t tso = (int64_t)p.geom.ts * p.dv;
 
   if (wave >= NCW) {
     // ---------------- movers ----------------
     const int mt = tid - 64 * NCW;
-    TileRegs<T, 64, DK> rK, rQ;
-    TileRegs<T, 64, BV> rV;
-    PlacedTri rTm, rP;
-    RowFactors fk, fq;
-    Scalars<GATE> rs;
-    rTm.init(LDC, mt), rP.init(LDC, mt);
+    struct Chunk {
+      TileRegs<T, 64, DK> K, Q;
+      TileRegs<T, 64, BV> V;
+      PlacedTri Tm, P;
+      RowFactors<L::AHEAD> fk, fq;
+      Scalars<GATE> sc;
+    };
+    Chunk a, b;
+    a.Tm.init(LDC, mt), a.P.init(LDC, mt), b.Tm.init(LDC, mt), b.P.init(LDC, mt);
     zero_upper(sTm, LDC, L::kC, mt);
     const int64_t tsk = (int64_t)p.geom.ts * DK, tsv = (int64_t)p.geom.ts * p.vcols;
-    auto fetch = [&](int n) {
+    // part 0: Q, 1: K, 2: the rest; < 0: everything.  Unconditional, as the commits: a load behind a branch cannot be counted
+    auto fetch = [&](Chunk& R, int n, int part = -1) __attribute__((always_inline)) {
+      n = min(n, c1 - 1);
       const int64_t slot = (int64_t)ch.row * N + n;
       int tok0, len;
       chunk_span(ch.span, n, tok0, len);
       const int64_t tbase = tok_index(p.geom, ch.row, tok0);
-      if constexpr (OUT) {
-        rQ.load(p.q + tbase * DK, tsk, len, mt);
-        fq.load(at<const float>(p.ws, p.off.Nq) + slot * 64, mt);
+      if (OUT && (part < 0 || part == 0)) {
+        R.Q.load(p.q + tbase * DK, tsk, len, mt);
+        R.fq.load(at<const float>(p.ws, p.off.Nq) + slot * 64, mt);
       }
-      rV.load(p.v + tbase * p.vcols + v0, tsv, (v0 < p.vcols) ? len : 0, mt);  // columns v does not hold read as zero
-      rTm.load(at<const T>(p.ws, p.off.Tm) + slot * 64 * 64, mt);
-      if constexpr (OUT) rP.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
-      rs.load(p, slot, tbase, len, mt);
-      rK.load(p.k + tbase * DK, tsk, len, mt);
-      fk.load(at<const float>(p.ws, p.off.Nk) + slot * 64, mt);
+      if (part < 0 || part == 2) {
+        R.V.load(p.v + tbase * p.vcols + v0, tsv, (v0 < p.vcols) ? len : 0, mt);  // columns v does not hold read as zero
+        R.Tm.load(at<const T>(p.ws, p.off.Tm) + slot * 64 * 64, mt);
+        if (OUT) R.P.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
+        R.sc.load(p, slot, tbase, len, mt);
+      }
+      if (part < 0 || part == 1) {
+        R.K.load(p.k + tbase * DK, tsk, len, mt);
+        R.fk.load(at<const float>(p.ws, p.off.Nk) + slot * 64, mt);
+      }
     };
-    auto commit = [&]() {
-      if constexpr (OUT) store_rows(rQ, fq, p.l2norm, sQ, LDK, mt);
-      rV.store(sV, LDV, mt);
-      rTm.store(sTm);
-      if constexpr (OUT) rP.store(sP);
+    auto normalise = [&](Chunk& R, int part = -1) __attribute__((always_inline)) {
+      if (OUT && p.l2norm && part != 1) scale_rows(R.Q, R.fq, mt);
+      if (p.l2norm && part != 0) scale_rows(R.K, R.fk, mt);
     };
-    auto commit_k = [&]() {  // the scalars with it: the last product's decay is read until here
-      store_rows(rK, fk, p.l2norm, sK, LDK, mt);
-      rs.put(sc, p.scale, mt);
+    auto commit = [&](const Chunk& R) __attribute__((always_inline)) {
+      if constexpr (OUT) store_rows(R.Q, sQ, LDK, mt);
+      R.V.store(sV, LDV, mt);
+      R.Tm.store(sTm);
+      if constexpr (OUT) R.P.store(sP);
+      R.sc.put(sc, p.scale, mt);
     };
-    if (c0 < c1) {
-      fetch(c0);
-      commit();
-      commit_k();
-    }
-    lds_barrier();  // B1 of the first chunk
-    for (int n = c0; n < c1; ++n) {
-      fetch(min(n + 1, c1 - 1));  // unconditional, as the commits: a load behind a branch cannot be counted
+    auto commit_k = [&](const Chunk& R, int n) __attribute__((always_inline)) { store_rows(R.K, k_tile(n), LDK, mt); };
+    // cur, whose chunk n is in LDS, takes chunk n + 2, a tile at a time between the conversions of nxt, which holds chunk n + 1 since the step
+    // before.  Without AHEAD the same registers take chunk n + 1.
+    auto step = [&](Chunk& cur, Chunk& nxt, int n) __attribute__((always_inline)) {
+      if constexpr (L::AHEAD) {
+        fetch(cur, n + 2, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        normalise(nxt, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(cur, n + 2, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        normalise(nxt, 1);
+        commit_k(nxt, n + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(cur, n + 2, 1);
+      } else {
+        fetch(cur, n + 1);
+      }
       lds_barrier();  // B2
       const int64_t slot = (int64_t)ch.row * N + n;
       int tok0, len;
@@ -300,10 +343,31 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
       if (std::is_same<OT, T>::value && p.o)
         unstage_tile_checked<T, 64, BV>(reinterpret_cast<T*>(p.o) + tok_index(p.geom, ch.row, tok0) * p.dv + v0, tso, sO, LDV, len, mt);
       if (OUT && p.save) unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.D) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sDT, LDT, BV, mt);
-      commit();
-      lds_barrier();  // B3
-      commit_k();
+      if (!L::AHEAD) normalise(nxt, 0);
+      commit(nxt);
+      if (!L::AHEAD) {
+        lds_barrier();  // B3
+        normalise(nxt, 1);
+        commit_k(nxt, n + 1);
+      }
       lds_barrier();  // B1 of the next chunk
+    };
+    if (c0 < c1) {
+      fetch(a, c0);
+      if (L::AHEAD) fetch(b, c0 + 1);
+      normalise(a);
+      commit(a);
+      commit_k(a, c0);
+    }
+    lds_barrier();  // B1 of the first chunk
+    if constexpr (L::AHEAD) {
+      for (int n = c0; n < c1;) {  // ways out lead out of the loop: they do not join the count of loads in flight
+        step(a, b, n);
+        if (++n >= c1) break;
+        step(b, a, n++);
+      }
+    } else {
+      for (int n = c0; n < c1; ++n) step(a, a, n);
     }
     return;
   }
@@ -333,7 +397,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
       for (int c = 0; c < NC; ++c) b[c] = S.operand(c, ks);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const Frag a = load_rows(sK, LDK, i, ks, lane);
+        const Frag a = load_rows(k_tile(n), LDK, i, ks, lane);
 #pragma unroll
         for (int c = 0; c < NC; ++c) S16::mma(y[c][i], a, b[c]);
       }
@@ -432,8 +496,8 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
     const float dec = sc[Sc::DEC];
     lds_barrier();  // B2
     if (GATE == LNX_GATE_SCALAR) S.scale(dec);
-    S.add(sK, LDK, bu, fresh(tid & 63));
-    lds_barrier();  // B3
+    S.add(k_tile(n), LDK, bu, fresh(tid & 63));
+    if (!L::AHEAD) lds_barrier();  // B3
     if (n + 1 < c1) save(n + 1);
     lds_barrier();  // B1 of the next chunk
   }
@@ -446,7 +510,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
   constexpr int BV = L::BV, LDK = L::LDK, LDC = L::LDC, LDV = L::LDV, LDT = L::LDT;
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);
-  T* sQ = sK + L::kRow;
+  T* sQ = sK + L::NK2 * L::kRow;
   T* sTm = sQ + L::kRow;
   T* sP = sTm + L::kC;
   T* sdO = sP + L::kC;
@@ -456,57 +520,97 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   Chain ch;
   if (!chain_of<BV>(p, ch)) return;
+  auto k_tile = [&](int n) { return sK + (L::AHEAD ? (n & 1) * L::kRow : 0); };
   const int N = p.geom.N, c0 = ch.c0, c1 = ch.c1, v0 = ch.v0;
 
   if (wave >= NCW) {
     // ---------------- movers ----------------
     const int mt = tid - 64 * NCW;
-    TileRegs<T, 64, DK> rK, rQ;
-    TileRegs<T, 64, BV> rdO;
-    PlacedTri rTm, rP;
-    RowFactors fk, fq;
-    Scalars<GATE> rs;
-    rTm.init(LDC, mt), rP.init(LDC, mt);
+    struct Chunk {
+      TileRegs<T, 64, DK> K, Q;
+      TileRegs<T, 64, BV> dO;
+      PlacedTri Tm, P;
+      RowFactors<L::AHEAD> fk, fq;
+      Scalars<GATE> sc;
+    };
+    Chunk a, b;
+    a.Tm.init(LDC, mt), a.P.init(LDC, mt), b.Tm.init(LDC, mt), b.P.init(LDC, mt);
     zero_upper(sTm, LDC, L::kC, mt);
     const int64_t tsk = (int64_t)p.geom.ts * DK, tsv = (int64_t)p.geom.ts * p.dv;
-    auto fetch = [&](int n) {
+    auto fetch = [&](Chunk& R, int n, int part = -1) __attribute__((always_inline)) {  // part 0: Q, 1: K, 2: the rest; < 0: everything
+      n = max(n, c0);
       const int64_t slot = (int64_t)ch.row * N + n;
       int tok0, len;
       chunk_span(ch.span, n, tok0, len);
       const int64_t tbase = tok_index(p.geom, ch.row, tok0);
-      rdO.load(p.d_o + tbase * p.dv + v0, tsv, len, mt);
-      rP.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
-      rTm.load(at<const T>(p.ws, p.off.Tm) + slot * 64 * 64, mt);
-      rs.load(p, slot, tbase, len, mt);
-      rQ.load(p.q + tbase * DK, tsk, len, mt);
-      fq.load(at<const float>(p.ws, p.off.Nq) + slot * 64, mt);
-      rK.load(p.k + tbase * DK, tsk, len, mt);
-      fk.load(at<const float>(p.ws, p.off.Nk) + slot * 64, mt);
+      if (part < 0 || part == 2) {
+        R.dO.load(p.d_o + tbase * p.dv + v0, tsv, len, mt);
+        R.P.load(at<const T>(p.ws, p.off.P) + slot * 64 * 64, mt);
+        R.Tm.load(at<const T>(p.ws, p.off.Tm) + slot * 64 * 64, mt);
+        R.sc.load(p, slot, tbase, len, mt);
+      }
+      if (part < 0 || part == 0) {
+        R.Q.load(p.q + tbase * DK, tsk, len, mt);
+        R.fq.load(at<const float>(p.ws, p.off.Nq) + slot * 64, mt);
+      }
+      if (part < 0 || part == 1) {
+        R.K.load(p.k + tbase * DK, tsk, len, mt);
+        R.fk.load(at<const float>(p.ws, p.off.Nk) + slot * 64, mt);
+      }
     };
-    auto commit = [&]() {
-      rdO.store(sdO, LDV, mt);
-      rP.store(sP);
-      rTm.store(sTm);
-      rs.put(sc, p.scale, mt);
-      store_rows(rQ, fq, p.l2norm, sQ, LDK, mt);
+    auto normalise = [&](Chunk& R, int part = -1) __attribute__((always_inline)) {
+      if (p.l2norm && part != 1) scale_rows(R.Q, R.fq, mt);
+      if (p.l2norm && part != 0) scale_rows(R.K, R.fk, mt);
     };
-    if (c0 < c1) {
-      fetch(c1 - 1);
-      commit();
-      store_rows(rK, fk, p.l2norm, sK, LDK, mt);
-    }
-    lds_barrier();  // B1 of the first chunk
-    for (int n = c1 - 1; n >= c0; --n) {
-      fetch(max(n - 1, c0));
+    auto commit = [&](const Chunk& R) __attribute__((always_inline)) {
+      R.dO.store(sdO, LDV, mt);
+      R.P.store(sP);
+      R.Tm.store(sTm);
+      R.sc.put(sc, p.scale, mt);
+      store_rows(R.Q, sQ, LDK, mt);
+    };
+    auto step = [&](Chunk& cur, Chunk& nxt, int n) __attribute__((always_inline)) {  // as in the forward pass
+      if constexpr (L::AHEAD) {
+        fetch(cur, n - 2, 2);
+        fetch(cur, n - 2, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        normalise(nxt, 1);
+        store_rows(nxt.K, k_tile(n - 1), LDK, mt);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(cur, n - 2, 1);
+      } else {
+        fetch(cur, n - 1);
+      }
       lds_barrier();  // B2
       int tok0, len;
       chunk_span(ch.span, n, tok0, len);
       unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.dD) + ((int64_t)ch.row * N + n) * p.dv * 64 + (int64_t)v0 * 64, 64, sdRT, LDT, BV, mt);
       unstage_tile_checked<T, 64, BV>(p.dv_out + tok_index(p.geom, ch.row, tok0) * p.dv + v0, tsv, sdV, LDV, len, mt);
-      commit();
-      lds_barrier();  // B3
-      store_rows(rK, fk, p.l2norm, sK, LDK, mt);
+      normalise(nxt, 0);
+      commit(nxt);
+      if (!L::AHEAD) {
+        lds_barrier();  // B3
+        normalise(nxt, 1);
+        store_rows(nxt.K, sK, LDK, mt);
+      }
       lds_barrier();  // B1 of the next chunk
+    };
+    if (c0 < c1) {
+      fetch(a, c1 - 1);
+      if (L::AHEAD) fetch(b, c1 - 2);
+      normalise(a);
+      commit(a);
+      store_rows(a.K, k_tile(c1 - 1), LDK, mt);
+    }
+    lds_barrier();  // B1 of the first chunk
+    if constexpr (L::AHEAD) {
+      for (int n = c1 - 1; n >= c0;) {
+        step(a, b, n);
+        if (--n < c0) break;
+        step(b, a, n--);
+      }
+    } else {
+      for (int n = c1 - 1; n >= c0; --n) step(a, a, n);
     }
     return;
   }
@@ -533,7 +637,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
       for (int c = 0; c < NC; ++c) b[c] = dS.operand(c, ks);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const Frag a = load_rows(sK, LDK, i, ks, lane);
+        const Frag a = load_rows(k_tile(n), LDK, i, ks, lane);
 #pragma unroll
         for (int c = 0; c < NC; ++c) S16::mma(z[c][i], a, b[c]);
       }
@@ -609,8 +713,8 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
     dS.add(sQ, LDK, foq, lane);
     lds_barrier();  // B2
     // ---- dS += K^T dY ----
-    dS.add(sK, LDK, by, lane);
-    lds_barrier();  // B3
+    dS.add(k_tile(n), LDK, by, lane);
+    if (!L::AHEAD) lds_barrier();  // B3
     if (n > c0) save(n - 1);
     lds_barrier();  // B1 of the next chunk
   }

@@ -65,3 +65,30 @@ def test_wide_slabs_against_the_oracle(gate, T):
         ref = delta_rule_adjoint(y["q"], y["k"], y["v"], y["beta"], c(do), y.get("g"), c(dS), None, y["s0"], False)
         err = {"o": max_rel(c(o), o_ref), "S": max_rel(c(S), S_ref), **{n: max_rel(c(got[n]), ref["dS0" if n == "s0" else "d" + n]) for n in got}}
         assert all(e < 2e-2 for e in err.values()), (b, h, err)
+
+
+@pytest.mark.parametrize("T,cu", [(1, None), (64, None), (129, None), (250, None), (330, None),
+                                  (500, [0, 0, 1, 64, 129, 129, 130, 131, 200, 264, 265, 270, 300, 500])])
+@pytest.mark.parametrize("gate", [False, True])
+def test_normalised_rows_at_every_width(gate, T, cu, monkeypatch):
+    """Rows normalised inside the kernels, where the narrow slabs' movers hold two chunks: no, one, even and odd numbers of chunks."""
+    from linearnexus_amd import linear_attn as m
+    B, H, dv = (1 if cu else 13), 16, 128
+    torch.manual_seed(T)
+    r = lambda *s: torch.randn(*s, device=DEV)
+    x = [r(B, H, T, 256).bfloat16(), r(B, H, T, 256).bfloat16(), r(B, H, T, dv).bfloat16(), -0.1 * torch.rand(B, H, T, device=DEV) if gate else None,
+         torch.rand(B, H, T, device=DEV)]
+    do, dS = r(B, H, T, dv).bfloat16(), r(13, H, 256, dv) * 0.1
+    cu = None if cu is None else torch.tensor(cu, dtype=torch.int32, device=DEV)
+
+    def run(slab):
+        monkeypatch.setitem(m._test_hooks, "scan_slab", slab)
+        t = [None if u is None else u.clone().requires_grad_(True) for u in x]
+        o, S = m._chunk_forward(*t, None, 256 ** -0.5, True, torch.bfloat16, cu, forward_only=False)[:2]
+        o2, S2 = m._chunk_forward(*x, None, 256 ** -0.5, True, torch.bfloat16, cu, forward_only=True)[:2]
+        assert torch.equal(o, o2) and torch.equal(S, S2)
+        return [o.detach(), S.detach(), *torch.autograd.grad([o, S], [u for u in t if u is not None], [do, dS])]
+
+    auto, wide, narrow = run(0), run(64), run(32)
+    for a, b, c in zip(auto, wide, narrow):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b) and torch.equal(a, c)
