@@ -55,7 +55,8 @@ typedef struct lnx_scan_args {
   int32_t gate;             /* lnx_gate */
   int32_t use_qk_l2norm;    /* normalise q, k rows as x / (|x|_2 + 1e-6) inside the op: always honoured by the decode step
                                and the token-by-token scan; by the chunk entry points where lnx_chunk_normalises_qk
-                               says so (ABI version 6), d_q and d_k are then the gradients of the raw q and k */
+                               says so (ABI version 9; before it lnx_chunk_fuses_l2norm, since version 6), d_q and d_k
+                               are then the gradients of the raw q and k */
   int32_t nseq;             /* number of packed sequences; 0 for a dense batch */
   float scale;              /* multiplies q (after normalisation) */
   int32_t forward_only;     /* lnx_chunk_fwd: no backward pass will follow, do not write the per-chunk tensors
@@ -109,13 +110,18 @@ typedef struct lnx_scan_args {
   float* d_gate_A_log;
   float* d_gate_bias;
 
-  /* Test hooks (ABI version 8); a binding leaves both 0 = the library's choice.  Neither changes results or the
-     workspace layout, only which of two tilings of the same kernel runs, so that tests reach both at small shapes. */
+  /* Test hooks (ABI version 8); a binding leaves both 0 = the library's choice.  Neither changes the workspace layout or, but for one
+     case, results, only which of two tilings of the same kernel runs, so that tests reach both at small shapes.  The case: the forward
+     pass of a per-channel gate in bf16 with dk <= 128 runs one of two kernels (32: the chain in registers, 64: the one through LDS),
+     whose results differ by the order of fp32 sums. */
   int32_t test_scan_slab;       /* 32 or 64: value columns per workgroup of the sequential kernels */
   int32_t test_out_slabs;       /* > 0: value slabs per workgroup of the fp32 output kernel */
 } lnx_scan_args;
 
-/* Library identification; also the symbol a loader probes first. */
+/* Library identification; also the symbol a loader probes first.  Version 9: lnx_chunk_bwd reads the values of a per-channel gate
+   again (bf16, dk <= 128; until then only whether g was given), so g must still hold what lnx_chunk_fwd was given; the chunk
+   entry points normalise q and k themselves for more shapes (lnx_chunk_normalises_qk, new; lnx_chunk_fuses_l2norm answers 1 at
+   dk = 256 too). */
 int lnx_abi_version(void);
 const char* lnx_last_error(void);
 
@@ -142,7 +148,8 @@ int lnx_recurrent_fwd(const lnx_scan_args* a, void* hip_stream);
  * workspace, unchanged, to lnx_chunk_bwd (unless forward_only was set), with the same shape, dtype, gate, nseq,
  * token_first, scale and use_qk_l2norm fields: the layout of the workspace follows from B, H, T, dk, dv, dtype, gate
  * and nseq alone (o_dtype does not enter it), and there is exactly one set of kernels per such shape.
- * q, k, v, beta and a per-channel gate (g or gate_raw) are read again by lnx_chunk_bwd and must hold the same values.
+ * q, k, v, beta and a per-channel gate (g since ABI version 9, or gate_raw) are read again by lnx_chunk_bwd and must hold the same
+ * values.
  * Shapes: dk in {64, 128, 256} (256 is the head_dim of the reference's Gated DeltaNet presets,
  * models.py:142-143), dv a multiple of 64.  q, k, v, o, a per-channel gate (g or gate_raw), the states, the workspace
  * and the gradients of all of these must be 16-byte aligned (the kernels move their rows as 16-byte vectors);

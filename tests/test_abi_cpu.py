@@ -36,7 +36,7 @@ def test_library_exports_every_declared_symbol():
     assert set(names) >= set(_lib.EXPORTS)
     for n in names:
         assert hasattr(lib, n), n
-    assert lib.lnx_abi_version() == 8
+    assert lib.lnx_abi_version() == 9
 
 
 def test_struct_layout_matches_header():
@@ -47,6 +47,28 @@ def test_struct_layout_matches_header():
     assert _lib.ScanArgs.gate_raw.offset == 216 and _lib.ScanArgs.gate_threshold.offset == 240
     assert _lib.ScanArgs.d_gate_raw.offset == 248 and _lib.ScanArgs.test_out_slabs.offset == 276
     assert ctypes.sizeof(_lib.ScanArgs) == 280
+
+
+def test_contract_of_version_9():
+    """What changed with the version: which shapes normalise q and k inside (the older query answers for calls without a per-channel gate
+    alone), and that a gate is needed again by the gradients.  What the queries deny, the entry points refuse."""
+    lib = _lib.load()
+    for dtype in (_lib.LNX_F32, _lib.LNX_BF16):
+        for dk in (64, 128, 256):
+            for gate in (_lib.GATE_NONE, _lib.GATE_SCALAR, _lib.GATE_VECTOR):
+                a = _lib.ScanArgs(B=1, H=1, T=64, dk=dk, dv=64, chunk=64, dtype=dtype, o_dtype=dtype, gate=gate, use_qk_l2norm=1)
+                vector = gate == _lib.GATE_VECTOR
+                inside = dtype == _lib.LNX_BF16 and not (vector and dk == 256)
+                assert lib.lnx_chunk_normalises_qk(a) == inside and lib.lnx_chunk_fuses_l2norm(a) == (inside and not vector)
+                a.q = a.k = a.v = a.beta = a.o = a.final_state = a.g = _aligned_dummy()
+                a.workspace, a.workspace_bytes = _aligned_dummy(), 0  # refused before anything is dereferenced
+                status, text = lib.lnx_chunk_fwd(a, None), lib.lnx_last_error()
+                assert (b"workspace" in text) if inside else (status == -2 and b"use_qk_l2norm" in text), (status, text)
+                if gate != _lib.GATE_NONE:
+                    a.d_o = a.d_q = a.d_k = a.d_v = a.d_beta = a.d_g = _aligned_dummy()
+                    a.use_qk_l2norm, a.g = 0, None
+                    assert lib.lnx_chunk_bwd(a, None) == -1 and b"needs g" in lib.lnx_last_error()
+    assert lib.lnx_chunk_normalises_qk(None) == 0
 
 
 def test_one_kernel_set_per_shape_and_no_environment_dispatch():
