@@ -34,7 +34,8 @@ struct BwdParams {
   float* ds0;
   int dv, gate, l2norm;
   int slab;  // lnx_scan_args.test_scan_slab
-  // per-channel gate activated inside the op (lnx_scan_args.gate_raw): bwd_wy2 carries dg through the activation
+  // per-channel gate activated inside the op (lnx_scan_args.gate_raw): bwd_wy2, or kda_bwd_chunk for 2-byte inputs with dk <= 128, carries
+  // dg through the activation
   const void* graw;
   const float* gA;
   const float* gbias;

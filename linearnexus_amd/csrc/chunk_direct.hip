@@ -1045,7 +1045,7 @@ int launch_scan_bwd(const DirectParams& p, int nstate, hipStream_t st) {
 // Measured per workgroup at B8 H16 T4096 d128 (wall clock of wave 0, 2 workgroups per CU): 4.3 us until the first slab
 // is there, 6.2 us for the loop, 2.1 us staging K, Q and the four small tiles, 1.8 us for the epilogue's products and
 // 3.4 us until dq, dk have left -- memory latency at every step; the kernel moves 4.9 TB/s.
-// dk = 256: 896 KB a chunk at dv = 512, most of it the two states; B8 H8 T4096 790 us, 4.6 TB/s.
+// dk = 256: 896 KB a chunk at dv = 512, most of it the two states; B8 H8 T4096 788 us, 4.8 TB/s.
 // ---------------------------------------------------------------------------------------
 template <int DK> struct BChunkL {
   // dk = 256: eight waves, one workgroup per CU -- the [64 x dk] accumulators of four would take 192 registers, the slabs of two
@@ -1070,7 +1070,8 @@ template <int DK> struct BChunkL {
   static_assert(kSt <= (OVER2 ? 2 : 4) * kC, "the staging tile overlays the small tiles");
   // The gate gradient's row dots <q_t, dq_t> - <k_t, dk_t> from the accumulators, before anything is rounded (what one pair of tokens gives
   // to both cancels along the chunk): dg is 4.0e-3 off instead of 6.5e-3.  dk <= 128 takes them from the staged rows, which its
-  // emit reads anyway: 7.0e-3.
+  // emit reads anyway: 7.0e-3.  The accumulators would halve that, too, but move the sums over all tokens that callers form of dg (A_log's and
+  // dt_bias' gradients, whose terms nearly cancel) by up to 3 %, as much as they are off: a change of results, left.
   static constexpr bool DOTS = DK == 256;
   static constexpr int nfloat = 64 * 10;
   static constexpr size_t bytes = sizeof(float) * nfloat + (epi_bytes > loop_bytes ? epi_bytes : loop_bytes);

@@ -1475,7 +1475,8 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   // forward only / states saved as well, by the number of its workgroups (two to a 64-column slab):
   //   dk = 128   8 .. 128: 57.5 -> 45 / 58.5 -> 49    192: 59.6 -> 46.3 / 87 -> 72    224: 71 -> 53.8 / 89.8 -> 87.5    240: 71.2 -> 59.6 / 91.3 -> 102    256: 74 -> 73 .. 79 / 93 -> 108
   //   dk = 64    8 .. 128: 64 -> 36 / 66 -> 38.5      192: 67.5 -> 40.2 / 90.8 -> 64.3    224: 70.8 -> 55.3 / 91.3 -> 78.9    256: 72.2 -> 68 / 95 -> 88.5
-  // On a full chip the tiles come at the rate of HBM, and at dk = 128 its one chunk in flight is too little.
+  // On a full chip the tiles come at the rate of HBM, and at dk = 128 its one chunk in flight is too little.  The line is that of the form that
+  // saves the states: forward only, 225 to 240 workgroups would still gain at dk = 128.
   if constexpr (sizeof(T) == 2 && DK <= 128) {
     const int64_t wide = (int64_t)nstate * p.geom.H * (p.dv / 64);
     if (p.slab ? p.slab == 32 : wide <= (DK == 128 ? 112 : 128)) return lnx_kda_scan_fwd(direct_params(p, GATE), DK, nstate, st);

@@ -722,7 +722,14 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
 }
 
 // Width of the slabs: the cheapest by rounds of 256 workgroups times the time of a chunk, which grows less than the width
-// because every workgroup loads the chunk's K, Q and W (relative times; at one round of workgroups 8.6 us with 128 columns).
+// because every workgroup loads the chunk's K and Q (relative times).  One round, us a chunk, few workgroups .. all 256:
+//   32 columns   forward 2.8 .. 3.3 (nothing saved 2.6 .. 2.8)   reverse 2.6 .. 3.2
+//   64           3.5 .. 4.9 (2.9 .. 3.7)                         3.1 .. 5.2
+//   128          6.9 .. 7.2 (5.5)                                6.1 .. 6.5
+// Up to 256 workgroups of 128 columns the choice is the fastest, also for forms that save nothing: T4096 dv128, forward / reverse, 64 heads
+// 209 / 203 us with 32 columns, 263 / 263 with 64; 96 heads 385 / 380 and 275 / 281; 128 heads 311 / 331 with 64 and 461 / 414 with 128; 160 heads
+// 545 / 545 and 476 / 431.  Beyond, where 128 columns take two rounds and 64 three, 64 would be faster by up to 15 % (T1024, 320 heads
+// 233 / 243 against 267 / 262; 448 heads 314 / 321 against 294 / 286).
 int slab_width(const DirectParams& p, int nstate) {
   if (p.slab == 32 || p.slab == 64) return p.slab;
   const int64_t chains = (int64_t)nstate * p.geom.H;

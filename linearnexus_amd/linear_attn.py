@@ -291,11 +291,11 @@ def _prefill_segments(B: int, H: int, T: int, dv: int, dk: int = 256, two_byte: 
 
     dk <= 128: the first pass has w = B H (dk + dv) / 64 workgroups per segment, so 256 / w segments fill the chip once.
     Segments of 16 chunks or more, but eight of them where the chip has room (a segment's step costs as much as two chunks).
-    The lines are where the gain starts, bf16 d128 unless said (both sides as they are now; where a call beside a line lost, as the line was
-    drawn): 4 heads of 4096 tokens 83 -> 62 us (2048: 52 -> 62), 4 heads of 16384 298 -> 107, 16 heads (w = 64) of 8192 170 -> 131 (4096:
-    98 -> 101), 32 heads never.  The kernels that form W and U prepare both passes: no gain at w = 64; fp32 4 heads of 4096
-    275 -> 175 us, bf16 per-channel gate 4 heads of 8192 185 -> 131 (4096: 104 -> 112).  From 512 chunks on, w = 64 gains from a second
-    round (32768 tokens: 806 -> 395).
+    bf16 d128 unless said, one chain -> cut, on the kernels as they are: 4 heads of 4096 tokens 85 -> 59 us, of 16384 306 -> 103; 16 heads
+    (w = 64) of 8192 174 -> 124, of 32768 690 -> 385 in eight segments (four: 422).  The kernels that form W and U prepare both passes: fp32 4
+    heads of 4096 275 -> 175, bf16 per-channel gate 4 heads of 8192 185 -> 130 (4096: 103 -> 111, so not), w = 64 never (8192: 289 -> 346).
+    The lines were drawn on a slower first pass: what lies before them would often gain, too, at w <= 32 from 48 chunks on (4 heads of 3072 tokens 67 -> 54; 2048: 49 -> 49), at w = 64 from 64 on (4096 tokens 93 -> 80; 3072: 73 ->
+    71), past w = 64 from 128 on at d64 (40 heads of 8192 tokens 164 -> 140) and from 256 on at d128 (20 heads of 16384 351 -> 311).
 
     dk = 256, and rows that would have to be copied to become heads: at most an eighth of the CUs busy and every segment keeps >= 64 chunks
     (fewer heads of 512 values gain less than their longer preparation costs: 16 workgroups of 4096 tokens 196 -> 216 us)."""
@@ -317,12 +317,12 @@ def _prefill_segments(B: int, H: int, T: int, dv: int, dk: int = 256, two_byte: 
 
 def _prefill_segments_256(B: int, H: int, T: int, dv: int) -> int:
     """The same for dk = 256 in bf16 without a per-channel gate, where the first pass forms no outputs and the second finds everything prepared.
-    A chain takes 3.3 us a chunk, cutting costs a setup and a short step per segment, so it pays from 32 chunks on while w <= 64 (H4 dv 512,
-    w = 48: 2048 tokens 117 -> 110 us, 4096 217 -> 153, 8192 420 -> 206) and from 64 on while w <= 128 (H8 dv 512, w = 96: 2048 tokens
-    117 -> 122, 4096 221 -> 174, 8192 427 -> 278; H16 dv 256, w = 128: 4096 227 -> 181), never beyond (H12 dv 512, w = 144:
-    8192 tokens 437 -> 495).  Eight segments; four where w or a short prompt leaves
-    them too little (2048 tokens, w = 24: 108 against 120 us; w = 96, 8192: 278 against 307), sixteen of few heads and long prompts
-    (16384 tokens, w = 24: 265 against 274; w = 48: 367 against 309)."""
+    A chain takes 2.5 us a chunk (3.3 when the lines were drawn), cutting costs a setup and a short step per segment.  One chain -> cut, us:
+    w <= 64 (H4 dv 512, w = 48) 3072 tokens 133 -> 119, 4096 171 -> 149, 8192 333 -> 196; w <= 128 (H8 dv 512, w = 96) 4096 175 -> 165, 8192 338 ->
+    258 (2048: 94 -> 119, so not); never beyond (H12 dv 512, w = 144: 8192 tokens 352 -> 450 and more).  Between 32 and some 40 chunks the cut now
+    loses (2048 tokens, w = 12 94 -> 98, w = 48 95 -> 102, w = 64 94 -> 104).  Eight segments; four where w or a short prompt leaves them too little
+    (w = 96, 8192 tokens: 258 against 300; they would be the better choice up to 96 chunks at w = 48, too: 4096 tokens 137 against 149), sixteen of
+    few heads and long prompts (w = 5, 32768 tokens: 284 against 348; w = 48: 544 against 484)."""
     chunks, w = -(-T // CHUNK), B * H * (4 + -(-dv // 64))
     if os.environ.get("LNX_PREFILL_SEGMENTS") is not None:
         return _prefill_segments(B, H, T, dv)
