@@ -1045,7 +1045,7 @@ int launch_scan_bwd(const DirectParams& p, int nstate, hipStream_t st) {
 // Measured per workgroup at B8 H16 T4096 d128 (wall clock of wave 0, 2 workgroups per CU): 4.3 us until the first slab
 // is there, 6.2 us for the loop, 2.1 us staging K, Q and the four small tiles, 1.8 us for the epilogue's products and
 // 3.4 us until dq, dk have left -- memory latency at every step; the kernel moves 4.9 TB/s.
-// dk = 256: 896 KB a chunk at dv = 512, most of it the two states; B8 H8 T4096 788 us, 4.8 TB/s.
+// dk = 256: 896 KB a chunk at dv = 512, most of it the two states; B8 H8 T4096 788 - 795 us, 4.8 TB/s.
 // ---------------------------------------------------------------------------------------
 template <int DK> struct BChunkL {
   // dk = 256: eight waves, one workgroup per CU -- the [64 x dk] accumulators of four would take 192 registers, the slabs of two

@@ -17,7 +17,7 @@
 // set s of 64 and all tokens, so that an accumulator element is at the place where pair_levels wants its channel and token:
 // lane (c = lane % 16, kq = lane / 16) holds the tokens 16 t + 4 kq + e of channel c, and everything between the loop and the
 // tiles on their way out happens in registers.  The four pair sums share their factors (pair_sums).
-// Measured at B4 H16 T8192 d128 (8192 chunks): 472 us for 280 KB a chunk, 4.9 TB/s, and two thirds of the time on vector instructions (the
+// Measured at B4 H16 T8192 d128 (8192 chunks): 461 - 472 us by box for 280 KB a chunk, 5 TB/s, and two thirds of the time on vector instructions (the
 // normalisation adds about 20 us to it and kda_prepare together, the gate's activation 65); bwd_dqk and bwd_wy2, which passed dW, a partial dk
 // and an fp32 partial gradient of the gate through memory, 402 + 497 us behind and before 217 us of normalisation outside.  The cumulative gate
 // is summed up again from the gate: 461 -> 470 us here, 25 less where the prepare kernel wrote it.  With eight waves and one workgroup per CU

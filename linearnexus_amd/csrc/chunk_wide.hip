@@ -23,10 +23,10 @@
 // With one chunk held and converted where it is stored, between the barriers, 4 heads dv 256 of 8192 tokens took 418 us forward only and 849
 // with gradients, more than the WY split's kernels (360 and 769, the normalisation ahead of them); so 331 and 743.  The movers' loads and
 // conversions in turn, a tile at a time, and Q's conversion behind B2 in reverse are 366 -> 349 and 368 -> 326 us of the scans.
-// Measured at B8 H8 T4096 dv512 (128-column slabs, 256 workgroups): forward 498 us, reverse 448 us, 7.8 and 7 us a chunk, of which
+// Measured at B8 H8 T4096 dv512 (128-column slabs, 256 workgroups): forward 498 - 510 us, reverse 448 - 459 us by box, 7.9 and 7.1 us a chunk, of which
 // 185 KB through the CU's memory path (64 KB of state per chunk and slab leave for the backward kernels) are most.  The WY split's
 // passes, which read W and U instead of Tm and V, took 521 and 435 us behind 205 us of preparation (now 68) and 221 us of normalisation
-// outside the kernels (now none), and before two more kernels of 804 and 289 us (now one of 788): the step 2478 -> 1830 us.
+// outside the kernels (now none), and before two more kernels of 804 and 289 us (now one of 788 - 795): the step 2478 -> 1830 us.
 // State stores among the products of the first phase instead of
 // behind the last barrier: 551 -> 587 and 464 -> 521 us (a wave whose store waits for a slot multiplies nothing).
 
