@@ -78,20 +78,24 @@ template <typename T, int DK> struct Prep2Cfg {
   static constexpr int kTile = 64 * LDC;
   static constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
   static constexpr size_t mat = sizeof(float) * 64 * LNX_LDA;  // one fp32 64x64 matrix
-  static constexpr size_t scr = sizeof(float) * 32 * 36;       // scratch of the inverse's block merges
-  // Two regions, each used by one thing at a time (2-byte inputs: 18 + 0.5 + 21.5 KB = 40 KB, four workgroups per CU):
-  //   region 0: A (fp32)                      -> after the inverse: Tw, Tu tiles
-  //   region 2: K, Q slab tiles, then P       -> Tm (fp32) + merge scratch -> loop-2 slab and result tiles
+  // Two regions, each used by one thing at a time:
+  //   region 0: A (fp32), inverted in place   -> Tw, Tu tiles
+  //   region 2: K, Q slab tiles, then P       -> loop-2 slab and result tiles
   static constexpr size_t r0 = cmax(mat, 2 * kTile * sizeof(T));
   static constexpr size_t r1 = sizeof(float) * 128;  // beta, G
-  static constexpr size_t r2 = cmax(mat + scr, 2 * kTile * sizeof(T));
+  static constexpr size_t r2 = 2 * kTile * sizeof(T);
   static constexpr size_t bytes = r0 + r1 + r2;
-  // LITE: the slab tiles, then A inverted in place + merge scratch | beta, G, row factors | P   (31.5 KB, five per CU)
-  static constexpr size_t lite_bytes = mat + scr + sizeof(float) * 256 + kTile * sizeof(T);
+  // LITE: the slab tiles, then A, inverted in place | beta, G, row factors | P   (28.5 KB, five per CU)
+  static constexpr size_t lite_tiles = cmax(mat, 2 * kTile * sizeof(T));
+  static constexpr size_t lite_bytes = lite_tiles + sizeof(float) * 256 + kTile * sizeof(T);
 };
 
 // LITE: stop after the inverse and leave Tm itself (row-major) next to Pm and G -- all that the kernels of
 // chunk_direct.hip read; V is not touched.
+// Bound by its 41 KB a chunk (d128) once the chip is full, by the chain of the inverse where it is not.  The pair products are formed
+// transposed, so that rows of A and P leave the fragments as vectors (25 LDS writes of 2 and 4 bytes a lane before), the wave whose tile lies
+// above the diagonal forms nothing, and the inverse takes a third of the instructions it took (tri_inverse_64): B8 H16 T4096 d128 88 -> 78 us
+// (71 with neither inverse nor decays), one prompt of 65536 tokens and 4 heads 46 -> 41, dk = 256 71.5 -> 68.
 template <typename T, int DK, int GATE, bool LITE = false>
 __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdParams p) {
   typedef Prep2Cfg<T, DK> L;
@@ -100,16 +104,14 @@ __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdPa
   float* sA = reinterpret_cast<float*>(smem);      // region 0 (LITE: over the slab tiles)
   T* sTw = reinterpret_cast<T*>(smem);             //   Tw, Tu once the inverse is done with A
   T* sTu = sTw + L::kTile;
-  float* sBeta = reinterpret_cast<float*>(smem + (LITE ? L::mat + L::scr : L::r0));
+  float* sBeta = reinterpret_cast<float*>(smem + (LITE ? L::lite_tiles : L::r0));
   float* sG = sBeta + 64;
   char* reg2 = LITE ? smem : smem + L::r0 + L::r1;  // region 2
   T* sKa = reinterpret_cast<T*>(reg2);             //   K slab of the first loop, then P
   T* sQa = sKa + L::kTile;                         //   Q slab
-  float* sT = reinterpret_cast<float*>(reg2);      //   Tm
-  float* sX = reinterpret_cast<float*>(reg2 + L::mat);
   T* sIn = sKa;                                    //   second loop: slab in, result out
   T* sOut = sQa;
-  T* sPt = LITE ? reinterpret_cast<T*>(smem + L::mat + L::scr + sizeof(float) * 256) : sKa;  // P on its way out
+  T* sPt = LITE ? reinterpret_cast<T*>(smem + L::lite_tiles + sizeof(float) * 256) : sKa;  // P on its way out
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int N = p.geom.N;
@@ -163,8 +165,9 @@ __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdPa
       rQ.load(qg + 64 * (s_ + 1), tsk, len, tid);
     }
     if (!(wi == 0 && wj == 1)) {
-      mma_nt<T, 1, 1>(ax, sKa + 32 * wi * LDC, LDC, sKa + 32 * wj * LDC, LDC, 64, lane);
-      mma_nt<T, 1, 1>(ap, sQa + 32 * wi * LDC, LDC, sKa + 32 * wj * LDC, LDC, 64, lane);
+      // transposed: the lane's token is i of tile wi, its elements are runs of four j of tile wj, what a row of A or P takes as one vector
+      mma_nt<T, 1, 1>(ax, sKa + 32 * wj * LDC, LDC, sKa + 32 * wi * LDC, LDC, 64, lane);
+      mma_nt<T, 1, 1>(ap, sKa + 32 * wj * LDC, LDC, sQa + 32 * wi * LDC, LDC, 64, lane);
     }
     if (LITE && p.l2norm) {
       const int r = tid >> 2, c0 = (tid & 3) * 16;
@@ -202,36 +205,41 @@ __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdPa
   };
   if (!LITE) fetch(0);
   lds_barrier();  // slab tiles dead
-  {
-    // the per-row scalars of this lane's sixteen fragment rows (four runs of four) first, as vectors: read one by one
-    // between the stores below, each read waited for its own round trip to LDS (the stores might alias them)
-    floatx4 gi[4], bi[4], nki[4], nqi[4];
-    const int j = 32 * wj + frag_col(lane);
+  if (wi >= wj) {  // the packed tiles hold nothing of the one above the diagonal
+    const int i = 32 * wi + frag_col(lane);
+    const float gi = sG[i], ba = sBeta[i] * (LITE ? sNk[i] : 1.f), sp = p.scale * (LITE ? sNq[i] : 1.f);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int i0 = 32 * wi + 8 * q + 4 * (lane >> 5);
-      gi[q] = load4(sG + i0);
-      bi[q] = load4(sBeta + i0);
-      if (LITE) nki[q] = load4(sNk + i0), nqi[q] = load4(sNq + i0);
-    }
-    const float gj = sG[j], nkj = LITE ? sNk[j] : 1.f;
-    floatx16 pe[1][1];
+      const int j0 = 32 * wj + 8 * q + 4 * (lane >> 5);
+      floatx4 f = {1.f, 1.f, 1.f, 1.f}, a, pe;
+      if (GATE != LNX_GATE_NONE) {
+        const floatx4 gj = load4(sG + j0);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int i = 32 * wi + frag_row(e, lane), q = e >> 2, u = e & 3;
-      const float dec = (GATE == LNX_GATE_NONE) ? 1.f : __expf(fminf(gi[q][u] - gj, 0.f));
-      const float fx = LITE ? nki[q][u] * nkj : 1.f, fp = LITE ? nqi[q][u] * nkj : 1.f;
-      sA[i * LNX_LDA + j] = (i > j) ? bi[q][u] * dec * fx * ax[0][0][e] : 0.f;
-      pe[0][0][e] = (i >= j) ? p.scale * dec * fp * ap[0][0][e] : 0.f;
+        for (int u = 0; u < 4; ++u) f[u] = __expf(fminf(gi - gj[u], 0.f));
+      }
+      if (LITE) f *= load4(sNk + j0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        a[u] = (wi > wj || i > j0 + u) ? ba * f[u] * ax[0][0][4 * q + u] : 0.f;
+        pe[u] = (wi > wj || i >= j0 + u) ? sp * f[u] * ap[0][0][4 * q + u] : 0.f;
+      }
+      store4(sA + i * LNX_LDA + j0, a);
+      store4(sPt + i * LDC + j0, pe);
     }
-    frag_store<T, 1, 1>(pe, sPt + 32 * wi * LDC + 32 * wj, LDC, lane);
+  } else if (!LITE) {
+    for (int q = 0; q < 4; ++q) {
+      const int o = 8 * q + 4 * (lane >> 5);
+      store4(sA + frag_col(lane) * LNX_LDA + 32 + o, floatx4{0.f, 0.f, 0.f, 0.f});
+      store4(sPt + frag_col(lane) * LDC + 32 + o, floatx4{0.f, 0.f, 0.f, 0.f});
+    }
   }
   lds_barrier();
   // LITE, 2-byte inputs: Pm and Tm leave packed (TriRegs in mma_tiles.h), only the vectors at or below the diagonal;
   // this thread's vector tid and, for tid < 32, vector 256 + tid
   int tr0 = 0, tc0 = 0, tr1 = 0, tc1 = 0;
   const bool tri2 = tid < LNX_TRI_VECS - 256;
-  if constexpr (LITE && sizeof(T) == 2) {
+  if constexpr (LITE) {
+    static_assert(sizeof(T) == 2, "packed tiles");
     tri_vec_pos(tid, tr0, tc0);
     tri_vec_pos(tri2 ? 256 + tid : 0, tr1, tc1);
     T* Pg = ws_ptr<T>(p, p.off.P) + slot * 64 * 64;
@@ -241,30 +249,18 @@ __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdPa
   } else {
     unstage_tile<T, 64, 64>(ws_ptr<T>(p, p.off.P) + slot * 64 * 64, 64, sPt, LDC, 64, tid);
   }
-  if constexpr (LITE) {
-    tri_inverse_64<true>(sA, sA, sX, tid);
-  } else {
-    lds_barrier();  // Tm is built over the P tile
-    tri_inverse_64(sA, sT, sX, tid);
-  }
+  tri_inverse_64<LITE>(sA, tid, (int)(slot >> 3) & 3);  // the solving wave differs between the workgroups of a CU
   if constexpr (LITE) {
     T* Tm = ws_ptr<T>(p, p.off.Tm) + slot * 64 * 64;
-    if constexpr (sizeof(T) == 2) {
-      typedef unsigned uint2_ __attribute__((ext_vector_type(2)));
-      typedef unsigned uint4_ __attribute__((ext_vector_type(4)));
-      auto put = [&](int idx, int r, int c) {
-        const float* src = sA + r * LNX_LDA + 8 * c;
-        const uint2_ lo = __builtin_bit_cast(uint2_, pack_bf16x4(load4(src))), hi = __builtin_bit_cast(uint2_, pack_bf16x4(load4(src + 4)));
-        *reinterpret_cast<uint4_*>(Tm + 8 * idx) = uint4_{lo[0], lo[1], hi[0], hi[1]};
-      };
-      put(tid, tr0, tc0);
-      if (tri2) put(256 + tid, tr1, tc1);
-    } else {
-      for (int idx = tid; idx < 64 * 16; idx += 256) {
-        const int r = idx >> 4, c = (idx & 15) * 4;
-        store4(Tm + r * 64 + c, load4(sA + r * LNX_LDA + c));
-      }
-    }
+    typedef unsigned uint2_ __attribute__((ext_vector_type(2)));
+    typedef unsigned uint4_ __attribute__((ext_vector_type(4)));
+    auto put = [&](int idx, int r, int c) {
+      const float* src = r >= 32 && c < 4 ? sA + (r - 32) * LNX_LDA + 32 + 8 * c : sA + r * LNX_LDA + 8 * c;
+      const uint2_ lo = __builtin_bit_cast(uint2_, pack_bf16x4(load4(src))), hi = __builtin_bit_cast(uint2_, pack_bf16x4(load4(src + 4)));
+      *reinterpret_cast<uint4_*>(Tm + 8 * idx) = uint4_{lo[0], lo[1], hi[0], hi[1]};
+    };
+    put(tid, tr0, tc0);
+    if (tri2) put(256 + tid, tr1, tc1);
     return;
   }
   {
@@ -273,7 +269,8 @@ __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdPa
     const int r0 = (tid >> 4) * 4, c0 = (tid & 15) * 4;
     floatx4 t[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) t[i] = load4(sT + (r0 + i) * LNX_LDA + c0);
+    for (int i = 0; i < 4; ++i) t[i] = load4(sA + (r0 + i) * LNX_LDA + c0);
+    lds_barrier();  // Tw and Tu take Tm's place
     const floatx4 bu = load4(sBeta + c0);
     floatx4 bw = bu;
     if (GATE != LNX_GATE_NONE) {
@@ -737,7 +734,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
     }
   }
   lds_barrier();
-  tri_inverse_64(sA, sT, sX, tid);
+  tri_inverse_64(sA, tid, (int)(slot >> 3) & 3);
 
   // ---- phase C: Tm^T to the workspace; Tm and Tm diag(beta) as MFMA operands ----
   T* sTm = sK;
@@ -748,7 +745,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
     const int r0 = (tid >> 4) * 4, c0 = (tid & 15) * 4;
     floatx4 t[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) t[i] = load4(sT + (r0 + i) * LNX_LDA + c0);
+    for (int i = 0; i < 4; ++i) t[i] = load4(sA + (r0 + i) * LNX_LDA + c0);
     const floatx4 bu = load4(sBeta + c0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

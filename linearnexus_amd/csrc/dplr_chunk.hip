@@ -543,7 +543,7 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
   put_tri(tx, w, ab, m.ab, [](floatx4 y_) { return -y_; });
   put_rows(tk, w, z);
   lds_barrier();
-  tri_inverse_64<true>(tx, tx, L.sx, threadIdx.x);
+  tri_inverse_64(tx, threadIdx.x);
   {
     floatx4 W[4], u[4];
     clear(W), clear(u);
@@ -851,7 +851,7 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   put_rows(tz, w, z);
   put_rows(ty, w, y);
   lds_barrier();
-  tri_inverse_64<true>(Tm, Tm, L.sx, threadIdx.x);
+  tri_inverse_64(Tm, threadIdx.x);
   floatx4 u[4], du[4];  // rows n, columns t
   clear(u), clear(du);
   upto(w.j, [&](auto b_) {

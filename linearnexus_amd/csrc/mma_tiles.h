@@ -571,79 +571,76 @@ __device__ __forceinline__ void rows_reduce_add(float (&v)[16 * MT], int row0, i
   if (MT == 2 || (lane & 1) == 0) atomicAdd(&rows[row0 + 32 * i + frag_row(e, lane)], total);
 }
 
-// ---------------------------------------------------------------------------------------
-// 16x16 fp32 products on v_mfma_f32_16x16x4_f32, operands row-major in LDS
-//   returns C[i][j] = sum_k A[i][k] * B[k][j];  fragment: c[e] is row 4*(lane>>4)+e, col lane&15
-// ---------------------------------------------------------------------------------------
-__device__ __forceinline__ floatx4 mm16_f32(const float* A, int lda, const float* B, int ldb, int K, int lane) {
-  floatx4 c = {0.f, 0.f, 0.f, 0.f};
-  const int i = lane & 15, kq = lane >> 4;
-  for (int k0 = 0; k0 < K; k0 += 4) {
-    const float a = A[i * lda + k0 + kq];
-    const float b = B[(k0 + kq) * ldb + i];
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  return c;
-}
-
-__device__ __forceinline__ void mm16_store(float* dst, int ld, floatx4 c, int lane, float sign) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) dst[(4 * (lane >> 4) + e) * ld + (lane & 15)] = sign * c[e];
-}
-
 #define LNX_LDA 68  // leading dimension of the fp32 64x64 matrices in LDS
 
-// In-LDS inverse of the unit lower-triangular matrix I + A (A strictly lower, 64x64, fp32,
-// leading dimension LNX_LDA):  Tm = (I + A)^-1.  `sA` is read only; `sT` receives the full
-// matrix (upper triangle zero); `sX` is a [32][36] fp32 scratch.  Must be called by all THREADS
-// threads of the workgroup, of which the first 256 work.  Diagonal 16x16 blocks by forward substitution, then two levels of block merges
-//   [[L0, 0], [B, L1]]^-1 = [[L0^-1, 0], [-L1^-1 B L0^-1, L1^-1]].
-// In place (sT == sA, INPLACE): A's upper triangle and diagonal must hold zeros; every block of A is read for the last
-// time before the barrier that precedes the write of the same block of Tm.
-template <bool INPLACE = false, int THREADS = 256>
-__device__ __forceinline__ void tri_inverse_64(const float* sA, float* sT, float* sX, int tid) {
-  const int wave = tid >> 6, lane = tid & 63;
-  if (!INPLACE) {
-    for (int idx = tid; idx < 64 * LNX_LDA; idx += THREADS) sT[idx] = 0.f;
-    lds_barrier();
-  }
-  if (lane < 16 && wave < 4) {
-    const int r0 = 16 * wave, c = lane;
+// In-LDS inverse of the unit lower-triangular matrix I + A: `M` holds A (strictly lower, zeros on and above the diagonal of the 16x16 diagonal
+// blocks, 64x64, fp32, leading dimension LNX_LDA) and receives Tm = (I + A)^-1.  Called by the 256 threads of a workgroup.  Wave `solver` takes
+// the four diagonal blocks by forward substitution, sixteen lanes each, a lane a column of the inverse; then two levels of block merges
+//   [[L0, 0], [B, L1]]^-1 = [[L0^-1, 0], [-L1^-1 B L0^-1, L1^-1]]
+// on v_mfma_f32_16x16x4_f32: a product's result fragment (rows 4 g + r, column l16) is the right operand of the next as it is, with the
+// contraction index of step r being 4 g + r in both (a left operand is then one 16-byte read), so a merge needs no scratch and no barrier of its
+// own.  ABOVE: the lower left 32x32 block of Tm stays in the place above the diagonal (rows 0 .., columns 32 ..), which spares the barrier
+// between the last reads of that block of A and its writes.
+// A chunk's inverse is a serial chain that other workgroups of the CU have to cover: with every wave solving a block and the merges' products
+// through LDS it took seven barriers and 730 instructions of forward substitution instead of 180 (B4 H16 T8192 d128 kda_prepare 374 -> 361 us,
+// RWKV-7's chunk kernels 994 -> 975 of 2095).
+template <bool ABOVE = false> __device__ __forceinline__ void tri_inverse_64(float* M, int tid, int solver = 0) {
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  if (wave == solver) {
+    float* D = M + 16 * g * (LNX_LDA + 1);
     float d[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float s = (i == c) ? 1.f : 0.f;
+    for (int i = 0; i < 16; ++i) d[i] = (i == l16) ? 1.f : 0.f;
 #pragma unroll
-      for (int m = 0; m < i; ++m) s -= sA[(r0 + i) * LNX_LDA + r0 + m] * d[m];
-      d[i] = s;
+    for (int m4 = 0; m4 < 4; ++m4) {  // by columns of A: what a solved row takes off the later ones
+      floatx4 a[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (i > 4 * m4) a[i] = load4(D + i * LNX_LDA + 4 * m4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (i > 4 * m4 + u) d[i] -= a[i][u] * d[4 * m4 + u];
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) sT[(r0 + i) * LNX_LDA + r0 + c] = d[i];
+    for (int i = 0; i < 16; ++i) D[i * LNX_LDA + l16] = d[i];
   }
   lds_barrier();
-  // level 1: blocks (1,0) and (3,2) of the 16x16 grid, one per wave 0/1
-  float* sXw = sX + (wave & 1) * 16 * 36;
-  const int b = 32 * (wave & 1);  // super-block origin
-  if (wave < 2) {
-    floatx4 x = mm16_f32(sA + (b + 16) * LNX_LDA + b, LNX_LDA, sT + b * LNX_LDA + b, LNX_LDA, 16, lane);
-    mm16_store(sXw, 36, x, lane, 1.f);
+  auto rows = [&](int i0, int k0) { return load4(M + (i0 + l16) * LNX_LDA + k0 + 4 * g); };
+  auto add = [&](floatx4& c, floatx4 a, floatx4 b) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
+  };
+  auto cols = [&](int k0, int j0) {
+    const float* p = M + (k0 + 4 * g) * LNX_LDA + j0 + l16;
+    return floatx4{p[0], p[LNX_LDA], p[2 * LNX_LDA], p[3 * LNX_LDA]};
+  };
+  auto put = [&](floatx4 c, int i0, int j0) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) M[(i0 + 4 * g + r) * LNX_LDA + j0 + l16] = -c[r];
+  };
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  if (wave < 2) {  // blocks (1, 0) and (3, 2) of the 16x16 grid
+    const int b = 32 * wave;
+    floatx4 x = zero, y = zero;
+    add(x, rows(b + 16, b), cols(b, b));
+    add(y, rows(b + 16, b + 16), x);
+    put(y, b + 16, b);
   }
   lds_barrier();
-  if (wave < 2) {
-    floatx4 y = mm16_f32(sT + (b + 16) * LNX_LDA + b + 16, LNX_LDA, sXw, 36, 16, lane);
-    mm16_store(sT + (b + 16) * LNX_LDA + b, LNX_LDA, y, lane, -1.f);
-  }
-  lds_barrier();
-  // level 2: the 32x32 lower-left block, one 16x16 output per wave
-  const int bi = 16 * (wave >> 1), bj = 16 * (wave & 1);
-  if (THREADS == 256 || wave < 4) {
-    floatx4 x = mm16_f32(sA + (32 + bi) * LNX_LDA, LNX_LDA, sT + bj, LNX_LDA, 32, lane);
-    mm16_store(sX + bi * 36 + bj, 36, x, lane, 1.f);
-  }
-  lds_barrier();
-  if (THREADS == 256 || wave < 4) {
-    floatx4 y = mm16_f32(sT + (32 + bi) * LNX_LDA + 32, LNX_LDA, sX + bj, 36, 32, lane);
-    mm16_store(sT + (32 + bi) * LNX_LDA + bj, LNX_LDA, y, lane, -1.f);
-  }
+  const int bi = wave >> 1, bj = wave & 1;  // block (2 + bi, bj); both triangular factors have one block of zeros
+  floatx4 y = zero;
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+    if (r <= bi) {
+      floatx4 x = zero;
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        if (k >= bj) add(x, rows(32 + 16 * r, 16 * k), cols(16 * k, 16 * bj));
+      add(y, rows(32 + 16 * bi, 32 + 16 * r), x);
+    }
+  if (!ABOVE) lds_barrier();  // the block of A has been read
+  put(y, ABOVE ? 16 * bi : 32 + 16 * bi, (ABOVE ? 32 : 0) + 16 * bj);
   lds_barrier();
 }
