@@ -127,6 +127,13 @@ inline bool lnx_chunk_direct(const lnx_scan_args* a) {
 // G then holds the chunks' last rows alone, [slot][dk]: the scans want e^{G_C}, and the gradient kernel sums the gate up itself.
 template <typename T, int DK> constexpr bool lnx_gate_last_only = sizeof(T) == 2 && DK <= 128;
 template <typename T, int DK> __device__ __forceinline__ int64_t gate_last(int64_t slot) { return lnx_gate_last_only<T, DK> ? slot * DK : (slot * LNX_C + LNX_C - 1) * DK; }
+// A chunk whose gates are none above zero and whose whole decay is above 2^-LNX_KDA_NEAR in every channel (of a set of 64): with the middle of a
+// channel's decay as the reference, e^{G - mid} and e^{mid - G} lie within 2^+-40, far from the ends of a bf16's or fp32's range also in the
+// products of pairs that are masked afterwards (up to 2^80), and one such factor a token takes the place of one per level.  A chunk of 64 tokens
+// forgets that much at 0.87 nats a token.  B4 H16 T8192 d128 forward and backward, one level against the levels: kda_prepare 317 and 372 us,
+// kda_bwd_chunk 454 - 466 and 480 - 488 (at the rate of HBM); B2 T2048 51 and 59, 74 and 84 of 237 and 256.  Either is as exact as the other or
+// better (o 3.8e-3 and 4.0e-3 off fp64, dg 3.6e-3 and 4.6e-3): the scaled rows of one level are held to more than bf16.
+constexpr float LNX_KDA_NEAR = 80.f;
 inline bool lnx_chunk_kda(const lnx_scan_args* a) { return a->dtype == LNX_BF16 && a->dk <= 128 && a->gate == LNX_GATE_VECTOR; }
 
 // The gradient that a chunk's right-hand side R = diag(beta) (V - ..) gets, dR, leaves the reverse scans once, as the rows of dv = beta dR, and

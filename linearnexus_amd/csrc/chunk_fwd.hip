@@ -413,6 +413,27 @@ template <bool LOG2> __device__ __forceinline__ void kda_pair_half(floatx4 (&a32
   }
 }
 
+// The same sums where a chunk's whole decay fits a factor (kda_near): E_ij = exp(G_i - m) exp(m - G_j) with one m per channel, so that every pair is
+// of one level and the tiles Kr, Qr (rows times exp(G - m)) and Kc (times exp(m - G)) are plain operands.  Kc comes in two parts, rounded and
+// what the rounding left: at the levels, too, a pair of neighbours has one operand or both with a factor of 1, unrounded, and with both rounded
+// here o was up to 4 % further off fp64 (gates of 0.4 a token).  A wave's blocks are those above; the diagonal one's accumulators are one a product.
+__device__ __forceinline__ void kda_pair_near(floatx4 (&a32)[2], floatx4& a16, floatx4 (&aF)[2], const bf16_t* __restrict__ Kr, const bf16_t* __restrict__ Qr,
+                                              const bf16_t* __restrict__ Kc, int ldc, int wave, int lane) {
+  const int o = (lane & 15) * ldc + 8 * (lane >> 4);
+  auto op = [&](const bf16_t* tile, int block) { return pair_row_raw(tile + 16 * block * ldc + o); };
+  const int ti = 2 + (wave >> 1), t16 = (wave < 2) ? 1 : 3;
+  const PairOp k32 = op(Kr, ti), q32 = op(Qr, ti), r16 = op((wave & 1) ? Qr : Kr, t16), kd = op(Kr, wave), qd = op(Qr, wave);
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const bf16_t* part = Kc + u * 64 * ldc;
+    const PairOp c32 = op(part, wave & 1), c16 = op(part, t16 - 1), cd = op(part, wave);
+    pair_mma(a32[0], k32, c32);
+    pair_mma(a32[1], q32, c32);
+    pair_mma(a16, r16, c16);
+    pair_mma(aF[0], kd, cd);
+    pair_mma(aF[1], qd, cd);
+  }
+}
 
 // ---------------------------------------------------------------------------------------
 // kda_prepare: chunk_prepare for a per-channel (vector) gate.  The pairwise products carry the
@@ -433,6 +454,8 @@ template <typename T, int DK> struct KdaPrepSmem {
   // output staging); the P accumulator / inverse; inverse scratch; beta, and where the rows are normalised inside their factors
   static constexpr bool NORM = sizeof(T) == 2 && DK <= 128;
   static constexpr size_t bytes = sizeof(T) * 2 * kTile + sizeof(float) * (64 * LDF + 2 * 64 * LNX_LDA + 32 * 36 + (NORM ? 192 : 64));
+  static __device__ __forceinline__ float* seg(float* sX) { return sX + 32 * 36 - 384; }  // 384 floats of phase A
+  static_assert(sizeof(T) == 4 || sizeof(T) * 2 * kTile <= sizeof(float) * (64 * LNX_LDA + 32 * 36 - 384), "the column operands end before them");
 };
 
 // GRAW: the gate arrives as the block's raw projection and is activated here, g = -exp(A_log[h]) softplus(raw + bias)
@@ -449,8 +472,10 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   float* sT = sA + 64 * LNX_LDA;
   T* sKb = reinterpret_cast<T*>(sA);  // LAST: beta K e^G [64][LDKB] from phase A to D
   constexpr int LDKB = DK + L::PAD;
+  T* sKc = reinterpret_cast<T*>(sT);  // LAST: K e^{mid - G} of the half, rounded, and behind it what the rounding left; reaches into sX
   float* sX = sT + 64 * LNX_LDA;
   float* sBeta = sX + 32 * 36;
+  float* sDiag = L::seg(sX) + 320;  // <q_t, k_t> over the halves whose pairs are of one level, from the rows themselves
   float* sNk = sBeta + 64;  // NORM: 1 / (|x| + eps) of the k and q rows
   float* sNq = sNk + 64;
 
@@ -567,14 +592,16 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   // (1, 0) or (3, 2) (level 16), and the diagonal block w of both products, one accumulator per level 8, 4, 2, 1 (each
   // level has its own mask) plus the plain <q_i, k_i> diagonal.
   constexpr bool LEVELS = sizeof(T) == 2;
-  floatx4 a32[2], a16, aD[5][2];
+  floatx4 a32[2], a16, aD[5][2], aF[2];
+  aF[0] = aF[1] = floatx4{0.f, 0.f, 0.f, 0.f};
   a32[0] = a32[1] = a16 = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < 5; ++u) aD[u][0] = aD[u][1] = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (int idx = tid; idx < 64 * LNX_LDA; idx += 256) {  // the diagonal blocks accumulate here over the halves
-    sA[idx] = 0.f;
-    sT[idx] = 0.f;
-  }
+  if constexpr (!LEVELS)
+    for (int idx = tid; idx < 64 * LNX_LDA; idx += 256) {  // the diagonal blocks accumulate here over the halves
+      sA[idx] = 0.f;
+      sT[idx] = 0.f;
+    }
 
 #pragma unroll 1
   for (int h = 0; h < NH; ++h) {
@@ -590,46 +617,80 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       float gs[16];  // the segment's sixteen values in registers: all loads in flight together, one write each
 #pragma unroll
       for (int i = 0; i < 16; ++i) gs[i] = sG[(16 * seg + i) * LDF + c] * UNIT;
+      float highest = -1.f;
+      if (LAST) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) highest = fmaxf(highest, gs[i]);
+      }
 #pragma unroll
       for (int i = 1; i < 16; ++i) gs[i] += gs[i - 1];
-      float* sSeg = sX;  // segment totals [4][64] (the inverse's scratch is free here)
+      float* sSeg = L::seg(sX);  // segment totals [4][64]
       sSeg[seg * 64 + c] = gs[15];
       lds_barrier();
       float off = 0.f;
       for (int s_ = 0; s_ < seg; ++s_) off += sSeg[s_ * 64 + c];
 #pragma unroll
       for (int i = 0; i < 16; ++i) sG[(16 * seg + i) * LDF + c] = gs[i] + off;
+      if (LAST) {
+        const bool all = __ballot(!(highest <= 0.f && gs[15] + off >= -LNX_KDA_NEAR)) == 0;  // (NaN shows in the sum)
+        if (c == 0) sSeg[256 + seg] = all ? 1.f : 0.f;
+      }
     }
     lds_barrier();
+    bool near = false;  // this half's pairs are of one level
+    if (LAST) {
+      const floatx4 f = load4(L::seg(sX) + 256);
+      near = __builtin_amdgcn_readfirstlane(f[0] + f[1] + f[2] + f[3] == 4.f);
+    }
     // G, K e^{G_last - G}, scale Q e^G of this half -> workspace.  LAST: of G only the last row, but beta K e^G for phase D into the tile that
     // later held A, which goes to the gate's instead.  The rows of G were 32 KB written a chunk, and a second exponential of all of them in
     // phase D (B4 H16 T8192 d128, forward and backward: 1568 us; beta K e^G through the place of W 1528, 16 KB that left and came back).
     {
       T* Krg = ws_ptr<T>(p, p.off.Kr) + slot * 64 * DK + 64 * h;
       T* Qgg = ws_ptr<T>(p, p.off.Qg) + slot * 64 * DK + 64 * h;
+      const int tid = LAST ? fresh(threadIdx.x) : (int)threadIdx.x, c = (tid & 15) * 4;
+      const floatx4 gl = load4(sG + 63 * LDF + c), mid = 0.5f * gl;
+      floatx4 em;  // e^mid
+#pragma unroll
+      for (int e = 0; e < 4; ++e) em[e] = near ? gate_exp<LAST>(mid[e]) : 1.f;
 #pragma unroll
       for (int it = 0; it < 4; ++it) {
-        const int idx = tid + 256 * it, r = idx >> 4, c = (idx & 15) * 4;
-        const floatx4 gr = load4(sG + r * LDF + c), gl = load4(sG + 63 * LDF + c);
+        const int r = (tid + 256 * it) >> 4;
+        const floatx4 gr = load4(sG + r * LDF + c);
         const floatx4 kk = load4(sK + r * LDC + c), qq = load4(sQ + r * LDC + c);
         const float bt = sBeta[r];
-        floatx4 kr, qgv, kb;
+        floatx4 f, fi, eg, er;  // e^{G - mid}, e^{mid - G}, e^G, e^{G_last - G}
+        if (near) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float eg = gate_exp<LAST>(gr[e]);
-          kr[e] = kk[e] * gate_exp<LAST>(fminf(gl[e] - gr[e], 0.f));
-          qgv[e] = qq[e] * p.scale * eg;
-          kb[e] = kk[e] * bt * eg;
+          for (int e = 0; e < 4; ++e) f[e] = gate_exp<LAST>(gr[e] - mid[e]), fi[e] = gate_exp<LAST>(mid[e] - gr[e]);
+          eg = f * em, er = fi * em;
+          store4(sK + r * LDC + c, kk * f);
+          store4(sQ + r * LDC + c, qq * f);
+          const floatx4 kc = kk * fi;
+          const bf16x4 hi = pack_bf16x4(kc);
+          *reinterpret_cast<bf16x4*>(sKc + r * LDC + c) = hi;
+          store4(sKc + L::kTile + r * LDC + c, kc - floatx4{(float)hi[0], (float)hi[1], (float)hi[2], (float)hi[3]});
+          const float d = row16_sum(qq[0] * kk[0] + qq[1] * kk[1] + qq[2] * kk[2] + qq[3] * kk[3]);
+          if ((tid & 15) == 0) sDiag[r] = h > 0 ? sDiag[r] + d : d;
+        } else {
+          if (LAST && h == 0 && (tid & 15) == 0) sDiag[r] = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) eg[e] = gate_exp<LAST>(gr[e]), er[e] = gate_exp<LAST>(fminf(gl[e] - gr[e], 0.f));
         }
-        if constexpr (LAST) store4(sKb + r * LDKB + 64 * h + c, kb);
+        if constexpr (LAST) store4(sKb + r * LDKB + 64 * h + c, kk * bt * eg);
         else store4(Gg + r * DK + 64 * h + c, gr);
-        store4(Krg + r * DK + c, kr);
-        store4(Qgg + r * DK + c, qgv);
+        store4(Krg + r * DK + c, kk * er);
+        store4(Qgg + r * DK + c, qq * p.scale * eg);
       }
       if (LAST && tid < 16) store4(Gg + 64 * h + 4 * tid, load4(sG + 63 * LDF + 4 * tid) * (1.f / LOG2E));
     }
-    if constexpr (LEVELS) {
-      kda_pair_half<LAST>(a32, a16, aD, reinterpret_cast<const bf16_t*>(sK), reinterpret_cast<const bf16_t*>(sQ), LDC, sG, LDF, wave, lane);
+    if (near) {
+      if constexpr (LAST) {
+        lds_barrier();
+        kda_pair_near(a32, a16, aF, reinterpret_cast<const bf16_t*>(sK), reinterpret_cast<const bf16_t*>(sQ), reinterpret_cast<const bf16_t*>(sKc), LDC, wave, lane);
+      }
+    } else if constexpr (LEVELS) {
+      kda_pair_half<LAST>(a32, a16, aD, reinterpret_cast<const bf16_t*>(sK), reinterpret_cast<const bf16_t*>(sQ), LDC, sG, LDF, wave, LAST ? fresh(lane) : lane);
     } else {
     // blocks below the diagonal: six blocks x two products = twelve tasks, three per wave
 #pragma unroll
@@ -702,8 +763,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       const int x = il ^ l16;
       const float va = x >= 8 ? aD[0][0][e] : x >= 4 ? aD[1][0][e] : x >= 2 ? aD[2][0][e] : aD[3][0][e];
       const float vp = x >= 8 ? aD[0][1][e] : x >= 4 ? aD[1][1][e] : x >= 2 ? aD[2][1][e] : x == 1 ? aD[3][1][e] : aD[4][1][e];
-      sA[(16 * wave + il) * LNX_LDA + 16 * wave + l16] = va;
-      sT[(16 * wave + il) * LNX_LDA + 16 * wave + l16] = vp;
+      sA[(16 * wave + il) * LNX_LDA + 16 * wave + l16] = va + aF[0][e];
+      sT[(16 * wave + il) * LNX_LDA + 16 * wave + l16] = vp + (LAST && x == 0 ? sDiag[16 * wave + il] : aF[1][e]);
     }
   } else {
 #pragma unroll

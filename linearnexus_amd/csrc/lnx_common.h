@@ -103,10 +103,14 @@ __device__ __forceinline__ float xor32_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-__device__ __forceinline__ float wave_sum(float x) {
-  // inside a row of 16 lanes with DPP (no LDS crossbar): quads, the two quads of a half row, the two half rows
+// Sum over a row of 16 lanes, in every lane, with DPP (no LDS crossbar): quads, the two quads of a half row, the two half rows
+__device__ __forceinline__ float row16_sum(float x) {
   x = quad_sum(x);
   x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x141, 0xF, 0xF, true));  // row_half_mirror: lane i <-> 7 - i
-  x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x128, 0xF, 0xF, true));  // row_ror:8 = lane ^ 8
+  return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x128, 0xF, 0xF, true));  // row_ror:8 = lane ^ 8
+}
+
+__device__ __forceinline__ float wave_sum(float x) {
+  x = row16_sum(x);
   return xor32_sum(xor16_sum(x));
 }

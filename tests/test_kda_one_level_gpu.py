@@ -1,0 +1,92 @@
+"""bf16 per-channel gates whose chunk's whole decay fits one factor a token (LNX_KDA_NEAR, csrc/chunk_common.h: 80 in units of log 2, per set of 64
+channels in kda_prepare and per sixteen channels in kda_bwd_chunk) take their pairs in one level, others in a hierarchy of levels: both, the
+limit between them and calls that mix them, against the fp64 oracle."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import max_rel
+from oracle import recurrent as rc
+from oracle.adjoint import delta_rule_adjoint
+from oracle.inputs import make_inputs, to_bf16_grid
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+LIMIT = 80 * np.log(2.0) / 64  # mean decay of a token at the limit, full chunk
+
+
+def _gates(which, T, dk, rng):
+    g = -rng.random((1, 2, T, dk)).astype(np.float32)
+    whole = lambda scale: g / g.reshape(1, 2, -1, 64, dk).sum(3).repeat(64, 2).reshape(g.shape) * -64 * LIMIT * scale if T % 64 == 0 else g
+    if which == "below":
+        return whole(0.999)
+    if which == "above":
+        return whole(1.001)
+    if which == "one_channel":  # of the second chunk, in the last set: the others stay in one level
+        g *= 0.1
+        g[:, :, 64:128, dk - 3] = -3.0
+        return g
+    if which == "one_token":
+        g *= 0.1
+        g[:, :, 70] = -200.0
+        return g
+    if which == "zero":
+        return np.zeros_like(g)
+    assert which == "ragged"
+    return g * 0.3
+
+
+@pytest.mark.parametrize("l2", [False, True])
+@pytest.mark.parametrize("dk", [64, 128])
+@pytest.mark.parametrize("which,T", [("below", 128), ("above", 128), ("one_channel", 192), ("one_token", 192), ("zero", 128), ("ragged", 65), ("ragged", 33), ("ragged", 143)])
+def test_forward_and_gradients(which, T, dk, l2):
+    import linearnexus_amd as la
+    x = make_inputs(7, 1, 2, T, dk, 64, gate="vector", with_state=True, with_grad=True, normalize=not l2)
+    x["g"] = np.ascontiguousarray(_gates(which, T, dk, np.random.default_rng(1)), np.float32)
+    for n in ("q", "k", "v", "dO"):
+        x[n] = to_bf16_grid(x[n])
+    leaves = {n: torch.from_numpy(x[n]).to(DEV).to(torch.bfloat16 if n in "qkv" else torch.float32).requires_grad_(True) for n in ("q", "k", "v", "g", "beta", "S0")}
+    o, S = la.kda_chunkwise(leaves["q"], leaves["k"], leaves["v"], leaves["g"], leaves["beta"], None, leaves["S0"], 64, l2)
+    grads = torch.autograd.grad([o, S], list(leaves.values()), [torch.from_numpy(x["dO"]).to(DEV), torch.from_numpy(x["dS"]).to(DEV)])
+    d = {n: a.astype(np.float64) for n, a in x.items()}
+    ro, rS = rc.kda_recurrent(d["q"], d["k"], d["v"], d["g"], d["beta"], None, d["S0"], l2)
+    ref = delta_rule_adjoint(x["q"], x["k"], x["v"], x["beta"], x["dO"], x["g"], x["dS"], None, x["S0"], l2)
+    errs = {"o": max_rel(o.detach().cpu().numpy(), ro), "S": max_rel(S.detach().cpu().numpy(), rS)}
+    errs.update({"d" + n: max_rel(t.float().cpu().numpy(), ref["d" + n]) for n, t in zip(leaves, grads)})
+    assert all(e < 2e-2 for e in errs.values()), errs
+
+
+@pytest.mark.parametrize("dk", [64, 128])
+def test_limit_joins_its_two_sides(dk):
+    """Gates a millionth on either side of the limit are the same gates to bf16: what differs is the way."""
+    import linearnexus_amd as la
+    x = make_inputs(8, 1, 2, 128, dk, 64, gate="vector", with_grad=True)
+    x["g"] = np.ascontiguousarray(_gates("below", 128, dk, np.random.default_rng(2)), np.float32)
+
+    def run(scale):
+        leaves = [torch.from_numpy(x[n] * (scale if n == "g" else 1)).to(DEV).to(torch.bfloat16 if n in "qkv" else torch.float32).requires_grad_(True)
+                  for n in ("q", "k", "v", "g", "beta")]
+        o, _ = la.kda_chunkwise(*leaves, use_qk_l2norm=False)
+        return [o.detach(), *torch.autograd.grad(o, leaves, torch.from_numpy(x["dO"]).to(DEV))]
+
+    for a, b in zip(run(1.0), run(1.0 / 0.998)):  # 0.999 -> 1.001 of the limit
+        a, b = a.float(), b.float()
+        assert (a - b).norm() < 2e-2 * b.norm()  # each within 1e-2 of the same values
+
+
+def test_gates_above_zero_and_nan_keep_the_levels():
+    """A gate above zero is outside the domain (its decay reads as 1 between neighbours at the levels) and is not taken to 2^+40 powers either:
+    finite results; NaN stays in its own head."""
+    import linearnexus_amd as la
+    x = make_inputs(9, 1, 2, 128, 64, 64, gate="vector", with_grad=True)
+    x["g"][:, 0, 5, 3] = 1e-3
+    leaves = [torch.from_numpy(x[n]).to(DEV).to(torch.bfloat16 if n in "qkv" else torch.float32).requires_grad_(True) for n in ("q", "k", "v", "g", "beta")]
+    o, _ = la.kda_chunkwise(*leaves, use_qk_l2norm=False)
+    gr = torch.autograd.grad(o, leaves, torch.from_numpy(x["dO"]).to(DEV))
+    assert all(torch.isfinite(t).all() for t in (o, *gr))
+    x["g"][:, 1, 70, 3] = np.nan
+    leaves = [torch.from_numpy(x[n]).to(DEV).to(torch.bfloat16 if n in "qkv" else torch.float32).requires_grad_(True) for n in ("q", "k", "v", "g", "beta")]
+    o2, _ = la.kda_chunkwise(*leaves, use_qk_l2norm=False)
+    gr2 = torch.autograd.grad(o2, leaves, torch.from_numpy(x["dO"]).to(DEV))
+    assert torch.equal(o2[:, 0], o[:, 0]) and torch.isnan(o2[:, 1, 70:]).any()
+    assert all(torch.equal(a[:, 0], b[:, 0]) for a, b in zip(gr, gr2))
