@@ -218,6 +218,14 @@ template <int NC> struct Strip {
 #pragma unroll
         for (int e = 0; e < 4; ++e) dst[(int64_t)(row0(ci) + grp(lane) + e) * dv + 16 * c + (lane & 15)] = x[c][ci][e];
   }
+  // What is formed of the state is formed again behind this: operands kept from one product for the next were 64 registers, which went to
+  // scratch memory
+  __device__ __forceinline__ void settle() {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int ci = 0; ci < KT; ++ci) asm volatile("" : "+v"(x[c][ci]));
+  }
   __device__ __forceinline__ Frag operand(int c, int ks) const { return S16::from_acc(x[c][2 * ks], x[c][2 * ks + 1]); }
   __device__ __forceinline__ void save(T* dst, int lane) const {  // [value column][dk] of the strip
 #pragma unroll
@@ -225,22 +233,77 @@ template <int NC> struct Strip {
 #pragma unroll
       for (int ks = 0; ks < NK; ++ks) *reinterpret_cast<bf16x8*>(dst + (16 * c + (lane & 15)) * DK + 32 * ks + 8 * (lane >> 4)) = operand(c, ks);
   }
-  __device__ __forceinline__ void scale(float f) {
+  // LDS reads go out two groups of products ahead (R rows of operands at a time) where a wave has two column tiles: left to the compiler they went
+  // out in front of the products that take them, 7950 cycles a chunk until D and O are there, 5900 so (2430 of products).  B8 H8 T4096 dv = 512
+  // forward scan 506 -> 452 us (5.1 TB/s of what HBM carries a chunk), nothing saved 375 -> 317.  With one column tile the compiler's order is as
+  // fast in reverse and 1 % faster forward.
+  static constexpr bool PIPED = NC == 2;
+  // x = f x + tile^T b: rows of the tile (tokens) contracted
+  template <bool SCALED> __device__ __forceinline__ void add(const T* tile, int ld, const Frag (&b)[NC][2], int lane, float f = 1.f) {
+    if constexpr (!PIPED) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int ci = 0; ci < KT; ++ci) x[c][ci] *= f;
-  }
-  // x += tile^T b: rows of the tile (tokens) contracted
-  __device__ __forceinline__ void add(const T* tile, int ld, const Frag (&b)[NC][2], int lane) {
+        for (int ci = 0; ci < KT; ++ci)
+          if (SCALED) x[c][ci] *= f;
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+      for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int ci = 0; ci < KT; ++ci) {
-        const Frag f = load_cols(tile, ld, s, ci, lane);
+        for (int ci = 0; ci < KT; ++ci) {
+          const Frag a = load_cols(tile, ld, s, ci, lane);
 #pragma unroll
-        for (int c = 0; c < NC; ++c) S16::mma(x[c][ci], f, b[c][s]);
+          for (int c = 0; c < NC; ++c) S16::mma(x[c][ci], a, b[c][s]);
+        }
+    } else {
+      constexpr int NG = 2 * KT / 4;
+      Frag a[3][4];
+      auto load = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[g % 3][j] = load_cols(tile, ld, 4 * g / KT, (4 * g) % KT + j, lane);
+      };
+      load(0), load(1);
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        if (g + 2 < NG) load(g + 2);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            floatx4& y = x[c][(4 * g) % KT + j];
+            if (SCALED && 4 * g < KT) y *= f;
+            S16::mma(y, a[g % 3][j], b[c][4 * g / KT]);
+          }
+        __builtin_amdgcn_sched_barrier(0);
       }
+    }
+  }
+  // y[c][i] += rows of tile i0 + i (tokens) times x, or the other way round (COLS: columns = tokens)
+  template <int NI, bool COLS> __device__ __forceinline__ void rows_times(floatx4 (&y)[NC][NI], const T* tile, int ld, int i0, int lane) const {
+    constexpr int AHEAD = PIPED ? (NI == 4 ? 2 : 3) : 0;
+    Frag a[AHEAD + 1][NI];
+    auto load = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) a[ks % (AHEAD + 1)][i] = load_rows(tile, ld, i0 + i, ks, lane);
+    };
+#pragma unroll
+    for (int ks = 0; ks < AHEAD; ++ks) load(ks);
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) {
+      if (PIPED && ks + AHEAD < NK) load(ks + AHEAD);
+      Frag b[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) b[c] = operand(c, ks);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        if (!PIPED) a[0][i] = load_rows(tile, ld, i0 + i, ks, lane);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          if (COLS) S16::mma(y[c][i], b[c], a[ks % (AHEAD + 1)][i]);
+          else S16::mma(y[c][i], a[ks % (AHEAD + 1)][i], b[c]);
+        }
+      }
+      if (PIPED) __builtin_amdgcn_sched_barrier(0);
+    }
   }
 };
 
@@ -390,18 +453,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i) y[c][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < NK; ++ks) {
-      Frag b[NC];
-#pragma unroll
-      for (int c = 0; c < NC; ++c) b[c] = S.operand(c, ks);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const Frag a = load_rows(k_tile(n), LDK, i, ks, lane);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) S16::mma(y[c][i], a, b[c]);
-      }
-    }
+    S.template rows_times<4, false>(y, k_tile(n), LDK, 0, lane);
     __builtin_amdgcn_sched_barrier(0);
     // ---- R = beta V - beta e^G Y, in place of Y ----
     Frag br[NC][2];
@@ -455,18 +507,8 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
       floatx4 o[NC][2];
 #pragma unroll
       for (int c = 0; c < NC; ++c) o[c][0] = o[c][1] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < NK; ++ks) {
-        Frag b[NC];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) b[c] = S.operand(c, ks);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const Frag q = load_rows(sQ, LDK, 2 * h + i, ks, lane);
-#pragma unroll
-          for (int c = 0; c < NC; ++c) S16::mma(o[c][i], b[c], q);
-        }
-      }
+      if (S.PIPED) S.settle();
+      S.template rows_times<2, true>(o, sQ, LDK, 2 * h, lane);
       int tok0, len;
       chunk_span(ch.span, n, tok0, len);
 #pragma unroll
@@ -495,8 +537,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
     }
     const float dec = sc[Sc::DEC];
     lds_barrier();  // B2
-    if (GATE == LNX_GATE_SCALAR) S.scale(dec);
-    S.add(k_tile(n), LDK, bu, fresh(tid & 63));
+    S.template add<GATE == LNX_GATE_SCALAR>(k_tile(n), LDK, bu, fresh(tid & 63), dec);
     if (!L::AHEAD) lds_barrier();  // B3
     if (n + 1 < c1) save(n + 1);
     lds_barrier();  // B1 of the next chunk
@@ -628,18 +669,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i) z[c][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < NK; ++ks) {
-      Frag b[NC];
-#pragma unroll
-      for (int c = 0; c < NC; ++c) b[c] = dS.operand(c, ks);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const Frag a = load_rows(k_tile(n), LDK, i, ks, lane);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) S16::mma(z[c][i], a, b[c]);
-      }
-    }
+    dS.template rows_times<4, false>(z, k_tile(n), LDK, 0, lane);
     // ---- dO as an operand, and its rows times scale e^G ----
     Frag fo[NC][2], foq[NC][2];
 #pragma unroll
@@ -704,11 +734,10 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
       for (int c = 0; c < NC; ++c) by[c][s] = S16::from_acc(-gm[0] * x[c][0], -gm[1] * x[c][1]);
     }
     // ---- dS <- e^{G_C} dS' + (scale e^G Q)^T dO ----
-    if (GATE == LNX_GATE_SCALAR) dS.scale(sc[Sc::DEC]);
-    dS.add(sQ, LDK, foq, lane);
+    dS.template add<GATE == LNX_GATE_SCALAR>(sQ, LDK, foq, lane, sc[Sc::DEC]);
     lds_barrier();  // B2
     // ---- dS += K^T dY ----
-    dS.add(k_tile(n), LDK, by, lane);
+    dS.template add<false>(k_tile(n), LDK, by, lane);
     if (!L::AHEAD) lds_barrier();  // B3
     if (n > c0) save(n - 1);
     lds_barrier();  // B1 of the next chunk
@@ -720,7 +749,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
 // because every workgroup loads the chunk's K and Q (relative times).  One round, us a chunk, few workgroups .. all 256:
 //   32 columns   forward 2.8 .. 3.3 (nothing saved 2.6 .. 2.8)   reverse 2.6 .. 3.2
 //   64           3.5 .. 4.9 (2.9 .. 3.7)                         3.1 .. 5.2
-//   128          6.9 .. 7.2 (5.5)                                6.1 .. 6.5
+//   128          6.9 .. 7.2 (5.5)                                6.1 .. 6.5     (at dv = 512 with LDS reads ahead 7.9 -> 7.1 (5.8 -> 5.0) forward)
 // Up to 256 workgroups of 128 columns the choice is the fastest, also for forms that save nothing: T4096 dv128, forward / reverse, 64 heads
 // 209 / 203 us with 32 columns, 263 / 263 with 64; 96 heads 385 / 380 and 275 / 281; 128 heads 311 / 331 with 64 and 461 / 414 with 128; 160 heads
 // 545 / 545 and 476 / 431.  Beyond, where 128 columns take two rounds and 64 three, 64 would be faster by up to 15 % (T1024, 320 heads
