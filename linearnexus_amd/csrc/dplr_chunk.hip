@@ -3,7 +3,7 @@
 // The token-by-token scan (dplr.hip) is one dependent step of some 270 wave instructions per token on the one or two waves
 // that a (batch, head) row has.  Over a chunk the recurrence is a linear map of the state, so everything but a 64 x 64
 // product per chunk can be done for all chunks at once, on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands and
-// accumulation, no operand is rounded to less).
+// accumulation; with v and dO in bf16 three bf16 products that add up to the same: no operand is rounded to less).
 //
 // Per chunk, w = e^gk, E_ts = product of w over the tokens after s up to and with t, per channel; e_t = E from the chunk's start, r_s = E
 // to its end, and t- the token before t (a token's own decay comes after its a):
@@ -219,6 +219,68 @@ template <typename F> __device__ __forceinline__ void put_row(float* tile, const
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) store4(tile + w.t * LD + 16 * cb + 4 * w.g, value(cb));
 }
+
+// ---- products with a tensor as the caller gave it ------------------------------------------------------------------
+// v and dO in bf16 are exact in one part, and an fp32 operand is the sum of three (its top eight bits, the next eight, the last eight: all
+// differences are exact), so a block of 16 of the contraction is two bf16 products of 16 cycles, {last, next} {x, x} and {top, 0} {x, x},
+// instead of four fp32 ones of 32, and no operand is rounded.  The small parts come first, so that c meets the large sum once (the other way round
+// h's error 0.76e-7 of its 2-norm instead of 0.53; four fp32 products 0.69; with ten times RWKV-7's gates 0.64, 0.49, 0.40).  B8 H16 T4096: dplr_prepare 486 -> 437, dplr_u 486 -> 443 us,
+// and with dPqk in dplr_grad 733 -> 724.  Where neither operand is given, six products of parts cost what they save: an operand takes 22
+// instructions to split, dplr_grad's pairs so 733 us, dAak alone 750.
+template <typename T> struct Parts {
+  floatx4 x;
+  __device__ __forceinline__ explicit Parts(floatx4 y) : x(y) {}
+};
+template <> struct Parts<bf16_t> {
+  typedef unsigned uint4_ __attribute__((ext_vector_type(4)));
+  uint4_ top, rest;
+  __device__ __forceinline__ explicit Parts(floatx4 x) {
+    const floatx4 y = x - high(x), z = y - high(y);
+    top = uint4_{pack(x[0], x[1]), pack(x[2], x[3]), 0, 0};
+    rest = uint4_{pack(z[0], z[1]), pack(z[2], z[3]), pack(y[0], y[1]), pack(y[2], y[3])};
+  }
+  static __device__ __forceinline__ floatx4 high(floatx4 x) { return __builtin_bit_cast(floatx4, __builtin_bit_cast(uint4_, x) & 0xffff0000u); }
+  static __device__ __forceinline__ unsigned pack(float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302); }
+};
+__device__ __forceinline__ void mfma_parts(floatx4& c, const Parts<float>& a, const Raw4<float>& b) { mfma4(c, a.x, b.x); }
+__device__ __forceinline__ void mfma_parts(floatx4& c, const Raw4<float>& a, const Parts<float>& b) { mfma4(c, a.x, b.x); }
+__device__ __forceinline__ void mfma_parts(floatx4& c, const Parts<bf16_t>& a, const Raw4<bf16_t>& b) {
+  const bf16x8 x = Mma16::join(b.x, b.x);
+  Mma16::mma(c, __builtin_bit_cast(bf16x8, a.rest), x);
+  Mma16::mma(c, __builtin_bit_cast(bf16x8, a.top), x);
+}
+__device__ __forceinline__ void mfma_parts(floatx4& c, const Raw4<bf16_t>& a, const Parts<bf16_t>& b) {
+  const bf16x8 x = Mma16::join(a.x, a.x);
+  Mma16::mma(c, x, __builtin_bit_cast(bf16x8, b.rest));
+  Mma16::mma(c, x, __builtin_bit_cast(bf16x8, b.top));
+}
+// Tiles of such a tensor in LDS, rows as given: bf16 rows 80 elements apart, which touch every bank once in both directions, and a wave's
+// sixteen where its rows of an fp32 tile begin (before a barrier they are the wave's alone)
+constexpr int LDG = 80;
+static_assert(16 * LDG * sizeof(bf16_t) <= 16 * LD * sizeof(float), "a wave's rows");
+__device__ __forceinline__ int given_at(int row) { return (row >> 4) * (16 * LD * 2) + (row & 15) * LDG; }
+__device__ __forceinline__ void put_given(float* tile, const Lane& w, const Row<float>& x) {
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) store4(tile + w.t * LD + 16 * cb + 4 * w.g, x[cb]);
+}
+__device__ __forceinline__ void put_given(float* tile, const Lane& w, const Row<bf16_t>& x) {
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16_t*>(tile) + given_at(w.t) + 16 * cb + 4 * w.g) = x.x[cb].x;
+}
+// Elements k .. k + 3 of row i; rows k .. k + 3 (of one block) of column c0 + l16
+template <typename T> __device__ __forceinline__ Raw4<T> given_row(const float* tile, int i, int k) {
+  Raw4<T> r;
+  if constexpr (sizeof(T) == 2) r.x = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const bf16_t*>(tile) + given_at(i) + k);
+  else r.x = frag<true>(tile, i, k);
+  return r;
+}
+template <typename T> __device__ __forceinline__ Raw4<T> given_col(const float* tile, int c0, int k, const Lane& w) {
+  Raw4<T> r;
+  if constexpr (sizeof(T) == 2) r.x = Mma16::rows4(reinterpret_cast<const bf16_t*>(tile) + given_at(k), LDG, 0, c0, threadIdx.x);
+  else r.x = frag<false>(tile, c0 + w.l16, k);
+  return r;
+}
+
 // A result whose columns are the wave's tokens (column l16, rows 16 nb + 4 g ..) into rows = tokens
 __device__ __forceinline__ void put_cols(float* tile, const Lane& w, const floatx4 (&c)[4]) {
   put_row(tile, w, [&](int cb) { return c[cb]; });
@@ -495,7 +557,7 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
     }
     put_row(tb, w, [&](int cb) { return x.b[cb] * e.s[cb]; });
     put_row(tk, w, [&](int cb) { return x.k[cb] * e.s[cb]; });
-    put_row(tx, w, [&](int cb) { return v[cb]; });
+    put_given(tx, w, v);
   }
   lds_barrier();
   before(w.j, [&](auto sb_) {
@@ -520,24 +582,28 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
   clear(nt), clear(z), clear(y);
 #pragma unroll
   for (int sb = 0; sb < 4; ++sb) {
-    const floatx4 kf = frag<false>(tk, 16 * w.j + l16, 16 * sb + g4) * end[sb];
+    const Parts<T> kf(frag<false>(tk, 16 * w.j + l16, 16 * sb + g4) * end[sb]);
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) mfma4(nt[nb], kf, frag<false>(tx, 16 * nb + l16, 16 * sb + g4));
+    for (int nb = 0; nb < 4; ++nb) mfma_parts(nt[nb], kf, given_col<T>(tx, 16 * nb, 16 * sb + g4, w));
   }
   before(w.j, [&](auto sb_) {
     constexpr int sb = decltype(sb_)::value;
+    const Parts<T> a(ak[sb]), q(qk[sb]);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
-      const floatx4 vf = frag<false>(tx, 16 * nb + l16, 16 * sb + g4);
-      mfma4(z[nb], ak[sb], vf);
-      mfma4(y[nb], vf, qk[sb]);
+      const Raw4<T> vf = given_col<T>(tx, 16 * nb, 16 * sb + g4, w);
+      mfma_parts(z[nb], a, vf);
+      mfma_parts(y[nb], vf, q);
     }
   });
+  {
+    const Parts<T> a(m.ak), q(m.qk);
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) {
-    const floatx4 vf = frag<false>(tx, 16 * nb + l16, 16 * w.j + g4);
-    mfma4(z[nb], m.ak, vf);
-    mfma4(y[nb], vf, m.qk);
+    for (int nb = 0; nb < 4; ++nb) {
+      const Raw4<T> vf = given_col<T>(tx, 16 * nb, 16 * w.j + g4, w);
+      mfma_parts(z[nb], a, vf);
+      mfma_parts(y[nb], vf, q);
+    }
   }
   lds_barrier();
   put_tri(tx, w, ab, m.ab, [](floatx4 y_) { return -y_; });
@@ -716,15 +782,15 @@ __global__ __launch_bounds__(256) void dplr_r_kernel(ChunkParams p) {
   x.load(p.X, s.kept * TG + w.t * D + g4);
   d.load(p.d_o, s, w);
   put_row(tX, w, [&](int cb) { return x[cb]; });
-  put_row(tO, w, [&](int cb) { return d[cb]; });
+  put_given(tO, w, d);
   lds_barrier();
   floatx4 acc[4];
   clear(acc);
 #pragma unroll
   for (int kb = 3; kb >= 0; --kb) {  // the chunk's first tokens, whose share is the largest, last
-    const floatx4 a = frag<false>(tX, w.t, 16 * kb + g4);
+    const Parts<T> a(frag<false>(tX, w.t, 16 * kb + g4));
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) mfma4(acc[nb], a, frag<false>(tO, 16 * nb + l16, 16 * kb + g4));
+    for (int nb = 0; nb < 4; ++nb) mfma_parts(acc[nb], a, given_col<T>(tO, 16 * nb, 16 * kb + g4, w));
   }
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb) store4(p.s2 + s.win * TG + (16 * nb + l16) * D + 16 * w.j + g4, acc[nb]);
@@ -808,8 +874,8 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   }
   lds_barrier();
   float *th = ta, *tO = tb, *tD = tk, *tv = tx;
-  put_row(tv, w, [&](int cb) { return v[cb]; });
-  put_row(tO, w, [&](int cb) { return d_o[cb]; });
+  put_given(tv, w, v);
+  put_given(tO, w, d_o);
   put_row(th, w, [&](int cb) { return h0[cb]; });  // [value column][channel]
   put_row(tD, w, [&](int cb) { return dC[cb]; });
   lds_barrier();
@@ -826,24 +892,29 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
     }
   before(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
+    const Parts<T> a(akT[b]);
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) mfma4(z[nb], akT[b], frag<false>(tv, 16 * nb + l16, 16 * b + g4));
+    for (int nb = 0; nb < 4; ++nb) mfma_parts(z[nb], a, given_col<T>(tv, 16 * nb, 16 * b + g4, w));
   });
   after(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
+    const Parts<T> pb(qb[b - 1]), pk(qk[b - 1]);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
-      const floatx4 of = frag<false>(tO, 16 * nb + l16, 16 * b + g4);
-      mfma4(y[nb], qb[b - 1], of);
-      mfma4(dv[nb], of, qk[b - 1]);
+      const Raw4<T> of = given_col<T>(tO, 16 * nb, 16 * b + g4, w);
+      mfma_parts(y[nb], pb, of);
+      mfma_parts(dv[nb], of, pk);
     }
   });
+  {
+    const Parts<T> a(akTd), pb(qbd), pk(qkd);
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) {
-    const floatx4 of = frag<false>(tO, 16 * nb + l16, 16 * w.j + g4);
-    mfma4(z[nb], akTd, frag<false>(tv, 16 * nb + l16, 16 * w.j + g4));
-    mfma4(y[nb], qbd, of);
-    mfma4(dv[nb], of, qkd);
+    for (int nb = 0; nb < 4; ++nb) {
+      const Raw4<T> of = given_col<T>(tO, 16 * nb, 16 * w.j + g4, w);
+      mfma_parts(z[nb], a, given_col<T>(tv, 16 * nb, 16 * w.j + g4, w));
+      mfma_parts(y[nb], pb, of);
+      mfma_parts(dv[nb], of, pk);
+    }
   }
   lds_barrier();
   float *Tm = tx, *tz = ta, *ty = tk, *tdu = tb;
@@ -1008,7 +1079,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
       const floatx4 y = sum_block(dC[cb] * h0[cb]);
       if (l16 == 0) store4(through + 64 * w.j + 16 * cb + g4, y);
     }
-    put_row(t0, w, [&](int cb) { return v[cb]; });
+    put_given(t0, w, v);
     put_row(t2, w, [&](int cb) { return u[cb]; });
     put_row(t1, w, [&](int cb) { return h0[cb]; });  // states: [value column][channel]
     put_row(t3, w, [&](int cb) { return dC[cb]; });
@@ -1029,23 +1100,32 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
   Pairs m{zero4(), zero4(), zero4(), zero4()};  // of the lane's own block
 #pragma unroll
   for (int i = 0; i < 3; ++i) pb[i] = pk[i] = nb_[i] = nk[i] = zero4();
-  before(w.j, [&](auto sb_) {
-    constexpr int sb = decltype(sb_)::value;
+  auto pair_sums = [&](floatx4& qb, floatx4& qk, floatx4& ab, floatx4& ak, int row) {
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
-      const floatx4 fu = frag<true>(t2, 16 * sb + l16, 16 * kb + g4), fv = frag<true>(t0, 16 * sb + l16, 16 * kb + g4), fo = d_o[kb], fd = du[kb];
-      mfma_block<4>({&pb[sb], &pk[sb], &nb_[sb], &nk[sb]}, [&](int i) { return i & 1 ? fv : fu; }, [&](int i) { return i & 2 ? fd : fo; });
+      const floatx4 fu = frag<true>(t2, row, 16 * kb + g4), fo = d_o[kb], fd = du[kb];
+      const Raw4<T> fv = given_row<T>(t0, row, 16 * kb + g4);
+      if constexpr (sizeof(T) == 4) {
+        mfma_block<4>({&qb, &qk, &ab, &ak}, [&](int i) { return i & 1 ? fv.x : fu; }, [&](int i) { return i & 2 ? fd : fo; });
+      } else {  // dPqk's operands are both as given: one product for two blocks
+        mfma_block<3>({&qb, &ab, &ak}, [&](int i) { return i == 2 ? fv.get() : fu; }, [&](int i) { return i ? fd : fo; });
+        if (kb & 1) Mma16::mma(qk, Mma16::join(given_row<T>(t0, row, 16 * kb - 16 + g4).x, fv.x), Mma16::join(d_o.x[kb - (kb & 1)].x, d_o.x[kb].x));
+      }
     }
+  };
+  before(w.j, [&](auto sb_) {
+    constexpr int sb = decltype(sb_)::value;
+    pair_sums(pb[sb], pk[sb], nb_[sb], nk[sb], 16 * sb + l16);
   });
   floatx4 dq[4], da[4];  // rows = channels, columns = tokens
   clear(dq), clear(da);
   float st[4];  // decays from the chunk's start to the lane's block, channels 16 cb + l16
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) st[cb] = L.start_to1(w.j, 16 * cb + l16);
+  pair_sums(m.qb, m.qk, m.ab, m.ak, w.t);
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
-    const floatx4 fo = d_o[kb], fd = du[kb], fu = frag<true>(t2, w.t, 16 * kb + g4), fv = frag<true>(t0, w.t, 16 * kb + g4);
-    mfma_block<4>({&m.qb, &m.qk, &m.ab, &m.ak}, [&](int i) { return i & 1 ? fv : fu; }, [&](int i) { return i & 2 ? fd : fo; });
+    const floatx4 fo = d_o[kb], fd = du[kb];
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {
       const floatx4 hf = frag<false>(t1, 16 * cb + l16, 16 * kb + g4) * st[cb];
@@ -1259,7 +1339,7 @@ constexpr int64_t kept_tiles(int64_t n) { return 3 * n + 1; }  // of a row that 
 
 template <typename K> int lds_limit(K* k) { return lnx_lds_limit(reinterpret_cast<const void*>(k), LDS_BYTES); }
 
-// B8 H16 T4096 bf16 (8192 chunks), us: dplr_prepare 507, dplr_chunk_scan 111, dplr_out 112 (48 KB of reads and 8 of writes per chunk: 4.1 TB/s)
+// B8 H16 T4096 bf16 (8192 chunks), us: dplr_prepare 437, dplr_chunk_scan 111, dplr_out 112 (48 KB of reads and 8 of writes per chunk: 4.1 TB/s)
 template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
   if (int rc = lds_limit(dplr_prepare_kernel<T>)) return rc;
@@ -1281,7 +1361,7 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
   return LNX_OK;
 }
 
-// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 490, dplr_grad 771 (two workgroups per CU leave 256 registers, and what a
+// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 443, dplr_grad 724 (two workgroups per CU leave 256 registers, and what a
 // token needs between the pair sums and the last products is more: rows stay as they were read, and three are loaded twice)
 template <typename T> int backward(const lnx_dplr_chunk_grads* g, const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
