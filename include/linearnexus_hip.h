@@ -207,6 +207,11 @@ int lnx_chunk_fwd_static(const lnx_scan_args* a, void* hip_stream);
  * rule would call.  Needs the workspace filled by lnx_chunk_fwd on the same inputs.
  */
 int lnx_chunk_bwd(const lnx_scan_args* a, void* hip_stream);
+/* The same for a gradient of the output that comes in fp32, [B,H,T,dv] in the call's layout, where lnx_chunk_rounds_d_o(a) answers 1 (bf16
+ * with a per-channel gate, dk <= 128): the kernels round it to dtype as they read it.  a->d_o is then an output, a scratch tensor of its
+ * rounded values (in dtype), and the results are those of lnx_chunk_bwd on that. */
+int lnx_chunk_bwd_d_o32(const lnx_scan_args* a, const float* d_o, void* hip_stream);
+int lnx_chunk_rounds_d_o(const lnx_scan_args* a);
 
 /*
  * Row-wise x / (|x|_2 + 1e-6) over the last dimension and its vector-Jacobian product,

@@ -25,6 +25,7 @@ struct BwdParams {
   const float* beta;
   const float* g;  // read again by chunk_kda.hip alone
   const void* d_o;
+  const float* d_o32;  // given in fp32: bwd_scan reads this and writes d_o, its rounding to T
   const float* d_sT;
   void* dq;
   void* dk;
@@ -100,16 +101,34 @@ __global__ __launch_bounds__(256) void bwd_local_kernel(BwdParams p) {
 // ---------------------------------------------------------------------------------------
 // BVW = columns of dv per workgroup: 64 by default; 32 for dk = 128 with 4-byte inputs (LDS capacity) and,
 // on request, for dk = 128 with 2-byte inputs when 64-column slabs would leave most CUs idle.
+// A slab of dO in fp32 as TileRegs<bf16_t, 64, BV> holds it in bf16
+template <int BV> struct RoundedSlab {
+  typedef TileRegs<bf16_t, 64, BV> Slab;
+  floatx4 x[Slab::IT][2];
+  __device__ __forceinline__ void load(const float* src, int64_t stride, int valid, int tid) {
+    const int bytes = valid > 0 ? (int)(valid * stride * (int64_t)sizeof(float)) : 0;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, bytes, 0x00020000);
+#pragma unroll
+    for (int it = 0; it < Slab::IT; ++it) {
+      const int idx = tid + 256 * it, r = idx / Slab::VPR, c = (idx - r * Slab::VPR) * Slab::N;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        x[it][h] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)((r * stride + c + 4 * h) * (int64_t)sizeof(float)), 0, 0));
+    }
+  }
+  __device__ __forceinline__ bf16x8 get(int it, int) const { return Mma16::join(pack_bf16x4(x[it][0]), pack_bf16x4(x[it][1])); }
+};
+
 template <typename T, int DK, int BVW = 64> struct BScanCfg {
   static constexpr int PAD = Mma<T>::PAD;
   static constexpr int BV = (DK > 128 && sizeof(T) == 4) ? 32 : BVW;
   static constexpr int LDK = DK + PAD, LDU = BV + PAD;
   static constexpr int LDC = LNX_C + PAD;
   static constexpr int kRow = 64 * LDK, kSlab = 64 * LDU, kdST = BV * LDK, kdDT = BV * LDC;
-  // 2-byte inputs: the chunk-local part dD_loc = P^T dO is formed here as well (P and the unscaled dO
-  // tile fit LDS), so bwd_local does not run
+  // 2-byte inputs: the chunk-local part dD_loc = P^T dO is formed here as well (P fits LDS, and with their per-channel gate dO's
+  // tile is the unscaled one), so bwd_local does not run
   static constexpr bool FUSE_LOCAL = sizeof(T) == 2;
-  static constexpr int kP = FUSE_LOCAL ? 64 * LDC : 0, kRaw = FUSE_LOCAL ? kSlab : 0;
+  static constexpr int kP = FUSE_LOCAL ? 64 * LDC : 0;
   static constexpr int kG = DK > 128 ? DK : 128;  // gate values: 64 tokens (scalar gate) or dk channels (vector gate)
   // 4-byte inputs with dk = 256: K (read for dD), Q and W (read for the dS update) of a chunk take turns in one tile
   static constexpr bool SHARE = sizeof(T) == 4 && DK > 128;
@@ -121,11 +140,14 @@ template <typename T, int DK, int BVW = 64> struct BScanCfg {
   // while chunk n is being read
   static constexpr bool DB = sizeof(T) == 2 && DK == 128 && BV == 32;
   static constexpr int NB = DB ? 2 : 1;
-  // K, Q, W rows [token][dk];  dO, dD slabs [token][BV];  -dD^T [BV][token];  dS^T [BV][dk];  P;  unscaled dO
-  static constexpr size_t bytes = sizeof(T) * (NB * (nRow * kRow + kSlab + kP + kRaw) + kSlab + kdDT + kdST) + sizeof(float) * NB * kG;
+  // K, Q, W rows [token][dk];  dO, dD slabs [token][BV];  -dD^T [BV][token];  dS^T [BV][dk];  P
+  static constexpr size_t bytes = sizeof(T) * (NB * (nRow * kRow + kSlab + kP) + kSlab + kdDT + kdST) + sizeof(float) * NB * kG;
 };
 
-template <typename T, int DK, int GATE, int BVW = 64>
+// ROUND: dO comes in fp32 (the default output type of the per-channel gate's rule).  The movers round it on its way into LDS and write the
+// rounded rows back for kda_bwd_chunk, in place of a pass of its own over 4 + 2 bytes per element of dO (B4 H16 T8192 d128: 76 us; here 248 -> 283,
+// dk = 64 with 512 workgroups 190 -> 250, held to the 128 registers of two workgroups per CU 473).
+template <typename T, int DK, int GATE, int BVW = 64, bool ROUND = false>
 __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
   typedef BScanCfg<T, DK, BVW> L;
   constexpr int LDK = L::LDK, LDU = L::LDU, LDC = L::LDC, BV = L::BV;
@@ -134,6 +156,7 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
   constexpr int RT = (DK >= 128) ? DK / 128 : 1;   // state tiles per wave: RT row tiles (from RT * wave, or wave & 1
   constexpr int NT = (DK >= 128) ? CT : 1;         //   for dk = 64) x NT column tiles
   static_assert(DK >= 128 || BV == 64, "dk = 64 needs a 64-column slab");
+  static_assert(!FUSE || GATE == LNX_GATE_VECTOR, "the fused local part reads dO unscaled");
   extern __shared__ __align__(16) char smem[];
   constexpr int NB = L::NB;  // buffers per input tile (the second of a pair follows the first)
   T* sK = reinterpret_cast<T*>(smem);
@@ -143,9 +166,8 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
   T* sdDl = sdO + NB * L::kSlab;
   T* sdDT = sdDl + L::kSlab;
   T* sdST = sdDT + L::kdDT;
-  T* sP = sdST + L::kdST;   // fused local part only: P [i][j] and the unscaled dO slab
-  T* sdOr = sP + NB * L::kP;
-  float* sG = reinterpret_cast<float*>(sdOr + NB * L::kRaw);
+  T* sP = sdST + L::kdST;   // fused local part only: P [i][j]
+  float* sG = reinterpret_cast<float*>(sP + NB * L::kP);
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int N = p.geom.N;
@@ -286,12 +308,8 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
       auto commit_main = [&]() {
         rK.store(sK, LDK, mt);
         rW.store(sW, LDK, mt);
-        if (FUSE) {
-          rP.store(sP, LDC, mt);
-          rdO.store(sdOr, LDU, mt);
-        } else {
-          rdD.store(sdDl, LDU, mt);
-        }
+        if (FUSE) rP.store(sP, LDC, mt);
+        else rdD.store(sdDl, LDU, mt);
 #pragma unroll
         for (int it = 0; it < Slab::IT; ++it) {
           const int idx = mt + 256 * it, r = idx / Slab::VPR, c = (idx - r * Slab::VPR) * Slab::N;
@@ -332,7 +350,8 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
     typedef TileRegs<T, 64, BV> Slab;
     struct Tiles {
       TileRegs<T, 64, DK> K, Q, W;
-      Slab dO, dD;                       // dD: the chunk-local part from bwd_local (not fused only)
+      typename std::conditional<ROUND, RoundedSlab<BV>, Slab>::type dO;
+      Slab dD;                           // the chunk-local part from bwd_local (not fused only)
       TileRegs<T, 64, FUSE ? 64 : 8> P;  // fused only
       float os[Slab::IT];  // G_i of the dO row each vector belongs to (scalar gate)
       float G;
@@ -355,7 +374,8 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
         else R.K.load(reinterpret_cast<const T*>(p.k) + tbase * DK, tsk, len, mt);
       }
       if (part < 0 || part == 1) {
-        R.dO.load(reinterpret_cast<const T*>(p.d_o) + tbase * p.dv + v0, (int64_t)p.geom.ts * p.dv, len, mt);
+        if constexpr (ROUND) R.dO.load(p.d_o32 + tbase * p.dv + v0, (int64_t)p.geom.ts * p.dv, len, mt);
+        else R.dO.load(reinterpret_cast<const T*>(p.d_o) + tbase * p.dv + v0, (int64_t)p.geom.ts * p.dv, len, mt);
         if (FUSE) R.P.load(wsp<T>(p, p.off.P) + slot * 64 * 64, 64, 64, mt);
         else R.dD.load(wsp<T>(p, p.off.dD) + slot * 64 * p.dv + v0, p.dv, 64, mt);
         // every thread loads (clamped index): a load behind a branch cannot be counted
@@ -379,12 +399,8 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
         R.W.store(sW + pb * L::kRow, LDK, mt);
       }
       if (part == 0 || part == 2) return;
-      if (FUSE) {
-        R.P.store(sP + pb * L::kP, LDC, mt);
-        R.dO.store(sdOr + pb * L::kRaw, LDU, mt);
-      } else {
-        R.dD.store(sdDl, LDU, mt);
-      }
+      if (FUSE) R.P.store(sP + pb * L::kP, LDC, mt);
+      else R.dD.store(sdDl, LDU, mt);
 #pragma unroll
       for (int it = 0; it < Slab::IT; ++it) {
         const int idx = mt + 256 * it, r = idx / Slab::VPR, c = (idx - r * Slab::VPR) * Slab::N;
@@ -397,6 +413,18 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
         if (idx < Slab::TOTAL) *reinterpret_cast<typename Vec16<T>::V*>(sdO + pb * L::kSlab + r * LDU + c) = o;
       }
       if (mt < L::kG) sG[pb * L::kG + mt] = R.G;
+    };
+    auto put_rounded = [&](const Tiles& R, int n) {  // dO of chunk n -> p.d_o
+      if constexpr (ROUND) {
+        int tok0, len;
+        chunk_span(span, n, tok0, len);
+        T* out = static_cast<T*>(const_cast<void*>(p.d_o)) + tok_index(p.geom, row, tok0) * p.dv + v0;
+#pragma unroll
+        for (int it = 0; it < Slab::IT; ++it) {
+          const int idx = mt + 256 * it, r = idx / Slab::VPR, c = (idx - r * Slab::VPR) * Slab::N;
+          if (r < len) *reinterpret_cast<typename Vec16<T>::V*>(out + (int64_t)r * p.geom.ts * p.dv + c) = R.dO.get(it, mt);
+        }
+      }
     };
     // Double-buffered form.  Chunk n - 1 goes to the buffers chunk n + 1 was read from, so no tile write waits for a
     // reader: loads of chunk n - 2 and the tile writes in the first two phases, dS', dD -> workspace in the second.
@@ -428,8 +456,11 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
       unstage_tile<T, BV, DK, true>(wsp<T>(p, p.off.dSn) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sdST, LDK, BV, mt);
       unstage_tile<T, 64, BV, true>(wsp<T>(p, p.off.dD) + slot * 64 * p.dv + v0, p.dv, sdDl, LDU, 64, mt);
       if constexpr (STEADY) {
+        put_rounded(nxt, n - 1);
         fetch(cur, n - 2, 2);
         commit_rest(nxt, pb ^ 1, 2);
+      } else if (n - 1 >= c0) {
+        put_rounded(nxt, n - 1);
       }
       lds_barrier();  // B3
       lds_barrier();  // B1 of the next chunk
@@ -445,13 +476,14 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
       unstage_tile<T, 64, BV, true>(wsp<T>(p, p.off.dD) + slot * 64 * p.dv + v0, p.dv, sdDl, LDU, 64, mt);
       lds_barrier();  // B3
       if (more && AHEAD == 2) fetch(cur, n - AHEAD, 2);
-      if (n - 1 >= c0) commit_rest(nxt, 0);
+      if (n - 1 >= c0) commit_rest(nxt, 0), put_rounded(nxt, n - 1);
       lds_barrier();  // B1 of the next chunk
     };
     if (c0 < c1) {
       fetch(ta, c1 - 1, -1);
       ta.K.store(sK, LDK, mt);
       commit_rest(ta, 0);
+      put_rounded(ta, c1 - 1);
     }
     if (AHEAD == 2 && c1 - 2 >= c0) fetch(tb, c1 - 2, -1);
     lds_barrier();  // B1 of the first chunk
@@ -505,7 +537,6 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
     const T* cW = sW + pb * L::kRow;
     const T* cdO = sdO + pb * L::kSlab;
     const T* cP = sP + pb * L::kP;
-    const T* cdOr = sdOr + pb * L::kRaw;
     const float* cG = sG + pb * L::kG;
     const float gl = (GATE == LNX_GATE_SCALAR) ? cG[63] : 0.f;
     // dD = dD_loc + r_j (K dS)_j
@@ -519,7 +550,7 @@ __global__ __launch_bounds__(512) void bwd_scan_kernel(BwdParams p) {
       if (FUSE) {  // dD_loc[j][v] = sum_i P[i][j] dO[i][v]: both operands contract along the rows of their tiles
         floatx16 l[1][1];
         frag_zero(l);
-        mma_x<T, 1, 1, true, true>(l, cP + 32 * wi, LDC, cdOr + 32 * wj, LDU, 64, lane);
+        mma_x<T, 1, 1, true, true>(l, cP + 32 * wi, LDC, cdO + 32 * wj, LDU, 64, lane);
 #pragma unroll
         for (int e = 0; e < 16; ++e) dl[e] = l[0][0][e];
       } else {
@@ -1425,6 +1456,8 @@ int launch_bwd(const BwdParams& p, int nstate, hipStream_t st) {
     hipLaunchKernelGGL(bwd_local_kernel<T>, dim3(lnx_xcd_grid(slots, p.dv / 64)), dim3(256), 0, st, p);
   }
   auto k1 = narrow ? bwd_scan_kernel<T, DK, GATE, NARROW> : bwd_scan_kernel<T, DK, GATE, WIDE>;
+  if constexpr (sizeof(T) == 2 && DK <= 128 && GATE == LNX_GATE_VECTOR)
+    if (p.d_o32) k1 = narrow ? bwd_scan_kernel<T, DK, GATE, NARROW, true> : bwd_scan_kernel<T, DK, GATE, WIDE, true>;
   const int bv = narrow ? BScanCfg<T, DK, NARROW>::BV : BScanCfg<T, DK, WIDE>::BV;
   const size_t b1 = narrow ? BScanCfg<T, DK, NARROW>::bytes : BScanCfg<T, DK, WIDE>::bytes;
   if ((rc = lnx_lds_limit((const void*)k1, b1)) != LNX_OK) return rc;
@@ -1471,7 +1504,7 @@ __global__ void copy_dstate_kernel(const float* src, float* dst, int64_t n) {
 
 }  // namespace
 
-extern "C" int lnx_chunk_bwd(const lnx_scan_args* a, void* stream) {
+static int chunk_bwd(const lnx_scan_args* a, const float* d_o32, void* stream) {
   int rc = lnx_chunk_check(a, true);
   if (rc != LNX_OK) return rc;
   hipStream_t st = (hipStream_t)stream;
@@ -1497,7 +1530,7 @@ extern "C" int lnx_chunk_bwd(const lnx_scan_args* a, void* stream) {
   p.geom.rows = packed ? a->H : a->B * a->H;
   p.geom.cu = a->cu_seqlens;
   p.geom.tab = packed ? reinterpret_cast<const int32_t*>(reinterpret_cast<char*>(a->workspace) + w.tab) : nullptr;
-  p.q = a->q; p.k = a->k; p.v = a->v; p.beta = a->beta; p.g = a->g; p.d_o = a->d_o; p.d_sT = a->d_final_state;
+  p.q = a->q; p.k = a->k; p.v = a->v; p.beta = a->beta; p.g = a->g; p.d_o = a->d_o; p.d_o32 = d_o32; p.d_sT = a->d_final_state;
   p.dq = a->d_q; p.dk = a->d_k; p.dv_out = a->d_v; p.dbeta = a->d_beta; p.dg = a->d_g; p.ds0 = a->d_initial_state;
   p.dv = a->dv; p.gate = a->gate; p.l2norm = a->use_qk_l2norm; p.scale = a->scale; p.slab = a->test_scan_slab;
   const bool raw_gate = a->gate == LNX_GATE_VECTOR && a->gate_raw != nullptr;
@@ -1539,4 +1572,15 @@ extern "C" int lnx_chunk_bwd(const lnx_scan_args* a, void* stream) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return lnx_set_error(LNX_ERR_LAUNCH, "chunk backward launch: %s", hipGetErrorString(e));
   return LNX_OK;
+}
+
+extern "C" int lnx_chunk_bwd(const lnx_scan_args* a, void* stream) { return chunk_bwd(a, nullptr, stream); }
+
+extern "C" int lnx_chunk_rounds_d_o(const lnx_scan_args* a) { return a && lnx_chunk_kda(a) ? 1 : 0; }
+
+extern "C" int lnx_chunk_bwd_d_o32(const lnx_scan_args* a, const float* d_o, void* stream) {
+  if (!a || !d_o) return lnx_set_error(LNX_ERR_NULL, "the arguments and d_o are required");
+  if (!lnx_chunk_rounds_d_o(a)) return lnx_set_error(LNX_ERR_DTYPE, "d_o in fp32: only where lnx_chunk_rounds_d_o says so");
+  if (reinterpret_cast<uintptr_t>(d_o) & 15) return lnx_set_error(LNX_ERR_SHAPE, "d_o must be 16-byte aligned");
+  return chunk_bwd(a, d_o, stream);
 }

@@ -510,7 +510,12 @@ struct ChunkFn : Function<ChunkFn> {
     a.test_scan_slab = (int32_t)m[11], a.test_out_slabs = (int32_t)m[12];
     const bool tf = m[10] != 0;
     const auto o = c.qn.options();
-    const Tensor d_o = as_layout(grads[0].defined() ? grads[0].to(c.qn.scalar_type()) : at::zeros({m[0], m[1], m[2], m[4]}, o), tf);
+    // in fp32 as the kernels can take it: rounded there, into a scratch tensor
+    const Tensor given = grads[0];
+    const bool rounds = given.defined() && given.scalar_type() == at::kFloat && given.numel() > 0 && !given.is_neg() && lnx_chunk_rounds_d_o(&a) &&
+                        reinterpret_cast<uintptr_t>(given.data_ptr()) % 16 == 0 && (tf ? is_token_first(given) : given.is_contiguous());
+    const Tensor d_o = rounds ? empty_layout(m[0], m[1], m[2], m[4], o, tf)
+                              : as_layout(given.defined() ? given.to(c.qn.scalar_type()) : at::zeros({m[0], m[1], m[2], m[4]}, o), tf);
     const Tensor d_sT = f32(grads[1]);
     Tensor dq = at::empty_like(c.qn), dk = at::empty_like(c.kn), dv = at::empty_like(c.v), dbeta = at::empty_like(c.beta);
     Tensor dg = c.g.defined() ? at::empty_like(c.g) : Tensor(), ds0, dA, dbias;
@@ -527,7 +532,8 @@ struct ChunkFn : Function<ChunkFn> {
       a.d_g = nullptr;
       a.d_gate_raw = ptr(dg), a.d_gate_A_log = fptr(dA), a.d_gate_bias = fptr(dbias);
     }
-    check_status(lnx_chunk_bwd(&a, stream_of(c.qn)), "lnx_chunk_bwd");
+    if (rounds) check_status(lnx_chunk_bwd_d_o32(&a, fptr(given), stream_of(c.qn)), "lnx_chunk_bwd_d_o32");
+    else check_status(lnx_chunk_bwd(&a, stream_of(c.qn)), "lnx_chunk_bwd");
     if (c.norm_outside) std::tie(dq, dk) = l2norm_pair_bwd(c.q_in, c.k_in, dq, dk);
     auto to = [](const Tensor& t, int64_t type) { return t.defined() ? t.to((at::ScalarType)type) : t; };
     return {dq, dk, dv, to(dg, m[14]), to(dbeta, m[13]), to(ds0, m[15]), to(dA, m[16]), to(dbias, m[17]), Tensor()};
