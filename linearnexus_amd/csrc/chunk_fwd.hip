@@ -1714,10 +1714,13 @@ int chunk_fwd_on(const lnx_scan_args* a, void* workspace, uint64_t workspace_byt
 // chain: s_in[0] = s0, s_in[i + 1] = B_i + A_i s_in[i], where segment i left [B_i | A_i] in ab [n, H, dk, dv + dk].
 // One workgroup per (head, 16 value columns): the columns stay in LDS (transposed) for all segments, wave w forms rows
 // 16 w .. on the fp32 matrix cores (16x16x4).  A step is a serial chain: barrier, the columns from LDS, 32 products a wave with two waves
-// on a matrix core (0.85 us of the step's 2), the sums back into LDS.  So its operands from LDS are requested at once, and the rows of
-// A_i two steps on (one at dk = 256) go out one by one between the products, each into the registers that have just been used: in front
-// of them they held the first product up.  16 segments of 4 heads d128 43.8 -> 37.3 us (with four sets in flight but in front 43.8, with
-// four waves of two row tiles 40.4), where a batched library product and two copies per step took 310.
+// on a matrix core (0.85 us of the step's 1.75), the sums back into LDS.  The rows of A_i two steps on (one at dk = 256) go out one by one
+// between the products, each into the registers that have just been used: in front of them they held the first product up.
+// They are loaded as they lie in memory, consecutive lanes side by side, and become operands through LDS of the wave's own (`turn`):
+// loaded as operands, 16 bytes of 16 rows, a CU takes a lane a cycle, 15.8 bytes, instead of a quad, 61 (measured with data in L2), and
+// its 64 KB were most of the step.  16 segments of 4 heads d128 38.5 -> 28.3 us (all of the state's operands requested at once, as
+// was best before, 32.9; slices of 16 28.9), 2 heads dk 256 dv 512 131 -> 86 (slices of 32: 49 registers spilled, 178), dk 64 the
+// same 13.2; a batched library product and two copies per step took 310 at the first.
 // ---------------------------------------------------------------------------------------
 __global__ void segment_setup_kernel(int32_t* cu, int32_t* tab, int N, int n, int seg, int T) {
   const int first = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
@@ -1737,46 +1740,67 @@ template <int DK> constexpr int segment_chain_threads = DK == 64 ? 256 : 512;
 template <int DK>
 __global__ __launch_bounds__(segment_chain_threads<DK>) void segment_chain_kernel(const float* ab, const float* s0, float* s_in, int n, int H, int dv) {
   constexpr int THREADS = segment_chain_threads<DK>, PW = DK / (THREADS / 4), NT = DK / 16;  // row tiles of a wave; 16-wide steps over k
-  constexpr int LD = DK + 4;
+  constexpr int LD = DK + 4, KS = DK <= 128 ? 32 : 16, NS = DK / KS, LDA = KS + 4;  // slices of KS k
   __shared__ __align__(16) float sS[2][16 * LD];  // [column][k]
+  __shared__ __align__(16) float sA[THREADS / 64][PW * 16 * LDA];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, kq = lane >> 4;
   const int h = blockIdx.x, v0 = 16 * blockIdx.y;
   const int ldab = dv + DK;
   auto tile = [&](int t) { return PW * wave + t; };
+  constexpr int VPR = KS / 4;  // vectors of a slice's row: consecutive lanes
   struct Rows {
-    floatx4 a[PW][NT], b[PW];
+    floatx4 a[NS][PW][KS / 16], b[PW];
+  };
+  struct Frags {
+    floatx4 a[PW][KS / 16];
   };
   auto fetch_a = [&](Rows& r, int i, int s) {
-    const float* m = ab + ((int64_t)i * H + h) * DK * ldab + dv + 16 * s + 4 * kq;
-#pragma unroll
-    for (int t = 0; t < PW; ++t) r.a[t][s] = load4(m + (int64_t)(16 * tile(t) + l16) * ldab);
-  };
-  auto fetch_b = [&](Rows& r, int i) {
-    const float* m = ab + ((int64_t)i * H + h) * DK * ldab + v0 + l16;
+    const float* m = ab + ((int64_t)i * H + h) * DK * ldab + dv + KS * s;  // the same for every lane
+    const int at = (16 * tile(0) + lane / VPR) * ldab + 4 * (lane % VPR);
 #pragma unroll
     for (int t = 0; t < PW; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) r.b[t][e] = m[(int64_t)(16 * tile(t) + 4 * kq + e) * ldab];
+      for (int u = 0; u < KS / 16; ++u) r.a[s][t][u] = load4(m + (16 * t + 64 / VPR * u) * ldab + at);
   };
-  auto fetch = [&](Rows& r, int i) {
+  auto fetch_b = [&](Rows& r, int i) {
+    const float* m = ab + ((int64_t)i * H + h) * DK * ldab + v0;
+    const int at = (16 * tile(0) + 4 * kq) * ldab + l16;
 #pragma unroll
-    for (int s = 0; s < NT; ++s) fetch_a(r, i, s);
-    fetch_b(r, i);
+    for (int t = 0; t < PW; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r.b[t][e] = (m + (16 * t + e) * ldab)[at];
+  };
+  auto turn = [&](Frags& f, const Rows& r, int s) {  // a slice as loaded -> operands, through the wave's own LDS
+#pragma unroll
+    for (int t = 0; t < PW; ++t)
+#pragma unroll
+      for (int u = 0; u < KS / 16; ++u) store4(sA[wave] + (16 * t + 64 / VPR * u + lane / VPR) * LDA + 4 * (lane % VPR), r.a[s][t][u]);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < PW; ++t)
+#pragma unroll
+      for (int j = 0; j < KS / 16; ++j) f.a[t][j] = load4(sA[wave] + (16 * t + l16) * LDA + 16 * j + 4 * kq);
+    __builtin_amdgcn_wave_barrier();
   };
   for (int i = tid; i < DK * 16; i += THREADS) sS[0][(i & 15) * LD + (i >> 4)] = s0 ? s0[((int64_t)h * DK + (i >> 4)) * dv + v0 + (i & 15)] : 0.f;
   constexpr int RING = DK <= 128 ? 2 : 1;
   Rows r[RING];
 #pragma unroll
   for (int i = 0; i < RING; ++i) {
-    fetch(r[i], min(i, n - 1));
+#pragma unroll
+    for (int s = 0; s < NS; ++s) fetch_a(r[i], min(i, n - 1), s);
+    fetch_b(r[i], min(i, n - 1));
     __builtin_amdgcn_sched_barrier(0);  // the sets' loads stay in order: the wait for one leaves the other in flight
   }
-  auto step = [&](Rows& r, int i) {
+  Frags f[2];
+  turn(f[0], r[0], 0);
+  fetch_a(r[0], min(RING, n - 1), 0);
+  auto step = [&](Rows& r, Rows& next, int i) {
     lds_barrier();
     const float* cur = sS[i & 1];
     // no load behind a branch, where its wait could not be counted: the last steps fetch and multiply what nobody reads
     const int ahead = min(i + RING, n - 1);
-    constexpr int XS = DK <= 128 ? NT : 2;
+    constexpr int XS = 2;
     floatx4 acc[PW][2], x[NT];
 #pragma unroll
     for (int s = 0; s < XS; ++s) x[s] = load4(cur + l16 * LD + 16 * s + 4 * kq);
@@ -1784,20 +1808,30 @@ __global__ __launch_bounds__(segment_chain_threads<DK>) void segment_chain_kerne
 #pragma unroll
     for (int t = 0; t < PW; ++t) acc[t][0] = acc[t][1] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < NT; ++s) {
+    for (int s = 0; s < NS; ++s) {
+      // the next slice becomes operands, and its registers take the rows RING steps on: a step's loads go out between its products and
+      // not in front of them
+      if (s + 1 < NS) {
+        turn(f[(s + 1) & 1], r, s + 1);
+        fetch_a(r, ahead, s + 1);
+      }
 #pragma unroll
-      for (int t = 0; t < PW; ++t)
+      for (int j = 0; j < KS / 16; ++j) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[t][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.a[t][s][e], x[s][e], acc[t][e & 1], 0, 0, 0);
-      // these registers take the rows RING steps on: a step's loads go out between its products and not in front of them
-      fetch_a(r, ahead, s);
-      if (s + XS < NT) x[s + XS] = load4(cur + l16 * LD + 16 * (s + XS) + 4 * kq);
+        for (int t = 0; t < PW; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[t][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[s & 1].a[t][j][e], x[KS / 16 * s + j][e], acc[t][e & 1], 0, 0, 0);
+        const int k = KS / 16 * s + j + XS;
+        if (k < NT) x[k] = load4(cur + l16 * LD + 16 * k + 4 * kq);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int t = 0; t < PW; ++t) store4(sS[(i + 1) & 1] + l16 * LD + 16 * tile(t) + 4 * kq, r.b[t] + (acc[t][0] + acc[t][1]));
     __builtin_amdgcn_sched_barrier(0);
     fetch_b(r, ahead);
+    turn(f[0], next, 0);
+    fetch_a(next, min(i + 1 + RING, n - 1), 0);
     if (i >= n) return;
     float* out = s_in + ((int64_t)i * H + h) * DK * dv + v0;
 #pragma unroll
@@ -1808,7 +1842,7 @@ __global__ __launch_bounds__(segment_chain_threads<DK>) void segment_chain_kerne
   };
   for (int i = 0; i < n; i += RING) {  // one exit: a way out between two steps would join the others' count of loads in flight
 #pragma unroll
-    for (int e = 0; e < RING; ++e) step(r[e], i + e);
+    for (int e = 0; e < RING; ++e) step(r[e], r[(e + 1) % RING], i + e);
   }
 }
 
