@@ -41,8 +41,15 @@ constexpr int C = 64, D = 64;       // tokens of a chunk, channels of a head
 constexpr int LD = LNX_LDA;         // leading dimension of the fp32 tiles in LDS: 68 floats, rows 4 banks apart
 constexpr int TS = C * LD;          // floats of a tile in LDS
 constexpr int TG = C * D;           // floats of a tile in the workspace
-constexpr int TRI = 10 * 256;       // floats of a lower-triangular one: the rows of block row j, 16 (j + 1) long, behind each other
+constexpr int TRI = 10 * 256;       // floats of a lower-triangular one: its ten blocks, row by row
 constexpr int RANGE = 60;           // products of decays of a block's first tokens lie within 2^+-RANGE, or the block is DIRECT
+
+// A tile in the workspace is sixteen blocks of 16 x 16, block row by block row, and a block lies as a wave holds it, four elements of a row
+// per lane: lane 16 g + l16 has row l16, columns 4 g ... to 4 g + 3.  Every kernel reads and writes the tiles that way, consecutive lanes
+// side by side.  With rows of 64 floats an instruction took 64 bytes of 16 rows, and such a one passes the CU's address path a lane a
+// cycle, 15.8 bytes instead of 61 (measured, data in L2).  B8 H16 T4096 forward and backward 1937 -> 1870 us (the scans 110 -> 89 and 101 -> 89,
+// dplr_out 112 -> 97), B1 H16 T16384 1228 -> 1143 (179 -> 135, 158 -> 142).
+__device__ __forceinline__ int block_at(int row, int col) { return (4 * row + col) * 256 + 4 * (threadIdx.x & 63); }
 
 struct ChunkParams {
   const void *q, *k, *v, *a, *b;
@@ -199,6 +206,10 @@ template <> struct Raw4<float> {
 // registers (B8 H16 T4096 forward and backward 2138 -> 2094 us).
 template <typename T> struct Row {
   Raw4<T> x[4];
+  __device__ __forceinline__ void load_tile(const float* tile, int row) {  // block row of a tile in the workspace
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) x[cb].load(tile + block_at(row, cb));
+  }
   __device__ __forceinline__ void load(const void* base, int64_t at) {  // at: element of the lane's first channel
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) x[cb].load(static_cast<const T*>(base) + at + 16 * cb);
@@ -506,8 +517,7 @@ template <bool BY_T, bool STRICT> __device__ __forceinline__ void mask(floatx4& 
     m[r] = (STRICT ? s >= t : s > t) ? 0.f : m[r];
   }
 }
-// The lane's row of a lower-triangular tile in the workspace
-__device__ __forceinline__ int tri_row(const Lane& w) { return 128 * w.j * (w.j + 1) + 16 * (w.j + 1) * w.l16; }
+__device__ __forceinline__ int tri_block(int row, int col) { return (row * (row + 1) / 2 + col) * 256 + 4 * (threadIdx.x & 63); }
 // The wave's rows of a lower-triangular matrix: what lies before block j, the block itself, zeros
 template <typename F> __device__ __forceinline__ void put_tri(float* tile, const Lane& w, const floatx4 (&x)[3], floatx4 d, F&& value) {
 #pragma unroll
@@ -620,7 +630,7 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
     upto(w.j, [&](auto sb_) {
       constexpr int sb = decltype(sb_)::value;
       const floatx4 tf = frag<true>(tx, w.t, 16 * sb + g4);
-      if (p.Tm) store4(p.Tm + s.kept * TRI + tri_row(w) + 16 * sb + g4, tf);
+      if (p.Tm) store4(p.Tm + s.kept * TRI + tri_block(w.j, sb), tf);
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
         mfma4(W[cb], tf, frag<false>(ta, 16 * cb + l16, 16 * sb + g4));
@@ -661,11 +671,11 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       if (16 * cb + g4 + e == w.t) r[e] += chunk;
-    const int at = w.t * D + 16 * cb + g4;
+    const int at = block_at(w.j, cb);
     store4(p.M + s.kept * TG + at, r);
     store4(p.X + s.kept * TG + at, xx[cb] + xw[cb]);
     store4(p.s2 + s.win * TG + at, y[cb] + yu[cb]);
-    store4(p.s1 + s.win * TG + (16 * cb + l16) * D + 16 * w.j + g4, nt[cb] + ntu[cb]);
+    store4(p.s1 + s.win * TG + block_at(cb, w.j), nt[cb] + ntu[cb]);
   }
 }
 
@@ -673,7 +683,8 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
 // One workgroup per row and 16 of the 64 value columns; wave w forms 16 rows of the new state, sixteen products of 32 cycles, from its
 // rows of M, which come straight into its registers three chunks ahead, and the old state, which the waves exchange
 // through LDS (transposed), one LDS barrier per chunk.  A whole chain on one wave per 16 columns took four times the products and
-// M through LDS: 1.85 us per chunk.
+// M through LDS: 1.85 us per chunk.  In reverse a wave's rows of M^T are columns of M: its blocks of M are turned through LDS of its own,
+// a chunk ahead (read from memory as columns, four rows at a time, the pass took 101 us instead of 89 at B8 H16 T4096).
 struct ScanParams {
   const float* M;    // kept tiles [rows][KN]
   const float* add;  // window tiles: N^T or R^T
@@ -684,17 +695,20 @@ struct ScanParams {
   int KN, at, nw;    // the window is chunks [at, at + nw) of the kept tensors
 };
 
+constexpr int LDT = 20;  // rows of 16 floats on their way through LDS: both ways touch every bank once
+
 template <bool BWD>
 __global__ __launch_bounds__(256) void dplr_chunk_scan_kernel(ScanParams p) {
-  __shared__ __align__(16) float buf[2][16 * LD];
+  __shared__ __align__(16) float buf[2][16 * LD], own_[BWD ? 4 : 1][BWD ? 64 * LDT : 4];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   int64_t row;
   int part;
   if (!xcd_slot_part(p.rows, 4, row, part)) return;  // the four parts read the same M: one XCD
   const int col = 16 * part + l16, r0 = 16 * wave + 4 * g;  // this lane's column and its first row of the state
-  const float* Mrow = p.M + (row * p.KN + p.at) * TG + (BWD ? 4 * g * D + 16 * wave + l16 : (16 * wave + l16) * D + 4 * g);
-  const float* Arow = p.add + row * p.nw * TG + col * D + r0;
-  float* Srow = p.st + (BWD ? row * p.nw : row * (p.KN + 1) + p.at) * TG + col * D + r0;
+  const float* Mrow = p.M + (row * p.KN + p.at) * TG + (BWD ? block_at(0, wave) : block_at(wave, 0));
+  const float* Arow = p.add + row * p.nw * TG + block_at(part, wave);
+  float* Srow = p.st + (BWD ? row * p.nw : row * (p.KN + 1) + p.at) * TG + block_at(part, wave);
+  float* own = own_[BWD ? wave : 0];
   auto chunk = [&](int i) { return (int64_t)(BWD ? p.nw - 1 - i : i); };
   floatx4 h;
 #pragma unroll
@@ -705,28 +719,37 @@ __global__ __launch_bounds__(256) void dplr_chunk_scan_kernel(ScanParams p) {
   auto fetch = [&](Ahead& x, int i) {
     const float* M = Mrow + chunk(min(i, p.nw - 1)) * TG;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      if (BWD) x.m[b] = floatx4{M[16 * b * D], M[(16 * b + 1) * D], M[(16 * b + 2) * D], M[(16 * b + 3) * D]};
-      else x.m[b] = load4(M + 16 * b);
-    }
+    for (int b = 0; b < 4; ++b) x.m[b] = load4(M + (BWD ? 4 * 256 : 256) * b);
     x.a = load4(Arow + chunk(min(i, p.nw - 1)) * TG);
   };
-  auto step = [&](Ahead& x, Ahead& next, int i) {  // next: the set that chunk i - 1 has used
+  floatx4 m[4];  // backward: the rows of M^T of the chunk at hand
+  auto turn = [&](const Ahead& x) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b) store4(own + (16 * b + l16) * LDT + 4 * g, x.m[b]);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m[b][e] = own[(16 * b + 4 * g + e) * LDT + l16];
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto step = [&](Ahead& x, const Ahead& next, Ahead& free, int i) {  // next: chunk i + 1; free: the set that chunk i - 1 has used
     lds_barrier();
     const float* cur = buf[i & 1] + l16 * LD + 4 * g;
     floatx4 f[4];
 #pragma unroll
     for (int b = 0; b < 4; ++b) f[b] = load4(cur + 16 * b);
-    fetch(next, i + 3);
+    fetch(free, i + 3);
     store4(Srow + chunk(i) * TG, h);
     floatx4 y0 = zero4(), y1 = zero4();
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[2 * b][r], f[2 * b][r], y0, 0, 0, 0);
-        y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[2 * b + 1][r], f[2 * b + 1][r], y1, 0, 0, 0);
+        y0 = __builtin_amdgcn_mfma_f32_16x16x4f32((BWD ? m[2 * b] : x.m[2 * b])[r], f[2 * b][r], y0, 0, 0, 0);
+        y1 = __builtin_amdgcn_mfma_f32_16x16x4f32((BWD ? m[2 * b + 1] : x.m[2 * b + 1])[r], f[2 * b + 1][r], y1, 0, 0, 0);
       }
+    if (BWD) turn(next);
     h = (y0 + y1) + x.a;
     store4(buf[(i + 1) & 1] + l16 * LD + r0, h);
   };
@@ -734,15 +757,17 @@ __global__ __launch_bounds__(256) void dplr_chunk_scan_kernel(ScanParams p) {
   fetch(x1, 1);
   fetch(x2, 2);
   store4(buf[0] + l16 * LD + r0, h);
-  for (int i = 0; i < p.nw; i += 4) {
-    step(x0, x3, i);
-    if (i + 1 >= p.nw) break;
-    step(x1, x0, i + 1);
-    if (i + 2 >= p.nw) break;
-    step(x2, x1, i + 2);
-    if (i + 3 >= p.nw) break;
-    step(x3, x2, i + 3);
+  if (BWD) turn(x0);
+  int i = 0;
+  for (; i + 4 <= p.nw; i += 4) {  // no way out in between: with one the compiler waited for the loads in flight here
+    step(x0, x1, x3, i);
+    step(x1, x2, x0, i + 1);
+    step(x2, x3, x1, i + 2);
+    step(x3, x0, x2, i + 3);
   }
+  if (i < p.nw) step(x0, x1, x3, i);
+  if (i + 1 < p.nw) step(x1, x2, x0, i + 1);
+  if (i + 2 < p.nw) step(x2, x3, x1, i + 2);
   if (!BWD && p.at + p.nw == p.KN) store4(Srow + (int64_t)p.nw * TG, h);
   if (p.s_out) {
 #pragma unroll
@@ -758,17 +783,17 @@ template <typename T>
 __global__ __launch_bounds__(256) void dplr_out_kernel(ChunkParams p) {
   const Slot s = slot_of(p);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4, t = 16 * wave + l16;
-  const float* X = p.X + s.kept * TG + t * D + 4 * g;
-  const float* Y = p.s2 + s.win * TG + t * D + 4 * g;
-  const float* h = p.hT + s.st * TG + l16 * D + 4 * g;
+  const float* X = p.X + s.kept * TG + block_at(wave, 0);
+  const float* Y = p.s2 + s.win * TG + block_at(wave, 0);
+  const float* h = p.hT + s.st * TG + block_at(0, 0);
   if (16 * wave >= s.len) return;
   floatx4 x[4], y[4], acc[4];
 #pragma unroll
-  for (int b = 0; b < 4; ++b) x[b] = load4(X + 16 * b), y[b] = load4(Y + 16 * b), acc[b] = zero4();
+  for (int b = 0; b < 4; ++b) x[b] = load4(X + 256 * b), y[b] = load4(Y + 256 * b), acc[b] = zero4();
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) mfma4(acc[nb], load4(h + 16 * nb * D + 16 * kb), x[kb]);
+    for (int kb = 0; kb < 4; ++kb) mfma4(acc[nb], load4(h + (4 * nb + kb) * 256), x[kb]);
   if (t < s.len) {
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) store_row4<T>(p.o, (s.tok + t) * D + 16 * nb + 4 * g, acc[nb] + y[nb]);
@@ -784,7 +809,7 @@ __global__ __launch_bounds__(256) void dplr_r_kernel(ChunkParams p) {
   const int l16 = w.l16, g4 = 4 * w.g;
   Row<float> x;
   Row<T> d;
-  x.load(p.X, s.kept * TG + w.t * D + g4);
+  x.load_tile(p.X + s.kept * TG, w.j);
   d.load(p.d_o, s, w);
   put_row(tX, w, [&](int cb) { return x[cb]; });
   put_given(tO, w, d);
@@ -798,7 +823,7 @@ __global__ __launch_bounds__(256) void dplr_r_kernel(ChunkParams p) {
     for (int nb = 0; nb < 4; ++nb) mfma_parts(acc[nb], a, given_col<T>(tO, 16 * nb, 16 * kb + g4, w));
   }
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) store4(p.s2 + s.win * TG + (16 * nb + l16) * D + 16 * w.j + g4, acc[nb]);
+  for (int nb = 0; nb < 4; ++nb) store4(p.s2 + s.win * TG + block_at(nb, w.j), acc[nb]);
 }
 
 // ---- backward: u, dU and dv of a chunk -----------------------------------------------------------------------
@@ -819,8 +844,8 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   v.load(p.v, s, w);
   d_o.load(p.d_o, s, w);
   Row<float> h0, dC;
-  h0.load(p.hT, s.st * TG + w.t * D + g4);
-  dC.load(p.s1, s.win * TG + w.t * D + g4);
+  h0.load_tile(p.hT + s.st * TG, w.j);
+  dC.load_tile(p.s1 + s.win * TG, w.j);
   floatx4 fa[4], fb[4], fk[4];  // the lane's row: a P of the token before, b S, k S
   floatx4 akT[3];               // Aak by t, with earlier blocks
   floatx4 ak[3], qb[3], qk[3];  // Aak, Pqb, Pqk by s, with later blocks (of block i + 1)
@@ -829,7 +854,7 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   for (int i = 0; i < 3; ++i) akT[i] = ak[i] = qb[i] = qk[i] = zero4();
   floatx4 tm[4];  // the lane's row of Tm
   clear(tm);
-  upto(w.j, [&](auto b_) { tm[decltype(b_)::value] = load4(p.Tm + s.kept * TRI + tri_row(w) + 16 * decltype(b_)::value + g4); });
+  upto(w.j, [&](auto b_) { tm[decltype(b_)::value] = load4(p.Tm + s.kept * TRI + tri_block(w.j, decltype(b_)::value)); });
   {
     const Gates gates(x.gk);
     const Decay e(gates, p, s, w);
@@ -944,11 +969,10 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) mfma4(du[nb], frag<true>(ty, 16 * nb + l16, 16 * b + g4), tf);
   });
-  const int64_t wt = s.win * TG + w.t * D + g4;
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb) {
-    store4(p.s3 + wt + 16 * nb, u[nb]);
-    store4(p.s4 + wt + 16 * nb, du[nb]);
+    store4(p.s3 + s.win * TG + block_at(w.j, nb), u[nb]);
+    store4(p.s4 + s.win * TG + block_at(w.j, nb), du[nb]);
   }
   put_cols(tdu, w, du);
   lds_barrier();
@@ -1067,20 +1091,20 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
   float* over = L.sx + 256;                          // [6][64]: row l (l - 1) / 2 + m has what flows into block l from before block m
   float* out_of = L.sx + 640;                        // [3][64]: from block j to D
   float *same_b = L.sx + 832, *same_k = L.sx + 896;  // [64]: the diagonals of dPqb and dPqk
-  const int64_t at = (s.tok + w.t) * D + g4, wt = s.win * TG + w.t * D + g4, ht = s.st * TG + w.t * D + g4;
+  const int64_t at = (s.tok + w.t) * D + g4, wt = s.win * TG;
   const bool ok = w.t < s.len;
   Own<T> x;
   Row<T> v, d_o;
   Row<float> u, du;
   {
     Row<float> h0, dC;
-    dC.load(p.s1, wt);
+    dC.load_tile(p.s1 + wt, w.j);
     x.load_gates(p, s, w);
     v.load(p.v, s, w);
     d_o.load(p.d_o, s, w);
-    u.load(p.s3, wt);
-    du.load(p.s4, wt);
-    h0.load(p.hT, ht);
+    u.load_tile(p.s3 + wt, w.j);
+    du.load_tile(p.s4 + wt, w.j);
+    h0.load_tile(p.hT + s.st * TG, w.j);
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) {  // the wave's sixteen value columns
       const floatx4 y = sum_block(dC[cb] * h0[cb]);
@@ -1205,7 +1229,7 @@ __global__ __launch_bounds__(256, 2) void dplr_grad_kernel(ChunkParams p) {
     }
   }
   keep_as_read(x.b), keep_as_read(x.k), keep_as_read(x.q), keep_as_read(x.a);
-  u.load(p.s3, wt), v.load(p.v, s, w);  // again, ahead of their use: in between the registers are full
+  u.load_tile(p.s3 + wt, w.j), v.load(p.v, s, w);  // again, ahead of their use: in between the registers are full
   lds_barrier();
   // db, dk, relative to the end of the lane's block: the matrices with the contraction along t, first those of q, then those of a
   floatx4 db[4], dk[4], own[4];  // own: b db + k dk of the block's own pairs
@@ -1347,7 +1371,7 @@ constexpr int64_t kept_tiles(int64_t n) { return 3 * n + 1; }  // of a row that 
 
 template <typename K> int lds_limit(K* k) { return lnx_lds_limit(reinterpret_cast<const void*>(k), LDS_BYTES); }
 
-// B8 H16 T4096 bf16 (8192 chunks), us: dplr_prepare 437, dplr_chunk_scan 111, dplr_out 112 (48 KB of reads and 8 of writes per chunk: 4.1 TB/s)
+// B8 H16 T4096 bf16 (8192 chunks), us: dplr_prepare 433, dplr_chunk_scan 89, dplr_out 97 (48 KB of reads and 8 of writes per chunk: 4.8 TB/s)
 template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
   if (int rc = lds_limit(dplr_prepare_kernel<T>)) return rc;
@@ -1369,7 +1393,7 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
   return LNX_OK;
 }
 
-// Same shape: dplr_r 60, dplr_chunk_scan_bwd 104, dplr_u 416, dplr_grad 717 (two workgroups per CU leave 256 registers, and what a
+// Same shape: dplr_r 54, dplr_chunk_scan_bwd 89, dplr_u 416, dplr_grad 709 (two workgroups per CU leave 256 registers, and what a
 // token needs between the pair sums and the last products is more: rows stay as they were read, and three are loaded twice)
 template <typename T> int backward(const lnx_dplr_chunk_grads* g, const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
