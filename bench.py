@@ -97,7 +97,7 @@ def chunk_flops(dk, dv, direct=False):
             "chunk_prepare": 2 * cc * dk,                     # K K^T, Q K^T
             "chunk_scan": 3 * cd + 2 * cc * dv,               # K S, Q S, Tm R, Pm D, K^T D
             "bwd_scan": 3 * cd + 2 * cc * dv,                 # K dS, Pm^T dO, Tm^T dD, Q^T dO, K^T dY
-            "bwd_chunk": 3 * cd + 2 * cc * dv + 4 * cc * dk,  # dO S^T, dv S^T, D dS^T, dO D^T, dv D^T, dPe K, dXe K, dPe^T Q, dXe^T K
+            "bwd_chunk": 3 * cd + 2 * cc * dv + 4 * cc * dk,  # dO S^T, dR S^T, D dS^T, dO D^T, dR D^T, dPe K, dXa K, dPe^T Q, dXe^T K
         }
     return {
         "chunk_prepare": cc * (3 * dk + dv),          # K K^T, Q K^T, Tm(beta K), Tm(beta V)

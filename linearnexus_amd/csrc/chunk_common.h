@@ -116,7 +116,7 @@ __device__ __forceinline__ float lnx_softplus_thr(float x, float thr) {
 }
 
 // 2-byte inputs without a per-channel gate take the kernels of chunk_direct.hip (dk = 256: the scans of chunk_wide.hip), which keep G, Pm, Tm, the
-// per-chunk states and state gradients and D in the workspace (no W, U, dW); every other shape takes the WY-split
+// per-chunk states and state gradients, D and dR in the workspace (no W, U, dW); every other shape takes the WY-split
 // kernels.  The choice reads only fields that the forward and the backward call of one step necessarily share (element
 // type, dk, gate kind), so both calls lay the workspace out the same way; there is one set of kernels per shape.
 inline bool lnx_chunk_direct(const lnx_scan_args* a) {
@@ -135,16 +135,6 @@ template <typename T, int DK> __device__ __forceinline__ int64_t gate_last(int64
 // better (o 3.8e-3 and 4.0e-3 off fp64, dg 3.6e-3 and 4.6e-3): the scaled rows of one level are held to more than bf16.
 constexpr float LNX_KDA_NEAR = 80.f;
 inline bool lnx_chunk_kda(const lnx_scan_args* a) { return a->dtype == LNX_BF16 && a->dk <= 128 && a->gate == LNX_GATE_VECTOR; }
-
-// The gradient that a chunk's right-hand side R = diag(beta) (V - ..) gets, dR, leaves the reverse scans once, as the rows of dv = beta dR, and
-// the chunk-local kernel reads those: whatever it forms of a row is linear in it, and rounded to bf16 one is as far off as the other.
-// (dR beside dv was 16 KB more per chunk of d128 on the way out: B8 H16 T4096 reverse scan 203 -> 180 us, dv = 512 behind
-// dk = 256 450 -> 425.)  A token whose |beta| is below
-// LNX_BETA_MIN (padding has beta = 0) says nothing of dR that way: its row goes out as dR_t, and the chunk-local kernel puts dv_t = beta dR_t
-// right.  2^-24: far from where an fp32 or bf16 product of gradients, values and a beta would leave the normal range.
-constexpr float LNX_BETA_MIN = 5.9604645e-8f;
-__device__ __forceinline__ bool lnx_dv_has_beta(float beta) { return fabsf(beta) >= LNX_BETA_MIN; }
-__device__ __forceinline__ float lnx_dv_factor(float beta) { return lnx_dv_has_beta(beta) ? beta : 1.f; }
 
 inline uint64_t lnx_align256(uint64_t x) { return (x + 255) & ~uint64_t(255); }
 
@@ -177,7 +167,7 @@ inline ChunkWs lnx_chunk_ws_layout(const lnx_scan_args* a) {
     w.SnT = take(bwd ? slots * dv * dk * es : 0);   // states entering the chunks, [v][k]
     w.dSn = take(bwd ? slots * dk * dv * es : 0);   // state gradients leaving the chunks, [v][k]
     w.D = take(bwd ? slots * dv * C * es : 0);      // D^T  [v][token]
-    w.dD = 0;                                       // the reverse scan's rows go out in the caller's dv (lnx_dv_factor)
+    w.dD = take(bwd ? slots * dv * C * es : 0);     // dR^T [v][token]
     w.total = off;
     return w;
   }

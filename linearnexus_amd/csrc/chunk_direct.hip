@@ -1,7 +1,7 @@
 // Chunked delta-rule forward and backward for 2-byte inputs with no / a scalar gate, in the
 // "direct solve" split (dk = 256: the scans are those of chunk_wide.hip): the only per-chunk tensors that cross kernels are Tm = (I + A)^-1, Pm = scale tril(E * Q K^T)
 // and the cumulative gate G from the chunk-parallel prepare kernel, the states entering the chunks and D (forward scan
-// -> chunk-local backward) and the state gradients leaving them (reverse scan -> chunk-local backward).  W, U,
+// -> chunk-local backward) and the state gradients leaving them and dR (reverse scan -> chunk-local backward).  W, U,
 // dD, dW of the WY form are never materialised: with S the state entering a chunk,
 //
 //   Y = K S          R = diag(beta) (V - diag(e^G) Y)      D = Tm R                     (forward substitution applied
@@ -19,7 +19,7 @@
 //   scan_fwd   (one workgroup per (state, slab of dv), sequential over chunks)   O, the entering states, S_T
 //   scan_bwd   (same grid, reverse)                                              the leaving state gradients, dS_0
 //   bwd_chunk  (one workgroup per chunk, all in parallel)                         dq, dk, dbeta, dg from q, k, v, dO, the
-//              two saved states, D and dv = beta dR as the scans left them
+//              two saved states and D, dR as the scans left them (dv leaves the reverse scan)
 //
 // Both scans split their waves into one compute wave per 16 value columns of the slab (matrix work on the tiles in LDS, the fp32 state in MFMA
 // accumulators for the whole sequence) and four or eight mover waves (global loads two chunks ahead into registers, the next chunk's tiles into
@@ -114,7 +114,7 @@ template <int DK, int BVW, bool OUT> struct FScanL {
   // movers carry.
   static constexpr bool CHAIN = BVW == 32;
   static constexpr int BV = BVW, PAD = M::PAD, OPAD = CHAIN ? 16 : 8, LDK = DK + OPAD, LDC = LNX_C + OPAD, LDV = BV + PAD, NCW = BV / 16, MT = CHAIN && DK == 128 ? 512 : 256;
-  static constexpr int LDS = DK + PAD, LDD = LNX_C + PAD;  // of the tiles on their way out: states, D
+  static constexpr int LDS = DK + PAD, LDD = LNX_C + PAD;  // of the tiles on their way out: states, D or dR
   static constexpr int kK = 64 * LDK, kST = BV * LDS, kV = 64 * LDV, kC = 64 * LDC;
   static constexpr int kDT = BV * LDD;
   static constexpr int NOW = OUT && CHAIN ? NCW : 0;  // output waves, one per strip
@@ -713,10 +713,10 @@ int launch_scan_fwd(const DirectParams& p, int nstate, hipStream_t st) {
 // scan_bwd: the reverse pass, same organisation as scan_fwd.  A compute wave owns a 16-column strip of dS (the
 // gradient of the state leaving the chunk); the chain  dS' -> Z = K dS' -> dD -> dR = Tm^T dD -> dY -> dS  stays in
 // its registers.  Needs no forward state: only K, Q, dO, Tm, Pm and the per-token scalars.
-//   B1    buffers of chunk n complete           compute: dS'^T -> LDS (saved), Z, Pm^T dO, dD, dR,
+//   B1    buffers of chunk n complete           compute: dS'^T -> LDS (saved), Z, Pm^T dO, dD, dR (-> LDS, transposed),
 //                                                        dv = beta dR -> LDS, dY
 //                                               movers:  loads of chunk n - 2; chunk n - 1 -> the other buffers
-//   Bmid  dS'^T and dv are in LDS               compute: dS update          movers: dS'^T -> workspace, dv out
+//   Bmid  dS'^T, dR^T and dv are in LDS         compute: dS update          movers: dS'^T, dR^T -> workspace, dv out
 // ---------------------------------------------------------------------------------------
 template <int DK, int BVW> struct BScanL {
   // 32-column slabs are taken where the chip has room for more workgroups, so what counts there is the time of a chunk's
@@ -724,17 +724,18 @@ template <int DK, int BVW> struct BScanL {
   // movers carry.
   static constexpr bool CHAIN = BVW == 32;
   static constexpr int BV = BVW, PAD = M::PAD, OPAD = CHAIN ? 16 : 8, LDK = DK + OPAD, LDC = LNX_C + OPAD, LDV = BV + PAD, NCW = BV / 16, MT = 256;
-  static constexpr int LDS = DK + PAD;  // of the states on their way out
+  static constexpr int LDS = DK + PAD, LDD = LNX_C + PAD;  // of the tiles on their way out: states, D or dR
   static constexpr int kK = 64 * LDK, kST = BV * LDS, kV = 64 * LDV, kC = 64 * LDC;
-  // [2] x (K, scaled Q, dO, Tm, Pm) | dS'^T | dv | scalars [2]
-  static constexpr size_t bytes = sizeof(T) * (2 * (2 * kK + kV + 2 * kC) + kST + kV) + sizeof(float) * 2 * Scal::SIZE;
+  static constexpr int kDT = BV * LDD;
+  // [2] x (K, scaled Q, dO, Tm, Pm) | dS'^T | dR^T | dv | scalars [2]
+  static constexpr size_t bytes = sizeof(T) * (2 * (2 * kK + kV + 2 * kC) + kST + kDT + kV) + sizeof(float) * 2 * Scal::SIZE;
   static constexpr int threads = 64 * NCW + MT;
 };
 
 template <int DK, int GATE, int BVW>
 __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(DirectParams p) {
   typedef BScanL<DK, BVW> L;
-  constexpr int LDK = L::LDK, LDC = L::LDC, BV = L::BV, LDV = L::LDV, NCW = L::NCW, LDS = L::LDS;
+  constexpr int LDK = L::LDK, LDC = L::LDC, BV = L::BV, LDV = L::LDV, NCW = L::NCW, LDS = L::LDS, LDD = L::LDD;
   constexpr bool CHAIN = L::CHAIN;
   constexpr int MT = L::MT;  // mover threads
   constexpr int KT = DK / 16;
@@ -745,7 +746,8 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
   T* sTm = sdO + 2 * L::kV;
   T* sP = sTm + 2 * L::kC;
   T* sdST = sP + 2 * L::kC;            // dS'^T [v][dk] on its way to the workspace
-  T* sdV = sdST + L::kST;              // dv = beta dR [token][v] on its way out
+  T* sdRT = sdST + L::kST;             // dR^T [v][token] on its way to the workspace
+  T* sdV = sdRT + L::kDT;              // dv = beta dR [token][v] on its way out
   float* sSc = reinterpret_cast<float*>(sdV + L::kV);
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -822,7 +824,7 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
         float* sc = sSc + pb * Scal::SIZE;
         const float gam = (GATE == LNX_GATE_SCALAR) ? __expf(R.g) : 1.f;
         const float bt = (mt < R.len) ? R.b : 0.f;
-        sc[Scal::BETA + mt] = lnx_dv_factor(bt);
+        sc[Scal::BETA + mt] = bt;
         sc[Scal::GAM + mt] = bt * gam;  // dY = -(beta e^G) dR
         sc[Scal::R + mt] = (GATE == LNX_GATE_SCALAR) ? __expf(fminf(R.gc - R.g, 0.f)) : 1.f;
         if (mt == 0) sc[Scal::DEC] = (GATE == LNX_GATE_SCALAR) ? __expf(R.gc) : 1.f;
@@ -846,6 +848,7 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
       lds_barrier();  // Bmid
       const int64_t slot = (int64_t)row * N + n;
       unstage_tile<T, BV, DK, true, MT>(at<T>(p.ws, p.off.dSn) + slot * p.dv * DK + (int64_t)v0 * DK, DK, sdST, LDS, BV, mt);
+      unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.dD) + slot * p.dv * 64 + (int64_t)v0 * 64, 64, sdRT, LDD, BV, mt);
       int tok0, len;
       chunk_span(span, n, tok0, len);
       unstage_tile_checked<T, 64, BV>(p.dv_out + tok_index(p.geom, row, tok0) * p.dv + v0, tsv, sdV, LDV, len, mt);
@@ -985,6 +988,8 @@ __global__ __launch_bounds__((BScanL<DK, BVW>::threads)) void scan_bwd_kernel(Di
 #pragma unroll
     for (int ci = 0; ci < KT; ++ci) S16::mma(dS[ci], fq[1][ci], fo[1]);
     __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) store_t(z[i], sdRT + vs * LDD + S16::row0(i), LDD, lane);
     // dY = -beta e^G dR
     bd0 = S16::from_acc(-sv[0] * z[0], -sv[1] * z[1]);
     bd1 = S16::from_acc(-sv[2] * z[2], -sv[3] * z[3]);
@@ -1024,19 +1029,16 @@ int launch_scan_bwd(const DirectParams& p, int nstate, hipStream_t st) {
 
 // ---------------------------------------------------------------------------------------
 // bwd_chunk: the chunk-local gradients, one workgroup per chunk, all chunks in parallel.  Reads q, k, v, dO of the
-// chunk, the states S (entering) and dS' (leaving), D and dv = beta dR from the two scans; writes dq, dk, dbeta, dg (dv left
+// chunk, the states S (entering) and dS' (leaving) and D, dR from the two scans; writes dq, dk, dbeta, dg (dv left
 // the reverse scan).  A loop over 32-column slabs of the value dimension accumulates every product that contracts
 // over value columns; the slabs arrive in two LDS buffers through loads that bypass the registers, two slabs ahead:
-//   dQa = dO S^T     dK1 = dv S^T     dK2 = D dS'^T     dPm = dO D^T     dAm = dv D^T     <dv_t, v_t>     <dS', S>
+//   dQa = dO S^T     dK1 = dR S^T     dK2 = D dS'^T     dPm = dO D^T     dAm = dR D^T     <dR_t, v_t>     <dS', S>
 // then an epilogue over the chunk's tokens:
-//   dPe = scale tril(E * dPm)          dXe = -tril(E * dAm, -1)
+//   dPe = scale tril(E * dPm)          dXa = -tril(E * dAm, -1)          dXe = diag(beta) dXa
 //   dq  = scale e^G dQa + dPe K
-//   row = dXe K - e^G dK1              m_t = <k_t, row_t>                 dbeta = (<dv, v> + m) / beta
-//   dk  = row + e^{G_C - G} dK2 + dPe^T Q + dXe^T K
-//   dG  = <q, dq> - <k, dk> + 2 m;   dG_C += sum_t e^{G_C - G_t} <k_t, dK2_t> + e^{G_C} <dS', S>;   dg = reverse cumsum(dG)
-// A token with next to no beta (lnx_dv_has_beta) comes as dR_t instead of dv_t: beta times its row of dXe and of `row` is what enters dk and
-// dG, dbeta_t = <dR_t, v_t> + m_t, and its dv_t is put right here.  (dbeta_t is also dAm_tt / beta_t^2, which needs no v, 20 us less here; but that
-// is off by all of D's error, where v is exact: 4.0e-3 instead of 3.1e-3.)
+//   row = dXa K - e^G dK1              m_t = <k_t, row_t>                 dbeta = <dR, v> + m
+//   dk  = beta row + e^{G_C - G} dK2 + dPe^T Q + dXe^T K
+//   dG  = <q, dq> - <k, dk> + 2 beta m;   dG_C += sum_t e^{G_C - G_t} <k_t, dK2_t> + e^{G_C} <dS', S>;   dg = reverse cumsum(dG)
 // Wave (wi, wj) owns the token-row tile wi and the key-column tiles NKT wj .. of the [64 x dk] accumulators and the
 // (wi, wj) tile of the [64 x 64] ones.  The epilogue's tiles that are only read through transposing LDS loads get a row
 // stride of 64 bytes mod 256, which spreads the four rows that half a wave reads over all banks.
@@ -1051,15 +1053,15 @@ template <int DK> struct BChunkL {
   static constexpr int NW = DK == 256 ? 8 : 4, THREADS = 64 * NW, NBUF = DK == 256 ? 3 : 2;
   static constexpr int SV = 32;
   static constexpr int SC = DK < 128 ? DK : 128, NH = DK / SC;  // a state slab is NH tiles of SC columns
-  typedef SwzTile<64, SV> TokT;            // dO, V, dv slabs [64][SV], read by rows
-  typedef SwzTile<SV, 64, false> TrT;      // D^T slabs [SV][64], transposing reads only
+  typedef SwzTile<64, SV> TokT;            // dO, V slabs [64][SV], read by rows
+  typedef SwzTile<SV, 64, false> TrT;      // D^T, dR^T slabs [SV][64], transposing reads only
   typedef SwzTile<SV, SC, false> StT;      // S^T, dS'^T slabs [SV][SC], transposing reads only
   static constexpr int LDKT = DK + 32;     // the epilogue's K, Q tiles [64][DK], transposing reads
   static constexpr int LDC = 64 + 8;       // dPe, dPe^T, dXa, dXe^T [64][64], read by rows
   static constexpr int LDK = DK + 8;       // staging tile for dq, dk [64][DK]
   static constexpr int kC = 64 * LDC, kRow = 64 * LDKT, kSt = 64 * LDK;
-  // one slab of the loop: dO | V | dv | D^T | S^T | dS'^T, unpadded; NBUF of them, filled by LDS-direct loads in turn
-  static constexpr int oV = TokT::BYTES, odV = 2 * TokT::BYTES, oDT = 3 * TokT::BYTES, oSn = oDT + TrT::BYTES, odSn = oSn + NH * StT::BYTES;
+  // one slab of the loop: dO | V | D^T | dR^T | S^T | dS'^T, unpadded; NBUF of them, filled by LDS-direct loads in turn
+  static constexpr int oV = TokT::BYTES, oDT = 2 * TokT::BYTES, odRT = oDT + TrT::BYTES, oSn = odRT + TrT::BYTES, odSn = oSn + NH * StT::BYTES;
   static constexpr int slab_bytes = odSn + NH * StT::BYTES;
   static constexpr size_t loop_bytes = NBUF * slab_bytes;
   // the staging tiles of dq and dk: over dPe and dPe^T, over dXa and dXe^T; dk = 256: dq over all four, dk's behind the Q tile
@@ -1089,7 +1091,7 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
   extern __shared__ __align__(16) char smem[];
   float* sG = reinterpret_cast<float*>(smem);
   float* sBeta = sG + 64;
-  float* sRdv = sBeta + 64;   // <dv_t, v_t>
+  float* sRdv = sBeta + 64;   // <dR_t, v_t>
   float* sM = sRdv + 64;      // [2]: m_t is the sum of the two
   float* sdG = sM + 128;      // [2]: <q_t, dq_t> - <k_t, dk_t> is the sum of the two
   float* sMisc = sdG + 128;    // [8 + wave] = the wave's share of sum_t r_t <k_t, dK2_t>, [16 + wave] = of <dS', S>
@@ -1157,9 +1159,9 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
   const T* gSn = at<const T>(p.ws, p.off.SnT) + slot * p.dv * DK;
   const T* gdSn = at<const T>(p.ws, p.off.dSn) + slot * p.dv * DK;
   const T* gDT = at<const T>(p.ws, p.off.D) + slot * p.dv * 64;
+  const T* gdRT = at<const T>(p.ws, p.off.dD) + slot * p.dv * 64;
   const T* gdO = p.d_o + tbase * p.dv;
   const T* gV = p.v + tbase * p.dv;
-  const T* gdV = p.dv_out + tbase * p.dv;
   auto issue = [&](int v0, int b) {
     const unsigned dst = slab0 + b * L::slab_bytes;
     int r, c;
@@ -1181,9 +1183,7 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
     if (NW == 4 || wave >= 4) {
       TrT::src(j, lane, r, c);
       dma16(gDT + (int64_t)(v0 + r) * 64 + c, dst + L::oDT + 1024 * j);
-      TokT::src(j, lane, r, c);
-      r = min(r, len - 1);
-      dma16(gdV + (int64_t)r * tsv + v0 + c, dst + L::odV + 1024 * j);
+      dma16(gdRT + (int64_t)(v0 + r) * 64 + c, dst + L::odRT + 1024 * j);
     }
   };
   constexpr int PER_WAVE = 2 * NH * StT::NINSTR / NW + 16 / NW;  // loads per wave and slab
@@ -1201,8 +1201,8 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
     lds_barrier();
     const T* sdO = reinterpret_cast<const T*>(sSlab + b * L::slab_bytes);
     const T* sV = reinterpret_cast<const T*>(sSlab + b * L::slab_bytes + L::oV);
-    const T* sdV = reinterpret_cast<const T*>(sSlab + b * L::slab_bytes + L::odV);
     const T* sDT = reinterpret_cast<const T*>(sSlab + b * L::slab_bytes + L::oDT);
+    const T* sdRT = reinterpret_cast<const T*>(sSlab + b * L::slab_bytes + L::odRT);
     const T* sSn = reinterpret_cast<const T*>(sSlab + b * L::slab_bytes + L::oSn);
     const T* sdSn = reinterpret_cast<const T*>(sSlab + b * L::slab_bytes + L::odSn);
     static_assert(SV == 32, "two 16-wide steps per slab");
@@ -1213,27 +1213,27 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
 #pragma unroll
     for (int k0 = 0; k0 < SV; k0 += 16) {
       const M::Frag fdO = TokT::load(sdO, 32 * wi + fr, k0 + kg8);
-      const M::Frag fdV = TokT::load(sdV, 32 * wi + fr, k0 + kg8);
+      const M::Frag fdR = TrT::load_t(sdRT, k0, 32 * wi, lane);
       const M::Frag fDi = TrT::load_t(sDT, k0, 32 * wi, lane);
       const M::Frag fDj = TrT::load_t(sDT, k0, 32 * jt, lane);
       if (has_p) M::mma(aP[0][0], fdO, fDj);
-      if (has_a) M::mma(aA[0][0], fdV, fDj);
+      if (has_a) M::mma(aA[0][0], fdR, fDj);
 #pragma unroll
       for (int c = 0; c < NKT; ++c) {
         const int col = 32 * (NKT * wj + c), st = NH == 1 ? 0 : (col / SC) * (StT::BYTES / 2);
         const M::Frag fS = StT::load_t(sSn + st, k0, NH == 1 ? col : col % SC, lane);
         const M::Frag fdS = StT::load_t(sdSn + st, k0, NH == 1 ? col : col % SC, lane);
         M::mma(aQ[0][c], fdO, fS);
-        M::mma(aK1[0][c], fdV, fS);
+        M::mma(aK1[0][c], fdR, fS);
         M::mma(aK2[0][c], fDi, fdS);
       }
     }
-    {  // <dv_t, v_t> over this slab: thread = (token tid / TPT, SV / TPT value columns)
+    {  // <dR_t, v_t> over this slab: thread = (token tid / TPT, SV / TPT value columns)
       typedef bf16_t VecV __attribute__((ext_vector_type(SV / TPT)));
-      const int at = TokT::at(tid / TPT, (SV / TPT) * (tid % TPT));
-      const VecV vv = *reinterpret_cast<const VecV*>(sV + at), dv = *reinterpret_cast<const VecV*>(sdV + at);
+      const int t = tid / TPT, c0 = (SV / TPT) * (tid % TPT);
+      const VecV vv = *reinterpret_cast<const VecV*>(sV + TokT::at(t, c0));
 #pragma unroll
-      for (int e = 0; e < SV / TPT; ++e) rdv += (float)vv[e] * (float)dv[e];
+      for (int e = 0; e < SV / TPT; ++e) rdv += (float)vv[e] * (float)sdRT[TrT::at(c0 + e, t)];
     }
     if (GATE == LNX_GATE_SCALAR) {  // <dS', S> over this slab: the two tiles share one layout, so granule by granule
 #pragma unroll
@@ -1255,19 +1255,9 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
     ss = wave_sum(ss);
     if (lane == 0) sMisc[16 + wave] = ss;  // one slot per wave, added in a fixed order below
   }
-  lds_barrier();  // slab tiles are dead from here on, and dv has been read
+  lds_barrier();  // slab tiles are dead from here on
 
   // ---- epilogue ----
-  if (__ballot(lane < len && !lnx_dv_has_beta(sBeta[lane])) != 0) {  // dv_t = beta dR_t, thread = (token tid / TPT, eight columns in turn)
-    const int t = tid / TPT;
-    if (t < len && !lnx_dv_has_beta(sBeta[t])) {
-#pragma unroll 1
-      for (int c = 8 * (tid % TPT); c < p.dv; c += 8 * TPT) {
-        M::Frag* x = reinterpret_cast<M::Frag*>(p.dv_out + (tbase + t * ts) * p.dv + c);
-        *x = scaled(*x, sBeta[t]);
-      }
-    }
-  }
   {  // K and Q rows, normalised
     typedef TileRegs<T, 64, DK, THREADS> RowTile;
 #pragma unroll
@@ -1281,17 +1271,14 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
       *reinterpret_cast<typename Vec16<T>::V*>(sQ + r * LDKT + c) = y;
     }
   }
-  // The cumulative gate and what the row's products lack in beta (1 or, where dR came, beta) of this lane's sixteen accumulator rows (four
-  // runs of four), as vectors and once: read one by one between the tile stores below, each read would wait out its own round trip to LDS
-  // (the stores might alias it).
+  // The cumulative gate and beta of this lane's sixteen accumulator rows (four runs of four), as vectors and once: read one
+  // by one between the tile stores below, each read would wait out its own round trip to LDS (the stores might alias it).
   floatx4 gi[4], bi[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int i0 = 32 * wi + 8 * q + 4 * (lane >> 5);
     gi[q] = load4(sG + i0);
     bi[q] = load4(sBeta + i0);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bi[q][e] = lnx_dv_has_beta(bi[q][e]) ? 1.f : bi[q][e];
   }
   const float gC = sG[63];
   {
@@ -1435,10 +1422,9 @@ __global__ __launch_bounds__(BChunkL<DK>::THREADS, 2) void bwd_chunk_kernel(Dire
   }
   if (wave == 0) {
     const int t = lane;
-    const float bt = sBeta[t], m = sM[t] + sM[64 + t];
-    if (t < len) p.dbeta[tbase + t * ts] = (sRdv[t] + m) / lnx_dv_factor(bt);
+    if (t < len) p.dbeta[tbase + t * ts] = sRdv[t] + (sM[t] + sM[64 + t]);
     if (GATE == LNX_GATE_SCALAR) {  // dg = reverse cumulative sum of dG over the chunk
-      float d = (L::DOTS ? sdG[t] + sdG[64 + t] : sdG[t]) + 2.f * (lnx_dv_has_beta(bt) ? m : bt * m);
+      float d = (L::DOTS ? sdG[t] + sdG[64 + t] : sdG[t]) + 2.f * sBeta[t] * (sM[t] + sM[64 + t]);
       if (t == 63) d += waves_sum(sMisc + 8) + __expf(gC) * waves_sum(sMisc + 16);
 #pragma unroll
       for (int s_ = 1; s_ < 64; s_ <<= 1) {

@@ -65,7 +65,7 @@ template <int NC, int NCW> struct WideL {
   static constexpr int kRow = 64 * LDK, kC = 64 * LDC, kV = 64 * LDV, kT = BV * LDT;
   static constexpr bool AHEAD = NC == 1;  // the movers hold two chunks, and LDS two K tiles
   static constexpr int NK2 = AHEAD ? 2 : 1;
-  // K [NK2] | Q | Tm | Pm | V (reverse: dO) | O (reverse: dv) on its way out | D^T on its way out (forward) | scalars
+  // K [NK2] | Q | Tm | Pm | V (reverse: dO) | O (reverse: dv) on its way out | D^T (reverse: dR^T) on its way out | scalars
   static constexpr size_t bytes = sizeof(T) * ((NK2 + 1) * kRow + 2 * kC + 2 * kV + kT) + sizeof(float) * 272;
   static constexpr int threads = 64 * NCW + 256;
   static_assert(bytes <= 160 * 1024, "LDS");
@@ -307,7 +307,7 @@ template <int NC> struct Strip {
   }
 };
 
-// D of a column tile as operands, transposed to LDS: 16 bytes are eight tokens of a value column
+// D (dR) of a column tile as operands, transposed to LDS: 16 bytes are eight tokens of a value column
 __device__ __forceinline__ void put_t(T* sT, int ld, int col, const Frag (&b)[2], int lane) {
 #pragma unroll
   for (int s = 0; s < 2; ++s) *reinterpret_cast<bf16x8*>(sT + (col + (lane & 15)) * ld + 32 * s + grp(lane)) = b[s];
@@ -548,7 +548,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_fwd_kerne
 template <int GATE, int NC, int NCW>
 __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kernel(DirectParams p) {
   typedef WideL<NC, NCW> L;
-  constexpr int BV = L::BV, LDK = L::LDK, LDC = L::LDC, LDV = L::LDV;
+  constexpr int BV = L::BV, LDK = L::LDK, LDC = L::LDC, LDV = L::LDV, LDT = L::LDT;
   extern __shared__ __align__(16) char smem[];
   T* sK = reinterpret_cast<T*>(smem);
   T* sQ = sK + L::NK2 * L::kRow;
@@ -556,7 +556,8 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
   T* sP = sTm + L::kC;
   T* sdO = sP + L::kC;
   T* sdV = sdO + L::kV;
-  float* sc = reinterpret_cast<float*>(sdV + L::kV);
+  T* sdRT = sdV + L::kV;
+  float* sc = reinterpret_cast<float*>(sdRT + L::kT);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   Chain ch;
   if (!chain_of<BV>(p, ch)) return;
@@ -624,6 +625,7 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
       lds_barrier();  // B2
       int tok0, len;
       chunk_span(ch.span, n, tok0, len);
+      unstage_tile<T, BV, 64, true>(at<T>(p.ws, p.off.dD) + ((int64_t)ch.row * N + n) * p.dv * 64 + (int64_t)v0 * 64, 64, sdRT, LDT, BV, mt);
       unstage_tile_checked<T, 64, BV>(p.dv_out + tok_index(p.geom, ch.row, tok0) * p.dv + v0, tsv, sdV, LDV, len, mt);
       normalise(nxt, 0);
       commit(nxt);
@@ -726,12 +728,15 @@ __global__ __launch_bounds__((WideL<NC, NCW>::threads)) void wide_scan_bwd_kerne
         }
         gm[h] = load4(sc + Sc::GAM + row0(i) + g8);
         const int t = row0(i) + row_of(lane);
-        const float bt = lnx_dv_factor(sc[Sc::BETA + t]);
+        const float bt = sc[Sc::BETA + t];
 #pragma unroll
         for (int c = 0; c < NC; ++c) store4(sdV + t * LDV + vs + 16 * c + 4 * (lane >> 4), w[c] * bt);
       }
 #pragma unroll
-      for (int c = 0; c < NC; ++c) by[c][s] = S16::from_acc(-gm[0] * x[c][0], -gm[1] * x[c][1]);
+      for (int c = 0; c < NC; ++c) {
+        *reinterpret_cast<bf16x8*>(sdRT + (vs + 16 * c + (lane & 15)) * LDT + 32 * s + g8) = S16::from_acc(x[c][0], x[c][1]);
+        by[c][s] = S16::from_acc(-gm[0] * x[c][0], -gm[1] * x[c][1]);
+      }
     }
     // ---- dS <- e^{G_C} dS' + (scale e^G Q)^T dO ----
     dS.template add<GATE == LNX_GATE_SCALAR>(sQ, LDK, foq, lane, sc[Sc::DEC]);

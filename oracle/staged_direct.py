@@ -14,8 +14,7 @@ triangular system is applied to the right-hand side of each chunk instead of bei
 
 (gated_deltanet.py:450-477 solves M [w | u] = rhs by forward substitution; D = u - w S is the same solve applied to
 rhs_u - rhs_w S.)  Tm, Pm and G leave the chunk-parallel prepare kernel; the forward scan keeps the states entering
-the chunks (Sn) and D; the reverse scan keeps the state gradients leaving the chunks (dSn) and writes dv, from which the chunk-local
-kernel has dR (tokens with |beta| < BETA_MIN leave as dR themselves).
+the chunks (Sn) and D; the reverse scan keeps the state gradients leaving the chunks (dSn) and dR, and writes dv.
 
 Reverse scan, given dO and the gradient dS' of the state leaving the chunk:
   dD = Pm^T dO + diag(r) K dS'        dR = Tm^T dD        dV = diag(beta) dR        dY = -diag(beta gam) dR
@@ -28,8 +27,6 @@ from __future__ import annotations
 import numpy as np
 
 from .staged import C, _chunks
-
-BETA_MIN = 2.0 ** -24
 
 
 def forward(q, k, v, beta, g=None, scale=None, initial_state=None, dtype=np.float64):
@@ -93,40 +90,37 @@ def backward(ws, dO, dS_T=None, dtype=np.float64):
               + np.swapaxes(k[:, :, n], -1, -2) @ dY)
     dS0 = dS
 
-    # ---- reverse scan, continued: per chunk it also leaves x = dv = beta dR, or dR where there is next to no beta ----
+    # ---- reverse scan, continued: per chunk it also leaves dR and dv = beta dR ----
     # (recomputed here for all chunks at once from the saved dSn)
     D = ws["D"]
     Z = k @ dSn
     dD = np.swapaxes(Pm, -1, -2) @ dOc + r * Z
     dR = TmT @ dD
-    has = np.abs(beta) >= BETA_MIN
-    x = np.where(has, beta, 1.0)[..., None] * dR
-    f = np.where(has, 1.0, beta)  # what x lacks
-    dv_ = f[..., None] * x
+    dv_ = beta[..., None] * dR
 
-    # ---- chunk-local kernel: reads q, k, v, dO, Pm's gate factors (G), beta, Sn, dSn, D, x ----
+    # ---- chunk-local kernel: reads q, k, v, dO, Pm's gate factors (G), beta, Sn, dSn, D, dR ----
     idx = np.arange(C)
     incl = idx[:, None] >= idx[None, :]
     strict = idx[:, None] > idx[None, :]
     E = np.exp(np.where(incl, G[..., :, None] - G[..., None, :], -np.inf))
     # loop over the value columns (every product contracts over v)
     dQa = dOc @ np.swapaxes(Sn, -1, -2)        # [C, dk]
-    dK1 = x @ np.swapaxes(Sn, -1, -2)
+    dK1 = dR @ np.swapaxes(Sn, -1, -2)
     dK2 = D @ np.swapaxes(dSn, -1, -2)
     dPm = dOc @ np.swapaxes(D, -1, -2)         # [C, C], masked below
-    dAm = x @ np.swapaxes(D, -1, -2)
-    x_v = np.sum(x * v, -1)                    # row dots <x_t, v_t>
+    dAm = dR @ np.swapaxes(D, -1, -2)
+    rd_v = np.sum(dR * v, -1)                  # row dots <dR_t, v_t>
     ss = np.sum(dSn * Sn, (-1, -2))            # <dS', S> per chunk
     # epilogue over the chunk's tokens
     dPe = np.where(incl, scale * E * dPm, 0.0)
     dXa = np.where(strict, -E * dAm, 0.0)      # dA * E
-    dXe = f[..., None] * dXa
+    dXe = beta[..., None] * dXa
     dq = scale * gam * dQa + dPe @ k
-    row = dXa @ k - gam * dK1                  # row-type part of dk but for the factor f
+    row = dXa @ k - gam * dK1                  # row-type part of dk before its factor beta
     m = np.sum(k * row, -1)
-    dk_ = f[..., None] * row + r * dK2 + np.swapaxes(dPe, -1, -2) @ q + np.swapaxes(dXe, -1, -2) @ k
-    dbeta = (x_v + m) / np.where(has, beta, 1.0)
-    dG = np.sum(q * dq, -1) - np.sum(k * dk_, -1) + 2.0 * f * m
+    dk_ = beta[..., None] * row + r * dK2 + np.swapaxes(dPe, -1, -2) @ q + np.swapaxes(dXe, -1, -2) @ k
+    dbeta = rd_v + m
+    dG = np.sum(q * dq, -1) - np.sum(k * dk_, -1) + 2.0 * beta * m
     dG[..., -1] += np.sum(r * dK2 * k, (-1, -2)) + np.exp(GC) * ss
     dg = np.flip(np.cumsum(np.flip(dG, 3), 3), 3)
 
