@@ -16,12 +16,9 @@
 // flight) forms dR and accumulates what contracts over value columns on 16x16x32 products: wave w owns the channels 64 s + 16 w .. of every
 // set s of 64 and all tokens, so that an accumulator element is at the place where pair_levels wants its channel and token:
 // lane (c = lane % 16, kq = lane / 16) holds the tokens 16 t + 4 kq + e of channel c, and everything between the loop and the
-// tiles on their way out happens in registers.  The four pair sums share their factors (pair_sums_near, or pair_sums where a channel forgets too
-// much for one factor a token).
-// Measured at B4 H16 T8192 d128 (8192 chunks): 454 - 466 us by box for 280 KB a chunk, 5.1 TB/s; with pair_sums 480 - 488.  (Nine addresses of the
-// output phase held in scratch memory over the pair sums cost 37 us: their reloads wait for the stores of dv.)  Measured with pair_sums: two thirds
-// of the time on vector instructions, the normalisation about 20 us of this kernel and kda_prepare together, the gate's activation 65; bwd_dqk and
-// bwd_wy2, which passed dW, a partial dk
+// tiles on their way out happens in registers.  The four pair sums share their factors (pair_sums).
+// Measured at B4 H16 T8192 d128 (8192 chunks): 461 - 472 us by box for 280 KB a chunk, 5 TB/s, and two thirds of the time on vector instructions (the
+// normalisation adds about 20 us to it and kda_prepare together, the gate's activation 65); bwd_dqk and bwd_wy2, which passed dW, a partial dk
 // and an fp32 partial gradient of the gate through memory, 402 + 497 us behind and before 217 us of normalisation outside.  The cumulative gate
 // is summed up again from the gate: 461 -> 470 us here, 25 less where the prepare kernel wrote it.  With eight waves and one workgroup per CU
 // 650 us: of 20.6 us a chunk 8.5 were pair sums with nothing in flight.
@@ -193,64 +190,6 @@ __device__ __forceinline__ void pair_sums(PairSums& s, const float (&g)[16], con
     sums_diag(s, g, dec, k4, q4, beta, P, A, t, lane);
   }
   s.settle();
-}
-
-// The same sums where one factor a token serves all pairs (LNX_KDA_NEAR): f = e^{G - mid} of a row token, fi = e^{mid - G} of a column token.
-// The scaled rows come in two parts, rounded and what the rounding left: at the levels, too, neighbours' rows often have a factor of 1, and
-// what the rounding of one token's row and of its partner's leaves does not cancel in the gate's gradient (gates of 0.4 a token, dg off by 8.6e-3
-// with rounded rows, 3.0e-3 so; at the levels 7.0e-3).
-struct Split {
-  bf16x4 hi, lo;
-  __device__ __forceinline__ explicit Split(floatx4 x) : hi(pack_bf16x4(x)) {
-    lo = pack_bf16x4(x - floatx4{(float)hi[0], (float)hi[1], (float)hi[2], (float)hi[3]});
-  }
-};
-__device__ __forceinline__ floatx4 widen4(bf16x4 x) { return floatx4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]}; }
-__device__ __forceinline__ floatx4 four(const float (&x)[16], int t) { return floatx4{x[4 * t], x[4 * t + 1], x[4 * t + 2], x[4 * t + 3]}; }
-__device__ __forceinline__ void pair_sums_near(PairSums& s, const float (&f)[16], const float (&fi)[16], const bf16x4 (&k4)[4], const bf16x4 (&q4)[4],
-                                               const float* __restrict__ beta, const T* __restrict__ P, const T* __restrict__ A, int lane_) {
-  const int lane = fresh(lane_);
-  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-  // Products over 32 throughout, half of one empty where a block has no neighbour: a 16x16x16 product whose sum the next 16x16x32 one went on
-  // with had two of its four elements lost (hipcc of ROCm 7.2 leaves too few wait states between the two kinds).
-  const bf16x4 none = {};
-  {
-    const Split b[4] = {Split(four(fi, 0) * widen4(k4[0])), Split(four(fi, 1) * widen4(k4[1])), Split(four(fi, 2) * widen4(k4[2])), Split(four(fi, 3) * widen4(k4[3]))};
-#pragma unroll
-    for (int ti = 0; ti < 4; ++ti) {
-      floatx4 xp = zero, xa = zero;
-#pragma unroll
-      for (int t = 0; t <= ti; t += 2) {
-        const bool two = t < ti;
-        const Frag p = S16::join(block_rows(P, ti, t, lane), two ? block_rows(P, ti, t + 1, lane) : none);
-        const Frag a = S16::join(block_rows(A, ti, t, lane), two ? block_rows(A, ti, t + 1, lane) : none);
-        const Frag hi = S16::join(b[t].hi, two ? b[t + 1].hi : none), lo = S16::join(b[t].lo, two ? b[t + 1].lo : none);
-        S16::mma(xp, p, hi), S16::mma(xa, a, hi), S16::mma(xp, p, lo), S16::mma(xa, a, lo);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s.rp[4 * ti + e] += f[4 * ti + e] * xp[e], s.ra[4 * ti + e] += f[4 * ti + e] * xa[e];
-    }
-  }
-  s.settle();
-#pragma unroll
-  for (int which = 0; which < 2; ++which) {  // the row tokens' f q through P, their f beta k through A
-    const T* M = which ? A : P;
-    auto row = [&](int t) { return four(f, t) * (which ? load4(beta + 16 * t + 4 * (lane >> 4)) * widen4(k4[t]) : widen4(q4[t])); };
-    const Split b[4] = {Split(row(0)), Split(row(1)), Split(row(2)), Split(row(3))};
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
-      floatx4 x = zero;
-#pragma unroll
-      for (int t = tj & 2; t < 4; t += 2) {
-        const bool two = t >= tj;
-        const Frag m = S16::join(two ? block_cols(M, t, tj, lane) : none, block_cols(M, t + 1, tj, lane));
-        S16::mma(x, m, S16::join(two ? b[t].hi : none, b[t + 1].hi)), S16::mma(x, m, S16::join(two ? b[t].lo : none, b[t + 1].lo));
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s.co[4 * tj + e] += fi[4 * tj + e] * x[e];
-    }
-    s.settle();
-  }
 }
 
 // One step of sixteen sums over sixteen lanes: of 2 M values a lane keeps M, adding what its partner sends
@@ -499,10 +438,9 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
     }
   dma_wait<0>();
   lds_barrier();
-  int near[NS];  // one factor a token serves the wave's channels of the set
 #pragma unroll
   for (int u = 0; u < NS; ++u) {
-    float gb = 0.f, highest = -1.f;
+    float gb = 0.f;
     if constexpr (GRAW) gb = p.gbias ? p.gbias[(row % p.geom.H) * DK + 64 * u + 16 * wave + l16] : 0.f;
     float before = 0.f;  // what the blocks of sixteen tokens before add
 #pragma unroll
@@ -513,7 +451,6 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
         if constexpr (GRAW) G[u][x] = gna * lnx_softplus_thr(G[u][x] + gb, p.gthr);
         G[u][x] *= LOG2E;
         G[u][x] = 16 * t + 4 * kq + e < len ? G[u][x] : 0.f;
-        highest = fmaxf(highest, G[u][x]);
         if (e) G[u][x] += G[u][x - (e ? 1 : 0)];
       }
       // as the reverse sum of its gradient below
@@ -526,16 +463,7 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
       for (int e = 0; e < 4; ++e) G[u][4 * t + e] += add;
       before += __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
     }
-    // NaN shows in the sum
-    near[u] = __ballot(!(highest <= 0.f && before >= -LNX_KDA_NEAR)) == 0 ? 1 : 0;
     settle16(G[u]);
-  }
-  // the second set's waits where the first one's gradient will, each lane in its own places
-  float* sG0 = reinterpret_cast<float*>(region + L::oG0);
-  auto waiting = [&](int x) { return (16 * (x >> 2) + 4 * kq + (x & 3)) * L::LDF + 16 * wave + l16; };
-  if constexpr (NS == 2) {
-#pragma unroll
-    for (int x = 0; x < 16; ++x) sG0[waiting(x)] = G[1][x];
   }
   float dq[NS][16], dk[NS][16], dG[16];
   // K and Q at this lane's channel and tokens, normalised (rounded as the op rounds the normalised rows), zero past the chunk's end
@@ -579,23 +507,7 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
         tot += kv * k2;
       }
     }
-    s.settle();
-    // One or the other, as two choices that the compiler cannot tell to be one: made into one, both sides started from copies of s (256
-    // registers and 85 in scratch memory).
-    int one_level = __builtin_amdgcn_readfirstlane(near[u]);
-    asm volatile("" : "+s"(one_level));
-#pragma unroll 1
-    for (int once = one_level; once == 0; once = 1) pair_sums(s, G[u], k4, q4, sBeta, sP, sA, lane);
-    s.settle();
-    asm volatile("" : "+s"(one_level));
-    if (one_level) {
-      settle16(G[u]);
-      const float mid = 0.5f * gC;
-      float f[16], fi[16];
-#pragma unroll
-      for (int x = 0; x < 16; ++x) f[x] = __builtin_amdgcn_exp2f(G[u][x] - mid), fi[x] = __builtin_amdgcn_exp2f(mid - G[u][x]);
-      pair_sums_near(s, f, fi, k4, q4, sBeta, sP, sA, lane);
-    }
+    pair_sums(s, G[u], k4, q4, sBeta, sP, sA, lane);
     float mv[16];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -640,11 +552,9 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
     }
     settle16(dG);
     if (u + 1 < NS) {
+      float* sG0 = reinterpret_cast<float*>(region + L::oG0);
 #pragma unroll
-      for (int x = 0; x < 16; ++x) G[u + 1][x] = sG0[waiting(x)];
-      settle16(G[u + 1]);
-#pragma unroll
-      for (int x = 0; x < 16; ++x) sG0[waiting(x)] = dG[x];
+      for (int x = 0; x < 16; ++x) sG0[(16 * (x >> 2) + 4 * kq + (x & 3)) * L::LDF + 16 * wave + l16] = dG[x];
     }
     settle16(dq[u]), settle16(dk[u]), settle16(dG);  // one set at a time
   }
@@ -680,12 +590,11 @@ __global__ __launch_bounds__(256, 2) void kda_bwd_chunk_kernel(KdaBwdParams p) {
     }
   }
   // ---- dq, dk out over the K and Q tiles, by rows ----
-  const int late = fresh(tid & 63);
 #pragma unroll
   for (int u = 0; u < NS; ++u)
 #pragma unroll
     for (int x = 0; x < 16; ++x) {
-      const int o = RowT::at(16 * (x >> 2) + 4 * (late >> 4) + (x & 3), 64 * u + 16 * wave + (late & 15));
+      const int o = RowT::at(16 * (x >> 2) + 4 * kq + (x & 3), 64 * u + 16 * wave + l16);
       sK[o] = (bf16_t)dk[u][x];
       sQ[o] = (bf16_t)dq[u][x];
     }

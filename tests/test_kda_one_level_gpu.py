@@ -1,6 +1,6 @@
 """bf16 per-channel gates whose chunk's whole decay fits one factor a token (LNX_KDA_NEAR, csrc/chunk_common.h: 80 in units of log 2, per set of 64
-channels in kda_prepare and per sixteen channels in kda_bwd_chunk) take their pairs in one level, others in a hierarchy of levels: both, the
-limit between them and calls that mix them, against the fp64 oracle."""
+channels) take their pairs in one level in kda_prepare, others in a hierarchy of levels: both, the limit between them and calls that mix them, against the
+fp64 oracle."""
 import numpy as np
 import pytest
 import torch
