@@ -1534,10 +1534,15 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   //   dk = 128   8 .. 128: 57.5 -> 45 / 58.5 -> 49    192: 59.6 -> 46.3 / 87 -> 72    224: 71 -> 53.8 / 89.8 -> 87.5    240: 71.2 -> 59.6 / 91.3 -> 102    256: 74 -> 73 .. 79 / 93 -> 108
   //   dk = 64    8 .. 128: 64 -> 36 / 66 -> 38.5      192: 67.5 -> 40.2 / 90.8 -> 64.3    224: 70.8 -> 55.3 / 91.3 -> 78.9    256: 72.2 -> 68 / 95 -> 88.5
   // On a full chip the tiles come at the rate of HBM, and at dk = 128 its one chunk in flight is too little.  The line is that of the form that
-  // saves the states: forward only, 225 to 240 workgroups would still gain at dk = 128.
+  // saves the states: forward only, 225 to 240 workgroups would still gain at dk = 128.  And only while what the call moves stays in the 256 MB
+  // cache: from HBM its one chunk in flight is too little for fewer slabs, too.  dk = dv = 128, chunk_scan -> with it, states saved, by chunks of
+  // all rows: 1024 (64 slabs) 60 -> 58, (32) 108 -> 93; 1152 52 -> 53; 1536 99 -> 110; 3072 158 -> 197; 6144 293 -> 371; forward only 1792 58 -> 50,
+  // 2048 104 -> 109 (64 slabs), 200 -> 189 (32); 3072 116 -> 146.  One line for both, so that a pass gives the same bits with states saved and without.
+  // At dk = 64 it is the faster one at any length (6144 chunks 316 -> 262).
   if constexpr (sizeof(T) == 2 && DK <= 128) {
     const int64_t wide = (int64_t)nstate * p.geom.H * (p.dv / 64);
-    if (p.slab ? p.slab == 32 : wide <= (DK == 128 ? 112 : 128)) return lnx_kda_scan_fwd(direct_params(p, GATE), DK, nstate, st);
+    const bool cached = DK == 64 || slots * (p.dv + 128) / 256 <= 2100;
+    if (p.slab ? p.slab == 32 : cached && wide <= (DK == 128 ? 112 : 128)) return lnx_kda_scan_fwd(direct_params(p, GATE), DK, nstate, st);
   }
   // 32-column slabs when 64-column ones would occupy at most half of the chip (256 CUs); always for 4-byte inputs
   // with dk = 256, whose tiles leave no room in LDS for a wider slab
