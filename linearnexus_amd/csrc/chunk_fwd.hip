@@ -94,8 +94,8 @@ template <typename T, int DK> struct Prep2Cfg {
 // chunk_direct.hip read; V is not touched.
 // Bound by its 41 KB a chunk (d128) once the chip is full, by the chain of the inverse where it is not.  The pair products are formed
 // transposed, so that rows of A and P leave the fragments as vectors (25 LDS writes of 2 and 4 bytes a lane before), the wave whose tile lies
-// above the diagonal forms nothing, and the inverse takes a third of the instructions it took (tri_inverse_64): B8 H16 T4096 d128 88 -> 78 us
-// (71 with neither inverse nor decays), one prompt of 65536 tokens and 4 heads 46 -> 41, dk = 256 71.5 -> 68.
+// above the diagonal forms nothing, and the inverse's scratch takes P's place: B8 H16 T4096 d128 88 -> 78 us (71 with neither inverse nor decays; with
+// tri_inverse_64's third of the instructions the same 78, but other last bits), one prompt of 65536 tokens and 4 heads 46 -> 43, dk = 256 71.5 -> 68.
 template <typename T, int DK, int GATE, bool LITE = false>
 __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdParams p) {
   typedef Prep2Cfg<T, DK> L;
@@ -249,13 +249,14 @@ __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdPa
   } else {
     unstage_tile<T, 64, 64>(ws_ptr<T>(p, p.off.P) + slot * 64 * 64, 64, sPt, LDC, 64, tid);
   }
-  tri_inverse_64<LITE>(sA, tid, (int)(slot >> 3) & 3);  // the solving wave differs between the workgroups of a CU
+  if constexpr (LITE) tri_inverse_64_ordered(sA, reinterpret_cast<float*>(sPt), tid);  // P has been read before the scratch's first use
+  else tri_inverse_64(sA, tid, (int)(slot >> 3) & 3);  // the solving wave differs between the workgroups of a CU
   if constexpr (LITE) {
     T* Tm = ws_ptr<T>(p, p.off.Tm) + slot * 64 * 64;
     typedef unsigned uint2_ __attribute__((ext_vector_type(2)));
     typedef unsigned uint4_ __attribute__((ext_vector_type(4)));
     auto put = [&](int idx, int r, int c) {
-      const float* src = r >= 32 && c < 4 ? sA + (r - 32) * LNX_LDA + 32 + 8 * c : sA + r * LNX_LDA + 8 * c;
+      const float* src = sA + r * LNX_LDA + 8 * c;
       const uint2_ lo = __builtin_bit_cast(uint2_, pack_bf16x4(load4(src))), hi = __builtin_bit_cast(uint2_, pack_bf16x4(load4(src + 4)));
       *reinterpret_cast<uint4_*>(Tm + 8 * idx) = uint4_{lo[0], lo[1], hi[0], hi[1]};
     };

@@ -571,6 +571,26 @@ __device__ __forceinline__ void rows_reduce_add(float (&v)[16 * MT], int row0, i
   if (MT == 2 || (lane & 1) == 0) atomicAdd(&rows[row0 + 32 * i + frag_row(e, lane)], total);
 }
 
+// ---------------------------------------------------------------------------------------
+// 16x16 fp32 products on v_mfma_f32_16x16x4_f32, operands row-major in LDS
+//   returns C[i][j] = sum_k A[i][k] * B[k][j];  fragment: c[e] is row 4*(lane>>4)+e, col lane&15
+// ---------------------------------------------------------------------------------------
+__device__ __forceinline__ floatx4 mm16_f32(const float* A, int lda, const float* B, int ldb, int K, int lane) {
+  floatx4 c = {0.f, 0.f, 0.f, 0.f};
+  const int i = lane & 15, kq = lane >> 4;
+  for (int k0 = 0; k0 < K; k0 += 4) {
+    const float a = A[i * lda + k0 + kq];
+    const float b = B[(k0 + kq) * ldb + i];
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  return c;
+}
+
+__device__ __forceinline__ void mm16_store(float* dst, int ld, floatx4 c, int lane, float sign) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) dst[(4 * (lane >> 4) + e) * ld + (lane & 15)] = sign * c[e];
+}
+
 #define LNX_LDA 68  // leading dimension of the fp32 64x64 matrices in LDS
 
 // In-LDS inverse of the unit lower-triangular matrix I + A: `M` holds A (strictly lower, zeros on and above the diagonal of the 16x16 diagonal
@@ -579,12 +599,11 @@ __device__ __forceinline__ void rows_reduce_add(float (&v)[16 * MT], int row0, i
 //   [[L0, 0], [B, L1]]^-1 = [[L0^-1, 0], [-L1^-1 B L0^-1, L1^-1]]
 // on v_mfma_f32_16x16x4_f32: a product's result fragment (rows 4 g + r, column l16) is the right operand of the next as it is, with the
 // contraction index of step r being 4 g + r in both (a left operand is then one 16-byte read), so a merge needs no scratch and no barrier of its
-// own.  ABOVE: the lower left 32x32 block of Tm stays in the place above the diagonal (rows 0 .., columns 32 ..), which spares the barrier
-// between the last reads of that block of A and its writes.
+// own.
 // A chunk's inverse is a serial chain that other workgroups of the CU have to cover: with every wave solving a block and the merges' products
 // through LDS it took seven barriers and 730 instructions of forward substitution instead of 180 (B4 H16 T8192 d128 kda_prepare 374 -> 361 us,
 // RWKV-7's chunk kernels 994 -> 975 of 2095).
-template <bool ABOVE = false> __device__ __forceinline__ void tri_inverse_64(float* M, int tid, int solver = 0) {
+__device__ __forceinline__ void tri_inverse_64(float* M, int tid, int solver = 0) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   if (wave == solver) {
     float* D = M + 16 * g * (LNX_LDA + 1);
@@ -640,7 +659,43 @@ template <bool ABOVE = false> __device__ __forceinline__ void tri_inverse_64(flo
         if (k >= bj) add(x, rows(32 + 16 * r, 16 * k), cols(16 * k, 16 * bj));
       add(y, rows(32 + 16 * bi, 32 + 16 * r), x);
     }
-  if (!ABOVE) lds_barrier();  // the block of A has been read
-  put(y, ABOVE ? 16 * bi : 32 + 16 * bi, (ABOVE ? 32 : 0) + 16 * bj);
+  lds_barrier();  // the block of A has been read
+  put(y, 32 + 16 * bi, 16 * bj);
   lds_barrier();
 }
+
+// The same with every sum in the order of its index: Tm of the bf16 calls without a per-channel gate.  A sequence whose keys are longer than one and
+// that has no gate grows until it overflows, and where it does hangs on Tm's last bits, so those stay what they are.  In place; A's upper triangle
+// within the 32x32 diagonal blocks must hold zeros, `sX` is a [32][36] scratch that is first written behind the first barrier.  Four waves solve a
+// diagonal block each (16 lanes a block), the merges' products go through the scratch.
+__device__ __forceinline__ void tri_inverse_64_ordered(float* M, float* sX, int tid) {
+  const int wave = tid >> 6, lane = tid & 63;
+  if (lane < 16) {
+    const int r0 = 16 * wave, c = lane;
+    float d[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float s = (i == c) ? 1.f : 0.f;
+#pragma unroll
+      for (int m = 0; m < i; ++m) s -= M[(r0 + i) * LNX_LDA + r0 + m] * d[m];
+      d[i] = s;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) M[(r0 + i) * LNX_LDA + r0 + c] = d[i];
+  }
+  lds_barrier();
+  // blocks (1,0) and (3,2) of the 16x16 grid, one per wave 0/1
+  float* sXw = sX + (wave & 1) * 16 * 36;
+  const int b = 32 * (wave & 1);
+  if (wave < 2) mm16_store(sXw, 36, mm16_f32(M + (b + 16) * LNX_LDA + b, LNX_LDA, M + b * LNX_LDA + b, LNX_LDA, 16, lane), lane, 1.f);
+  lds_barrier();
+  if (wave < 2) mm16_store(M + (b + 16) * LNX_LDA + b, LNX_LDA, mm16_f32(M + (b + 16) * LNX_LDA + b + 16, LNX_LDA, sXw, 36, 16, lane), lane, -1.f);
+  lds_barrier();
+  // the 32x32 lower-left block, one 16x16 output per wave
+  const int bi = 16 * (wave >> 1), bj = 16 * (wave & 1);
+  mm16_store(sX + bi * 36 + bj, 36, mm16_f32(M + (32 + bi) * LNX_LDA, LNX_LDA, M + bj, LNX_LDA, 32, lane), lane, 1.f);
+  lds_barrier();
+  mm16_store(M + (32 + bi) * LNX_LDA + bj, LNX_LDA, mm16_f32(M + (32 + bi) * LNX_LDA + 32, LNX_LDA, sX + bj, 36, 32, lane), lane, -1.f);
+  lds_barrier();
+}
+
