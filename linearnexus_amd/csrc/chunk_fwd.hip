@@ -249,8 +249,7 @@ __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdPa
   } else {
     unstage_tile<T, 64, 64>(ws_ptr<T>(p, p.off.P) + slot * 64 * 64, 64, sPt, LDC, 64, tid);
   }
-  if constexpr (LITE) tri_inverse_64_ordered(sA, reinterpret_cast<float*>(sPt), tid);  // P has been read before the scratch's first use
-  else tri_inverse_64(sA, tid, (int)(slot >> 3) & 3);  // the solving wave differs between the workgroups of a CU
+  tri_inverse_64_ordered(sA, reinterpret_cast<float*>(sPt), tid);  // P has been read before the scratch's first use
   if constexpr (LITE) {
     T* Tm = ws_ptr<T>(p, p.off.Tm) + slot * 64 * 64;
     typedef unsigned uint2_ __attribute__((ext_vector_type(2)));

@@ -664,7 +664,7 @@ __device__ __forceinline__ void tri_inverse_64(float* M, int tid, int solver = 0
   lds_barrier();
 }
 
-// The same with every sum in the order of its index: Tm of the bf16 calls without a per-channel gate.  A sequence whose keys are longer than one and
+// The same with every sum in the order of its index: Tm of the calls without a per-channel gate.  A sequence whose keys are longer than one and
 // that has no gate grows until it overflows, and where it does hangs on Tm's last bits, so those stay what they are.  In place; A's upper triangle
 // within the 32x32 diagonal blocks must hold zeros, `sX` is a [32][36] scratch that is first written behind the first barrier.  Four waves solve a
 // diagonal block each (16 lanes a block), the merges' products go through the scratch.
