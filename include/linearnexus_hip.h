@@ -325,7 +325,7 @@ int lnx_dplr_recurrent_bwd(const lnx_dplr_bwd_args* a, void* hip_stream);
  * lnx_dplr_recurrent_fwd with o_dtype == dtype and 16-byte aligned tensors; the forward call leaves what the backward call
  * needs in `kept` (NULL: no backward pass will follow).  lnx_dplr_chunk_bytes gives the bytes of `kept` (LNX_DPLR_KEPT, both
  * calls) and of the scratch areas (forward with kept, forward without, backward), which hold nothing between calls and are
- * bounded (about 1 GiB) however long the sequence is.  `kept` is 58 KB per chunk of a row; the token kernels keep nothing between
+ * bounded (about 1 GiB) however long the sequence is.  `kept` is 48 KB per chunk of a row; the token kernels keep nothing between
  * the passes.  The token gradients dq, dk, dv, da, db have args->dtype; dgk (read back within the call) and d_initial_state
  * (may be NULL) are fp32; d_final_state may be NULL (zero).  Gates may be anything that the token kernels take, down to -inf.
  * No atomics: the result is the same from run to run.

@@ -41,7 +41,6 @@ constexpr int C = 64, D = 64;       // tokens of a chunk, channels of a head
 constexpr int LD = LNX_LDA;         // leading dimension of the fp32 tiles in LDS: 68 floats, rows 4 banks apart
 constexpr int TS = C * LD;          // floats of a tile in LDS
 constexpr int TG = C * D;           // floats of a tile in the workspace
-constexpr int TRI = 10 * 256;       // floats of a lower-triangular one: its ten blocks, row by row
 constexpr int RANGE = 60;           // products of decays of a block's first tokens lie within 2^+-RANGE, or the block is DIRECT
 
 // A tile in the workspace is sixteen blocks of 16 x 16, block row by block row, and a block lies as a wave holds it, four elements of a row
@@ -59,7 +58,6 @@ struct ChunkParams {
   void *dq, *dk, *dv, *da, *db;
   float* dgk;
   float *M, *X, *hT;         // kept for the backward pass: [rows][KN] tiles, hT [rows][KN + 1] (states transposed: [dv][dk])
-  float* Tm;                 // with a backward pass: [rows][KN], lower-triangular
   float *s1, *s2, *s3, *s4;  // of a window of chunks, [rows][nw] tiles.  forward: N^T, Y; backward: D^T, R^T, u, dU
   int T, N, n0, nw;          // tokens, chunks of a row, the window [n0, n0 + nw)
   int KN, k0;                // the kept tensors hold chunks [k0, k0 + KN) of every row: all, or without a backward pass the window
@@ -517,7 +515,6 @@ template <bool BY_T, bool STRICT> __device__ __forceinline__ void mask(floatx4& 
     m[r] = (STRICT ? s >= t : s > t) ? 0.f : m[r];
   }
 }
-__device__ __forceinline__ int tri_block(int row, int col) { return (row * (row + 1) / 2 + col) * 256 + 4 * (threadIdx.x & 63); }
 // The wave's rows of a lower-triangular matrix: what lies before block j, the block itself, zeros
 template <typename F> __device__ __forceinline__ void put_tri(float* tile, const Lane& w, const floatx4 (&x)[3], floatx4 d, F&& value) {
 #pragma unroll
@@ -630,7 +627,6 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
     upto(w.j, [&](auto sb_) {
       constexpr int sb = decltype(sb_)::value;
       const floatx4 tf = frag<true>(tx, w.t, 16 * sb + g4);
-      if (p.Tm) store4(p.Tm + s.kept * TRI + tri_block(w.j, sb), tf);
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
         mfma4(W[cb], tf, frag<false>(ta, 16 * cb + l16, 16 * sb + g4));
@@ -827,9 +823,8 @@ __global__ __launch_bounds__(256) void dplr_r_kernel(ChunkParams p) {
 }
 
 // ---- backward: u, dU and dv of a chunk -----------------------------------------------------------------------
-// The inverse comes from the forward pass, 10 KB per chunk (B8 H16 T4096: 443 -> 416 us, with fp32 tensors
-// 523 -> 516); the pair matrices are formed again: keeping them, too, would
-// add 60 KB to the 128 that this kernel and dplr_prepare move, and their factors are needed here in any case.
+// The pair matrices and the inverse are formed again: keeping the pairs would move 128 KB per chunk through memory, and the inverse alone (10 KB of
+// 48 more to hold between the passes) gave 1.4 % of forward and backward, 0.4 % with fp32 tensors.
 template <typename T>
 __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   extern __shared__ __align__(16) char smem[];
@@ -847,14 +842,11 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   h0.load_tile(p.hT + s.st * TG, w.j);
   dC.load_tile(p.s1 + s.win * TG, w.j);
   floatx4 fa[4], fb[4], fk[4];  // the lane's row: a P of the token before, b S, k S
-  floatx4 akT[3];               // Aak by t, with earlier blocks
+  floatx4 ab[3], akT[3];        // Aab, Aak by t, with earlier blocks
   floatx4 ak[3], qb[3], qk[3];  // Aak, Pqb, Pqk by s, with later blocks (of block i + 1)
-  floatx4 akTd = zero4(), akd = zero4(), qbd = zero4(), qkd = zero4();  // the lane's own block
+  floatx4 abd = zero4(), akTd = zero4(), akd = zero4(), qbd = zero4(), qkd = zero4();  // the lane's own block
 #pragma unroll
-  for (int i = 0; i < 3; ++i) akT[i] = ak[i] = qb[i] = qk[i] = zero4();
-  floatx4 tm[4];  // the lane's row of Tm
-  clear(tm);
-  upto(w.j, [&](auto b_) { tm[decltype(b_)::value] = load4(p.Tm + s.kept * TRI + tri_block(w.j, decltype(b_)::value)); });
+  for (int i = 0; i < 3; ++i) ab[i] = akT[i] = ak[i] = qb[i] = qk[i] = zero4();
   {
     const Gates gates(x.gk);
     const Decay e(gates, p, s, w);
@@ -869,27 +861,28 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
         const floatx4 r = rcp4(e.p[cb]), b = x.b[cb] * r, k = x.k[cb] * r;
-        mfma_block<4>({&akTd, &akd, &qbd, &qkd}, [&](int i) { return i == 0 ? k : i == 1 ? fa[cb] : fq[cb]; }, [&](int i) { return i == 0 ? fa[cb] : i == 2 ? b : k; });
+        mfma_block<5>({&abd, &akTd, &akd, &qbd, &qkd}, [&](int i) { return i == 0 ? b : i == 1 ? k : i == 2 ? fa[cb] : fq[cb]; },
+                      [&](int i) { return i < 2 ? fa[cb] : i == 3 ? b : k; });
       }
-      mask<true, true>(akTd, w), mask<false, true>(akd, w), mask<false, false>(qbd, w), mask<false, false>(qkd, w);
+      mask<true, true>(abd, w), mask<true, true>(akTd, w), mask<false, true>(akd, w), mask<false, false>(qbd, w), mask<false, false>(qkd, w);
     } else {
       floatx4 decays[4];
       token_decays(p, s, w, decays);
       put_cols(tx, w, decays);
       __builtin_amdgcn_wave_barrier();
       const Pairs byt = direct_pairs<T, true>(p, s, w, tx), bys = direct_pairs<T, false>(p, s, w, tx);
-      akTd = byt.ak, akd = bys.ak, qbd = bys.qb, qkd = bys.qk;
+      abd = byt.ab, akTd = byt.ak, akd = bys.ak, qbd = bys.qb, qkd = bys.qk;
       __builtin_amdgcn_wave_barrier();
     }
-    put_cols(ta, w, fa), put_cols(tk, w, fk), put_cols(tx, w, fq);
+    put_cols(ta, w, fa), put_cols(tb, w, fb), put_cols(tk, w, fk), put_cols(tx, w, fq);
   }
   lds_barrier();
   before(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
-      const floatx4 rk = frag<true>(tk, 16 * b + l16, 16 * kb + g4), ra = fa[kb] * L.from<b>(w.j, 16 * kb + g4);
-      mfma_block<1>({&akT[b]}, [&](int) { return rk; }, [&](int) { return ra; });
+      const floatx4 rb = frag<true>(tb, 16 * b + l16, 16 * kb + g4), rk = frag<true>(tk, 16 * b + l16, 16 * kb + g4), ra = fa[kb] * L.from<b>(w.j, 16 * kb + g4);
+      mfma_block<2>({&ab[b], &akT[b]}, [&](int i) { return i ? rk : rb; }, [&](int) { return ra; });
     }
   });
   after(w.j, [&](auto b_) {
@@ -952,16 +945,18 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
   }
   lds_barrier();
   float *Tm = tx, *tz = ta, *ty = tk, *tdu = tb;
-  put_cols(Tm, w, tm);
+  put_tri(Tm, w, ab, abd, [](floatx4 x_) { return -x_; });
   put_rows(tz, w, z);
   put_rows(ty, w, y);
   lds_barrier();
+  tri_inverse_64(Tm, threadIdx.x);
   floatx4 u[4], du[4];  // rows n, columns t
   clear(u), clear(du);
   upto(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
+    const floatx4 tf = frag<true>(Tm, w.t, 16 * b + g4);
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) mfma4(u[nb], frag<true>(tz, 16 * nb + l16, 16 * b + g4), tm[b]);
+    for (int nb = 0; nb < 4; ++nb) mfma4(u[nb], frag<true>(tz, 16 * nb + l16, 16 * b + g4), tf);
   });
   downto(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
@@ -1361,13 +1356,12 @@ ChunkParams params(const lnx_dplr_args* a) {
   p.T = a->T, p.N = (a->T + C - 1) / C, p.scale = a->scale;
   return p;
 }
-void set_kept(ChunkParams& p, float* kept, int64_t rows, int k0, int KN, bool backward) {
+void set_kept(ChunkParams& p, float* kept, int64_t rows, int k0, int KN) {
   const int64_t n = rows * KN * TG;
   p.M = kept, p.X = p.M + n, p.hT = p.X + n;
-  p.Tm = backward ? p.hT + n + rows * TG : nullptr;
   p.k0 = k0, p.KN = KN;
 }
-constexpr int64_t kept_tiles(int64_t n) { return 3 * n + 1; }  // of a row that keeps n chunks, without Tm
+constexpr int64_t kept_tiles(int64_t n) { return 3 * n + 1; }  // of a row that keeps n chunks
 
 template <typename K> int lds_limit(K* k) { return lnx_lds_limit(reinterpret_cast<const void*>(k), LDS_BYTES); }
 
@@ -1379,8 +1373,8 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
   p.s1 = scratch, p.s2 = scratch + rows * W * TG;
   for (int n0 = 0; n0 < p.N; n0 += W) {
     p.n0 = n0, p.nw = p.N - n0 < W ? p.N - n0 : W;
-    if (kept) set_kept(p, kept, rows, 0, p.N, true);
-    else set_kept(p, scratch + 2 * rows * W * TG, rows, n0, p.nw, false);
+    if (kept) set_kept(p, kept, rows, 0, p.N);
+    else set_kept(p, scratch + 2 * rows * W * TG, rows, n0, p.nw);
     const unsigned grid = (unsigned)(rows * p.nw);
     lnx_profile_mark("dplr_prepare", st);
     hipLaunchKernelGGL(dplr_prepare_kernel<T>, dim3(grid), dim3(256), LDS_BYTES, st, p);
@@ -1393,11 +1387,11 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
   return LNX_OK;
 }
 
-// Same shape: dplr_r 54, dplr_chunk_scan_bwd 89, dplr_u 416, dplr_grad 709 (two workgroups per CU leave 256 registers, and what a
+// Same shape: dplr_r 54, dplr_chunk_scan_bwd 89, dplr_u 443, dplr_grad 709 (two workgroups per CU leave 256 registers, and what a
 // token needs between the pair sums and the last products is more: rows stay as they were read, and three are loaded twice)
 template <typename T> int backward(const lnx_dplr_chunk_grads* g, const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
-  set_kept(p, kept, rows, 0, p.N, true);
+  set_kept(p, kept, rows, 0, p.N);
   if (int rc = lds_limit(dplr_u_kernel<T>)) return rc;
   if (int rc = lds_limit(dplr_grad_kernel<T>)) return rc;
   const int W = window(rows, p.N, 4);
@@ -1441,7 +1435,7 @@ extern "C" uint64_t lnx_dplr_chunk_bytes(int32_t B, int32_t H, int32_t T, int32_
   const int64_t rows = (int64_t)B * H;
   const int N = (T + C - 1) / C;
   switch (what) {
-    case LNX_DPLR_KEPT: return (uint64_t)(tiles(rows, kept_tiles(N)) + rows * N * TRI * (int64_t)sizeof(float));
+    case LNX_DPLR_KEPT: return (uint64_t)tiles(rows, kept_tiles(N));
     case LNX_DPLR_ONLY_SCRATCH: return (uint64_t)tiles(rows, 2 * (int64_t)window(rows, N, 5) + kept_tiles(window(rows, N, 5)));
     case LNX_DPLR_FWD_SCRATCH: return (uint64_t)tiles(rows, 2 * (int64_t)window(rows, N, 2));
     case LNX_DPLR_BWD_SCRATCH: return (uint64_t)tiles(rows, 4 * (int64_t)window(rows, N, 4) + 1);

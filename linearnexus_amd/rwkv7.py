@@ -7,7 +7,7 @@ output in ``q.dtype``, fp32 state).  Heads of 64 x 64 -- RWKV-7's own -- with at
 tokens on the fp32 matrix cores (csrc/dplr_chunk.hip; the reference has no chunked form of this recurrence), anything else
 token by token (csrc/dplr.hip).  Both take any gate: a large negative one, down to -inf, ends a document inside a row.
 Both ops are differentiable with respect to q, k, v, a, b, gk and the state, as the reference's are under jax.grad (its
-RWKV-7 block trains through the scan).  Between the two passes the chunked scan keeps 58 KB per chunk of a (batch, head)
+RWKV-7 block trains through the scan).  Between the two passes the chunked scan keeps 48 KB per chunk of a (batch, head)
 row, as much again as a bf16 call's inputs; the token kernels keep nothing and recompute the states from checkpoints.
 Additive: ``dplr_delta_rule_step(..., inplace=True)`` updates the state buffer in place (not differentiable).  There
 is no other code path: the ops raise if the library is missing.
