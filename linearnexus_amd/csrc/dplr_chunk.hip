@@ -238,11 +238,15 @@ template <typename F> __device__ __forceinline__ void put_row(float* tile, const
 // h's error 0.76e-7 of its 2-norm instead of 0.53; four fp32 products 0.69; with ten times RWKV-7's gates 0.64, 0.49, 0.40).  B8 H16 T4096: dplr_prepare 486 -> 437, dplr_u 486 -> 443 us,
 // and with dPqk in dplr_grad 733 -> 724.  Where neither operand is given, six products of parts cost what they save: an operand takes 22
 // instructions to split, dplr_grad's pairs so 733 us, dAak alone 750.
-template <typename T> struct Parts {
+//
+// Whatever an infinite operand reaches is NaN by parts: inf - inf where it is the one split, inf times the empty half of `top` where it is the
+// given one.  A workgroup that finds a NaN among its sums begins again with FULL products, fp32 ones, which leave infinite what the fp32
+// kernels do (B8 H16 T4096 forward and backward 1895 -> 1905 us, of that dplr_prepare 434 -> 443).
+template <typename T, bool FULL> struct Parts {
   floatx4 x;
   __device__ __forceinline__ explicit Parts(floatx4 y) : x(y) {}
 };
-template <> struct Parts<bf16_t> {
+template <> struct Parts<bf16_t, false> {
   typedef unsigned uint4_ __attribute__((ext_vector_type(4)));
   uint4_ top, rest;
   __device__ __forceinline__ explicit Parts(floatx4 x) {
@@ -253,17 +257,33 @@ template <> struct Parts<bf16_t> {
   static __device__ __forceinline__ floatx4 high(floatx4 x) { return __builtin_bit_cast(floatx4, __builtin_bit_cast(uint4_, x) & 0xffff0000u); }
   static __device__ __forceinline__ unsigned pack(float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302); }
 };
-__device__ __forceinline__ void mfma_parts(floatx4& c, const Parts<float>& a, const Raw4<float>& b) { mfma4(c, a.x, b.x); }
-__device__ __forceinline__ void mfma_parts(floatx4& c, const Raw4<float>& a, const Parts<float>& b) { mfma4(c, a.x, b.x); }
-__device__ __forceinline__ void mfma_parts(floatx4& c, const Parts<bf16_t>& a, const Raw4<bf16_t>& b) {
+template <typename T> __device__ __forceinline__ void mfma_parts(floatx4& c, const Parts<T, true>& a, const Raw4<T>& b) { mfma4(c, a.x, b.get()); }
+template <typename T> __device__ __forceinline__ void mfma_parts(floatx4& c, const Raw4<T>& a, const Parts<T, true>& b) { mfma4(c, a.get(), b.x); }
+__device__ __forceinline__ void mfma_parts(floatx4& c, const Parts<bf16_t, false>& a, const Raw4<bf16_t>& b) {
   const bf16x8 x = Mma16::join(b.x, b.x);
   Mma16::mma(c, __builtin_bit_cast(bf16x8, a.rest), x);
   Mma16::mma(c, __builtin_bit_cast(bf16x8, a.top), x);
 }
-__device__ __forceinline__ void mfma_parts(floatx4& c, const Raw4<bf16_t>& a, const Parts<bf16_t>& b) {
+__device__ __forceinline__ void mfma_parts(floatx4& c, const Raw4<bf16_t>& a, const Parts<bf16_t, false>& b) {
   const bf16x8 x = Mma16::join(a.x, a.x);
   Mma16::mma(c, x, __builtin_bit_cast(bf16x8, b.rest));
   Mma16::mma(c, x, __builtin_bit_cast(bf16x8, b.top));
+}
+// NaN in any lane's sums
+template <typename... S> __device__ __forceinline__ bool any_nan(const S&... sums) {
+  bool x = false;
+  auto look = [&](const floatx4(&c)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x |= __builtin_isunordered(c[i][0], c[i][1]) | __builtin_isunordered(c[i][2], c[i][3]);
+  };
+  (look(sums), ...);
+  return __ballot(x) != 0;
+}
+// ... of the workgroup's waves: four words of LDS between the two, and a barrier
+__device__ __forceinline__ void put_flag(float* flags, bool x) { flags[threadIdx.x >> 6] = x ? 1.f : 0.f; }
+__device__ __forceinline__ bool any_flag(const float* flags) {
+  const floatx4 f = load4(flags);
+  return __builtin_amdgcn_readfirstlane(f[0] + f[1] + f[2] + f[3] != 0.f);
 }
 // Tiles of such a tensor in LDS, rows as given: bf16 rows 80 elements apart, which touch every bank once in both directions, and a wave's
 // sixteen where its rows of an fp32 tile begin (before a barrier they are the wave's alone)
@@ -526,10 +546,7 @@ template <typename F> __device__ __forceinline__ void put_tri(float* tile, const
 }
 
 // ---- forward: M, X, N^T, Y of a chunk ------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
-  extern __shared__ __align__(16) char smem[];
-  const Lds L(smem);
+template <typename T, bool FULL> __device__ __forceinline__ bool prepare_chunk(const ChunkParams& p, const Lds& L) {
   const Slot s = slot_of(p);
   const Lane w;
   const int l16 = w.l16, g = w.g, g4 = 4 * w.g;
@@ -593,13 +610,13 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
   clear(nt), clear(z), clear(y);
 #pragma unroll
   for (int sb = 0; sb < 4; ++sb) {
-    const Parts<T> kf(frag<false>(tk, 16 * w.j + l16, 16 * sb + g4) * end[sb]);
+    const Parts<T, FULL> kf(frag<false>(tk, 16 * w.j + l16, 16 * sb + g4) * end[sb]);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) mfma_parts(nt[nb], kf, given_col<T>(tx, 16 * nb, 16 * sb + g4, w));
   }
   before(w.j, [&](auto sb_) {
     constexpr int sb = decltype(sb_)::value;
-    const Parts<T> a(ak[sb]), q(qk[sb]);
+    const Parts<T, FULL> a(ak[sb]), q(qk[sb]);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       const Raw4<T> vf = given_col<T>(tx, 16 * nb, 16 * sb + g4, w);
@@ -608,7 +625,7 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
     }
   });
   {
-    const Parts<T> a(m.ak), q(m.qk);
+    const Parts<T, FULL> a(m.ak), q(m.qk);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       const Raw4<T> vf = given_col<T>(tx, 16 * nb, 16 * w.j + g4, w);
@@ -670,9 +687,22 @@ __global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
     const int at = block_at(w.j, cb);
     store4(p.M + s.kept * TG + at, r);
     store4(p.X + s.kept * TG + at, xx[cb] + xw[cb]);
-    store4(p.s2 + s.win * TG + at, y[cb] + yu[cb]);
-    store4(p.s1 + s.win * TG + block_at(cb, w.j), nt[cb] + ntu[cb]);
+    y[cb] += yu[cb], nt[cb] += ntu[cb];
+    store4(p.s2 + s.win * TG + at, y[cb]);
+    store4(p.s1 + s.win * TG + block_at(cb, w.j), nt[cb]);
   }
+  if constexpr (!FULL) {  // (what z had, N has in the whole column)
+    put_flag(L.sx, any_nan(nt, y));
+    lds_barrier();
+    return !any_flag(L.sx);
+  }
+  return true;
+}
+template <typename T>
+__global__ __launch_bounds__(256, 2) void dplr_prepare_kernel(ChunkParams p) {
+  extern __shared__ __align__(16) char smem[];
+  const Lds L(smem);
+  if (!prepare_chunk<T, sizeof(T) == 4>(p, L)) prepare_chunk<T, true>(p, L);
 }
 
 // ---- the sequential pass: h <- M h + N (forward), D <- M^T D + R (backward) ------------------------------------
@@ -811,13 +841,17 @@ __global__ __launch_bounds__(256) void dplr_r_kernel(ChunkParams p) {
   put_given(tO, w, d);
   lds_barrier();
   floatx4 acc[4];
-  clear(acc);
+  auto sums = [&](auto full) {
+    clear(acc);
 #pragma unroll
-  for (int kb = 3; kb >= 0; --kb) {  // the chunk's first tokens, whose share is the largest, last
-    const Parts<T> a(frag<false>(tX, w.t, 16 * kb + g4));
+    for (int kb = 3; kb >= 0; --kb) {  // the chunk's first tokens, whose share is the largest, last
+      const Parts<T, decltype(full)::value> a(frag<false>(tX, w.t, 16 * kb + g4));
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) mfma_parts(acc[nb], a, given_col<T>(tO, 16 * nb, 16 * kb + g4, w));
-  }
+      for (int nb = 0; nb < 4; ++nb) mfma_parts(acc[nb], a, given_col<T>(tO, 16 * nb, 16 * kb + g4, w));
+    }
+  };
+  sums(std::bool_constant<sizeof(T) == 4>{});
+  if (sizeof(T) == 2 && any_nan(acc)) sums(std::true_type{});
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb) store4(p.s2 + s.win * TG + block_at(nb, w.j), acc[nb]);
 }
@@ -825,10 +859,7 @@ __global__ __launch_bounds__(256) void dplr_r_kernel(ChunkParams p) {
 // ---- backward: u, dU and dv of a chunk -----------------------------------------------------------------------
 // The pair matrices and the inverse are formed again: keeping the pairs would move 128 KB per chunk through memory, and the inverse alone (10 KB of
 // 48 more to hold between the passes) gave 1.4 % of forward and backward, 0.4 % with fp32 tensors.
-template <typename T>
-__global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
-  extern __shared__ __align__(16) char smem[];
-  const Lds L(smem);
+template <typename T, bool FULL> __device__ __forceinline__ bool u_chunk(const ChunkParams& p, const Lds& L) {
   const Slot s = slot_of(p);
   const Lane w;
   const int l16 = w.l16, g4 = 4 * w.g;
@@ -919,13 +950,13 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
     }
   before(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
-    const Parts<T> a(akT[b]);
+    const Parts<T, FULL> a(akT[b]);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) mfma_parts(z[nb], a, given_col<T>(tv, 16 * nb, 16 * b + g4, w));
   });
   after(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
-    const Parts<T> pb(qb[b - 1]), pk(qk[b - 1]);
+    const Parts<T, FULL> pb(qb[b - 1]), pk(qk[b - 1]);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       const Raw4<T> of = given_col<T>(tO, 16 * nb, 16 * b + g4, w);
@@ -934,7 +965,7 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
     }
   });
   {
-    const Parts<T> a(akTd), pb(qbd), pk(qkd);
+    const Parts<T, FULL> a(akTd), pb(qbd), pk(qkd);
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       const Raw4<T> of = given_col<T>(tO, 16 * nb, 16 * w.j + g4, w);
@@ -943,7 +974,10 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
       mfma_parts(dv[nb], of, pk);
     }
   }
+  if constexpr (!FULL) put_flag(L.sx, any_nan(z, y, dv));
   lds_barrier();
+  if constexpr (!FULL)
+    if (any_flag(L.sx)) return false;
   float *Tm = tx, *tz = ta, *ty = tk, *tdu = tb;
   put_tri(Tm, w, ab, abd, [](floatx4 x_) { return -x_; });
   put_rows(tz, w, z);
@@ -984,6 +1018,13 @@ __global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) store_row4<T>(p.dv, (s.tok + w.t) * D + 16 * nb + g4, dv[nb] + dva[nb]);
   }
+  return true;
+}
+template <typename T>
+__global__ __launch_bounds__(256, 2) void dplr_u_kernel(ChunkParams p) {
+  extern __shared__ __align__(16) char smem[];
+  const Lds L(smem);
+  if (!u_chunk<T, sizeof(T) == 4>(p, L)) u_chunk<T, true>(p, L);
 }
 
 // ---- backward: dq, dk, da, db, dgk of a chunk ----------------------------------------------------------------
