@@ -948,6 +948,12 @@ template <typename T, bool FULL> __device__ __forceinline__ bool u_chunk(const C
       mfma4(y[nb], fb[kb], df);
       mfma4(dv[nb], df, fk[kb]);
     }
+  // The sums go on from fp32 to bf16 matrix instructions.  hipcc's wait states for a change of kind on one accumulator have been too few once
+  // (16x16x16 into 16x16x32, both bf16, lost elements), so whatever the schedule none of the first kind's results, of eight passes, is under way
+  // behind these 32 states.  Sums of their own for the two kinds cost 150 spills (no difference in time measured with the states).
+  if constexpr (sizeof(T) == 2 && !FULL)
+    asm volatile("s_nop 15\n\ts_nop 15"
+                 : "+v"(z[0]), "+v"(z[1]), "+v"(z[2]), "+v"(z[3]), "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]), "+v"(dv[0]), "+v"(dv[1]), "+v"(dv[2]), "+v"(dv[3]));
   before(w.j, [&](auto b_) {
     constexpr int b = decltype(b_)::value;
     const Parts<T, FULL> a(akT[b]);
