@@ -235,9 +235,9 @@ template <typename F> __device__ __forceinline__ void put_row(float* tile, const
 // v and dO in bf16 are exact in one part, and an fp32 operand is the sum of three (its top eight bits, the next eight, the last eight: all
 // differences are exact), so a block of 16 of the contraction is two bf16 products of 16 cycles, {last, next} {x, x} and {top, 0} {x, x},
 // instead of four fp32 ones of 32, and no operand is rounded.  The small parts come first, so that c meets the large sum once (the other way round
-// h's error 0.76e-7 of its 2-norm instead of 0.53; four fp32 products 0.69; with ten times RWKV-7's gates 0.64, 0.49, 0.40).  B8 H16 T4096: dplr_prepare 486 -> 437, dplr_u 486 -> 443 us,
-// and with dPqk in dplr_grad 733 -> 724.  Where neither operand is given, six products of parts cost what they save: an operand takes 22
+// h's error 0.76e-7 of its 2-norm instead of 0.53; four fp32 products 0.69).  B8 H16 T4096: dplr_prepare 486 -> 437, dplr_u 486 -> 443 us, and with dPqk in dplr_grad 733 -> 724.  Where neither operand is given, six products of parts cost what they save: an operand takes 22
 // instructions to split, dplr_grad's pairs so 733 us, dAak alone 750.
+// An operand below 2^-110 loses those of its bits that lie under the smallest bf16 number, 2^-133.
 //
 // Whatever an infinite operand reaches is NaN by parts: inf - inf where it is the one split, inf times the empty half of `top` where it is the
 // given one.  A workgroup that finds a NaN among its sums begins again with FULL products, fp32 ones, which leave infinite what the fp32
@@ -608,12 +608,24 @@ template <typename T, bool FULL> __device__ __forceinline__ bool prepare_chunk(c
   L.ends(w.t, end, chunk);
   floatx4 nt[4], z[4], y[4];  // N (rows i, columns n), Aak v (rows t, columns n), Y^T (rows n, columns t)
   clear(nt), clear(z), clear(y);
+  auto new_sums = [&](auto full) {
 #pragma unroll
-  for (int sb = 0; sb < 4; ++sb) {
-    const Parts<T, FULL> kf(frag<false>(tk, 16 * w.j + l16, 16 * sb + g4) * end[sb]);
+    for (int sb = 0; sb < 4; ++sb) {
+      const Parts<T, decltype(full)::value> kf(frag<false>(tk, 16 * w.j + l16, 16 * sb + g4) * end[sb]);
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) mfma_parts(nt[nb], kf, given_col<T>(tx, 16 * nb, 16 * sb + g4, w));
+      for (int nb = 0; nb < 4; ++nb) mfma_parts(nt[nb], kf, given_col<T>(tx, 16 * nb, 16 * sb + g4, w));
+    }
+  };
+  // Where a channel's decay over the last block is below 2^-24, N is the sum of a few tokens: the matrix instruction cuts a sum of bf16 products off
+  // where it rounds one of fp32 ones, and with so few terms no rounding of a longer sum outweighs that.  h's error, 1e-7 of its 2-norm, by parts and
+  // in fp32: RWKV-7's decays (2^-14 and above) 0.53 and 0.69, three times those 0.47 and 0.50, four 0.46 and 0.45, six 0.46 and 0.41, ten 0.48
+  // and 0.37.  Parts' sums apart, added at the end: 0.59 .. 0.54.
+  bool full = FULL;
+  if constexpr (!FULL) {
+    full = __ballot(end[2] < 0x1p-24f) != 0;
+    if (!full) new_sums(std::false_type{});
   }
+  if (full) new_sums(std::true_type{});
   before(w.j, [&](auto sb_) {
     constexpr int sb = decltype(sb_)::value;
     const Parts<T, FULL> a(ak[sb]), q(qk[sb]);
