@@ -413,6 +413,37 @@ template <bool LOG2> __device__ __forceinline__ void kda_pair_half(floatx4 (&a32
   }
 }
 
+// Anything among two tiles' rows that a factor of 2^+-40 could take out of its type's range, or the remainder that Kc carries beside it.  Mostly the
+// sizes of all groups of eight elements are within 2^-50 .. 2^60, which their sums of squares show in 24 instructions (B4 H16 T8192 d128 363 -> 368 us;
+// with the look at every element 10 more instead of 5).  Otherwise every element has to be zero or within 2^-64 .. 2^80; infinities and NaN lie beyond.
+template <int IT> __device__ __forceinline__ bool kda_odd_sizes(const bf16x8 (&a)[IT], const bf16x8 (&b)[IT]) {
+  typedef bf16_t bf16x2_ __attribute__((ext_vector_type(2)));
+  float most = 0.f, least = 1.f;
+  auto square = [&](bf16x8 x) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) s = __builtin_amdgcn_fdot2_f32_bf16(bf16x2_{x[i], x[i + 1]}, bf16x2_{x[i], x[i + 1]}, s, false);
+    return s;
+  };
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const float s = square(a[it]), t = square(b[it]);
+    most = fmaxf(most, fmaxf(s, t)), least = fminf(least, fminf(s, t));
+  }
+  const bool plain = most <= 0x1p120f && least >= 0x1p-100f;
+  if (__ballot(!plain) == 0) return false;
+  typedef unsigned short ushort8_ __attribute__((ext_vector_type(8)));
+  constexpr unsigned short LOW = (127 - 64) << 7, HIGH = (127 + 80) << 7;
+  ushort8_ high = (unsigned short)0, low = (unsigned short)0xffff;  // of the magnitudes' bits; of those less one, which leaves zero out
+  auto look = [&](bf16x8 x) {
+    const ushort8_ m = __builtin_bit_cast(ushort8_, x) & (unsigned short)0x7fff;
+    high = __builtin_elementwise_max(high, m), low = __builtin_elementwise_min(low, m - (unsigned short)1);
+  };
+#pragma unroll
+  for (int it = 0; it < IT; ++it) look(a[it]), look(b[it]);
+  return __builtin_reduce_max(high) >= HIGH || __builtin_reduce_min(low) < LOW - 1;
+}
+
 // The same sums where a chunk's whole decay fits a factor (kda_near): E_ij = exp(G_i - m) exp(m - G_j) with one m per channel, so that every pair is
 // of one level and the tiles Kr, Qr (rows times exp(G - m)) and Kc (times exp(m - G)) are plain operands.  Kc comes in two parts, rounded and
 // what the rounding left: at the levels, too, a pair of neighbours has one operand or both with a factor of 1, unrounded, and with both rounded
@@ -609,6 +640,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
     if (norm) scale_rows(rK, sNk), scale_rows(rQ, sNq);
     rK.store(sK, LDC, tid);
     rQ.store(sQ, LDC, tid);
+    bool odd = false;
+    if constexpr (LAST) odd = kda_odd_sizes(rK.x, rQ.x);
     store_gate(h);
     lds_barrier();
     if (h + 1 < NH) fetch_half(h + 1);
@@ -632,7 +665,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
 #pragma unroll
       for (int i = 0; i < 16; ++i) sG[(16 * seg + i) * LDF + c] = gs[i] + off;
       if (LAST) {
-        const bool all = __ballot(!(highest <= 0.f && gs[15] + off >= -LNX_KDA_NEAR)) == 0;  // (NaN shows in the sum)
+        const bool all = __ballot(odd || !(highest <= 0.f && gs[15] + off >= -LNX_KDA_NEAR)) == 0;  // (NaN shows in the sum)
         if (c == 0) sSeg[256 + seg] = all ? 1.f : 0.f;
       }
     }

@@ -90,3 +90,53 @@ def test_gates_above_zero_and_nan_keep_the_levels():
     gr2 = torch.autograd.grad(o2, leaves, torch.from_numpy(x["dO"]).to(DEV))
     assert torch.equal(o2[:, 0], o[:, 0]) and torch.isnan(o2[:, 1, 70:]).any()
     assert all(torch.equal(a[:, 0], b[:, 0]) for a, b in zip(gr, gr2))
+
+
+@pytest.mark.parametrize("dk", [64, 128])
+@pytest.mark.parametrize("size", [2.0 ** 100, 2.0 ** -100])
+def test_sizes_at_the_ends_of_the_range(size, dk):
+    """Rows near the ends of the range keep the levels, whose factors are none above one: o is linear in q, whatever the size of q."""
+    import linearnexus_amd as la
+    x = make_inputs(10, 1, 2, 128, dk, 64, gate="vector", with_state=True)
+    x["g"] = np.ascontiguousarray(_gates("below", 128, dk, np.random.default_rng(3)), np.float32)
+    t = {n: torch.from_numpy(a).to(DEV).to(torch.bfloat16 if n in "qkv" else torch.float32) for n, a in x.items()}
+    run = lambda q: la.kda_chunkwise(q, t["k"], t["v"], t["g"], t["beta"], None, t["S0"], 64, False)[0].double()
+    want, got = run(t["q"]), run(t["q"] * size) / size
+    assert (got - want).norm() < 2e-2 * want.norm()  # each within 1e-2 of the same values
+
+
+@pytest.mark.parametrize("dk", [64, 128])
+def test_one_key_beyond_a_factor(dk):
+    """A key of 2^100 in one channel of one late token of a chunk, queries of 2^-100 in that channel: their products are ordinary numbers."""
+    import linearnexus_amd as la
+    x = make_inputs(11, 1, 2, 128, dk, 64, gate="vector", with_state=True)
+    x["g"] = np.ascontiguousarray(_gates("below", 128, dk, np.random.default_rng(4)), np.float32)
+    x["k"][..., 7], x["S0"][..., 7, :] = 0.0, 0.0
+    x["k"][:, :, 60, 7] = 2.0 ** 100
+    x["q"][..., 7] *= 2.0 ** -100
+    for n in "qkv":
+        x[n] = to_bf16_grid(x[n])
+    x["beta"][:, :, 60] = 0.5
+    t = {n: torch.from_numpy(a).to(DEV).to(torch.bfloat16 if n in "qkv" else torch.float32) for n, a in x.items()}
+    o, _ = la.kda_chunkwise(t["q"], t["k"], t["v"], t["g"], t["beta"], None, t["S0"], 64, False)
+    d = {n: a.astype(np.float64) for n, a in x.items()}
+    ro, _ = rc.kda_recurrent(d["q"], d["k"], d["v"], d["g"], d["beta"], None, d["S0"], False)
+    assert max_rel(o.cpu().numpy(), ro) < 2e-2
+
+
+@pytest.mark.parametrize("t", [1, 37, 63])
+def test_an_infinite_query_is_infinite(t):
+    """Positive values all along the one channel that the infinite query reads: the sum is +inf, and only in that token's row."""
+    import linearnexus_amd as la
+    gen = torch.Generator(device=DEV).manual_seed(t)
+    T, D, c = 64, 64, 5
+    q, k = torch.randn(1, 1, T, D, device=DEV, generator=gen), torch.zeros(1, 1, T, D, device=DEV)
+    k[..., c] = 0.1 + 0.1 * torch.rand(1, 1, T, device=DEV, generator=gen)
+    q[0, 0, t] = 0.0
+    q[0, 0, t, c] = float("inf")
+    v = 1 + torch.rand(1, 1, T, D, device=DEV, generator=gen)
+    S0 = torch.zeros(1, 1, D, D, device=DEV)
+    S0[:, :, c] = 0.5
+    o, _ = la.kda_chunkwise(q.bfloat16(), k.bfloat16(), v.bfloat16(), torch.full((1, 1, T, D), -0.02, device=DEV), torch.full((1, 1, T), 0.1, device=DEV), None, S0, 64, False)
+    others = torch.arange(T, device=DEV) != t
+    assert torch.isfinite(o[:, :, others]).all() and (o[0, 0, t] == float("inf")).all()
