@@ -129,12 +129,12 @@ template <typename T, int DK> constexpr bool lnx_gate_last_only = sizeof(T) == 2
 template <typename T, int DK> __device__ __forceinline__ int64_t gate_last(int64_t slot) { return lnx_gate_last_only<T, DK> ? slot * DK : (slot * LNX_C + LNX_C - 1) * DK; }
 // A chunk whose gates are none above zero and whose whole decay is above 2^-LNX_KDA_NEAR in every channel (of a set of 64): with the middle of a
 // channel's decay as the reference, e^{G - mid} and e^{mid - G} lie within 2^+-40, far from the ends of a bf16's or fp32's range also in the
-// products of pairs that are masked afterwards (up to 2^80), and one such factor a token takes the place of one per level (where the rows' own sizes
-// leave room for it, kda_odd_sizes in chunk_fwd.hip).  A chunk of 64 tokens
-// forgets that much at 0.87 nats a token.  B4 H16 T8192 d128, kda_prepare in one level against the levels: 317 and 372 us, B2 T2048 51 and 59.
-// One level is as exact as the levels or better (o 3.8e-3 and 4.0e-3 off fp64): its scaled rows are held to more than bf16.  kda_bwd_chunk keeps
-// the levels: in one level it took 466 us instead of 484, and the gates' gradient was closer to fp64 (3.6e-3 and 4.6e-3), but by that much another
-// that its sums over all tokens moved by 1 to 2.4 %, more than the 1 % that results may move.
+// products of pairs that are masked afterwards (up to 2^80), and one such factor a token takes the place of one per level (where the rows' own
+// sizes leave room for it, kda_odd_sizes in chunk_fwd.hip).  A chunk of 64 tokens forgets that much at 0.87 nats a token.  B4 H16 T8192 d128,
+// kda_prepare in one level against the levels: 317 and 372 us, B2 T2048 51 and 59.  One level is as exact as the levels or better (o 3.8e-3 and
+// 4.0e-3 off fp64): its scaled rows are held to more than bf16.  kda_bwd_chunk keeps the levels: in one level it took 466 us instead of 484, and the
+// gates' gradient was closer to fp64 (3.6e-3 and 4.6e-3), but a training program's gradients of A_log and dt_bias, sums of it over all tokens in
+// which most cancels, came out 1 to 2.4 % of their norm from those that it had had.
 constexpr float LNX_KDA_NEAR = 80.f;
 inline bool lnx_chunk_kda(const lnx_scan_args* a) { return a->dtype == LNX_BF16 && a->dk <= 128 && a->gate == LNX_GATE_VECTOR; }
 

@@ -85,7 +85,7 @@ template <typename T, int DK> struct Prep2Cfg {
   static constexpr size_t r1 = sizeof(float) * 128;  // beta, G
   static constexpr size_t r2 = 2 * kTile * sizeof(T);
   static constexpr size_t bytes = r0 + r1 + r2;
-  // LITE: the slab tiles, then A, inverted in place | beta, G, row factors | P   (28.5 KB, five per CU)
+  // LITE: the slab tiles, then A, inverted in place | beta, G, row factors | P   (28 KB, five per CU)
   static constexpr size_t lite_tiles = cmax(mat, 2 * kTile * sizeof(T));
   static constexpr size_t lite_bytes = lite_tiles + sizeof(float) * 256 + kTile * sizeof(T);
 };
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(256, LITE ? 5 : 1) void chunk_prepare2_kernel(FwdPa
   } else {
     unstage_tile<T, 64, 64>(ws_ptr<T>(p, p.off.P) + slot * 64 * 64, 64, sPt, LDC, 64, tid);
   }
-  tri_inverse_64_ordered(sA, reinterpret_cast<float*>(sPt), tid);  // P has been read before the scratch's first use
+  tri_inverse_64_rows(sA, reinterpret_cast<float*>(sPt), tid);  // P has been read before the scratch's first use
   if constexpr (LITE) {
     T* Tm = ws_ptr<T>(p, p.off.Tm) + slot * 64 * 64;
     typedef unsigned uint2_ __attribute__((ext_vector_type(2)));
@@ -481,12 +481,12 @@ template <typename T, int DK> struct KdaPrepSmem {
   static constexpr int PAD = Mma<T>::PAD;
   static constexpr int LDC = LNX_C + PAD, LDF = 64 + 4;
   static constexpr int kTile = 64 * LDC;
-  // K half (later Tm), Q half (later Tm diag(beta)); gate half (later the staged slab); A (later the
-  // output staging); the P accumulator / inverse; inverse scratch; beta, and where the rows are normalised inside their factors
+  // K half (later Tm), Q half (later Tm diag(beta)); gate half (later the staged slab, or A); A, inverted in place (later the
+  // output staging), or beta K e^G; the P accumulator, before it the column operands of one level, which are longer by kCol floats; phase A's
+  // segment totals [4][64], flags and diagonal; beta, and where the rows are normalised inside their factors
   static constexpr bool NORM = sizeof(T) == 2 && DK <= 128;
-  static constexpr size_t bytes = sizeof(T) * 2 * kTile + sizeof(float) * (64 * LDF + 2 * 64 * LNX_LDA + 32 * 36 + (NORM ? 192 : 64));
-  static __device__ __forceinline__ float* seg(float* sX) { return sX + 32 * 36 - 384; }  // 384 floats of phase A
-  static_assert(sizeof(T) == 4 || sizeof(T) * 2 * kTile <= sizeof(float) * (64 * LNX_LDA + 32 * 36 - 384), "the column operands end before them");
+  static constexpr int kCol = NORM ? (int)(sizeof(T) * 2 * kTile / sizeof(float)) - 64 * LNX_LDA : 0, kA = NORM ? 384 : 256;
+  static constexpr size_t bytes = sizeof(T) * 2 * kTile + sizeof(float) * (64 * LDF + 2 * 64 * LNX_LDA + kCol + kA + (NORM ? 192 : 64));
 };
 
 // GRAW: the gate arrives as the block's raw projection and is activated here, g = -exp(A_log[h]) softplus(raw + bias)
@@ -503,10 +503,10 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
   float* sT = sA + 64 * LNX_LDA;
   T* sKb = reinterpret_cast<T*>(sA);  // LAST: beta K e^G [64][LDKB] from phase A to D
   constexpr int LDKB = DK + L::PAD;
-  T* sKc = reinterpret_cast<T*>(sT);  // LAST: K e^{mid - G} of the half, rounded, and behind it what the rounding left; reaches into sX
-  float* sX = sT + 64 * LNX_LDA;
-  float* sBeta = sX + 32 * 36;
-  float* sDiag = L::seg(sX) + 320;  // <q_t, k_t> over the halves whose pairs are of one level, from the rows themselves
+  T* sKc = reinterpret_cast<T*>(sT);  // LAST: K e^{mid - G} of the half, rounded, and behind it what the rounding left
+  float* sSeg = sT + 64 * LNX_LDA + L::kCol;  // segment totals [4][64]
+  float* sBeta = sSeg + L::kA;
+  float* sDiag = sSeg + 320;  // <q_t, k_t> over the halves whose pairs are of one level, from the rows themselves
   float* sNk = sBeta + 64;  // NORM: 1 / (|x| + eps) of the k and q rows
   float* sNq = sNk + 64;
 
@@ -657,7 +657,6 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
       }
 #pragma unroll
       for (int i = 1; i < 16; ++i) gs[i] += gs[i - 1];
-      float* sSeg = L::seg(sX);  // segment totals [4][64]
       sSeg[seg * 64 + c] = gs[15];
       lds_barrier();
       float off = 0.f;
@@ -672,7 +671,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 ? 2 : 1)) void kda_prepare_ker
     lds_barrier();
     bool near = false;  // this half's pairs are of one level
     if (LAST) {
-      const floatx4 f = load4(L::seg(sX) + 256);
+      const floatx4 f = load4(sSeg + 256);
       near = __builtin_amdgcn_readfirstlane(f[0] + f[1] + f[2] + f[3] == 4.f);
     }
     // G, K e^{G_last - G}, scale Q e^G of this half -> workspace.  LAST: of G only the last row, but beta K e^G for phase D into the tile that
@@ -1570,7 +1569,10 @@ int launch_fwd(const FwdParams& p, int nstate, hipStream_t st) {
   // saves the states: forward only, 225 to 240 workgroups would still gain at dk = 128.  And only while what the call moves stays in the 256 MB
   // cache: from HBM its one chunk in flight is too little for fewer slabs, too.  dk = dv = 128, chunk_scan -> with it, states saved, by chunks of
   // all rows: 1024 (64 slabs) 60 -> 58, (32) 108 -> 93; 1152 52 -> 53; 1536 99 -> 110; 3072 158 -> 197; 6144 293 -> 371; forward only 1792 58 -> 50,
-  // 2048 104 -> 109 (64 slabs), 200 -> 189 (32); 3072 116 -> 146.  One line for both, so that a pass gives the same bits with states saved and without.
+  // 2048 104 -> 109 (64 slabs), 200 -> 189 (32); 3072 116 -> 146.  At 16, 8, 4, 2 slabs: 2400 chunks, states saved 477 -> 553, 948 -> 1041, 1883 -> 2016,
+  // 3757 -> 3991, forward only 459 -> 472, 910 -> 914, 1820 -> 1736, 3615 -> 3257; 8192 chunks 1615 -> 1864 .. 12749 -> 13625 and 1547 -> 1656 .. 12335 -> 12649.
+  // One line for both, so that a pass gives the same bits with states saved and without, and it is that of forward only: with states saved
+  // between 1150 and 2100 chunks the choice gives up to 11 % of this scan, and forward only two slabs give 10 % up to some 3000 chunks.
   // At dk = 64 it is the faster one at any length (6144 chunks 316 -> 262).
   if constexpr (sizeof(T) == 2 && DK <= 128) {
     const int64_t wide = (int64_t)nstate * p.geom.H * (p.dv / 64);

@@ -351,11 +351,12 @@ __device__ __forceinline__ floatx4 product_from(floatx4 x) {  // row_shl
 }
 
 constexpr int LDS_TILES = 4;
-constexpr unsigned LDS_BYTES = (LDS_TILES * TS + 5 * 64 + 32 * 36) * sizeof(float);
+constexpr int SX = 15 * 64;  // dplr_grad's sums that cross waves; the flags of the others
+constexpr unsigned LDS_BYTES = (LDS_TILES * TS + 5 * 64 + SX) * sizeof(float);
 static_assert(LDS_BYTES <= 80 * 1024, "two workgroups per CU");
 struct Lds {
   float *base, *total, *one;  // total: [4][64], decays of the whole blocks; one: 64 ones
-  float* sx;                  // 32 x 36 floats
+  float* sx;                  // SX floats
   __device__ __forceinline__ Lds(char* smem) {
     base = reinterpret_cast<float*>(smem);
     total = base + LDS_TILES * TS, one = total + 256, sx = one + 64;

@@ -664,11 +664,14 @@ __device__ __forceinline__ void tri_inverse_64(float* M, int tid, int solver = 0
   lds_barrier();
 }
 
-// The same with every sum in the order of its index: Tm of the calls without a per-channel gate.  A sequence whose keys are longer than one and
-// that has no gate grows until it overflows, and where it does hangs on Tm's last bits, so those stay what they are.  In place; A's upper triangle
+// The same with the sums grouped another way: Tm of the calls without a per-channel gate.  Neither is the more exact one.  This one's bits are those
+// that these calls' results have had, which shows only where a sequence grows to the end of fp32's range (keys longer than one, no gate) and the
+// last bits decide which values are infinite.  They are so by measurement: -ffast-math lets the compiler regroup the substitution, and it does
+// (held to the order written here, fp32 results have other last bits).  Price: chunk_prepare2 43 instead of 41 us on one prompt of 65536 tokens and
+// 4 heads, none at B8 H16 T4096.  In place; A's upper triangle
 // within the 32x32 diagonal blocks must hold zeros, `sX` is a [32][36] scratch that is first written behind the first barrier.  Four waves solve a
 // diagonal block each (16 lanes a block), the merges' products go through the scratch.
-__device__ __forceinline__ void tri_inverse_64_ordered(float* M, float* sX, int tid) {
+__device__ __forceinline__ void tri_inverse_64_rows(float* M, float* sX, int tid) {
   const int wave = tid >> 6, lane = tid & 63;
   if (lane < 16) {
     const int r0 = 16 * wave, c = lane;
