@@ -1425,7 +1425,7 @@ constexpr int64_t kept_tiles(int64_t n) { return 3 * n + 1; }  // of a row that 
 
 template <typename K> int lds_limit(K* k) { return lnx_lds_limit(reinterpret_cast<const void*>(k), LDS_BYTES); }
 
-// B8 H16 T4096 bf16 (8192 chunks), us: dplr_prepare 433, dplr_chunk_scan 89, dplr_out 97 (48 KB of reads and 8 of writes per chunk: 4.8 TB/s)
+// B8 H16 T4096 bf16 (8192 chunks), us: dplr_prepare 447, dplr_chunk_scan 90, dplr_out 93 (48 KB of reads and 8 of writes per chunk: 5.0 TB/s)
 template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
   if (int rc = lds_limit(dplr_prepare_kernel<T>)) return rc;
@@ -1447,7 +1447,7 @@ template <typename T> int forward(const lnx_dplr_args* a, ChunkParams p, float* 
   return LNX_OK;
 }
 
-// Same shape: dplr_r 54, dplr_chunk_scan_bwd 89, dplr_u 443, dplr_grad 709 (two workgroups per CU leave 256 registers, and what a
+// Same shape: dplr_r 53, dplr_chunk_scan_bwd 88, dplr_u 441, dplr_grad 709 (two workgroups per CU leave 256 registers, and what a
 // token needs between the pair sums and the last products is more: rows stay as they were read, and three are loaded twice)
 template <typename T> int backward(const lnx_dplr_chunk_grads* g, const lnx_dplr_args* a, ChunkParams p, float* kept, float* scratch, hipStream_t st) {
   const int64_t rows = (int64_t)a->B * a->H;
